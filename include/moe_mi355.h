@@ -67,7 +67,7 @@ typedef struct moe_router_params {
 /*
  * Fused router: replaces MoEGate.forward (modeling_deepseek_v3.py:500-561,
  * modeling_deepseek_v2.py:483-533) and the routing lines of
- * MixtralSparseMoeBlock.forward (transformers 4.42.0).  One kernel computes the
+ * MixtralSparseMoeBlock.forward (transformers 4.42.0).  Computes the
  * fp32 logits x @ W^T, the scores (softmax, or sigmoid + e_score_correction_bias),
  * the group-limited selection, top-k (descending score, ties to the lower expert
  * index), renormalisation and routed scaling.
@@ -76,7 +76,10 @@ typedef struct moe_router_params {
  *   bias       device fp32 [E] (e_score_correction_bias) or NULL
  *   topk_idx   device int32 [n, k]   out
  *   topk_w     device fp32 [n, k]    out
- *   logits_out device fp32 [n, E]    out, may be NULL
+ *   logits_out device fp32 [n, E]    out, may be NULL.  With it the call is two launches: logits into the
+ *              buffer, routing from it.  Without it one launch keeps the logits on chip, which spreads
+ *              fewer than about 4000 tokens over fewer CUs (256 experts, 64 tokens: about three times the time)
+ * hidden: a multiple of 8 below 2^22.
  */
 int moe_router(const void* x, const void* w_gate, const float* bias,
                const moe_router_params* params, int32_t* topk_idx, float* topk_w,
@@ -257,13 +260,9 @@ int moe_rmsnorm(const void* x, const void* weight, float eps, int32_t n_tokens, 
 /*
  * moe_router reading its tokens THROUGH post_attention_layernorm (modeling_deepseek_v3.py:1361-1364:
  * hidden_states = self.post_attention_layernorm(hidden_states); self.mlp(hidden_states) -> the gate's
- * F.linear at :504-508): x holds the raw hidden states, each workgroup first computes the rstd of
- * its tokens (moe_rmsnorm's summation order), normalises every chunk on its way to the matrix
- * cores, xn = bf16(weight * bf16(f32(x) * rstd)), and writes the normalised rows once to x_norm
- * for the expert GEMMs.  Results (x_norm, indices, weights, logits) are bit-identical to
- * moe_rmsnorm followed by moe_router (with 32 experts or fewer, and with more than 64 experts and a
- * small batch -- up to 1024 tokens, 2048 above 128 experts --, where the fused form does not pay,
- * the call is those two launches).
+ * F.linear at :504-508): x holds the raw hidden states and x_norm receives
+ * xn = bf16(weight * bf16(f32(x) * rstd)) for the expert GEMMs.  moe_rmsnorm followed by moe_router,
+ * in one call.
  *   x           device bf16 [n, h]  raw hidden states
  *   norm_weight device bf16 [h]
  *   x_norm      device bf16 [n, h]  out (must not alias x)

@@ -73,7 +73,7 @@ def router(x: torch.Tensor, gate_w: torch.Tensor, bias, spec: RouterSpec, want_l
         raise ValueError("noaux_tc routing needs e_score_correction_bias")
     idx = torch.empty((n, k), dtype=torch.int32, device=x.device)
     w = torch.empty((n, k), dtype=torch.float32, device=x.device)
-    lg = torch.empty((n, E), dtype=torch.float32, device=x.device) if want_logits else None
+    lg = torch.empty((n, E), dtype=torch.float32, device=x.device)     # (the library routes from a logits matrix in memory)
     p = N.RouterParams(n, h, E, k, spec.n_group or 1, spec.topk_group or 1, SCORE[spec.scoring],
                        METHOD[spec.method], int(spec.norm_topk_prob), spec.scale_mode,
                        int(spec.logits_bf16), int(spec.weights_bf16), spec.norm_eps,
@@ -84,10 +84,10 @@ def router(x: torch.Tensor, gate_w: torch.Tensor, bias, spec: RouterSpec, want_l
         N.check(N.lib().moe_router_rmsnorm(_ptr(x), _ptr(norm_weight), float(eps), _ptr(gate_w), _ptr(bias),
                                            ctypes.byref(p), _ptr(xn), _ptr(idx), _ptr(w), _ptr(lg), _stream()),
                 "moe_router_rmsnorm")
-        return idx, w, lg, xn
+        return idx, w, lg if want_logits else None, xn
     N.check(N.lib().moe_router(_ptr(x), _ptr(gate_w), _ptr(bias), ctypes.byref(p), _ptr(idx), _ptr(w),
                                _ptr(lg), _stream()), "moe_router")
-    return idx, w, lg
+    return idx, w, lg if want_logits else None
 
 
 class Dispatch(NamedTuple):

@@ -248,3 +248,50 @@ def test_router_nan_inputs_keep_indices_valid(name):
                       2 if name == "mixtral_8" else 0)
     torch.cuda.synchronize()
     assert np.array_equal(torch.isnan(out.float()).all(dim=1).cpu().numpy(), np.isnan(ow).any(axis=1))
+
+
+@pytest.mark.parametrize("E,n", [(256, 4100), (256, 8200), (64, 16400), (128, 16400), (200, 6000), (192, 11000), (160, 9000)])
+def test_wave_tiles_of_two_by_two_stage_counts(E, n):
+    """Many tokens: 2 x 2 tiles per wave in workgroups of 4 and 8 waves (and one tile per wave where the last block of
+    64 experts would be half empty), rings of 4 and 3 stages of 128 k: hidden sizes with and without a last stage of
+    fewer k and with fewer stages than the ring, the last token block ragged.  The first and last rows (a token's
+    logits depend on its own row) bit for bit against the oracle."""
+    for h in (16, 128, 392, 640, 1160):
+        print(f"2x2 tiles E={E} n={n} h={h}", flush=True)
+        spec = O.RouterSpec.deepseek_v3(E, 6, 4, 2, True, 2.5)
+        g = torch.Generator().manual_seed(h + E)
+        x = torch.randn(n, h, generator=g).to(torch.bfloat16)
+        wg = (torch.randn(E, h, generator=g) * 0.1).to(torch.bfloat16)
+        bias = torch.randn(E, generator=g) * 0.01
+        idx, w, lg = gpu_router(x, wg, bias, spec)
+        for rows in (slice(0, 130), slice(n - 130, n)):
+            oi, ow, ol = O.router(bits(x[rows]), bits(wg), bias.numpy(), spec)
+            assert np.array_equal(lg[rows].view(np.uint32), ol.view(np.uint32)), (E, n, h)
+            assert np.array_equal(idx[rows], oi), (E, n, h)
+            assert np.array_equal(w[rows].view(np.uint32), ow.view(np.uint32)), (E, n, h)
+
+
+@pytest.mark.parametrize("E", [3, 8, 16, 17, 32, 33, 64, 72, 160, 256])
+@pytest.mark.parametrize("n,h", [(1, 8), (33, 136), (70, 1160)])
+def test_router_without_a_logits_buffer(E, n, h):
+    """A C caller that passes no logits buffer: the workgroup walks the expert blocks itself and routes from LDS."""
+    import ctypes
+    from moe_gen_amd import _native as N
+    spec = O.RouterSpec.deepseek_v3(E, 2, 4, 2, True, 2.5) if E % 8 == 0 else O.RouterSpec.deepseek_v2(E, 2, "greedy")
+    g = torch.Generator().manual_seed(E + h)
+    x = torch.randn(n, h, generator=g).to(torch.bfloat16)
+    wg = (torch.randn(E, h, generator=g) * 0.1).to(torch.bfloat16)
+    bias = (torch.randn(E, generator=g) * 0.01) if spec.method == "noaux_tc" else None
+    from moe_gen_amd import ops
+    p = N.RouterParams(n, h, E, 2, spec.n_group, spec.topk_group, ops.SCORE[spec.scoring], ops.METHOD[spec.method],
+                       int(spec.norm_topk_prob), spec.scale_mode, 0, 0, spec.norm_eps, spec.routed_scaling_factor)
+    xd, wd, bd = x.cuda(), wg.cuda(), None if bias is None else bias.cuda()
+    idx = torch.full((n, 2), -1, dtype=torch.int32, device="cuda")
+    w = torch.full((n, 2), -1.0, device="cuda")
+    print(f"no logits buffer E={E} n={n} h={h}", flush=True)
+    N.check(N.lib().moe_router(xd.data_ptr(), wd.data_ptr(), None if bd is None else bd.data_ptr(), ctypes.byref(p),
+                               idx.data_ptr(), w.data_ptr(), None, torch.cuda.current_stream().cuda_stream), "moe_router")
+    torch.cuda.synchronize()
+    oi, ow, _ = O.router(bits(x), bits(wg), None if bias is None else bias.numpy(), spec)
+    assert np.array_equal(idx.cpu().numpy(), oi)
+    assert np.array_equal(w.cpu().numpy().view(np.uint32), ow.view(np.uint32))
