@@ -174,8 +174,10 @@ int moe_dispatch_static(const int32_t* topk_idx, int32_t n_tokens, int32_t top_k
  * weights, never on the row's place among its expert's rows, on any expert's count or on the kernel that computes
  * it.  With bf16 weights that holds across calls too.  With fp8 weights a call that the one-workgroup-per-tile kernel
  * serves alone adds a row's products in another order than a call that launches both kernels (other starting stages
- * of its k loops, and another order within a stage for experts of up to 64 rows), and a row's last bit may differ
- * between the two kinds of call.
+ * of its k loops), and its experts of up to 64 rows are multiplied by the fp8 values as they are, the block scale being
+ * applied to the fp32 sum of each 128 k instead of to the weight before it is rounded to bf16: a row may then differ
+ * between the two kinds of call by the rounding of the weights (2^-9).
+ * Calls in which no expert has more than 16 rows run on a kernel of one wave per 32 weight rows.
  */
 enum { MOE_PHASE_GATE_UP = 1, MOE_PHASE_DOWN = 2, MOE_PHASE_BOTH = 3 };
 size_t moe_grouped_workspace_bytes(int32_t n_rows, int32_t n_experts);
@@ -189,7 +191,7 @@ int moe_grouped_swiglu_bf16(const void* x, int32_t x_rows, const int32_t* row_ma
 /*
  * W8A16 variant: weights are fp8 e4m3fn with one fp32 scale per 128x128 block;
  * each weight element is dequantised in registers as bf16(f32(q) * scale)
- * (deepseek_v3_dequantization, Wrapper.py:109-138) before it reaches the MFMA.
+ * (deepseek_v3_dequantization, Wrapper.py:109-138) before it reaches the MFMA (few rows: see above).
  *   s_gate/s_up  device arrays of E pointers to fp32 [ceil(I/128), ceil(h/128)]
  *   s_down       device array  of E pointers to fp32 [ceil(h/128), ceil(I/128)]
  * Requires h % 128 == 0 and I % 128 == 0.
@@ -202,6 +204,38 @@ int moe_grouped_swiglu_w8a16(const void* x, int32_t x_rows, const int32_t* row_m
                              int32_t n_rows, int32_t n_experts, int32_t hidden, int32_t inter,
                              void* act, void* y, int32_t phases, void* workspace,
                              size_t workspace_bytes, void* stream);
+
+/*
+ * One expert MLP problem: the arguments of the two calls above (the bf16 form leaves the scales NULL), plus
+ *   max_rows  no expert has more rows than this (0: not known).  A layer call on n tokens knows it: a token goes to an
+ *             expert at most once
+ */
+typedef struct moe_mlp_group {
+    const void* x;
+    int32_t x_rows, n_rows;
+    const int32_t* row_map;
+    const void* const* w_gate;
+    const void* const* w_up;
+    const void* const* w_down;
+    const float* const* s_gate;
+    const float* const* s_up;
+    const float* const* s_down;
+    const int32_t* offsets;
+    int32_t n_experts, inter, max_rows, reserved;
+    void* act;
+    void* y;
+} moe_mlp_group;
+
+/*
+ * The routed experts and the shared expert(s) of a layer (DeepseekV3MoE.forward, modeling_deepseek_v3.py:618-625; one MLP
+ * of any intermediate size, n_experts == 1) in one call, both of the same weight type (fp8 != 0: fp8 with block scales).
+ * Where moe_shared_joins says 1 they share their launches: the shared expert's tiles run next to the routed experts';
+ * otherwise they run one after the other.  shared == NULL: the routed experts alone.  With bf16 weights the bits are
+ * those of separate calls.
+ */
+int moe_grouped_swiglu_joint(const moe_mlp_group* routed, const moe_mlp_group* shared, int32_t hidden, int32_t fp8,
+                             int32_t phases, void* stream);
+int moe_shared_joins(const moe_mlp_group* routed, const moe_mlp_group* shared, int32_t hidden);
 
 /*
  * Write n 64-bit words (device pointers of a wave of experts, say) into device memory at dst, from host memory

@@ -25,6 +25,17 @@ class RouterParams(ctypes.Structure):
     ]
 
 
+class MlpGroup(ctypes.Structure):
+    """struct moe_mlp_group."""
+    _fields_ = [
+        ("x", c_void_p), ("x_rows", c_int32), ("n_rows", c_int32), ("row_map", c_void_p),
+        ("w_gate", c_void_p), ("w_up", c_void_p), ("w_down", c_void_p),
+        ("s_gate", c_void_p), ("s_up", c_void_p), ("s_down", c_void_p), ("offsets", c_void_p),
+        ("n_experts", c_int32), ("inter", c_int32), ("max_rows", c_int32), ("reserved", c_int32),
+        ("act", c_void_p), ("y", c_void_p),
+    ]
+
+
 # name -> (restype, argtypes); every symbol include/moe_mi355.h declares
 SIGNATURES = {
     "moe_last_error": (ctypes.c_char_p, []),
@@ -45,6 +56,9 @@ SIGNATURES = {
     "moe_grouped_swiglu_w8a16": (ctypes.c_int, [c_void_p, c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                                 c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_int32,
                                                 c_int32, c_void_p, c_void_p, c_int32, c_void_p, c_size_t, c_void_p]),
+    "moe_grouped_swiglu_joint": (ctypes.c_int, [ctypes.POINTER(MlpGroup), ctypes.POINTER(MlpGroup), c_int32, c_int32, c_int32,
+                                                c_void_p]),
+    "moe_shared_joins": (ctypes.c_int, [ctypes.POINTER(MlpGroup), ctypes.POINTER(MlpGroup), c_int32]),
     "moe_dequant_fp8_block128": (ctypes.c_int, [c_void_p, c_void_p, c_int32, c_int32, c_void_p, c_void_p]),
     "moe_combine": (ctypes.c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_int32,
                                    c_int32, c_int32, c_void_p, c_void_p]),

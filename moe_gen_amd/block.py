@@ -55,17 +55,22 @@ def _span(timer, name):
     return timer.span(name) if timer is not None else _NoSpan()
 
 
-def _grouped(timer, tag, x, row_map, ptrs, offsets, n_rows):
+def _grouped(timer, tag, x, row_map, ptrs, offsets, n_rows, max_rows=0):
     """Both launches of the expert MLP; split (and timed per launch) when a timer is attached."""
-    if timer is None:
-        return ops.grouped_swiglu(x, row_map, ptrs, offsets, n_rows)
-    act = torch.empty((n_rows, ptrs.inter), dtype=torch.bfloat16, device=x.device)
-    y = torch.empty((n_rows, ptrs.hidden), dtype=torch.bfloat16, device=x.device)
-    with timer.span(tag + "_gate_up"):
-        ops.grouped_swiglu(x, row_map, ptrs, offsets, n_rows, act, y, ops.PHASE_GATE_UP)
-    with timer.span(tag + "_down"):
-        ops.grouped_swiglu(x, row_map, ptrs, offsets, n_rows, act, y, ops.PHASE_DOWN)
+    m, _, y = ops.mlp_group(x, row_map, ptrs, offsets, n_rows, max_rows)
+    if n_rows:
+        _launch(timer, tag, m, None, ptrs.hidden, ptrs.fp8)
     return y
+
+
+def _launch(timer, tag, routed, shared, hidden, fp8):
+    if timer is None:
+        ops.grouped_swiglu_joint(routed, shared, hidden, fp8)
+        return
+    with timer.span(tag + "_gate_up"):
+        ops.grouped_swiglu_joint(routed, shared, hidden, fp8, ops.PHASE_GATE_UP)
+    with timer.span(tag + "_down"):
+        ops.grouped_swiglu_joint(routed, shared, hidden, fp8, ops.PHASE_DOWN)
 
 
 def _require_silu(config):
@@ -380,42 +385,6 @@ def _engine_experts(block, timer, tag, experts, a_rows, row_map, offsets, n_rows
     return y
 
 
-def _shared_joins_routed(block, experts, staged, shared, n, k, fused_gather, cache):
-    """Whether this call runs the shared expert as one more group of the routed experts' grouped call, and if so the
-    pointer tables of the 1 + E groups and the offset / row-map buffers of the joint call (cached per token count).
-
-    It does when the shared expert alone would leave most CUs without a tile -- (n / 256 + 1) row tiles times I / 128
-    column tiles fewer than 3/8 of the device's CUs: DeepSeek-V3 up to 1024 tokens, where the step gains 2-5 %; from
-    2048 tokens on a launch pair of its own, with 256-row tiles, is the faster by 0.6 % -- and has the routed experts'
-    shapes and dtype (one shared expert: DeepSeek-V3 / R1; DeepSeek-V2's two are one MLP of twice the width), with all
-    weights resident.  `block.join_shared = False` keeps the two calls apart."""
-    if shared is None or not fused_gather or not getattr(block, "join_shared", True):
-        return None
-    if staged or engine_backed(shared):
-        return None
-    E = len(experts)
-    fit = cache.get("joint_fit")
-    if fit is None or fit[0] != (id(shared), id(experts[0]), E):
-        ts, tr = _tensors_of(shared), _tensors_of(experts[0])
-        same = ts[0].shape == tr[0].shape and ts[0].dtype == tr[0].dtype and ts[2].shape == tr[2].shape
-        dev = ts[0].device
-        fit = ((id(shared), id(experts[0]), E), same, -(-ts[0].shape[0] // 128), dev,
-               torch.cuda.get_device_properties(dev).multi_processor_count)
-        cache["joint_fit"] = fit
-    _, same, col_tiles, dev, cus = fit
-    if not same or (n // 256 + 1) * col_tiles * 8 >= 3 * cus:
-        return None
-    ptrs = collect_pointers([shared] + experts, cache.setdefault("shared+routed", {}))
-    bufs = cache.get("joint")
-    if bufs is None or bufs[0] != (n, k, E, dev):
-        off = torch.zeros(E + 2, dtype=torch.int32, device=dev)        # [0, n, n + routed offsets 1 .. E]
-        rows = torch.empty(n + n * k, dtype=torch.int32, device=dev)   # [0 .. n-1, routed row map]
-        rows[:n] = torch.arange(n, dtype=torch.int32, device=dev)
-        bufs = ((n, k, E, dev), off, rows)
-        cache["joint"] = bufs
-    return ptrs, bufs[1], bufs[2]
-
-
 @torch.no_grad()
 def moe_forward(block, hidden_states: torch.Tensor, spec: ops.RouterSpec, gate_weight: torch.Tensor,
                 bias, experts, shared, combine_mode: int, want_logits: bool = False):
@@ -447,38 +416,37 @@ def moe_forward(block, hidden_states: torch.Tensor, spec: ops.RouterSpec, gate_w
     fused_gather = getattr(block, "fused_gather", True)
     experts = list(experts)
     staged = any_engine_backed(experts)            # decided expert by expert, as the reference's initializers do
-    joined = _shared_joins_routed(block, experts, staged, shared, n, k, fused_gather, cache)
-    if joined is not None:
-        # The shared expert as one more group of the routed call: all n token rows IN FRONT of the n*k routed rows
-        # (identity entries at the head of the row map, written once; the routed offsets shifted by n).  Its tiles
-        # then fill the CUs next to the routed experts' instead of a launch pair of their own that has a tile for a
-        # fraction of them -- in front, because they are the tallest of the call and would be its tail at the end.
-        ptrs_all, off_all, map_all = joined
-        with _span(timer, "dispatch"):
-            d = ops.dispatch(idx, E, None, out_row_map=map_all[n:])
-            torch.add(d.offsets, n, out=off_all[1:])
-        block.last_counts = d.counts
-        y_all = _grouped(timer, "routed", x, map_all, ptrs_all, off_all, n * k + n)
-        with _span(timer, "combine"):
-            out = ops.combine(y_all[n:], d.pos, idx, w, y_all[:n], combine_mode, residual=residual)
-        return out.view(*shape), logits
     with _span(timer, "dispatch"):
         d = ops.dispatch(idx, E, None if fused_gather else x, want_row_map=fused_gather)
     counts, offsets, pos, row_map = d.counts, d.offsets, d.pos, d.row_map
     block.last_counts = counts
     a_rows = x if fused_gather else d.xs
-    if staged:
-        y = _engine_experts(block, timer, "routed", experts, a_rows, row_map, offsets, n * k, counts)
-    else:
-        y = _grouped(timer, "routed", a_rows, row_map, collect_pointers(experts, cache.setdefault("routed", {})),
-                     offsets, n * k)
-    sh = None
+    so = None
     if shared is not None:
         so = cache.get("shared_off")
         if so is None or so[0] != n or so[1].device != x.device:
             so = (n, torch.tensor([0, n], dtype=torch.int32, device=x.device))
             cache["shared_off"] = so
-        if engine_backed(shared):
+    sh, shared_staged = None, shared is not None and engine_backed(shared)
+    if staged:
+        y = _engine_experts(block, timer, "routed", experts, a_rows, row_map, offsets, n * k, counts)
+    else:
+        ptrs = collect_pointers(experts, cache.setdefault("routed", {}))
+        if shared is not None and not shared_staged and n and getattr(block, "join_shared", True):
+            # the shared expert's tiles in the routed experts' launches where that pays (a small batch: alone it has a
+            # tile for a fraction of the CUs); `block.join_shared = False` keeps the two apart
+            sp = collect_pointers([shared], cache.setdefault("shared", {}))
+            routed_m, _, y = ops.mlp_group(a_rows, row_map, ptrs, offsets, n * k, n)
+            shared_m, _, sh = ops.mlp_group(x, None, sp, so[1], n)
+            if sp.fp8 == ptrs.fp8 and ops.shared_joins(routed_m, shared_m, h):
+                _launch(timer, "routed", routed_m, shared_m, h, ptrs.fp8)
+            else:
+                _launch(timer, "routed", routed_m, None, h, ptrs.fp8)
+                _launch(timer, "shared", shared_m, None, h, sp.fp8)
+        else:
+            y = _grouped(timer, "routed", a_rows, row_map, ptrs, offsets, n * k, n)
+    if shared is not None and sh is None:
+        if shared_staged:
             sh = _engine_experts(block, timer, "shared", [shared], x, None, so[1], n, None)
         else:
             sh = _grouped(timer, "shared", x, None, collect_pointers([shared], cache.setdefault("shared", {})), so[1], n)

@@ -96,6 +96,15 @@ struct GemmArgs {
                                 // is left goes to the other kernel as 128-row half tiles if that pays (tail_tiles)
 };
 
+// What a launch of the one-workgroup-per-tile kernel or of the thin kernel works on: the routed experts and, in front of
+// them, the first `shared_tiles` (units) of a second problem with matrices and buffers of its own, the layer's shared
+// expert.  A launch pair for the shared expert alone has a tile for a fraction of the CUs (DeepSeek-V2-236B, 64 tokens:
+// 24 and 20 tiles, 70 + 44 us for 94 MB).
+struct GemmPair {
+    GemmArgs p[2];              // routed, shared
+    int shared_tiles;
+};
+
 // LDS rows are 128 bytes = 8 chunks of 16 bytes; chunk c of row r is stored at chunk c ^ swz(r).
 // swz makes any 8 consecutive rows hit 8 different chunks (32 banks x 4 B = one 128-byte row per
 // cycle) AND any 16 consecutive rows hit 16 different (row parity, chunk) slots (64 banks =
@@ -172,6 +181,17 @@ __device__ __forceinline__ u32x4 dequant8(uint32_t q0, uint32_t q1, float sc) {
     const f32x2 c2 = __builtin_amdgcn_cvt_pk_f32_fp8(q1, false), c3 = __builtin_amdgcn_cvt_pk_f32_fp8(q1, true);
     return u32x4{pack_bf16(c0[0] * sc, c0[1] * sc), pack_bf16(c1[0] * sc, c1[1] * sc),
                  pack_bf16(c2[0] * sc, c2[1] * sc), pack_bf16(c3[0] * sc, c3[1] * sc)};
+}
+
+// 8 fp8 weights (two dwords) -> the same values as bf16 (exact), one instruction per pair.  The streamers for few rows
+// multiply them unscaled and apply the block scale to the fp32 sum of each 128 k: a quarter of dequant8's vector
+// instructions, and a weight keeps the bits that bf16(f32(q) * s) rounds away.
+__device__ __forceinline__ bf16x8 widen8(uint32_t q0, uint32_t q1) {
+    const u32x4 v = {__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(q0, 1.0f, false)),
+                     __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(q0, 1.0f, true)),
+                     __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(q1, 1.0f, false)),
+                     __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(q1, 1.0f, true))};
+    return __builtin_bit_cast(bf16x8, v);
 }
 
 // Epilogue values of one lane for one pair of accumulators: 4 consecutive output columns of one row.
@@ -776,14 +796,17 @@ __device__ __forceinline__ void stream8_tile(const GemmArgs& g, SBuf buf0, SBuf 
         asm volatile("" ::: "memory");
         scales(p + 1, sset ^ 1);
         __builtin_amdgcn_sched_barrier(0);
+        f32x4 part[TG][2];                      // the block's sums of unscaled weights
+#pragma unroll
+        for (int t = 0; t < TG; ++t) { part[t][0] = f32x4{0}; part[t][1] = f32x4{0}; }
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             bf16x8 wa[2][2];
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 const u32x4 raw = *reinterpret_cast<const u32x4*>(rd.w + w_rd + j * 2048 + (((4 * h + fq) ^ wkey) << 4));
-                wa[j][0] = __builtin_bit_cast(bf16x8, dequant8(raw[0], raw[1], rsc[sset][j]));
-                wa[j][1] = __builtin_bit_cast(bf16x8, dequant8(raw[2], raw[3], rsc[sset][j]));
+                wa[j][0] = widen8(raw[0], raw[1]);
+                wa[j][1] = widen8(raw[2], raw[3]);
             }
 #pragma unroll
             for (int s2 = 0; s2 < 2; ++s2) {
@@ -791,8 +814,8 @@ __device__ __forceinline__ void stream8_tile(const GemmArgs& g, SBuf buf0, SBuf 
 #pragma unroll
                 for (int t = 0; t < TG; ++t) {
                     const bf16x8 tf = *reinterpret_cast<const bf16x8*>(rd.t + t_rd + t * 16 * 256 + coff);
-                    acc[t][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[0][s2], tf, acc[t][0], 0, 0, 0);
-                    acc[t][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[1][s2], tf, acc[t][1], 0, 0, 0);
+                    part[t][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[0][s2], tf, part[t][0], 0, 0, 0);
+                    part[t][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[1][s2], tf, part[t][1], 0, 0, 0);
                 }
                 // the refill of the freed buffer goes out between the four groups of matrix instructions (2, 2, 1, 1
                 // DMA instructions): a wave that issues all six first stands in the memory pipeline's queue while its
@@ -804,6 +827,12 @@ __device__ __forceinline__ void stream8_tile(const GemmArgs& g, SBuf buf0, SBuf 
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
+#pragma unroll
+        for (int t = 0; t < TG; ++t)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[t][j][i] = __builtin_fmaf(part[t][j][i], rsc[sset][j], acc[t][j][i]);
     };
     scales(0, 0);
     dma(0, buf0);
@@ -1239,7 +1268,7 @@ __device__ __forceinline__ int tail_tiles(const GemmArgs& g, int total, int own)
 }
 
 template <bool PAIR>   // whether an expert of PAIR_LO .. PAIR_HI rows is cut in the middle (bf16 weights)
-__device__ __forceinline__ int tiles_of(int count) {
+__host__ __device__ __forceinline__ int tiles_of(int count) {
     constexpr int SINGLE = 192;   // rows that one tile may hold
     if (count <= SINGLE) return count > 0 ? 1 : 0;
     // bf16 weights: an expert of 257 to 384 rows is cut in the middle, into two tiles of the 192-row body that run
@@ -1459,7 +1488,7 @@ __device__ __forceinline__ void stream8x(const GemmArgs& g, SBuf b0, SBuf b1, SB
 
 // One workgroup per (M tile, N tile); serves what the persistent kernel does not take (few rows per expert, odd K).
 template <int WN, bool SWIGLU, bool W8>
-__global__ __launch_bounds__(128 * WN) void grouped_gemm_kernel(GemmArgs g) {
+__global__ __launch_bounds__(128 * WN) void grouped_gemm_kernel(GemmPair pair_of) {
     constexpr int NT = 128 * WN;
     // Three weight arrays of 32 KiB and token arrays of 16 KiB (fp8 weights: three, 128 rows; the second one 24 KiB)
     // or 24 KiB (bf16: two, 192 rows) -- the buffers of the weight streamers, written by DMA, as separate objects so
@@ -1481,18 +1510,22 @@ __global__ __launch_bounds__(128 * WN) void grouped_gemm_kernel(GemmArgs g) {
     __shared__ int s_sel[5];
     const int tid = threadIdx.x;
 
-    // ---- M-tile prefix over experts ----
-    ExpertOfThread mine;
-    const bool s8_ok = !g.row_map || g.a_bytes < (1ull << 32);   // (the weight streamer addresses gathered rows with 32-bit offsets)
-    int run = mtile_prefix_scan<NT>(g, tid, s_pref, s_wtot, mine, [&](int c) { return own_tiles<W8>(g, c); }, [](int, int, int) {});
-    const int total = run * g.n_tiles_n;
-
     // ---- XCD-aware id: groups of 4 consecutive tiles (the M tiles of one N tile first) go round-robin to the XCDs
     // (workgroup ids are dealt to the XCDs one by one).  The tiles of a multi-tile expert that read the same
     // weights then share them through one XCD's L2, and dealing small groups round keeps the XCDs even whatever
     // the number of tiles and however much one expert's tiles cost more than another's ----
     const int slot = blockIdx.x >> 3;
     int v = (((slot >> 2) << 3) + (blockIdx.x & 7)) * 4 + (slot & 3);
+    const bool of_shared = v < pair_of.shared_tiles;
+    const GemmArgs& g = pair_of.p[of_shared ? 1 : 0];
+    if (!of_shared) v -= pair_of.shared_tiles;
+
+    // ---- M-tile prefix over experts ----
+    ExpertOfThread mine;
+    const bool s8_ok = !g.row_map || g.a_bytes < (1ull << 32);   // (the weight streamer addresses gathered rows with 32-bit offsets)
+    int run = mtile_prefix_scan<NT>(g, tid, s_pref, s_wtot, mine, [&](int c) { return own_tiles<W8>(g, c); }, [](int, int, int) {});
+    const int total = run * g.n_tiles_n;
+
     // Past this kernel's own tiles: the tiles that the persistent kernel leaves at the end of ITS tile space, two
     // workgroups (128-row halves, neighbours on one XCD) per tile.  The prefix is rebuilt over that space.
     int half = -1;
@@ -1593,6 +1626,182 @@ __global__ __launch_bounds__(128 * WN) void grouped_gemm_kernel(GemmArgs g) {
         if (t1 - t0 > 128) {
             __syncthreads();
             gemm_tile<2, WN, SWIGLU, W8, false>(g, stage(0), stage(1), e, t0 + 128, t1, n_tile);
+        }
+    }
+}
+
+// ---- thin kernel: calls in which no expert has more than 16 rows (decoding a few sequences) ----
+//
+// Such a call touches a few experts, and cut into tiles of 256 weight rows it has fewer tiles than the chip has CUs
+// (one token of DeepSeek-V2-Lite: 66) or two and a half rounds of them.  Here the unit is a WAVE with 32 weight rows --
+// 16 gate rows and the matching up rows, or 32 down rows -- and the whole K, each wave a workgroup of its own: no
+// barrier, six of them per CU, and nothing to wait for but its own DMA.  A stage is 128 bytes of each weight row (64 k of
+// bf16, 128 of fp8: whole lines) and the same k of 16 token rows (rows that do not exist cost no request), NB stages in
+// a ring.  Every matrix instruction gets the k values that the streamers above give it, in the same lanes and the same
+// order, so a row's bits are those of a larger call (fp8: of a larger call whose experts have up to 64 rows).
+// Measured (us, tile kernel -> this): DeepSeek-V2-Lite, one token (8 x 1408 of 2048) 25 + 25 and 19 + 33 -> 21 and 11;
+// DeepSeek-V3, 5 tokens (38 experts, fp8) 190 and 115 -> 171 and 88 = 6.4 TB/s.  Weights loaded into registers instead
+// reach 4 ... 5 TB/s: a fragment load then takes half a line from each of 16 rows.
+template <bool SWIGLU, bool W8>
+__global__ __launch_bounds__(64) void grouped_gemm_thin_kernel(GemmPair pair_of) {
+    constexpr int TBYTES = W8 ? 4096 : 2048;      // 16 token rows of a stage
+    constexpr int NB = W8 ? 3 : 4;                // stages in LDS
+    constexpr int NDT = TBYTES / 1024, NI = 4 + NDT;   // DMA instructions per stage: 4 for the weights
+    constexpr int NCOL = SWIGLU ? 16 : 32;        // output columns of a wave
+    constexpr int SB = 4096 + TBYTES;
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[NB * SB];
+    const int lane = threadIdx.x;
+    const bool of_shared = (int)blockIdx.x < pair_of.shared_tiles;
+    const GemmArgs& g = pair_of.p[of_shared ? 1 : 0];
+    const int unit = (int)blockIdx.x - (of_shared ? 0 : pair_of.shared_tiles);
+    const int K = g.K, N = g.N;
+    const int tiles = (N + NCOL - 1) / NCOL;
+
+    // the (unit / tiles)-th expert that has rows: 256 experts at a time, 4 per lane
+    int left = unit / tiles, e = -1, row0 = 0, row_end = 0;
+    for (int base = 0; base < g.E; base += 256) {
+        int o[5], c = 0;
+#pragma unroll
+        for (int j = 0; j < 5; ++j) o[j] = g.offsets[min(base + 4 * lane + j, g.E)];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) c += o[j + 1] > o[j] ? 1 : 0;
+        int inc = c;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int up = __shfl_up(inc, d);
+            if (lane >= d) inc += up;
+        }
+        const int tot = __builtin_amdgcn_readlane(inc, 63);
+        if (left < tot) {
+            int k = left - (inc - c), ce = 0, c0 = 0, c1 = 0;
+            const uint64_t owner = __ballot(k >= 0 && k < c);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (o[j + 1] > o[j]) {
+                    if (k == 0) { ce = base + 4 * lane + j; c0 = o[j]; c1 = o[j + 1]; }
+                    --k;
+                }
+            const int l = __builtin_ctzll(owner);
+            e = __builtin_amdgcn_readlane(ce, l);
+            row0 = __builtin_amdgcn_readlane(c0, l);
+            row_end = __builtin_amdgcn_readlane(c1, l);
+            break;
+        }
+        left -= tot;
+    }
+    if (e < 0) return;
+    const int n0 = (unit % tiles) * NCOL;
+    const int nk = K / (W8 ? 128 : 64);
+    const int rot = (n0 / (SWIGLU ? 128 : 256)) % nk;      // the k rotation of the N tile these columns belong to
+    auto stage_at = [&](int k) { const int s = min(k, nk - 1) + rot; return s >= nk ? s - nk : s; };
+
+    const uint8_t* bm0 = uni_ptr(g.b0[e]);
+    const uint8_t* bm1 = SWIGLU ? uni_ptr(g.b1[e]) : bm0;
+    gptr_f32 sc0 = nullptr, sc1 = nullptr;                 // scales of the 128 rows the wave's columns lie in
+    if (W8) {
+        sc0 = (gptr_f32)(uintptr_t)uni_ptr(g.s0[e]) + (n0 >> 7) * nk;
+        sc1 = SWIGLU ? (gptr_f32)(uintptr_t)uni_ptr(g.s1[e]) + (n0 >> 7) * nk : sc0;
+    }
+    // DMA: weights, instruction i: fragment i / 2 (gate / up, or the two halves of the 32 down rows), rows 8 (i & 1) +
+    // lane / 8; tokens, instruction i: 8 (fp8: 4) rows; chunks swizzled as in the streamers
+    const int lr = lane >> 3, pp = lane & 7;
+    const uint32_t row_bytes = (uint32_t)K * (W8 ? 1 : 2);
+    uint32_t w_voff[4], t_voff[4];                         // (NDT of the latter are used)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int fr = 8 * (i & 1) + lr;
+        w_voff[i] = (uint32_t)min(n0 + (SWIGLU ? 0 : 16 * (i >> 1)) + fr, N - 1) * row_bytes + (uint32_t)((pp ^ (W8 ? wsw(fr) : swz(fr))) << 4);
+    }
+    const int frow = lane & 15, q = lane >> 4;
+    const int fq = ((q & 1) << 1) | (q >> 1);
+    const uint32_t w_rd = (uint32_t)(frow * 128), wkey = (uint32_t)(W8 ? wsw(frow) : swz(frow));
+    const uint32_t t_rd = 4096u + (uint32_t)(frow * (W8 ? 256 : 128)), tkey = (uint32_t)(W8 ? tsw(frow) : swz(frow));
+
+    for (int r0 = row0; r0 < row_end; r0 += 16) {          // (more than once only if a caller's row bound was wrong)
+        const uint8_t* a_base = reinterpret_cast<const uint8_t*>(g.a) + (g.row_map ? (size_t)0 : (size_t)r0 * K * 2);
+        const int a_records = g.row_map ? (int)(uint32_t)g.a_bytes : min(16, row_end - r0) * K * 2;
+#pragma unroll
+        for (int i = 0; i < NDT; ++i) {
+            const int tr = W8 ? 4 * i + (lane >> 4) : 8 * i + lr;
+            const int r = min(r0 + tr, row_end - 1);
+            const int src = g.row_map ? ((gptr_i32)(uintptr_t)g.row_map)[r] : r - r0;
+            t_voff[i] = (uint32_t)src * (uint32_t)(K * 2) + (uint32_t)((W8 ? (lane & 15) ^ tsw(tr) : pp ^ swz(tr)) << 4);
+            if (r0 + tr >= row_end || (g.row_map && (unsigned)src >= (unsigned)g.a_rows)) t_voff[i] = 0xfffffff0u;
+        }
+        auto dma = [&](int k, int buf) __attribute__((always_inline)) {
+            const int live = uni(k < nk ? -1 : 0);         // past the end: empty descriptors, the instructions still count
+            uint8_t* d = lds + buf * SB;
+            const uint32_t so = (uint32_t)stage_at(k) * 128u;
+            const __amdgpu_buffer_rsrc_t r0d = __builtin_amdgcn_make_buffer_rsrc((void*)bm0, 0, live, 0x00020000);
+            const __amdgpu_buffer_rsrc_t r1d = __builtin_amdgcn_make_buffer_rsrc((void*)bm1, 0, live, 0x00020000);
+            const __amdgpu_buffer_rsrc_t rad = __builtin_amdgcn_make_buffer_rsrc((void*)a_base, 0, live & a_records, 0x00020000);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r0d, (lds_u8)d, 16, w_voff[0], so, 0, 2);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r0d, (lds_u8)(d + 1024), 16, w_voff[1], so, 0, 2);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r1d, (lds_u8)(d + 2048), 16, w_voff[2], so, 0, 2);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r1d, (lds_u8)(d + 3072), 16, w_voff[3], so, 0, 2);
+#pragma unroll
+            for (int i = 0; i < NDT; ++i)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rad, (lds_u8)(d + 4096 + i * 1024), 16, t_voff[i], W8 ? 2 * so : so, 0, 0);
+        };
+        f32x4 acc[2] = {f32x4{0}, f32x4{0}};
+        float v0 = 0.0f, v1 = 0.0f;                        // fp8: lane l holds the scales of stage 64 i + l
+        if (W8) { v0 = sc0[stage_at(lane)]; v1 = sc1[stage_at(lane)]; }
+        for (int i = 0; i < NB - 1; ++i) dma(i, i);
+        // (waits by hand: the compiler's own, in front of the readlane below, would cover the DMA of the next stage too)
+        if (W8) asm volatile("s_waitcnt vmcnt(%2)" : "+v"(v0), "+v"(v1) : "n"((NB - 1) * NI));
+        int buf = 0;
+        for (int k = 0; k < nk; ++k) {
+            // this wave's DMA of stage k has landed and its reads of stage k - 1, whose buffer is refilled, have returned
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"((NB - 2) * NI) : "memory");
+            if (W8 && (k & 63) == 0 && k > 0) {
+                v0 = sc0[stage_at(k + lane)];
+                v1 = sc1[stage_at(k + lane)];
+                asm volatile("s_waitcnt vmcnt(0)" : "+v"(v0), "+v"(v1));
+            }
+            dma(k + NB - 1, buf == 0 ? NB - 1 : buf - 1);
+            const uint8_t* b = lds + buf * SB;
+            if (W8) {
+                f32x4 part[2] = {f32x4{0}, f32x4{0}};
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    u32x4 raw[2];
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) raw[j] = *reinterpret_cast<const u32x4*>(b + j * 2048 + w_rd + (((4 * h + fq) ^ wkey) << 4));
+#pragma unroll
+                    for (int s2 = 0; s2 < 2; ++s2) {
+                        const bf16x8 tf = *reinterpret_cast<const bf16x8*>(b + t_rd + (((8 * h + 2 * fq + s2) ^ tkey) << 4));
+#pragma unroll
+                        for (int j = 0; j < 2; ++j)
+                            part[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(widen8(raw[j][2 * s2], raw[j][2 * s2 + 1]), tf, part[j], 0, 0, 0);
+                    }
+                }
+                const float c0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v0), k & 63));
+                const float c1 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v1), k & 63));
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    acc[0][i] = __builtin_fmaf(part[0][i], c0, acc[0][i]);
+                    acc[1][i] = __builtin_fmaf(part[1][i], c1, acc[1][i]);
+                }
+            } else {
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    const uint32_t coff = (uint32_t)((4 * s + fq) ^ wkey) << 4;      // (wkey == tkey)
+                    const bf16x8 tf = *reinterpret_cast<const bf16x8*>(b + t_rd + coff);
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+                        acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(b + j * 2048 + w_rd + coff), tf, acc[j], 0, 0, 0);
+                }
+            }
+            buf = buf + 1 == NB ? 0 : buf + 1;
+        }
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");   // no DMA may land in LDS after the workgroup has gone
+        const int r = r0 + frow;
+        if (r < row_end) {
+#pragma unroll
+            for (int j = 0; j < (SWIGLU ? 1 : 2); ++j) {
+                const int col = n0 + 16 * j + 4 * q;
+                if (col < N) *reinterpret_cast<u32x2*>(g.c + (size_t)r * N + col) = epilogue_pack<SWIGLU>(acc[j], acc[SWIGLU ? 1 : j]);
+            }
         }
     }
 }
@@ -1928,18 +2137,44 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmArgs g
     }
 }
 
+// shared: the second problem of the launch (NULL: none), of n_shared rows
 template <int WN, bool SWIGLU, bool W8>
-int launch_tiles(const GemmArgs& g, int n_rows, hipStream_t st) {
+int launch_tiles(const GemmArgs& g, int n_rows, const GemmArgs* shared, int n_shared, hipStream_t st) {
     auto kern = grouped_gemm_kernel<WN, SWIGLU, W8>;
     // sum_e tiles_of(c_e) <= sum_e (c_e / 128 + 1); with the larger experts elsewhere, one tile per expert that has rows
     const long max_mtiles = g.cold_max <= 192 ? (g.pair_rows ? 2 : 1) * (long)(g.E < n_rows ? g.E : n_rows) : (long)n_rows / 128 + g.E;
+    GemmPair pair{};
+    pair.p[0] = g;
+    if (shared) {
+        pair.p[1] = *shared;
+        pair.shared_tiles = tiles_of<!W8>(n_shared) * shared->n_tiles_n;
+    }
     // (+ the persistent kernel's last tiles, less than a round of them, as two half tiles each)
-    const long grid = ((max_mtiles * g.n_tiles_n + 2 * g.tail_cus + 31) / 32) * 32;   // whole rounds of 8 groups of 4 tiles
+    const long grid = ((max_mtiles * g.n_tiles_n + pair.shared_tiles + 2 * g.tail_cus + 31) / 32) * 32;   // whole rounds of 8 groups of 4 tiles
     if (grid > 0x7fffffffL) {
         set_error("grouped gemm: %ld workgroups exceed the grid limit", grid);
         return MOE_ERR_INVALID;
     }
-    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(128 * WN), 0, st, g);
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(128 * WN), 0, st, pair);
+    MOE_HIP_CHECK(hipGetLastError());
+    return MOE_OK;
+}
+
+template <bool SWIGLU, bool W8>
+int launch_thin(const GemmArgs& g, int n_rows, const GemmArgs* shared, hipStream_t st) {
+    constexpr int NCOL = SWIGLU ? 16 : 32;
+    GemmPair pair{};
+    pair.p[0] = g;
+    if (shared) {
+        pair.p[1] = *shared;
+        pair.shared_tiles = (shared->N + NCOL - 1) / NCOL;
+    }
+    const long grid = (long)(g.E < n_rows ? g.E : n_rows) * ((g.N + NCOL - 1) / NCOL) + pair.shared_tiles;
+    if (grid > 0x7fffffffL) {
+        set_error("grouped gemm: %ld workgroups exceed the grid limit", grid);
+        return MOE_ERR_INVALID;
+    }
+    hipLaunchKernelGGL((grouped_gemm_thin_kernel<SWIGLU, W8>), dim3((unsigned)grid), dim3(64), 0, st, pair);
     MOE_HIP_CHECK(hipGetLastError());
     return MOE_OK;
 }
@@ -1968,17 +2203,21 @@ int launch_persistent(const GemmArgs& g, int n_rows, hipStream_t st) {
     return MOE_OK;
 }
 
+// 4 GiB of gathered rows or more: only the register-staged body addresses them
+inline bool gather_fits(const GemmArgs& g) { return !g.row_map || g.a_bytes < (1ull << 32); }
+
+// max_rows: no expert has more rows (callers that do not know pass n_rows)
 template <bool SWIGLU, bool W8>
-int launch_mt(const GemmArgs& g0, int n_rows, hipStream_t st) {
+int launch_mt(const GemmArgs& g0, int n_rows, int max_rows, hipStream_t st) {
     GemmArgs g = g0;
     const long mean = g.E > 0 ? (long)n_rows / g.E : 0;
+    if (max_rows <= 16 && gather_fits(g)) return launch_thin<SWIGLU, W8>(g, n_rows, nullptr, st);
     // the persistent kernel needs an even number of k-stages for its hand-over (fp8 sizes always have
     // one), keeps per-expert tables for up to 512 experts and addresses gathered rows with 32-bit offsets
-    const bool fits = !g.row_map || g.a_bytes < (1ull << 32);
     // (below a mean of 128 rows an expert above one tile is rare and is cut into 128-row tiles where it occurs)
-    if (mean < 128 || !(g.K % 128 == 0 && g.E <= 512 && fits && cu_count() >= 8)) {
+    if (mean < 128 || !(g.K % 128 == 0 && g.E <= 512 && gather_fits(g) && cu_count() >= 8)) {
         g.cold_max = 0x7fffffff;
-        return launch_tiles<4, SWIGLU, W8>(g, n_rows, st);
+        return launch_tiles<4, SWIGLU, W8>(g, n_rows, nullptr, 0, st);
     }
     // The counts themselves live on the device; only their mean is known here.  Both kernels are launched and every
     // expert goes by its own count: what fits one tile of the one-workgroup-per-tile kernel runs there, at its own
@@ -2009,50 +2248,99 @@ int launch_mt(const GemmArgs& g0, int n_rows, hipStream_t st) {
     g.tail_cus = (cu_count() / 8) * 8;     // the persistent launch's grid when there is a round of tiles or more
     int rc = launch_persistent<SWIGLU, W8>(g, n_rows, st);
     if (rc != MOE_OK) return rc;
-    return launch_tiles<4, SWIGLU, W8>(g, n_rows, st);
+    return launch_tiles<4, SWIGLU, W8>(g, n_rows, nullptr, 0, st);
+}
+
+// The shared expert's tiles in the routed experts' launch.
+template <bool SWIGLU, bool W8>
+int launch_joint(const GemmArgs& routed, int n_rows, int max_rows, const GemmArgs& shared, int n_shared, hipStream_t st) {
+    if (max_rows <= 16 && n_shared <= 16) return launch_thin<SWIGLU, W8>(routed, n_rows, &shared, st);
+    GemmArgs r = routed, s = shared;
+    r.cold_max = s.cold_max = 0x7fffffff;
+    return launch_tiles<4, SWIGLU, W8>(r, n_rows, &s, n_shared, st);
+}
+
+int check_group(const moe_mlp_group& m, int32_t hidden, bool w8, const char* who) {
+    MOE_REQUIRE(m.n_rows >= 0, "%s: n_rows %d < 0", who, m.n_rows);
+    if (m.n_rows == 0) return MOE_OK;
+    MOE_REQUIRE(m.x && m.w_gate && m.w_up && m.w_down && m.offsets && m.act && m.y, "%s: NULL pointer argument", who);
+    MOE_REQUIRE(m.x_rows >= 1, "%s: x_rows %d < 1", who, m.x_rows);
+    MOE_REQUIRE(!w8 || (m.s_gate && m.s_up && m.s_down), "%s: NULL scale pointer array", who);
+    MOE_REQUIRE(m.n_experts >= 1 && m.n_experts <= MAX_E, "%s: n_experts %d outside [1,%d]", who, m.n_experts, MAX_E);
+    const int align = w8 ? 128 : 64;
+    MOE_REQUIRE(hidden > 0 && hidden % align == 0, "%s: hidden %d must be a positive multiple of %d", who, hidden, align);
+    MOE_REQUIRE(m.inter > 0 && m.inter % align == 0, "%s: intermediate %d must be a positive multiple of %d", who, m.inter,
+                align);
+    return MOE_OK;
+}
+
+GemmArgs gate_up_args(const moe_mlp_group& m, int32_t hidden) {
+    GemmArgs g{};
+    g.a = static_cast<const uint16_t*>(m.x);
+    g.row_map = m.row_map;
+    g.a_bytes = (size_t)m.x_rows * (size_t)hidden * 2;
+    g.a_rows = m.x_rows;
+    g.b0 = m.w_gate; g.b1 = m.w_up; g.s0 = m.s_gate; g.s1 = m.s_up;
+    g.offsets = m.offsets;
+    g.c = static_cast<uint16_t*>(m.act);
+    g.E = m.n_experts; g.K = hidden; g.N = m.inter;
+    g.n_tiles_n = (m.inter + 127) / 128;
+    return g;
+}
+
+GemmArgs down_args(const moe_mlp_group& m, int32_t hidden) {
+    GemmArgs g{};
+    g.a = static_cast<const uint16_t*>(m.act);
+    g.b0 = m.w_down; g.s0 = m.s_down;
+    g.offsets = m.offsets;
+    g.c = static_cast<uint16_t*>(m.y);
+    g.E = m.n_experts; g.K = m.inter; g.N = hidden;
+    g.n_tiles_n = (hidden + 255) / 256;
+    return g;
+}
+
+// no expert of the group has more rows than this
+int row_bound(const moe_mlp_group& m) { return m.max_rows > 0 && m.max_rows < m.n_rows ? m.max_rows : m.n_rows; }
+
+// Whether the shared expert's tiles join the routed experts' launch: it is small -- (n / 256 + 1) row tiles times I / 128
+// column tiles fewer than 3/8 of the device's CUs: alone it would leave most of them without a tile -- and the routed
+// call is one that the one-workgroup-per-tile kernel (or the thin one) serves alone.  DeepSeek-V3 up to 1024 tokens: the
+// step gains 2-5 %, from 2048 tokens on a launch pair of its own, with 256-row tiles, is the faster by 0.6 %.
+bool joins(const moe_mlp_group& routed, const moe_mlp_group& shared, int32_t hidden) {
+    if (routed.n_rows == 0 || shared.n_rows == 0 || shared.n_experts != 1) return false;
+    if (routed.n_rows / routed.n_experts >= 128) return false;
+    if (routed.row_map && (size_t)routed.x_rows * (size_t)hidden * 2 >= (1ull << 32)) return false;
+    return (long)(shared.n_rows / 256 + 1) * ((shared.inter + 127) / 128) * 8 < 3L * cu_count();
 }
 
 template <bool W8>
-int grouped_swiglu(const void* x, int32_t x_rows, const int32_t* row_map, const void* const* w_gate, const void* const* w_up,
-                   const void* const* w_down, const float* const* s_gate, const float* const* s_up,
-                   const float* const* s_down, const int32_t* offsets, int32_t n_rows, int32_t n_experts,
-                   int32_t hidden, int32_t inter, void* act, void* y, int32_t phases, void* stream, const char* who) {
-    MOE_REQUIRE(n_rows >= 0, "%s: n_rows %d < 0", who, n_rows);
+int grouped_swiglu(const moe_mlp_group& m, int32_t hidden, int32_t phases, void* stream, const char* who) {
     MOE_REQUIRE(phases >= MOE_PHASE_GATE_UP && phases <= MOE_PHASE_BOTH, "%s: bad phases %d", who, phases);
-    if (n_rows == 0) return MOE_OK;
-    MOE_REQUIRE(x && w_gate && w_up && w_down && offsets && act && y, "%s: NULL pointer argument", who);
-    MOE_REQUIRE(x_rows >= 1, "%s: x_rows %d < 1", who, x_rows);
-    MOE_REQUIRE(!W8 || (s_gate && s_up && s_down), "%s: NULL scale pointer array", who);
-    MOE_REQUIRE(n_experts >= 1 && n_experts <= MAX_E, "%s: n_experts %d outside [1,%d]", who, n_experts, MAX_E);
-    const int align = W8 ? 128 : 64;
-    MOE_REQUIRE(hidden > 0 && hidden % align == 0, "%s: hidden %d must be a positive multiple of %d", who, hidden, align);
-    MOE_REQUIRE(inter > 0 && inter % align == 0, "%s: intermediate %d must be a positive multiple of %d", who, inter,
-                align);
+    int rc = check_group(m, hidden, W8, who);
+    if (rc != MOE_OK || m.n_rows == 0) return rc;
     hipStream_t st = as_stream(stream);
-    GemmArgs g1{};
-    g1.a = static_cast<const uint16_t*>(x);
-    g1.row_map = row_map;
-    g1.a_bytes = (size_t)x_rows * (size_t)hidden * 2;
-    g1.a_rows = x_rows;
-    g1.b0 = w_gate; g1.b1 = w_up; g1.s0 = s_gate; g1.s1 = s_up;
-    g1.offsets = offsets;
-    g1.c = static_cast<uint16_t*>(act);
-    g1.E = n_experts; g1.K = hidden; g1.N = inter;
-    g1.n_tiles_n = (inter + 127) / 128;
-    if (phases & MOE_PHASE_GATE_UP) {
-        int rc = launch_mt<true, W8>(g1, n_rows, st);
-        if (rc != MOE_OK) return rc;
+    if (phases & MOE_PHASE_GATE_UP) rc = launch_mt<true, W8>(gate_up_args(m, hidden), m.n_rows, row_bound(m), st);
+    if (rc == MOE_OK && (phases & MOE_PHASE_DOWN)) rc = launch_mt<false, W8>(down_args(m, hidden), m.n_rows, row_bound(m), st);
+    return rc;
+}
+
+template <bool W8>
+int grouped_swiglu_joint(const moe_mlp_group& r, const moe_mlp_group& s, int32_t hidden, int32_t phases, void* stream) {
+    const char* who = "moe_grouped_swiglu_joint";
+    if (!joins(r, s, hidden)) {
+        const int rc = grouped_swiglu<W8>(r, hidden, phases, stream, who);
+        return rc != MOE_OK ? rc : grouped_swiglu<W8>(s, hidden, phases, stream, who);
     }
-    if (!(phases & MOE_PHASE_DOWN)) return MOE_OK;
-    GemmArgs g2{};
-    g2.a = static_cast<const uint16_t*>(act);
-    g2.row_map = nullptr;
-    g2.b0 = w_down; g2.b1 = nullptr; g2.s0 = s_down; g2.s1 = nullptr;
-    g2.offsets = offsets;
-    g2.c = static_cast<uint16_t*>(y);
-    g2.E = n_experts; g2.K = inter; g2.N = hidden;
-    g2.n_tiles_n = (hidden + 255) / 256;
-    return launch_mt<false, W8>(g2, n_rows, st);
+    MOE_REQUIRE(phases >= MOE_PHASE_GATE_UP && phases <= MOE_PHASE_BOTH, "%s: bad phases %d", who, phases);
+    int rc = check_group(r, hidden, W8, who);
+    if (rc == MOE_OK) rc = check_group(s, hidden, W8, who);
+    if (rc != MOE_OK) return rc;
+    hipStream_t st = as_stream(stream);
+    if (phases & MOE_PHASE_GATE_UP)
+        rc = launch_joint<true, W8>(gate_up_args(r, hidden), r.n_rows, row_bound(r), gate_up_args(s, hidden), s.n_rows, st);
+    if (rc == MOE_OK && (phases & MOE_PHASE_DOWN))
+        rc = launch_joint<false, W8>(down_args(r, hidden), r.n_rows, row_bound(r), down_args(s, hidden), s.n_rows, st);
+    return rc;
 }
 
 // out = bf16(f32(q) * scale[i/128, j/128]); one thread per 16 consecutive elements of a row
@@ -2087,8 +2375,8 @@ extern "C" int moe_grouped_swiglu_bf16(const void* x, int32_t x_rows, const int3
                                        const void* const* w_up, const void* const* w_down, const int32_t* offsets,
                                        int32_t n_rows, int32_t n_experts, int32_t hidden, int32_t inter, void* act,
                                        void* y, int32_t phases, void*, size_t, void* stream) {
-    return moe::grouped_swiglu<false>(x, x_rows, row_map, w_gate, w_up, w_down, nullptr, nullptr, nullptr, offsets, n_rows,
-                                      n_experts, hidden, inter, act, y, phases, stream, "moe_grouped_swiglu_bf16");
+    const moe_mlp_group m{x, x_rows, n_rows, row_map, w_gate, w_up, w_down, nullptr, nullptr, nullptr, offsets, n_experts, inter, 0, 0, act, y};
+    return moe::grouped_swiglu<false>(m, hidden, phases, stream, "moe_grouped_swiglu_bf16");
 }
 
 extern "C" int moe_grouped_swiglu_w8a16(const void* x, int32_t x_rows, const int32_t* row_map, const void* const* w_gate,
@@ -2097,8 +2385,23 @@ extern "C" int moe_grouped_swiglu_w8a16(const void* x, int32_t x_rows, const int
                                         const float* const* s_down, const int32_t* offsets, int32_t n_rows,
                                         int32_t n_experts, int32_t hidden, int32_t inter, void* act, void* y,
                                         int32_t phases, void*, size_t, void* stream) {
-    return moe::grouped_swiglu<true>(x, x_rows, row_map, w_gate, w_up, w_down, s_gate, s_up, s_down, offsets, n_rows,
-                                     n_experts, hidden, inter, act, y, phases, stream, "moe_grouped_swiglu_w8a16");
+    const moe_mlp_group m{x, x_rows, n_rows, row_map, w_gate, w_up, w_down, s_gate, s_up, s_down, offsets, n_experts, inter, 0, 0, act, y};
+    return moe::grouped_swiglu<true>(m, hidden, phases, stream, "moe_grouped_swiglu_w8a16");
+}
+
+extern "C" int moe_grouped_swiglu_joint(const moe_mlp_group* routed, const moe_mlp_group* shared, int32_t hidden, int32_t fp8,
+                                        int32_t phases, void* stream) {
+    using namespace moe;
+    MOE_REQUIRE(routed != nullptr, "moe_grouped_swiglu_joint: NULL group");
+    if (shared == nullptr)
+        return fp8 ? grouped_swiglu<true>(*routed, hidden, phases, stream, "moe_grouped_swiglu_joint")
+                   : grouped_swiglu<false>(*routed, hidden, phases, stream, "moe_grouped_swiglu_joint");
+    return fp8 ? grouped_swiglu_joint<true>(*routed, *shared, hidden, phases, stream)
+               : grouped_swiglu_joint<false>(*routed, *shared, hidden, phases, stream);
+}
+
+extern "C" int moe_shared_joins(const moe_mlp_group* routed, const moe_mlp_group* shared, int32_t hidden) {
+    return routed && shared && moe::joins(*routed, *shared, hidden) ? 1 : 0;
 }
 
 extern "C" int moe_dequant_fp8_block128(const void* q, const float* scale, int32_t rows, int32_t cols, void* out,

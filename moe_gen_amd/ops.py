@@ -304,6 +304,39 @@ def grouped_swiglu(x: torch.Tensor, row_map, ptrs: ExpertPointers, offsets: torc
     return y
 
 
+def mlp_group(x: torch.Tensor, row_map, ptrs: ExpertPointers, offsets: torch.Tensor, n_rows: int, max_rows: int = 0,
+              act: torch.Tensor | None = None, y: torch.Tensor | None = None):
+    """One expert MLP problem for grouped_swiglu_joint: (struct, act, y).  Arguments as grouped_swiglu; max_rows: no expert
+    has more rows than this (0: not known)."""
+    h, I, E = ptrs.hidden, ptrs.inter, ptrs.n_experts
+    _need(x, torch.bfloat16, "x")
+    if x.shape[1] != h:
+        raise ValueError(f"x has hidden size {x.shape[1]}, experts expect {h}")
+    if row_map is None and x.shape[0] < n_rows:
+        raise ValueError(f"x has {x.shape[0]} rows, need {n_rows}")
+    if row_map is not None:
+        _need(row_map, torch.int32, "row_map", (n_rows,))
+    _need(offsets, torch.int32, "offsets", (E + 1,))
+    act = torch.empty((n_rows, I), dtype=torch.bfloat16, device=x.device) if act is None else act
+    y = torch.empty((n_rows, h), dtype=torch.bfloat16, device=x.device) if y is None else y
+    _need(act, torch.bfloat16, "act", (n_rows, I))
+    _need(y, torch.bfloat16, "y", (n_rows, h))
+    m = N.MlpGroup(_ptr(x), x.shape[0], n_rows, _ptr(row_map), _ptr(ptrs.w_gate), _ptr(ptrs.w_up), _ptr(ptrs.w_down),
+                   _ptr(ptrs.s_gate), _ptr(ptrs.s_up), _ptr(ptrs.s_down), _ptr(offsets), E, I, max_rows, 0, _ptr(act), _ptr(y))
+    return m, act, y
+
+
+def shared_joins(routed, shared, hidden: int) -> bool:
+    """Whether grouped_swiglu_joint runs the shared expert inside the routed experts' launches."""
+    return bool(N.lib().moe_shared_joins(ctypes.byref(routed), ctypes.byref(shared), hidden))
+
+
+def grouped_swiglu_joint(routed, shared, hidden: int, fp8: bool, phases: int = PHASE_BOTH) -> None:
+    """The expert MLPs of `routed` and of `shared` (structs of mlp_group, of the same weight type; shared may be None)."""
+    N.check(N.lib().moe_grouped_swiglu_joint(ctypes.byref(routed), None if shared is None else ctypes.byref(shared), hidden,
+                                             int(fp8), phases, _stream()), "moe_grouped_swiglu_joint")
+
+
 def dequant_fp8_block128(q: torch.Tensor, scale: torch.Tensor) -> torch.Tensor:
     """bf16(f32(q) * scale[i//128, j//128]) -- deepseek_v3_dequantization (Wrapper.py:109-138)."""
     _need(q, torch.float8_e4m3fn, "q")

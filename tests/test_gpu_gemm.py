@@ -747,3 +747,89 @@ def test_swiglu_epilogue_alone(fp8):
     assert diff.max() <= 2, f"epilogue off by {diff.max()} bf16 steps"
     assert (diff > 0).mean() < 0.01, f"{(diff > 0).mean():.2%} of the elements differ"
     assert (diff > 1).mean() < 0.001, f"{(diff > 1).mean():.3%} of the elements differ by two steps"
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("h,I", [(128, 128), (640, 384), (1024, 896), (256, 8320)])    # 1 ... 130 stages; more than 64 fp8 scales per row
+def test_thin_kernel_matches_larger_calls(fp8, h, I):
+    """Calls whose experts have at most 16 rows run on one wave per 32 weight rows.  Experts of 0 ... 16 rows, empty ones
+    in front, between and behind, more experts than a wave scans at once; rows gathered through a row map with an entry
+    outside x (zeros).  Against the oracle, and bit for bit against the same rows in a call with an expert of 40 rows
+    (the tile kernel: fp8 in its form for up to 64 rows)."""
+    from moe_gen_amd import ops
+    E = 263
+    counts = [0] * E
+    for e, c in ((1, 1), (2, 16), (4, 15), (63, 2), (64, 7), (255, 3), (256, 16), (261, 1)):
+        counts[e] = c
+    print(f"thin fp8={fp8} h={h} I={I}", flush=True)
+    offsets = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    n = int(offsets[-1])
+    g = torch.Generator().manual_seed(401)
+    x = torch.randn(n + 40, h, generator=g).to(torch.bfloat16)
+    mats = make_experts(2, h, I, fp8, 402)                       # experts alternate between two sets of weights
+    dev = lambda m: tuple(t.cuda() for t in m) if isinstance(m, tuple) else m.cuda()
+    dm = [[dev(m) for m in one] for one in mats]
+    pick = lambda i, j: [dm[e % 2][i][j] if fp8 else dm[e % 2][i] for e in range(E)]
+    ptrs = ops.expert_pointers(*(pick(i, 0) for i in range(3)), *((pick(i, 1) for i in range(3)) if fp8 else ()))
+    rm = torch.randperm(n, generator=g).to(torch.int32)
+    xd = x.cuda()
+    m, _, y = ops.mlp_group(xd, rm.cuda(), ptrs, torch.from_numpy(offsets).cuda(), n, 16)
+    ops.grouped_swiglu_joint(m, None, h, fp8)
+    bad = rm.clone()
+    bad[[0, 20]] = torch.tensor([n + 40, -3], dtype=torch.int32)
+    mb, _, yb = ops.mlp_group(xd, bad.cuda(), ptrs, torch.from_numpy(offsets).cuda(), n, 16)
+    ops.grouped_swiglu_joint(mb, None, h, fp8)
+    big = list(counts)
+    big[262] = 40                                                # behind all others: their rows keep their places
+    off_big = np.concatenate([[0], np.cumsum(big)]).astype(np.int32)
+    rm_big = torch.cat([rm, torch.arange(n, n + 40, dtype=torch.int32)])
+    y_big = ops.grouped_swiglu(xd, rm_big.cuda(), ptrs, torch.from_numpy(off_big).cuda(), n + 40)
+    torch.cuda.synchronize()
+    assert torch.equal(y, y_big[:n])
+    keep = torch.ones(n, dtype=torch.bool)
+    keep[[0, 20]] = False
+    assert torch.equal(yb.cpu()[keep], y.cpu()[keep]) and (yb.cpu()[~keep].float() == 0).all()
+    xf = O.bf16_to_f32(bits(x[rm.long()]))
+    ref = np.zeros((n, h), np.float32)
+    for e in range(E):
+        a, b = offsets[e], offsets[e + 1]
+        if b > a:
+            ref[a:b] = O.mlp_f32(xf[a:b], *(f32_of(w) for w in mats[e % 2]))
+    assert rel_max(O.bf16_to_f32(bits(y)), ref) <= TOL
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("n,shared_inter", [(1, 256), (16, 768), (17, 256), (100, 768), (192, 256), (193, 512), (300, 256)])
+def test_shared_expert_in_the_routed_launches(fp8, n, shared_inter):
+    """A shared expert of another intermediate size next to the routed experts: few rows (thin kernel), one tile, two
+    halves of 257 ... 384 rows and 128-row slices (tile kernel).  Bit for bit what the two calls give apart; with fp8
+    weights too as long as both calls are ones that the tile kernel serves alone (mean rows per expert below 128)."""
+    from moe_gen_amd import ops
+    E, k, h, I = 12, 2, 384, 256
+    print(f"joint fp8={fp8} n={n} shared_inter={shared_inter}", flush=True)
+    g = torch.Generator().manual_seed(n)
+    dev = lambda m: tuple(t.cuda() for t in m) if isinstance(m, tuple) else m.cuda()
+    tables = []
+    for count, inter, seed in ((E, I, 11), (1, shared_inter, 12)):
+        dm = [[dev(m) for m in one] for one in make_experts(count, h, inter, fp8, seed)]
+        col = lambda i, j: [o[i][j] if fp8 else o[i] for o in dm]
+        tables.append(ops.expert_pointers(*(col(i, 0) for i in range(3)), *((col(i, 1) for i in range(3)) if fp8 else ())))
+    idx = torch.rand((n, E), generator=g).topk(k, dim=1).indices.to(torch.int32)
+    x = torch.randn(n, h, generator=g).to(torch.bfloat16).cuda()
+    d = ops.dispatch(idx.cuda(), E, None, want_row_map=True)
+    so = torch.tensor([0, n], dtype=torch.int32, device="cuda")
+    r1, _, y1 = ops.mlp_group(x, d.row_map, tables[0], d.offsets, n * k, n)
+    s1, _, sh1 = ops.mlp_group(x, None, tables[1], so, n)
+    assert ops.shared_joins(r1, s1, h)
+    ops.grouped_swiglu_joint(r1, s1, h, fp8)
+    r2, _, y2 = ops.mlp_group(x, d.row_map, tables[0], d.offsets, n * k, n)
+    s2, _, sh2 = ops.mlp_group(x, None, tables[1], so, n)
+    ops.grouped_swiglu_joint(r2, None, h, fp8)
+    ops.grouped_swiglu_joint(s2, None, h, fp8)
+    torch.cuda.synchronize()
+    assert torch.equal(y1, y2)
+    if not fp8 or n < 128:
+        assert torch.equal(sh1, sh2)
+    else:
+        a, b = sh1.float(), sh2.float()
+        assert (a - b).abs().max().item() <= TOL * b.abs().max().item()
