@@ -221,7 +221,8 @@ typedef struct moe_mlp_group {
     const float* const* s_up;
     const float* const* s_down;
     const int32_t* offsets;
-    int32_t n_experts, inter, max_rows, reserved;
+    int32_t n_experts, inter, max_rows;
+    int32_t fp8;                 /* weight type, read by moe_layer_forward (elsewhere the call says it) */
     void* act;
     void* y;
 } moe_mlp_group;
@@ -236,6 +237,42 @@ typedef struct moe_mlp_group {
 int moe_grouped_swiglu_joint(const moe_mlp_group* routed, const moe_mlp_group* shared, int32_t hidden, int32_t fp8,
                              int32_t phases, void* stream);
 int moe_shared_joins(const moe_mlp_group* routed, const moe_mlp_group* shared, int32_t hidden);
+
+/*
+ * A whole layer call with resident weights: [rmsnorm,] router, dispatch, expert MLPs, combine [, residual add], the
+ * launches of the separate entry points with their buffers carved out of one workspace
+ * (DeepseekV3MoE.forward, modeling_deepseek_v3.py:614-626; with norm_weight the MLP half of the decoder layer, :1361-1365).
+ *   x            device bf16 [n, h] hidden states
+ *   norm_weight  device bf16 [h] or NULL: the experts and the router read x through the RMSNorm, and x is added to the result
+ *   w_gate, bias, router   as moe_router (router->n_tokens, ->hidden are the call's sizes)
+ *   routed       weights, scales, n_experts, inter and fp8 of the routed experts; the other fields are not read
+ *   shared       the same of the shared expert (n_experts 1), NULL: none
+ *   topk_idx [n,k], topk_w [n,k], counts [E]   out
+ *   logits_bf16  device bf16 [n, E] out (Mixtral's second result), may be NULL
+ *   out          device bf16 [n, h]; must not alias x (with norm_weight it may)
+ *   workspace    moe_layer_workspace_bytes() bytes
+ */
+typedef struct moe_layer_args {
+    const void* x;
+    const void* norm_weight;
+    const void* w_gate;
+    const float* bias;
+    const moe_router_params* router;
+    const moe_mlp_group* routed;
+    const moe_mlp_group* shared;
+    int32_t* topk_idx;
+    float* topk_w;
+    int32_t* counts;
+    void* logits_bf16;
+    void* out;
+    void* workspace;
+    size_t workspace_bytes;
+    float norm_eps;
+    int32_t combine_mode;        /* as moe_combine */
+    int32_t join_shared;         /* 0: never run the shared expert inside the routed experts' launches */
+} moe_layer_args;
+size_t moe_layer_workspace_bytes(const moe_layer_args* args);
+int moe_layer_forward(const moe_layer_args* args, void* stream);
 
 /*
  * Write n 64-bit words (device pointers of a wave of experts, say) into device memory at dst, from host memory

@@ -31,8 +31,19 @@ class MlpGroup(ctypes.Structure):
         ("x", c_void_p), ("x_rows", c_int32), ("n_rows", c_int32), ("row_map", c_void_p),
         ("w_gate", c_void_p), ("w_up", c_void_p), ("w_down", c_void_p),
         ("s_gate", c_void_p), ("s_up", c_void_p), ("s_down", c_void_p), ("offsets", c_void_p),
-        ("n_experts", c_int32), ("inter", c_int32), ("max_rows", c_int32), ("reserved", c_int32),
+        ("n_experts", c_int32), ("inter", c_int32), ("max_rows", c_int32), ("fp8", c_int32),
         ("act", c_void_p), ("y", c_void_p),
+    ]
+
+
+class LayerArgs(ctypes.Structure):
+    """struct moe_layer_args."""
+    _fields_ = [
+        ("x", c_void_p), ("norm_weight", c_void_p), ("w_gate", c_void_p), ("bias", c_void_p),
+        ("router", c_void_p), ("routed", c_void_p), ("shared", c_void_p),      # addresses of a RouterParams and two MlpGroup
+        ("topk_idx", c_void_p), ("topk_w", c_void_p), ("counts", c_void_p), ("logits_bf16", c_void_p), ("out", c_void_p),
+        ("workspace", c_void_p), ("workspace_bytes", c_size_t), ("norm_eps", c_float), ("combine_mode", c_int32),
+        ("join_shared", c_int32),
     ]
 
 
@@ -59,6 +70,8 @@ SIGNATURES = {
     "moe_grouped_swiglu_joint": (ctypes.c_int, [ctypes.POINTER(MlpGroup), ctypes.POINTER(MlpGroup), c_int32, c_int32, c_int32,
                                                 c_void_p]),
     "moe_shared_joins": (ctypes.c_int, [ctypes.POINTER(MlpGroup), ctypes.POINTER(MlpGroup), c_int32]),
+    "moe_layer_workspace_bytes": (c_size_t, [ctypes.POINTER(LayerArgs)]),
+    "moe_layer_forward": (ctypes.c_int, [ctypes.POINTER(LayerArgs), c_void_p]),
     "moe_dequant_fp8_block128": (ctypes.c_int, [c_void_p, c_void_p, c_int32, c_int32, c_void_p, c_void_p]),
     "moe_combine": (ctypes.c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_int32,
                                    c_int32, c_int32, c_void_p, c_void_p]),

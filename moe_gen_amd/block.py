@@ -116,14 +116,17 @@ class SwiGLUMLP(nn.Module):
         n = x2d.shape[0]
         if engine_backed(self):
             raise RuntimeError("SwiGLUMLP.forward: engine-backed weights are handled by the MoE block")
-        ptrs = collect_pointers([self], None)
-        offsets = torch.tensor([0, n], dtype=torch.int32, device=x.device)
-        return ops.grouped_swiglu(x2d, None, ptrs, offsets, n).view(*shape)
+        ptrs = collect_pointers([self], self.__dict__.setdefault("_moe_cache", {}))
+        # (the row range travels in kernel arguments: a copy from the host would stop the stream)
+        offsets = ops._upload_words([n << 32], x.device).view(torch.int32)
+        return _grouped(None, "mlp", x2d, None, ptrs, offsets, n, n).view(*shape)
 
 
 def _unwrap(expert):
     """MoE-Gen replaces experts by Expert_Wrapper objects that keep the MLP in `.module`
     (Wrapper.py:449); accept both."""
+    if isinstance(expert, SwiGLUMLP) and "module" not in expert.__dict__:
+        return expert
     return getattr(expert, "module", expert)
 
 
@@ -147,18 +150,33 @@ def _tensors_of(expert, fetched=None):
         if wrap_scales:
             return (w0, fetched[wk[1]], fetched[wk[2]], wrap_scales.get(sk[0]), wrap_scales.get(sk[1]), wrap_scales.get(sk[2]))
     mlp = _unwrap(expert)
-    wrap_scales = getattr(expert, "weight_dequant_scale", None) or {}
+    wrap_scales = {} if mlp is expert else getattr(expert, "weight_dequant_scale", None) or {}
     ws, ss = [], []
     for name in mlp.names:
-        lin = getattr(mlp, name)
-        w = fetched[name + ".weight"] if fetched is not None else lin.weight.data
+        lin = _linear(mlp, name)
+        w = fetched[name + ".weight"] if fetched is not None else _param(lin, "weight")
         s = wrap_scales.get(name + ".weight_scale_inv")
         if s is None:
-            s = getattr(lin, "weight_scale_inv", None)
-            s = None if s is None else s.data
+            s = _param(lin, "weight_scale_inv")
         ws.append(w)
         ss.append(s)
     return (*ws, *ss)
+
+
+def _linear(mlp, name):
+    """mlp.<name> without nn.Module's attribute protocol where the Linear is an ordinary submodule."""
+    mods = mlp.__dict__.get("_modules")
+    lin = mods.get(name) if mods else None
+    return getattr(mlp, name) if lin is None else lin
+
+
+def _param(lin, name):
+    """The parameter's tensor (None if there is none), also without the protocol."""
+    params = lin.__dict__.get("_parameters")
+    p = params.get(name) if params else None
+    if p is None:
+        p = getattr(lin, name, None) if name == "weight" or name in lin.__dict__ or hasattr(type(lin), name) else None
+    return None if p is None else p.data
 
 
 def _pointer_table(rows):
@@ -192,9 +210,9 @@ def any_engine_backed(experts) -> bool:
 def collect_pointers(experts, cache):
     """Pointer tables for a list of RESIDENT expert modules, cached in `cache` (a dict) keyed on
     the storage addresses of the first and last expert."""
-    f = _tensors_of(experts[0])
-    last = _tensors_of(experts[-1])
-    stamp = (len(experts), f[0].data_ptr(), f[0].dtype, tuple(f[0].shape), last[2].data_ptr())
+    first, last = _unwrap(experts[0]), _unwrap(experts[-1])
+    f = _param(_linear(first, first.names[0]), "weight")
+    stamp = (len(experts), f.data_ptr(), f.dtype, f.shape, _param(_linear(last, last.names[2]), "weight").data_ptr())
     if cache is not None and cache.get("stamp") == stamp:
         return cache["ptrs"]
     p = _pointer_table([_tensors_of(ex) for ex in experts])
@@ -385,10 +403,18 @@ def _engine_experts(block, timer, tag, experts, a_rows, row_map, offsets, n_rows
     return y
 
 
+def _option(block, name, default):
+    """block.<name> or the default: an attribute of the block or of its class (nn.Module answers for a missing attribute by
+    way of an exception)."""
+    d = block.__dict__
+    return d[name] if name in d else getattr(type(block), name, default)
+
+
 @torch.no_grad()
 def moe_forward(block, hidden_states: torch.Tensor, spec: ops.RouterSpec, gate_weight: torch.Tensor,
                 bias, experts, shared, combine_mode: int, want_logits: bool = False):
-    """The whole layer for one call.  Returns (out [same shape as hidden_states], logits | None)."""
+    """The whole layer for one call.  Returns (out [same shape as hidden_states], logits | None).  With resident weights that
+    is one call into the library; attached timers, staged weights and the materialised gather take it stage by stage."""
     if not hidden_states.is_cuda:
         raise RuntimeError("MoE block called on a CPU tensor: this implementation runs on the GPU only")
     if hidden_states.dtype != torch.bfloat16:
@@ -399,12 +425,22 @@ def moe_forward(block, hidden_states: torch.Tensor, spec: ops.RouterSpec, gate_w
         x = x.contiguous()
     n, h = x.shape
     k, E = spec.top_k, spec.n_experts
-    residual = None
-    fuse = getattr(block, "_norm_residual", None)
-    timer = getattr(block, "stage_timer", None)
+    fuse, timer = _option(block, "_norm_residual", None), _option(block, "stage_timer", None)
+    fused_gather, join = _option(block, "fused_gather", True), _option(block, "join_shared", True)
     cache = block.__dict__.setdefault("_moe_cache", {})
     gw = _gate_weight_bf16(gate_weight, cache)
     b = None if bias is None else bias.data.to(torch.float32)
+    experts = list(experts)
+    staged = any_engine_backed(experts)            # decided expert by expert, as the reference's initializers do
+    if timer is None and fused_gather and not staged and (shared is None or not engine_backed(shared)):
+        ptrs = collect_pointers(experts, cache.setdefault("routed", {}))
+        sp = None if shared is None else collect_pointers([shared], cache.setdefault("shared", {}))
+        out, idx, w, counts, logits = ops.layer_forward(x, *(fuse or (None, 0.0)), gw, b, spec, ptrs, sp, combine_mode, bool(join),
+                                                        want_logits)
+        d = block.__dict__
+        d["last_topk_idx"], d["last_topk_weight"], d["last_counts"] = idx, w, counts
+        return out.view(shape), logits
+    residual = None
     if fuse is not None:                      # see norm_moe_residual: the router reads x through the norm
         residual = x
         with _span(timer, "router"):
@@ -413,9 +449,6 @@ def moe_forward(block, hidden_states: torch.Tensor, spec: ops.RouterSpec, gate_w
         with _span(timer, "router"):
             idx, w, logits = ops.router(x, gw, b, spec, want_logits)
     block.last_topk_idx, block.last_topk_weight = idx, w
-    fused_gather = getattr(block, "fused_gather", True)
-    experts = list(experts)
-    staged = any_engine_backed(experts)            # decided expert by expert, as the reference's initializers do
     with _span(timer, "dispatch"):
         d = ops.dispatch(idx, E, None if fused_gather else x, want_row_map=fused_gather)
     counts, offsets, pos, row_map = d.counts, d.offsets, d.pos, d.row_map
@@ -432,7 +465,7 @@ def moe_forward(block, hidden_states: torch.Tensor, spec: ops.RouterSpec, gate_w
         y = _engine_experts(block, timer, "routed", experts, a_rows, row_map, offsets, n * k, counts)
     else:
         ptrs = collect_pointers(experts, cache.setdefault("routed", {}))
-        if shared is not None and not shared_staged and n and getattr(block, "join_shared", True):
+        if shared is not None and not shared_staged and n and join:
             # the shared expert's tiles in the routed experts' launches where that pays (a small batch: alone it has a
             # tile for a fraction of the CUs); `block.join_shared = False` keeps the two apart
             sp = collect_pointers([shared], cache.setdefault("shared", {}))

@@ -21,6 +21,7 @@
 #include <mutex>
 
 #include "common.h"
+#include "dispatch_small.h"
 
 namespace moe {
 namespace {
@@ -28,7 +29,7 @@ namespace {
 constexpr int SEG_PER_WAVE = 512;   // flat entries ranked by one wave
 constexpr int SEG_WAVES = 4;
 constexpr int SEG = SEG_PER_WAVE * SEG_WAVES;  // entries per block
-constexpr int MAX_E = 256;
+constexpr int MAX_E = kDispatchMaxE;
 
 __global__ void zero_i32(int32_t* a, int na, int32_t* b, int nb) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -79,7 +80,8 @@ __global__ __launch_bounds__(256) void rank_scatter(const int32_t* __restrict__ 
                                                     const int32_t* __restrict__ seg_base,
                                                     const int32_t* __restrict__ counts,
                                                     int32_t* __restrict__ offsets, int32_t* __restrict__ perm,
-                                                    int32_t* __restrict__ pos, int32_t* __restrict__ row_map, int k) {
+                                                    int32_t* __restrict__ pos, int32_t* __restrict__ row_map, int k,
+                                                    int32_t* __restrict__ one_group) {
     __shared__ int off[MAX_E];                 // exclusive prefix sum of counts
     __shared__ int whist[SEG_WAVES][MAX_E];    // per-wave counts, then per-wave running cursors
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -102,6 +104,7 @@ __global__ __launch_bounds__(256) void rank_scatter(const int32_t* __restrict__ 
     if (blockIdx.x == 0) {
         if (tid < E) offsets[tid] = wpre + inc - cv;
         if (tid == E - 1) offsets[E] = wpre + inc;
+        if (one_group && tid < 2) one_group[tid] = tid ? (int32_t)(nk / k) : 0;
     }
 
     // pass 1: counts of this wave's 512-entry slice
@@ -155,92 +158,11 @@ __global__ __launch_bounds__(256) void rank_scatter(const int32_t* __restrict__ 
     }
 }
 
-// The three kernels above as one workgroup of 16 waves, for index lists of up to SMALL_MAX entries (a decode or small
-// prefill batch: three dependent launches of a few microseconds each cost more than their work).  Wave w owns the
-// w-th slice of the list (a multiple of 64 entries): counts it, the first 256 threads turn the 16 x E counts into
-// counts[], offsets[] and one cursor per (wave, expert) -- offsets[e] + entries of e in earlier slices -- and every
-// wave ranks its slice as rank_scatter does.  The sorted position of an entry is the same pure function of the list.
-constexpr int SMALL_WAVES = 16;
 constexpr int SMALL_MAX = 12288;   // one launch of 18.6 us against three of 21.7 (16384 entries: 23.7)
 
-__global__ __launch_bounds__(64 * SMALL_WAVES) void dispatch_small(const int32_t* __restrict__ idx, int nk, int E,
-                                                                   int32_t* __restrict__ counts,
-                                                                   int32_t* __restrict__ offsets,
-                                                                   int32_t* __restrict__ perm, int32_t* __restrict__ pos,
-                                                                   int32_t* __restrict__ row_map, int k) {
-    constexpr int IT = SMALL_MAX / (SMALL_WAVES * 64);   // 64-entry steps of a wave's slice, at most
-    __shared__ int whist[SMALL_WAVES][MAX_E];
-    __shared__ int wtot[4];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int slice = (nk + SMALL_WAVES * 64 - 1) / (SMALL_WAVES * 64) * 64;
-    const int wbase = wave * slice;
-    // the lane's entries of the slice, all requested at once (both passes use them: a load per step would put the
-    // memory latency into every step); -1 marks an entry past the list or an id outside [0, E)
-    int ev[IT];
-#pragma unroll
-    for (int it = 0; it < IT; ++it) ev[it] = idx[min(wbase + 64 * it + lane, nk - 1)];
-    for (int e = tid; e < SMALL_WAVES * MAX_E; e += 64 * SMALL_WAVES) (&whist[0][0])[e] = 0;
-    __syncthreads();
-#pragma unroll
-    for (int it = 0; it < IT; ++it) {
-        const int g = wbase + 64 * it + lane;
-        if (64 * it >= slice || g >= nk || (unsigned)ev[it] >= (unsigned)E) ev[it] = -1;
-        if (ev[it] >= 0) atomicAdd(&whist[wave][ev[it]], 1);
-    }
-    __syncthreads();
-    int cv = 0, inc = 0;
-    if (tid < MAX_E) {                         // waves 0 .. 3, whole waves
-        if (tid < E) {
-#pragma unroll
-            for (int w = 0; w < SMALL_WAVES; ++w) cv += whist[w][tid];
-        }
-        inc = cv;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const int o = __shfl_up(inc, d);
-            if (lane >= d) inc += o;
-        }
-        if (lane == 63) wtot[wave] = inc;
-    }
-    __syncthreads();
-    if (tid < E) {
-        int run = inc - cv;
-        for (int w = 0; w < wave; ++w) run += wtot[w];
-        counts[tid] = cv;
-        offsets[tid] = run;
-        if (tid == E - 1) offsets[E] = run + cv;
-#pragma unroll
-        for (int w = 0; w < SMALL_WAVES; ++w) {
-            const int c = whist[w][tid];
-            whist[w][tid] = run;
-            run += c;
-        }
-    }
-    __syncthreads();
-    int* cur = whist[wave];
-#pragma unroll
-    for (int it = 0; it < IT; ++it) {
-        if (64 * it >= slice) break;
-        const int g = wbase + 64 * it + lane;
-        const int e = ev[it];
-        const bool ok = e >= 0;
-        if (g < nk && !ok) pos[g] = -1;        // as in rank_scatter: no sorted row, the combine skips the slot
-        uint64_t peers = __ballot(ok);
-#pragma unroll
-        for (int b = 0; b < 8; ++b) {
-            const bool bit = (e >> b) & 1;
-            const uint64_t bal = __ballot(bit);
-            peers &= bit ? bal : ~bal;
-        }
-        const uint64_t below = peers & ((1ull << lane) - 1ull);
-        if (ok) {
-            const int r = cur[e] + __popcll(below);
-            perm[r] = g;
-            pos[g] = r;
-            if (row_map) row_map[r] = g / k;
-        }
-        if (ok && below == 0) cur[e] += __popcll(peers);
-    }
+__global__ __launch_bounds__(64 * SMALL_WAVES) void dispatch_small(const int32_t* __restrict__ idx, int nk, int E, DispatchOut out,
+                                                                   int k) {
+    dispatch_one_workgroup<SMALL_MAX / (SMALL_WAVES * 64)>(nk, E, out, k, [&](int i) { return idx[i]; });
 }
 
 __global__ __launch_bounds__(256) void gather_rows(const u32x4* __restrict__ x, const int32_t* __restrict__ perm,
@@ -268,22 +190,20 @@ namespace moe {
 namespace {
 
 // The launches behind both entry points; `seg` holds nseg * n_experts per-segment counts.
-int dispatch_launch(const int32_t* topk_idx, int64_t nk, int32_t top_k, int32_t n_experts, int32_t* counts,
-                    int32_t* offsets, int32_t* perm, int32_t* pos, int32_t* row_map, const void* x, int32_t hidden,
-                    void* xs, int32_t* seg, hipStream_t st) {
+int dispatch_launch(const int32_t* topk_idx, int64_t nk, int32_t top_k, int32_t n_experts, const DispatchOut& out, const void* x,
+                    int32_t hidden, void* xs, int32_t* seg, hipStream_t st) {
     if (nk <= SMALL_MAX) {
-        hipLaunchKernelGGL(dispatch_small, dim3(1), dim3(64 * SMALL_WAVES), 0, st, topk_idx, (int)nk, n_experts, counts,
-                           offsets, perm, pos, row_map, top_k);
+        hipLaunchKernelGGL(dispatch_small, dim3(1), dim3(64 * SMALL_WAVES), 0, st, topk_idx, (int)nk, n_experts, out, top_k);
     } else {
         const int nseg = (int)((nk + SEG - 1) / SEG);
         hipLaunchKernelGGL(block_histogram, dim3(nseg), dim3(256), 0, st, topk_idx, nk, n_experts, seg);
-        hipLaunchKernelGGL(scan_segments, dim3((n_experts + 3) / 4), dim3(256), 0, st, seg, nseg, n_experts, counts);
-        hipLaunchKernelGGL(rank_scatter, dim3(nseg), dim3(256), 0, st, topk_idx, nk, n_experts, seg, counts, offsets,
-                           perm, pos, row_map, top_k);
+        hipLaunchKernelGGL(scan_segments, dim3((n_experts + 3) / 4), dim3(256), 0, st, seg, nseg, n_experts, out.counts);
+        hipLaunchKernelGGL(rank_scatter, dim3(nseg), dim3(256), 0, st, topk_idx, nk, n_experts, seg, out.counts, out.offsets,
+                           out.perm, out.pos, out.row_map, top_k, out.one_group);
     }
     if (x) {
         hipLaunchKernelGGL(gather_rows, dim3((unsigned)((nk + 3) / 4)), dim3(256), 0, st,
-                           static_cast<const u32x4*>(x), perm, nk, top_k, hidden / 8, static_cast<u32x4*>(xs));
+                           static_cast<const u32x4*>(x), out.perm, nk, top_k, hidden / 8, static_cast<u32x4*>(xs));
     }
     MOE_HIP_CHECK(hipGetLastError());
     return MOE_OK;
@@ -330,9 +250,17 @@ extern "C" int moe_dispatch(const int32_t* topk_idx, int32_t n_tokens, int32_t t
         set_error("moe_dispatch: workspace %zu bytes, need %zu", workspace_bytes, need);
         return MOE_ERR_WORKSPACE;
     }
-    return dispatch_launch(topk_idx, nk, top_k, n_experts, counts, offsets, perm, pos, row_map, x, hidden, xs,
+    return dispatch_launch(topk_idx, nk, top_k, n_experts, DispatchOut{counts, offsets, perm, pos, row_map, nullptr}, x, hidden, xs,
                            static_cast<int32_t*>(workspace), st);
 }
+
+namespace moe {
+int dispatch_on_stream(const int32_t* topk_idx, int32_t n_tokens, int32_t top_k, int32_t n_experts, const DispatchOut& out,
+                       void* workspace, hipStream_t st) {
+    return dispatch_launch(topk_idx, (int64_t)n_tokens * top_k, top_k, n_experts, out, nullptr, 0, nullptr,
+                           static_cast<int32_t*>(workspace), st);
+}
+}  // namespace moe
 
 // ---- moe_dispatch_static: the same launches with the per-segment counts in a file-scope device
 // array instead of a caller workspace, for callers that cannot allocate.
@@ -393,7 +321,8 @@ extern "C" int moe_dispatch_static(const int32_t* topk_idx, int32_t n_tokens, in
     int32_t* seg = nullptr;
     rc = static_scratch(&seg);
     if (rc != MOE_OK) return rc;
-    return dispatch_launch(topk_idx, nk, top_k, n_experts, counts, offsets, perm, pos, row_map, x, hidden, xs, seg, st);
+    return dispatch_launch(topk_idx, nk, top_k, n_experts, DispatchOut{counts, offsets, perm, pos, row_map, nullptr}, x, hidden, xs,
+                           seg, st);
 }
 
 // ---- 64-bit words from the host into device memory inside kernel arguments ----

@@ -15,6 +15,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "dispatch_small.h"
 #include "moe_math.h"
 
 namespace moe {
@@ -107,7 +108,7 @@ __device__ __forceinline__ int first_lane(bool hit, int gbase) {
 template <int GW, int MAX_EJ>
 __device__ void route_token(const float* row, const float* __restrict__ bias, const moe_router_params& p,
                             int32_t* __restrict__ idx_out, float* __restrict__ w_out,
-                            float* logits_out, float* val, bool live) {
+                            float* logits_out, uint16_t* logits_bf16, float* val, bool live) {
     // MAX_EJ: experts per lane, ceil(padded experts / GW)
     const int lane = threadIdx.x & 63, gl = lane & (GW - 1), gbase = lane - gl;
     const int E = p.n_experts;
@@ -125,6 +126,7 @@ __device__ void route_token(const float* row, const float* __restrict__ bias, co
         if (!valid[j]) L[j] = 0.0f;
         if (p.logits_bf16) L[j] = round_to_bf16(L[j]);
         if (logits_out && valid[j] && live) logits_out[gl + GW * j] = L[j];
+        if (logits_bf16 && valid[j] && live) logits_bf16[gl + GW * j] = (uint16_t)f32_to_bf16_bits(L[j]);
     }
     if (p.scoring == MOE_SCORE_SIGMOID) {
 #pragma unroll
@@ -463,7 +465,7 @@ __global__ __launch_bounds__(64 * WT * WE, 1) void router_logits_kernel(
             const bool live = t < n;
             const int tr = live ? t : n - 1, tlr = live ? tl : tb;
             route_token<GW, EJ>(lg + tlr * LG, bias, p, topk_idx + (size_t)tr * p.top_k, topk_w + (size_t)tr * p.top_k,
-                                nullptr, val + wave * 64 * EJ + lane / GW * (EJ * GW), live);
+                                nullptr, nullptr, val + wave * 64 * EJ + lane / GW * (EJ * GW), live);
         }
     }
 }
@@ -471,19 +473,42 @@ __global__ __launch_bounds__(64 * WT * WE, 1) void router_logits_kernel(
 // Routes the tokens of a logits matrix in memory, a lane group per token (the group width follows from the expert count
 // alone: it fixes the order of the softmax sum).  logits_bf16 (Mixtral): the rounded values are written back.
 template <int GW, int EJ>
-__global__ __launch_bounds__(256) void router_select_kernel(const float* __restrict__ bias, moe_router_params p,
-                                                            int32_t* __restrict__ topk_idx, float* __restrict__ topk_w,
-                                                            float* logits) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    __shared__ float val[4][64 * EJ];
-    constexpr int TPW = 64 / GW;
-    const int t = (blockIdx.x * 4 + wave) * TPW + lane / GW;
-    if (t - lane / GW >= p.n_tokens) return;
+__device__ __forceinline__ void select_tokens(int tb, const float* bias, const moe_router_params& p, int32_t* topk_idx, float* topk_w,
+                                              float* logits, uint16_t* logits_bf16, float* val) {
+    const int lane = threadIdx.x & 63, t = tb + lane / GW;
     const bool live = t < p.n_tokens;
     const int tr = live ? t : p.n_tokens - 1;
     float* row = logits + (size_t)tr * p.n_experts;
     route_token<GW, EJ>(row, bias, p, topk_idx + (size_t)tr * p.top_k, topk_w + (size_t)tr * p.top_k,
-                        p.logits_bf16 ? row : nullptr, val[wave] + lane / GW * (EJ * GW), live);
+                        p.logits_bf16 ? row : nullptr, logits_bf16 ? logits_bf16 + (size_t)tr * p.n_experts : nullptr,
+                        val + lane / GW * (EJ * GW), live);
+}
+
+template <int GW, int EJ>
+__global__ __launch_bounds__(256) void router_select_kernel(const float* __restrict__ bias, moe_router_params p,
+                                                            int32_t* __restrict__ topk_idx, float* __restrict__ topk_w,
+                                                            float* logits, uint16_t* logits_bf16) {
+    const int wave = threadIdx.x >> 6;
+    __shared__ float val[4][64 * EJ];
+    const int tb = (blockIdx.x * 4 + wave) * (64 / GW);
+    if (tb < p.n_tokens) select_tokens<GW, EJ>(tb, bias, p, topk_idx, topk_w, logits, logits_bf16, val[wave]);
+}
+
+// Selection and dispatch of a few tokens by one workgroup: its 16 waves route them, then it sorts the indices (5 tokens of
+// 256 experts: 8.3 us; the two launches 5.8 + 4.8 and the gap between them).
+template <int GW, int EJ>
+__global__ __launch_bounds__(64 * SMALL_WAVES) void router_select_dispatch_kernel(const float* __restrict__ bias, moe_router_params p,
+                                                                                  int32_t* topk_idx, float* topk_w, float* logits,
+                                                                                  uint16_t* logits_bf16, DispatchOut out) {
+    const int wave = threadIdx.x >> 6;
+    __shared__ float val[SMALL_WAVES][64 * EJ];
+    for (int tb = wave * (64 / GW); tb < p.n_tokens; tb += SMALL_WAVES * (64 / GW))
+        select_tokens<GW, EJ>(tb, bias, p, topk_idx, topk_w, logits, logits_bf16, val[wave]);
+    __threadfence_block();
+    __syncthreads();                                            // the other waves' indices are in memory
+    const volatile int32_t* idx = topk_idx;
+    constexpr int IT = kSelectDispatchTokens * 16 / (SMALL_WAVES * 64);   // (top_k <= 16)
+    dispatch_one_workgroup<IT>(p.n_tokens * p.top_k, p.n_experts, out, p.top_k, [&](int i) { return idx[i]; });
 }
 
 template <int WT, int WE, int TT, int TE, int S>
@@ -499,14 +524,62 @@ void launch_fused(const void* x, const void* w, const float* bias, const moe_rou
     hipLaunchKernelGGL((router_logits_kernel<WT, WE, 1, 1, 4, true, GW>), dim3((p.n_tokens + BT - 1) / BT), dim3(64 * WT * WE), 0, st,
                        (const uint16_t*)x, (const uint16_t*)w, bias, p, idx, tw, nullptr);
 }
-template <int GW, int EJ>
-void launch_select(const float* bias, const moe_router_params& p, int32_t* idx, float* tw, float* logits, hipStream_t st) {
-    const int per_block = 4 * (64 / GW);
-    hipLaunchKernelGGL((router_select_kernel<GW, EJ>), dim3((p.n_tokens + per_block - 1) / per_block), dim3(256), 0, st, bias, p,
-                       idx, tw, logits);
-}
 
 }  // namespace
+
+// f(GW, EJ) with the lane-group width and the experts per lane that the expert count asks for
+template <typename F>
+static void for_expert_count(int E, F f) {
+    using std::integral_constant;
+    if (E <= 16) f(integral_constant<int, 16>{}, integral_constant<int, 1>{});
+    else if (E <= 32) f(integral_constant<int, 32>{}, integral_constant<int, 1>{});
+    else if (E <= 64) f(integral_constant<int, 64>{}, integral_constant<int, 1>{});
+    else if (E <= 128) f(integral_constant<int, 64>{}, integral_constant<int, 2>{});
+    else if (E <= 192) f(integral_constant<int, 64>{}, integral_constant<int, 3>{});
+    else f(integral_constant<int, 64>{}, integral_constant<int, 4>{});
+}
+
+int router_select(const float* bias, const moe_router_params& p, int32_t* topk_idx, float* topk_w, float* logits,
+                  uint16_t* logits_bf16, hipStream_t st) {
+    for_expert_count(p.n_experts, [&](auto gw, auto ej) {
+        constexpr int GW = decltype(gw)::value, EJ = decltype(ej)::value, per_block = 4 * (64 / GW);
+        hipLaunchKernelGGL((router_select_kernel<GW, EJ>), dim3((p.n_tokens + per_block - 1) / per_block), dim3(256), 0, st, bias, p,
+                           topk_idx, topk_w, logits, logits_bf16);
+    });
+    MOE_HIP_CHECK(hipGetLastError());
+    return MOE_OK;
+}
+
+int router_select_dispatch(const float* bias, const moe_router_params& p, int32_t* topk_idx, float* topk_w, float* logits,
+                           uint16_t* logits_bf16, const DispatchOut& out, hipStream_t st) {
+    for_expert_count(p.n_experts, [&](auto gw, auto ej) {
+        constexpr int GW = decltype(gw)::value, EJ = decltype(ej)::value;
+        hipLaunchKernelGGL((router_select_dispatch_kernel<GW, EJ>), dim3(1), dim3(64 * SMALL_WAVES), 0, st, bias, p, topk_idx, topk_w,
+                           logits, logits_bf16, out);
+    });
+    MOE_HIP_CHECK(hipGetLastError());
+    return MOE_OK;
+}
+
+int router_logits(const void* x, const void* w_gate, const moe_router_params& p, float* logits, hipStream_t st) {
+    const int E = p.n_experts, n = p.n_tokens;
+    // One tile per wave up to 4096 tokens of 256 experts: the matrix cores of all CUs are then busy for less than about
+    // four rounds of it, and smaller workgroups leave less of the last round idle; and where the last block of 64 experts
+    // would be half empty (160 experts: 32-expert blocks fit).  Beyond, 2 x 2 tiles per wave, in workgroups of 8 waves
+    // where 128-expert blocks fit and there is one for every CU.  Measured, logits alone (us, h = 7168):
+    //   256 experts  1024 tokens: one tile 33;  3000: 86;  4096: 121, 2 x 2 in 4 waves 110, in 8 waves 208
+    //                8192: 2 x 2 in 4 waves 215, in 8 waves 211;  65536: one tile 1890, 1690, 1645
+    //   160 experts  16384 tokens: one tile 264, 2 x 2 with 32-expert blocks 301
+    //   8 experts    16384 tokens (h = 6144): 4 waves along the tokens 35, 2 waves 38
+    const int64_t work = (int64_t)n * E;
+    if (E <= 16) launch_logits<4, 1, 1, 1, 4>(x, w_gate, p, logits, st);
+    else if (work < (1 << 20) || (E % 64 != 0 && E % 64 <= 32)) launch_logits<2, 2, 1, 1, 4>(x, w_gate, p, logits, st);
+    else if (work < (1 << 21) || (E % 128 != 0 && E % 128 <= 64)) launch_logits<2, 2, 2, 2, 4>(x, w_gate, p, logits, st);
+    else launch_logits<2, 4, 2, 2, 3>(x, w_gate, p, logits, st);
+    MOE_HIP_CHECK(hipGetLastError());
+    return MOE_OK;
+}
+
 }  // namespace moe
 
 namespace moe {
@@ -537,9 +610,7 @@ extern "C" int moe_router_rmsnorm(const void* x, const void* norm_weight, float 
 }
 
 namespace moe {
-namespace {
-int route(const void* x, const void* w_gate, const float* bias, const moe_router_params* params, int32_t* topk_idx,
-          float* topk_w, float* logits_out, void* stream) {
+int check_router(const void* x, const void* w_gate, const moe_router_params* params, const int32_t* topk_idx, const float* topk_w) {
     MOE_REQUIRE(params != nullptr, "moe_router: params is NULL");
     const moe_router_params& p = *params;
     MOE_REQUIRE(p.n_tokens >= 0, "moe_router: n_tokens %d < 0", p.n_tokens);
@@ -564,8 +635,19 @@ int route(const void* x, const void* w_gate, const float* bias, const moe_router
                     "moe_router: noaux_tc needs at least 2 experts per group");
     }
     MOE_REQUIRE(p.hidden < 1 << 22, "moe_router: hidden %d: 256 rows have to lie within 2 GiB", p.hidden);
+    return MOE_OK;
+}
+}  // namespace moe
+
+namespace moe {
+namespace {
+int route(const void* x, const void* w_gate, const float* bias, const moe_router_params* params, int32_t* topk_idx,
+          float* topk_w, float* logits_out, void* stream) {
+    const int ok = check_router(x, w_gate, params, topk_idx, topk_w);
+    if (ok != MOE_OK || params->n_tokens == 0) return ok;
+    const moe_router_params& p = *params;
     hipStream_t st = as_stream(stream);
-    const int E = p.n_experts, n = p.n_tokens;
+    const int E = p.n_experts;
     if (logits_out == nullptr) {
         if (E <= 16) launch_fused<2, 1, 16>(x, w_gate, bias, p, topk_idx, topk_w, st);
         else if (E <= 32) launch_fused<1, 4, 32>(x, w_gate, bias, p, topk_idx, topk_w, st);
@@ -573,27 +655,8 @@ int route(const void* x, const void* w_gate, const float* bias, const moe_router
         MOE_HIP_CHECK(hipGetLastError());
         return MOE_OK;
     }
-    // One tile per wave up to 4096 tokens of 256 experts: the matrix cores of all CUs are then busy for less than about
-    // four rounds of it, and smaller workgroups leave less of the last round idle; and where the last block of 64 experts
-    // would be half empty (160 experts: 32-expert blocks fit).  Beyond, 2 x 2 tiles per wave, in workgroups of 8 waves
-    // where 128-expert blocks fit and there is one for every CU.  Measured, logits alone (us, h = 7168):
-    //   256 experts  1024 tokens: one tile 33;  3000: 86;  4096: 121, 2 x 2 in 4 waves 110, in 8 waves 208
-    //                8192: 2 x 2 in 4 waves 215, in 8 waves 211;  65536: one tile 1890, 1690, 1645
-    //   160 experts  16384 tokens: one tile 264, 2 x 2 with 32-expert blocks 301
-    //   8 experts    16384 tokens (h = 6144): 4 waves along the tokens 35, 2 waves 38
-    const int64_t work = (int64_t)n * E;
-    if (E <= 16) launch_logits<4, 1, 1, 1, 4>(x, w_gate, p, logits_out, st);
-    else if (work < (1 << 20) || (E % 64 != 0 && E % 64 <= 32)) launch_logits<2, 2, 1, 1, 4>(x, w_gate, p, logits_out, st);
-    else if (work < (1 << 21) || (E % 128 != 0 && E % 128 <= 64)) launch_logits<2, 2, 2, 2, 4>(x, w_gate, p, logits_out, st);
-    else launch_logits<2, 4, 2, 2, 3>(x, w_gate, p, logits_out, st);
-    if (E <= 16) launch_select<16, 1>(bias, p, topk_idx, topk_w, logits_out, st);
-    else if (E <= 32) launch_select<32, 1>(bias, p, topk_idx, topk_w, logits_out, st);
-    else if (E <= 64) launch_select<64, 1>(bias, p, topk_idx, topk_w, logits_out, st);
-    else if (E <= 128) launch_select<64, 2>(bias, p, topk_idx, topk_w, logits_out, st);
-    else if (E <= 192) launch_select<64, 3>(bias, p, topk_idx, topk_w, logits_out, st);
-    else launch_select<64, 4>(bias, p, topk_idx, topk_w, logits_out, st);
-    MOE_HIP_CHECK(hipGetLastError());
-    return MOE_OK;
+    const int rc = router_logits(x, w_gate, p, logits_out, st);
+    return rc != MOE_OK ? rc : router_select(bias, p, topk_idx, topk_w, logits_out, nullptr, st);
 }
 }  // namespace
 }  // namespace moe

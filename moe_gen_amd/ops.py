@@ -51,6 +51,19 @@ def _need(t: torch.Tensor, dtype, name: str, shape=None):
         raise ValueError(f"{name} must have shape {tuple(shape)}, got {tuple(t.shape)}")
 
 
+def router_params(spec: RouterSpec, n: int, h: int, bias) -> "N.RouterParams":
+    if spec.scoring not in SCORE:
+        raise NotImplementedError(f"insupportable scoring function for MoE gating: {spec.scoring}")
+    if spec.method not in METHOD:
+        raise NotImplementedError(f"insupportable TopK function for MoE gating: {spec.method}")
+    if spec.method == "noaux_tc" and bias is None:
+        raise ValueError("noaux_tc routing needs e_score_correction_bias")
+    return N.RouterParams(n, h, spec.n_experts, spec.top_k, spec.n_group or 1, spec.topk_group or 1, SCORE[spec.scoring],
+                          METHOD[spec.method], int(spec.norm_topk_prob), spec.scale_mode,
+                          int(spec.logits_bf16), int(spec.weights_bf16), spec.norm_eps,
+                          spec.routed_scaling_factor)
+
+
 def router(x: torch.Tensor, gate_w: torch.Tensor, bias, spec: RouterSpec, want_logits: bool = False,
            norm_weight: torch.Tensor | None = None, eps: float = 1e-6):
     """x bf16 [n,h], gate_w bf16 [E,h], bias fp32 [E] | None ->
@@ -65,19 +78,10 @@ def router(x: torch.Tensor, gate_w: torch.Tensor, bias, spec: RouterSpec, want_l
     _need(gate_w, torch.bfloat16, "gate weight", (E, h))
     if bias is not None:
         _need(bias, torch.float32, "e_score_correction_bias", (E,))
-    if spec.scoring not in SCORE:
-        raise NotImplementedError(f"insupportable scoring function for MoE gating: {spec.scoring}")
-    if spec.method not in METHOD:
-        raise NotImplementedError(f"insupportable TopK function for MoE gating: {spec.method}")
-    if spec.method == "noaux_tc" and bias is None:
-        raise ValueError("noaux_tc routing needs e_score_correction_bias")
+    p = router_params(spec, n, h, bias)
     idx = torch.empty((n, k), dtype=torch.int32, device=x.device)
     w = torch.empty((n, k), dtype=torch.float32, device=x.device)
     lg = torch.empty((n, E), dtype=torch.float32, device=x.device)     # (the library routes from a logits matrix in memory)
-    p = N.RouterParams(n, h, E, k, spec.n_group or 1, spec.topk_group or 1, SCORE[spec.scoring],
-                       METHOD[spec.method], int(spec.norm_topk_prob), spec.scale_mode,
-                       int(spec.logits_bf16), int(spec.weights_bf16), spec.norm_eps,
-                       spec.routed_scaling_factor)
     if norm_weight is not None:
         _need(norm_weight, torch.bfloat16, "norm weight", (h,))
         xn = torch.empty_like(x)
@@ -151,6 +155,11 @@ class ExpertPointers:
     s_down: torch.Tensor | None = None
     keep: tuple = ()
 
+    def __post_init__(self):
+        # the part of a moe_mlp_group that does not change from call to call
+        self.weights = N.MlpGroup(None, 0, 0, None, _ptr(self.w_gate), _ptr(self.w_up), _ptr(self.w_down), _ptr(self.s_gate),
+                                  _ptr(self.s_up), _ptr(self.s_down), None, self.n_experts, self.inter, 0, int(self.fp8), None, None)
+
 
 def expert_pointers(gates, ups, downs, s_gates=None, s_ups=None, s_downs=None, device=None) -> ExpertPointers:
     """Build pointer tables from lists of per-expert tensors: gate/up [I,h], down [h,I]
@@ -159,27 +168,24 @@ def expert_pointers(gates, ups, downs, s_gates=None, s_ups=None, s_downs=None, d
     I, h = gates[0].shape
     fp8 = gates[0].dtype == torch.float8_e4m3fn
     want = torch.float8_e4m3fn if fp8 else torch.bfloat16
-    for i in range(E):
-        _need(gates[i], want, f"experts[{i}].gate weight", (I, h))
-        _need(ups[i], want, f"experts[{i}].up weight", (I, h))
-        _need(downs[i], want, f"experts[{i}].down weight", (h, I))
-    dev = device or gates[0].device
-
-    def table(ts):
-        return torch.tensor([t.data_ptr() for t in ts], dtype=torch.int64).to(dev, non_blocking=False)
-
-    sg = su = sd = None
+    cols = [("gate weight", gates, want, (I, h)), ("up weight", ups, want, (I, h)), ("down weight", downs, want, (h, I))]
     if fp8:
         if s_gates is None or s_ups is None or s_downs is None:
             raise ValueError("fp8 expert weights need their *_scale_inv block scales")
         bi, bh = -(-I // 128), -(-h // 128)
+        cols += [("gate scale", s_gates, torch.float32, (bi, bh)), ("up scale", s_ups, torch.float32, (bi, bh)),
+                 ("down scale", s_downs, torch.float32, (bh, bi))]
+    vals = []
+    for what, ts, dtype, shape in cols:
         for i in range(E):
-            _need(s_gates[i], torch.float32, f"experts[{i}].gate scale", (bi, bh))
-            _need(s_ups[i], torch.float32, f"experts[{i}].up scale", (bi, bh))
-            _need(s_downs[i], torch.float32, f"experts[{i}].down scale", (bh, bi))
-        sg, su, sd = table(s_gates), table(s_ups), table(s_downs)
-    keep = (tuple(gates), tuple(ups), tuple(downs), tuple(s_gates or ()), tuple(s_ups or ()), tuple(s_downs or ()))
-    return ExpertPointers(E, h, I, fp8, table(gates), table(ups), table(downs), sg, su, sd, keep)
+            t = ts[i]
+            if not (t.dtype is dtype and t.shape == shape and t.is_cuda and t.is_contiguous()):
+                _need(t, dtype, f"experts[{i}].{what}", shape)
+            vals.append(t.data_ptr())
+    t = _upload_words(vals, device or gates[0].device)        # all tables in one array, written by one small launch
+    tab = [t[c * E:(c + 1) * E] for c in range(len(cols))]
+    keep = tuple(tuple(ts) for _, ts, _, _ in cols)
+    return ExpertPointers(E, h, I, fp8, tab[0], tab[1], tab[2], *(tab[3:] if fp8 else (None, None, None)), keep)
 
 
 def _upload_words(values, device) -> torch.Tensor:
@@ -322,7 +328,7 @@ def mlp_group(x: torch.Tensor, row_map, ptrs: ExpertPointers, offsets: torch.Ten
     _need(act, torch.bfloat16, "act", (n_rows, I))
     _need(y, torch.bfloat16, "y", (n_rows, h))
     m = N.MlpGroup(_ptr(x), x.shape[0], n_rows, _ptr(row_map), _ptr(ptrs.w_gate), _ptr(ptrs.w_up), _ptr(ptrs.w_down),
-                   _ptr(ptrs.s_gate), _ptr(ptrs.s_up), _ptr(ptrs.s_down), _ptr(offsets), E, I, max_rows, 0, _ptr(act), _ptr(y))
+                   _ptr(ptrs.s_gate), _ptr(ptrs.s_up), _ptr(ptrs.s_down), _ptr(offsets), E, I, max_rows, int(ptrs.fp8), _ptr(act), _ptr(y))
     return m, act, y
 
 
@@ -335,6 +341,37 @@ def grouped_swiglu_joint(routed, shared, hidden: int, fp8: bool, phases: int = P
     """The expert MLPs of `routed` and of `shared` (structs of mlp_group, of the same weight type; shared may be None)."""
     N.check(N.lib().moe_grouped_swiglu_joint(ctypes.byref(routed), None if shared is None else ctypes.byref(shared), hidden,
                                              int(fp8), phases, _stream()), "moe_grouped_swiglu_joint")
+
+
+def layer_forward(x: torch.Tensor, norm_weight, eps: float, gate_w: torch.Tensor, bias, spec: RouterSpec, routed: ExpertPointers,
+                  shared, combine_mode: int, join_shared: bool, want_logits: bool):
+    """A whole layer call on x bf16 [n,h] with resident weights as one call into the library (moe_layer_forward):
+    (out, topk_idx, topk_weight, counts, logits bf16 | None)."""
+    n, h = x.shape
+    E, k, dev = spec.n_experts, spec.top_k, x.device
+    _need(x, torch.bfloat16, "x")
+    _need(gate_w, torch.bfloat16, "gate weight", (E, h))
+    if bias is not None:
+        _need(bias, torch.float32, "e_score_correction_bias", (E,))
+    if norm_weight is not None:
+        _need(norm_weight, torch.bfloat16, "norm weight", (h,))
+    if routed.hidden != h or routed.n_experts != E or (shared is not None and shared.hidden != h):
+        raise ValueError(f"x has hidden size {h} and the gate {E} experts, the experts are {routed.n_experts} of hidden size {routed.hidden}")
+    p = router_params(spec, n, h, bias)
+    out = torch.empty_like(x)
+    idx = torch.empty((n, k), dtype=torch.int32, device=dev)
+    w = torch.empty((n, k), dtype=torch.float32, device=dev)
+    counts = torch.empty(E, dtype=torch.int32, device=dev)
+    logits = torch.empty((n, E), dtype=torch.bfloat16, device=dev) if want_logits else None
+    a = N.LayerArgs(_ptr(x), _ptr(norm_weight), gate_w.data_ptr(), _ptr(bias), ctypes.addressof(p), ctypes.addressof(routed.weights),
+                    None if shared is None else ctypes.addressof(shared.weights), idx.data_ptr(), w.data_ptr(), counts.data_ptr(),
+                    _ptr(logits), out.data_ptr(), None, 0, eps, combine_mode, int(join_shared))
+    L, ref = N.lib(), ctypes.byref(a)
+    a.workspace_bytes = L.moe_layer_workspace_bytes(ref)
+    ws = torch.empty(a.workspace_bytes, dtype=torch.uint8, device=dev)
+    a.workspace = ws.data_ptr()
+    N.check(L.moe_layer_forward(ref, _stream()), "moe_layer_forward")
+    return out, idx, w, counts, logits
 
 
 def dequant_fp8_block128(q: torch.Tensor, scale: torch.Tensor) -> torch.Tensor:

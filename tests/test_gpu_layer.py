@@ -191,3 +191,32 @@ def test_single_shared_expert_joins_the_routed_call_at_small_batches(fp8):
         assert (a - b).abs().max().item() <= 2e-2 * b.abs().max().item()
     else:
         assert torch.equal(joined, apart)
+
+
+@pytest.mark.parametrize("name,E", [("deepseek_v3_w8a16", 256), ("deepseek_v2_236b", 160), ("deepseek_v2_lite", 64), ("deepseek_v2_lite", 24),
+                                    ("mixtral_8x7b", 8)])
+def test_layer_call_equals_the_separate_calls(name, E):
+    """The whole-layer call of the library (selection and dispatch in one launch up to 16 ... 64 tokens) against the stage-by-stage
+    path that an attached timer takes, at both sides of 64 tokens and of 16, where the experts change kernels, with and
+    without the norm around the layer: output, routing, counts and Mixtral's logits bit for bit."""
+    from moe_gen_amd import norm_moe_residual, synthetic
+    from moe_gen_amd.block import StageTimer
+    w = synthetic.WORKLOADS[name].scaled(n=200, h=512, I=256, seq=200, E=E)
+    blk = synthetic.build_block(w, device="cuda", gen_device="cpu")
+    xs = synthetic.hidden_states(w, "cpu").cuda()
+    nw = (1 + 0.1 * torch.randn(512, generator=torch.Generator().manual_seed(1))).to(torch.bfloat16).cuda()
+    for n in (1, 15, 16, 17, 63, 64, 65, 200):
+        x = xs[:, :n].contiguous()
+        for norm in (False, True):
+            print(f"layer call {name} E={E} n={n} norm={norm}", flush=True)
+            run = lambda: norm_moe_residual(blk, x, nw) if norm else blk(x)
+            got = []
+            for timer in (None, StageTimer()):
+                blk.stage_timer = timer
+                res = run()
+                res = res if isinstance(res, tuple) else (res,)
+                got.append([*res, blk.last_topk_idx, blk.last_topk_weight, blk.last_counts])
+            torch.cuda.synchronize()
+            assert len(got[0]) == len(got[1])
+            for a, b in zip(*got):
+                assert a.dtype == b.dtype and torch.equal(a, b), (n, norm)
