@@ -116,8 +116,9 @@ class SwiGLUMLP(nn.Module):
         n = x2d.shape[0]
         if engine_backed(self):
             raise RuntimeError("SwiGLUMLP.forward: engine-backed weights are handled by the MoE block")
-        ptrs = collect_pointers([self], self.__dict__.setdefault("_moe_cache", {}))
-        # (the row range travels in kernel arguments: a copy from the host would stop the stream)
+        # (tables and row range travel in kernel arguments: a copy from the host would stop the stream, and tables kept
+        # for the next call would hide a weight or scale that has been replaced in between)
+        ptrs = collect_pointers([self], None)
         offsets = ops._upload_words([n << 32], x.device).view(torch.int32)
         return _grouped(None, "mlp", x2d, None, ptrs, offsets, n, n).view(*shape)
 
@@ -179,12 +180,12 @@ def _param(lin, name):
     return None if p is None else p.data
 
 
-def _pointer_table(rows):
+def _pointer_table(rows, one_call):
     """ExpertPointers from a list of (gate, up, down, s_gate, s_up, s_down) tuples."""
     cols = list(zip(*rows))
     fp8 = cols[0][0].dtype == FP8
     return ops.expert_pointers(list(cols[0]), list(cols[1]), list(cols[2]),
-                               *((list(c) for c in cols[3:]) if fp8 else (None, None, None)))
+                               *((list(c) for c in cols[3:]) if fp8 else (None, None, None)), one_call=one_call)
 
 
 def engine_backed(expert) -> bool:
@@ -209,13 +210,13 @@ def any_engine_backed(experts) -> bool:
 
 def collect_pointers(experts, cache):
     """Pointer tables for a list of RESIDENT expert modules, cached in `cache` (a dict) keyed on
-    the storage addresses of the first and last expert."""
+    the storage addresses of the first and last expert; without one they serve this call on this stream only."""
     first, last = _unwrap(experts[0]), _unwrap(experts[-1])
     f = _param(_linear(first, first.names[0]), "weight")
     stamp = (len(experts), f.data_ptr(), f.dtype, f.shape, _param(_linear(last, last.names[2]), "weight").data_ptr())
     if cache is not None and cache.get("stamp") == stamp:
         return cache["ptrs"]
-    p = _pointer_table([_tensors_of(ex) for ex in experts])
+    p = _pointer_table([_tensors_of(ex) for ex in experts], one_call=cache is None)
     if cache is not None:
         cache["stamp"], cache["ptrs"] = stamp, p
     return p

@@ -156,12 +156,20 @@ class ExpertPointers:
     keep: tuple = ()
 
     def __post_init__(self):
-        # the part of a moe_mlp_group that does not change from call to call
+        # The part of a moe_mlp_group that does not change from call to call.  It holds addresses of the tables above: a
+        # copy (copy.deepcopy or pickle of a block that has run) gets one of its own tables.
         self.weights = N.MlpGroup(None, 0, 0, None, _ptr(self.w_gate), _ptr(self.w_up), _ptr(self.w_down), _ptr(self.s_gate),
                                   _ptr(self.s_up), _ptr(self.s_down), None, self.n_experts, self.inter, 0, int(self.fp8), None, None)
 
+    def __getstate__(self):
+        return {k: v for k, v in self.__dict__.items() if k != "weights"}
 
-def expert_pointers(gates, ups, downs, s_gates=None, s_ups=None, s_downs=None, device=None) -> ExpertPointers:
+    def __setstate__(self, state):
+        self.__dict__.update(state)
+        self.__post_init__()
+
+
+def expert_pointers(gates, ups, downs, s_gates=None, s_ups=None, s_downs=None, device=None, one_call=False) -> ExpertPointers:
     """Build pointer tables from lists of per-expert tensors: gate/up [I,h], down [h,I]
     (bf16, or float8_e4m3fn with fp32 scales [ceil(r/128), ceil(c/128)])."""
     E = len(gates)
@@ -182,7 +190,10 @@ def expert_pointers(gates, ups, downs, s_gates=None, s_ups=None, s_downs=None, d
             if not (t.dtype is dtype and t.shape == shape and t.is_cuda and t.is_contiguous()):
                 _need(t, dtype, f"experts[{i}].{what}", shape)
             vals.append(t.data_ptr())
-    t = _upload_words(vals, device or gates[0].device)        # all tables in one array, written by one small launch
+    # All tables in one array.  The copy from the host returns when they are there, for a later call on any stream; tables
+    # of one call (one_call) are written on its own stream by a small launch, without a wait.
+    dev = device or gates[0].device
+    t = _upload_words(vals, dev) if one_call else torch.tensor(vals, dtype=torch.int64).to(dev)
     tab = [t[c * E:(c + 1) * E] for c in range(len(cols))]
     keep = tuple(tuple(ts) for _, ts, _, _ in cols)
     return ExpertPointers(E, h, I, fp8, tab[0], tab[1], tab[2], *(tab[3:] if fp8 else (None, None, None)), keep)

@@ -220,3 +220,27 @@ def test_layer_call_equals_the_separate_calls(name, E):
             assert len(got[0]) == len(got[1])
             for a, b in zip(*got):
                 assert a.dtype == b.dtype and torch.equal(a, b), (n, norm)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+def test_dense_mlp_sees_replaced_weights_and_a_copied_block_its_own(fp8):
+    """A dense MLP whose up projection (fp8: or its block scales) is replaced between two calls computes with the new one,
+    and a deep copy of a block that has run gives the block's results after the block's weights are gone."""
+    import copy
+    from moe_gen_amd import synthetic
+    w = synthetic.WORKLOADS["deepseek_v3_w8a16" if fp8 else "deepseek_v2_lite"].scaled(n=24, h=512, I=256, seq=24)
+    blk = synthetic.build_block(w, device="cuda", gen_device="cpu")
+    x = synthetic.hidden_states(w, "cpu").cuda()
+    mlp = blk.shared_experts
+    first = mlp(x)
+    lin = mlp.up_proj
+    name = "weight_scale_inv" if fp8 else "weight"
+    setattr(lin, name, torch.nn.Parameter(getattr(lin, name).data * 2, requires_grad=False))
+    second = mlp(x)
+    assert torch.equal(second, 2 * first)                  # (a power of two: every product, sum and rounding scales)
+    out = blk(x)
+    twin = copy.deepcopy(blk)
+    for ex in blk.experts:
+        for lin in (ex.gate_proj, ex.up_proj, ex.down_proj):
+            lin.weight.data.view(torch.uint8).zero_()
+    assert torch.equal(twin(x), out)

@@ -1,9 +1,12 @@
 """Host-side behaviour of the blocks that needs no GPU: parameter tree, errors, no CPU fallback."""
+import copy
+import pickle
+
 import pytest
 import torch
 
 import moe_gen_amd as M
-from moe_gen_amd import deepseek_v2, synthetic
+from moe_gen_amd import deepseek_v2, ops, synthetic
 
 
 def tiny(family):
@@ -41,6 +44,17 @@ def test_no_cpu_fallback():
     with pytest.raises((RuntimeError, TypeError)):
         M.ops.router(torch.zeros(4, 16, dtype=torch.bfloat16), torch.zeros(8, 16, dtype=torch.bfloat16), None,
                      M.ops.RouterSpec(8, 2))
+
+
+def test_pointer_tables_survive_a_copy():
+    """A block that has run keeps its tables: copy.deepcopy and pickle of it go through, and the copy's struct holds the
+    addresses of the copy's tables."""
+    table = [torch.arange(4) for _ in range(3)]
+    p = ops.ExpertPointers(4, 64, 128, False, *table)
+    for q in (copy.deepcopy(p), pickle.loads(pickle.dumps(p))):
+        assert torch.equal(q.w_up, p.w_up) and q.w_up.data_ptr() != p.w_up.data_ptr()
+        assert q.weights.w_up == q.w_up.data_ptr() and q.weights.w_gate == q.w_gate.data_ptr()
+        assert (q.weights.n_experts, q.weights.inter, q.weights.s_down) == (4, 128, None)
 
 
 def test_unsupported_rules_raise_like_the_reference():
