@@ -222,10 +222,20 @@ typedef struct moe_mlp_group {
     const float* const* s_down;
     const int32_t* offsets;
     int32_t n_experts, inter, max_rows;
-    int32_t fp8;                 /* weight type, read by moe_layer_forward (elsewhere the call says it) */
+    int32_t fp8;                 /* weight type, read by moe_layer_forward and moe_mlp_workspace_bytes (elsewhere the call says it) */
     void* act;
     void* y;
+    void* workspace;             /* moe_mlp_workspace_bytes() bytes, or NULL */
+    size_t workspace_bytes;
 } moe_mlp_group;
+
+/*
+ * Device scratch with which a group runs faster, 0 if none does: ONE fp8 MLP (n_experts 1) of few rows and a long
+ * intermediate size (DeepSeek-V3's dense layers, up to 512 rows) gives every column tile of the down projection to several
+ * workgroups, which leave their fp32 sums here.  Without it, or with less, the call runs as the two above.  A row's bits may differ
+ * between the two by the order of its sums.
+ */
+size_t moe_mlp_workspace_bytes(const moe_mlp_group* group, int32_t hidden);
 
 /*
  * The routed experts and the shared expert(s) of a layer (DeepseekV3MoE.forward, modeling_deepseek_v3.py:618-625; one MLP

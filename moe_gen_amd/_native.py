@@ -32,7 +32,7 @@ class MlpGroup(ctypes.Structure):
         ("w_gate", c_void_p), ("w_up", c_void_p), ("w_down", c_void_p),
         ("s_gate", c_void_p), ("s_up", c_void_p), ("s_down", c_void_p), ("offsets", c_void_p),
         ("n_experts", c_int32), ("inter", c_int32), ("max_rows", c_int32), ("fp8", c_int32),
-        ("act", c_void_p), ("y", c_void_p),
+        ("act", c_void_p), ("y", c_void_p), ("workspace", c_void_p), ("workspace_bytes", c_size_t),
     ]
 
 
@@ -69,6 +69,7 @@ SIGNATURES = {
                                                 c_int32, c_void_p, c_void_p, c_int32, c_void_p, c_size_t, c_void_p]),
     "moe_grouped_swiglu_joint": (ctypes.c_int, [ctypes.POINTER(MlpGroup), ctypes.POINTER(MlpGroup), c_int32, c_int32, c_int32,
                                                 c_void_p]),
+    "moe_mlp_workspace_bytes": (c_size_t, [ctypes.POINTER(MlpGroup), c_int32]),
     "moe_shared_joins": (ctypes.c_int, [ctypes.POINTER(MlpGroup), ctypes.POINTER(MlpGroup), c_int32]),
     "moe_layer_workspace_bytes": (c_size_t, [ctypes.POINTER(LayerArgs)]),
     "moe_layer_forward": (ctypes.c_int, [ctypes.POINTER(LayerArgs), c_void_p]),

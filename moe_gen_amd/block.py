@@ -120,7 +120,7 @@ class SwiGLUMLP(nn.Module):
         # for the next call would hide a weight or scale that has been replaced in between)
         ptrs = collect_pointers([self], None)
         offsets = ops._upload_words([n << 32], x.device).view(torch.int32)
-        return _grouped(None, "mlp", x2d, None, ptrs, offsets, n, n).view(*shape)
+        return ops.grouped_swiglu_one(x2d, ptrs, offsets, n).view(*shape)
 
 
 def _unwrap(expert):

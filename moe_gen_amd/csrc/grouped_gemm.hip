@@ -690,9 +690,21 @@ struct SBuf {
     uint8_t *w, *t;
 };
 
-template <int TG, bool SWIGLU>   // TG: 16-row token groups multiplied (the expert has at most 16 TG <= 64 rows)
+// How the split kernel cuts one problem: row tiles of `rows`, k into `slices` of up to `blocks` blocks of 128
+struct SplitPlan {
+    int m_tiles, rows, slices, blocks;
+};
+
+// A slice of k for a tile whose sums other workgroups share (split kernel): blocks first .. first + count - 1 of 128 k, and
+// where the fp32 sums go: part[(row - row_base) * N + column]
+struct KSlice {
+    int first, count, row_base;
+    float* part;
+};
+
+template <int TG, bool SWIGLU, bool SPLIT = false>   // TG: 16-row token groups multiplied (the expert has at most 16 TG <= 64 rows)
 __device__ __forceinline__ void stream8_tile(const GemmArgs& g, SBuf buf0, SBuf buf1, SBuf buf2, int e, int row0,
-                                             int row_end, int n_tile) {
+                                             int row_end, int n_tile, KSlice ks = {}) {
     constexpr int NBLK = SWIGLU ? 128 : 256;
     constexpr int NDW = 4, NDT = 2;               // DMA instructions per wave and 128-k block: weights, tokens
     // Operations that may stay in flight at the wait for a block: the DMA of the next block, NDW + NDT instructions
@@ -700,11 +712,13 @@ __device__ __forceinline__ void stream8_tile(const GemmArgs& g, SBuf buf0, SBuf 
     // older still: not counting them costs at most a wait for two small loads that hit in L2, and keeps the count
     // right for the first block, which has no scale loads of a block before it behind its DMA.
     constexpr int VM_BLOCK = NDW + NDT;
+    static_assert(!(SPLIT && SWIGLU), "slices of k: the down projection");
     static_assert(TG >= 1 && 16 * TG <= S8_TROWS, "token rows staged");
     const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
     const int n0 = n_tile * NBLK;
     const int K = g.K, N = g.N;
-    const int npair = K >> 7;
+    const int npair = SPLIT ? ks.count : K >> 7;             // blocks of 128 k multiplied
+    const int kfirst = SPLIT ? ks.first : 0;
     // N tile t walks k from 128-k block t (mod the number of blocks), so that the requests in flight on the chip do
     // not share their low address bits (weight rows are K bytes apart); a column's order depends on its tile alone
     const int prot = n_tile % npair;
@@ -720,7 +734,7 @@ __device__ __forceinline__ void stream8_tile(const GemmArgs& g, SBuf buf0, SBuf 
     for (int j = 0; j < 2; ++j) {
         bmat[j] = uni_ptr((SWIGLU && j == 1) ? g.b1[e] : g.b0[e]);
         sc[j] = (gptr_f32)(uintptr_t)uni_ptr((SWIGLU && j == 1) ? g.s1[e] : g.s0[e]);
-        srow[j] = min((n0 + (SWIGLU ? 0 : 32 * wave)) >> 7, (N >> 7) - 1) * npair;
+        srow[j] = min((n0 + (SWIGLU ? 0 : 32 * wave)) >> 7, (N >> 7) - 1) * (K >> 7) + kfirst;
     }
 #pragma unroll
     for (int i = 0; i < NDW; ++i) {
@@ -763,11 +777,11 @@ __device__ __forceinline__ void stream8_tile(const GemmArgs& g, SBuf buf0, SBuf 
         pr = pr >= npair ? pr - npair : pr;
         if (i < NDW) {
             const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)bmat[i >> 1], 0, live, 0x00020000);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_u8)(buf.w + wave * 4096 + i * 1024), 16, w_voff[i], (uint32_t)(pr * 128), 0, 2);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_u8)(buf.w + wave * 4096 + i * 1024), 16, w_voff[i], (uint32_t)((pr + kfirst) * 128), 0, 2);
         } else {
             const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)a_base, 0, live & a_records, 0x00020000);
             __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_u8)(buf.t + wave * 2048 + (i - NDW) * 1024), 16, t_voff[i - NDW],
-                                                     (uint32_t)(pr * 256), 0, 0);
+                                                     (uint32_t)((pr + kfirst) * 256), 0, 0);
         }
     };
     auto dma = [&](int p_pipe, SBuf buf) {
@@ -865,7 +879,9 @@ __device__ __forceinline__ void stream8_tile(const GemmArgs& g, SBuf buf0, SBuf 
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 const int col = n0 + 32 * wave + 16 * j + 4 * q;
-                if (col < N) *reinterpret_cast<u32x2*>(g.c + (size_t)r * N + col) = epilogue_pack<false>(acc[t][j], acc[t][j]);
+                if (col >= N) continue;
+                if (SPLIT) *reinterpret_cast<f32x4*>(ks.part + (size_t)(r - ks.row_base) * N + col) = acc[t][j];
+                else *reinterpret_cast<u32x2*>(g.c + (size_t)r * N + col) = epilogue_pack<false>(acc[t][j], acc[t][j]);
             }
         }
     }
@@ -886,16 +902,18 @@ __device__ __forceinline__ void stream8_tile(const GemmArgs& g, SBuf buf0, SBuf 
 // weights keep their three buffers of 128 k: 96 + 48 KiB.  Per half-block a wave issues 2 weight DMA instructions (of
 // the block two ahead) and 2 token DMA instructions (of the half two ahead), and the wait before a half's barrier
 // leaves the 4 of the half before in flight.  k starts at block 0 unless the kernel has the call to itself.
-template <int TG, bool SWIGLU>   // TG: 16-row token groups multiplied (1 .. 8)
+template <int TG, bool SWIGLU, bool SPLIT = false>   // TG: 16-row token groups multiplied (1 .. 8)
 __device__ __forceinline__ void stream8x_tile(const GemmArgs& g, SBuf b0, SBuf b1, SBuf b2, int e, int row0, int row_end,
-                                              int n_tile, bool rotate) {
+                                              int n_tile, bool rotate, KSlice ks = {}) {
     constexpr int NBLK = SWIGLU ? 128 : 256;
     constexpr int VM_HALF = 4;                    // DMA instructions per wave and half-block: 2 weights + 2 tokens
+    static_assert(!(SPLIT && SWIGLU), "slices of k: the down projection");
     static_assert(TG >= 1 && TG <= 8, "token rows staged");
     const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
     const int n0 = n_tile * NBLK;
     const int K = g.K, N = g.N;
-    const int npair = K >> 7;
+    const int npair = SPLIT ? ks.count : K >> 7;             // blocks of 128 k multiplied
+    const int kfirst = SPLIT ? ks.first : 0;
     const int prot = rotate ? n_tile % npair : 0;             // k_rotation in blocks of 128 k
 
     // ---- DMA coordinates ----
@@ -910,7 +928,7 @@ __device__ __forceinline__ void stream8x_tile(const GemmArgs& g, SBuf b0, SBuf b
     for (int j = 0; j < 2; ++j) {
         bmat[j] = uni_ptr((SWIGLU && j == 1) ? g.b1[e] : g.b0[e]);
         sc[j] = (cptr_f32)(uintptr_t)uni_ptr((SWIGLU && j == 1) ? g.s1[e] : g.s0[e]);
-        srow[j] = min((n0 + (SWIGLU ? 0 : 32 * wave)) >> 7, (N >> 7) - 1) * npair;
+        srow[j] = min((n0 + (SWIGLU ? 0 : 32 * wave)) >> 7, (N >> 7) - 1) * (K >> 7) + kfirst;
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -944,7 +962,7 @@ __device__ __forceinline__ void stream8x_tile(const GemmArgs& g, SBuf b0, SBuf b
         int pr = min(p_pipe, npair - 1) + prot;
         pr = pr >= npair ? pr - npair : pr;
         const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)bmat[i >> 1], 0, live, 0x00020000);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_u8)(buf.w + wave * 4096 + i * 1024), 16, w_voff[i], (uint32_t)(pr * 128), 0, 2);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_u8)(buf.w + wave * 4096 + i * 1024), 16, w_voff[i], (uint32_t)((pr + kfirst) * 128), 0, 2);
     };
     auto dma_t = [&](int hb_pipe, SBuf buf, int i) __attribute__((always_inline)) {
         const int live = uni(hb_pipe < 2 * npair ? -1 : 0);
@@ -953,7 +971,7 @@ __device__ __forceinline__ void stream8x_tile(const GemmArgs& g, SBuf b0, SBuf b
         pr = pr >= npair ? pr - npair : pr;
         const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)a_base, 0, live & a_records, 0x00020000);
         __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_u8)(buf.t + wave * 2048 + i * 1024), 16, t_voff[i],
-                                                 (uint32_t)(pr * 256 + (hb & 1) * 128), 0, 0);
+                                                 (uint32_t)((pr + kfirst) * 256 + (hb & 1) * 128), 0, 0);
     };
 
     const int frow = lane & 15, q = lane >> 4;
@@ -1055,7 +1073,9 @@ __device__ __forceinline__ void stream8x_tile(const GemmArgs& g, SBuf b0, SBuf b
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 const int col = n0 + 32 * wave + 16 * j + 4 * q;
-                if (col < N) *reinterpret_cast<u32x2*>(g.c + (size_t)r * N + col) = epilogue_pack<false>(acc[t][j], acc[t][j]);
+                if (col >= N) continue;
+                if (SPLIT) *reinterpret_cast<f32x4*>(ks.part + (size_t)(r - ks.row_base) * N + col) = acc[t][j];
+                else *reinterpret_cast<u32x2*>(g.c + (size_t)r * N + col) = epilogue_pack<false>(acc[t][j], acc[t][j]);
             }
         }
     }
@@ -1806,6 +1826,64 @@ __global__ __launch_bounds__(64) void grouped_gemm_thin_kernel(GemmPair pair_of)
     }
 }
 
+// ---- split kernel: the down projection of a dense fp8 MLP at few rows ----
+//
+// One MLP of few rows has hidden / 256 column tiles (DeepSeek-V3: 28) with a long k (18432), and a workgroup takes 0.8 to
+// 1.7 us per 128 k however few others run: 28 CUs worked while the rest waited.  Here a tile's k is cut into slices, one
+// workgroup each, so that tiles x slices fill the CUs once; the fp32 sums of the slices go to the workspace and
+// add_slices_kernel adds them, in order, and rounds once.  Rows past 128 are cut into tiles of equal height; all tiles of a
+// call run the same body, chosen by that height, so a row's bits do not depend on its place.  The M tiles of one piece of
+// the weights are neighbours on one XCD.
+// Measured (DeepSeek-V3's dense MLP, whole forward, us, one workgroup per tile -> this): 1 token 103 -> 79, 17: 171 -> 86,
+// 64: 203 -> 106, 128: 363 -> 174, 192: 521 -> 255, 256: 427 -> 285, 384: 471 -> 424, 512: 507 -> 441; of those the gate and up
+// products take 44, 56, 66, 113, 156, 193, 238 and 275.
+__global__ __launch_bounds__(512) void grouped_gemm_split_kernel(GemmArgs g, int n_rows, SplitPlan plan, float* part) {
+    __shared__ __attribute__((aligned(1024))) uint8_t lw0[S8_WBYTES];
+    __shared__ __attribute__((aligned(1024))) uint8_t lw1[S8_WBYTES];
+    __shared__ __attribute__((aligned(1024))) uint8_t lw2[S8_WBYTES];
+    __shared__ __attribute__((aligned(1024))) uint8_t lt0[128 * ROW_B];
+    __shared__ __attribute__((aligned(1024))) uint8_t lt1[128 * ROW_B];
+    __shared__ __attribute__((aligned(1024))) uint8_t lt2[128 * ROW_B];
+    const SBuf b0{lw0, lt0}, b1{lw1, lt1}, b2{lw2, lt2};
+    const int local = blockIdx.x >> 3;
+    const int piece = local / plan.m_tiles * 8 + (blockIdx.x & 7), m_tile = local % plan.m_tiles;
+    if (piece >= plan.slices * g.n_tiles_n) return;
+    const int slice = piece / g.n_tiles_n, n_tile = piece % g.n_tiles_n;
+    const int base = uni(g.offsets[0]), stop = min(uni(g.offsets[1]), base + n_rows);
+    const int r0 = base + m_tile * plan.rows, r1 = min(r0 + plan.rows, stop);
+    if (r0 >= r1) return;
+    const int first = slice * plan.blocks;
+    const KSlice ks{first, min(plan.blocks, (g.K >> 7) - first), base, part + (size_t)slice * n_rows * g.N};
+    const int groups = (r1 - r0 + 15) >> 4;
+    if (plan.rows <= 64) {
+        if (groups == 1) stream8_tile<1, false, true>(g, b0, b1, b2, 0, r0, r1, n_tile, ks);
+        else if (groups == 2) stream8_tile<2, false, true>(g, b0, b1, b2, 0, r0, r1, n_tile, ks);
+        else if (groups == 3) stream8_tile<3, false, true>(g, b0, b1, b2, 0, r0, r1, n_tile, ks);
+        else stream8_tile<4, false, true>(g, b0, b1, b2, 0, r0, r1, n_tile, ks);
+    } else {
+        if (groups <= 5) stream8x_tile<5, false, true>(g, b0, b1, b2, 0, r0, r1, n_tile, true, ks);
+        else if (groups == 6) stream8x_tile<6, false, true>(g, b0, b1, b2, 0, r0, r1, n_tile, true, ks);
+        else if (groups == 7) stream8x_tile<7, false, true>(g, b0, b1, b2, 0, r0, r1, n_tile, true, ks);
+        else stream8x_tile<8, false, true>(g, b0, b1, b2, 0, r0, r1, n_tile, true, ks);
+    }
+}
+
+// y = bf16(part[0] + part[1] + ...), 4 columns per thread
+__global__ __launch_bounds__(256) void add_slices_kernel(const float* __restrict__ part, const int32_t* __restrict__ offsets,
+                                                         uint16_t* __restrict__ y, int n_rows, int N, int slices) {
+    const int base = offsets[0], rows = min(offsets[1] - base, n_rows);
+    const size_t at = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4, stride = (size_t)n_rows * N;
+    if (rows <= 0 || at >= (size_t)rows * N) return;
+    f32x4 sum = *reinterpret_cast<const f32x4*>(part + at);
+#pragma unroll 4
+    for (int s = 1; s < slices; ++s) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(part + s * stride + at);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sum[i] += v[i];
+    }
+    *reinterpret_cast<u32x2*>(y + (size_t)base * N + at) = epilogue_pack<false>(sum, sum);
+}
+
 // lane id produced where it is used: the compiler cannot hoist it (and everything derived from it)
 // out of the tile loop and keep it in registers through the k loop
 __device__ __forceinline__ int fresh_lane() {
@@ -2206,11 +2284,42 @@ int launch_persistent(const GemmArgs& g, int n_rows, hipStream_t st) {
 // 4 GiB of gathered rows or more: only the register-staged body addresses them
 inline bool gather_fits(const GemmArgs& g) { return !g.row_map || g.a_bytes < (1ull << 32); }
 
+// The split kernel's plan, slices == 0 where it does not pay: as many slices as fill the CUs once, of 8 blocks or more (a
+// shorter k loop is mostly its own start), at most 16; and only where k is long: 32 blocks (4096), so that what the slices save
+// outweighs their sums' way through memory.  (A long k without two tiles' worth of idle CUs, from 513 rows of DeepSeek-V3:
+// the persistent kernel.)
+SplitPlan split_plan(int n_rows, int K, int n_tiles_n) {
+    const int nblk = K / 128;
+    int m = (n_rows + 127) / 128;
+    const int rows = m <= 1 ? n_rows : ((n_rows + m - 1) / m + 15) / 16 * 16;
+    if (nblk < 32 || n_rows < 1 || (long)m * n_tiles_n * 2 > cu_count()) return SplitPlan{};
+    m = (n_rows + rows - 1) / rows;
+    int s = cu_count() / (m * n_tiles_n);
+    s = s < nblk / 8 ? s : nblk / 8;
+    s = s < 16 ? s : 16;
+    const int blocks = (nblk + s - 1) / s;
+    return SplitPlan{m, rows, (nblk + blocks - 1) / blocks, blocks};
+}
+
+int launch_split(const GemmArgs& g, int n_rows, const SplitPlan& plan, float* part, hipStream_t st) {
+    const int pieces = plan.slices * g.n_tiles_n;
+    hipLaunchKernelGGL(grouped_gemm_split_kernel, dim3((pieces + 7) / 8 * 8 * plan.m_tiles), dim3(512), 0, st, g, n_rows, plan, part);
+    hipLaunchKernelGGL(add_slices_kernel, dim3((unsigned)(((size_t)n_rows * g.N / 4 + 255) / 256)), dim3(256), 0, st, part, g.offsets, g.c,
+                       n_rows, g.N, plan.slices);
+    MOE_HIP_CHECK(hipGetLastError());
+    return MOE_OK;
+}
+
 // max_rows: no expert has more rows (callers that do not know pass n_rows)
 template <bool SWIGLU, bool W8>
-int launch_mt(const GemmArgs& g0, int n_rows, int max_rows, hipStream_t st) {
+int launch_mt(const GemmArgs& g0, int n_rows, int max_rows, void* workspace, size_t workspace_bytes, hipStream_t st) {
     GemmArgs g = g0;
     const long mean = g.E > 0 ? (long)n_rows / g.E : 0;
+    if constexpr (W8 && !SWIGLU) {
+        const SplitPlan plan = g.E == 1 && workspace ? split_plan(n_rows, g.K, g.n_tiles_n) : SplitPlan{};
+        if (plan.slices > 1 && workspace_bytes >= (size_t)plan.slices * n_rows * g.N * 4)
+            return launch_split(g, n_rows, plan, static_cast<float*>(workspace), st);
+    }
     if (max_rows <= 16 && gather_fits(g)) return launch_thin<SWIGLU, W8>(g, n_rows, nullptr, st);
     // the persistent kernel needs an even number of k-stages for its hand-over (fp8 sizes always have
     // one), keeps per-expert tables for up to 512 experts and addresses gathered rows with 32-bit offsets
@@ -2319,8 +2428,9 @@ int grouped_swiglu(const moe_mlp_group& m, int32_t hidden, int32_t phases, void*
     int rc = check_group(m, hidden, W8, who);
     if (rc != MOE_OK || m.n_rows == 0) return rc;
     hipStream_t st = as_stream(stream);
-    if (phases & MOE_PHASE_GATE_UP) rc = launch_mt<true, W8>(gate_up_args(m, hidden), m.n_rows, row_bound(m), st);
-    if (rc == MOE_OK && (phases & MOE_PHASE_DOWN)) rc = launch_mt<false, W8>(down_args(m, hidden), m.n_rows, row_bound(m), st);
+    if (phases & MOE_PHASE_GATE_UP) rc = launch_mt<true, W8>(gate_up_args(m, hidden), m.n_rows, row_bound(m), nullptr, 0, st);
+    if (rc == MOE_OK && (phases & MOE_PHASE_DOWN)) 
+        rc = launch_mt<false, W8>(down_args(m, hidden), m.n_rows, row_bound(m), m.workspace, m.workspace_bytes, st);
     return rc;
 }
 
@@ -2375,7 +2485,7 @@ extern "C" int moe_grouped_swiglu_bf16(const void* x, int32_t x_rows, const int3
                                        const void* const* w_up, const void* const* w_down, const int32_t* offsets,
                                        int32_t n_rows, int32_t n_experts, int32_t hidden, int32_t inter, void* act,
                                        void* y, int32_t phases, void*, size_t, void* stream) {
-    const moe_mlp_group m{x, x_rows, n_rows, row_map, w_gate, w_up, w_down, nullptr, nullptr, nullptr, offsets, n_experts, inter, 0, 0, act, y};
+    const moe_mlp_group m{x, x_rows, n_rows, row_map, w_gate, w_up, w_down, nullptr, nullptr, nullptr, offsets, n_experts, inter, 0, 0, act, y, nullptr, 0};
     return moe::grouped_swiglu<false>(m, hidden, phases, stream, "moe_grouped_swiglu_bf16");
 }
 
@@ -2385,7 +2495,7 @@ extern "C" int moe_grouped_swiglu_w8a16(const void* x, int32_t x_rows, const int
                                         const float* const* s_down, const int32_t* offsets, int32_t n_rows,
                                         int32_t n_experts, int32_t hidden, int32_t inter, void* act, void* y,
                                         int32_t phases, void*, size_t, void* stream) {
-    const moe_mlp_group m{x, x_rows, n_rows, row_map, w_gate, w_up, w_down, s_gate, s_up, s_down, offsets, n_experts, inter, 0, 0, act, y};
+    const moe_mlp_group m{x, x_rows, n_rows, row_map, w_gate, w_up, w_down, s_gate, s_up, s_down, offsets, n_experts, inter, 0, 0, act, y, nullptr, 0};
     return moe::grouped_swiglu<true>(m, hidden, phases, stream, "moe_grouped_swiglu_w8a16");
 }
 
@@ -2398,6 +2508,13 @@ extern "C" int moe_grouped_swiglu_joint(const moe_mlp_group* routed, const moe_m
                    : grouped_swiglu<false>(*routed, hidden, phases, stream, "moe_grouped_swiglu_joint");
     return fp8 ? grouped_swiglu_joint<true>(*routed, *shared, hidden, phases, stream)
                : grouped_swiglu_joint<false>(*routed, *shared, hidden, phases, stream);
+}
+
+extern "C" size_t moe_mlp_workspace_bytes(const moe_mlp_group* m, int32_t hidden) {
+    using namespace moe;
+    if (m == nullptr || !m->fp8 || m->n_experts != 1 || m->n_rows < 1 || hidden < 1) return 0;
+    const SplitPlan plan = split_plan(m->n_rows, m->inter, (hidden + 255) / 256);
+    return plan.slices > 1 ? (size_t)plan.slices * m->n_rows * hidden * 4 : 0;
 }
 
 extern "C" int moe_shared_joins(const moe_mlp_group* routed, const moe_mlp_group* shared, int32_t hidden) {

@@ -343,6 +343,17 @@ def mlp_group(x: torch.Tensor, row_map, ptrs: ExpertPointers, offsets: torch.Ten
     return m, act, y
 
 
+def grouped_swiglu_one(x: torch.Tensor, ptrs: ExpertPointers, offsets: torch.Tensor, n_rows: int) -> torch.Tensor:
+    """One dense MLP on all n_rows rows of x, with the scratch that its down projection asks for."""
+    m, _, y = mlp_group(x, None, ptrs, offsets, n_rows, n_rows)
+    need = N.lib().moe_mlp_workspace_bytes(ctypes.byref(m), ptrs.hidden)
+    if need:
+        ws = torch.empty(need, dtype=torch.uint8, device=x.device)
+        m.workspace, m.workspace_bytes = ws.data_ptr(), need
+    grouped_swiglu_joint(m, None, ptrs.hidden, ptrs.fp8)
+    return y
+
+
 def shared_joins(routed, shared, hidden: int) -> bool:
     """Whether grouped_swiglu_joint runs the shared expert inside the routed experts' launches."""
     return bool(N.lib().moe_shared_joins(ctypes.byref(routed), ctypes.byref(shared), hidden))

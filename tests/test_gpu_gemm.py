@@ -833,3 +833,42 @@ def test_shared_expert_in_the_routed_launches(fp8, n, shared_inter):
     else:
         a, b = sh1.float(), sh2.float()
         assert (a - b).abs().max().item() <= TOL * b.abs().max().item()
+
+
+@pytest.mark.parametrize("I", [4096, 4224, 18432])      # 32 blocks of 128 k (the rule's least), 33 (a short last slice), DeepSeek-V3's
+@pytest.mark.parametrize("h", [128, 768])               # half a column tile; three
+def test_dense_fp8_down_projection_in_slices_of_k(h, I):
+    """The down projection of one fp8 MLP with its scratch, at the edges of its row tiles: against float64 on the dequantised
+    weights, nothing written past the scratch, and a row's bits independent of its place."""
+    import ctypes
+    from moe_gen_amd import _native as N, ops
+    from moe_gen_amd.synthetic import quantize_fp8_block128
+    g = torch.Generator(device="cuda").manual_seed(h + I)
+    q, sc = quantize_fp8_block128(torch.randn(h, I, generator=g, device="cuda") * 0.02)
+    qi = torch.zeros(I, h, device="cuda").to(torch.float8_e4m3fn)      # (gate and up are not run)
+    si = torch.ones(I // 128, h // 128, device="cuda")
+    ptrs = ops.expert_pointers([qi], [qi], [q], [si], [si], [sc])
+    wd = q.double() * sc.double().repeat_interleave(128, 0).repeat_interleave(128, 1)
+    for n in (1, 16, 17, 63, 64, 65, 80, 81, 128, 129, 160, 161, 256, 257, 384, 512, 513):
+        print(f"slices of k h={h} I={I} n={n}", flush=True)
+        act = torch.randn(n, I, generator=g, device="cuda").to(torch.bfloat16)
+        x = torch.zeros(n, h, dtype=torch.bfloat16, device="cuda")
+        off = torch.tensor([0, n], dtype=torch.int32, device="cuda")
+
+        def down(a, need):
+            m, _, y = ops.mlp_group(x, None, ptrs, off, n, n, act=a)
+            ws = torch.full((need // 4 + 64,), 7.0, device="cuda")
+            m.workspace, m.workspace_bytes = (ws.data_ptr(), need) if need else (None, 0)
+            ops.grouped_swiglu_joint(m, None, h, True, ops.PHASE_DOWN)
+            assert torch.equal(ws[need // 4:], torch.full((64,), 7.0, device="cuda"))
+            return y
+        m, _, _ = ops.mlp_group(x, None, ptrs, off, n, n, act=act)
+        need = N.lib().moe_mlp_workspace_bytes(ctypes.byref(m), h)
+        assert need > 0 and need % (4 * n * h) == 0
+        y = down(act, need)
+        ref = act.double() @ wd.t()
+        # weights (above 64 rows) and result are each rounded to bf16: relative 2^-9 at most, independent per element
+        for out in (y, down(act, 0)):
+            assert (out.double() - ref).norm() <= 2.0 ** -8 * ref.norm()
+        perm = torch.randperm(n, generator=torch.Generator().manual_seed(n)).cuda()
+        assert torch.equal(down(act[perm].contiguous(), need), y[perm])
