@@ -170,13 +170,12 @@ int moe_dispatch_static(const int32_t* topk_idx, int32_t n_tokens, int32_t top_k
  * one per CU, take whole rounds of tiles; a last, partial round is cut into 128-row halves and runs with the first
  * kind when that shortens the two launches (alone: if it is at most half the CUs' worth of tiles).  Below a mean of 128 rows per expert (n_rows / E), with K not a multiple of
  * 128, with more than 512 experts or with 4 GiB or more of gathered x, the one-workgroup-per-tile kernel serves the
- * call alone (larger experts cut into 128-row tiles).  An output row's bits depend on the row and its expert's
- * weights, never on the row's place among its expert's rows, on any expert's count or on the kernel that computes
- * it.  With bf16 weights that holds across calls too.  With fp8 weights a call that the one-workgroup-per-tile kernel
- * serves alone adds a row's products in another order than a call that launches both kernels (other starting stages
- * of its k loops), and its experts of up to 64 rows are multiplied by the fp8 values as they are, the block scale being
- * applied to the fp32 sum of each 128 k instead of to the weight before it is rounded to bf16: a row may then differ
- * between the two kinds of call by the rounding of the weights (2^-9).
+ * call alone (larger experts cut into 128-row tiles).  With bf16 weights an output row's bits depend on the row and its
+ * expert's weights alone, never on the row's place among its expert's rows, on any expert's count, on the kernel that
+ * computes it or on the call.  With fp8 weights that holds inside a call that launches both kernels, and two things
+ * change the order in which a row's products are added, and with it the last bit: a call that the
+ * one-workgroup-per-tile kernel serves alone starts its k loops at other stages, and there an expert of up to 64 rows
+ * adds the products of a stage in another order than one of more.
  * Calls in which no expert has more than 16 rows run on a kernel of one wave per 32 weight rows.
  */
 enum { MOE_PHASE_GATE_UP = 1, MOE_PHASE_DOWN = 2, MOE_PHASE_BOTH = 3 };
@@ -191,7 +190,7 @@ int moe_grouped_swiglu_bf16(const void* x, int32_t x_rows, const int32_t* row_ma
 /*
  * W8A16 variant: weights are fp8 e4m3fn with one fp32 scale per 128x128 block;
  * each weight element is dequantised in registers as bf16(f32(q) * scale)
- * (deepseek_v3_dequantization, Wrapper.py:109-138) before it reaches the MFMA (few rows: see above).
+ * (deepseek_v3_dequantization, Wrapper.py:109-138) before it reaches the MFMA.
  *   s_gate/s_up  device arrays of E pointers to fp32 [ceil(I/128), ceil(h/128)]
  *   s_down       device array  of E pointers to fp32 [ceil(h/128), ceil(I/128)]
  * Requires h % 128 == 0 and I % 128 == 0.

@@ -183,19 +183,6 @@ __device__ __forceinline__ u32x4 dequant8(uint32_t q0, uint32_t q1, float sc) {
                  pack_bf16(c2[0] * sc, c2[1] * sc), pack_bf16(c3[0] * sc, c3[1] * sc)};
 }
 
-// 8 fp8 weights (two dwords) -> the same values as bf16 (exact), one instruction per pair.  The streamers for few rows
-// multiply them unscaled and apply the block scale to the fp32 sum of each 128 k: a quarter of dequant8's vector
-// instructions, and a weight keeps the bits that bf16(f32(q) * s) rounds away.
-// Relative 2-norm error of a DeepSeek-V3 layer (1 ... 64 tokens) and dense MLP (1, 64) against float64 on q * s: 5.3e-3 and 4.9e-3
-// with the weights rounded to bf16, 4.3e-3 and 3.9e-3 so (against float64 on bf16(f32(q) * s): 4.4e-3 -> 5.2e-3).
-__device__ __forceinline__ bf16x8 widen8(uint32_t q0, uint32_t q1) {
-    const u32x4 v = {__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(q0, 1.0f, false)),
-                     __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(q0, 1.0f, true)),
-                     __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(q1, 1.0f, false)),
-                     __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(q1, 1.0f, true))};
-    return __builtin_bit_cast(bf16x8, v);
-}
-
 // Epilogue values of one lane for one pair of accumulators: 4 consecutive output columns of one row.
 // SWIGLU: act = bf16(bf16(silu(bf16(g))) * bf16(u)), the rounding points of the reference's bf16
 // Linear / SiLU / mul modules (silu through the hardware exp and reciprocal); else bf16(acc).
@@ -812,17 +799,14 @@ __device__ __forceinline__ void stream8_tile(const GemmArgs& g, SBuf buf0, SBuf 
         asm volatile("" ::: "memory");
         scales(p + 1, sset ^ 1);
         __builtin_amdgcn_sched_barrier(0);
-        f32x4 part[TG][2];                      // the block's sums of unscaled weights
-#pragma unroll
-        for (int t = 0; t < TG; ++t) { part[t][0] = f32x4{0}; part[t][1] = f32x4{0}; }
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             bf16x8 wa[2][2];
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 const u32x4 raw = *reinterpret_cast<const u32x4*>(rd.w + w_rd + j * 2048 + (((4 * h + fq) ^ wkey) << 4));
-                wa[j][0] = widen8(raw[0], raw[1]);
-                wa[j][1] = widen8(raw[2], raw[3]);
+                wa[j][0] = __builtin_bit_cast(bf16x8, dequant8(raw[0], raw[1], rsc[sset][j]));
+                wa[j][1] = __builtin_bit_cast(bf16x8, dequant8(raw[2], raw[3], rsc[sset][j]));
             }
 #pragma unroll
             for (int s2 = 0; s2 < 2; ++s2) {
@@ -830,8 +814,8 @@ __device__ __forceinline__ void stream8_tile(const GemmArgs& g, SBuf buf0, SBuf 
 #pragma unroll
                 for (int t = 0; t < TG; ++t) {
                     const bf16x8 tf = *reinterpret_cast<const bf16x8*>(rd.t + t_rd + t * 16 * 256 + coff);
-                    part[t][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[0][s2], tf, part[t][0], 0, 0, 0);
-                    part[t][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[1][s2], tf, part[t][1], 0, 0, 0);
+                    acc[t][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[0][s2], tf, acc[t][0], 0, 0, 0);
+                    acc[t][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[1][s2], tf, acc[t][1], 0, 0, 0);
                 }
                 // the refill of the freed buffer goes out between the four groups of matrix instructions (2, 2, 1, 1
                 // DMA instructions): a wave that issues all six first stands in the memory pipeline's queue while its
@@ -843,12 +827,6 @@ __device__ __forceinline__ void stream8_tile(const GemmArgs& g, SBuf buf0, SBuf 
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
-#pragma unroll
-        for (int t = 0; t < TG; ++t)
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) acc[t][j][i] = __builtin_fmaf(part[t][j][i], rsc[sset][j], acc[t][j][i]);
     };
     scales(0, 0);
     dma(0, buf0);
@@ -1783,7 +1761,8 @@ __global__ __launch_bounds__(64) void grouped_gemm_thin_kernel(GemmPair pair_of)
             dma(k + NB - 1, buf == 0 ? NB - 1 : buf - 1);
             const uint8_t* b = lds + buf * SB;
             if (W8) {
-                f32x4 part[2] = {f32x4{0}, f32x4{0}};
+                const float c[2] = {__builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v0), k & 63)),
+                                    __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v1), k & 63))};
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
                     u32x4 raw[2];
@@ -1794,15 +1773,9 @@ __global__ __launch_bounds__(64) void grouped_gemm_thin_kernel(GemmPair pair_of)
                         const bf16x8 tf = *reinterpret_cast<const bf16x8*>(b + t_rd + (((8 * h + 2 * fq + s2) ^ tkey) << 4));
 #pragma unroll
                         for (int j = 0; j < 2; ++j)
-                            part[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(widen8(raw[j][2 * s2], raw[j][2 * s2 + 1]), tf, part[j], 0, 0, 0);
+                            acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                                __builtin_bit_cast(bf16x8, dequant8(raw[j][2 * s2], raw[j][2 * s2 + 1], c[j])), tf, acc[j], 0, 0, 0);
                     }
-                }
-                const float c0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v0), k & 63));
-                const float c1 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v1), k & 63));
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    acc[0][i] = __builtin_fmaf(part[0][i], c0, acc[0][i]);
-                    acc[1][i] = __builtin_fmaf(part[1][i], c1, acc[1][i]);
                 }
             } else {
 #pragma unroll

@@ -867,8 +867,59 @@ def test_dense_fp8_down_projection_in_slices_of_k(h, I):
         assert need > 0 and need % (4 * n * h) == 0
         y = down(act, need)
         ref = act.double() @ wd.t()
-        # weights (above 64 rows) and result are each rounded to bf16: relative 2^-9 at most, independent per element
+        # weights and result are each rounded to bf16: relative 2^-9 at most, independent per element
         for out in (y, down(act, 0)):
             assert (out.double() - ref).norm() <= 2.0 ** -8 * ref.norm()
         perm = torch.randperm(n, generator=torch.Generator().manual_seed(n)).cuda()
         assert torch.equal(down(act[perm].contiguous(), need), y[perm])
+
+
+@pytest.mark.parametrize("n,inter", [(1, 256), (16, 256), (17, 256), (64, 256), (65, 256), (128, 256), (192, 256), (193, 256), (256, 256),
+                                     (1, 4096), (16, 4096), (64, 4096), (65, 4096), (128, 4096)])
+def test_fp8_weights_are_dequantised_to_bf16_at_every_row_count(n, inter):
+    """A weight is bf16(f32(q) * s) in every kernel (one wave per 32 weight rows, the streamers, the persistent kernel, slices
+    of k with scratch from 4096 on), over all finite byte values.  A token row takes the difference of two neighbouring
+    codes: both products and their sum are exact in fp32, so the down projection's result is pinned to the bit, and the
+    rounding of the two weights is 3 % of it and more.  The up projection is read through a gate of exactly 1: one bf16
+    step for silu by the hardware exponential."""
+    import ctypes
+    from moe_gen_amd import _native as N, ops
+    print(f"fp8 rounding n={n} inter={inter}", flush=True)
+    h = 384
+    codes = torch.tensor([c for c in range(256) if c & 0x7f != 0x7f], dtype=torch.uint8)
+    g = torch.Generator().manual_seed(n + inter)
+
+    def weight(rows, cols):
+        i = torch.arange(cols).unsqueeze(0) + 37 * torch.arange(rows).unsqueeze(1)
+        q = codes[i % len(codes)].view(torch.float8_e4m3fn)
+        s = 0.01 + 0.01 * torch.rand(-(-rows // 128), -(-cols // 128), generator=g)
+        w = (q.float() * s.repeat_interleave(128, 0)[:rows].repeat_interleave(128, 1)[:, :cols]).to(torch.bfloat16).float()
+        return q.cuda(), s.cuda(), w
+
+    def rows_of(width):                                  # (+1 at an even k, -1 behind it)
+        k = torch.randint(0, width // 2, (n,), generator=g) * 2
+        a = torch.zeros(n, width)
+        a[torch.arange(n), k], a[torch.arange(n), k + 1] = 1.0, -1.0
+        return k, a.to(torch.bfloat16).cuda()
+
+    up, down = weight(inter, h), weight(h, inter)
+    one = torch.zeros(inter, h)
+    one[:, ::2] = 1.0
+    ptrs = ops.expert_pointers([one.to(torch.float8_e4m3fn).cuda()], [up[0]], [down[0]],
+                               [torch.ones(inter // 128, h // 128).cuda()], [up[1]], [down[1]])
+    off = torch.tensor([0, n], dtype=torch.int32, device="cuda")
+    kx, x = rows_of(h)
+    m, act, _ = ops.mlp_group(x, None, ptrs, off, n, n)
+    ops.grouped_swiglu_joint(m, None, h, True, ops.PHASE_GATE_UP)
+    u = (up[2][:, kx] - up[2][:, kx + 1]).t().to(torch.bfloat16)
+    want = torch.nn.functional.silu(torch.ones((), dtype=torch.bfloat16)) * u
+    assert ((act.cpu().float() - want.float()).abs() <= 2.0 ** -7 * want.float().abs()).all()
+
+    ka, a = rows_of(inter)
+    m, _, y = ops.mlp_group(x, None, ptrs, off, n, n, act=a)
+    need = N.lib().moe_mlp_workspace_bytes(ctypes.byref(m), h)
+    assert (need > 0) == (inter >= 4096)
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    m.workspace, m.workspace_bytes = (ws.data_ptr(), need) if need else (None, 0)
+    ops.grouped_swiglu_joint(m, None, h, True, ops.PHASE_DOWN)
+    assert torch.equal(y.cpu().float(), (down[2][:, ka] - down[2][:, ka + 1]).t().to(torch.bfloat16).float())
