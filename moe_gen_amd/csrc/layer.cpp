@@ -104,11 +104,13 @@ extern "C" int moe_layer_forward(const moe_layer_args* args, void* stream) {
     routed.x = x; routed.x_rows = n; routed.n_rows = n * k; routed.row_map = d.row_map; routed.offsets = d.offsets;
     routed.max_rows = n;
     routed.act = ws + l.act; routed.y = ws + l.y;
+    routed.workspace = nullptr; routed.workspace_bytes = 0;       // (the caller's fields may hold anything)
     const void* y_shared = nullptr;
     if (a.shared) {
         moe_mlp_group shared = *a.shared;
         shared.x = x; shared.x_rows = shared.n_rows = shared.max_rows = n; shared.row_map = nullptr; shared.offsets = d.one_group;
         shared.act = ws + l.act_shared; shared.y = ws + l.y_shared;
+        shared.workspace = nullptr; shared.workspace_bytes = 0;
         y_shared = shared.y;
         if (a.join_shared && shared.fp8 == routed.fp8) {
             rc = moe_grouped_swiglu_joint(&routed, &shared, h, routed.fp8, MOE_PHASE_BOTH, stream);

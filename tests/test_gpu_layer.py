@@ -244,3 +244,22 @@ def test_dense_mlp_sees_replaced_weights_and_a_copied_block_its_own(fp8):
         for lin in (ex.gate_proj, ex.up_proj, ex.down_proj):
             lin.weight.data.view(torch.uint8).zero_()
     assert torch.equal(twin(x), out)
+
+
+@pytest.mark.parametrize("E", [1, 8])
+def test_layer_call_reads_only_the_weights_of_its_groups(E):
+    """The other fields of a layer call's groups may hold anything.  The sizes are ones at which an fp8 MLP with a
+    workspace of its own cuts its down projection into slices of k (one expert, 4096 inner columns, few rows): a buffer
+    offered in those fields stays as it was, and the output is that of a call without one."""
+    from moe_gen_amd import synthetic
+    w = synthetic.WORKLOADS["deepseek_v2_lite"].scaled(n=16, h=512, I=4096, S=1, seq=16, E=E, k=1, fp8=True)
+    blk = synthetic.build_block(w, device="cuda", gen_device="cpu")
+    blk.join_shared = False
+    x = synthetic.hidden_states(w, "cpu").cuda()
+    print(f"layer call with a foreign workspace E={E}", flush=True)
+    want = blk(x)
+    sentinel = torch.full((64 * 2 ** 20,), 7, dtype=torch.uint8, device="cuda")
+    for tables in (blk._moe_cache["routed"]["ptrs"], blk._moe_cache["shared"]["ptrs"]):
+        tables.weights.workspace, tables.weights.workspace_bytes = sentinel.data_ptr(), sentinel.numel()
+    assert torch.equal(blk(x), want)
+    assert (sentinel == 7).all()
