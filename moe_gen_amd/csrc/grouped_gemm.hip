@@ -2391,7 +2391,7 @@ int row_bound(const moe_mlp_group& m) { return m.max_rows > 0 && m.max_rows < m.
 // call is one that the one-workgroup-per-tile kernel (or the thin one) serves alone.  DeepSeek-V3 up to 1024 tokens: the
 // step gains 2-5 %, from 2048 tokens on a launch pair of its own, with 256-row tiles, is the faster by 0.6 %.
 bool joins(const moe_mlp_group& routed, const moe_mlp_group& shared, int32_t hidden) {
-    if (routed.n_rows == 0 || shared.n_rows == 0 || shared.n_experts != 1) return false;
+    if (routed.n_rows < 1 || shared.n_rows < 1 || routed.n_experts < 1 || shared.n_experts != 1 || hidden < 1) return false;
     if (routed.n_rows / routed.n_experts >= 128) return false;
     if (routed.row_map && (size_t)routed.x_rows * (size_t)hidden * 2 >= (1ull << 32)) return false;
     return (long)(shared.n_rows / 256 + 1) * ((shared.inter + 127) / 128) * 8 < 3L * cu_count();
@@ -2412,14 +2412,14 @@ int grouped_swiglu(const moe_mlp_group& m, int32_t hidden, int32_t phases, void*
 template <bool W8>
 int grouped_swiglu_joint(const moe_mlp_group& r, const moe_mlp_group& s, int32_t hidden, int32_t phases, void* stream) {
     const char* who = "moe_grouped_swiglu_joint";
-    if (!joins(r, s, hidden)) {
-        const int rc = grouped_swiglu<W8>(r, hidden, phases, stream, who);
-        return rc != MOE_OK ? rc : grouped_swiglu<W8>(s, hidden, phases, stream, who);
-    }
     MOE_REQUIRE(phases >= MOE_PHASE_GATE_UP && phases <= MOE_PHASE_BOTH, "%s: bad phases %d", who, phases);
     int rc = check_group(r, hidden, W8, who);
     if (rc == MOE_OK) rc = check_group(s, hidden, W8, who);
     if (rc != MOE_OK) return rc;
+    if (!joins(r, s, hidden)) {
+        rc = grouped_swiglu<W8>(r, hidden, phases, stream, who);
+        return rc != MOE_OK ? rc : grouped_swiglu<W8>(s, hidden, phases, stream, who);
+    }
     hipStream_t st = as_stream(stream);
     if (phases & MOE_PHASE_GATE_UP)
         rc = launch_joint<true, W8>(gate_up_args(r, hidden), r.n_rows, row_bound(r), gate_up_args(s, hidden), s.n_rows, st);

@@ -52,3 +52,26 @@ def test_argument_validation_needs_no_gpu():
     assert lib.moe_grouped_swiglu_bf16(1, 8, None, 1, 1, 1, 1, 8, 2, 100, 64, 1, 1, 3, None, 0, None) == -1
     assert "hidden" in N.last_error()
     assert lib.moe_dispatch(1, 4, 2, 300, 1, 1, 1, 1, None, None, 0, None, None, 0, None) == -1
+
+
+def test_joint_calls_check_their_groups_first():
+    """No expert, or fewer than no rows: an error code (a division by zero would end the process), and a bad second group
+    is refused before the first one is launched.  In a process of its own, which reports how it ended."""
+    import subprocess
+    import sys
+    code = """
+import ctypes
+from moe_gen_amd import _native as N
+lib = N.lib()
+group = lambda rows, E, inter: N.MlpGroup(1, 8, rows, None, 1, 1, 1, 1, 1, 1, 1, E, inter, 0, 0, 1, 1, None, 0)
+good, none = group(8, 2, 64), group(8, 1, 64)
+for bad in (group(8, 0, 64), group(-1, 2, 64), group(8, -1, 64)):
+    assert lib.moe_shared_joins(ctypes.byref(bad), ctypes.byref(none), 64) == 0
+    for fp8 in (0, 1):
+        assert lib.moe_grouped_swiglu_joint(ctypes.byref(bad), ctypes.byref(none), 64, fp8, 3, None) == -1, N.last_error()
+assert lib.moe_grouped_swiglu_joint(ctypes.byref(good), ctypes.byref(group(8, 1, 65)), 64, 0, 3, None) == -1 and "intermediate" in N.last_error()
+assert lib.moe_grouped_swiglu_joint(ctypes.byref(good), ctypes.byref(none), 64, 0, 9, None) == -1 and "phases" in N.last_error()
+"""
+    r = subprocess.run([sys.executable, "-c", code], cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
+                       capture_output=True, text=True)
+    assert r.returncode == 0, (r.returncode, r.stderr)
