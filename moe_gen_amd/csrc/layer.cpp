@@ -77,15 +77,14 @@ extern "C" int moe_layer_forward(const moe_layer_args* args, void* stream) {
                                     nullptr, 0, nullptr, nullptr, 0, stream);
     MOE_REQUIRE(a.x && a.out, "%s: NULL pointer argument", who);
     const hipStream_t st = as_stream(stream);
+    rc = check_router(a.x, a.w_gate, &p, a.topk_idx, a.topk_w);
+    if (rc != MOE_OK) return rc;
     const void* x = a.x;
     if (a.norm_weight) {
         rc = moe_rmsnorm(a.x, a.norm_weight, a.norm_eps, n, h, ws + l.x_norm, stream);
         if (rc != MOE_OK) return rc;
         x = ws + l.x_norm;
     }
-    rc = check_router(x, a.w_gate, &p, a.topk_idx, a.topk_w);
-    if (rc != MOE_OK) return rc;
-
     float* logits = reinterpret_cast<float*>(ws + l.logits);
     auto ints = [&](size_t off) { return reinterpret_cast<int32_t*>(ws + off); };
     const DispatchOut d{a.counts, ints(l.offsets), ints(l.perm), ints(l.pos), ints(l.row_map), a.shared ? ints(l.one_group) : nullptr};

@@ -602,9 +602,10 @@ extern "C" int moe_router_rmsnorm(const void* x, const void* norm_weight, float 
     MOE_REQUIRE(norm_weight && x_norm, "moe_router_rmsnorm: NULL norm weight or output");
     MOE_REQUIRE(x_norm != x, "moe_router_rmsnorm: x_norm must not alias x (rows are read twice)");
     MOE_REQUIRE(eps >= 0.0f, "moe_router_rmsnorm: eps %g < 0", (double)eps);
+    int rc = check_router(x, w_gate, params, topk_idx, topk_w);       // (a refused call leaves x_norm as it was)
+    if (rc != MOE_OK) return rc;
     // The norm as a kernel of its own: the logit engine takes its operands by DMA and has no place to normalise them.
-    MOE_REQUIRE(params != nullptr, "moe_router_rmsnorm: params is NULL");
-    const int rc = moe_rmsnorm(x, norm_weight, eps, params->n_tokens, params->hidden, x_norm, stream);
+    rc = moe_rmsnorm(x, norm_weight, eps, params->n_tokens, params->hidden, x_norm, stream);
     if (rc != MOE_OK) return rc;
     return route(x_norm, w_gate, bias, params, topk_idx, topk_w, logits_out, stream);
 }

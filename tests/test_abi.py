@@ -48,6 +48,8 @@ def test_argument_validation_needs_no_gpu():
     p = N.RouterParams(4, 16, 8, 2, 1, 1, 7, 0, 0, 1, 0, 0, 1e-20, 1.0)       # unknown scoring function
     assert lib.moe_router(1, 1, None, ctypes.byref(p), 1, 1, None, None) == -1
     assert "scoring" in N.last_error()
+    assert lib.moe_router_rmsnorm(1, 1, 1e-6, 1, None, ctypes.byref(p), 2, 1, 1, None, None) == -1     # (before the norm is launched)
+    assert "scoring" in N.last_error()
     assert lib.moe_combine(1, 1, None, 1, None, 4, 99, 64, 0, 1, None) == -1 and "top_k" in N.last_error()
     assert lib.moe_grouped_swiglu_bf16(1, 8, None, 1, 1, 1, 1, 8, 2, 100, 64, 1, 1, 3, None, 0, None) == -1
     assert "hidden" in N.last_error()
