@@ -178,7 +178,7 @@ def expert_pointers(gates, ups, downs, s_gates=None, s_ups=None, s_downs=None, d
     want = torch.float8_e4m3fn if fp8 else torch.bfloat16
     cols = [("gate weight", gates, want, (I, h)), ("up weight", ups, want, (I, h)), ("down weight", downs, want, (h, I))]
     if fp8:
-        if s_gates is None or s_ups is None or s_downs is None:
+        if any(ts is None or any(t is None for t in ts) for ts in (s_gates, s_ups, s_downs)):
             raise ValueError("fp8 expert weights need their *_scale_inv block scales")
         bi, bh = -(-I // 128), -(-h // 128)
         cols += [("gate scale", s_gates, torch.float32, (bi, bh)), ("up scale", s_ups, torch.float32, (bi, bh)),

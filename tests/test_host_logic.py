@@ -311,3 +311,41 @@ def test_layer_with_resident_and_engine_backed_experts():
         for ex in experts:
             ex.get_weights = False
         block.staged_experts_forward(experts, launch, counts)
+
+
+@pytest.mark.parametrize("form", ["parameter", "buffer", "attribute", "own_dict", "wrapped"])
+def test_block_scales_are_found_wherever_a_module_keeps_them(form):
+    """weight_scale_inv as a parameter, a registered buffer or a plain attribute of the Linear, and weight_dequant_scale on
+    the MLP itself or on a wrapper around it; a table of tensors without scales says what is missing."""
+    from moe_gen_amd.block import SwiGLUMLP, _tensors_of
+    mlp = SwiGLUMLP(128, 256)
+    scales = {}
+    for i, name in enumerate(mlp.names):
+        lin = getattr(mlp, name)
+        lin.weight = torch.nn.Parameter(torch.zeros(lin.weight.shape).to(torch.float8_e4m3fn), requires_grad=False)
+        s = torch.full((-(-lin.weight.shape[0] // 128), -(-lin.weight.shape[1] // 128)), 2.0 + i)
+        scales[name + ".weight_scale_inv"] = s
+        if form == "parameter":
+            lin.weight_scale_inv = torch.nn.Parameter(s, requires_grad=False)
+        elif form == "buffer":
+            lin.register_buffer("weight_scale_inv", s)
+        elif form == "attribute":
+            lin.weight_scale_inv = s
+    expert = mlp
+    if form == "own_dict":
+        mlp.weight_dequant_scale = scales
+    elif form == "wrapped":
+        class Wrapper(torch.nn.Module):
+            def __init__(self, module):
+                super().__init__()
+                self.module, self.weight_dequant_scale = module, scales
+        expert = Wrapper(mlp)
+    t = _tensors_of(expert)
+    assert [x.data_ptr() for x in t[:3]] == [getattr(mlp, n).weight.data_ptr() for n in mlp.names]
+    assert [float(x[0, 0]) for x in t[3:]] == [2.0, 3.0, 4.0]
+
+
+def test_missing_block_scales_are_named():
+    q = torch.zeros(128, 128).to(torch.float8_e4m3fn)
+    with pytest.raises(ValueError, match="block scales"):
+        ops.expert_pointers([q], [q], [q], [None], [None], [None])
