@@ -407,13 +407,6 @@ def _engine_experts(block, timer, tag, experts, a_rows, row_map, offsets, n_rows
     return y
 
 
-def _option(block, name, default):
-    """block.<name> or the default: an attribute of the block or of its class (nn.Module answers for a missing attribute by
-    way of an exception)."""
-    d = block.__dict__
-    return d[name] if name in d else getattr(type(block), name, default)
-
-
 @torch.no_grad()
 def moe_forward(block, hidden_states: torch.Tensor, spec: ops.RouterSpec, gate_weight: torch.Tensor,
                 bias, experts, shared, combine_mode: int, want_logits: bool = False):
@@ -429,8 +422,8 @@ def moe_forward(block, hidden_states: torch.Tensor, spec: ops.RouterSpec, gate_w
         x = x.contiguous()
     n, h = x.shape
     k, E = spec.top_k, spec.n_experts
-    fuse, timer = _option(block, "_norm_residual", None), _option(block, "stage_timer", None)
-    fused_gather, join = _option(block, "fused_gather", True), _option(block, "join_shared", True)
+    fuse, timer = _attr(block, "_norm_residual"), _attr(block, "stage_timer")
+    fused_gather, join = _attr(block, "fused_gather", True), _attr(block, "join_shared", True)
     cache = block.__dict__.setdefault("_moe_cache", {})
     gw = _gate_weight_bf16(gate_weight, cache)
     b = None if bias is None else bias.data.to(torch.float32)

@@ -349,3 +349,33 @@ def test_missing_block_scales_are_named():
     q = torch.zeros(128, 128).to(torch.float8_e4m3fn)
     with pytest.raises(ValueError, match="block scales"):
         ops.expert_pointers([q], [q], [q], [None], [None], [None])
+
+
+def test_attributes_of_a_block_are_what_getattr_gives():
+    """A stage timer that is itself a module, a switch kept as a buffer, a class attribute, a property, a class with a
+    __getattr__ of its own, and an object that is no module."""
+    from moe_gen_amd.block import _attr
+
+    class Timer(torch.nn.Module):
+        pass
+
+    class Forwarding(torch.nn.Module):
+        join_shared = False
+
+        @property
+        def fused_gather(self):
+            return 3
+
+        def __getattr__(self, name):
+            return 5 if name == "stage_timer" else super().__getattr__(name)
+
+    class Plain:
+        __slots__ = ("module",)
+
+    blk, fwd, plain = tiny("v3"), Forwarding(), Plain()
+    blk.stage_timer = timer = Timer()
+    blk.register_buffer("join_shared", torch.zeros(()))
+    plain.module = blk
+    assert _attr(blk, "stage_timer") is timer and _attr(blk, "join_shared") is blk.join_shared and _attr(blk, "fused_gather", 7) == 7
+    assert (_attr(fwd, "join_shared"), _attr(fwd, "fused_gather"), _attr(fwd, "stage_timer"), _attr(fwd, "absent", 9)) == (False, 3, 5, 9)
+    assert _attr(plain, "module") is blk and _attr(plain, "absent") is None
