@@ -372,7 +372,7 @@ def test_attributes_of_a_block_are_what_getattr_gives():
     class Plain:
         __slots__ = ("module",)
 
-    blk, fwd, plain = tiny("v3"), Forwarding(), Plain()
+    blk, fwd, plain = synthetic.build_block(tiny("v3"), device="cpu"), Forwarding(), Plain()
     blk.stage_timer = timer = Timer()
     blk.register_buffer("join_shared", torch.zeros(()))
     plain.module = blk
