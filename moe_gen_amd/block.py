@@ -4,6 +4,8 @@ slot, in waves when its pool is smaller than the layer) and the fused forward
 router -> dispatch -> grouped SwiGLU -> combine."""
 from __future__ import annotations
 
+import operator
+
 import torch
 from torch import nn
 
@@ -129,12 +131,13 @@ def _unwrap(expert):
     return _attr(expert, "module", expert)
 
 
-def _tensors_of(expert, fetched=None):
+def _tensors_of(expert, fetched=None, places=None):
     """(gate, up, down, s_gate, s_up, s_down) of one expert.
 
     fetched: optional dict `"<proj>.weight" -> tensor` obtained from an engine's get_weights();
     block scales come from the Linear's `weight_scale_inv` or, for a wrapped expert, from the
-    wrapper's `weight_dequant_scale["<proj>.weight_scale_inv"]` (Wrapper.py:482-489)."""
+    wrapper's `weight_dequant_scale["<proj>.weight_scale_inv"]` (Wrapper.py:482-489).
+    places: a _Places that notes where each of them was found."""
     if fetched is not None:                     # hot path of the staged walk: no attribute look-ups on the modules
         keys = expert.__dict__.get("_moe_keys")
         if keys is None:                        # the tensor names of this expert, built once
@@ -148,18 +151,23 @@ def _tensors_of(expert, fetched=None):
         wrap_scales = expert.__dict__.get("weight_dequant_scale")
         if wrap_scales:
             return (w0, fetched[wk[1]], fetched[wk[2]], wrap_scales.get(sk[0]), wrap_scales.get(sk[1]), wrap_scales.get(sk[2]))
-    mlp = _unwrap(expert)
-    wrap_scales = _attr(expert, "weight_dequant_scale") or {}
+    look = _attr if places is None else places.look
+    mlp = look(expert, "module", expert)
+    wrap_scales = None
     ws, ss = [], []
     for name in mlp.names:
-        lin = _attr(mlp, name)
-        w = fetched[name + ".weight"] if fetched is not None else _attr(lin, "weight").data
+        lin = look(mlp, name)
+        w = fetched[name + ".weight"] if fetched is not None else look(lin, "weight").data
         s = None
         if w.dtype == FP8:                      # (bf16 weights have no scales to look for)
+            if wrap_scales is None:
+                wrap_scales = look(expert, "weight_dequant_scale") or {}
             s = wrap_scales.get(name + ".weight_scale_inv")
             if s is None:
-                s = _attr(lin, "weight_scale_inv")
+                s = look(lin, "weight_scale_inv")
                 s = None if s is None else s.data
+            elif places is not None:
+                places.tensor(wrap_scales, name + ".weight_scale_inv", s)
         ws.append(w)
         ss.append(s)
     return (*ws, *ss)
@@ -181,6 +189,113 @@ def _attr(obj, name, default=None):
         if name in d[table]:
             return d[table][name]
     return default
+
+
+class _Places:
+    """Where the weights and scales of a list of experts were found: the dicts that attribute look-up came down to, so that
+    a later call can tell in a few passes of C code whether every one of them is still the tensor that the pointer tables
+    were made from (256 fp8 experts: 0.17 ms; following the attributes again takes 8 ms).  An expert that answers through
+    properties or a __getattr__ of its own is asked again, tensor by tensor."""
+
+    def __init__(self, experts=()):
+        self.experts, self.traced = list(experts), True
+        self.submodules = [], []                        # _modules dicts, and copies of them
+        self.links, self.tensors = ([], [], []), ([], [], [])      # dicts, keys, and the objects / addresses found there
+        self.kinds = {}                                 # (class, name) -> where its objects may keep it (0: they have to be asked)
+
+    def note(self):
+        """Follows every expert's attributes: [(gate, up, down, s_gate, s_up, s_down)]."""
+        rows = [_tensors_of(ex, None, self) for ex in self.experts]
+        self.form = rows[0][0].dtype, rows[0][0].shape
+        if not self.traced:
+            self.addresses = _addresses(rows)
+        return rows
+
+    def look(self, obj, name, default=None):
+        """_attr, noting where the value lay."""
+        cls = type(obj)
+        kind = self.kinds.get((cls, name))
+        if kind is None:
+            kind = 0 if hasattr(cls, name) or not hasattr(obj, "__dict__") else 1        # 1: in its __dict__ or nowhere
+            if kind and hasattr(cls, "__getattr__"):
+                kind = 2 if cls.__getattr__ is nn.Module.__getattr__ else 0              # 2: or in a module's tables
+            self.kinds[cls, name] = kind
+        if not kind:
+            self.traced = False
+            return getattr(obj, name, default)
+        own = obj.__dict__
+        if name in own:
+            d = own
+        elif kind == 1:
+            return self._absent(own, name, default)
+        elif name in own["_parameters"]:
+            d = own["_parameters"]
+        elif name in own["_modules"]:
+            d = own["_modules"]
+            if not self.submodules[0] or self.submodules[0][-1] is not d:
+                self.submodules[0].append(d)
+                self.submodules[1].append(d.copy())
+            return d[name]
+        elif name in own["_buffers"]:
+            d = own["_buffers"]
+        else:
+            return self._absent(own, name, default)
+        value = d[name]
+        if isinstance(value, torch.Tensor):
+            self.tensor(d, name, value)
+        else:
+            self.link(d, name, value)
+        return value
+
+    def _absent(self, own, name, default):
+        if name == "weight_dequant_scale":              # (of what an expert may lack, this can be given to it later)
+            self.link(own, name, None)
+        return default
+
+    def tensor(self, d, key, value):
+        dicts, keys, found = self.tensors
+        dicts.append(d)
+        keys.append(key)
+        found.append(value.data_ptr())
+
+    def link(self, d, key, value):
+        dicts, keys, found = self.links
+        dicts.append(d)
+        keys.append(key)
+        found.append(value)
+
+    def ends_hold(self, experts) -> bool:
+        """hold() for the first and the last tensor alone (which a block moved to another device or type does not pass)."""
+        if not self.traced:
+            return self.hold(experts)
+        if len(experts) != len(self.experts) or experts[0] is not self.experts[0]:
+            return False
+        dicts, keys, found = self.tensors
+        first, last = dicts[0].get(keys[0]), dicts[-1].get(keys[-1])
+        return (first is not None and last is not None and (first.dtype, first.shape) == self.form
+                and first.data_ptr() == found[0] and last.data_ptr() == found[-1])
+
+    def hold(self, experts) -> bool:
+        """Whether these are the experts noted, with every weight and scale where it was."""
+        if len(experts) != len(self.experts) or not all(map(operator.is_, experts, self.experts)):
+            return False
+        if not self.traced:
+            return _addresses([_tensors_of(ex) for ex in experts]) == self.addresses
+        dicts, keys, found = self.links
+        if not (all(map(operator.eq, *self.submodules)) and all(map(operator.is_, map(dict.get, dicts, keys), found))):
+            return False
+        dicts, keys, found = self.tensors
+        try:
+            return list(map(torch.Tensor.data_ptr, map(operator.getitem, dicts, keys))) == found
+        except (KeyError, TypeError):                   # (a tensor was taken away)
+            return False
+
+    def __reduce__(self):
+        return _Places, ()                              # (a copy's weights are tensors of its own)
+
+
+def _addresses(rows):
+    return [None if t is None else t.data_ptr() for row in rows for t in row]
 
 
 def _pointer_table(rows, one_call):
@@ -211,18 +326,25 @@ def any_engine_backed(experts) -> bool:
     return any(engine_backed(ex) for ex in experts)
 
 
+def _cached_pointers(experts, cache):
+    """The pointer tables of the last call if the first and the last tensor are where they were, else None.  What lies in
+    between is not looked at: `ptrs.places.hold(experts)` does."""
+    ptrs = cache.get("ptrs")
+    return ptrs if ptrs is not None and ptrs.places.ends_hold(experts) else None
+
+
 def collect_pointers(experts, cache):
-    """Pointer tables for a list of RESIDENT expert modules, cached in `cache` (a dict) keyed on
-    the storage addresses of the first and last expert; without one they serve this call on this stream only."""
-    first, last = _unwrap(experts[0]), _unwrap(experts[-1])
-    f = _attr(_attr(first, first.names[0]), "weight").data
-    stamp = (len(experts), f.data_ptr(), f.dtype, f.shape, _attr(_attr(last, last.names[2]), "weight").data.data_ptr())
-    if cache is not None and cache.get("stamp") == stamp:
-        return cache["ptrs"]
-    p = _pointer_table([_tensors_of(ex) for ex in experts], one_call=cache is None)
-    if cache is not None:
-        cache["stamp"], cache["ptrs"] = stamp, p
-    return p
+    """Pointer tables for a list of RESIDENT expert modules, kept in `cache` (a dict) for as long as every weight and scale
+    is the tensor it was; without one they serve this call on this stream only."""
+    if cache is None:
+        return _pointer_table([_tensors_of(ex) for ex in experts], one_call=True)
+    ptrs = _cached_pointers(experts, cache)
+    if ptrs is None or not ptrs.places.hold(experts):
+        places = _Places(experts)
+        ptrs = _pointer_table(places.note(), one_call=False)
+        ptrs.places = places
+        cache["ptrs"] = ptrs
+    return ptrs
 
 
 def pool_size(expert, module_type: str = "routed_expert") -> int:
@@ -430,10 +552,19 @@ def moe_forward(block, hidden_states: torch.Tensor, spec: ops.RouterSpec, gate_w
     experts = list(experts)
     staged = any_engine_backed(experts)            # decided expert by expert, as the reference's initializers do
     if timer is None and fused_gather and not staged and (shared is None or not engine_backed(shared)):
-        ptrs = collect_pointers(experts, cache.setdefault("routed", {}))
-        sp = None if shared is None else collect_pointers([shared], cache.setdefault("shared", {}))
-        out, idx, w, counts, logits = ops.layer_forward(x, *(fuse or (None, 0.0)), gw, b, spec, ptrs, sp, combine_mode, bool(join),
-                                                        want_logits)
+        groups = [(experts, cache.setdefault("routed", {}))]
+        if shared is not None:
+            groups.append(([shared], cache.setdefault("shared", {})))
+        # The tables of the last call are used at once and held against the modules while the GPU runs (256 fp8 experts:
+        # 0.17 ms of host time); where one is out of date the call is made again.
+        kept = [_cached_pointers(*g) for g in groups]
+        while True:
+            tables = [t or collect_pointers(*g) for t, g in zip(kept, groups)]
+            out, idx, w, counts, logits = ops.layer_forward(x, *(fuse or (None, 0.0)), gw, b, spec, tables[0],
+                                                            tables[1] if shared is not None else None, combine_mode, bool(join), want_logits)
+            if all(t is None or t.places.hold(g[0]) for t, g in zip(kept, groups)):
+                break
+            kept = [None] * len(groups)
         d = block.__dict__
         d["last_topk_idx"], d["last_topk_weight"], d["last_counts"] = idx, w, counts
         return out.view(shape), logits

@@ -263,3 +263,43 @@ def test_layer_call_reads_only_the_weights_of_its_groups(E):
         tables.weights.workspace, tables.weights.workspace_bytes = sentinel.data_ptr(), sentinel.numel()
     assert torch.equal(blk(x), want)
     assert (sentinel == 7).all()
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("path", ["layer", "stages"])
+def test_layer_sees_every_replaced_weight_and_scale(fp8, path):
+    """A block that has run, and then gets a middle expert's up projection, the shared expert's up projection (fp8: and one
+    expert's block scales) anew, computes what a block that never ran before computes with them."""
+    from moe_gen_amd import synthetic
+    from moe_gen_amd.block import StageTimer
+    w = synthetic.WORKLOADS["deepseek_v3_w8a16" if fp8 else "deepseek_v2_lite"].scaled(n=96, h=512, I=256, seq=96)
+    x = synthetic.hidden_states(w, "cpu").cuda()
+    print(f"replaced weights fp8={fp8} {path}", flush=True)
+
+    def block():
+        b = synthetic.build_block(w, device="cuda", gen_device="cpu")
+        b.stage_timer = StageTimer() if path == "stages" else None
+        return b
+
+    def replace(b, what):
+        ex = b.shared_experts if what == "shared" else b.experts[len(b.experts) // 2]
+        lin, name = (ex.down_proj, "weight_scale_inv") if what == "scale" else (ex.up_proj, "weight")
+        old = getattr(lin, name).data
+        new = old * 2 if what == "scale" else old.flip(0).contiguous() if not fp8 else old.view(torch.uint8).flip(0).contiguous().view(old.dtype)
+        if what == "data":
+            getattr(lin, name).data = new
+        else:
+            setattr(lin, name, torch.nn.Parameter(new, requires_grad=False))
+
+    ran, last = block(), None
+    last = ran(x).clone()
+    done = []
+    for what in ["weight", "shared", "data"] + (["scale"] if fp8 else []):
+        replace(ran, what)
+        done.append(what)
+        got, fresh = ran(x), block()
+        for d in done:
+            replace(fresh, d)
+        assert torch.equal(got, fresh(x)), what
+        assert not torch.equal(got, last), what
+        last = got.clone()

@@ -379,3 +379,87 @@ def test_attributes_of_a_block_are_what_getattr_gives():
     assert _attr(blk, "stage_timer") is timer and _attr(blk, "join_shared") is blk.join_shared and _attr(blk, "fused_gather", 7) == 7
     assert (_attr(fwd, "join_shared"), _attr(fwd, "fused_gather"), _attr(fwd, "stage_timer"), _attr(fwd, "absent", 9)) == (False, 3, 5, 9)
     assert _attr(plain, "module") is blk and _attr(plain, "absent") is None
+
+
+@pytest.mark.parametrize("form", ["bf16", "parameter", "buffer", "own_dict", "wrapped", "property"])
+def test_pointer_tables_follow_every_weight_and_scale(form, monkeypatch):
+    """Tables are kept while nothing changed, and made anew when any tensor of any expert is another one, whichever way it
+    came there: a middle expert's Parameter, its .data, a block scale, a Linear, an expert; never taken over by a copy."""
+    import copy
+    from moe_gen_amd import block
+    from moe_gen_amd.block import SwiGLUMLP, collect_pointers
+
+    class Table:
+        def __init__(self, rows, one_call):
+            self.addresses = [None if t is None else t.data_ptr() for r in rows for t in r]
+
+    class Wrapper(torch.nn.Module):
+        def __init__(self, module, scales):
+            super().__init__()
+            self.module, self.weight_dequant_scale = module, scales
+
+    class Owner(SwiGLUMLP):
+        @property
+        def up_proj(self):
+            return self.kept_up
+
+        @up_proj.setter
+        def up_proj(self, lin):
+            self.kept_up = lin
+
+    monkeypatch.setattr(block, "_pointer_table", Table)
+    fp8 = form not in ("bf16", "property")
+
+    def weight(lin):
+        w = torch.randn(lin.weight.shape)
+        return torch.nn.Parameter(w.to(torch.float8_e4m3fn if fp8 else torch.bfloat16), requires_grad=False)
+
+    def expert():
+        mlp, scales = (Owner if form == "property" else SwiGLUMLP)(128, 256), {}
+        for name in mlp.names:
+            lin = getattr(mlp, name)
+            lin.weight = weight(lin)
+            s = torch.ones(-(-lin.weight.shape[0] // 128), -(-lin.weight.shape[1] // 128))
+            if form == "parameter":
+                lin.weight_scale_inv = torch.nn.Parameter(s, requires_grad=False)
+            elif form == "buffer":
+                lin.register_buffer("weight_scale_inv", s)
+            scales[name + ".weight_scale_inv"] = s
+        if form == "own_dict":
+            mlp.weight_dequant_scale = scales
+        return Wrapper(mlp, scales) if form == "wrapped" else mlp
+
+    experts, cache = [expert() for _ in range(5)], {}
+    inner = lambda: getattr(experts[2], "module", experts[2])
+
+    def replace_scale():
+        if form in ("own_dict", "wrapped"):
+            experts[2].weight_dequant_scale["up_proj.weight_scale_inv"] = torch.ones(2, 1)
+        elif "weight_scale_inv" in inner().up_proj._parameters:
+            inner().up_proj.weight_scale_inv = torch.nn.Parameter(torch.ones(2, 1), requires_grad=False)
+        else:
+            inner().up_proj.weight_scale_inv = torch.ones(2, 1)
+
+    def replace_linear():
+        lin = torch.nn.Linear(128, 256, bias=False)
+        lin.weight = weight(lin)
+        if fp8:
+            lin.weight_scale_inv = torch.nn.Parameter(torch.ones(2, 1), requires_grad=False)
+        inner().up_proj = lin
+
+    changes = [lambda: setattr(inner().up_proj, "weight", weight(inner().up_proj)),
+               lambda: setattr(inner().gate_proj.weight, "data", weight(inner().gate_proj).data),
+               lambda: experts.__setitem__(3, expert())] + ([replace_scale] if fp8 else []) + [replace_linear]
+    for change in changes:
+        kept = collect_pointers(experts, cache)
+        assert collect_pointers(experts, cache) is kept
+        change()
+        new = collect_pointers(experts, cache)
+        assert new is not kept
+        assert new.addresses == [None if t is None else t.data_ptr() for ex in experts for t in block._tensors_of(ex)]
+    twin = copy.deepcopy((experts, cache))
+    assert not twin[1]["ptrs"].places.hold(twin[0])
+    if fp8 and form not in ("own_dict", "wrapped"):
+        kept = collect_pointers(experts, cache)
+        experts[1].weight_dequant_scale = {n + ".weight_scale_inv": torch.ones(2, 2) for n in experts[1].names}
+        assert collect_pointers(experts, cache) is not kept
