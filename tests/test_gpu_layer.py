@@ -303,3 +303,27 @@ def test_layer_sees_every_replaced_weight_and_scale(fp8, path):
         assert torch.equal(got, fresh(x)), what
         assert not torch.equal(got, last), what
         last = got.clone()
+
+
+def test_first_call_of_a_block_on_another_stream_finds_its_tables():
+    """A block whose first call runs on one stream and whose next call follows at once on another: the tables that the
+    first call made are there for both."""
+    from moe_gen_amd import synthetic
+    w = synthetic.WORKLOADS["deepseek_v3_w8a16"].scaled(n=48, h=512, I=256, seq=48)
+    x = synthetic.hidden_states(w, "cpu").cuda()
+    print("first call on a stream of its own", flush=True)
+    want = synthetic.build_block(w, device="cuda", gen_device="cpu")(x).clone()
+    busy = torch.randn(4096, 4096, device="cuda")
+    for _ in range(3):
+        blk = synthetic.build_block(w, device="cuda", gen_device="cpu")
+        streams = torch.cuda.Stream(), torch.cuda.Stream()
+        torch.cuda.synchronize()
+        outs = []
+        for i, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                if i == 0:                          # (the first stream is busy when its call comes, the second is not)
+                    for _ in range(20):
+                        busy = busy @ busy * 1e-3
+                outs.append(blk(x))
+        torch.cuda.synchronize()
+        assert torch.equal(outs[0], want) and torch.equal(outs[1], want)
