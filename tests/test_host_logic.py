@@ -463,3 +463,15 @@ def test_pointer_tables_follow_every_weight_and_scale(form, monkeypatch):
         kept = collect_pointers(experts, cache)
         experts[1].weight_dequant_scale = {n + ".weight_scale_inv": torch.ones(2, 2) for n in experts[1].names}
         assert collect_pointers(experts, cache) is not kept
+
+
+def test_engine_backed_experts_that_answer_by_getattr():
+    """An MLP class that hands its staging attributes on from a helper is as engine-backed in a layer as on its own."""
+    from moe_gen_amd.block import SwiGLUMLP, any_engine_backed, engine_backed
+
+    class Delegating(SwiGLUMLP):
+        def __getattr__(self, name):
+            return {"get_weights": True, "core_engine": self}[name] if name in ("get_weights", "core_engine") else super().__getattr__(name)
+
+    assert engine_backed(Delegating(16, 16)) and any_engine_backed([Delegating(16, 16)])
+    assert not any_engine_backed([SwiGLUMLP(16, 16)])
