@@ -78,7 +78,7 @@ typedef struct moe_router_params {
  *   topk_w     device fp32 [n, k]    out
  *   logits_out device fp32 [n, E]    out, may be NULL.  With it the call is two launches: logits into the
  *              buffer, routing from it.  Without it one launch keeps the logits on chip, which spreads
- *              fewer than about 4000 tokens over fewer CUs (256 experts, 64 tokens: about three times the time)
+ *              them over fewer CUs (256 experts, 64 tokens: 84 us against 36; 65536 tokens: 2106 against 1715)
  * hidden: a multiple of 8 below 2^22.
  */
 int moe_router(const void* x, const void* w_gate, const float* bias,

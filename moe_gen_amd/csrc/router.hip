@@ -274,7 +274,8 @@ __device__ void route_token(const float* row, const float* __restrict__ bias, co
 // 92 ... 95, 100 and 2153 us.)
 // FUSED == false: the logits of the tile go to `logits` [n, E] in memory, router_select_kernel routes the tokens.
 // FUSED == true (a caller without a logits buffer): the workgroup walks the expert blocks of its tokens one after the
-// other, keeps the logits in LDS and routes the tokens itself.
+// other, keeps the logits in LDS and routes the tokens itself.  Where that leaves most CUs without tokens
+// router_tokens_kernel takes the call.
 typedef __attribute__((address_space(3))) uint8_t* lds_u8;
 
 constexpr int kStageBytes = 256, kStepsPerStage = 32;    // 128 k of a row per stage, 4 k per step
@@ -297,7 +298,7 @@ __device__ __forceinline__ void read_bf16_as_f32(float& v, uint32_t addr) {
     asm volatile("ds_read_u16_d16_hi %0, %1 offset:%2" : "+v"(v) : "v"(addr), "n"(OFF));
 }
 
-template <int WT, int WE, int TT, int TE, int S, bool FUSED, int GW>
+template <int WT, int WE, int TT, int TE, int S, bool FUSED, int GW, int EJ>   // (GW, EJ: route_token; read where FUSED)
 __global__ __launch_bounds__(64 * WT * WE, 1) void router_logits_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ wg, const float* __restrict__ bias,
     moe_router_params p, int32_t* __restrict__ topk_idx, float* __restrict__ topk_w, float* __restrict__ logits) {
@@ -306,12 +307,14 @@ __global__ __launch_bounds__(64 * WT * WE, 1) void router_logits_kernel(
     constexpr int NX = BT / (4 * NW), NE = BE / (4 * NW), NI = NX + NE;   // DMA instructions (4 rows each) per wave and stage
     constexpr int SB = (BT + BE) / 4 * kBlock;                  // bytes of a stage, token rows first
     constexpr int R = TT + TE, DEPTH = ring_depth(R), RING = DEPTH > 3 ? 8 : 4;
-    static_assert((TT == 1 ? RING == 8 : RING == 4) && NI <= 8 && DEPTH < RING && DEPTH >= 2 && S >= 3 && (S - 2) * NI < 64, "counters");
-    constexpr int LG = FUSED ? (BE == 16 ? 16 : 256) : 1;       // row of the logits kept in LDS
+    static_assert((TT == 1 ? RING == 8 : RING == 4) && NI <= 10 && DEPTH < RING && DEPTH >= 2 && S >= 3 && (S - 2) * NI < 64, "counters");
+    constexpr int LG = GW == 64 ? 64 * EJ : BE;                 // row of the logits kept in LDS: whole expert blocks
+    static_assert(LG % BE == 0, "expert blocks");
     __shared__ __attribute__((aligned(1024))) uint8_t lds[S * SB];
     __shared__ float lg[FUSED ? BT * LG : 1];
-    constexpr int EJ = GW == 64 ? 4 : 1;                        // experts per lane in the selection (GW lanes: E <= GW below 64)
-    __shared__ float val[FUSED ? NW * 64 * EJ : 1];
+    constexpr bool VAL_IN_STAGES = S == 3;                      // the selection's values in the stage buffers: two workgroups per CU then fit
+    static_assert(NW * 64 * EJ * 4 <= S * SB, "selection");
+    __shared__ float val_own[FUSED && !VAL_IN_STAGES ? NW * 64 * EJ : 1];
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -330,7 +333,7 @@ __global__ __launch_bounds__(64 * WT * WE, 1) void router_logits_kernel(
         // the buffer: neither is multiplied
         const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void*)(x + (size_t)t0 * h), 0, min(BT, n - t0) * h * 2, 0x00020000);
         const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)(wg + (size_t)e0 * h), 0, min(BE, E - e0) * h * 2, 0x00020000);
-        int voff[8];                                                // (NI <= 8 are used)
+        int voff[10];                                               // (NI <= 10 are used)
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
             const int g = 4 * (wave + NW * i) + (lane & 3);         // row of the stage
@@ -458,6 +461,7 @@ __global__ __launch_bounds__(64 * WT * WE, 1) void router_logits_kernel(
         e0 += BE;
     } while (FUSED && e0 < E);
     if constexpr (FUSED) {
+        float* const val = VAL_IN_STAGES ? reinterpret_cast<float*>(lds) : val_own;       // (behind the barrier above)
         constexpr int TPW = 64 / GW;
         for (int tb = wave * TPW; tb < BT; tb += NW * TPW) {
             if (t0 + tb >= n) break;
@@ -469,6 +473,150 @@ __global__ __launch_bounds__(64 * WT * WE, 1) void router_logits_kernel(
         }
     }
 }
+
+// Logits and selection in one launch for more than 128 experts and up to 1024 tokens whose caller has no logits buffer.
+// Sixteen tokens per workgroup, as above, are 64 CUs at most, each with four blocks of experts one after the other
+// (DeepSeek-V3's gate, 64 tokens: 143 us).  Here a workgroup takes 4 tokens and a wave 64 experts, in the 4 x 64 layout
+// of the 4x4 MFMA: lane l of a wave the expert 64 wave + l.
+//  * The 128-byte lines of a wave's 64 gate rows reach its own LDS region as bf16 by DMA (8 instructions per 64 k; chunk c
+//    of row r in 16-byte slot c ^ g(r), so that the 16 lanes the LDS serves together -- rows 8i .. 8i+7 and
+//    32+8i .. 39+8i -- fall on 16 different bank groups); a lane reads the 8 weights of its expert with one
+//    ds_read_b128 and widens them to fp32 between the MFMAs (a shift or a mask each).
+//  * The token values never touch LDS: the MFMA broadcasts the A operand of one block to all 16, so a register that
+//    holds the 4 tokens' values of 16 consecutive k (one 2-byte load per lane) feeds 16 instructions.
+//  * One wave's LDS reads execute in order and its DMA is ordered by vmcnt, so the k loop has no barrier.
+// Each logit is the same chain of one fused multiply-add per k as in the engine above.  Per k a wave issues one
+// MFMA, one conversion and an eighth of a 16-byte LDS read: 11.9 ns; 9.7 ns without the conversion and 8.3 ns without
+// the LDS read either, which is the MFMA chain itself.
+__device__ __forceinline__ int thin_slot(int r) { return ((r >> 1) & 3) | (((r >> 5) & 1) << 2); }
+
+// The A operand of block B is broadcast to all 16 blocks of the instruction (cbsz = 4, abid = B), so ONE register holds
+// the token values of 16 consecutive k: lanes 4b .. 4b+3 the 4 tokens at k0 + b.  The B operand of lane l is expert l
+// of the wave's 64.
+template <int B>
+__device__ __forceinline__ f32x4 mfma_4_tokens(float a, float b, f32x4 acc) {
+    return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, acc, 4, B, 0);
+}
+
+template <int WE>
+__global__ __launch_bounds__(64 * WE, 1) void router_tokens_kernel(
+    const uint16_t* __restrict__ x, const uint16_t* __restrict__ wg, const float* __restrict__ bias,
+    moe_router_params p, int32_t* __restrict__ topk_idx, float* __restrict__ topk_w) {
+    constexpr int KC = 64, BT = 4, EP = 64 * WE, WBYTES = 64 * 128;
+    // (one workgroup per CU) one array per weight buffer: a read of one then never waits for the DMA in flight into another
+    __shared__ __attribute__((aligned(1024))) uint8_t wb0[WE * WBYTES];           // written by DMA only
+    __shared__ __attribute__((aligned(1024))) uint8_t wb1[WE * WBYTES];
+    __shared__ __attribute__((aligned(1024))) uint8_t wb2[WE * WBYTES];
+    __shared__ __attribute__((aligned(16))) float lg[BT * EP];
+    __shared__ float val[WE * EP];                                                // selection: EP per wave
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n = p.n_tokens, h = p.hidden, E = p.n_experts;
+    const int t0 = blockIdx.x * BT;
+    const int nfull = h / KC, rem8 = (h % KC) / 8, nstage = nfull + (rem8 ? 1 : 0);
+
+    // weight DMA: instruction i brings rows 8i .. 8i+7 of the wave's 64, a lane the chunk that belongs in its slot
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)wg, 0, E * h * 2, 0x00020000);
+    int w_voff[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const int r = 8 * i + (lane >> 3), c = (lane & 7) ^ thin_slot(r);
+        w_voff[i] = (min(64 * wave + r, E - 1) * h + c * 8) * 2;
+    }
+    auto dma_w = [&](uint8_t* buf, int st) {
+        uint8_t* dst = buf + wave * WBYTES;
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_u8)(dst + i * 1024), 16, w_voff[i], (uint32_t)(st * (KC * 2)), 0, 0);
+    };
+    // token values straight from memory into the broadcast layout: register g of a stage holds, in lanes
+    // 4b .. 4b+3, element 16 g + b of the 4 tokens (one 2-byte load per lane and 16 k), widened when its 16 k come up
+    const uint16_t* const xrow = x + (size_t)min(t0 + (lane & 3), n - 1) * h;
+    uint32_t xr[2][4];
+    auto load_x = [&](int set, int st) {       // (elements past h are never multiplied: any address inside the row will do)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const int k = st * KC + 16 * g + (lane >> 2);
+            xr[set][g] = xrow[k < h ? k : 0];
+        }
+    };
+
+    f32x4 acc = {0, 0, 0, 0};                  // register i: token i, expert 64 wave + lane
+    int w_roff[8];                             // chunk c of the lane's row inside a buffer
+#pragma unroll
+    for (int c = 0; c < 8; ++c) w_roff[c] = wave * WBYTES + lane * 128 + ((c ^ thin_slot(lane)) << 4);
+
+    auto wf = [](const u32x4& v, int j) {      // element j of 8 bf16 as fp32
+        return __uint_as_float((j & 1) ? (v[j >> 1] & 0xffff0000u) : (v[j >> 1] << 16));
+    };
+    // Stage st; the register set st & 1 and the buffers are literals at every call site.  The DMA of stage
+    // st + 2 leaves first, then the wait for the DMA of stage st.  Its count is the DMA instructions issued
+    // since -- 8 per stage ahead -- and nothing else: the token loads sit behind the wait in program order, but the
+    // compiler may place a register load on either side of it, and every one that is in the window only makes the
+    // wait stricter (the oldest operations in the window are token loads of a stage ago, long complete).
+    auto stage = [&](int st, int set, const uint8_t* wb, uint8_t* wb_refill, int nch) {
+        uint32_t xs[4];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) xs[g] = xr[set][g];
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the reads of stage st - 1, a stage old, before their buffer is refilled
+        dma_w(wb_refill, min(st + 2, nstage - 1));
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * 8) : "memory");
+        load_x(set, min(st + 2, nstage - 1));            // (tokens of stage st + 2 into the set that held stage st)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            if (2 * g >= nch) break;
+            const u32x4 w0 = *reinterpret_cast<const u32x4*>(wb + w_roff[2 * g]);
+            const u32x4 w1 = *reinterpret_cast<const u32x4*>(wb + w_roff[2 * g + 1]);
+            const float xa = __uint_as_float(xs[g] << 16);
+#define MOE_THIN_K(B) \
+    if (2 * g + ((B) >> 3) < nch) acc = mfma_4_tokens<B>(xa, wf((B) < 8 ? w0 : w1, (B) & 7), acc);
+            MOE_THIN_K(0) MOE_THIN_K(1) MOE_THIN_K(2) MOE_THIN_K(3) MOE_THIN_K(4) MOE_THIN_K(5) MOE_THIN_K(6) MOE_THIN_K(7)
+            MOE_THIN_K(8) MOE_THIN_K(9) MOE_THIN_K(10) MOE_THIN_K(11) MOE_THIN_K(12) MOE_THIN_K(13) MOE_THIN_K(14) MOE_THIN_K(15)
+#undef MOE_THIN_K
+        }
+    };
+
+    int st = 0;
+    load_x(0, 0);
+    load_x(1, min(1, nstage - 1));
+    dma_w(wb0, 0);
+    dma_w(wb1, min(1, nstage - 1));
+    for (; st + 6 <= nfull; st += 6) {
+        stage(st, 0, wb0, wb2, 8);
+        stage(st + 1, 1, wb1, wb0, 8);
+        stage(st + 2, 0, wb2, wb1, 8);
+        stage(st + 3, 1, wb0, wb2, 8);
+        stage(st + 4, 0, wb1, wb0, 8);
+        stage(st + 5, 1, wb2, wb1, 8);
+    }
+    // up to 5 whole stages and one of fewer than 64 k are left; stage st + i has the literals of i
+    const int left = nfull - st;
+    if (left > 0) stage(st, 0, wb0, wb2, 8);
+    if (left > 1) stage(st + 1, 1, wb1, wb0, 8);
+    if (left > 2) stage(st + 2, 0, wb2, wb1, 8);
+    if (left > 3) stage(st + 3, 1, wb0, wb2, 8);
+    if (left > 4) stage(st + 4, 0, wb1, wb0, 8);
+    if (rem8) {
+        if (left == 0) stage(st, 0, wb0, wb2, rem8);
+        else if (left == 1) stage(st + 1, 1, wb1, wb0, rem8);
+        else if (left == 2) stage(st + 2, 0, wb2, wb1, rem8);
+        else if (left == 3) stage(st + 3, 1, wb0, wb2, rem8);
+        else if (left == 4) stage(st + 4, 0, wb1, wb0, rem8);
+        else stage(st + 5, 1, wb2, wb1, rem8);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // no DMA may land in LDS after the workgroup has gone
+
+#pragma unroll
+    for (int i = 0; i < 4; ++i) lg[i * EP + 64 * wave + lane] = acc[i];
+    __syncthreads();
+    for (int tb = wave; tb < BT; tb += WE) {
+        if (t0 + tb >= n) break;
+        const int t = t0 + tb;
+        route_token<64, WE>(lg + tb * EP, bias, p, topk_idx + (size_t)t * p.top_k, topk_w + (size_t)t * p.top_k, nullptr, nullptr,
+                            val + wave * EP, true);
+    }
+}
+
 
 // Routes the tokens of a logits matrix in memory, a lane group per token (the group width follows from the expert count
 // alone: it fixes the order of the softmax sum).  logits_bf16 (Mixtral): the rounded values are written back.
@@ -515,13 +663,18 @@ template <int WT, int WE, int TT, int TE, int S>
 void launch_logits(const void* x, const void* w, const moe_router_params& p, float* logits, hipStream_t st) {
     constexpr int BT = 16 * TT * WT, BE = 16 * TE * WE;
     const int ntb = (p.n_tokens + BT - 1) / BT, neb = (p.n_experts + BE - 1) / BE;
-    hipLaunchKernelGGL((router_logits_kernel<WT, WE, TT, TE, S, false, 64>), dim3((ntb + 7) / 8 * 8 * neb), dim3(64 * WT * WE), 0, st,
+    hipLaunchKernelGGL((router_logits_kernel<WT, WE, TT, TE, S, false, 64, 2>), dim3((ntb + 7) / 8 * 8 * neb), dim3(64 * WT * WE), 0, st,
                        (const uint16_t*)x, (const uint16_t*)w, nullptr, p, nullptr, nullptr, logits);
 }
-template <int WT, int WE, int GW>
+template <int WE>
+void launch_tokens(const void* x, const void* w, const float* bias, const moe_router_params& p, int32_t* idx, float* tw, hipStream_t st) {
+    hipLaunchKernelGGL((router_tokens_kernel<WE>), dim3((p.n_tokens + 3) / 4), dim3(64 * WE), 0, st, (const uint16_t*)x, (const uint16_t*)w,
+                       bias, p, idx, tw);
+}
+template <int WT, int WE, int TT, int S, int GW, int EJ>
 void launch_fused(const void* x, const void* w, const float* bias, const moe_router_params& p, int32_t* idx, float* tw, hipStream_t st) {
-    constexpr int BT = 16 * WT;
-    hipLaunchKernelGGL((router_logits_kernel<WT, WE, 1, 1, 4, true, GW>), dim3((p.n_tokens + BT - 1) / BT), dim3(64 * WT * WE), 0, st,
+    constexpr int BT = 16 * TT * WT;
+    hipLaunchKernelGGL((router_logits_kernel<WT, WE, TT, TT, S, true, GW, EJ>), dim3((p.n_tokens + BT - 1) / BT), dim3(64 * WT * WE), 0, st,
                        (const uint16_t*)x, (const uint16_t*)w, bias, p, idx, tw, nullptr);
 }
 
@@ -650,9 +803,29 @@ int route(const void* x, const void* w_gate, const float* bias, const moe_router
     hipStream_t st = as_stream(stream);
     const int E = p.n_experts;
     if (logits_out == nullptr) {
-        if (E <= 16) launch_fused<2, 1, 16>(x, w_gate, bias, p, topk_idx, topk_w, st);
-        else if (E <= 32) launch_fused<1, 4, 32>(x, w_gate, bias, p, topk_idx, topk_w, st);
-        else launch_fused<1, 4, 64>(x, w_gate, bias, p, topk_idx, topk_w, st);
+        // 4 tokens per workgroup while 16 leave most CUs without any, where that beats three or four expert blocks one
+        // after the other; a ring of 4 stages while every CU has one block of 16 tokens; then two workgroups per CU, so that
+        // one selects while the other multiplies; and 2 x 2 tiles per wave where 128-expert blocks fit and there are many
+        // rounds.  Measured (us, h = 7168 / 5120 / 4096 / 2048 for 256 / 160 / 128 / 64 experts; the engines that took
+        // one k per instruction -> this):
+        //   64 tokens     256 experts 94 -> 84 (16 tokens per workgroup 143), 160: 77 -> 64 (81), 128: 57 -> 48
+        //   4096          235 -> 145, 136 -> 81, 76 -> 49, 41 -> 19      8192: ring of 4 288, of 3 267
+        //   16384         635 -> 530, 427 -> 287, 248 -> 167, 82 -> 54
+        //   65536         2127 -> 2106 (one tile per wave 2161), 1174 -> 1172, 678 -> 682, 260 -> 214
+        for_expert_count(E, [&](auto gw, auto ej) {
+            constexpr int GW = decltype(gw)::value, EJ = decltype(ej)::value;
+            const int n = p.n_tokens;
+            if constexpr (GW == 16) {
+                launch_fused<2, 1, 1, 4, GW, EJ>(x, w_gate, bias, p, topk_idx, topk_w, st);
+            } else {
+                if constexpr (EJ > 2)
+                    if (n <= 1024) return launch_tokens<EJ>(x, w_gate, bias, p, topk_idx, topk_w, st);
+                if constexpr (EJ % 2 == 0)
+                    if (n > 32768) return launch_fused<1, 4, 2, 3, GW, EJ>(x, w_gate, bias, p, topk_idx, topk_w, st);
+                if (n <= 4096) launch_fused<1, 4, 1, 4, GW, EJ>(x, w_gate, bias, p, topk_idx, topk_w, st);
+                else launch_fused<1, 4, 1, 3, GW, EJ>(x, w_gate, bias, p, topk_idx, topk_w, st);
+            }
+        });
         MOE_HIP_CHECK(hipGetLastError());
         return MOE_OK;
     }

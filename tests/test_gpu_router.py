@@ -295,3 +295,29 @@ def test_router_without_a_logits_buffer(E, n, h):
     oi, ow, _ = O.router(bits(x), bits(wg), None if bias is None else bias.numpy(), spec)
     assert np.array_equal(idx.cpu().numpy(), oi)
     assert np.array_equal(w.cpu().numpy().view(np.uint32), ow.view(np.uint32))
+
+
+@pytest.mark.parametrize("E", [9, 24, 64, 65, 128, 129, 192, 193, 256])
+def test_router_without_a_logits_buffer_at_every_size(E):
+    """The kernels behind a call without a logits buffer -- 4 tokens per workgroup up to 1024 tokens of more than 128 experts,
+    rings of 4 and (from 4097 tokens) of 3 stages, 2 x 2 tiles per wave from 32769 -- against the call with one, bit for bit: both
+    sides of each switch, ragged last blocks, and hidden sizes with 0 ... 6 stages of 64 k before a last one of 8 ... 64."""
+    import ctypes
+    from moe_gen_amd import _native as N, ops
+    L, st = N.lib(), torch.cuda.current_stream().cuda_stream
+    for n, hs in ((1, (8, 64, 72, 136, 200, 264, 328, 384, 392, 456, 824)), (7, (64, 1160)), (1023, (392, 512)), (1024, (72,)), (1025, (72, 640)),
+                  (4096, (264,)), (4097, (136, 512)), (8500, (392,)), (32768, (72,)), (32769, (16, 392)), (33000, (128, 640))):
+        for h in hs:
+            print(f"no logits buffer E={E} n={n} h={h}", flush=True)
+            g = torch.Generator().manual_seed(h + E + n)
+            x = torch.randn(n, h, generator=g).to(torch.bfloat16).cuda()
+            wg = (torch.randn(E, h, generator=g) * 0.1).to(torch.bfloat16).cuda()
+            p = N.RouterParams(n, h, E, 5, 1, 1, ops.SCORE["softmax"], ops.METHOD["greedy"], 1, 0, 0, 0, 1e-20, 1.0)
+            got = []
+            for lg in (None, torch.empty(n, E, device="cuda")):
+                idx = torch.full((n, 5), -1, dtype=torch.int32, device="cuda")
+                w = torch.full((n, 5), -1.0, device="cuda")
+                N.check(L.moe_router(x.data_ptr(), wg.data_ptr(), None, ctypes.byref(p), idx.data_ptr(), w.data_ptr(),
+                                     None if lg is None else lg.data_ptr(), st), "moe_router")
+                got.append((idx, w))
+            assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]), (E, n, h)
