@@ -569,7 +569,7 @@ def moe_forward(block, hidden_states: torch.Tensor, spec: ops.RouterSpec, gate_w
         d["last_topk_idx"], d["last_topk_weight"], d["last_counts"] = idx, w, counts
         return out.view(shape), logits
     residual = None
-    if fuse is not None:                      # see norm_moe_residual: the router reads x through the norm
+    if fuse is not None:                      # see norm_moe_residual
         residual = x
         with _span(timer, "router"):
             idx, w, logits, x = ops.router(x, gw, b, spec, want_logits, norm_weight=fuse[0], eps=fuse[1])
@@ -626,8 +626,8 @@ def norm_moe_residual(block, hidden_states: torch.Tensor, norm_weight: torch.Ten
         hidden_states = mlp(hidden_states)
         hidden_states = residual + hidden_states
 
-    with the norm folded into the router's read of the rows (its normalised copy is a side output
-    that the expert GEMMs read) and the residual add folded into the combine's output pass.
+    in one call: the norm writes the rows that the router and the expert GEMMs read, and the residual add is folded
+    into the combine's output pass.
     Returns what `block(...)` returns with the new residual stream in place of the block output
     (Mixtral: a tuple with the router logits second)."""
     w = norm_weight.data if isinstance(norm_weight, torch.nn.Parameter) else norm_weight

@@ -1639,8 +1639,8 @@ __global__ __launch_bounds__(128 * WN) void grouped_gemm_kernel(GemmPair pair_of
 // bf16, 128 of fp8: whole lines) and the same k of 16 token rows (rows that do not exist cost no request), NB stages in
 // a ring.  Every matrix instruction gets the k values that the streamers above give it, in the same lanes and the same
 // order, so a row's bits are those of a larger call (fp8: of a larger call whose experts have up to 64 rows).
-// Measured (us, tile kernel -> this): DeepSeek-V2-Lite, one token (8 x 1408 of 2048) 25 + 25 and 19 + 33 -> 21 and 11;
-// DeepSeek-V3, 5 tokens (38 experts, fp8) 190 and 115 -> 171 and 88 = 6.4 TB/s.  Weights loaded into registers instead
+// Measured (us, tile kernel -> this): DeepSeek-V2-Lite, one token (8 x 1408 of 2048) 25 + 25 and 19 + 33 -> 17 and 14;
+// DeepSeek-V3, 5 tokens (39 experts, fp8) 190 and 115 -> 187 and 92 = 6.0 TB/s.  Weights loaded into registers instead
 // reach 4 ... 5 TB/s: a fragment load then takes half a line from each of 16 rows.
 template <bool SWIGLU, bool W8>
 __global__ __launch_bounds__(64) void grouped_gemm_thin_kernel(GemmPair pair_of) {
@@ -1809,9 +1809,9 @@ __global__ __launch_bounds__(64) void grouped_gemm_thin_kernel(GemmPair pair_of)
 // add_slices_kernel adds them, in order, and rounds once.  Rows past 128 are cut into tiles of equal height; all tiles of a
 // call run the same body, chosen by that height, so a row's bits do not depend on its place.  The M tiles of one piece of
 // the weights are neighbours on one XCD.
-// Measured (DeepSeek-V3's dense MLP, whole forward, us, one workgroup per tile -> this): 1 token 103 -> 79, 17: 171 -> 86,
-// 64: 203 -> 106, 128: 363 -> 174, 192: 521 -> 255, 256: 427 -> 285, 384: 471 -> 424, 512: 507 -> 441; of those the gate and up
-// products take 44, 56, 66, 113, 156, 193, 238 and 275.
+// Measured (DeepSeek-V3's dense MLP, both launches, us, without scratch -> with it): 1 token 119 -> 75, 17: 185 -> 87,
+// 64: 231 -> 115, 128: 356 -> 161, 192: 516 -> 220, 256: 426 -> 273, 384: 465 -> 402, 512: 502 -> 415; of those the gate and up
+// products take 49, 58, 76, 104, 150, 186, 232 and 273.
 __global__ __launch_bounds__(512) void grouped_gemm_split_kernel(GemmArgs g, int n_rows, SplitPlan plan, float* part) {
     __shared__ __attribute__((aligned(1024))) uint8_t lw0[S8_WBYTES];
     __shared__ __attribute__((aligned(1024))) uint8_t lw1[S8_WBYTES];

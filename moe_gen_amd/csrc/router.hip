@@ -268,10 +268,10 @@ __device__ void route_token(const float* row, const float* __restrict__ bias, co
 //    instruction brings four rows as 16 chunks of 4 x 16 bytes, and blocks of four rows lie 1088 bytes apart: the 16
 //    rows of a read fall on 64 different banks and the next k are at a constant distance.
 //  * The last stage of a hidden size that is no multiple of 128 stops after its h / 4 steps: nothing is padded.
-// Measured (DeepSeek-V3, h = 7168, logits and selection): 1 ... 256 tokens 35 ... 37 us (the chain alone at 32 cycles per
-// step and 2.4 GHz: 24), 1024: 39, 65536: 1716 = 140 TFLOP/s.  Without the LDS reads the 65536-token logits take 1587,
+// Measured (DeepSeek-V3, h = 7168, logits and selection in a loop on the same rows): 1 ... 256 tokens 35 ... 37 us (the chain
+// alone at 32 cycles per step and 2.4 GHz: 24), 1024: 37, 65536: 1716 = 140 TFLOP/s (between the other kernels of a layer 1807 + 80).  Without the LDS reads the 65536-token logits take 1587,
 // without the DMA 1674, with both 1645.  (Before, on the 4x4x1 and 32x32x1 forms, which take one k per instruction:
-// 92 ... 95, 100 and 2153 us.)
+// 92 ... 96, 96 and 2133 us.)
 // FUSED == false: the logits of the tile go to `logits` [n, E] in memory, router_select_kernel routes the tokens.
 // FUSED == true (a caller without a logits buffer): the workgroup walks the expert blocks of its tokens one after the
 // other, keeps the logits in LDS and routes the tokens itself.  Where that leaves most CUs without tokens
