@@ -176,7 +176,7 @@ int moe_dispatch_static(const int32_t* topk_idx, int32_t n_tokens, int32_t top_k
  * change the order in which a row's products are added, and with it the last bit: a call that the
  * one-workgroup-per-tile kernel serves alone starts its k loops at other stages, and there an expert of up to 64 rows
  * adds the products of a stage in another order than one of more.
- * Calls in which no expert has more than 16 rows run on a kernel of one wave per 32 weight rows.
+ * Calls in which no expert has more than 16 rows run on a kernel of one wave per 32 weight rows where that is the faster one.
  */
 enum { MOE_PHASE_GATE_UP = 1, MOE_PHASE_DOWN = 2, MOE_PHASE_BOTH = 3 };
 size_t moe_grouped_workspace_bytes(int32_t n_rows, int32_t n_experts);

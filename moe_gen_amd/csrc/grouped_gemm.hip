@@ -46,6 +46,7 @@
 // a lane ends up holding 4 consecutive output columns of one token row per accumulator;
 // the epilogue transposes them through LDS into 16-byte-per-lane row-contiguous stores.
 
+#include <cmath>
 #include <type_traits>
 
 #include "common.h"
@@ -1630,7 +1631,7 @@ __global__ __launch_bounds__(128 * WN) void grouped_gemm_kernel(GemmPair pair_of
     }
 }
 
-// ---- thin kernel: calls in which no expert has more than 16 rows (decoding a few sequences) ----
+// ---- thin kernel: calls in which no expert has more than 16 rows (decoding a few sequences), where thin_pays ----
 //
 // Such a call touches a few experts, and cut into tiles of 256 weight rows it has fewer tiles than the chip has CUs
 // (one token of DeepSeek-V2-Lite: 66) or two and a half rounds of them.  Here the unit is a WAVE with 32 weight rows --
@@ -2285,6 +2286,27 @@ int launch_split(const GemmArgs& g, int n_rows, const SplitPlan& plan, float* pa
     return MOE_OK;
 }
 
+// Whether a call in which no expert has more than 16 rows goes to the thin kernel, `shared` a second problem of the launch
+// or NULL.  Where rows are few for the number of experts it does: which experts have rows, and so how many tiles there are, is not
+// known here, and the tile kernel loses most where they fill its last round badly.  From three rows per expert on nearly all
+// have some.  Both kernels then stream the same weights, and what differs is how full their rounds are: a tile of 256 weight rows is
+// a workgroup of the tile kernel, one per CU, and 8 waves of the thin kernel, six per CU, so a round of the latter is 3/4 as many
+// tiles.  A wave's token rows cost it 1 % each; K up to 2048 costs the tile kernel 7 % around its short k loop; and with K of 8192
+// and more the tile kernel streams at the full rate from 139 of 256 tiles on, the thin one not always.  Measured (us, thin / tile):
+//   Mixtral-8x22B, 3 rows each  gate/up 474 / 466, down 279 / 234;  16 rows 526 / 480, 266 / 234;  layer, 12 tokens 687 / 675, 16: 778 / 739
+//   Mixtral-8x7B, 3 rows each   gate/up 278 / 289, down 138 / 182;  16 rows 298 / 294, 150 / 187
+//   DeepSeek-V2-236B, 4 rows    gate/up 758 / 751, down 382 / 396;  16 rows 844 / 769, 454 / 434
+//   DeepSeek-V3, 4 rows         gate/up 1128 / 1104, down 585 / 594;  16 rows 1367 / 1146, 751 / 680
+// and below three rows per expert, layers: Mixtral-8x22B, 8 tokens 408 / 461; DeepSeek-V2-236B, 6 tokens 221 / 261; V2-Lite, 16: 99 / 114.
+bool thin_pays(const GemmArgs& g, int n_rows, const GemmArgs* shared) {
+    if (n_rows < 3L * g.E) return true;
+    const double tiles = (double)g.E * g.n_tiles_n + (shared ? shared->n_tiles_n : 0);
+    const double cus = cu_count(), round = 0.75 * cus;
+    if (g.K >= 8192 && tiles <= round && tiles > 139.0 / 256 * cus) return false;
+    const double thin = std::ceil(tiles / round) * round * (1.0 + 0.01 * ((double)n_rows / g.E - 1.0));
+    return thin < std::ceil(tiles / cus) * cus * (g.K <= 2048 ? 1.07 : 1.0);
+}
+
 // max_rows: no expert has more rows (callers that do not know pass n_rows)
 template <bool SWIGLU, bool W8>
 int launch_mt(const GemmArgs& g0, int n_rows, int max_rows, void* workspace, size_t workspace_bytes, hipStream_t st) {
@@ -2295,7 +2317,7 @@ int launch_mt(const GemmArgs& g0, int n_rows, int max_rows, void* workspace, siz
         if (plan.slices > 1 && workspace_bytes >= (size_t)plan.slices * n_rows * g.N * 4)
             return launch_split(g, n_rows, plan, static_cast<float*>(workspace), st);
     }
-    if (max_rows <= 16 && gather_fits(g)) return launch_thin<SWIGLU, W8>(g, n_rows, nullptr, st);
+    if (max_rows <= 16 && gather_fits(g) && thin_pays(g, n_rows, nullptr)) return launch_thin<SWIGLU, W8>(g, n_rows, nullptr, st);
     // the persistent kernel needs an even number of k-stages for its hand-over (fp8 sizes always have
     // one), keeps per-expert tables for up to 512 experts and addresses gathered rows with 32-bit offsets
     // (below a mean of 128 rows an expert above one tile is rare and is cut into 128-row tiles where it occurs)
@@ -2338,7 +2360,7 @@ int launch_mt(const GemmArgs& g0, int n_rows, int max_rows, void* workspace, siz
 // The shared expert's tiles in the routed experts' launch.
 template <bool SWIGLU, bool W8>
 int launch_joint(const GemmArgs& routed, int n_rows, int max_rows, const GemmArgs& shared, int n_shared, hipStream_t st) {
-    if (max_rows <= 16 && n_shared <= 16) return launch_thin<SWIGLU, W8>(routed, n_rows, &shared, st);
+    if (max_rows <= 16 && n_shared <= 16 && thin_pays(routed, n_rows, &shared)) return launch_thin<SWIGLU, W8>(routed, n_rows, &shared, st);
     GemmArgs r = routed, s = shared;
     r.cold_max = s.cold_max = 0x7fffffff;
     return launch_tiles<4, SWIGLU, W8>(r, n_rows, &s, n_shared, st);

@@ -923,3 +923,29 @@ def test_fp8_weights_are_dequantised_to_bf16_at_every_row_count(n, inter):
     m.workspace, m.workspace_bytes = (ws.data_ptr(), need) if need else (None, 0)
     ops.grouped_swiglu_joint(m, None, h, True, ops.PHASE_DOWN)
     assert torch.equal(y.cpu().float(), (down[2][:, ka] - down[2][:, ka + 1]).t().to(torch.bfloat16).float())
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("E,h,I", [(8, 4608, 8192), (40, 512, 384)])     # long k and 144 tiles; short k, whole and part-filled rounds
+def test_kernel_choice_for_few_rows_leaves_the_bits(fp8, E, h, I):
+    """Calls of at most 16 rows per expert on both sides of three rows per expert, where the rounds of the thin and the tile
+    kernel begin to be compared: a row's bits are those of a call that names no bound (the tile kernel) and do not
+    depend on how many rows the others have.  All experts share one set of weights."""
+    from moe_gen_amd import ops
+    print(f"few rows fp8={fp8} E={E} h={h} I={I}", flush=True)
+    m = [t if isinstance(t, tuple) else (t,) for t in make_experts(1, h, I, fp8, 21)[0]]
+    m = [[t.cuda() for t in one] for one in m]
+    ptrs = ops.expert_pointers(*([one[0]] * E for one in m), *(([one[1]] * E for one in m) if fp8 else ()))
+    x = torch.randn(E, 16, h, generator=torch.Generator().manual_seed(22)).to(torch.bfloat16).cuda()
+
+    def call(rows, bound):
+        xs = x[:, :rows].reshape(-1, h).contiguous()
+        off = torch.arange(0, E * rows + 1, rows, dtype=torch.int32, device="cuda")
+        g, _, y = ops.mlp_group(xs, None, ptrs, off, E * rows, bound)
+        ops.grouped_swiglu_joint(g, None, h, fp8)
+        return y.view(E, rows, h)
+
+    want = call(16, 0)
+    assert want.float().abs().max() > 0
+    for rows in (1, 2, 3, 4, 16):
+        assert torch.equal(call(rows, 16), want[:, :rows]), rows
