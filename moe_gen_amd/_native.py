@@ -10,6 +10,7 @@ import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libmoe_mi355.so")
+PLACES_PATH = os.path.join(_HERE, "_places.so")
 
 c_void_p, c_int32, c_size_t, c_float, c_int64 = (ctypes.c_void_p, ctypes.c_int32, ctypes.c_size_t,
                                                  ctypes.c_float, ctypes.c_int64)
@@ -127,6 +128,21 @@ SIGNATURES = {
 }
 
 _lib = None
+_places_hold = None
+
+
+def places_hold(objects: list, tensors: list, addresses) -> bool:
+    """Whether every object of [dict, key, object, ...] is still there and every tensor of [dict, key, ...] at its address (an
+    array of 64-bit integers)."""
+    global _places_hold
+    if _places_hold is None:
+        if not os.path.exists(PLACES_PATH):
+            raise RuntimeError(f"{PLACES_PATH} is missing: build it with `make -C {os.path.join(_HERE, 'csrc')}`")
+        import torch  # noqa: F401  (its libraries are what _places.so is linked against)
+        f = ctypes.PyDLL(PLACES_PATH).moe_places_hold
+        f.argtypes, f.restype = [ctypes.py_object, ctypes.py_object, c_void_p], ctypes.c_int
+        _places_hold = f
+    return bool(_places_hold(objects, tensors, addresses.buffer_info()[0]))
 
 
 def lib() -> ctypes.CDLL:

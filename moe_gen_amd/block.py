@@ -4,11 +4,14 @@ slot, in waves when its pool is smaller than the layer) and the fused forward
 router -> dispatch -> grouped SwiGLU -> combine."""
 from __future__ import annotations
 
+import array
 import operator
+from collections import OrderedDict
 
 import torch
 from torch import nn
 
+from . import _native as N
 from . import ops
 
 FP8 = torch.float8_e4m3fn
@@ -193,14 +196,13 @@ def _attr(obj, name, default=None):
 
 class _Places:
     """Where the weights and scales of a list of experts were found: the dicts that attribute look-up came down to, so that
-    a later call can tell in a few passes of C code whether every one of them is still the tensor that the pointer tables
-    were made from (256 fp8 experts: 0.17 ms; following the attributes again takes 8 ms).  An expert that answers through
-    properties or a __getattr__ of its own is asked again, tensor by tensor."""
+    a later call can tell without following attributes (8 ms for 256 fp8 experts) whether every one of them is still
+    the tensor that the pointer tables were made from.  An expert that answers through properties or a __getattr__ of its
+    own is asked again, tensor by tensor."""
 
     def __init__(self, experts=()):
         self.experts, self.traced = list(experts), True
-        self.submodules = [], []                        # _modules dicts, and copies of them
-        self.links, self.tensors = ([], [], []), ([], [], [])      # dicts, keys, and the objects / addresses found there
+        self.objects, self.tensors, self.found = [], [], array.array("q")     # as _native.places_hold takes them
         self.kinds = {}                                 # (class, name) -> where its objects may keep it (0: they have to be asked)
 
     def note(self):
@@ -223,46 +225,28 @@ class _Places:
         if not kind:
             self.traced = False
             return getattr(obj, name, default)
-        own = obj.__dict__
-        if name in own:
-            d = own
-        elif kind == 1:
-            return self._absent(own, name, default)
-        elif name in own["_parameters"]:
-            d = own["_parameters"]
-        elif name in own["_modules"]:
-            d = own["_modules"]
-            if not self.submodules[0] or self.submodules[0][-1] is not d:
-                self.submodules[0].append(d)
-                self.submodules[1].append(d.copy())
-            return d[name]
-        elif name in own["_buffers"]:
-            d = own["_buffers"]
-        else:
-            return self._absent(own, name, default)
+        d = own = obj.__dict__
+        if name not in own:
+            for table in _MODULE_TABLES if kind == 2 else ():
+                if name in own[table]:
+                    d = own[table]
+                    break
+            else:
+                if name == "weight_dequant_scale":      # (of what an expert may lack, this can be given to it later)
+                    self.objects += own, name, None
+                return default
         value = d[name]
         if isinstance(value, torch.Tensor):
             self.tensor(d, name, value)
         else:
-            self.link(d, name, value)
+            self.objects += d, name, value
         return value
 
-    def _absent(self, own, name, default):
-        if name == "weight_dequant_scale":              # (of what an expert may lack, this can be given to it later)
-            self.link(own, name, None)
-        return default
-
     def tensor(self, d, key, value):
-        dicts, keys, found = self.tensors
-        dicts.append(d)
-        keys.append(key)
-        found.append(value.data_ptr())
-
-    def link(self, d, key, value):
-        dicts, keys, found = self.links
-        dicts.append(d)
-        keys.append(key)
-        found.append(value)
+        if type(d) not in (dict, OrderedDict):
+            self.traced = False
+        self.tensors += d, key
+        self.found.append(value.data_ptr())
 
     def ends_hold(self, experts) -> bool:
         """hold() for the first and the last tensor alone (which a block moved to another device or type does not pass)."""
@@ -270,10 +254,10 @@ class _Places:
             return self.hold(experts)
         if len(experts) != len(self.experts) or experts[0] is not self.experts[0]:
             return False
-        dicts, keys, found = self.tensors
-        first, last = dicts[0].get(keys[0]), dicts[-1].get(keys[-1])
+        t = self.tensors
+        first, last = t[0].get(t[1]), t[-2].get(t[-1])
         return (first is not None and last is not None and (first.dtype, first.shape) == self.form
-                and first.data_ptr() == found[0] and last.data_ptr() == found[-1])
+                and first.data_ptr() == self.found[0] and last.data_ptr() == self.found[-1])
 
     def hold(self, experts) -> bool:
         """Whether these are the experts noted, with every weight and scale where it was."""
@@ -281,14 +265,7 @@ class _Places:
             return False
         if not self.traced:
             return _addresses([_tensors_of(ex) for ex in experts]) == self.addresses
-        dicts, keys, found = self.links
-        if not (all(map(operator.eq, *self.submodules)) and all(map(operator.is_, map(dict.get, dicts, keys), found))):
-            return False
-        dicts, keys, found = self.tensors
-        try:
-            return list(map(torch.Tensor.data_ptr, map(operator.getitem, dicts, keys))) == found
-        except (KeyError, TypeError):                   # (a tensor was taken away)
-            return False
+        return N.places_hold(self.objects, self.tensors, self.found)
 
     def __reduce__(self):
         return _Places, ()                              # (a copy's weights are tensors of its own)
@@ -555,8 +532,8 @@ def moe_forward(block, hidden_states: torch.Tensor, spec: ops.RouterSpec, gate_w
         groups = [(experts, cache.setdefault("routed", {}))]
         if shared is not None:
             groups.append(([shared], cache.setdefault("shared", {})))
-        # The tables of the last call are used at once and held against the modules while the GPU runs (256 fp8 experts:
-        # 0.17 ms of host time); where one is out of date the call is made again.
+        # The tables of the last call are used at once and held against the modules while the GPU runs (host time, 256 fp8
+        # experts: 0.04 ms); where one is out of date the call is made again.
         kept = [_cached_pointers(*g) for g in groups]
         while True:
             tables = [t or collect_pointers(*g) for t, g in zip(kept, groups)]

@@ -459,6 +459,13 @@ def test_pointer_tables_follow_every_weight_and_scale(form, monkeypatch):
         assert new.addresses == [None if t is None else t.data_ptr() for ex in experts for t in block._tensors_of(ex)]
     twin = copy.deepcopy((experts, cache))
     assert not twin[1]["ptrs"].places.hold(twin[0])
+    meta, kept = collect_pointers(experts, cache), inner().down_proj.weight
+    inner().down_proj.weight = torch.nn.Parameter(kept.data.to("meta"), requires_grad=False)
+    assert not meta.places.hold(experts)
+    del inner().down_proj.weight
+    assert form == "property" or not meta.places.hold(experts)
+    inner().down_proj.weight = kept
+    assert meta.places.hold(experts)
     if fp8 and form not in ("own_dict", "wrapped"):
         kept = collect_pointers(experts, cache)
         experts[1].weight_dequant_scale = {n + ".weight_scale_inv": torch.ones(2, 2) for n in experts[1].names}
