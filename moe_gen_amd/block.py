@@ -194,6 +194,10 @@ def _attr(obj, name, default=None):
     return default
 
 
+_LACKS = "module", "weight_dequant_scale"                # what an ordinary MLP has nowhere
+_LINEAR = frozenset(("weight", "weight_scale_inv"))     # and what its Linears have among their parameters only
+
+
 class _Places:
     """Where the weights and scales of a list of experts were found: the dicts that attribute look-up came down to, so that
     a later call can tell without following attributes (8 ms for 256 fp8 experts) whether every one of them is still
@@ -207,11 +211,53 @@ class _Places:
 
     def note(self):
         """Follows every expert's attributes: [(gate, up, down, s_gate, s_up, s_down)]."""
-        rows = [_tensors_of(ex, None, self) for ex in self.experts]
+        rows = [self._ordinary(ex) or _tensors_of(ex, None, self) for ex in self.experts]
         self.form = rows[0][0].dtype, rows[0][0].shape
         if not self.traced:
             self.addresses = _addresses(rows)
         return rows
+
+    def _ordinary(self, mlp):
+        """What _tensors_of gives and notes, for an MLP of plain Linears whose weights and scales are parameters (None: it is
+        not one), in a third of the time: a block's first call waits for all of its experts."""
+        cls = type(mlp)
+        hidden = self.kinds.get(cls)                    # names that must not be in the MLP's __dict__
+        if hidden is None:
+            names = getattr(cls, "names", ())
+            plain = issubclass(cls, SwiGLUMLP) and cls.__getattr__ is nn.Module.__getattr__ and not any(hasattr(cls, n) for n in (*_LACKS, *names))
+            self.kinds[cls] = hidden = frozenset((*_LACKS, *names, "names")) if plain else ()
+        if not hidden:
+            return None
+        own, names = mlp.__dict__, cls.names
+        mods = own["_modules"]
+        if own["_parameters"] or own["_buffers"] or "module" in mods or not hidden.isdisjoint(own):
+            return None
+        objects, tensors, weights, scales = [], [], [], []
+        for name in names:
+            lin = mods.get(name)
+            if type(lin) is not nn.Linear or not _LINEAR.isdisjoint(lin.__dict__):
+                return None
+            params = lin.__dict__["_parameters"]
+            w = params.get("weight")
+            if w is None:
+                return None
+            objects += mods, name, lin
+            tensors += params, "weight"
+            w, s = w.data, None
+            if w.dtype is FP8:
+                s = params.get("weight_scale_inv")
+                if s is None:
+                    return None
+                tensors += params, "weight_scale_inv"
+                s = s.data
+            weights.append(w)
+            scales.append(s)
+        if weights[0].dtype is FP8:
+            objects += own, "weight_dequant_scale", None
+        self.objects += objects
+        self.tensors += tensors
+        self.found.extend([t.data_ptr() for pair in zip(weights, scales) for t in pair if t is not None])
+        return (*weights, *scales)
 
     def look(self, obj, name, default=None):
         """_attr, noting where the value lay."""
