@@ -39,12 +39,12 @@
 // operand reads are bank-conflict free.  Token rows and bf16 weights come into LDS by DMA
 // (buffer_load ... lds); fp8 weights of the persistent kernel go through registers, converted on the way,
 // two k-stages ahead, every wave interleaving its share of that with its MFMAs, one piece per group of
-// MFMAs, between the one barrier per k-stage.  gemm_tile, the register-staged body of the other kernel,
+// MFMAs, between the two barriers per k-stage.  gemm_tile, the register-staged body of the other kernel,
 // remains for calls that gather from 4 GiB of rows or more (the DMA paths address them with 32 bits).
 //
 // The MFMA is issued with the WEIGHT fragment as srcA and the TOKEN fragment as srcB, so
 // a lane ends up holding 4 consecutive output columns of one token row per accumulator;
-// the epilogue transposes them through LDS into 16-byte-per-lane row-contiguous stores.
+// the epilogues put them together, between lanes or through LDS, into 16-byte stores of row segments.
 
 #include <cmath>
 #include <type_traits>
@@ -201,6 +201,21 @@ __device__ __forceinline__ u32x2 epilogue_pack(const f32x4& a, const f32x4& up) 
         return u32x2{pack_bf16(o[0], o[1]), pack_bf16(o[2], o[3])};
     }
     return u32x2{pack_bf16(a[0], a[1]), pack_bf16(a[2], a[3])};
+}
+
+// A lane's 4 columns (8 bytes) of two neighbouring 16-column fragments of one row -> 16 consecutive bytes of that row: lane
+// group q gets columns 8 (q / 2) .. + 7 of fragment q % 2, so the four groups write 64 consecutive bytes of a row.
+__device__ __forceinline__ u32x4 pair_columns(u32x2 p0, u32x2 p1) {
+    const auto lo = __builtin_amdgcn_permlane16_swap(p0[0], p1[0], false, false);   // odd groups of p0 <-> even groups of p1
+    const auto hi = __builtin_amdgcn_permlane16_swap(p0[1], p1[1], false, false);
+    return u32x4{lo[0], hi[0], lo[1], hi[1]};
+}
+
+// 16 bytes to base + offset; an offset of 2 GiB or more stores nothing, and the instruction still counts.  AUX 2: non-temporal
+template <int AUX>
+__device__ __forceinline__ void store16(u32x4 v, const uint8_t* base, uint32_t offset) {
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, 0x7fffffff, 0x00020000);
+    __builtin_amdgcn_raw_buffer_store_b128(v, r, offset, 0, AUX);
 }
 
 // Exclusive scan of the experts' M-tile counts, tiles_of(count), by the whole workgroup: s_pref[e] = number of
@@ -1870,42 +1885,50 @@ __device__ __forceinline__ int fresh_lane() {
 
 // Persistent kernel for BM = 256: one workgroup per CU walks its share of the tiles, and the software
 // pipeline runs on across the tile boundary (a tile's last k-iterations already fetch the next tile's
-// first stages, the epilogue goes through the idle stage, and the next tile starts with its first stage
-// in LDS).  What a fresh workgroup pays per tile -- launch, tile-prefix scan, pointer chase, first fetch,
-// store drain: 6-8 us against 57 us of k loop for K = 2048 -- is paid once per workgroup or overlaps
-// the previous tile's work.
+// first stages, and the epilogue runs beside them).  What a fresh workgroup pays per tile -- launch,
+// tile-prefix scan, pointer chase, first fetch, store drain: 6-8 us against 57 us of k loop for K = 2048 --
+// is paid once per workgroup or overlaps the previous tile's work.
 //
 // Token rows (and bf16 weights) reach LDS by DMA: buffer_load_dwordx4 ... lds writes 64 lanes x 16 bytes
 // to 1 KiB of consecutive LDS, each lane fetching the 16 bytes that belong at its position of the
 // swizzled layout, so there are no staging registers, no LDS store instructions and no per-chunk load
-// waits in the MFMA stream: a wave waits once per k-iteration, before the barrier, for its own DMA of the
-// next stage.  fp8 weights still go through registers (they are converted on the way), two k-stages
-// ahead.  Three things make this worth it (the same loads issued as global_load ... lds in one array per
+// waits in the MFMA stream.  fp8 weights still go through registers (they are converted on the way), two
+// k-stages ahead.  Three things make this worth it (the same loads issued as global_load ... lds in one array per
 // stage measured 2 % slower than register staging; this form 3-5 % faster):
 //  * buffer (MUBUF) loads.  The compiler models the FLAT-encoded global_load ... lds as a possible LDS
 //    access through the flat aperture and from then on waits for ALL outstanding LDS operations
 //    (lgkmcnt(0)) wherever an operand fragment is needed, which serialises the fragment reads.
-//  * token stages and weight stages are separate LDS arrays.  An LDS store that may alias the target of
-//    an outstanding DMA gets a vmcnt(0) in front of it; the fp8 weight stores must not.
+//  * whatever a DMA fills while something else is read is an LDS array of its own.  An LDS access that may alias the
+//    target of an outstanding DMA gets a wait for it in front.
 //  * stage parities are literals (the k loop is unrolled by two), so reads of one stage provably do not
 //    alias the DMA into the other.
+//
+// What bounds it: matrix cores 81 % (bf16) and 68 % (fp8) of the cycles at 1.71 and 1.83 GHz, the chip's power limit.  A
+// stage lives in LDS for two iterations, but its pieces are read in the first half of one: replaced piece by piece
+// (`iteration` below) every DMA has one to one and a half iterations to land, where refilling a whole stage behind one barrier
+// left the last pieces half an iteration, less than a trip to L2 under load.  TFLOP/s, one barrier per iteration -> this,
+// both in one process (vendor library: 1500): bf16, one group of 65536 rows, 7168 -> 2 x 2048 1369 -> 1466, 2048 -> 7168 1344 -> 1358;
+// 8 experts, 32768 rows, 4096 <-> 14336 1258 -> 1350 and 1265 -> 1353; 160 experts, 196608 rows, 5120 <-> 1536 1177 -> 1232 and
+// 1063 -> 1142.  fp8, 64 experts, 131072 rows, 7168 <-> 2048: 1231 -> 1251 and 1182 -> 1193; there the conversion, 64 vector
+// instructions per 64 matrix instructions, is what is left (1360 and 1292 with most of it taken out).
 template <bool SWIGLU, bool W8>
 __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmArgs g) {
     constexpr int MT = 4, WN = 4;
     constexpr int NT = 128 * WN;
     constexpr int BM = 64 * MT;
-    constexpr int A_STAGE = BM * ROW_B;
+    constexpr int A_HALF = BM / 2 * ROW_B;      // half of a token stage: the first or the last 64 rows of either wave row
     constexpr int B_STAGE = BN_ROWS * ROW_B;
     constexpr int RB = NT / 4;                  // fp8: B rows per pass (rows are 4 chunks of 16 weights)
     constexpr int NB = BN_ROWS / RB;            // fp8: 16-byte global B chunks per thread per stage (2)
     constexpr int NBLK = SWIGLU ? 128 : 256;
-    constexpr int NJ = 8 / WN;
     constexpr int ND = 4;                       // DMA instructions per wave and tile half (32 rows of 128 bytes = 4 x 1 KiB)
-    // four separate arrays: the DMA writes the token stages, the fp8 path writes the weight stages with
-    // ordinary LDS stores; as separate objects the two provably do not alias (otherwise every LDS store
-    // waits for all outstanding DMA)
-    __shared__ __attribute__((aligned(1024))) uint8_t sA0[A_STAGE];
-    __shared__ __attribute__((aligned(1024))) uint8_t sA1[A_STAGE];
+    // Every piece that a DMA writes while another is read is an array of its own: as separate objects they provably do
+    // not alias (otherwise a read waits for every outstanding DMA).  The fp8 path writes the weight stages with
+    // ordinary LDS stores.
+    __shared__ __attribute__((aligned(1024))) uint8_t sA0a[A_HALF];
+    __shared__ __attribute__((aligned(1024))) uint8_t sA0b[A_HALF];
+    __shared__ __attribute__((aligned(1024))) uint8_t sA1a[A_HALF];
+    __shared__ __attribute__((aligned(1024))) uint8_t sA1b[A_HALF];
     __shared__ __attribute__((aligned(1024))) uint8_t sB0[B_STAGE];
     __shared__ __attribute__((aligned(1024))) uint8_t sB1[B_STAGE];
     __shared__ int s_pref[MAX_E + 1];
@@ -1944,11 +1967,14 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmArgs g
     // descriptor over all of x, whose size the launcher has checked against 4 GiB, so a row_map entry
     // outside x reads zeros instead of faulting.  Sorted rows: the descriptor starts at the tile's first row.
     const uint8_t *a_base = reinterpret_cast<const uint8_t*>(g.a), *a_base_n = a_base;
-    const int a_records = g.row_map ? (int)(uint32_t)g.a_bytes : -1;
-    uint32_t a_voff[ND], a_voff_n[ND];          // this wave's DMA offsets of the tile being fetched / of the next one
-    // bf16 weights also by DMA: descriptors of the expert's matrices and per-lane offsets
-    uint32_t b_voff[ND], b_voff_n[ND];
-    const uint8_t *bm_cur = nullptr, *bm_next = nullptr;   // matrix this wave's weight rows come from (gate or up / down)
+    const int a_records = SWIGLU && g.row_map ? (int)(uint32_t)g.a_bytes : -1;
+    uint32_t a_voff[ND];                        // this wave's DMA offsets of the tile being fetched
+    int a_row_n[ND];                            // and its rows of x of the next one
+    // bf16 weights also by DMA: descriptors of the expert's matrices and per-lane offsets (gate and up: rows n0 .. n0 + 127
+    // of either matrix, so one pair of offsets)
+    constexpr int NBO = SWIGLU ? 2 : 4;
+    uint32_t b_voff[ND], b_voff_n[ND];          // (NBO of them are used)
+    const uint8_t *bm0 = nullptr, *bm1 = nullptr, *bm0_n = nullptr, *bm1_n = nullptr;
     // fp8 weights through registers
     uint32_t b8_voff[NB];
     const uint8_t *b8m0 = nullptr, *b8m1 = nullptr;
@@ -1975,18 +2001,18 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmArgs g
         row_end = uni(s_off[e + 1]);
         n0 = n_tile * NBLK;
         rot_n = W8 ? 0 : k_rotation<false>(n_tile, nk);
-        // DMA instruction i of this wave fills rows 32*wave + 8*i .. +7 of a stage: lane l supplies row +l/8 and
-        // the 16 bytes that belong at physical chunk l%8, i.e. logical chunk (l%8) ^ swz(row)
+        // DMA instruction i of this wave fills rows 16*wave + 8*(i&1) .. +7 of the 128 rows of half i/2: lane l supplies
+        // row +l/8 and the 16 bytes that belong at physical chunk l%8, i.e. logical chunk (l%8) ^ swz(row).  Row r of
+        // half h of the token stage is row 128*(r/64) + 64*h + r%64 of the tile, row r of half h of the weight stage its
+        // row 128*h + r.
         const int lr = l >> 3, pc = l & 7;
 #pragma unroll
         for (int i = 0; i < ND; ++i) {
-            const int rt = 32 * wave_s + 8 * i + lr;                 // row of the tile
-            const int lc = pc ^ (lr ^ (i & 1));                       // swz(rt): rt & 7 == lr, (rt >> 3) & 1 == i & 1
+            const int rt = ((wave_s >> 2) << 7) + ((i >> 1) << 6) + 16 * (wave_s & 3) + 8 * (i & 1) + lr;   // row of the tile
             const int r = min(row0 + rt, row_end - 1);
-            const int src = g.row_map ? ((gptr_i32)(uintptr_t)g.row_map)[r] : r - row0;
-            a_voff_n[i] = (uint32_t)src * (uint32_t)(K * 2) + (uint32_t)(lc * 16);
+            a_row_n[i] = SWIGLU && g.row_map ? ((gptr_i32)(uintptr_t)g.row_map)[r] : r - row0;   // (down: sorted rows)
         }
-        if (!g.row_map) a_base_n = reinterpret_cast<const uint8_t*>(g.a) + (size_t)row0 * K * 2;
+        if (!(SWIGLU && g.row_map)) a_base_n = reinterpret_cast<const uint8_t*>(g.a) + (size_t)row0 * K * 2;
         const uint8_t* bmat0 = uni_ptr(reinterpret_cast<const void*>((uintptr_t)s_ptr[0][e]));
         const uint8_t* bmat1 = SWIGLU ? uni_ptr(reinterpret_cast<const void*>((uintptr_t)s_ptr[1][e])) : bmat0;
         if (W8) {
@@ -2003,33 +2029,41 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmArgs g
             if (SWIGLU) { srow0 = (n0 >> 7) * KB; srow1 = srow0; }
             else        { srow0 = (n0 >> 7) * KB; srow1 = min((n0 >> 7) + 1, (N >> 7) - 1) * KB; }
         } else {
-            // rows 32*wave .. +31 of the weight tile: waves 0-3 the first 128 rows (gate), 4-7 the second (up)
-            bm_next = (SWIGLU && wave_s >= 4) ? bmat1 : bmat0;
+            bm0_n = bmat0; bm1_n = bmat1;
 #pragma unroll
-            for (int i = 0; i < ND; ++i) {
-                const int rt = 32 * wave_s + 8 * i + lr;
+            for (int i = 0; i < NBO; ++i) {
+                const int n = n0 + 128 * (i >> 1) + 16 * wave_s + 8 * (i & 1) + lr;
                 const int lc = pc ^ (lr ^ (i & 1));
-                const int n = SWIGLU ? (n0 + (rt & 127)) : (n0 + rt);
                 b_voff_n[i] = (uint32_t)min(n, N - 1) * (uint32_t)(K * 2) + (uint32_t)(lc * 16);
             }
         }
     };
     auto adopt = [&]() {   // the next tile's DMA coordinates become the current ones
+        // (the row loads are waited for here, half an iteration after they were issued, not where they are issued: such a wait
+        // covers every older DMA)
+        const int l = fresh_lane(), lr = l >> 3;
 #pragma unroll
-        for (int i = 0; i < ND; ++i) { a_voff[i] = a_voff_n[i]; if (!W8) b_voff[i] = b_voff_n[i]; }
-        if (!W8) bm_cur = bm_next;
+        for (int i = 0; i < ND; ++i)             // swz(row): row & 7 == lr, (row >> 3) & 1 == i & 1
+            a_voff[i] = (uint32_t)a_row_n[i] * (uint32_t)(K * 2) + (uint32_t)(((l & 7) ^ lr ^ (i & 1)) << 4);
+        if (!W8) {
+#pragma unroll
+            for (int i = 0; i < NBO; ++i) b_voff[i] = b_voff_n[i];
+            bm0 = bm0_n; bm1 = bm1_n;
+        }
         a_base = a_base_n;
         rot = rot_n;
     };
-    auto dma_a = [&](uint8_t* stA, int kt, int i) {
+    auto dma_a = [&](int st, int kt, int i) __attribute__((always_inline)) {
+        uint8_t* d = st ? (i >= 2 ? sA1b : sA1a) : (i >= 2 ? sA0b : sA0a);
         const __amdgpu_buffer_rsrc_t rsrcA = __builtin_amdgcn_make_buffer_rsrc((void*)a_base, 0, a_records, 0x00020000);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrcA, (lds_u8)(stA + (32 * wave_s + 8 * i) * ROW_B), 16, a_voff[i],
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrcA, (lds_u8)(d + (16 * wave_s + 8 * (i & 1)) * ROW_B), 16, a_voff[i],
                                                  (uint32_t)((W8 ? kt : stage_of(kt, rot)) * BK * 2), 0, 0);
     };
-    auto dma_b = [&](uint8_t* stB, int kt, int i) {
-        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)bm_cur, 0, -1, 0x00020000);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_u8)(stB + (32 * wave_s + 8 * i) * ROW_B), 16, b_voff[i],
-                                                 (uint32_t)((W8 ? kt : stage_of(kt, rot)) * BK * 2), 0, 0);
+    auto dma_b = [&](int st, int kt, int i) __attribute__((always_inline)) {
+        uint8_t* d = st ? sB1 : sB0;
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)((SWIGLU && i >= 2) ? bm1 : bm0), 0, -1, 0x00020000);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_u8)(d + (128 * (i >> 1) + 16 * wave_s + 8 * (i & 1)) * ROW_B), 16,
+                                                 b_voff[SWIGLU ? (i & 1) : i], (uint32_t)(stage_of(kt, rot) * BK * 2), 0, 0);
     };
     // fp8 weight path (registers): thread t owns row t/4 (+128 i), chunks 2q, 2q+1 of the bf16 row
     const int brow = tid >> 2;
@@ -2053,142 +2087,195 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmArgs g
         const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)(uintptr_t)sc, 0, -1, 0x00020000);
         return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, 0, idx * 4, 0));
     };
-    auto gload_b = [&](int kt) {
-        const size_t kofs = (size_t)kt * BK;
-#pragma unroll
-        for (int i = 0; i < NB; ++i) rb[i] = load_b8(i, (uint32_t)kofs);
-        rs[0] = load_scale(sc0, srow0 + (kt >> 1));
-        rs[1] = load_scale(sc1, srow1 + (kt >> 1));
-    };
-    auto store_b_all = [&](uint8_t* Bs) {
-#pragma unroll
-        for (int i = 0; i < NB; ++i) {
-            u32x4 l, h;
-            dequant16(rb[i], rs[i / (NB / 2)], l, h);
-            *reinterpret_cast<u32x4*>(Bs + b_lds[0] + i * RB * ROW_B) = b_swap ? h : l;
-            *reinterpret_cast<u32x4*>(Bs + b_lds[1] + i * RB * ROW_B) = b_swap ? l : h;
-        }
+    auto load_chunk = [&](int b, int kt) {      // chunk b of stage kt and its block scale: two loads
+        rb[b] = load_b8(b, (uint32_t)(kt * BK));
+        if (b / (NB / 2) == 0) rs[0] = load_scale(sc0, srow0 + (kt >> 1));
+        else rs[1] = load_scale(sc1, srow1 + (kt >> 1));
     };
     auto b_item = [&](int it, uint8_t* Bs, int kn) {   // it in 0 .. 2*NB-1: half it%2 of chunk it/2
         const int b = it >> 1, half = it & 1;
         const u32x4 o = dequant8(rb[b][2 * half], rb[b][2 * half + 1], rs[b / (NB / 2)]);
         *reinterpret_cast<u32x4*>(Bs + ((half ^ (b_swap ? 1 : 0)) ? b_lds[1] : b_lds[0]) + b * RB * ROW_B) = o;
-        if (half == 1) {
-            rb[b] = load_b8(b, (uint32_t)(kn * BK));
-            if (b / (NB / 2) == 0) rs[0] = load_scale(sc0, srow0 + (kn >> 1));
-            else rs[1] = load_scale(sc1, srow1 + (kn >> 1));
-        }
+        if (half == 1) load_chunk(b, kn);
     };
 
     const int frow = lane & 15, fquad = lane >> 4, fkey = swz(frow);
     const int fchunk = ((fquad & 1) << 1) | (fquad >> 1);
-    constexpr int TM = 2 * MT, TN = 2 * NJ;
-    uint32_t tok_off[TM], w_off[TN];
-    fragment_rows<MT, TN, SWIGLU>(wm, wn, frow, tok_off, w_off);
+    constexpr int TM = 2 * MT, TN = 4;
+    // operand rows: fragment row = base + lane % 16; tokens: 64 rows of either half per wave row; weights: TN fragments
+    // of 16 rows, for SWIGLU the first half from the gate rows and the second from the matching up rows
+    const uint32_t t_rd = (uint32_t)((wm * 64 + frow) * ROW_B);
+    const uint32_t w_rd = (uint32_t)((wn * (SWIGLU ? 32 : 64) + frow) * ROW_B);
+    auto w_row = [](int j) { return SWIGLU ? (j < TN / 2 ? 0 : 128) + 16 * (j % (TN / 2)) : 16 * j; };
+    const uint32_t coff[2] = {(uint32_t)((fchunk ^ fkey) << 4), (uint32_t)(((4 + fchunk) ^ fkey) << 4)};
     f32x4 acc[TM][TN];
-    constexpr int TQ = MT / 2;
-    constexpr int NP = TM / TQ;
-    constexpr int NU = 2 * NP;
-    bf16x8 wfr[2][TN], tq[2][TQ];
-    auto read_w1 = [&](const uint8_t* Bs, int s, int j) {
-        const uint32_t coff = (uint32_t)(((4 * s + fchunk) ^ fkey) << 4);
-        wfr[s][j] = *reinterpret_cast<const bf16x8*>(Bs + w_off[j] + coff);
-    };
-    auto read_tq = [&](const uint8_t* As, int u) {
-        const int s = u / NP, q = u % NP;
-        const uint32_t coff = (uint32_t)(((4 * s + fchunk) ^ fkey) << 4);
+    // A stage is multiplied in 8 sub-phases: token part q = u/2 (two 16-row tiles of the wave's 128 rows) x 32-wide
+    // k-step s = u%2.  Slot v of an iteration issues the matrix instructions of sub-phase v - 2 and requests the
+    // operands of sub-phase v.
+    bf16x8 wfr[2][TN], tq[2][2];
+    auto read_w = [&](const uint8_t* Bs, int s) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < TQ; ++i) tq[u & 1][i] = *reinterpret_cast<const bf16x8*>(As + tok_off[q * TQ + i] + coff);
+        for (int j = 0; j < TN; ++j) wfr[s][j] = *reinterpret_cast<const bf16x8*>(Bs + w_rd + w_row(j) * ROW_B + coff[s]);
     };
-    auto mfma_sub = [&](int u) {
-        const int s = u / NP, q = u % NP;
+    auto read_tq = [&](int st, int u) __attribute__((always_inline)) {
+        const int q = u >> 1, s = u & 1;
+        const uint8_t* As = st ? (q >= 2 ? sA1b : sA1a) : (q >= 2 ? sA0b : sA0a);
 #pragma unroll
-        for (int i = 0; i < TQ; ++i)
+        for (int i = 0; i < 2; ++i) tq[u & 1][i] = *reinterpret_cast<const bf16x8*>(As + t_rd + (32 * (q & 1) + 16 * i) * ROW_B + coff[s]);
+    };
+    auto mfma_sub = [&](int u, bool zero) __attribute__((always_inline)) {
+        const int q = u >> 1, s = u & 1;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
 #pragma unroll
             for (int jx = 0; jx < TN; ++jx) {
                 const int j = ((i + u) & 1) ? TN - 1 - jx : jx;
-                acc[q * TQ + i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wfr[s][j], tq[u & 1][i], acc[q * TQ + i][j], 0, 0, 0);
+                const f32x4 c = zero && s == 0 ? f32x4{0} : acc[q * 2 + i][j];
+                acc[q * 2 + i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wfr[s][j], tq[u & 1][i], c, 0, 0, 0);
             }
     };
-    constexpr int WPS = TN / NP;
-    // iteration kt multiplies stage par; the DMA brings k-stage ka (of the tile whose coordinates are current) into
-    // the other token stage (and weight stage, bf16); fp8 converts the weight registers (k-stage kt+1) into the other
-    // weight stage and refills them with k-stage kb
-    // Vector-memory operations a wave issues per k-iteration AFTER its DMA of the next stage; they may stay in flight
-    // at the iteration's barrier: the fp8 weight chunks (NB buffer loads) and their two block scales (buffer loads).
-    constexpr int VM_TAIL = W8 ? NB + 2 : 0;
-    auto iteration = [&](int kt, int ka, int kb, int par) {
-        const uint8_t* rdA = par ? sA1 : sA0; const uint8_t* rdB = par ? sB1 : sB0;
-        uint8_t* wrA = par ? sA0 : sA1; uint8_t* wrB = par ? sB0 : sB1;
+    // Iteration kt multiplies stage kt out of buffer par.  Two barriers: behind the first every wave has left stage
+    // kt - 1, whose weights and second half of the token rows are replaced (by stage kt + 1); the first four slots
+    // read all of a stage's weights and the first half of its token rows, and behind the second barrier those are
+    // replaced in turn, by stage kt + 2.
+    //   bf16: slots 0-3 bring weights 2, 3 and tokens 2, 3 of stage k1 (= kt + 1), slots 4-7 tokens 0, 1 and weights 0, 1 of
+    //   stage k2 (= kt + 2).  fp8: slots 0, 1 tokens 2, 3 of stage k1; slots 2-5 convert the weight registers (stage kt + 1)
+    //   into the other weight buffer and refill them with stage k2; slots 6, 7 tokens 0, 1 of stage k2.
+    // Waits: the counter retires in issue order.  VM_X: operations issued after the last one that the first four slots
+    // read; VM_Y: after the last one that the others read; S: the stores of an epilogue, which lie in between in a tile's first
+    // iteration (the first tile, which has none in front, finds everything landed).  Operations the compiler adds only make
+    // the waits stricter.
+    // first / second: the tile's first two iterations (sub-phases 6 and 7 of the first run in the second); turn: from the second
+    // half on the DMA belongs to the next tile.
+    constexpr int VM_X = W8 ? 8 : 6, VM_Y = W8 ? 10 : 8;
+    constexpr int S = SWIGLU ? 8 : 16;
+    auto iteration = [&](int k1, int k2, int par, auto first, auto second, auto turn) __attribute__((always_inline)) {
+        constexpr bool FIRST = decltype(first)::value, SECOND = decltype(second)::value;
+        const uint8_t* rdB = par ? sB1 : sB0;
+        uint8_t* wrB = par ? sB0 : sB1;
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(VM_X + (FIRST ? S : 0)) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
 #pragma unroll
-        for (int v = 0; v < NU; ++v) {
-            if (v < ND) {
-                dma_a(wrA, ka, v);
-                if (!W8) dma_b(wrB, ka, v);
-            } else if (W8) {
-                b_item(v - ND, wrB, kb);
+        for (int v = 0; v < 8; ++v) {
+            if (v == 4) {
+                if (turn) adopt();
+                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(VM_Y + (FIRST ? S : 0)) : "memory");
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
             }
-            if (!W8) __builtin_amdgcn_sched_barrier(0);
-            if (v >= 2) mfma_sub(v - 2);
-            else if (kt > 0) mfma_sub(NU - 2 + v);
-            read_tq(rdA, v);
-            if (v == 0) {
+            if (W8) {
+                if (v < 2) dma_a(par ^ 1, k1, v + 2);
+                else if (v < 4) b_item(v - 2, wrB, k2);
+                else if (v < 6) b_item(v - 2, wrB, k2);
+                else dma_a(par, k2, v - 6);
+            } else {
+                if (v < 2) dma_b(par ^ 1, k1, v + 2);
+                else if (v < 4) dma_a(par ^ 1, k1, v);
+                else if (v < 6) dma_a(par, k2, v - 4);
+                else dma_b(par, k2, v - 6);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (v >= 2) mfma_sub(v - 2, FIRST);
+            else if (!FIRST) mfma_sub(6 + v, SECOND);
+            read_tq(par, v);
+            if (v < 2) read_w(rdB, v);
+            // (fp8: two vector instructions of the conversion behind every matrix instruction, which hides them; in a clump
+            // in front the waves of a SIMD, in step, leave the matrix core idle.  Gate and up 1226 -> 1251 TFLOP/s; the down
+            // projection, whose registers hold less, runs the same either way and is left to the compiler)
+            if (W8 && SWIGLU && v >= 2 && v < 6) {
 #pragma unroll
-                for (int j = 0; j < TN; ++j) read_w1(rdB, 0, j);
-            } else if (v >= 2 && v < 2 + NP) {
-#pragma unroll
-                for (int j = (v - 2) * WPS; j < (v - 1) * WPS; ++j) read_w1(rdB, 1, j);
+                for (int i = 0; i < 8; ++i) {
+                    __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x2, 2, 0);
+                }
             }
             __builtin_amdgcn_sched_barrier(0);
         }
-        // this wave's DMA has landed (the younger loads are the fp8 weight chunks and scales), then everybody's
-        asm volatile("s_waitcnt vmcnt(%0)" :: "n"(VM_TAIL) : "memory");
-        __syncthreads();
     };
-    static_assert(NU == 8 && ND == 4 && (!W8 || NB == 2), "slot plan");
+    static_assert(ND == 4 && (!W8 || NB == 2), "slot plan");
     // ---- tiles ----
     setup(tile_of(slot));
     adopt();
+    // prologue: what the iterations before the first would have issued, all of it landed (the scheduler orders it as it likes)
 #pragma unroll
-    for (int i = 0; i < ND; ++i) { dma_a(sA0, 0, i); if (!W8) dma_b(sB0, 0, i); }
+    for (int i = 0; i < ND; ++i) { dma_a(0, 0, i); if (!W8) dma_b(0, 0, i); }
+    dma_a(1, 1, 0); dma_a(1, 1, 1);
     if (W8) {
-        gload_b(0);
-        store_b_all(sB0);
-        gload_b(1);
+        load_chunk(0, 0);
+        load_chunk(1, 0);
+#pragma unroll
+        for (int it = 0; it < 4; ++it) b_item(it, sB0, 1);
+    } else {
+        dma_b(1, 1, 0); dma_b(1, 1, 1);
     }
-    asm volatile("s_waitcnt vmcnt(%0)" :: "n"(VM_TAIL) : "memory");   // (all but gload_b(1)'s NB + 2 loads)
-    __syncthreads();
+    __builtin_amdgcn_s_waitcnt(0x0f70);     // vmcnt(0), as an instruction that the compiler's own count knows
     constexpr int CW = SWIGLU ? 8 * TN : 16 * TN;    // output columns of this wave
     for (;;) {
         const int out_row0 = row0, out_row_end = row_end, out_n0 = n0;
-#pragma unroll
-        for (int mi = 0; mi < TM; ++mi)
-#pragma unroll
-            for (int j = 0; j < TN; ++j) acc[mi][j] = f32x4{0};
         bool more = false;
-        for (int kt = 0; kt + 2 <= nk - 2; kt += 2) {
-            iteration(kt, kt + 1, kt + 2, 0);
-            iteration(kt + 1, kt + 2, kt + 3, 1);
+        auto next_tile = [&]() {
+            slot += slots;
+            more = tile_of(slot) < total;
+            setup(tile_of(more ? slot : slot - slots));
+        };
+        constexpr std::true_type yes{};
+        constexpr std::false_type no{};
+        const bool only = nk == 2;               // (the first pair is the last one: not a copy of its own)
+        if (only) next_tile();
+        iteration(1, only ? 0 : 2, 0, yes, no, only);
+        iteration(only ? 0 : 2, only ? 1 : 3, 1, no, yes, no);
+        if (!only) {
+            for (int kt = 2; kt < nk - 2; kt += 2) {
+                iteration(kt + 1, kt + 2, 0, no, no, no);
+                iteration(kt + 2, kt + 3, 1, no, no, no);
+            }
+            next_tile();
+            iteration(nk - 1, 0, 0, no, no, yes);
+            iteration(0, 1, 1, no, no, no);
         }
-        slot += slots;
-        more = tile_of(slot) < total;
-        setup(tile_of(more ? slot : slot - slots));
-        iteration(nk - 2, nk - 1, more ? 0 : nk - 1, 0);
-        adopt();
-        iteration(nk - 1, more ? 0 : nk - 1, more ? 1 : nk - 1, 1);
-        mfma_sub(NU - 2);
-        mfma_sub(NU - 1);
-
-        // epilogue: stage 0 already holds the next tile; stage 1 is idle until the next tile's first iteration writes
-        // it, so each wave transposes through its 8 KiB slice of stage 1 (64 or 128 rows at a time).  The lane id is
-        // produced here, so that nothing derived from it stays live through the k loop.
-        const int ncol0 = out_n0 + wn * CW;
-        store_wave_outputs<MT, TN, SWIGLU, 8192 / (CW * 2), !SWIGLU>(
-            acc, ((wave_s < 4) ? sA1 : sB1) + (wave_s & 3) * 8192, fresh_lane(),
-            g.c + (size_t)(out_row0 + wm * 32 * MT) * N + ncol0, N, min(BM, out_row_end - out_row0) - wm * 32 * MT, N - ncol0);
-        if (!more) return;
-        __syncthreads();
+        // Epilogue.  A lane holds 4 consecutive columns (8 bytes) of one row per accumulator.  Gate and up: a wave has 32
+        // columns, 64 bytes of a row; neighbouring lane groups exchange halves and store them from the registers.  Down: 64
+        // columns, a whole 128-byte line of a row, put together in LDS, 16 rows at a time, in the wave's 2 KiB of the one piece
+        // of a stage that no DMA writes before the next tile's first barrier.
+        if (!SWIGLU) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // every wave has read that piece
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+        }
+        mfma_sub(6, false);
+        mfma_sub(7, false);
+        {
+            const int l = fresh_lane();
+            const int fr = l & 15, q = l >> 4;
+            const int rows_here = min(BM, out_row_end - out_row0) - wm * 128, ncol0 = out_n0 + wn * CW;
+            const uint8_t* out = uni_ptr(g.c + (size_t)(out_row0 + wm * 128) * N + ncol0);
+            uint8_t* ep = sA1b + wave_s * 2048;
+#pragma unroll
+            for (int mi = 0; mi < TM; ++mi) {
+                if (SWIGLU) {
+                    const u32x4 o = pair_columns(epilogue_pack<true>(acc[mi][0], acc[mi][2]), epilogue_pack<true>(acc[mi][1], acc[mi][3]));
+                    const int r = 16 * mi + fr, col = 16 * (q & 1) + 8 * (q >> 1);
+                    store16<0>(o, out, r < rows_here && ncol0 + col < N ? (uint32_t)(r * N + col) * 2u : 0x80000000u);
+                } else {
+#pragma unroll
+                    for (int jj = 0; jj < 2; ++jj) {
+                        const u32x4 o = pair_columns(epilogue_pack<false>(acc[mi][2 * jj], acc[mi][2 * jj]),
+                                                     epilogue_pack<false>(acc[mi][2 * jj + 1], acc[mi][2 * jj + 1]));
+                        *reinterpret_cast<u32x4*>(ep + fr * 128 + (((4 * jj + 2 * (q & 1) + (q >> 1)) ^ (fr & 7)) << 4)) = o;
+                    }
+#pragma unroll
+                    for (int ps = 0; ps < 2; ++ps) {
+                        const int rr = 8 * ps + (l >> 3), r = 16 * mi + rr, col = 8 * (l & 7);
+                        const u32x4 o = *reinterpret_cast<const u32x4*>(ep + rr * 128 + (((l & 7) ^ (rr & 7)) << 4));
+                        store16<2>(o, out, r < rows_here && ncol0 + col < N ? (uint32_t)(r * N + col) * 2u : 0x80000000u);
+                    }
+                }
+            }
+        }
+        if (!more) break;
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no DMA may land in LDS after the workgroup has gone
 }
 
 // shared: the second problem of the launch (NULL: none), of n_shared rows

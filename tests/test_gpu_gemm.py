@@ -194,6 +194,17 @@ def test_rounds_of_the_persistent_kernel_and_its_last_tiles(fp8, I, counts):
 
 
 @pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("h,I", [(128, 1280), (256, 1280), (384, 1280), (512, 1280), (2560, 128), (2688, 256), (2560, 384)])
+def test_persistent_kernel_turns_between_tiles_at_short_k(fp8, h, I):
+    """More tiles than CUs at 2, 4, 6 and 8 stages of 64 k (gate/up: h; down projection: I), so that workgroups go on from
+    tile to tile where a tile's first pair of stages is also its last, or its last but one; 2688: half a column tile at
+    the end.  Ragged row counts, gathered rows.  Against the oracle."""
+    print(f"turns fp8={fp8} h={h} I={I}", flush=True)
+    y, ref32, refr = run_case(5, h, I, [1100, 2047, 1500, 1793, 1750], fp8, seed=97, use_row_map=True)
+    assert np.isfinite(y).all() and rel_max(y, ref32) <= TOL and rel_max(y, refr) <= TOL
+
+
+@pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("counts", [[300, 640, 129, 70], [2100, 1700], [40, 3, 77]])
 def test_a_row_does_not_depend_on_its_place_in_its_expert(fp8, counts):
     """The same rows in another order within every expert give the same output rows, bit for bit, whichever kernel
