@@ -1907,10 +1907,10 @@ __device__ __forceinline__ int fresh_lane() {
 // stage lives in LDS for two iterations, but its pieces are read in the first half of one: replaced piece by piece
 // (`iteration` below) every DMA has one to one and a half iterations to land, where refilling a whole stage behind one barrier
 // left the last pieces half an iteration, less than a trip to L2 under load.  TFLOP/s, one barrier per iteration -> this,
-// both in one process (vendor library: 1500): bf16, one group of 65536 rows, 7168 -> 2 x 2048 1369 -> 1466, 2048 -> 7168 1344 -> 1358;
-// 8 experts, 32768 rows, 4096 <-> 14336 1258 -> 1350 and 1265 -> 1353; 160 experts, 196608 rows, 5120 <-> 1536 1177 -> 1232 and
-// 1063 -> 1142.  fp8, 64 experts, 131072 rows, 7168 <-> 2048: 1231 -> 1251 and 1182 -> 1193; there the conversion, 64 vector
-// instructions per 64 matrix instructions, is what is left (1360 and 1292 with most of it taken out).
+// both in one process (vendor library: 1520, 1428): bf16, one group of 65536 rows, 7168 -> 2 x 2048 1392 -> 1498, 2048 -> 7168
+// 1378 -> 1396; 8 experts, 32768 rows, 4096 <-> 14336 1273 -> 1383 and 1277 -> 1390; 160 experts, 196608 rows, 5120 <-> 1536
+// 1190 -> 1271 and 1076 -> 1164.  fp8, 64 experts, 131072 rows, 7168 <-> 2048: 1259 -> 1282 and 1201 -> 1217; there the
+// conversion, 64 vector instructions per 64 matrix instructions, is what is left (a tenth more with most of it taken out).
 template <bool SWIGLU, bool W8>
 __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmArgs g) {
     constexpr int MT = 4, WN = 4;
@@ -2081,8 +2081,7 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmArgs g
         return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, b8_voff[i], kofs, 0));
     };
     // Block scales come through buffer loads too, although their address is the same for every lane: as loads
-    // through a pointer the compiler would be free to make them scalar loads, and the hand-written vmcnt
-    // immediates below count them as vector-memory operations.
+    // through a pointer they could become scalar loads, which share a counter with the operand reads and return out of order.
     auto load_scale = [&](gptr_f32 sc, int idx) {
         const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)(uintptr_t)sc, 0, -1, 0x00020000);
         return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, 0, idx * 4, 0));
@@ -2141,26 +2140,28 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmArgs g
     //   bf16: slots 0-3 bring weights 2, 3 and tokens 2, 3 of stage k1 (= kt + 1), slots 4-7 tokens 0, 1 and weights 0, 1 of
     //   stage k2 (= kt + 2).  fp8: slots 0, 1 tokens 2, 3 of stage k1; slots 2-5 convert the weight registers (stage kt + 1)
     //   into the other weight buffer and refill them with stage k2; slots 6, 7 tokens 0, 1 of stage k2.
-    // Waits: the counter retires in issue order.  VM_X: operations issued after the last one that the first four slots
-    // read; VM_Y: after the last one that the others read; S: the stores of an epilogue, which lie in between in a tile's first
-    // iteration (the first tile, which has none in front, finds everything landed).  Operations the compiler adds only make
-    // the waits stricter.
+    // Waits.  DMA into LDS retires in issue order, but loads into registers issued after it may retire before it (counted as in
+    // order, a DMA's rows were now and then read before they had landed, gathered ones first), and nothing is known of
+    // stores: the waits count DMA operations only, so whatever else is in flight makes them stricter.  VM_X: DMA
+    // issued after the last one that the first four slots read; VM_Y: after the last one that the others read; VM_TURN: after a
+    // tile's first stage, waited for in front of the stores of the tile before, so that the first iteration need not wait.
     // first / second: the tile's first two iterations (sub-phases 6 and 7 of the first run in the second); turn: from the second
     // half on the DMA belongs to the next tile.
-    constexpr int VM_X = W8 ? 8 : 6, VM_Y = W8 ? 10 : 8;
-    constexpr int S = SWIGLU ? 8 : 16;
+    constexpr int VM_X = W8 ? 4 : 6, VM_Y = W8 ? 4 : 8, VM_TURN = W8 ? 2 : 4;
     auto iteration = [&](int k1, int k2, int par, auto first, auto second, auto turn) __attribute__((always_inline)) {
         constexpr bool FIRST = decltype(first)::value, SECOND = decltype(second)::value;
         const uint8_t* rdB = par ? sB1 : sB0;
         uint8_t* wrB = par ? sB0 : sB1;
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(VM_X + (FIRST ? S : 0)) : "memory");
+        if (FIRST) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(VM_X) : "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
 #pragma unroll
         for (int v = 0; v < 8; ++v) {
             if (v == 4) {
                 if (turn) adopt();
-                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(VM_Y + (FIRST ? S : 0)) : "memory");
+                if (FIRST) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(VM_Y) : "memory");
                 __builtin_amdgcn_s_barrier();
                 asm volatile("" ::: "memory");
             }
@@ -2245,6 +2246,8 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmArgs g
         }
         mfma_sub(6, false);
         mfma_sub(7, false);
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_waitcnt vmcnt(%0)" :: "n"(VM_TURN) : "memory");
         {
             const int l = fresh_lane();
             const int fr = l & 15, q = l >> 4;
