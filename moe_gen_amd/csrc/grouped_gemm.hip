@@ -27,7 +27,7 @@
 //    leave over if that is at most 192 rows; work that mostly streams weights): one
 //    workgroup per tile, grid = upper bound on the tile count, surplus workgroups exit at once;
 //    the tile height (16 ... 192 rows in steps of 16) follows the expert, groups of 4 tiles go round-robin
-//    to the XCDs.  Its tiles run through the weight streamers (stream16_tile, stream8x_tile, stream8w_tile, stream8_tile):
+//    to the XCDs.  Its tiles run through the weight streamers (stream16_tile, stream8x_tile, stream8_tile):
 //    weights AND token rows reach LDS by DMA, three weight buffers, one barrier per stage.
 //
 // Workgroup = 8 waves, two per SIMD.  v_mfma_f32_16x16x32_bf16 throughout: on real (non-zero) data this
@@ -695,6 +695,12 @@ struct SBuf {
     uint8_t *w, *t;
 };
 
+// LDS of a workgroup of the tile kernel or of the split kernel, an array each: three weight buffers of 32 KiB, token buffers of
+// 16, 24 (split kernel: 16) and 16 KiB
+struct TileLds {
+    uint8_t *w0, *w1, *w2, *t0, *t1, *t2;
+};
+
 // How the split kernel cuts one problem: row tiles of `rows`, k into `slices` of up to `blocks` blocks of 128
 struct SplitPlan {
     int m_tiles, rows, slices, blocks;
@@ -884,177 +890,259 @@ __device__ __forceinline__ void stream8_tile(const GemmArgs& g, SBuf buf0, SBuf 
 }
 
 
-// ---- fp8 weight streamer in the persistent kernel's summation order: tiles of up to 128 rows ----
+// ---- fp8 weight streamer in the persistent kernel's summation order: tiles of up to 192 rows ----
 //
 // The same division of labour as stream8_tile (8 waves x 32 weight rows, fp8 weights by DMA in whole lines, every wave
-// multiplies all token rows), for tiles whose rows another kernel might have computed: what an fp8 expert's full
-// 256-row tiles leave over, the halves of the persistent kernel's last tiles, and in calls that this kernel serves
-// alone the experts (or 128-row slices of experts) above 64 rows.  A row's bits must then not depend on who computes
-// it, so every matrix instruction gets the k values the persistent kernel gives it, in the same lanes: lane group q
-// holds k = 32 s + 8 f(q) + (0..7) of k-step s, f = 0, 2, 1, 3.  Those are 8 consecutive fp8 weights, one half of a
-// 16-byte part (read whole; the weights are a ninth of the LDS reads), and the 16-byte token chunk 4 s + f(q) of a
-// 64-k half.  128 token rows x 128 k would not fit LDS three times over next to the weights, so token rows travel in
-// halves of 64 k (128 rows x 128 bytes = 16 KiB) through three buffers of their own, one barrier per half, while the
-// weights keep their three buffers of 128 k: 96 + 48 KiB.  Per half-block a wave issues 2 weight DMA instructions (of
-// the block two ahead) and 2 token DMA instructions (of the half two ahead), and the wait before a half's barrier
-// leaves the 4 of the half before in flight.  k starts at block 0 unless the kernel has the call to itself.
-template <int TG, bool SWIGLU, bool SPLIT = false>   // TG: 16-row token groups multiplied (1 .. 8)
-__device__ __forceinline__ void stream8x_tile(const GemmArgs& g, SBuf b0, SBuf b1, SBuf b2, int e, int row0, int row_end,
-                                              int n_tile, bool rotate, KSlice ks = {}) {
+// multiplies all token rows, a weight is converted once, by the wave that multiplies it), for tiles whose rows another
+// kernel might have computed: what an fp8 expert's full 256-row tiles leave over, the halves of the persistent kernel's last
+// tiles, and in calls that this kernel serves alone the experts (or 128-row slices of experts) above 64 rows.  A row's bits
+// must then not depend on who computes it, so every matrix instruction gets the k values the persistent kernel gives it,
+// in the same lanes: lane group q holds k = 32 s + 8 f(q) + (0..7) of k-step s, f = 0, 2, 1, 3.  Those are 8 consecutive
+// fp8 weights, one half of a 16-byte part (read whole; the lane group two further on uses the other half, a broadcast, where
+// 8-byte reads of every other half collide), and the 16-byte token chunk 4 s + f(q) of a 64-k half.
+//
+// Weights travel in blocks of 128 k through three buffers, token rows in halves of 64 k with one barrier per half: up to 128
+// rows through three buffers of 16 KiB, two halves ahead, above through two of 24 KiB (one is two arrays), one half ahead.
+// A wave brings and reads its own weight rows, so only token rows need the barrier.
+//
+// The k loop is a pipeline of slots, one per k-step of 32 and part of at most 4 token groups.  Slot n multiplies part n - 2,
+// requests the token operands of part n, and converts its share of the weights of the step after the one that is multiplied, so
+// the LDS latency and the conversion stand beside matrix instructions instead of in front of them.  Slots run on across
+// the barriers; in front of the first one operands and accumulators are zero.
+//
+// What bounds it: the chip's power.  It runs at 1.7 to 1.8 GHz, and a half of 16 KiB of weights takes 1075 cycles and 126 more
+// for every 16 token rows: the stream and the products add up (96 / 176 rows: matrix cores 42 / 57 %, vector ALU 36 / 28 % of the
+// cycles).  Against one form each for up to 128 and up to 192 rows, in which every half read, converted and multiplied
+// in turn, DeepSeek-V3 shapes, 256 experts, us: 96 rows each 1913 -> 1861 (gate and up), 1091 -> 1055 (down), 176 rows
+// 2782 -> 2583 and 1566 -> 1468; 512 rows each (leftovers of full tiles) 6144 -> 6082, 3247 -> 3226 for 64 experts.
+template <int TG, bool SWIGLU, bool SPLIT = false>   // TG: 16-row token groups multiplied (1 .. 12)
+__device__ __forceinline__ void stream8x_tile(const GemmArgs& g, const TileLds& lds, int e, int row0, int row_end, int n_tile,
+                                              bool rotate, KSlice ks = {}) {
     constexpr int NBLK = SWIGLU ? 128 : 256;
-    constexpr int VM_HALF = 4;                    // DMA instructions per wave and half-block: 2 weights + 2 tokens
+    constexpr bool WIDE = TG > 8;                 // two token buffers
+    constexpr int NP = (TG + 3) / 4;              // parts of a k-step
+    constexpr int V = 2 * NP;                     // slots of a half
+    constexpr int NDT = (2 * TG + 7) / 8;         // token DMA instructions per wave and half (8 rows each)
+    constexpr int NS = SWIGLU ? 2 : 1;            // block scales of a wave's columns
+    // Order of issue in half h of block p: the tokens two halves ahead (above 128 rows: one), h = 0: the scales of block p + 1, and
+    // the weights of block p + 2 (all four instructions in h = 0; above 128 rows two in either half).  VM: DMA operations that may
+    // stay in flight at the barrier of a half, those issued after its tokens.  (The scales do not count: loads into registers
+    // may retire before older DMA, see the persistent kernel)
+    constexpr int VM = WIDE ? 2 : 4 + NDT;
     static_assert(!(SPLIT && SWIGLU), "slices of k: the down projection");
-    static_assert(TG >= 1 && TG <= 8, "token rows staged");
+    static_assert(TG >= 1 && TG <= 12, "token rows staged");
     const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
     const int n0 = n_tile * NBLK;
     const int K = g.K, N = g.N;
     const int npair = SPLIT ? ks.count : K >> 7;             // blocks of 128 k multiplied
     const int kfirst = SPLIT ? ks.first : 0;
     const int prot = rotate ? n_tile % npair : 0;             // k_rotation in blocks of 128 k
+    auto block_of = [&](int p_pipe) { const int pr = min(p_pipe, npair - 1) + prot; return pr >= npair ? pr - npair : pr; };
 
     // ---- DMA coordinates ----
     // weights, instruction i (0..3): rows 8 i + lane / 8 of the wave's 32 (fragment i / 2, fragment row 8 (i & 1) + lane / 8);
     // 16-byte part c of fragment row r at part c ^ wsw(r)
     const int lr = lane >> 3, pp = lane & 7;
-    uint32_t w_voff[4];
+    uint32_t w_voff[4], t_voff[3];                // (NDT of the latter are used)
     const uint8_t* bmat[2];
-    cptr_f32 sc[2];
-    int srow[2];
+    const uint8_t* sc[2];
+    int srow = 0;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         bmat[j] = uni_ptr((SWIGLU && j == 1) ? g.b1[e] : g.b0[e]);
-        sc[j] = (cptr_f32)(uintptr_t)uni_ptr((SWIGLU && j == 1) ? g.s1[e] : g.s0[e]);
-        srow[j] = min((n0 + (SWIGLU ? 0 : 32 * wave)) >> 7, (N >> 7) - 1) * (K >> 7) + kfirst;
+        sc[j] = uni_ptr((SWIGLU && j == 1) ? g.s1[e] : g.s0[e]);
     }
+    srow = min((n0 + (SWIGLU ? 0 : 32 * wave)) >> 7, (N >> 7) - 1) * (K >> 7) + kfirst;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int fr = 8 * (i & 1) + lr;
         const int rt = SWIGLU ? 16 * wave + fr : 32 * wave + 16 * (i >> 1) + fr;      // row of the tile's N range
         w_voff[i] = (uint32_t)min(n0 + rt, N - 1) * (uint32_t)K + (uint32_t)((pp ^ wsw(fr)) << 4);
     }
-    // tokens, instruction i (0..1): rows 16 wave + 8 i + lane / 8 of the 128 staged, 16-byte chunk c of row r at chunk
-    // c ^ swz(r) (the persistent kernel's layout of a 64-k stage).  Rows past the tile's last: zeros, no request.
-    uint32_t t_voff[2];
+    // tokens, instruction i: rows 64 i + 8 wave + lane / 8, 16-byte chunk c of row r at chunk c ^ swz(r) (the persistent
+    // kernel's layout of a 64-k stage).  Rows past the tile's last: zeros, no request.
     const uint8_t* a_base = reinterpret_cast<const uint8_t*>(g.a) + (g.row_map ? (size_t)0 : (size_t)row0 * K * 2);
     const int a_records = g.row_map ? (int)(uint32_t)g.a_bytes : (row_end - row0) * K * 2;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int tr = 16 * wave + 8 * i + lr;
+    for (int i = 0; i < NDT; ++i) {
+        const int tr = 64 * i + 8 * wave + lr;
         const int r = min(row0 + tr, row_end - 1);
         const int src = g.row_map ? ((gptr_i32)(uintptr_t)g.row_map)[r] : r - row0;
         t_voff[i] = (uint32_t)src * (uint32_t)(K * 2) + (uint32_t)((pp ^ swz(tr)) << 4);
         if (row0 + tr >= row_end || (g.row_map && (unsigned)src >= (unsigned)g.a_rows)) t_voff[i] = 0xfffffff0u;
     }
-    float rsc[2][2];                              // block scales of the block being multiplied / of the next one
-    auto scales = [&](int p_pipe, int set) {      // scalar loads (uniform addresses in the constant address space)
-        int pr = min(p_pipe, npair - 1) + prot;
-        pr = pr >= npair ? pr - npair : pr;
+    float rsc[3][2];                              // block scales, block p in set p % 3
+    auto scales = [&](int p_pipe, int set) __attribute__((always_inline)) {   // (buffer loads: the waits count them)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) rsc[set][j] = sc[j][srow[j] + pr];
+        for (int j = 0; j < NS; ++j) {
+            const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)sc[j], 0, -1, 0x00020000);
+            rsc[set][j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, 0, (srow + block_of(p_pipe)) * 4, 0));
+        }
     };
-    // weight DMA instruction i of block p_pipe (pipeline order) / token DMA instruction i of half-block hb_pipe
-    auto dma_w = [&](int p_pipe, SBuf buf, int i) __attribute__((always_inline)) {
+    // weight DMA instruction i of block p_pipe (pipeline order) / token DMA instruction i of half-block hb_pipe, into token
+    // buffer tb
+    auto dma_w = [&](int p_pipe, uint8_t* wb, int i) __attribute__((always_inline)) {
         const int live = uni(p_pipe < npair ? -1 : 0);   // past the end: an empty descriptor, zeros without a request
-        int pr = min(p_pipe, npair - 1) + prot;
-        pr = pr >= npair ? pr - npair : pr;
         const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)bmat[i >> 1], 0, live, 0x00020000);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_u8)(buf.w + wave * 4096 + i * 1024), 16, w_voff[i], (uint32_t)((pr + kfirst) * 128), 0, 2);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_u8)(wb + wave * 4096 + i * 1024), 16, w_voff[i],
+                                                 (uint32_t)((block_of(p_pipe) + kfirst) * 128), 0, 2);
     };
-    auto dma_t = [&](int hb_pipe, SBuf buf, int i) __attribute__((always_inline)) {
+    auto dma_t = [&](int hb_pipe, int tb, int i) __attribute__((always_inline)) {
         const int live = uni(hb_pipe < 2 * npair ? -1 : 0);
         const int hb = min(hb_pipe, 2 * npair - 1);
-        int pr = (hb >> 1) + prot;
-        pr = pr >= npair ? pr - npair : pr;
+        uint8_t* d = WIDE ? (tb == 0 ? lds.t1 + i * 8192 : i < 2 ? lds.t0 + i * 8192 : lds.t2)
+                          : (tb == 0 ? lds.t0 : tb == 1 ? lds.t1 : lds.t2) + i * 8192;
         const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)a_base, 0, live & a_records, 0x00020000);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_u8)(buf.t + wave * 2048 + i * 1024), 16, t_voff[i],
-                                                 (uint32_t)((pr + kfirst) * 256 + (hb & 1) * 128), 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_u8)(d + wave * 1024), 16, t_voff[i],
+                                                 (uint32_t)((block_of(hb >> 1) + kfirst) * 256 + (hb & 1) * 128), 0, 0);
     };
 
-    const int frow = lane & 15, q = lane >> 4;
-    const int fq = ((q & 1) << 1) | (q >> 1);
+    // ---- operands ----
+    const int frow = lane & 15, q4 = lane >> 4;
+    const int fq = ((q4 & 1) << 1) | (q4 >> 1);
     // weights: the 8 bytes at 32 s + 8 f(q) of the 64-byte half h of fragment row frow: 16-byte part 4 h + 2 s + f(q) / 2
     const uint32_t w_rd = (uint32_t)(wave * 4096 + frow * 128), wkey = (uint32_t)wsw(frow);
     const uint32_t t_rd = (uint32_t)(frow * 128), tkey = (uint32_t)swz(frow);   // (group bases are multiples of 16 rows)
     f32x4 acc[TG][2];
+    bf16x8 tf[2][4], wa[2][2];
+    u32x4 raw[2] = {u32x4{0}, u32x4{0}};
 #pragma unroll
     for (int t = 0; t < TG; ++t) { acc[t][0] = f32x4{0}; acc[t][1] = f32x4{0}; }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) tf[0][t] = tf[1][t] = __builtin_bit_cast(bf16x8, u32x4{0});
+#pragma unroll
+    for (int j = 0; j < 2; ++j) wa[0][j] = wa[1][j] = __builtin_bit_cast(bf16x8, u32x4{0});
+    auto part_lo = [](int q) { return q * TG / NP; };
+    auto read_tokens = [&](int tb, int v) __attribute__((always_inline)) {      // part v % NP of step v / NP
+        const int s = v / NP, q = v % NP;
+        const uint32_t coff = (uint32_t)(((4 * s + fq) ^ tkey) << 4);
+#pragma unroll
+        for (int t = part_lo(q); t < part_lo(q + 1); ++t) {
+            const uint8_t* b = WIDE ? (tb == 0 ? lds.t1 + t * 2048 : t < 8 ? lds.t0 + t * 2048 : lds.t2 + (t - 8) * 2048)
+                                    : (tb == 0 ? lds.t0 : tb == 1 ? lds.t1 : lds.t2) + t * 2048;
+            tf[v & 1][t - part_lo(q)] = *reinterpret_cast<const bf16x8*>(b + t_rd + coff);
+        }
+    };
+    auto read_weights = [&](const uint8_t* wb, int h, int s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+            raw[j] = *reinterpret_cast<const u32x4*>(wb + w_rd + j * 2048 + (((4 * h + 2 * s + (fq >> 1)) ^ wkey) << 4));
+    };
+    auto convert = [&](int s, int part, int set) __attribute__((always_inline)) {   // share `part` of NP of raw -> wa[s]
+#pragma unroll
+        for (int u = part * 4 / NP; u < (part + 1) * 4 / NP; ++u) {              // 4 weights of fragment u / 2
+            const int j = u >> 1, d = u & 1;
+            const float scale = rsc[set][SWIGLU ? j : 0];
+            const uint32_t qv = (fq & 1) ? raw[j][2 + d] : raw[j][d];
+            const f32x2 c0 = __builtin_amdgcn_cvt_pk_f32_fp8(qv, false), c1 = __builtin_amdgcn_cvt_pk_f32_fp8(qv, true);
+            u32x4 o = __builtin_bit_cast(u32x4, wa[s][j]);
+            o[2 * d] = pack_bf16(c0[0] * scale, c0[1] * scale);
+            o[2 * d + 1] = pack_bf16(c1[0] * scale, c1[1] * scale);
+            wa[s][j] = __builtin_bit_cast(bf16x8, o);
+        }
+    };
+    auto multiply = [&](int v) __attribute__((always_inline)) {                  // part v % NP of step v / NP
+        const int s = v / NP, q = v % NP;
+#pragma unroll
+        for (int t = part_lo(q); t < part_lo(q + 1); ++t) {
+            acc[t][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[s][0], tf[v & 1][t - part_lo(q)], acc[t][0], 0, 0, 0);
+            acc[t][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[s][1], tf[v & 1][t - part_lo(q)], acc[t][1], 0, 0, 0);
+        }
+    };
 
-    // Half-block H = 2 p + h multiplies half h of block p: weights out of buffer p % 3, tokens out of token buffer
-    // H % 3.  Before it: this wave's DMA of its tokens (issued two halves ago) and of everything older has landed and
-    // its LDS reads have returned, then everybody's (a bare s_barrier).  After the barrier every wave has left half
-    // H - 1, whose token buffer takes half H + 2, and (h == 0) block p - 1, whose weight buffer takes block p + 2 over
-    // the two halves of block p.
-    auto half = [&](int p, int h, SBuf wb, SBuf tb, SBuf w_refill, SBuf t_refill, int sset) __attribute__((always_inline)) {
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(VM_HALF) : "memory");
+    // Half h of block p: weights out of wb (block p; the next block's out of w_next), tokens out of buffer tb.  Before it: this
+    // wave's DMA of its tokens and of everything older has landed and its LDS reads have returned, then everybody's (a
+    // bare s_barrier).  After the barrier every wave has left the half before, whose token buffer is t_refill, and (h == 0) this
+    // wave block p - 1, whose weight buffer is w_refill.
+    auto half = [&](int p, int h, const uint8_t* wb, const uint8_t* w_next, uint8_t* w_refill, int tb, int t_refill, int set) __attribute__((always_inline)) {
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(VM) : "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        // every operand of the half is requested up front (2 + TG reads per k-step): the matrix instructions then run
-        // behind the LDS pipeline instead of waiting out its latency one token group at a time
-        u32x2 wraw[2][2];
-        bf16x8 tf[2][TG];
 #pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2) {
+        for (int i = 0; i < NDT; ++i) dma_t(2 * p + h + (WIDE ? 1 : 2), t_refill, i);
+        if (h == 0) scales(p + 1, (set + 1) % 3);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                // (the whole 16-byte part, of which this lane group uses one half and the group two further on the
-                // other: the two read the same address in the same LDS pass, a broadcast, where 8-byte reads of
-                // every other half collide -- SQ_LDS_BANK_CONFLICT was three times the LDS instruction cycles)
-                const u32x4 part = *reinterpret_cast<const u32x4*>(wb.w + w_rd + j * 2048 + (((4 * h + 2 * s2 + (fq >> 1)) ^ wkey) << 4));
-                wraw[s2][j] = (fq & 1) ? u32x2{part[2], part[3]} : u32x2{part[0], part[1]};
+        for (int v = 0; v < V; ++v) {
+            const int s = v / NP, mq = (v + V - 2) % NP;       // step of this slot, part that it multiplies
+            multiply((v + V - 2) % V);
+            read_tokens(tb, v);
+            // the step after the one that is multiplied: its share of the conversion
+            if (NP == 1) convert(s ^ 1, 0, h == 0 && v == 0 ? (set + 2) % 3 : set);
+            else if (NP == 2 || mq) convert(s, mq, set);
+            else convert(s ^ 1, 0, h == 1 && s == 1 ? (set + 1) % 3 : set);
+            if (NP == 1) read_weights(wb, h, s);
+            else if (mq == NP - 1) read_weights(s == 0 || h == 0 ? wb : w_next, s == 0 ? h : h ^ 1, s ^ 1);
+            // the weights of block p + 2: behind the first slots of the half
+            if (!WIDE && h == 0) {
+                if (V == 2) { dma_w(p + 2, w_refill, 2 * v); dma_w(p + 2, w_refill, 2 * v + 1); }
+                else dma_w(p + 2, w_refill, v);
             }
-            const uint32_t coff = (uint32_t)(((4 * s2 + fq) ^ tkey) << 4);
-#pragma unroll
-            for (int t = 0; t < TG; ++t) tf[s2][t] = *reinterpret_cast<const bf16x8*>(tb.t + t_rd + t * 16 * 128 + coff);
+            if (WIDE && v < 2) dma_w(p + 2, w_refill, 2 * h + v);
+            __builtin_amdgcn_sched_barrier(0);
         }
-#pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2) {
-            bf16x8 wa[2];
-#pragma unroll
-            for (int j = 0; j < 2; ++j) wa[j] = __builtin_bit_cast(bf16x8, dequant8(wraw[s2][j][0], wraw[s2][j][1], rsc[sset][j]));
-#pragma unroll
-            for (int t = 0; t < TG; ++t) {
-                acc[t][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[0], tf[s2][t], acc[t][0], 0, 0, 0);
-                acc[t][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[1], tf[s2][t], acc[t][1], 0, 0, 0);
-            }
-            dma_w(p + 2, w_refill, 2 * h + s2);
-            dma_t(2 * p + h + 2, t_refill, s2);
-        }
-        // (the next block's scales: scalar loads, issued where no LDS read is outstanding -- the two share a counter
-        // and scalar loads return out of order, which would turn every operand wait into a full drain)
-        if (h == 0) scales(p + 1, sset ^ 1);
     };
-    // Prologue: blocks 0 and 1 and halves 0 and 1, the tokens of half 0 before the weights of block 1, so that the
-    // first half's wait (all but the 4 youngest instructions) covers what it reads, as in the steady state.
-    scales(0, 0);
+    // Prologue: what the halves before the first would have issued, in their order
+    if (WIDE) scales(0, 0);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) dma_w(0, b0, i);
+    for (int i = 0; i < 4; ++i) dma_w(0, lds.w0, i);
+    __builtin_amdgcn_sched_barrier(0);
+    if (WIDE) {
+        dma_w(1, lds.w1, 0); dma_w(1, lds.w1, 1);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int i = 0; i < 2; ++i) dma_t(0, b0, i);
+        for (int i = 0; i < NDT; ++i) dma_t(0, 0, i);
+        __builtin_amdgcn_sched_barrier(0);
+        dma_w(1, lds.w1, 2); dma_w(1, lds.w1, 3);
+    } else {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) dma_w(1, b1, i);
+        for (int i = 0; i < NDT; ++i) dma_t(0, 0, i);
+        __builtin_amdgcn_sched_barrier(0);
+        scales(0, 0);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int i = 0; i < 2; ++i) dma_t(1, b1, i);
-    // Six halves = three blocks bring both rotations back to where they started: literal buffers in the loop body.
+        for (int i = 0; i < 4; ++i) dma_w(1, lds.w1, i);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < NDT; ++i) dma_t(1, 1, i);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (NP > 1) {
+        asm volatile("s_waitcnt vmcnt(%0)" :: "n"(VM) : "memory");     // this wave's weights of block 0
+        read_weights(lds.w0, 0, 0);
+    }
+    if (NP == 3) convert(0, 0, 0);
+    rsc[2][0] = rsc[2][1] = 0.0f;
+    // Six halves = three blocks bring the rotations back to where they started: literal buffers in the loop body.
+    uint8_t *const w0 = lds.w0, *const w1 = lds.w1, *const w2 = lds.w2;
+    constexpr int T1 = 1, T2 = WIDE ? 0 : 2, T3 = WIDE ? 1 : 0, T4 = WIDE ? 0 : 1, T5 = WIDE ? 1 : 2;   // token buffers of halves 1 .. 5
+    auto refill = [](int b) { return WIDE ? b ^ 1 : (b + 2) % 3; };
     int p = 0;
     for (; p + 3 <= npair; p += 3) {
-        half(p, 0, b0, b0, b2, b2, 0);
-        half(p, 1, b0, b1, b2, b0, 0);
-        half(p + 1, 0, b1, b2, b0, b1, 1);
-        half(p + 1, 1, b1, b0, b0, b2, 1);
-        half(p + 2, 0, b2, b1, b1, b0, 0);
-        half(p + 2, 1, b2, b2, b1, b1, 0);
-        const float t0 = rsc[0][0], t1 = rsc[0][1];
-        rsc[0][0] = rsc[1][0]; rsc[0][1] = rsc[1][1];
-        rsc[1][0] = t0; rsc[1][1] = t1;
+        half(p, 0, w0, w1, w2, 0, refill(0), 0);
+        half(p, 1, w0, w1, w2, T1, refill(T1), 0);
+        half(p + 1, 0, w1, w2, w0, T2, refill(T2), 1);
+        half(p + 1, 1, w1, w2, w0, T3, refill(T3), 1);
+        half(p + 2, 0, w2, w0, w1, T4, refill(T4), 2);
+        half(p + 2, 1, w2, w0, w1, T5, refill(T5), 2);
     }
     if (p < npair) {
-        half(p, 0, b0, b0, b2, b2, 0);
-        half(p, 1, b0, b1, b2, b0, 0);
+        half(p, 0, w0, w1, w2, 0, refill(0), 0);
+        half(p, 1, w0, w1, w2, T1, refill(T1), 0);
         if (p + 1 < npair) {
-            half(p + 1, 0, b1, b2, b0, b1, 1);
-            half(p + 1, 1, b1, b0, b0, b2, 1);
+            half(p + 1, 0, w1, w2, w0, T2, refill(T2), 1);
+            half(p + 1, 1, w1, w2, w0, T3, refill(T3), 1);
         }
     }
+    multiply(V - 2);
+    if (NP == 1) {                                // (the step after the last slot's: the last block's scales)
+        const int rem = npair % 3;
+        if (rem == 1) convert(1, 0, 0);
+        else if (rem == 2) convert(1, 0, 1);
+        else convert(1, 0, 2);
+    }
+    multiply(V - 1);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no DMA may land in LDS after the workgroup has gone
 
     // ---- epilogue: a lane holds 4 consecutive columns of one row per accumulator and stores them itself ----
@@ -1063,192 +1151,18 @@ __device__ __forceinline__ void stream8x_tile(const GemmArgs& g, SBuf b0, SBuf b
         const int r = row0 + 16 * t + frow;
         if (r >= row_end) continue;
         if (SWIGLU) {
-            const int col = n0 + 16 * wave + 4 * q;
+            const int col = n0 + 16 * wave + 4 * q4;
             if (col < N) *reinterpret_cast<u32x2*>(g.c + (size_t)r * N + col) = epilogue_pack<true>(acc[t][0], acc[t][1]);
         } else {
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
-                const int col = n0 + 32 * wave + 16 * j + 4 * q;
+                const int col = n0 + 32 * wave + 16 * j + 4 * q4;
                 if (col >= N) continue;
                 if (SPLIT) *reinterpret_cast<f32x4*>(ks.part + (size_t)(r - ks.row_base) * N + col) = acc[t][j];
                 else *reinterpret_cast<u32x2*>(g.c + (size_t)r * N + col) = epilogue_pack<false>(acc[t][j], acc[t][j]);
             }
         }
     }
-}
-
-// ---- fp8 weight streamer in the persistent kernel's summation order: tiles of 129 to 192 rows ----
-//
-// stream8x_tile for 9 to 12 groups of 16 token rows: what an fp8 expert's full 256-row tiles leave over when that is
-// more than 128 rows (as a padded 256-row tile of the persistent kernel such rows cost a third to a half more matrix
-// work than they hold), and experts of that size in calls that this kernel serves alone.  Same weight DMA and LDS
-// layouts, the same division of labour (a weight is converted once, by the wave that multiplies it: with two sets of
-// 4 waves over the token groups, as in the bf16 streamer, every weight is converted twice, and the conversion then
-// takes the vector ALU as long as the products take the matrix cores -- DeepSeek-V3 at 4096 tokens 4.52 against 4.31
-// ms), same k values in the same lanes.  What differs: such a tile is bound by the matrix cores, not by the weight
-// stream, and 192 token rows x 64 k are 24 KiB, so there are two weight buffers, the next block requested right
-// after a block's first barrier (a block of 128 k takes the matrix cores about 2 us, more than a trip to memory), and
-// two token buffers, one per half of a block, each refilled right after the barrier that retires it, one half ahead
-// (token rows come out of L2).
-// Before a block's first half everything this wave requested must have landed (vmcnt 0); before its second half all
-// but the 4 weight instructions of the next block, which were issued behind that half's token rows.
-template <int TG, bool SWIGLU>   // TG: 16-row token groups multiplied (9 .. 12)
-__device__ __forceinline__ void stream8w_tile(const GemmArgs& g, uint8_t* w0, uint8_t* w1, uint8_t* t0, uint8_t* t1, int e,
-                                              int row0, int row_end, int n_tile, bool rotate) {
-    constexpr int NBLK = SWIGLU ? 128 : 256;
-    constexpr int NF = 2;                         // 16-row weight fragments per wave
-    constexpr int NDT = (2 * TG + 7) / 8;         // token DMA instructions per wave and half (8 rows each)
-    static_assert(TG >= 9 && TG <= 12 && NDT == 3, "token rows staged");
-    const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
-    const int n0 = n_tile * NBLK;
-    const int K = g.K, N = g.N;
-    const int npair = K >> 7;
-    const int prot = rotate ? n_tile % npair : 0;             // k_rotation in blocks of 128 k
-
-    // ---- DMA coordinates (weights as in stream8x_tile: wave w brings LDS rows 32 w .. 32 w + 31, fragments 2 w, 2 w + 1) ----
-    const int lr = lane >> 3, pp = lane & 7;
-    uint32_t w_voff[4], t_voff[NDT];
-    const uint8_t* bmat[2];
-    cptr_f32 sc[2];
-    int srow[2];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        bmat[j] = uni_ptr((SWIGLU && j == 1) ? g.b1[e] : g.b0[e]);
-        sc[j] = (cptr_f32)(uintptr_t)uni_ptr((SWIGLU && j == 1) ? g.s1[e] : g.s0[e]);
-        srow[j] = min((n0 + (SWIGLU ? 0 : 32 * wave)) >> 7, (N >> 7) - 1) * npair;
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int fr = 8 * (i & 1) + lr;
-        const int rt = SWIGLU ? 16 * wave + fr : 32 * wave + 16 * (i >> 1) + fr;      // row of the tile's N range
-        w_voff[i] = (uint32_t)min(n0 + rt, N - 1) * (uint32_t)K + (uint32_t)((pp ^ wsw(fr)) << 4);
-    }
-    const uint8_t* a_base = reinterpret_cast<const uint8_t*>(g.a) + (g.row_map ? (size_t)0 : (size_t)row0 * K * 2);
-    const int a_records = g.row_map ? (int)(uint32_t)g.a_bytes : (row_end - row0) * K * 2;
-#pragma unroll
-    for (int i = 0; i < NDT; ++i) {               // token rows 64 i + 8 wave + lr; rows past the tile's last: zeros, no request
-        const int tr = 64 * i + 8 * wave + lr;
-        const int r = min(row0 + tr, row_end - 1);
-        const int src = g.row_map ? ((gptr_i32)(uintptr_t)g.row_map)[r] : r - row0;
-        t_voff[i] = (uint32_t)src * (uint32_t)(K * 2) + (uint32_t)((pp ^ swz(tr)) << 4);
-        if (row0 + tr >= row_end || (g.row_map && (unsigned)src >= (unsigned)g.a_rows)) t_voff[i] = 0xfffffff0u;
-    }
-    float rsc[2][2];                              // block scales of the block being multiplied / of the next one
-    auto block_of = [&](int p_pipe) { int pr = min(p_pipe, npair - 1) + prot; return pr >= npair ? pr - npair : pr; };
-    auto scales = [&](int p_pipe, int set) {      // scalar loads (uniform addresses in the constant address space)
-        const int pr = block_of(p_pipe);
-#pragma unroll
-        for (int j = 0; j < 2; ++j) rsc[set][j] = sc[j][srow[j] + pr];
-    };
-    auto dma_w = [&](int p_pipe, uint8_t* wb, int i) __attribute__((always_inline)) {
-        const int live = uni(p_pipe < npair ? -1 : 0);   // past the end: an empty descriptor, zeros without a request
-        const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)bmat[i >> 1], 0, live, 0x00020000);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_u8)(wb + wave * 4096 + i * 1024), 16, w_voff[i], (uint32_t)(block_of(p_pipe) * 128), 0, 2);
-    };
-    auto dma_t = [&](int hb_pipe, uint8_t* tb, int i) __attribute__((always_inline)) {
-        const int live = uni(hb_pipe < 2 * npair ? -1 : 0);
-        const int hb = min(hb_pipe, 2 * npair - 1);
-        const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)a_base, 0, live & a_records, 0x00020000);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_u8)(tb + (64 * i + 8 * wave) * 128), 16, t_voff[i],
-                                                 (uint32_t)(block_of(hb >> 1) * 256 + (hb & 1) * 128), 0, 0);
-    };
-
-    // ---- operand coordinates: a wave multiplies the two fragments it brought ----
-    const int frow = lane & 15, q = lane >> 4;
-    const int fq = ((q & 1) << 1) | (q >> 1);
-    const uint32_t wkey = (uint32_t)wsw(frow), tkey = (uint32_t)swz(frow);
-    const uint32_t w_rd = (uint32_t)(wave * 4096 + frow * 128), t_rd = (uint32_t)(frow * 128);
-    f32x4 acc[TG][NF];
-#pragma unroll
-    for (int t = 0; t < TG; ++t)
-#pragma unroll
-        for (int f = 0; f < NF; ++f) acc[t][f] = f32x4{0};
-
-    // Half h of block p: weights out of wb (block p), token rows out of tb (half 2 p + h).
-    auto half = [&](int p, int h, const uint8_t* wb, const uint8_t* tb, uint8_t* w_refill, uint8_t* t_refill, int sset) __attribute__((always_inline)) {
-        if (h == 0) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        // every wave has left half 2 p + h - 1 (its token buffer takes half 2 p + h + 1) and, h == 0, block p - 1 (its
-        // weight buffer takes block p + 1)
-#pragma unroll
-        for (int i = 0; i < NDT; ++i) dma_t(2 * p + h + 1, t_refill, i);
-        if (h == 0) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) dma_w(p + 1, w_refill, i);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        u32x2 wraw[2][NF];
-        bf16x8 tf[2][TG];
-#pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2) {
-#pragma unroll
-            for (int f = 0; f < NF; ++f) {
-                // (the whole 16-byte part, of which this lane group uses one half and the group two further on the other)
-                const u32x4 part = *reinterpret_cast<const u32x4*>(wb + w_rd + f * 2048 + (((4 * h + 2 * s2 + (fq >> 1)) ^ wkey) << 4));
-                wraw[s2][f] = (fq & 1) ? u32x2{part[2], part[3]} : u32x2{part[0], part[1]};
-            }
-            const uint32_t coff = (uint32_t)(((4 * s2 + fq) ^ tkey) << 4);
-#pragma unroll
-            for (int t = 0; t < TG; ++t) tf[s2][t] = *reinterpret_cast<const bf16x8*>(tb + t_rd + t * 16 * 128 + coff);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2) {
-            bf16x8 wa[NF];
-#pragma unroll
-            for (int f = 0; f < NF; ++f)
-                wa[f] = __builtin_bit_cast(bf16x8, dequant8(wraw[s2][f][0], wraw[s2][f][1], rsc[sset][f]));
-#pragma unroll
-            for (int t = 0; t < TG; ++t)
-#pragma unroll
-                for (int f = 0; f < NF; ++f) acc[t][f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[f], tf[s2][t], acc[t][f], 0, 0, 0);
-        }
-        // (the next block's scales: scalar loads, issued where no LDS read is outstanding)
-        if (h == 0) scales(p + 1, sset ^ 1);
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    scales(0, 0);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) dma_w(0, w0, i);
-#pragma unroll
-    for (int i = 0; i < NDT; ++i) dma_t(0, t0, i);
-    // Two blocks bring the weight buffers and the scale sets back to where they started: literal buffers in the loop body.
-    int p = 0;
-    for (; p + 2 <= npair; p += 2) {
-        half(p, 0, w0, t0, w1, t1, 0);
-        half(p, 1, w0, t1, w1, t0, 0);
-        half(p + 1, 0, w1, t0, w0, t1, 1);
-        half(p + 1, 1, w1, t1, w0, t0, 1);
-    }
-    if (p < npair) {
-        half(p, 0, w0, t0, w1, t1, 0);
-        half(p, 1, w0, t1, w1, t0, 0);
-    }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no DMA may land in LDS after the workgroup has gone
-
-    // ---- epilogue: a lane holds 4 consecutive columns of one row per accumulator and stores them itself ----
-#pragma unroll
-    for (int t = 0; t < TG; ++t) {
-        const int r = row0 + 16 * t + frow;
-        if (r >= row_end) continue;
-#pragma unroll
-        for (int f = 0; f < (SWIGLU ? 1 : NF); ++f) {
-            const int col = n0 + (SWIGLU ? 16 : 32) * wave + 16 * f + 4 * q;
-            if (col < N) *reinterpret_cast<u32x2*>(g.c + (size_t)r * N + col) = epilogue_pack<SWIGLU>(acc[t][f], acc[t][SWIGLU ? 1 : f]);
-        }
-    }
-}
-
-template <bool SWIGLU>
-__device__ __forceinline__ void stream8w(const GemmArgs& g, uint8_t* w0, uint8_t* w1, uint8_t* t0, uint8_t* t1, int e, int row0,
-                                         int row_end, int n_tile, bool rotate) {
-    const int rows = row_end - row0;
-    if (rows <= 144) stream8w_tile<9, SWIGLU>(g, w0, w1, t0, t1, e, row0, row_end, n_tile, rotate);
-    else if (rows <= 160) stream8w_tile<10, SWIGLU>(g, w0, w1, t0, t1, e, row0, row_end, n_tile, rotate);
-    else if (rows <= 176) stream8w_tile<11, SWIGLU>(g, w0, w1, t0, t1, e, row0, row_end, n_tile, rotate);
-    else stream8w_tile<12, SWIGLU>(g, w0, w1, t0, t1, e, row0, row_end, n_tile, rotate);
 }
 
 // M tiles of an expert with `count` rows in the one-workgroup-per-tile kernel: one tile of up to 192 rows if that
@@ -1489,17 +1403,14 @@ __device__ __forceinline__ void stream16(const GemmArgs& g, uint8_t* w0, uint8_t
 }
 
 template <bool SWIGLU>
-__device__ __forceinline__ void stream8x(const GemmArgs& g, SBuf b0, SBuf b1, SBuf b2, int e, int row0, int row_end, int n_tile,
-                                         bool rotate) {
-    const int rows = row_end - row0;
-    if (rows <= 16) stream8x_tile<1, SWIGLU>(g, b0, b1, b2, e, row0, row_end, n_tile, rotate);
-    else if (rows <= 32) stream8x_tile<2, SWIGLU>(g, b0, b1, b2, e, row0, row_end, n_tile, rotate);
-    else if (rows <= 48) stream8x_tile<3, SWIGLU>(g, b0, b1, b2, e, row0, row_end, n_tile, rotate);
-    else if (rows <= 64) stream8x_tile<4, SWIGLU>(g, b0, b1, b2, e, row0, row_end, n_tile, rotate);
-    else if (rows <= 80) stream8x_tile<5, SWIGLU>(g, b0, b1, b2, e, row0, row_end, n_tile, rotate);
-    else if (rows <= 96) stream8x_tile<6, SWIGLU>(g, b0, b1, b2, e, row0, row_end, n_tile, rotate);
-    else if (rows <= 112) stream8x_tile<7, SWIGLU>(g, b0, b1, b2, e, row0, row_end, n_tile, rotate);
-    else stream8x_tile<8, SWIGLU>(g, b0, b1, b2, e, row0, row_end, n_tile, rotate);
+__device__ __forceinline__ void stream8x(const GemmArgs& g, const TileLds& lds, int e, int row0, int row_end, int n_tile, bool rotate) {
+    switch ((row_end - row0 + 15) >> 4) {
+#define MOE_S8X_CASE(n) case n: stream8x_tile<n, SWIGLU>(g, lds, e, row0, row_end, n_tile, rotate); break;
+    MOE_S8X_CASE(1) MOE_S8X_CASE(2) MOE_S8X_CASE(3) MOE_S8X_CASE(4) MOE_S8X_CASE(5) MOE_S8X_CASE(6)
+    MOE_S8X_CASE(7) MOE_S8X_CASE(8) MOE_S8X_CASE(9) MOE_S8X_CASE(10) MOE_S8X_CASE(11)
+#undef MOE_S8X_CASE
+    default: stream8x_tile<12, SWIGLU>(g, lds, e, row0, row_end, n_tile, rotate); break;
+    }
 }
 
 // One workgroup per (M tile, N tile); serves what the persistent kernel does not take (few rows per expert, odd K).
@@ -1509,8 +1420,8 @@ __global__ __launch_bounds__(128 * WN) void grouped_gemm_kernel(GemmPair pair_of
     // Three weight arrays of 32 KiB and token arrays of 16 KiB (fp8 weights: three, 128 rows; the second one 24 KiB)
     // or 24 KiB (bf16: two, 192 rows) -- the buffers of the weight streamers, written by DMA, as separate objects so
     // that a read of one waits for no DMA into another; gemm_tile's two stages (up to 128 token rows + 256 weight
-    // rows) are two pairs of them.  The fp8 streamer for 129 to 192 rows has two weight buffers and keeps its token
-    // rows (24 KiB per half) in the third weight array and the 24 KiB token array.
+    // rows) are two pairs of them.  fp8 tiles of 129 to 192 rows have two token buffers, the second array and the
+    // first and third together.
     constexpr int TB = W8 ? 128 * ROW_B : 192 * ROW_B;
     __shared__ __attribute__((aligned(1024))) uint8_t lw0[S8_WBYTES];
     __shared__ __attribute__((aligned(1024))) uint8_t lw1[S8_WBYTES];
@@ -1521,6 +1432,7 @@ __global__ __launch_bounds__(128 * WN) void grouped_gemm_kernel(GemmPair pair_of
     static_assert(S8_TROWS * 256 <= 128 * ROW_B && S8_WBYTES == BN_ROWS * ROW_B, "regions of a streamer buffer");
     auto stage = [&](int i) { return Stage{i ? lt1 : lt0, i ? lw1 : lw0, i ? lw1 : lw0}; };
     const SBuf sb0{lw0, lt0}, sb1{lw1, lt1}, sb2{lw2, lt2};
+    const TileLds lds{lw0, lw1, lw2, lt0, lt1, lt2};
     __shared__ int s_pref[MAX_E + 1];
     __shared__ int s_wtot[NT / 64];
     __shared__ int s_sel[5];
@@ -1588,7 +1500,7 @@ __global__ __launch_bounds__(128 * WN) void grouped_gemm_kernel(GemmPair pair_of
         const int r0 = uni(s_sel[3]) + m_tile * 256 + half * 128;
         const int r1 = min(uni(s_sel[4]), uni(s_sel[3]) + (m_tile + 1) * 256);
         if (r0 >= r1) return;
-        if (W8 && s8_ok) stream8x<SWIGLU>(g, sb0, sb1, sb2, e, r0, r1, n_tile, false);
+        if (W8 && s8_ok) stream8x<SWIGLU>(g, lds, e, r0, min(r1, r0 + 128), n_tile, false);
         else if (s8_ok) stream16<SWIGLU, true>(g, lw0, lw1, lw2, lt0, lt1, e, r0, min(r1, r0 + 128), n_tile);
         else gemm_tile<2, WN, SWIGLU, W8, false>(g, stage(0), stage(1), e, r0, r1, n_tile);
         return;
@@ -1608,10 +1520,8 @@ __global__ __launch_bounds__(128 * WN) void grouped_gemm_kernel(GemmPair pair_of
             else if (rows <= 32) stream8_tile<2, SWIGLU>(g, sb0, sb1, sb2, e, r0, r1, n_tile);
             else if (rows <= 48) stream8_tile<3, SWIGLU>(g, sb0, sb1, sb2, e, r0, r1, n_tile);
             else stream8_tile<4, SWIGLU>(g, sb0, sb1, sb2, e, r0, r1, n_tile);
-        } else if (rows > 128) {                 // (one tile of 129 to 192 rows)
-            stream8w<SWIGLU>(g, lw0, lw1, lw2, lt1, e, r0, r1, n_tile, alone);
         } else {
-            stream8x<SWIGLU>(g, sb0, sb1, sb2, e, r0, r1, n_tile, alone);
+            stream8x<SWIGLU>(g, lds, e, r0, r1, n_tile, alone);
         }
         return;
     }
@@ -1836,6 +1746,7 @@ __global__ __launch_bounds__(512) void grouped_gemm_split_kernel(GemmArgs g, int
     __shared__ __attribute__((aligned(1024))) uint8_t lt1[128 * ROW_B];
     __shared__ __attribute__((aligned(1024))) uint8_t lt2[128 * ROW_B];
     const SBuf b0{lw0, lt0}, b1{lw1, lt1}, b2{lw2, lt2};
+    const TileLds lds{lw0, lw1, lw2, lt0, lt1, lt2};
     const int local = blockIdx.x >> 3;
     const int piece = local / plan.m_tiles * 8 + (blockIdx.x & 7), m_tile = local % plan.m_tiles;
     if (piece >= plan.slices * g.n_tiles_n) return;
@@ -1852,10 +1763,10 @@ __global__ __launch_bounds__(512) void grouped_gemm_split_kernel(GemmArgs g, int
         else if (groups == 3) stream8_tile<3, false, true>(g, b0, b1, b2, 0, r0, r1, n_tile, ks);
         else stream8_tile<4, false, true>(g, b0, b1, b2, 0, r0, r1, n_tile, ks);
     } else {
-        if (groups <= 5) stream8x_tile<5, false, true>(g, b0, b1, b2, 0, r0, r1, n_tile, true, ks);
-        else if (groups == 6) stream8x_tile<6, false, true>(g, b0, b1, b2, 0, r0, r1, n_tile, true, ks);
-        else if (groups == 7) stream8x_tile<7, false, true>(g, b0, b1, b2, 0, r0, r1, n_tile, true, ks);
-        else stream8x_tile<8, false, true>(g, b0, b1, b2, 0, r0, r1, n_tile, true, ks);
+        if (groups <= 5) stream8x_tile<5, false, true>(g, lds, 0, r0, r1, n_tile, true, ks);
+        else if (groups == 6) stream8x_tile<6, false, true>(g, lds, 0, r0, r1, n_tile, true, ks);
+        else if (groups == 7) stream8x_tile<7, false, true>(g, lds, 0, r0, r1, n_tile, true, ks);
+        else stream8x_tile<8, false, true>(g, lds, 0, r0, r1, n_tile, true, ks);
     }
 }
 

@@ -385,6 +385,17 @@ def test_fp8_weight_streamer_tiles_of_129_to_192_rows(counts, h, I):
     assert rel_max(O.bf16_to_f32(bits(ys[0])), ref) <= TOL
 
 
+@pytest.mark.parametrize("more", [[], [1100]])      # the tile kernel alone; with the persistent kernel next to it
+@pytest.mark.parametrize("h,I", [(128, 384), (256, 512), (384, 128), (640, 256)])     # 1 ... 5 blocks of 128 k
+def test_fp8_weight_streamer_every_tile_height(h, I, more):
+    """Tiles of 1 to 12 groups of 16 rows, first and last row counts of a group, at block counts around the three that a turn of
+    the k loop takes.  Against the oracle."""
+    counts = [16, 17, 33, 49, 65, 80, 81, 96, 97, 112, 113, 128, 129, 144, 145, 160, 161, 176, 177, 192] + more
+    print(f"tile heights h={h} I={I} more={more}", flush=True)
+    y, ref32, refr = run_case(len(counts), h, I, counts, True, seed=67, use_row_map=True)
+    assert np.isfinite(y).all() and rel_max(y, ref32) <= TOL and rel_max(y, refr) <= TOL
+
+
 @pytest.mark.parametrize("h,I", [(512, 640), (640, 896), (896, 512)])      # 4 / 5 / 7 blocks of 128 k (gate/up), 5 / 7 / 4 (down)
 def test_fp8_weight_streamer_shapes_and_gather(h, I):
     """The fp8 weight streamer on every token-group count and both sides of each boundary, with block counts that
