@@ -97,13 +97,14 @@ struct GemmArgs {
                                 // is left goes to the other kernel as 128-row half tiles if that pays (tail_tiles)
 };
 
-// What a launch of the one-workgroup-per-tile kernel or of the thin kernel works on: the routed experts and, in front of
-// them, the first `shared_tiles` (units) of a second problem with matrices and buffers of its own, the layer's shared
-// expert.  A launch pair for the shared expert alone has a tile for a fraction of the CUs (DeepSeek-V2-236B, 64 tokens:
-// 24 and 20 tiles, 70 + 44 us for 94 MB).
+// What a launch works on: the routed experts and, in front of them, a second problem of one expert with matrices, sizes and
+// buffers of its own, the layer's shared expert: its `shared_tiles` tiles (units) of the one-workgroup-per-tile or the thin
+// kernel, its `shared_ptiles` tiles of the persistent kernel.  A launch pair for the shared expert alone has a tile for a
+// fraction of the CUs at small batches (DeepSeek-V2-236B, 64 tokens: 24 and 20 tiles, 70 + 44 us for 94 MB) and rounds of its own
+// that end part-filled at larger ones.
 struct GemmPair {
     GemmArgs p[2];              // routed, shared
-    int shared_tiles;
+    int shared_tiles, shared_ptiles;
 };
 
 // LDS rows are 128 bytes = 8 chunks of 16 bytes; chunk c of row r is stored at chunk c ^ swz(r).
@@ -1173,10 +1174,10 @@ __device__ __forceinline__ void stream8x_tile(const GemmArgs& g, const TileLds& 
 // the weights with plain loads, so that all but the first read of a line come out of that XCD's L2.
 // 256-row tiles of an expert with `count` rows in the persistent kernel's tile space
 // whether an expert of `count` rows belongs to the one-workgroup-per-tile kernel (no rem_split)
-__device__ __forceinline__ bool is_cold(const GemmArgs& g, int count) {
+__host__ __device__ __forceinline__ bool is_cold(const GemmArgs& g, int count) {
     return count <= g.cold_max || (g.pair_rows && count >= PAIR_LO && count <= PAIR_HI);
 }
-__device__ __forceinline__ int persistent_tiles(const GemmArgs& g, int count) {
+__host__ __device__ __forceinline__ int persistent_tiles(const GemmArgs& g, int count) {
     if (g.rem_split) return (count >> 8) + ((count & 255) > g.cold_max ? 1 : 0);
     return is_cold(g, count) ? 0 : (count + 255) >> 8;
 }
@@ -1215,7 +1216,7 @@ __device__ __forceinline__ int half_rows(int count) { return ((count + 1) / 2 + 
 
 // M tiles of an expert with `count` rows in the one-workgroup-per-tile kernel's own tile space
 template <bool W8>
-__device__ __forceinline__ int own_tiles(const GemmArgs& g, int c) {
+__host__ __device__ __forceinline__ int own_tiles(const GemmArgs& g, int c) {
     if (g.rem_split) c &= 255;      // the rows the persistent kernel's full tiles leave over
     return (g.rem_split ? c > g.cold_max : !is_cold(g, c)) ? 0 : tiles_of<!W8>(c);
 }
@@ -1445,29 +1446,36 @@ __global__ __launch_bounds__(128 * WN) void grouped_gemm_kernel(GemmPair pair_of
     const int slot = blockIdx.x >> 3;
     int v = (((slot >> 2) << 3) + (blockIdx.x & 7)) * 4 + (slot & 3);
     const bool of_shared = v < pair_of.shared_tiles;
-    const GemmArgs& g = pair_of.p[of_shared ? 1 : 0];
     if (!of_shared) v -= pair_of.shared_tiles;
+    const GemmArgs* gp = &pair_of.p[of_shared ? 1 : 0];
 
     // ---- M-tile prefix over experts ----
     ExpertOfThread mine;
-    const bool s8_ok = !g.row_map || g.a_bytes < (1ull << 32);   // (the weight streamer addresses gathered rows with 32-bit offsets)
-    int run = mtile_prefix_scan<NT>(g, tid, s_pref, s_wtot, mine, [&](int c) { return own_tiles<W8>(g, c); }, [](int, int, int) {});
-    const int total = run * g.n_tiles_n;
+    int run = mtile_prefix_scan<NT>(*gp, tid, s_pref, s_wtot, mine, [&](int c) { return own_tiles<W8>(*gp, c); }, [](int, int, int) {});
+    const int total = run * gp->n_tiles_n;
 
     // Past this kernel's own tiles: the tiles that the persistent kernel leaves at the end of ITS tile space, two
     // workgroups (128-row halves, neighbours on one XCD) per tile.  The prefix is rebuilt over that space.
     int half = -1;
     if (v >= total) {
-        if (g.tail_cus <= 0 || g.E > NT) return;
+        if (of_shared || gp->tail_cus <= 0 || gp->E > NT) return;
         const int t = v - total;
         __syncthreads();                 // s_wtot of the first scan has been read by everyone
-        run = mtile_prefix_scan<NT>(g, tid, s_pref, s_wtot, mine, [&](int c) { return persistent_tiles(g, c); }, [](int, int, int) {});
-        const int total_p = run * g.n_tiles_n;
-        const int tail = tail_tiles(g, total_p, total);
+        run = mtile_prefix_scan<NT>(*gp, tid, s_pref, s_wtot, mine, [&](int c) { return persistent_tiles(*gp, c); }, [](int, int, int) {});
+        const int total_p = run * gp->n_tiles_n + pair_of.shared_ptiles;
+        const int tail = tail_tiles(*gp, total_p, total + pair_of.shared_tiles);
         if (t >= 2 * tail) return;
         v = total_p - tail + (t >> 1);
         half = t & 1;
+        if (v < pair_of.shared_ptiles) {             // the shared expert's: its one expert belongs to thread 0
+            gp = &pair_of.p[1];
+            mine = ExpertOfThread{0, tid == 0 ? pair_of.shared_ptiles / gp->n_tiles_n : 0, gp->offsets[0], gp->offsets[1]};
+        } else {
+            v -= pair_of.shared_ptiles;
+        }
     }
+    const GemmArgs& g = *gp;
+    const bool s8_ok = !g.row_map || g.a_bytes < (1ull << 32);   // (the weight streamer addresses gathered rows with 32-bit offsets)
     const int q = v / g.n_tiles_n;  // global M-tile number
     // find e with prefix[e] <= q < prefix[e+1].  Up to NT experts every thread still holds its own
     // expert's prefix, tile count and row range: the one that owns q publishes them (one barrier,
@@ -1823,7 +1831,8 @@ __device__ __forceinline__ int fresh_lane() {
 // 1190 -> 1271 and 1076 -> 1164.  fp8, 64 experts, 131072 rows, 7168 <-> 2048: 1259 -> 1282 and 1201 -> 1217; there the
 // conversion, 64 vector instructions per 64 matrix instructions, is what is left (a tenth more with most of it taken out).
 template <bool SWIGLU, bool W8>
-__global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmArgs g) {
+__global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmPair pair_of) {
+    const GemmArgs& g = pair_of.p[0];            // the routed experts; the tiles of the second problem come first
     constexpr int MT = 4, WN = 4;
     constexpr int NT = 128 * WN;
     constexpr int BM = 64 * MT;
@@ -1846,7 +1855,8 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmArgs g
     __shared__ int s_wtot[NT / 64];
     constexpr int PE = 512;
     __shared__ int s_off[PE + 1];
-    __shared__ unsigned long long s_ptr[4][PE];
+    __shared__ unsigned long long s_ptr[4][PE + 1];        // (the last column: the second problem's)
+    __shared__ int s_off1[2];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wave_s = uni(wave);
@@ -1862,23 +1872,31 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmArgs g
         s_ptr[2][e] = W8 ? (unsigned long long)(uintptr_t)g.s0[e] : 0ull;
         s_ptr[3][e] = (W8 && SWIGLU) ? (unsigned long long)(uintptr_t)g.s1[e] : 0ull;
     });
+    const int ptiles1 = pair_of.shared_ptiles;
     if (tid == 0) s_pref[g.E] = run;
+    if (ptiles1 > 0 && tid == 0) {
+        const GemmArgs& s = pair_of.p[1];
+        s_off1[0] = s.offsets[0];
+        s_off1[1] = s.offsets[1];
+        s_ptr[0][PE] = (unsigned long long)(uintptr_t)s.b0[0];
+        s_ptr[1][PE] = SWIGLU ? (unsigned long long)(uintptr_t)s.b1[0] : 0ull;
+        s_ptr[2][PE] = W8 ? (unsigned long long)(uintptr_t)s.s0[0] : 0ull;
+        s_ptr[3][PE] = (W8 && SWIGLU) ? (unsigned long long)(uintptr_t)s.s1[0] : 0ull;
+    }
     __syncthreads();
     // whole rounds, and the last one unless it is better off with the other kernel, whose own tiles are counted for that
-    const int own = g.tail_cus > 0 ? sum_over_experts<NT>(g, tid, s_wtot, [&](int c) { return own_tiles<W8>(g, c); }) * g.n_tiles_n : 0;
-    const int total = run * g.n_tiles_n - tail_tiles(g, run * g.n_tiles_n, own);
+    const int own = g.tail_cus > 0 ? sum_over_experts<NT>(g, tid, s_wtot, [&](int c) { return own_tiles<W8>(g, c); }) * g.n_tiles_n + pair_of.shared_tiles : 0;
+    const int all = run * g.n_tiles_n + ptiles1, total = all - tail_tiles(g, all, own);
     const int xcd = blockIdx.x & 7, slots = gridDim.x >> 3;
     int slot = blockIdx.x >> 3;
     auto tile_of = [&](int sl) { return ((sl / slots) * 8 + xcd) * slots + (sl % slots); };
     if (tile_of(slot) >= total) return;
-    const int K = g.K, N = g.N;
-    const int KB = K >> 7;
 
     // Token rows come through a buffer descriptor and 32-bit byte offsets.  Gathered rows (row_map): one
     // descriptor over all of x, whose size the launcher has checked against 4 GiB, so a row_map entry
     // outside x reads zeros instead of faulting.  Sorted rows: the descriptor starts at the tile's first row.
-    const uint8_t *a_base = reinterpret_cast<const uint8_t*>(g.a), *a_base_n = a_base;
-    const int a_records = SWIGLU && g.row_map ? (int)(uint32_t)g.a_bytes : -1;
+    const uint8_t *a_base = nullptr, *a_base_n = nullptr;
+    int a_records = -1, a_records_n = -1;
     uint32_t a_voff[ND];                        // this wave's DMA offsets of the tile being fetched
     int a_row_n[ND];                            // and its rows of x of the next one
     // bf16 weights also by DMA: descriptors of the expert's matrices and per-lane offsets (gate and up: rows n0 .. n0 + 127
@@ -1893,24 +1911,41 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmArgs g
     gptr_f32 sc0 = nullptr, sc1 = nullptr;
     int row0 = 0, row_end = 0, n0 = 0;
     int cur_e = 0;
+    uint16_t* c_out = nullptr;                  // of the tile set up last: outputs and their row length
+    int N_out = 0;
     // bf16 weights: k starts at another stage for every N tile (k_rotation); stage_of is the stage that pipeline step
     // kt fetches.  The rotation is adopted with the tile's DMA coordinates.
-    const int nk = K / BK;
-    int rot = 0, rot_n = 0;
-    auto stage_of = [&](int kt, int r) { const int kp = kt + r; return kp >= nk ? kp - nk : kp; };
+    // (So are the stages of a tile and the length of its token rows: the two problems may differ in them.)
+    int rot = 0, rot_n = 0, nk_dma = 0, K_n = 0;
+    auto stage_of = [&](int kt, int r) { const int kp = kt + r; return kp >= nk_dma ? kp - nk_dma : kp; };
     auto setup = [&](int v) {
         const int l = fresh_lane();
         const int t = wave_s * 64 + l;
-        const int q = v / g.n_tiles_n;
-        while (uni(s_pref[cur_e + 1]) <= q) ++cur_e;
-        const int e = cur_e;
-        const int pe = uni(s_pref[e]);
-        const int mt_e = uni(s_pref[e + 1]) - pe;
-        int m_tile, n_tile;
-        tile_in_expert(v - pe * g.n_tiles_n, mt_e, g.n_tiles_n, m_tile, n_tile);
-        row0 = uni(s_off[e]) + m_tile * BM;
-        row_end = uni(s_off[e + 1]);
+        const bool second = v < ptiles1;
+        const GemmArgs& pr = pair_of.p[second ? 1 : 0];
+        const int K = pr.K, N = pr.N, nk = K / BK;
+        int m_tile, n_tile, e, first;
+        if (second) {
+            e = PE;
+            first = uni(s_off1[0]);
+            row_end = uni(s_off1[1]);
+            tile_in_expert(v, ptiles1 / pr.n_tiles_n, pr.n_tiles_n, m_tile, n_tile);
+        } else {
+            v -= ptiles1;
+            const int q = v / pr.n_tiles_n;
+            while (uni(s_pref[cur_e + 1]) <= q) ++cur_e;
+            e = cur_e;
+            const int pe = uni(s_pref[e]);
+            const int mt_e = uni(s_pref[e + 1]) - pe;
+            first = uni(s_off[e]);
+            row_end = uni(s_off[e + 1]);
+            tile_in_expert(v - pe * pr.n_tiles_n, mt_e, pr.n_tiles_n, m_tile, n_tile);
+        }
+        row0 = first + m_tile * BM;
         n0 = n_tile * NBLK;
+        c_out = pr.c;
+        N_out = N;
+        K_n = K;
         rot_n = W8 ? 0 : k_rotation<false>(n_tile, nk);
         // DMA instruction i of this wave fills rows 16*wave + 8*(i&1) .. +7 of the 128 rows of half i/2: lane l supplies
         // row +l/8 and the 16 bytes that belong at physical chunk l%8, i.e. logical chunk (l%8) ^ swz(row).  Row r of
@@ -1921,15 +1956,17 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmArgs g
         for (int i = 0; i < ND; ++i) {
             const int rt = ((wave_s >> 2) << 7) + ((i >> 1) << 6) + 16 * (wave_s & 3) + 8 * (i & 1) + lr;   // row of the tile
             const int r = min(row0 + rt, row_end - 1);
-            a_row_n[i] = SWIGLU && g.row_map ? ((gptr_i32)(uintptr_t)g.row_map)[r] : r - row0;   // (down: sorted rows)
+            a_row_n[i] = SWIGLU && pr.row_map ? ((gptr_i32)(uintptr_t)pr.row_map)[r] : r - row0;   // (down: sorted rows)
         }
-        if (!(SWIGLU && g.row_map)) a_base_n = reinterpret_cast<const uint8_t*>(g.a) + (size_t)row0 * K * 2;
+        const bool gathered = SWIGLU && pr.row_map;
+        a_base_n = uni_ptr(reinterpret_cast<const uint8_t*>(pr.a) + (gathered ? (size_t)0 : (size_t)row0 * K * 2));
+        a_records_n = uni(gathered ? (int)(uint32_t)pr.a_bytes : -1);
         const uint8_t* bmat0 = uni_ptr(reinterpret_cast<const void*>((uintptr_t)s_ptr[0][e]));
         const uint8_t* bmat1 = SWIGLU ? uni_ptr(reinterpret_cast<const void*>((uintptr_t)s_ptr[1][e])) : bmat0;
         if (W8) {
             sc0 = (gptr_f32)(uintptr_t)uni_ptr(reinterpret_cast<const void*>((uintptr_t)s_ptr[2][e]));
             sc1 = SWIGLU ? (gptr_f32)(uintptr_t)uni_ptr(reinterpret_cast<const void*>((uintptr_t)s_ptr[3][e])) : sc0;
-            const int brow = t >> 2, bcol_b = (t & 3) << 4;
+            const int brow = t >> 2, bcol_b = (t & 3) << 4, KB = K >> 7;
 #pragma unroll
             for (int i = 0; i < NB; ++i) {
                 int r = brow + RB * i;
@@ -1955,13 +1992,15 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmArgs g
         const int l = fresh_lane(), lr = l >> 3;
 #pragma unroll
         for (int i = 0; i < ND; ++i)             // swz(row): row & 7 == lr, (row >> 3) & 1 == i & 1
-            a_voff[i] = (uint32_t)a_row_n[i] * (uint32_t)(K * 2) + (uint32_t)(((l & 7) ^ lr ^ (i & 1)) << 4);
+            a_voff[i] = (uint32_t)a_row_n[i] * (uint32_t)(K_n * 2) + (uint32_t)(((l & 7) ^ lr ^ (i & 1)) << 4);
         if (!W8) {
 #pragma unroll
             for (int i = 0; i < NBO; ++i) b_voff[i] = b_voff_n[i];
             bm0 = bm0_n; bm1 = bm1_n;
         }
         a_base = a_base_n;
+        a_records = a_records_n;
+        nk_dma = K_n / BK;
         rot = rot_n;
     };
     auto dma_a = [&](int st, int kt, int i) __attribute__((always_inline)) {
@@ -2124,7 +2163,8 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmArgs g
     __builtin_amdgcn_s_waitcnt(0x0f70);     // vmcnt(0), as an instruction that the compiler's own count knows
     constexpr int CW = SWIGLU ? 8 * TN : 16 * TN;    // output columns of this wave
     for (;;) {
-        const int out_row0 = row0, out_row_end = row_end, out_n0 = n0;
+        const int out_row0 = row0, out_row_end = row_end, out_n0 = n0, N = N_out, nk = nk_dma;
+        uint16_t* const c = c_out;
         bool more = false;
         auto next_tile = [&]() {
             slot += slots;
@@ -2163,7 +2203,7 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmArgs g
             const int l = fresh_lane();
             const int fr = l & 15, q = l >> 4;
             const int rows_here = min(BM, out_row_end - out_row0) - wm * 128, ncol0 = out_n0 + wn * CW;
-            const uint8_t* out = uni_ptr(g.c + (size_t)(out_row0 + wm * 128) * N + ncol0);
+            const uint8_t* out = uni_ptr(c + (size_t)(out_row0 + wm * 128) * N + ncol0);
             uint8_t* ep = sA1b + wave_s * 2048;
 #pragma unroll
             for (int mi = 0; mi < TM; ++mi) {
@@ -2192,18 +2232,12 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmArgs g
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no DMA may land in LDS after the workgroup has gone
 }
 
-// shared: the second problem of the launch (NULL: none), of n_shared rows
 template <int WN, bool SWIGLU, bool W8>
-int launch_tiles(const GemmArgs& g, int n_rows, const GemmArgs* shared, int n_shared, hipStream_t st) {
+int launch_tiles(const GemmPair& pair, int n_rows, hipStream_t st) {
     auto kern = grouped_gemm_kernel<WN, SWIGLU, W8>;
+    const GemmArgs& g = pair.p[0];
     // sum_e tiles_of(c_e) <= sum_e (c_e / 128 + 1); with the larger experts elsewhere, one tile per expert that has rows
     const long max_mtiles = g.cold_max <= 192 ? (g.pair_rows ? 2 : 1) * (long)(g.E < n_rows ? g.E : n_rows) : (long)n_rows / 128 + g.E;
-    GemmPair pair{};
-    pair.p[0] = g;
-    if (shared) {
-        pair.p[1] = *shared;
-        pair.shared_tiles = tiles_of<!W8>(n_shared) * shared->n_tiles_n;
-    }
     // (+ the persistent kernel's last tiles, less than a round of them, as two half tiles each)
     const long grid = ((max_mtiles * g.n_tiles_n + pair.shared_tiles + 2 * g.tail_cus + 31) / 32) * 32;   // whole rounds of 8 groups of 4 tiles
     if (grid > 0x7fffffffL) {
@@ -2248,12 +2282,13 @@ inline int cu_count() {
 }
 
 template <bool SWIGLU, bool W8>
-int launch_persistent(const GemmArgs& g, int n_rows, hipStream_t st) {
+int launch_persistent(const GemmPair& pair, int n_rows, hipStream_t st) {
+    const GemmArgs& g = pair.p[0];
     const long max_mtiles = (long)n_rows / 256 + g.E;
-    long grid = ((max_mtiles * g.n_tiles_n + 7) / 8) * 8;
+    long grid = ((max_mtiles * g.n_tiles_n + pair.shared_ptiles + 7) / 8) * 8;
     const long ncu = (cu_count() / 8) * 8;
     if (grid > ncu) grid = ncu;
-    hipLaunchKernelGGL((grouped_gemm_persistent_kernel<SWIGLU, W8>), dim3((unsigned)grid), dim3(512), 0, st, g);
+    hipLaunchKernelGGL((grouped_gemm_persistent_kernel<SWIGLU, W8>), dim3((unsigned)grid), dim3(512), 0, st, pair);
     MOE_HIP_CHECK(hipGetLastError());
     return MOE_OK;
 }
@@ -2308,6 +2343,26 @@ bool thin_pays(const GemmArgs& g, int n_rows, const GemmArgs* shared) {
     return thin < std::ceil(tiles / cus) * cus * (g.K <= 2048 ? 1.07 : 1.0);
 }
 
+// The persistent kernel needs an even number of k-stages for its hand-over (fp8 sizes always have one), keeps per-expert
+// tables for up to 512 experts and addresses gathered rows with 32-bit offsets.
+inline bool persistent_fits(const GemmArgs& g) { return g.K % 128 == 0 && g.E <= 512 && gather_fits(g) && cu_count() >= 8; }
+
+// the rules by which a call's tiles fall to the two kernels (reasons in launch_mt)
+template <bool W8>
+GemmArgs both_kernels(GemmArgs g) {
+    g.cold_max = 192;
+    g.rem_split = W8 ? 1 : 0;
+    g.pair_rows = W8 ? 0 : 1;
+    g.tail_cus = (cu_count() / 8) * 8;     // the persistent launch's grid when there is a round of tiles or more
+    return g;
+}
+
+template <bool SWIGLU, bool W8>
+int launch_both(const GemmPair& pair, int n_rows, hipStream_t st) {
+    const int rc = launch_persistent<SWIGLU, W8>(pair, n_rows, st);
+    return rc != MOE_OK ? rc : launch_tiles<4, SWIGLU, W8>(pair, n_rows, st);
+}
+
 // max_rows: no expert has more rows (callers that do not know pass n_rows)
 template <bool SWIGLU, bool W8>
 int launch_mt(const GemmArgs& g0, int n_rows, int max_rows, void* workspace, size_t workspace_bytes, hipStream_t st) {
@@ -2319,12 +2374,11 @@ int launch_mt(const GemmArgs& g0, int n_rows, int max_rows, void* workspace, siz
             return launch_split(g, n_rows, plan, static_cast<float*>(workspace), st);
     }
     if (max_rows <= 16 && gather_fits(g) && thin_pays(g, n_rows, nullptr)) return launch_thin<SWIGLU, W8>(g, n_rows, nullptr, st);
-    // the persistent kernel needs an even number of k-stages for its hand-over (fp8 sizes always have
-    // one), keeps per-expert tables for up to 512 experts and addresses gathered rows with 32-bit offsets
-    // (below a mean of 128 rows an expert above one tile is rare and is cut into 128-row tiles where it occurs)
-    if (mean < 128 || !(g.K % 128 == 0 && g.E <= 512 && gather_fits(g) && cu_count() >= 8)) {
+    GemmPair pair{};
+    if (mean < 128 || !persistent_fits(g)) {
         g.cold_max = 0x7fffffff;
-        return launch_tiles<4, SWIGLU, W8>(g, n_rows, nullptr, 0, st);
+        pair.p[0] = g;
+        return launch_tiles<4, SWIGLU, W8>(pair, n_rows, st);
     }
     // The counts themselves live on the device; only their mean is known here.  Both kernels are launched and every
     // expert goes by its own count: what fits one tile of the one-workgroup-per-tile kernel runs there, at its own
@@ -2345,26 +2399,29 @@ int launch_mt(const GemmArgs& g0, int n_rows, int max_rows, void* workspace, siz
     // weights it is break-even (Mixtral-8x7B 9.28 -> 9.23 ms, DeepSeek-V2-236B 11.34 -> 11.42) and not done.
     // (Both launches at every mean: from 1536 rows per expert a small expert is rare, but the second launch is there
     // for the persistent kernel's last round anyway.)
-    g.cold_max = 192;
-    g.rem_split = W8 ? 1 : 0;
-    g.pair_rows = W8 ? 0 : 1;
     // Last round of the persistent kernel (tail_tiles above): Mixtral-8x22B, 8192 tokens, down projection (6.4 rounds
     // of 0.4 ms) 2.82 -> 2.66 ms, step 8.31 -> 8.13; Mixtral-8x7B 9.39 -> 9.27 ms; DeepSeek-V2-Lite 0.855 -> 0.821 ms
     // (its shared expert's 128 down tiles become 256 half tiles: 0.071 -> 0.055 ms); DeepSeek-V2-236B 11.43 -> 11.46,
     // DeepSeek-V3 46.56 -> 46.54: short rounds gain nothing, a partial round of few CUs runs at a higher clock anyway.
-    g.tail_cus = (cu_count() / 8) * 8;     // the persistent launch's grid when there is a round of tiles or more
-    int rc = launch_persistent<SWIGLU, W8>(g, n_rows, st);
-    if (rc != MOE_OK) return rc;
-    return launch_tiles<4, SWIGLU, W8>(g, n_rows, nullptr, 0, st);
+    pair.p[0] = both_kernels<W8>(g);
+    return launch_both<SWIGLU, W8>(pair, n_rows, st);
 }
 
-// The shared expert's tiles in the routed experts' launch.
+// The shared expert's tiles in the routed experts' launches.
 template <bool SWIGLU, bool W8>
 int launch_joint(const GemmArgs& routed, int n_rows, int max_rows, const GemmArgs& shared, int n_shared, hipStream_t st) {
     if (max_rows <= 16 && n_shared <= 16 && thin_pays(routed, n_rows, &shared)) return launch_thin<SWIGLU, W8>(routed, n_rows, &shared, st);
-    GemmArgs r = routed, s = shared;
-    r.cold_max = s.cold_max = 0x7fffffff;
-    return launch_tiles<4, SWIGLU, W8>(r, n_rows, &s, n_shared, st);
+    GemmPair pair{{routed, shared}, 0, 0};
+    if (n_rows / routed.E < 128) {
+        pair.p[0].cold_max = pair.p[1].cold_max = 0x7fffffff;
+        pair.shared_tiles = tiles_of<!W8>(n_shared) * shared.n_tiles_n;
+        return launch_tiles<4, SWIGLU, W8>(pair, n_rows, st);
+    }
+    pair.p[0] = both_kernels<W8>(routed);
+    pair.p[1] = both_kernels<W8>(shared);
+    pair.shared_tiles = own_tiles<W8>(pair.p[1], n_shared) * shared.n_tiles_n;
+    pair.shared_ptiles = persistent_tiles(pair.p[1], n_shared) * shared.n_tiles_n;
+    return launch_both<SWIGLU, W8>(pair, n_rows, st);
 }
 
 int check_group(const moe_mlp_group& m, int32_t hidden, bool w8, const char* who) {
@@ -2409,15 +2466,20 @@ GemmArgs down_args(const moe_mlp_group& m, int32_t hidden) {
 // no expert of the group has more rows than this
 int row_bound(const moe_mlp_group& m) { return m.max_rows > 0 && m.max_rows < m.n_rows ? m.max_rows : m.n_rows; }
 
-// Whether the shared expert's tiles join the routed experts' launch: it is small -- (n / 256 + 1) row tiles times I / 128
-// column tiles fewer than 3/8 of the device's CUs: alone it would leave most of them without a tile -- and the routed
-// call is one that the one-workgroup-per-tile kernel (or the thin one) serves alone.  DeepSeek-V3 up to 1024 tokens: the
-// step gains 2-5 %, from 2048 tokens on a launch pair of its own, with 256-row tiles, is the faster by 0.6 %.
+// Whether the shared expert's tiles join the routed experts' launches.  Where the routed call goes to both kernels they
+// do: the two then fill their last rounds together.  Where it is one that the one-workgroup-per-tile kernel (or the thin
+// one) serves alone, whose 128-row tiles would be all the shared expert gets, up to two such tiles per CU.
+// Layers, us, apart -> joined.  Both kernels: DeepSeek-V2-Lite 1400 / 2000 / 2777 / 4096 tokens 439 / 514 / 585 / 725 -> 397 / 470 /
+// 563 / 699; DeepSeek-V3 4096 / 6000 4046 / 5498 -> 4004 / 5367, 16384 the same.  One kernel: DeepSeek-V2-Lite 1024 / 1300 366 /
+// 409 -> 322 / 351; DeepSeek-V2-236B 1024 / 1500 1463 / 1641 -> 1416 / 1615, 2048 the same, 3000 2074 -> 2090 (not joined: 576 tiles);
+// DeepSeek-V3 1500 / 2997 / 4000 2507 / 3437 / 4139 -> 2470 / 3382 / 4120.
 bool joins(const moe_mlp_group& routed, const moe_mlp_group& shared, int32_t hidden) {
     if (routed.n_rows < 1 || shared.n_rows < 1 || routed.n_experts < 1 || shared.n_experts != 1 || hidden < 1) return false;
-    if (routed.n_rows / routed.n_experts >= 128) return false;
     if (routed.row_map && (size_t)routed.x_rows * (size_t)hidden * 2 >= (1ull << 32)) return false;
-    return (long)(shared.n_rows / 256 + 1) * ((shared.inter + 127) / 128) * 8 < 3L * cu_count();
+    if (shared.row_map && (size_t)shared.x_rows * (size_t)hidden * 2 >= (1ull << 32)) return false;
+    if (routed.n_rows / routed.n_experts >= 128)
+        return hidden % 128 == 0 && routed.inter % 128 == 0 && shared.inter % 128 == 0 && routed.n_experts <= 512 && cu_count() >= 8;
+    return (long)((shared.n_rows + 127) / 128) * ((shared.inter + 127) / 128) <= 2L * cu_count();
 }
 
 template <bool W8>

@@ -857,6 +857,43 @@ def test_shared_expert_in_the_routed_launches(fp8, n, shared_inter):
         assert (a - b).abs().max().item() <= TOL * b.abs().max().item()
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("n,E,I,shared_inter", [
+    (700, 4, 256, 128),       # the shared expert's k is shorter than the routed experts', every tile of it a half tile
+    (1500, 4, 128, 640),      # longer; all of the persistent kernel's tiles are half tiles, the shared expert's among them
+    (3000, 8, 1280, 2560),    # rounds of tiles of both
+    (2900, 3, 256, 2048),     # mostly the shared expert's
+    (200, 2, 256, 384)])      # one tile of up to 192 rows next to 256-row tiles
+def test_shared_expert_in_the_launches_of_both_kernels(fp8, n, E, I, shared_inter):
+    """From a mean of 128 rows per expert on the shared expert's tiles come first in the launches of the persistent kernel and of
+    the other one.  Bit for bit what the calls give apart, with fp8 weights too (both start every tile at k 0 there)."""
+    from moe_gen_amd import ops
+    k, h = 2, 384
+    print(f"joint, both kernels fp8={fp8} n={n} E={E} I={I} shared_inter={shared_inter}", flush=True)
+    g = torch.Generator().manual_seed(n)
+    dev = lambda m: tuple(t.cuda() for t in m) if isinstance(m, tuple) else m.cuda()
+    tables = []
+    for count, inter, seed in ((E, I, 11), (1, shared_inter, 12)):
+        dm = [[dev(m) for m in one] for one in make_experts(count, h, inter, fp8, seed)]
+        col = lambda i, j: [o[i][j] if fp8 else o[i] for o in dm]
+        tables.append(ops.expert_pointers(*(col(i, 0) for i in range(3)), *((col(i, 1) for i in range(3)) if fp8 else ())))
+    idx = (torch.rand((n, E), generator=g) + 0.2 * torch.arange(E)).topk(k, dim=1).indices.to(torch.int32)
+    x = torch.randn(n, h, generator=g).to(torch.bfloat16).cuda()
+    d = ops.dispatch(idx.cuda(), E, None, want_row_map=True)
+    so = torch.tensor([0, n], dtype=torch.int32, device="cuda")
+    r1, _, y1 = ops.mlp_group(x, d.row_map, tables[0], d.offsets, n * k, n)
+    s1, _, sh1 = ops.mlp_group(x, None, tables[1], so, n)
+    y1.fill_(7.0); sh1.fill_(7.0)
+    assert ops.shared_joins(r1, s1, h)
+    ops.grouped_swiglu_joint(r1, s1, h, fp8)
+    r2, _, y2 = ops.mlp_group(x, d.row_map, tables[0], d.offsets, n * k, n)
+    s2, _, sh2 = ops.mlp_group(x, None, tables[1], so, n)
+    ops.grouped_swiglu_joint(r2, None, h, fp8)
+    ops.grouped_swiglu_joint(s2, None, h, fp8)
+    torch.cuda.synchronize()
+    assert torch.equal(y1, y2) and torch.equal(sh1, sh2)
+
+
 @pytest.mark.parametrize("I", [4096, 4224, 18432])      # 32 blocks of 128 k (the rule's least), 33 (a short last slice), DeepSeek-V3's
 @pytest.mark.parametrize("h", [128, 768])               # half a column tile; three
 def test_dense_fp8_down_projection_in_slices_of_k(h, I):
