@@ -1189,13 +1189,17 @@ __host__ __device__ __forceinline__ int persistent_tiles(const GemmArgs& g, int 
 // that is a last round of at most half the CUs; next to other work also a longer one (Mixtral-8x22B, 1024 tokens,
 // down projection: 144 tiles here and 144 there are two half-empty launches in a row, 0.71 ms; as one launch of 432
 // tiles 0.56).  Both kernels evaluate this on the same offsets[].
+struct RoundCost { int keep, move; };       // the two launches with the last round in the persistent kernel / in the other
+__host__ __device__ __forceinline__ RoundCost round_cost(int total, int own, int cus) {
+    return RoundCost{100 * ((total + cus - 1) / cus) + 72 * ((own + cus - 1) / cus),
+                     100 * (total / cus) + 72 * ((own + 2 * (total % cus) + cus - 1) / cus)};
+}
 __device__ __forceinline__ int tail_tiles(const GemmArgs& g, int total, int own) {
     if (g.tail_cus <= 0) return 0;
-    const int cus = g.tail_cus, tail = total % cus;
+    const int tail = total % g.tail_cus;
     if (tail == 0) return 0;
-    const int keep = 100 * (total / cus + 1) + 72 * ((own + cus - 1) / cus);
-    const int move = 100 * (total / cus) + 72 * ((own + 2 * tail + cus - 1) / cus);
-    return move < keep ? tail : 0;
+    const RoundCost c = round_cost(total, own, g.tail_cus);
+    return c.move < c.keep ? tail : 0;
 }
 
 template <bool PAIR>   // whether an expert of PAIR_LO .. PAIR_HI rows is cut in the middle (bf16 weights)
@@ -2404,6 +2408,17 @@ int launch_mt(const GemmArgs& g0, int n_rows, int max_rows, void* workspace, siz
     // (its shared expert's 128 down tiles become 256 half tiles: 0.071 -> 0.055 ms); DeepSeek-V2-236B 11.43 -> 11.46,
     // DeepSeek-V3 46.56 -> 46.54: short rounds gain nothing, a partial round of few CUs runs at a higher clock anyway.
     pair.p[0] = both_kernels<W8>(g);
+    // One fp8 expert (a dense MLP): the rows are known here.  What its full tiles leave over goes to the persistent kernel too,
+    // as a padded tile, where that shortens the two launches by the same count: the last round has room, or the other launch
+    // is saved.  DeepSeek-V3's dense MLP, us: 1300 / 1800 / 2200 / 4000 / 6000 tokens (leftovers of 20, 8, 152, 160 and 112 rows) 1129 /
+    // 1352 / 1567 / 2726 / 3998 -> 1015 / 1263 / 1465 / 2606 / 3887; done always, 600 / 1100 / 3500 tokens would be 616 / 931 / 2370
+    // instead of 534 / 816 / 2265.
+    if (W8 && g.E == 1 && own_tiles<W8>(pair.p[0], n_rows) > 0) {
+        const int cus = pair.p[0].tail_cus, full = (n_rows >> 8) * g.n_tiles_n;
+        const RoundCost apart = round_cost(full, g.n_tiles_n, cus), padded = round_cost(full + g.n_tiles_n, 0, cus);
+        const int a = apart.move < apart.keep ? apart.move : apart.keep, b = padded.move < padded.keep ? padded.move : padded.keep;
+        if (b < a) pair.p[0].cold_max = 0;
+    }
     return launch_both<SWIGLU, W8>(pair, n_rows, st);
 }
 

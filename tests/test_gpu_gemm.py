@@ -894,6 +894,25 @@ def test_shared_expert_in_the_launches_of_both_kernels(fp8, n, E, I, shared_inte
     assert torch.equal(y1, y2) and torch.equal(sh1, sh2)
 
 
+@pytest.mark.parametrize("left", [1, 72, 192])
+def test_dense_fp8_leftover_rows_as_a_padded_tile(left):
+    """One fp8 MLP of 11 full tiles and a leftover whose gate and up tiles (240 of 128 columns with the leftover's) fit one round
+    of the persistent kernel: it takes them all.  The last rows come out bit for bit as in a call of their own, where
+    the other kernel serves the leftover, and the first as in a call without one."""
+    from moe_gen_amd import ops
+    h, I, n = 256, 2560, 11 * 256 + left
+    print(f"padded leftover {left}", flush=True)
+    g = torch.Generator().manual_seed(left)
+    x = torch.randn(n, h, generator=g).to(torch.bfloat16).cuda()
+    mats = [tuple(t.cuda() for t in m) for m in make_experts(1, h, I, True, 31)[0]]
+    ptrs = ops.expert_pointers(*([m[0]] for m in mats), *([m[1]] for m in mats))
+    def call(rows):
+        return ops.grouped_swiglu(rows, None, ptrs, torch.tensor([0, len(rows)], dtype=torch.int32, device="cuda"), len(rows))
+    y = call(x)
+    assert torch.equal(y[10 * 256:], call(x[10 * 256:].contiguous()))
+    assert torch.equal(y[:11 * 256], call(x[:11 * 256].contiguous()))
+
+
 @pytest.mark.parametrize("I", [4096, 4224, 18432])      # 32 blocks of 128 k (the rule's least), 33 (a short last slice), DeepSeek-V3's
 @pytest.mark.parametrize("h", [128, 768])               # half a column tile; three
 def test_dense_fp8_down_projection_in_slices_of_k(h, I):
