@@ -1834,7 +1834,8 @@ __device__ __forceinline__ int fresh_lane() {
 // 1378 -> 1396; 8 experts, 32768 rows, 4096 <-> 14336 1273 -> 1383 and 1277 -> 1390; 160 experts, 196608 rows, 5120 <-> 1536
 // 1190 -> 1271 and 1076 -> 1164.  fp8, 64 experts, 131072 rows, 7168 <-> 2048: 1259 -> 1282 and 1201 -> 1217; there the
 // conversion, 64 vector instructions per 64 matrix instructions, is what is left (a tenth more with most of it taken out).
-template <bool SWIGLU, bool W8>
+// PAIRED: with a second problem.  (An instantiation of its own: the choice per tile costs DeepSeek-V3's 65536 tokens 0.4 %.)
+template <bool SWIGLU, bool W8, bool PAIRED>
 __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmPair pair_of) {
     const GemmArgs& g = pair_of.p[0];            // the routed experts; the tiles of the second problem come first
     constexpr int MT = 4, WN = 4;
@@ -1876,9 +1877,9 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmPair p
         s_ptr[2][e] = W8 ? (unsigned long long)(uintptr_t)g.s0[e] : 0ull;
         s_ptr[3][e] = (W8 && SWIGLU) ? (unsigned long long)(uintptr_t)g.s1[e] : 0ull;
     });
-    const int ptiles1 = pair_of.shared_ptiles;
+    const int ptiles1 = PAIRED ? pair_of.shared_ptiles : 0;
     if (tid == 0) s_pref[g.E] = run;
-    if (ptiles1 > 0 && tid == 0) {
+    if (PAIRED && tid == 0) {
         const GemmArgs& s = pair_of.p[1];
         s_off1[0] = s.offsets[0];
         s_off1[1] = s.offsets[1];
@@ -1925,29 +1926,31 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmPair p
     auto setup = [&](int v) {
         const int l = fresh_lane();
         const int t = wave_s * 64 + l;
-        const bool second = v < ptiles1;
-        const GemmArgs& pr = pair_of.p[second ? 1 : 0];
-        const int K = pr.K, N = pr.N, nk = K / BK;
+        const bool second = PAIRED && v < ptiles1;
+        // (selects, not a reference to either: that would be loads from the arguments, waited for on every tile)
+        const GemmArgs& g1 = pair_of.p[1];
+        const int K = second ? g1.K : g.K, N = second ? g1.N : g.N, nk = K / BK, tiles_n = second ? g1.n_tiles_n : g.n_tiles_n;
+        const int32_t* const row_map = SWIGLU ? (second ? g1.row_map : g.row_map) : nullptr;
         int m_tile, n_tile, e, first;
         if (second) {
             e = PE;
             first = uni(s_off1[0]);
             row_end = uni(s_off1[1]);
-            tile_in_expert(v, ptiles1 / pr.n_tiles_n, pr.n_tiles_n, m_tile, n_tile);
+            tile_in_expert(v, ptiles1 / tiles_n, tiles_n, m_tile, n_tile);
         } else {
             v -= ptiles1;
-            const int q = v / pr.n_tiles_n;
+            const int q = v / tiles_n;
             while (uni(s_pref[cur_e + 1]) <= q) ++cur_e;
             e = cur_e;
             const int pe = uni(s_pref[e]);
             const int mt_e = uni(s_pref[e + 1]) - pe;
             first = uni(s_off[e]);
             row_end = uni(s_off[e + 1]);
-            tile_in_expert(v - pe * pr.n_tiles_n, mt_e, pr.n_tiles_n, m_tile, n_tile);
+            tile_in_expert(v - pe * tiles_n, mt_e, tiles_n, m_tile, n_tile);
         }
         row0 = first + m_tile * BM;
         n0 = n_tile * NBLK;
-        c_out = pr.c;
+        c_out = second ? g1.c : g.c;
         N_out = N;
         K_n = K;
         rot_n = W8 ? 0 : k_rotation<false>(n_tile, nk);
@@ -1960,11 +1963,10 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmPair p
         for (int i = 0; i < ND; ++i) {
             const int rt = ((wave_s >> 2) << 7) + ((i >> 1) << 6) + 16 * (wave_s & 3) + 8 * (i & 1) + lr;   // row of the tile
             const int r = min(row0 + rt, row_end - 1);
-            a_row_n[i] = SWIGLU && pr.row_map ? ((gptr_i32)(uintptr_t)pr.row_map)[r] : r - row0;   // (down: sorted rows)
+            a_row_n[i] = row_map ? ((gptr_i32)(uintptr_t)row_map)[r] : r - row0;   // (down: sorted rows)
         }
-        const bool gathered = SWIGLU && pr.row_map;
-        a_base_n = uni_ptr(reinterpret_cast<const uint8_t*>(pr.a) + (gathered ? (size_t)0 : (size_t)row0 * K * 2));
-        a_records_n = uni(gathered ? (int)(uint32_t)pr.a_bytes : -1);
+        a_base_n = reinterpret_cast<const uint8_t*>(second ? g1.a : g.a) + (row_map ? (size_t)0 : (size_t)row0 * K * 2);
+        a_records_n = row_map ? (int)(uint32_t)(second ? g1.a_bytes : g.a_bytes) : -1;
         const uint8_t* bmat0 = uni_ptr(reinterpret_cast<const void*>((uintptr_t)s_ptr[0][e]));
         const uint8_t* bmat1 = SWIGLU ? uni_ptr(reinterpret_cast<const void*>((uintptr_t)s_ptr[1][e])) : bmat0;
         if (W8) {
@@ -2292,7 +2294,8 @@ int launch_persistent(const GemmPair& pair, int n_rows, hipStream_t st) {
     long grid = ((max_mtiles * g.n_tiles_n + pair.shared_ptiles + 7) / 8) * 8;
     const long ncu = (cu_count() / 8) * 8;
     if (grid > ncu) grid = ncu;
-    hipLaunchKernelGGL((grouped_gemm_persistent_kernel<SWIGLU, W8>), dim3((unsigned)grid), dim3(512), 0, st, pair);
+    if (pair.shared_ptiles > 0) hipLaunchKernelGGL((grouped_gemm_persistent_kernel<SWIGLU, W8, true>), dim3((unsigned)grid), dim3(512), 0, st, pair);
+    else hipLaunchKernelGGL((grouped_gemm_persistent_kernel<SWIGLU, W8, false>), dim3((unsigned)grid), dim3(512), 0, st, pair);
     MOE_HIP_CHECK(hipGetLastError());
     return MOE_OK;
 }
@@ -2482,7 +2485,7 @@ GemmArgs down_args(const moe_mlp_group& m, int32_t hidden) {
 int row_bound(const moe_mlp_group& m) { return m.max_rows > 0 && m.max_rows < m.n_rows ? m.max_rows : m.n_rows; }
 
 // Whether the shared expert's tiles join the routed experts' launches.  Where the routed call goes to both kernels they
-// do: the two then fill their last rounds together.  Where it is one that the one-workgroup-per-tile kernel (or the thin
+// do, up to four rounds of tiles of its own (beyond, the same within 0.2 %): the two then fill their last rounds together.  Where it is one that the one-workgroup-per-tile kernel (or the thin
 // one) serves alone, whose 128-row tiles would be all the shared expert gets, up to two such tiles per CU.
 // Layers, us, apart -> joined.  Both kernels: DeepSeek-V2-Lite 1400 / 2000 / 2777 / 4096 tokens 439 / 514 / 585 / 725 -> 397 / 470 /
 // 563 / 699; DeepSeek-V3 4096 / 6000 4046 / 5498 -> 4004 / 5367, 16384 the same.  One kernel: DeepSeek-V2-Lite 1024 / 1300 366 /
@@ -2493,7 +2496,7 @@ bool joins(const moe_mlp_group& routed, const moe_mlp_group& shared, int32_t hid
     if (routed.row_map && (size_t)routed.x_rows * (size_t)hidden * 2 >= (1ull << 32)) return false;
     if (shared.row_map && (size_t)shared.x_rows * (size_t)hidden * 2 >= (1ull << 32)) return false;
     if (routed.n_rows / routed.n_experts >= 128)
-        return hidden % 128 == 0 && routed.inter % 128 == 0 && shared.inter % 128 == 0 && routed.n_experts <= 512 && cu_count() >= 8;
+        return (long)((shared.n_rows + 255) / 256) * ((shared.inter + 127) / 128) <= 4L * cu_count() && hidden % 128 == 0 && routed.inter % 128 == 0 && shared.inter % 128 == 0 && routed.n_experts <= 512 && cu_count() >= 8;
     return (long)((shared.n_rows + 127) / 128) * ((shared.inter + 127) / 128) <= 2L * cu_count();
 }
 
