@@ -241,7 +241,7 @@ size_t moe_mlp_workspace_bytes(const moe_mlp_group* group, int32_t hidden);
  * of any intermediate size, n_experts == 1) in one call, both of the same weight type (fp8 != 0: fp8 with block scales).
  * Where moe_shared_joins says 1 they share their launches: the shared expert's tiles run next to the routed experts';
  * otherwise they run one after the other.  shared == NULL: the routed experts alone.  With bf16 weights the bits are
- * those of separate calls.
+ * those of separate calls, with fp8 weights too from a mean of 128 rows per routed expert on.
  */
 int moe_grouped_swiglu_joint(const moe_mlp_group* routed, const moe_mlp_group* shared, int32_t hidden, int32_t fp8,
                              int32_t phases, void* stream);
