@@ -97,14 +97,17 @@ struct GemmArgs {
                                 // is left goes to the other kernel as 128-row half tiles if that pays (tail_tiles)
 };
 
-// What a launch works on: the routed experts and, in front of them, a second problem of one expert with matrices, sizes and
-// buffers of its own, the layer's shared expert: its `shared_tiles` tiles (units) of the one-workgroup-per-tile or the thin
-// kernel, its `shared_ptiles` tiles of the persistent kernel.  A launch pair for the shared expert alone has a tile for a
-// fraction of the CUs at small batches (DeepSeek-V2-236B, 64 tokens: 24 and 20 tiles, 70 + 44 us for 94 MB) and rounds of its own
-// that end part-filled at larger ones.
+// What a launch works on: the routed experts and a second problem of one expert with matrices, sizes and buffers of its own,
+// the layer's shared expert.  A launch pair for the shared expert alone has a tile for a fraction of the CUs at small batches
+// (DeepSeek-V2-236B, 64 tokens: 24 and 20 tiles, 70 + 44 us for 94 MB) and rounds of its own that end part-filled at larger ones.
+// The host knows a bound of its rows, the kernels its rows (offsets[], like every expert's):
+//  * one kernel serves the call: `shared_tiles` workgroups in front of the routed experts' are the shared expert's; those past
+//    its rows return at once.
+//  * both kernels do: `shared_rows` > 0 bounds its rows, and each kernel counts its tiles as it does any expert's (persistent
+//    kernel: in front of the routed experts'; the other one: behind them, in front of the half tiles).
 struct GemmPair {
     GemmArgs p[2];              // routed, shared
-    int shared_tiles, shared_ptiles;
+    int shared_tiles, shared_rows;
 };
 
 // LDS rows are 128 bytes = 8 chunks of 16 bytes; chunk c of row r is stored at chunk c ^ swz(r).
@@ -1225,6 +1228,18 @@ __host__ __device__ __forceinline__ int own_tiles(const GemmArgs& g, int c) {
     return (g.rem_split ? c > g.cold_max : !is_cold(g, c)) ? 0 : tiles_of<!W8>(c);
 }
 
+// The shared expert's rows and its tiles in the spaces of the two kernels when both run, all 0 without one
+struct SharedTiles { int first, end, own, persistent; };
+template <bool W8>
+__host__ __device__ __forceinline__ SharedTiles shared_tiles_of(const GemmArgs& g, int first, int end) {
+    return SharedTiles{first, end, own_tiles<W8>(g, end - first) * g.n_tiles_n, persistent_tiles(g, end - first) * g.n_tiles_n};
+}
+// The most tiles of each kind that up to `rows` rows can have (fewer rows can have more: 200 rows one 256-row tile, 300 none)
+template <bool W8>
+inline SharedTiles shared_tiles_bound(const GemmArgs& g, int rows) {
+    return SharedTiles{0, rows, (!W8 && rows >= PAIR_LO ? 2 : 1) * g.n_tiles_n, rows > g.cold_max ? ((rows + 255) >> 8) * g.n_tiles_n : 0};
+}
+
 // sum over the experts of f(count) (every thread gets it; two barriers)
 template <int NT, typename F>
 __device__ __forceinline__ int sum_over_experts(const GemmArgs& g, int tid, int* s_wtot, F f) {
@@ -1449,36 +1464,50 @@ __global__ __launch_bounds__(128 * WN) void grouped_gemm_kernel(GemmPair pair_of
     // the number of tiles and however much one expert's tiles cost more than another's ----
     const int slot = blockIdx.x >> 3;
     int v = (((slot >> 2) << 3) + (blockIdx.x & 7)) * 4 + (slot & 3);
-    const bool of_shared = v < pair_of.shared_tiles;
-    if (!of_shared) v -= pair_of.shared_tiles;
-    const GemmArgs* gp = &pair_of.p[of_shared ? 1 : 0];
+    const bool in_front = v < pair_of.shared_tiles;
+    if (!in_front) v -= pair_of.shared_tiles;
+    int problem = in_front ? 1 : 0;
 
     // ---- M-tile prefix over experts ----
+    const GemmArgs& ga = pair_of.p[problem];
+    int shared_first = 0, shared_end = 0;    // (requested here, so that the answer comes with that to the scan's loads)
+    if (pair_of.shared_rows > 0) {
+        shared_first = pair_of.p[1].offsets[0];
+        shared_end = pair_of.p[1].offsets[1];
+    }
     ExpertOfThread mine;
-    int run = mtile_prefix_scan<NT>(*gp, tid, s_pref, s_wtot, mine, [&](int c) { return own_tiles<W8>(*gp, c); }, [](int, int, int) {});
-    const int total = run * gp->n_tiles_n;
+    int run = mtile_prefix_scan<NT>(ga, tid, s_pref, s_wtot, mine, [&](int c) { return own_tiles<W8>(ga, c); }, [](int, int, int) {});
+    const int total = run * ga.n_tiles_n;
 
-    // Past this kernel's own tiles: the tiles that the persistent kernel leaves at the end of ITS tile space, two
-    // workgroups (128-row halves, neighbours on one XCD) per tile.  The prefix is rebuilt over that space.
+    // Past the routed experts' tiles, where the persistent kernel runs too: the shared expert's, and then the tiles that the
+    // persistent kernel leaves at the end of ITS tile space, two workgroups (128-row halves, neighbours on one XCD) per
+    // tile.  The prefix is rebuilt over that space.
     int half = -1;
     if (v >= total) {
-        if (of_shared || gp->tail_cus <= 0 || gp->E > NT) return;
-        const int t = v - total;
-        __syncthreads();                 // s_wtot of the first scan has been read by everyone
-        run = mtile_prefix_scan<NT>(*gp, tid, s_pref, s_wtot, mine, [&](int c) { return persistent_tiles(*gp, c); }, [](int, int, int) {});
-        const int total_p = run * gp->n_tiles_n + pair_of.shared_ptiles;
-        const int tail = tail_tiles(*gp, total_p, total + pair_of.shared_tiles);
-        if (t >= 2 * tail) return;
-        v = total_p - tail + (t >> 1);
-        half = t & 1;
-        if (v < pair_of.shared_ptiles) {             // the shared expert's: its one expert belongs to thread 0
-            gp = &pair_of.p[1];
-            mine = ExpertOfThread{0, tid == 0 ? pair_of.shared_ptiles / gp->n_tiles_n : 0, gp->offsets[0], gp->offsets[1]};
+        if (in_front || ga.tail_cus <= 0 || ga.E > NT) return;
+        SharedTiles s{0, 0, 0, 0};
+        if (pair_of.shared_rows > 0) s = shared_tiles_of<W8>(pair_of.p[1], uni(shared_first), uni(shared_end));
+        v -= total;
+        int shared = s.own;                          // of the shared expert in the tile space that v counts in
+        if (v >= shared) {
+            const int t = v - shared;
+            __syncthreads();             // s_wtot of the first scan has been read by everyone
+            run = mtile_prefix_scan<NT>(ga, tid, s_pref, s_wtot, mine, [&](int c) { return persistent_tiles(ga, c); }, [](int, int, int) {});
+            shared = s.persistent;
+            const int total_p = run * ga.n_tiles_n + shared;
+            const int tail = tail_tiles(ga, total_p, total + s.own);
+            if (t >= 2 * tail) return;
+            v = total_p - tail + (t >> 1);
+            half = t & 1;
+        }
+        if (v < shared) {                            // its one expert belongs to thread 0
+            problem = 1;
+            mine = ExpertOfThread{0, tid == 0 ? shared / pair_of.p[1].n_tiles_n : 0, s.first, s.end};
         } else {
-            v -= pair_of.shared_ptiles;
+            v -= shared;
         }
     }
-    const GemmArgs& g = *gp;
+    const GemmArgs& g = pair_of.p[problem];
     const bool s8_ok = !g.row_map || g.a_bytes < (1ull << 32);   // (the weight streamer addresses gathered rows with 32-bit offsets)
     const int q = v / g.n_tiles_n;  // global M-tile number
     // find e with prefix[e] <= q < prefix[e+1].  Up to NT experts every thread still holds its own
@@ -1877,7 +1906,6 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmPair p
         s_ptr[2][e] = W8 ? (unsigned long long)(uintptr_t)g.s0[e] : 0ull;
         s_ptr[3][e] = (W8 && SWIGLU) ? (unsigned long long)(uintptr_t)g.s1[e] : 0ull;
     });
-    const int ptiles1 = PAIRED ? pair_of.shared_ptiles : 0;
     if (tid == 0) s_pref[g.E] = run;
     if (PAIRED && tid == 0) {
         const GemmArgs& s = pair_of.p[1];
@@ -1890,7 +1918,9 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmPair p
     }
     __syncthreads();
     // whole rounds, and the last one unless it is better off with the other kernel, whose own tiles are counted for that
-    const int own = g.tail_cus > 0 ? sum_over_experts<NT>(g, tid, s_wtot, [&](int c) { return own_tiles<W8>(g, c); }) * g.n_tiles_n + pair_of.shared_tiles : 0;
+    const SharedTiles second_tiles = PAIRED ? shared_tiles_of<W8>(pair_of.p[1], uni(s_off1[0]), uni(s_off1[1])) : SharedTiles{0, 0, 0, 0};
+    const int ptiles1 = second_tiles.persistent;
+    const int own = g.tail_cus > 0 ? sum_over_experts<NT>(g, tid, s_wtot, [&](int c) { return own_tiles<W8>(g, c); }) * g.n_tiles_n + second_tiles.own : 0;
     const int all = run * g.n_tiles_n + ptiles1, total = all - tail_tiles(g, all, own);
     const int xcd = blockIdx.x & 7, slots = gridDim.x >> 3;
     int slot = blockIdx.x >> 3;
@@ -2245,7 +2275,8 @@ int launch_tiles(const GemmPair& pair, int n_rows, hipStream_t st) {
     // sum_e tiles_of(c_e) <= sum_e (c_e / 128 + 1); with the larger experts elsewhere, one tile per expert that has rows
     const long max_mtiles = g.cold_max <= 192 ? (g.pair_rows ? 2 : 1) * (long)(g.E < n_rows ? g.E : n_rows) : (long)n_rows / 128 + g.E;
     // (+ the persistent kernel's last tiles, less than a round of them, as two half tiles each)
-    const long grid = ((max_mtiles * g.n_tiles_n + pair.shared_tiles + 2 * g.tail_cus + 31) / 32) * 32;   // whole rounds of 8 groups of 4 tiles
+    const int shared = pair.shared_rows > 0 ? shared_tiles_bound<W8>(pair.p[1], pair.shared_rows).own : pair.shared_tiles;
+    const long grid = ((max_mtiles * g.n_tiles_n + shared + 2 * g.tail_cus + 31) / 32) * 32;   // whole rounds of 8 groups of 4 tiles
     if (grid > 0x7fffffffL) {
         set_error("grouped gemm: %ld workgroups exceed the grid limit", grid);
         return MOE_ERR_INVALID;
@@ -2291,10 +2322,11 @@ template <bool SWIGLU, bool W8>
 int launch_persistent(const GemmPair& pair, int n_rows, hipStream_t st) {
     const GemmArgs& g = pair.p[0];
     const long max_mtiles = (long)n_rows / 256 + g.E;
-    long grid = ((max_mtiles * g.n_tiles_n + pair.shared_ptiles + 7) / 8) * 8;
+    const int shared = pair.shared_rows > 0 ? shared_tiles_bound<W8>(pair.p[1], pair.shared_rows).persistent : 0;
+    long grid = ((max_mtiles * g.n_tiles_n + shared + 7) / 8) * 8;
     const long ncu = (cu_count() / 8) * 8;
     if (grid > ncu) grid = ncu;
-    if (pair.shared_ptiles > 0) hipLaunchKernelGGL((grouped_gemm_persistent_kernel<SWIGLU, W8, true>), dim3((unsigned)grid), dim3(512), 0, st, pair);
+    if (pair.shared_rows > 0) hipLaunchKernelGGL((grouped_gemm_persistent_kernel<SWIGLU, W8, true>), dim3((unsigned)grid), dim3(512), 0, st, pair);
     else hipLaunchKernelGGL((grouped_gemm_persistent_kernel<SWIGLU, W8, false>), dim3((unsigned)grid), dim3(512), 0, st, pair);
     MOE_HIP_CHECK(hipGetLastError());
     return MOE_OK;
@@ -2437,8 +2469,7 @@ int launch_joint(const GemmArgs& routed, int n_rows, int max_rows, const GemmArg
     }
     pair.p[0] = both_kernels<W8>(routed);
     pair.p[1] = both_kernels<W8>(shared);
-    pair.shared_tiles = own_tiles<W8>(pair.p[1], n_shared) * shared.n_tiles_n;
-    pair.shared_ptiles = persistent_tiles(pair.p[1], n_shared) * shared.n_tiles_n;
+    pair.shared_rows = n_shared;
     return launch_both<SWIGLU, W8>(pair, n_rows, st);
 }
 

@@ -894,6 +894,51 @@ def test_shared_expert_in_the_launches_of_both_kernels(fp8, n, E, I, shared_inte
     assert torch.equal(y1, y2) and torch.equal(sh1, sh2)
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("E", [2, 16])          # routed experts of 256 rows (both kernels) and of 32 (one kernel)
+@pytest.mark.parametrize("n_rows,rows", [
+    (192, 150), (300, 150), (300, 200), (384, 200), (384, 260), (600, 0), (600, 150), (600, 200), (600, 300), (600, 384), (600, 500),
+    (1100, 513)])
+def test_joint_call_with_fewer_shared_rows_than_its_bound(fp8, E, n_rows, rows):
+    """n_rows bounds the shared expert's rows, offsets[] has them: its tiles follow the rows, on both sides of 192, 256 and 384, and
+    rows past them are neither read (NaN) nor written.  Bit for bit a call of its own with the same arguments (one kernel, fp8
+    weights: the joint call with the exact bound, the call of its own starts its sums elsewhere)."""
+    from moe_gen_amd import ops
+    n, k, h, I = 256, 2, 256, 384
+    print(f"joint, rows below the bound fp8={fp8} E={E} n_rows={n_rows} rows={rows}", flush=True)
+    g = torch.Generator().manual_seed(n_rows + rows)
+    dev = lambda m: tuple(t.cuda() for t in m) if isinstance(m, tuple) else m.cuda()
+    tables = []
+    for count, seed in ((E, 21), (1, 22)):
+        dm = [[dev(m) for m in one] for one in make_experts(count, h, I, fp8, seed)]
+        col = lambda i, j: [o[i][j] if fp8 else o[i] for o in dm]
+        tables.append(ops.expert_pointers(*(col(i, 0) for i in range(3)), *((col(i, 1) for i in range(3)) if fp8 else ())))
+    idx = torch.rand((n, E), generator=g).topk(k, dim=1).indices.to(torch.int32)
+    x = torch.randn(n, h, generator=g).to(torch.bfloat16).cuda()
+    xs = torch.randn(n_rows, h, generator=g).to(torch.bfloat16)
+    xs[rows:] = float("nan")
+    xs = xs.cuda()
+    d = ops.dispatch(idx.cuda(), E, None, want_row_map=True)
+    so = torch.tensor([0, rows], dtype=torch.int32, device="cuda")
+    def call(bound, joint):
+        r, _, y = ops.mlp_group(x, d.row_map, tables[0], d.offsets, n * k, n)
+        s, _, sh = ops.mlp_group(xs, None, tables[1], so, bound)
+        y.fill_(7.0); sh.fill_(7.0)
+        if joint:
+            assert ops.shared_joins(r, s, h)
+            ops.grouped_swiglu_joint(r, s, h, fp8)
+        else:
+            ops.grouped_swiglu_joint(r, None, h, fp8)
+            ops.grouped_swiglu_joint(s, None, h, fp8)
+        torch.cuda.synchronize()
+        return y, sh
+    y1, sh1 = call(n_rows, True)
+    y2, sh2 = call(n_rows, False) if E == 2 or not fp8 or rows == 0 else call(rows, True)
+    assert torch.equal(y1, y2)
+    assert torch.equal(sh1[:rows], sh2[:rows]) and torch.isfinite(sh1[:rows].float()).all()
+    assert (sh1[rows:] == 7.0).all()
+
+
 @pytest.mark.parametrize("left", [1, 72, 192])
 def test_dense_fp8_leftover_rows_as_a_padded_tile(left):
     """One fp8 MLP of 11 full tiles and a leftover whose gate and up tiles (240 of 128 columns with the leftover's) fit one round
