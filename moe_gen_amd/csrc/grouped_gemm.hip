@@ -93,6 +93,8 @@ struct GemmArgs {
                                 // instead of to its count: the persistent kernel takes the full tiles, and the
                                 // last, ragged one only if it holds more than cold_max rows
     int pair_rows;              // 1: experts of PAIR_LO .. PAIR_HI rows also belong to the one-workgroup-per-tile kernel
+    int alone;                  // 1 (fp8): no other kernel's sums have to be matched: k_rotation, and the stage order of
+                                // stream8_tile for tiles of up to 64 rows
     int tail_cus;               // > 0: the persistent kernel runs whole rounds of this many tiles (one per CU); what
                                 // is left goes to the other kernel as 128-row half tiles if that pays (tail_tiles)
 };
@@ -123,8 +125,8 @@ __device__ __forceinline__ int swz(int row) { return (row & 7) ^ ((row >> 3) & 1
 // TB/s; 128 / 160 / 192 rows next to the persistent kernel: gate/up 0.63 / 0.64 / 0.66 -> 0.55 / 0.58 / 0.62 ms).
 // bf16 weights: every path of both kernels uses this rule, so which kernel or tile computes a row does not change the
 // order its products are added in (the persistent kernel itself runs within 0.5 % either way).  fp8 weights (a scale
-// per 128 k: pairs of stages stay together): only in calls that the one-workgroup-per-tile kernel serves alone; the
-// persistent kernel loses 1.6 % of the DeepSeek-V3 step to a rotated walk, so calls that launch it start every tile
+// per 128 k: pairs of stages stay together): only in calls that the one-workgroup-per-tile kernel serves alone (and not for
+// a large shared expert in them, joint_alone); the persistent kernel loses 1.6 % of the DeepSeek-V3 step to a rotated walk, so calls that launch it start every tile
 // at stage 0, in both kernels.
 template <bool W8>
 __device__ __forceinline__ int k_rotation(int n_tile, int nk) { return (W8 ? 2 * n_tile : n_tile) % nk; }
@@ -1548,21 +1550,20 @@ __global__ __launch_bounds__(128 * WN) void grouped_gemm_kernel(GemmPair pair_of
     }
     const int row_end = uni(s_sel[4]);
     const int first_row = uni(s_sel[3]) + (g.rem_split ? ((row_end - uni(s_sel[3])) & ~255) : 0);
-    const bool alone = g.cold_max == 0x7fffffff;
     if (W8 && s8_ok) {
-        // fp8 weights: the weight streamers.  Up to 64 rows in a call that this kernel has to itself, where no other
-        // kernel's summation order has to be matched: the form that reads a lane's 16 weights at once.  Everything
-        // else -- up to 192 rows; what an expert's full 256-row tiles leave over; 128-row slices of larger experts
-        // when the kernel is alone -- in the persistent kernel's order.
+        // fp8 weights: the weight streamers.  Up to 64 rows where no other kernel's summation order has to be matched: the
+        // form that reads a lane's 16 weights at once.  Everything else -- up to 192 rows; what an expert's full 256-row
+        // tiles leave over; 128-row slices of larger experts when the kernel serves the call by itself -- in the
+        // persistent kernel's order.
         const int r0 = first_row + (mt_e > 1 ? m_tile * 128 : 0), r1 = mt_e > 1 ? min(row_end, r0 + 128) : row_end;
         const int rows = r1 - r0;
-        if (alone && mt_e == 1 && rows <= 64) {
+        if (g.alone && mt_e == 1 && rows <= 64) {
             if (rows <= 16) stream8_tile<1, SWIGLU>(g, sb0, sb1, sb2, e, r0, r1, n_tile);
             else if (rows <= 32) stream8_tile<2, SWIGLU>(g, sb0, sb1, sb2, e, r0, r1, n_tile);
             else if (rows <= 48) stream8_tile<3, SWIGLU>(g, sb0, sb1, sb2, e, r0, r1, n_tile);
             else stream8_tile<4, SWIGLU>(g, sb0, sb1, sb2, e, r0, r1, n_tile);
         } else {
-            stream8x<SWIGLU>(g, lds, e, r0, r1, n_tile, alone);
+            stream8x<SWIGLU>(g, lds, e, r0, r1, n_tile, g.alone);
         }
         return;
     }
@@ -2389,6 +2390,7 @@ inline bool persistent_fits(const GemmArgs& g) { return g.K % 128 == 0 && g.E <=
 // the rules by which a call's tiles fall to the two kernels (reasons in launch_mt)
 template <bool W8>
 GemmArgs both_kernels(GemmArgs g) {
+    g.alone = 0;
     g.cold_max = 192;
     g.rem_split = W8 ? 1 : 0;
     g.pair_rows = W8 ? 0 : 1;
@@ -2416,6 +2418,7 @@ int launch_mt(const GemmArgs& g0, int n_rows, int max_rows, void* workspace, siz
     GemmPair pair{};
     if (mean < 128 || !persistent_fits(g)) {
         g.cold_max = 0x7fffffff;
+        g.alone = 1;
         pair.p[0] = g;
         return launch_tiles<4, SWIGLU, W8>(pair, n_rows, st);
     }
@@ -2457,13 +2460,14 @@ int launch_mt(const GemmArgs& g0, int n_rows, int max_rows, void* workspace, siz
     return launch_both<SWIGLU, W8>(pair, n_rows, st);
 }
 
-// The shared expert's tiles in the routed experts' launches.
+// The shared expert's tiles in the routed experts' launches.  shared.alone: see joint_alone.
 template <bool SWIGLU, bool W8>
 int launch_joint(const GemmArgs& routed, int n_rows, int max_rows, const GemmArgs& shared, int n_shared, hipStream_t st) {
     if (max_rows <= 16 && n_shared <= 16 && thin_pays(routed, n_rows, &shared)) return launch_thin<SWIGLU, W8>(routed, n_rows, &shared, st);
     GemmPair pair{{routed, shared}, 0, 0};
     if (n_rows / routed.E < 128) {
         pair.p[0].cold_max = pair.p[1].cold_max = 0x7fffffff;
+        pair.p[0].alone = 1;
         pair.shared_tiles = tiles_of<!W8>(n_shared) * shared.n_tiles_n;
         return launch_tiles<4, SWIGLU, W8>(pair, n_rows, st);
     }
@@ -2531,6 +2535,15 @@ bool joins(const moe_mlp_group& routed, const moe_mlp_group& shared, int32_t hid
     return (long)((shared.n_rows + 127) / 128) * ((shared.inter + 127) / 128) <= 2L * cu_count();
 }
 
+// fp8 weights, a joint call that one kernel serves: whether the shared expert's sums start at the stages of that kernel's own
+// calls.  They do where it is small, 256-row tiles for less than 3/8 of the CUs, and where a call of its own would do the same (a
+// mean below 128); else at stage 0, as in a call of its own, whose bits it then has.  DeepSeek-V3, us, 1300 /
+// 1500 / 2997 / 4000 tokens (all of the second kind): started as the first kind 2337 / 2437 / 3387 / 4082, at stage 0
+// 2340 / 2449 / 3392 / 4081.
+int joint_alone(const moe_mlp_group& shared) {
+    return shared.n_rows < 128 || (long)(shared.n_rows / 256 + 1) * ((shared.inter + 127) / 128) * 8 < 3L * cu_count();
+}
+
 template <bool W8>
 int grouped_swiglu(const moe_mlp_group& m, int32_t hidden, int32_t phases, void* stream, const char* who) {
     MOE_REQUIRE(phases >= MOE_PHASE_GATE_UP && phases <= MOE_PHASE_BOTH, "%s: bad phases %d", who, phases);
@@ -2555,10 +2568,12 @@ int grouped_swiglu_joint(const moe_mlp_group& r, const moe_mlp_group& s, int32_t
         return rc != MOE_OK ? rc : grouped_swiglu<W8>(s, hidden, phases, stream, who);
     }
     hipStream_t st = as_stream(stream);
+    GemmArgs gate_up = gate_up_args(s, hidden), down = down_args(s, hidden);
+    gate_up.alone = down.alone = joint_alone(s);
     if (phases & MOE_PHASE_GATE_UP)
-        rc = launch_joint<true, W8>(gate_up_args(r, hidden), r.n_rows, row_bound(r), gate_up_args(s, hidden), s.n_rows, st);
+        rc = launch_joint<true, W8>(gate_up_args(r, hidden), r.n_rows, row_bound(r), gate_up, s.n_rows, st);
     if (rc == MOE_OK && (phases & MOE_PHASE_DOWN))
-        rc = launch_joint<false, W8>(down_args(r, hidden), r.n_rows, row_bound(r), down_args(s, hidden), s.n_rows, st);
+        rc = launch_joint<false, W8>(down_args(r, hidden), r.n_rows, row_bound(r), down, s.n_rows, st);
     return rc;
 }
 

@@ -939,6 +939,35 @@ def test_joint_call_with_fewer_shared_rows_than_its_bound(fp8, E, n_rows, rows):
     assert (sh1[rows:] == 7.0).all()
 
 
+@pytest.mark.parametrize("n,shared_inter", [(280, 6144), (500, 6144), (700, 4096)])     # the least sizes of the rule
+def test_large_fp8_shared_expert_in_a_one_kernel_call_has_the_bits_of_its_own_call(n, shared_inter):
+    """Below a mean of 128 rows per routed expert a shared expert of 3/8 of the CUs' worth of 256-row tiles or more is summed as in a
+    call of its own, where both kernels run.  Last tiles of 24, 116 and 60 rows."""
+    from moe_gen_amd import ops
+    E, k, h, I = 12, 2, 256, 128
+    print(f"large shared expert n={n} shared_inter={shared_inter}", flush=True)
+    g = torch.Generator().manual_seed(n)
+    tables = []
+    for count, inter, seed in ((E, I, 41), (1, shared_inter, 42)):
+        dm = [[tuple(t.cuda() for t in m) for m in one] for one in make_experts(count, h, inter, True, seed)]
+        col = lambda i, j: [o[i][j] for o in dm]
+        tables.append(ops.expert_pointers(*(col(i, 0) for i in range(3)), *(col(i, 1) for i in range(3))))
+    idx = torch.rand((n, E), generator=g).topk(k, dim=1).indices.to(torch.int32)
+    x = torch.randn(n, h, generator=g).to(torch.bfloat16).cuda()
+    d = ops.dispatch(idx.cuda(), E, None, want_row_map=True)
+    so = torch.tensor([0, n], dtype=torch.int32, device="cuda")
+    r1, _, y1 = ops.mlp_group(x, d.row_map, tables[0], d.offsets, n * k, n)
+    s1, _, sh1 = ops.mlp_group(x, None, tables[1], so, n)
+    assert ops.shared_joins(r1, s1, h)
+    ops.grouped_swiglu_joint(r1, s1, h, True)
+    r2, _, y2 = ops.mlp_group(x, d.row_map, tables[0], d.offsets, n * k, n)
+    s2, _, sh2 = ops.mlp_group(x, None, tables[1], so, n)
+    ops.grouped_swiglu_joint(r2, None, h, True)
+    ops.grouped_swiglu_joint(s2, None, h, True)
+    torch.cuda.synchronize()
+    assert torch.equal(y1, y2) and torch.equal(sh1, sh2)
+
+
 @pytest.mark.parametrize("left", [1, 72, 192])
 def test_dense_fp8_leftover_rows_as_a_padded_tile(left):
     """One fp8 MLP of 11 full tiles and a leftover whose gate and up tiles (240 of 128 columns with the leftover's) fit one round
