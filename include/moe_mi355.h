@@ -240,10 +240,10 @@ size_t moe_mlp_workspace_bytes(const moe_mlp_group* group, int32_t hidden);
  * The routed experts and the shared expert(s) of a layer (DeepseekV3MoE.forward, modeling_deepseek_v3.py:618-625; one MLP
  * of any intermediate size, n_experts == 1) in one call, both of the same weight type (fp8 != 0: fp8 with block scales).
  * Where moe_shared_joins says 1 they share their launches: the shared expert's tiles run next to the routed experts';
- * otherwise they run one after the other.  shared == NULL: the routed experts alone.  The bits are those of separate calls
- * without scratch, but for one case: with fp8 weights, below a mean of 128 rows per routed expert, a shared expert of 128
- * rows or more that is small (256-row tiles for less than 3/8 of the CUs) starts its sums at other stages than a call
- * of its own does.
+ * otherwise they run one after the other.  shared == NULL: the routed experts alone.  The bits are those of separate calls,
+ * but for one case: with fp8 weights, below a mean of 128 rows per routed expert, a shared expert that is small (256-row
+ * tiles for less than 3/8 of the CUs) starts its sums at other stages than a call of its own with 128 rows or more does,
+ * and is not cut into slices of k as that is if it brings scratch.
  */
 int moe_grouped_swiglu_joint(const moe_mlp_group* routed, const moe_mlp_group* shared, int32_t hidden, int32_t fp8,
                              int32_t phases, void* stream);

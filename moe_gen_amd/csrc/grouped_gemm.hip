@@ -2519,9 +2519,20 @@ GemmArgs down_args(const moe_mlp_group& m, int32_t hidden) {
 // no expert of the group has more rows than this
 int row_bound(const moe_mlp_group& m) { return m.max_rows > 0 && m.max_rows < m.n_rows ? m.max_rows : m.n_rows; }
 
-// Whether the shared expert's tiles join the routed experts' launches.  Where the routed call goes to both kernels they
-// do, up to four rounds of tiles of its own (beyond, the same within 0.2 %): the two then fill their last rounds together.  Where it is one that the one-workgroup-per-tile kernel (or the thin
-// one) serves alone, whose 128-row tiles would be all the shared expert gets, up to two such tiles per CU.
+// Whether a call of the group by itself, with the scratch that it brings, cuts its down projection into slices of k
+bool sliced(const moe_mlp_group& m, int32_t hidden) {
+    const size_t need = moe_mlp_workspace_bytes(&m, hidden);
+    return need > 0 && m.workspace && m.workspace_bytes >= need;
+}
+
+// Whether 256-row tiles of the group (its gate and up projection) are fewer than 3/8 of the CUs
+bool few_tiles(const moe_mlp_group& m) { return (long)(m.n_rows / 256 + 1) * ((m.inter + 127) / 128) * 8 < 3L * cu_count(); }
+
+// Whether the shared expert's tiles join the routed experts' launches.  Where the routed call goes to both kernels they do if a
+// call of its own would go to both as well (128 rows, no slices of k), up to four rounds of tiles of its own (beyond, the same
+// within 0.2 %): the two then fill their last rounds together.  Where the routed call is one that the one-workgroup-per-tile
+// kernel (or the thin one) serves alone, a few tiles always do; more of them up to two of that kernel's 128-row tiles, all that
+// the shared expert gets there, per CU, unless its own call is in slices.
 // Layers, us, apart -> joined.  Both kernels: DeepSeek-V2-Lite 1400 / 2000 / 2777 / 4096 tokens 439 / 514 / 585 / 725 -> 397 / 470 /
 // 563 / 699; DeepSeek-V3 4096 / 6000 4046 / 5498 -> 4004 / 5367, 16384 the same.  One kernel: DeepSeek-V2-Lite 1024 / 1300 366 /
 // 409 -> 322 / 351; DeepSeek-V2-236B 1024 / 1500 1463 / 1641 -> 1416 / 1615, 2048 the same, 3000 2074 -> 2090 (not joined: 576 tiles);
@@ -2530,9 +2541,11 @@ bool joins(const moe_mlp_group& routed, const moe_mlp_group& shared, int32_t hid
     if (routed.n_rows < 1 || shared.n_rows < 1 || routed.n_experts < 1 || shared.n_experts != 1 || hidden < 1) return false;
     if (routed.row_map && (size_t)routed.x_rows * (size_t)hidden * 2 >= (1ull << 32)) return false;
     if (shared.row_map && (size_t)shared.x_rows * (size_t)hidden * 2 >= (1ull << 32)) return false;
+    const long cus = cu_count(), cols = (shared.inter + 127) / 128, rows = shared.n_rows;
     if (routed.n_rows / routed.n_experts >= 128)
-        return (long)((shared.n_rows + 255) / 256) * ((shared.inter + 127) / 128) <= 4L * cu_count() && hidden % 128 == 0 && routed.inter % 128 == 0 && shared.inter % 128 == 0 && routed.n_experts <= 512 && cu_count() >= 8;
-    return (long)((shared.n_rows + 127) / 128) * ((shared.inter + 127) / 128) <= 2L * cu_count();
+        return rows >= 128 && (rows + 255) / 256 * cols <= 4 * cus && hidden % 128 == 0 && routed.inter % 128 == 0 &&
+               shared.inter % 128 == 0 && routed.n_experts <= 512 && cus >= 8 && !sliced(shared, hidden);
+    return few_tiles(shared) || ((rows + 127) / 128 * cols <= 2 * cus && !sliced(shared, hidden));
 }
 
 // fp8 weights, a joint call that one kernel serves: whether the shared expert's sums start at the stages of that kernel's own
@@ -2540,9 +2553,7 @@ bool joins(const moe_mlp_group& routed, const moe_mlp_group& shared, int32_t hid
 // mean below 128); else at stage 0, as in a call of its own, whose bits it then has.  DeepSeek-V3, us, 1300 /
 // 1500 / 2997 / 4000 tokens (all of the second kind): started as the first kind 2337 / 2437 / 3387 / 4082, at stage 0
 // 2340 / 2449 / 3392 / 4081.
-int joint_alone(const moe_mlp_group& shared) {
-    return shared.n_rows < 128 || (long)(shared.n_rows / 256 + 1) * ((shared.inter + 127) / 128) * 8 < 3L * cu_count();
-}
+int joint_alone(const moe_mlp_group& shared) { return shared.n_rows < 128 || few_tiles(shared); }
 
 template <bool W8>
 int grouped_swiglu(const moe_mlp_group& m, int32_t hidden, int32_t phases, void* stream, const char* who) {

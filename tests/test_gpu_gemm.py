@@ -968,6 +968,44 @@ def test_large_fp8_shared_expert_in_a_one_kernel_call_has_the_bits_of_its_own_ca
     assert torch.equal(y1, y2) and torch.equal(sh1, sh2)
 
 
+@pytest.mark.parametrize("E,rows,shared_inter,scratch", [
+    (12, 17, 12288, True),     # one kernel for the routed experts, slices of k for the shared one
+    (2, 300, 4096, True),      # both kernels
+    (2, 100, 640, False)])     # both kernels, and one that would start its sums elsewhere
+def test_joint_call_leaves_apart_what_its_own_call_sums_in_another_way(E, rows, shared_inter, scratch):
+    """fp8.  Bit for bit two separate calls on the same groups, scratch included."""
+    from moe_gen_amd import _native as N
+    from moe_gen_amd import ops
+    import ctypes
+    n, k, h, I = 256, 2, 512, 128
+    print(f"apart E={E} rows={rows} shared_inter={shared_inter} scratch={scratch}", flush=True)
+    g = torch.Generator().manual_seed(rows)
+    tables = []
+    for count, inter, seed in ((E, I, 51), (1, shared_inter, 52)):
+        dm = [[tuple(t.cuda() for t in m) for m in one] for one in make_experts(count, h, inter, True, seed)]
+        col = lambda i, j: [o[i][j] for o in dm]
+        tables.append(ops.expert_pointers(*(col(i, 0) for i in range(3)), *(col(i, 1) for i in range(3))))
+    idx = torch.rand((n, E), generator=g).topk(k, dim=1).indices.to(torch.int32)
+    x = torch.randn(n, h, generator=g).to(torch.bfloat16).cuda()
+    xs = torch.randn(rows, h, generator=g).to(torch.bfloat16).cuda()
+    d = ops.dispatch(idx.cuda(), E, None, want_row_map=True)
+    so = torch.tensor([0, rows], dtype=torch.int32, device="cuda")
+    out = []
+    for joint in (True, False):
+        r, _, y = ops.mlp_group(x, d.row_map, tables[0], d.offsets, n * k, n)
+        s, _, sh = ops.mlp_group(xs, None, tables[1], so, rows)
+        if scratch:
+            need = N.lib().moe_mlp_workspace_bytes(ctypes.byref(s), h)
+            ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+            assert need > 0
+            s.workspace, s.workspace_bytes = ws.data_ptr(), need
+        for a, b in ((r, s),) if joint else ((r, None), (s, None)):
+            ops.grouped_swiglu_joint(a, b, h, True)
+        torch.cuda.synchronize()
+        out.append((y, sh))
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+
+
 @pytest.mark.parametrize("left", [1, 72, 192])
 def test_dense_fp8_leftover_rows_as_a_padded_tile(left):
     """One fp8 MLP of 11 full tiles and a leftover whose gate and up tiles (240 of 128 columns with the leftover's) fit one round
