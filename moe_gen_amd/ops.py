@@ -32,9 +32,15 @@ class RouterSpec:
     weights_bf16: bool = False        # Mixtral: routing weights cast to bf16
 
 
+# torch.cuda.current_stream().cuda_stream without the Stream object around it, 3 to 5 us of a call's 60.  No part of torch's
+# public interface: a torch without it takes the public form.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream() -> int:
-    # torch.cuda.current_stream().cuda_stream without the Stream object around it (3 to 5 us of a call's 60)
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    if _raw_stream is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(torch.cuda.current_device())
 
 
 def _ptr(t):

@@ -1,6 +1,8 @@
 """Host-side behaviour of the blocks that needs no GPU: parameter tree, errors, no CPU fallback."""
 import copy
+import importlib.util
 import pickle
+import sys
 
 import pytest
 import torch
@@ -44,6 +46,19 @@ def test_no_cpu_fallback():
     with pytest.raises((RuntimeError, TypeError)):
         M.ops.router(torch.zeros(4, 16, dtype=torch.bfloat16), torch.zeros(8, 16, dtype=torch.bfloat16), None,
                      M.ops.RouterSpec(8, 2))
+
+
+def test_stream_handle_without_torchs_own_shortcut(monkeypatch):
+    """A torch that does not have the function for the raw handle: the operators take the public form."""
+    class Current:
+        cuda_stream = 0x1234
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: Current)
+    spec = importlib.util.spec_from_file_location("moe_gen_amd.ops_of_another_torch", ops.__file__)
+    fresh = importlib.util.module_from_spec(spec)
+    monkeypatch.setitem(sys.modules, spec.name, fresh)      # (its dataclasses look their module up)
+    spec.loader.exec_module(fresh)
+    assert fresh._stream() == 0x1234
 
 
 def test_pointer_tables_survive_a_copy():
