@@ -863,7 +863,9 @@ def test_shared_expert_in_the_routed_launches(fp8, n, shared_inter):
     (1500, 4, 128, 640),      # longer; all of the persistent kernel's tiles are half tiles, the shared expert's among them
     (3000, 8, 1280, 2560),    # rounds of tiles of both
     (2900, 3, 256, 2048),     # mostly the shared expert's
-    (200, 2, 256, 384)])      # one tile of up to 192 rows next to 256-row tiles
+    (200, 2, 256, 384),       # 200 rows each, one 256-row tile
+    (150, 2, 256, 384),       # 150 rows each, one tile of up to 192 rows: nothing for the persistent kernel
+    (300, 3, 256, 640)])      # bf16: two tiles of up to 192 rows next to a 256-row tile; fp8: 44 rows over a full tile
 def test_shared_expert_in_the_launches_of_both_kernels(fp8, n, E, I, shared_inter):
     """From a mean of 128 rows per expert on the shared expert's tiles come first in the launches of the persistent kernel and of
     the other one.  Bit for bit what the calls give apart, with fp8 weights too (both start every tile at k 0 there)."""
