@@ -166,7 +166,8 @@ int moe_dispatch_static(const int32_t* topk_idx, int32_t n_tokens, int32_t top_k
  * up to 192 rows run one workgroup per tile, at a tile height chosen per expert on the device in steps of 16 rows
  * (bf16 weights: also experts of 257 to 384 rows, as two such tiles);
  * larger experts run on 256-row tiles of persistent workgroups (with fp8 weights: their full 256-row tiles, and the
- * rows these leave over as one tile of the first kind if they are at most 192).  The persistent workgroups,
+ * rows these leave over as one tile of the first kind if they are at most 192; those of a single expert, E = 1, as a padded tile
+ * of the second kind where that shortens the call).  The persistent workgroups,
  * one per CU, take whole rounds of tiles; a last, partial round is cut into 128-row halves and runs with the first
  * kind when that shortens the two launches (alone: if it is at most half the CUs' worth of tiles).  Below a mean of 128 rows per expert (n_rows / E), with K not a multiple of
  * 128, with more than 512 experts or with 4 GiB or more of gathered x, the one-workgroup-per-tile kernel serves the
@@ -175,7 +176,7 @@ int moe_dispatch_static(const int32_t* topk_idx, int32_t n_tokens, int32_t top_k
  * computes it or on the call.  With fp8 weights that holds inside a call that launches both kernels, and two things
  * change the order in which a row's products are added, and with it the last bit: a call that the
  * one-workgroup-per-tile kernel serves alone starts its k loops at other stages, and there an expert of up to 64 rows
- * adds the products of a stage in another order than one of more.
+ * adds the products of a stage in another order than one of more.  (The scratch of moe_mlp_workspace_bytes changes it too.)
  * Calls in which no expert has more than 16 rows run on a kernel of one wave per 32 weight rows where that is the faster one.
  */
 enum { MOE_PHASE_GATE_UP = 1, MOE_PHASE_DOWN = 2, MOE_PHASE_BOTH = 3 };

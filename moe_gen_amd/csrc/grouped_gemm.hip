@@ -24,8 +24,8 @@
 //    A and B panels through that XCD's L2), and a workgroup's k pipeline runs on from one of
 //    its tiles into the next.
 //  * grouped_gemm_kernel (experts of up to 192 rows, and with fp8 weights what an expert's full 256-row tiles
-//    leave over if that is at most 192 rows; work that mostly streams weights): one
-//    workgroup per tile, grid = upper bound on the tile count, surplus workgroups exit at once;
+//    leave over if that is at most 192 rows, a single MLP's where a padded tile of the other kernel is not the
+//    shorter way; work that mostly streams weights): one workgroup per tile, grid = upper bound on the tile count, surplus workgroups exit at once;
 //    the tile height (16 ... 192 rows in steps of 16) follows the expert, groups of 4 tiles go round-robin
 //    to the XCDs.  Its tiles run through the weight streamers (stream16_tile, stream8x_tile, stream8_tile):
 //    weights AND token rows reach LDS by DMA, three weight buffers, one barrier per stage.
@@ -138,7 +138,6 @@ typedef const __attribute__((address_space(1))) u32x4* gptr_u32x4;
 typedef const __attribute__((address_space(1))) float* gptr_f32;
 typedef const __attribute__((address_space(1))) int32_t* gptr_i32;
 typedef __attribute__((address_space(3))) uint8_t* lds_u8;
-typedef const __attribute__((address_space(4))) float* cptr_f32;   // constant address space: uniform addresses become scalar loads
 
 __device__ __forceinline__ u32x4 gload16(const void* p) { return *(gptr_u32x4)(uintptr_t)p; }
 // Weights under the one-workgroup-per-tile kernel are streamed: a tile of them is used by one workgroup (two
@@ -916,9 +915,11 @@ __device__ __forceinline__ void stream8_tile(const GemmArgs& g, SBuf buf0, SBuf 
 // the LDS latency and the conversion stand beside matrix instructions instead of in front of them.  Slots run on across
 // the barriers; in front of the first one operands and accumulators are zero.
 //
-// What bounds it: the chip's power.  It runs at 1.7 to 1.8 GHz, and a half of 16 KiB of weights takes 1075 cycles and 126 more
-// for every 16 token rows: the stream and the products add up (96 / 176 rows: matrix cores 42 / 57 %, vector ALU 36 / 28 % of the
-// cycles).  Against one form each for up to 128 and up to 192 rows, in which every half read, converted and multiplied
+// What bounds it: a half of 16 KiB of weights takes 1075 cycles and 126 more for every 16 token rows, so the stream and the products
+// add up, and neither is busy (96 / 176 rows: matrix cores 42 / 57 %, vector ALU 36 / 28 % of the cycles).  The clock falls
+// little meanwhile (16 -> 176 rows 1.81 -> 1.71 GHz), and a CU takes 0.122 to 0.125 lines per cycle at every height (the persistent
+// kernel about 0.20): products that do not overlap the stream or token lines that queue with the weights' both fit; which of
+// them it is has not been established.  Against one form each for up to 128 and up to 192 rows, in which every half read, converted and multiplied
 // in turn, DeepSeek-V3 shapes, 256 experts, us: 96 rows each 1913 -> 1861 (gate and up), 1091 -> 1055 (down), 176 rows
 // 2782 -> 2583 and 1566 -> 1468; 512 rows each (leftovers of full tiles) 6144 -> 6082, 3247 -> 3226 for 64 experts.
 template <int TG, bool SWIGLU, bool SPLIT = false>   // TG: 16-row token groups multiplied (1 .. 12)
@@ -932,8 +933,8 @@ __device__ __forceinline__ void stream8x_tile(const GemmArgs& g, const TileLds& 
     constexpr int NS = SWIGLU ? 2 : 1;            // block scales of a wave's columns
     // Order of issue in half h of block p: the tokens two halves ahead (above 128 rows: one), h = 0: the scales of block p + 1, and
     // the weights of block p + 2 (all four instructions in h = 0; above 128 rows two in either half).  VM: DMA operations that may
-    // stay in flight at the barrier of a half, those issued after its tokens.  (The scales do not count: loads into registers
-    // may retire before older DMA, see the persistent kernel)
+    // stay in flight at the barrier of a half, those issued after its tokens.  (The scales do not count: nothing holds their
+    // place among the DMA, see the persistent kernel)
     constexpr int VM = WIDE ? 2 : 4 + NDT;
     static_assert(!(SPLIT && SWIGLU), "slices of k: the down projection");
     static_assert(TG >= 1 && TG <= 12, "token rows staged");
@@ -978,7 +979,7 @@ __device__ __forceinline__ void stream8x_tile(const GemmArgs& g, const TileLds& 
         if (row0 + tr >= row_end || (g.row_map && (unsigned)src >= (unsigned)g.a_rows)) t_voff[i] = 0xfffffff0u;
     }
     float rsc[3][2];                              // block scales, block p in set p % 3
-    auto scales = [&](int p_pipe, int set) __attribute__((always_inline)) {   // (buffer loads: the waits count them)
+    auto scales = [&](int p_pipe, int set) __attribute__((always_inline)) {   // (buffer loads: scalar ones share a counter with the operand reads)
 #pragma unroll
         for (int j = 0; j < NS; ++j) {
             const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)sc[j], 0, -1, 0x00020000);
@@ -1715,7 +1716,8 @@ __global__ __launch_bounds__(64) void grouped_gemm_thin_kernel(GemmPair pair_of)
         float v0 = 0.0f, v1 = 0.0f;                        // fp8: lane l holds the scales of stage 64 i + l
         if (W8) { v0 = sc0[stage_at(lane)]; v1 = sc1[stage_at(lane)]; }
         for (int i = 0; i < NB - 1; ++i) dma(i, i);
-        // (waits by hand: the compiler's own, in front of the readlane below, would cover the DMA of the next stage too)
+        // (waits by hand: the compiler's own, in front of the readlane below, would cover the DMA of the next stage too.  The
+        // scales were requested before the DMA; where the compiler moves them behind some of it, it waits for them here itself)
         if (W8) asm volatile("s_waitcnt vmcnt(%2)" : "+v"(v0), "+v"(v1) : "n"((NB - 1) * NI));
         int buf = 0;
         for (int k = 0; k < nk; ++k) {
@@ -2127,9 +2129,9 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmPair p
     //   bf16: slots 0-3 bring weights 2, 3 and tokens 2, 3 of stage k1 (= kt + 1), slots 4-7 tokens 0, 1 and weights 0, 1 of
     //   stage k2 (= kt + 2).  fp8: slots 0, 1 tokens 2, 3 of stage k1; slots 2-5 convert the weight registers (stage kt + 1)
     //   into the other weight buffer and refill them with stage k2; slots 6, 7 tokens 0, 1 of stage k2.
-    // Waits.  DMA into LDS retires in issue order, but loads into registers issued after it may retire before it (counted as in
-    // order, a DMA's rows were now and then read before they had landed, gathered ones first), and nothing is known of
-    // stores: the waits count DMA operations only, so whatever else is in flight makes them stricter.  VM_X: DMA
+    // Waits.  Loads retire in issue order, DMA into LDS and loads into registers alike (measured), but the compiler may move a
+    // load into registers across a DMA, and nothing is known of stores: the waits count DMA operations only, whose number
+    // and order the source fixes, so whatever else is in flight makes them stricter.  VM_X: DMA
     // issued after the last one that the first four slots read; VM_Y: after the last one that the others read; VM_TURN: after a
     // tile's first stage, waited for in front of the stores of the tile before, so that the first iteration need not wait.
     // first / second: the tile's first two iterations (sub-phases 6 and 7 of the first run in the second); turn: from the second
@@ -2526,7 +2528,7 @@ bool sliced(const moe_mlp_group& m, int32_t hidden) {
 }
 
 // Whether 256-row tiles of the group (its gate and up projection) are fewer than 3/8 of the CUs
-bool few_tiles(const moe_mlp_group& m) { return (long)(m.n_rows / 256 + 1) * ((m.inter + 127) / 128) * 8 < 3L * cu_count(); }
+bool few_tiles(const moe_mlp_group& m, long cus) { return (long)(m.n_rows / 256 + 1) * ((m.inter + 127) / 128) * 8 < 3 * cus; }
 
 // Whether the shared expert's tiles join the routed experts' launches.  Where the routed call goes to both kernels they do if a
 // call of its own would go to both as well (128 rows, no slices of k), up to four rounds of tiles of its own (beyond, the same
@@ -2545,7 +2547,7 @@ bool joins(const moe_mlp_group& routed, const moe_mlp_group& shared, int32_t hid
     if (routed.n_rows / routed.n_experts >= 128)
         return rows >= 128 && (rows + 255) / 256 * cols <= 4 * cus && hidden % 128 == 0 && routed.inter % 128 == 0 &&
                shared.inter % 128 == 0 && routed.n_experts <= 512 && cus >= 8 && !sliced(shared, hidden);
-    return few_tiles(shared) || ((rows + 127) / 128 * cols <= 2 * cus && !sliced(shared, hidden));
+    return few_tiles(shared, cus) || ((rows + 127) / 128 * cols <= 2 * cus && !sliced(shared, hidden));
 }
 
 // fp8 weights, a joint call that one kernel serves: whether the shared expert's sums start at the stages of that kernel's own
@@ -2553,7 +2555,7 @@ bool joins(const moe_mlp_group& routed, const moe_mlp_group& shared, int32_t hid
 // mean below 128); else at stage 0, as in a call of its own, whose bits it then has.  DeepSeek-V3, us, 1300 /
 // 1500 / 2997 / 4000 tokens (all of the second kind): started as the first kind 2337 / 2437 / 3387 / 4082, at stage 0
 // 2340 / 2449 / 3392 / 4081.
-int joint_alone(const moe_mlp_group& shared) { return shared.n_rows < 128 || few_tiles(shared); }
+int joint_alone(const moe_mlp_group& shared) { return shared.n_rows < 128 || few_tiles(shared, cu_count()); }
 
 template <bool W8>
 int grouped_swiglu(const moe_mlp_group& m, int32_t hidden, int32_t phases, void* stream, const char* who) {
@@ -2580,7 +2582,7 @@ int grouped_swiglu_joint(const moe_mlp_group& r, const moe_mlp_group& s, int32_t
     }
     hipStream_t st = as_stream(stream);
     GemmArgs gate_up = gate_up_args(s, hidden), down = down_args(s, hidden);
-    gate_up.alone = down.alone = joint_alone(s);
+    if (W8) gate_up.alone = down.alone = joint_alone(s);
     if (phases & MOE_PHASE_GATE_UP)
         rc = launch_joint<true, W8>(gate_up_args(r, hidden), r.n_rows, row_bound(r), gate_up, s.n_rows, st);
     if (rc == MOE_OK && (phases & MOE_PHASE_DOWN))
