@@ -613,7 +613,7 @@ def main():
     ap.add_argument("--headline-only", action="store_true", help="only the workload named by --workload")
     ap.add_argument("--tokens", type=int, default=0, help="override the token count (parity/debug only)")
     ap.add_argument("--no-join-shared", action="store_true", help="keep a single shared expert in a grouped call of "
-                    "its own at every token count (by default it joins the routed call at small batches)")
+                    "its own at every token count (by default it joins the routed call where the library says so)")
     ap.add_argument("--materialize", action="store_true", help="gather rows into a sorted copy instead of "
                     "reading them through the row map inside the GEMM")
     ap.add_argument("--no-cpu-baseline", action="store_true")
