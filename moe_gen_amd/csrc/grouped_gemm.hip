@@ -25,7 +25,8 @@
 //    its tiles into the next.
 //  * grouped_gemm_kernel (experts of up to 192 rows, and with fp8 weights what an expert's full 256-row tiles
 //    leave over if that is at most 192 rows, a single MLP's where a padded tile of the other kernel is not the
-//    shorter way; work that mostly streams weights): one workgroup per tile, grid = upper bound on the tile count, surplus workgroups exit at once;
+//    shorter way; work that mostly streams weights): one workgroup per tile, grid = upper bound on the tile count,
+//    surplus workgroups exit at once;
 //    the tile height (16 ... 192 rows in steps of 16) follows the expert, groups of 4 tiles go round-robin
 //    to the XCDs.  Its tiles run through the weight streamers (stream16_tile, stream8x_tile, stream8_tile):
 //    weights AND token rows reach LDS by DMA, three weight buffers, one barrier per stage.
@@ -126,8 +127,8 @@ __device__ __forceinline__ int swz(int row) { return (row & 7) ^ ((row >> 3) & 1
 // bf16 weights: every path of both kernels uses this rule, so which kernel or tile computes a row does not change the
 // order its products are added in (the persistent kernel itself runs within 0.5 % either way).  fp8 weights (a scale
 // per 128 k: pairs of stages stay together): only in calls that the one-workgroup-per-tile kernel serves alone (and not for
-// a large shared expert in them, joint_alone); the persistent kernel loses 1.6 % of the DeepSeek-V3 step to a rotated walk, so calls that launch it start every tile
-// at stage 0, in both kernels.
+// a large shared expert in them, joint_alone); the persistent kernel loses 1.6 % of the DeepSeek-V3 step to a rotated
+// walk, so calls that launch it start every tile at stage 0, in both kernels.
 template <bool W8>
 __device__ __forceinline__ int k_rotation(int n_tile, int nk) { return (W8 ? 2 * n_tile : n_tile) % nk; }
 
@@ -358,7 +359,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, Stage st0, Stage st
     // (fp8 weights under tiles below 256 rows are fetched 128 k at a time, see PAIR8 below: k_rotation keeps their
     // pairs of stages together)
     constexpr bool PAIR8 = W8;
-    const int rot = (W8 && g.cold_max != 0x7fffffff) ? 0 : k_rotation<W8>(n_tile, nk);
+    const int rot = (W8 && !g.alone) ? 0 : k_rotation<W8>(n_tile, nk);
     auto stage_at = [&](int kt) { const int kp = kt + rot; return kp >= nk ? kp - nk : kp; };
 
     // ---- per-thread load coordinates ----
@@ -919,7 +920,8 @@ __device__ __forceinline__ void stream8_tile(const GemmArgs& g, SBuf buf0, SBuf 
 // add up, and neither is busy (96 / 176 rows: matrix cores 42 / 57 %, vector ALU 36 / 28 % of the cycles).  The clock falls
 // little meanwhile (16 -> 176 rows 1.81 -> 1.71 GHz), and a CU takes 0.122 to 0.125 lines per cycle at every height (the persistent
 // kernel about 0.20): products that do not overlap the stream or token lines that queue with the weights' both fit; which of
-// them it is has not been established.  Against one form each for up to 128 and up to 192 rows, in which every half read, converted and multiplied
+// them it is has not been established.
+// Against one form each for up to 128 and up to 192 rows, in which every half read, converted and multiplied
 // in turn, DeepSeek-V3 shapes, 256 experts, us: 96 rows each 1913 -> 1861 (gate and up), 1091 -> 1055 (down), 176 rows
 // 2782 -> 2583 and 1566 -> 1468; 512 rows each (leftovers of full tiles) 6144 -> 6082, 3247 -> 3226 for 64 experts.
 template <int TG, bool SWIGLU, bool SPLIT = false>   // TG: 16-row token groups multiplied (1 .. 12)
