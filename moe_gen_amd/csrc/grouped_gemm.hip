@@ -903,27 +903,32 @@ __device__ __forceinline__ void stream8_tile(const GemmArgs& g, SBuf buf0, SBuf 
 // kernel might have computed: what an fp8 expert's full 256-row tiles leave over, the halves of the persistent kernel's last
 // tiles, and in calls that this kernel serves alone the experts (or 128-row slices of experts) above 64 rows.  A row's bits
 // must then not depend on who computes it, so every matrix instruction gets the k values the persistent kernel gives it,
-// in the same lanes: lane group q holds k = 32 s + 8 f(q) + (0..7) of k-step s, f = 0, 2, 1, 3.  Those are 8 consecutive
-// fp8 weights, one half of a 16-byte part (read whole; the lane group two further on uses the other half, a broadcast, where
-// 8-byte reads of every other half collide), and the 16-byte token chunk 4 s + f(q) of a 64-k half.
+// in the same lanes: lane group q holds k = 32 s + 8 f(q) + (0..7) of k-step s, f = 0, 2, 1, 3.  Those are the 16-byte token
+// chunk 4 s + f(q) of a 64-k half, and 8 consecutive fp8 weights, one half of the 16-byte part 2 s + (q & 1): lane groups q and
+// q + 2 use the two halves of one part.  So lane group q reads part q, the lower half of the wave those of step 0 and the upper
+// those of step 1, and one v_permlane32_swap per pair of dwords gives every lane its 8 weights of either step: every weight
+// leaves LDS once.
 //
 // Weights travel in blocks of 128 k through three buffers, token rows in halves of 64 k with one barrier per half: up to 128
 // rows through three buffers of 16 KiB, two halves ahead, above through two of 24 KiB (one is two arrays), one half ahead.
 // A wave brings and reads its own weight rows, so only token rows need the barrier.
 //
-// The k loop is a pipeline of slots, one per k-step of 32 and part of at most 4 token groups.  Slot n multiplies part n - 2,
-// requests the token operands of part n, and converts its share of the weights of the step after the one that is multiplied, so
-// the LDS latency and the conversion stand beside matrix instructions instead of in front of them.  Slots run on across
-// the barriers; in front of the first one operands and accumulators are zero.
+// The k loop is a pipeline of slots, one per k-step of 32 and part of at most 4 token groups.  Slot n requests the token operands of
+// part n, multiplies part n - 1 and converts its share of the weights of the step after the one that is multiplied, so the LDS
+// latency and the conversion stand beside matrix instructions instead of in front of them.  Slots run on across the barriers; in
+// front of the first one operands and accumulators are zero.
 //
-// What bounds it: a half of 16 KiB of weights takes 1075 cycles and 126 more for every 16 token rows, so the stream and the products
-// add up, and neither is busy (96 / 176 rows: matrix cores 42 / 57 %, vector ALU 36 / 28 % of the cycles).  The clock falls
-// little meanwhile (16 -> 176 rows 1.81 -> 1.71 GHz), and a CU takes 0.122 to 0.125 lines per cycle at every height (the persistent
-// kernel about 0.20): products that do not overlap the stream or token lines that queue with the weights' both fit; which of
-// them it is has not been established.
-// Against one form each for up to 128 and up to 192 rows, in which every half read, converted and multiplied
-// in turn, DeepSeek-V3 shapes, 256 experts, us: 96 rows each 1913 -> 1861 (gate and up), 1091 -> 1055 (down), 176 rows
-// 2782 -> 2583 and 1566 -> 1468; 512 rows each (leftovers of full tiles) 6144 -> 6082, 3247 -> 3226 for 64 experts.
+// What bounds it: power.  DeepSeek-V3 shapes, 256 experts of 96 rows, gate and up 1833 us; with operands of zero, the same
+// instructions and bytes, 1447 (5.2 TB/s of weights), at 176 rows 2519 and 1792; without any load 1201 and 1652, weights alone
+// 1312.  Behind that come the instruction slots of a SIMD: a matrix instruction takes 8 of its 16 cycles from the vector ALU, a
+// vector instruction 4, an LDS read about 6, which at 96 rows adds up to 1200 cycles a half, 600 of them the conversion.
+// Against reads at the end of a slot, which the next slot waited for, two LDS reads a fragment and half, and the compiler's order of
+// products and conversion, same box, us: 96 rows each 1863 -> 1828 (gate and up), 1067 -> 1045 (down), 176 rows 2569 -> 2525 and
+// 1460 -> 1442.
+// weights in LDS: 16-byte part c of fragment row r at part c ^ wsx(r).  A 16-byte read serves lanes 0-3, 12-15, 20-27 together, then
+// 4-11, 16-19, 28-31, and the same of the upper half-wave: with lane group q on part q their 16 reads fall on 16 different bank
+// groups (wsw gives two on each)
+__device__ __forceinline__ int wsx(int r) { return (r & 2) | ((r >> 1) & 4); }
 template <int TG, bool SWIGLU, bool SPLIT = false>   // TG: 16-row token groups multiplied (1 .. 12)
 __device__ __forceinline__ void stream8x_tile(const GemmArgs& g, const TileLds& lds, int e, int row0, int row_end, int n_tile,
                                               bool rotate, KSlice ks = {}) {
@@ -950,7 +955,7 @@ __device__ __forceinline__ void stream8x_tile(const GemmArgs& g, const TileLds& 
 
     // ---- DMA coordinates ----
     // weights, instruction i (0..3): rows 8 i + lane / 8 of the wave's 32 (fragment i / 2, fragment row 8 (i & 1) + lane / 8);
-    // 16-byte part c of fragment row r at part c ^ wsw(r)
+    // 16-byte part c of fragment row r at part c ^ wsx(r)
     const int lr = lane >> 3, pp = lane & 7;
     uint32_t w_voff[4], t_voff[3];                // (NDT of the latter are used)
     const uint8_t* bmat[2];
@@ -966,7 +971,7 @@ __device__ __forceinline__ void stream8x_tile(const GemmArgs& g, const TileLds& 
     for (int i = 0; i < 4; ++i) {
         const int fr = 8 * (i & 1) + lr;
         const int rt = SWIGLU ? 16 * wave + fr : 32 * wave + 16 * (i >> 1) + fr;      // row of the tile's N range
-        w_voff[i] = (uint32_t)min(n0 + rt, N - 1) * (uint32_t)K + (uint32_t)((pp ^ wsw(fr)) << 4);
+        w_voff[i] = (uint32_t)min(n0 + rt, N - 1) * (uint32_t)K + (uint32_t)((pp ^ wsx(fr)) << 4);
     }
     // tokens, instruction i: rows 64 i + 8 wave + lane / 8, 16-byte chunk c of row r at chunk c ^ swz(r) (the persistent
     // kernel's layout of a 64-k stage).  Rows past the tile's last: zeros, no request.
@@ -1009,12 +1014,11 @@ __device__ __forceinline__ void stream8x_tile(const GemmArgs& g, const TileLds& 
     // ---- operands ----
     const int frow = lane & 15, q4 = lane >> 4;
     const int fq = ((q4 & 1) << 1) | (q4 >> 1);
-    // weights: the 8 bytes at 32 s + 8 f(q) of the 64-byte half h of fragment row frow: 16-byte part 4 h + 2 s + f(q) / 2
-    const uint32_t w_rd = (uint32_t)(wave * 4096 + frow * 128), wkey = (uint32_t)wsw(frow);
+    const uint32_t w_rd = (uint32_t)(wave * 4096 + frow * 128), wkey = (uint32_t)wsx(frow);
     const uint32_t t_rd = (uint32_t)(frow * 128), tkey = (uint32_t)swz(frow);   // (group bases are multiples of 16 rows)
     f32x4 acc[TG][2];
     bf16x8 tf[2][4], wa[2][2];
-    u32x4 raw[2] = {u32x4{0}, u32x4{0}};
+    u32x4 raw[2][2];                              // [half & 1][fragment]
 #pragma unroll
     for (int t = 0; t < TG; ++t) { acc[t][0] = f32x4{0}; acc[t][1] = f32x4{0}; }
 #pragma unroll
@@ -1032,17 +1036,27 @@ __device__ __forceinline__ void stream8x_tile(const GemmArgs& g, const TileLds& 
             tf[v & 1][t - part_lo(q)] = *reinterpret_cast<const bf16x8*>(b + t_rd + coff);
         }
     };
-    auto read_weights = [&](const uint8_t* wb, int h, int s) __attribute__((always_inline)) {
+    auto read_weights = [&](const uint8_t* wb, int h) __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < 2; ++j)
-            raw[j] = *reinterpret_cast<const u32x4*>(wb + w_rd + j * 2048 + (((4 * h + 2 * s + (fq >> 1)) ^ wkey) << 4));
+            raw[h][j] = *reinterpret_cast<const u32x4*>(wb + w_rd + j * 2048 + (((4 * h + q4) ^ wkey) << 4));
     };
-    auto convert = [&](int s, int part, int set) __attribute__((always_inline)) {   // share `part` of NP of raw -> wa[s]
+    // dwords 0 and 1: step 0's weights of this lane, 2 and 3: step 1's
+    auto sort_weights = [&](int h, int j) __attribute__((always_inline)) {
+#pragma unroll
+        for (int d = 0; d < 2; ++d) {
+            const auto r = __builtin_amdgcn_permlane32_swap(raw[h][j][d], raw[h][j][2 + d], false, false);
+            raw[h][j][d] = r[0];
+            raw[h][j][2 + d] = r[1];
+        }
+    };
+    auto convert = [&](int h, int s, int part, int set) __attribute__((always_inline)) {   // share `part` of NP of raw[h] -> wa[s]
 #pragma unroll
         for (int u = part * 4 / NP; u < (part + 1) * 4 / NP; ++u) {              // 4 weights of fragment u / 2
             const int j = u >> 1, d = u & 1;
             const float scale = rsc[set][SWIGLU ? j : 0];
-            const uint32_t qv = (fq & 1) ? raw[j][2 + d] : raw[j][d];
+            if (s == 0 && d == 0) sort_weights(h, j);
+            const uint32_t qv = raw[h][j][2 * s + d];
             const f32x2 c0 = __builtin_amdgcn_cvt_pk_f32_fp8(qv, false), c1 = __builtin_amdgcn_cvt_pk_f32_fp8(qv, true);
             u32x4 o = __builtin_bit_cast(u32x4, wa[s][j]);
             o[2 * d] = pack_bf16(c0[0] * scale, c0[1] * scale);
@@ -1068,26 +1082,36 @@ __device__ __forceinline__ void stream8x_tile(const GemmArgs& g, const TileLds& 
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
 #pragma unroll
-        for (int i = 0; i < NDT; ++i) dma_t(2 * p + h + (WIDE ? 1 : 2), t_refill, i);
-        if (h == 0) scales(p + 1, (set + 1) % 3);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
         for (int v = 0; v < V; ++v) {
-            const int s = v / NP, mq = (v + V - 2) % NP;       // step of this slot, part that it multiplies
-            multiply((v + V - 2) % V);
             read_tokens(tb, v);
-            // the step after the one that is multiplied: its share of the conversion
-            if (NP == 1) convert(s ^ 1, 0, h == 0 && v == 0 ? (set + 2) % 3 : set);
-            else if (NP == 2 || mq) convert(s, mq, set);
-            else convert(s ^ 1, 0, h == 1 && s == 1 ? (set + 1) % 3 : set);
-            if (NP == 1) read_weights(wb, h, s);
-            else if (mq == NP - 1) read_weights(s == 0 || h == 0 ? wb : w_next, s == 0 ? h : h ^ 1, s ^ 1);
+            if (v == NP) read_weights(h == 0 ? wb : w_next, h ^ 1);
+            __builtin_amdgcn_sched_barrier(0);
+            if (v == 0) {
+#pragma unroll
+                for (int i = 0; i < NDT; ++i) dma_t(2 * p + h + (WIDE ? 1 : 2), t_refill, i);
+                if (h == 0) scales(p + 1, (set + 1) % 3);
+                __builtin_amdgcn_sched_barrier(0);
+            }
             // the weights of block p + 2: behind the first slots of the half
             if (!WIDE && h == 0) {
                 if (V == 2) { dma_w(p + 2, w_refill, 2 * v); dma_w(p + 2, w_refill, 2 * v + 1); }
                 else dma_w(p + 2, w_refill, v);
             }
             if (WIDE && v < 2) dma_w(p + 2, w_refill, 2 * h + v);
+            multiply((v + V - 1) % V);
+            // the step after the one that is multiplied: its share of the conversion
+            const int share = (v + V - 1) % NP;
+            if (v == 0) convert(h, 0, share, set);
+            else if (v <= NP) convert(h, 1, share, set);
+            else convert(h ^ 1, 0, share, h == 0 ? set : (set + 1) % 3);
+            // two vector instructions are free beside a matrix instruction of 16 cycles, the third costs 4
+            const int nm = 2 * (part_lo((v + V - 1) % NP + 1) - part_lo((v + V - 1) % NP));
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                if (i < nm) {
+                    __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x2, 2, 0);
+                }
             __builtin_amdgcn_sched_barrier(0);
         }
     };
@@ -1117,12 +1141,10 @@ __device__ __forceinline__ void stream8x_tile(const GemmArgs& g, const TileLds& 
         for (int i = 0; i < NDT; ++i) dma_t(1, 1, i);
     }
     __builtin_amdgcn_sched_barrier(0);
-    if (NP > 1) {
-        asm volatile("s_waitcnt vmcnt(%0)" :: "n"(VM) : "memory");     // this wave's weights of block 0
-        read_weights(lds.w0, 0, 0);
-    }
-    if (NP == 3) convert(0, 0, 0);
-    rsc[2][0] = rsc[2][1] = 0.0f;
+    asm volatile("s_waitcnt vmcnt(%0)" :: "n"(VM) : "memory");         // this wave's weights of block 0
+    read_weights(lds.w0, 0);
+#pragma unroll
+    for (int part = 0; part < NP - 1; ++part) convert(0, 0, part, 0);
     // Six halves = three blocks bring the rotations back to where they started: literal buffers in the loop body.
     uint8_t *const w0 = lds.w0, *const w1 = lds.w1, *const w2 = lds.w2;
     constexpr int T1 = 1, T2 = WIDE ? 0 : 2, T3 = WIDE ? 1 : 0, T4 = WIDE ? 0 : 1, T5 = WIDE ? 1 : 2;   // token buffers of halves 1 .. 5
@@ -1143,13 +1165,6 @@ __device__ __forceinline__ void stream8x_tile(const GemmArgs& g, const TileLds& 
             half(p + 1, 0, w1, w2, w0, T2, refill(T2), 1);
             half(p + 1, 1, w1, w2, w0, T3, refill(T3), 1);
         }
-    }
-    multiply(V - 2);
-    if (NP == 1) {                                // (the step after the last slot's: the last block's scales)
-        const int rem = npair % 3;
-        if (rem == 1) convert(1, 0, 0);
-        else if (rem == 2) convert(1, 0, 1);
-        else convert(1, 0, 2);
     }
     multiply(V - 1);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no DMA may land in LDS after the workgroup has gone
