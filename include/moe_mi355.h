@@ -230,8 +230,8 @@ typedef struct moe_mlp_group {
 } moe_mlp_group;
 
 /*
- * Device scratch with which a group runs faster, 0 if none does: ONE fp8 MLP (n_experts 1) of few rows and a long
- * intermediate size (DeepSeek-V3's dense layers, up to 512 rows) gives every column tile of the down projection to several
+ * Device scratch with which a group runs faster, 0 if none does: ONE fp8 MLP (n_experts 1) with a long intermediate size whose
+ * down projection has too few tiles for the chip (DeepSeek-V3's dense layers, up to 1536 rows) gives every tile of it to several
  * workgroups, which leave their fp32 sums here.  Without it, or with less, the call runs as the two above.  A row's bits may differ
  * between the two by the order of its sums.
  */

@@ -707,9 +707,15 @@ struct TileLds {
     uint8_t *w0, *w1, *w2, *t0, *t1, *t2;
 };
 
-// How the split kernel cuts one problem: row tiles of `rows`, k into `slices` of up to `blocks` blocks of 128
+// How the down projection of one MLP is cut when its k is: row tiles of `rows` (256: on the persistent kernel, else on the split
+// kernel), k into `slices` of up to `blocks` blocks of 128.  part: where the fp32 sums go, [slices][n_rows][N].
 struct SplitPlan {
     int m_tiles, rows, slices, blocks;
+};
+struct SplitArgs {
+    SplitPlan plan;
+    int n_rows;
+    float* part;
 };
 
 // A slice of k for a tile whose sums other workgroups share (split kernel): blocks first .. first + count - 1 of 128 k, and
@@ -1795,10 +1801,10 @@ __global__ __launch_bounds__(64) void grouped_gemm_thin_kernel(GemmPair pair_of)
 // workgroup each, so that tiles x slices fill the CUs once; the fp32 sums of the slices go to the workspace and
 // add_slices_kernel adds them, in order, and rounds once.  Rows past 128 are cut into tiles of equal height; all tiles of a
 // call run the same body, chosen by that height, so a row's bits do not depend on its place.  The M tiles of one piece of
-// the weights are neighbours on one XCD.
+// the weights are neighbours on one XCD.  (From 257 rows on the slices run as 256-row tiles of the persistent kernel, split_plan.)
 // Measured (DeepSeek-V3's dense MLP, both launches, us, without scratch -> with it): 1 token 119 -> 75, 17: 185 -> 87,
-// 64: 231 -> 115, 128: 356 -> 161, 192: 516 -> 220, 256: 426 -> 273, 384: 465 -> 402, 512: 502 -> 415; of those the gate and up
-// products take 49, 58, 76, 104, 150, 186, 232 and 273.
+// 64: 231 -> 115, 128: 356 -> 161, 192: 516 -> 220, 256: 426 -> 273; of those the gate and up products take 49, 58, 76, 104, 150
+// and 186.
 __global__ __launch_bounds__(512) void grouped_gemm_split_kernel(GemmArgs g, int n_rows, SplitPlan plan, float* part) {
     __shared__ __attribute__((aligned(1024))) uint8_t lw0[S8_WBYTES];
     __shared__ __attribute__((aligned(1024))) uint8_t lw1[S8_WBYTES];
@@ -1884,8 +1890,10 @@ __device__ __forceinline__ int fresh_lane() {
 // 1190 -> 1271 and 1076 -> 1164.  fp8, 64 experts, 131072 rows, 7168 <-> 2048: 1259 -> 1282 and 1201 -> 1217; there the
 // conversion, 64 vector instructions per 64 matrix instructions, is what is left (a tenth more with most of it taken out).
 // PAIRED: with a second problem.  (An instantiation of its own: the choice per tile costs DeepSeek-V3's 65536 tokens 0.4 %.)
-template <bool SWIGLU, bool W8, bool PAIRED>
-__global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmPair pair_of) {
+// SPLIT: the down projection of one MLP, its tiles once per slice of k, all of them here; the fp32 sums go to `split`.
+template <bool SWIGLU, bool W8, bool PAIRED, bool SPLIT>
+__global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmPair pair_of, SplitArgs split) {
+    static_assert(!SPLIT || (!SWIGLU && W8 && !PAIRED), "slices of k: the down projection of one fp8 MLP");
     const GemmArgs& g = pair_of.p[0];            // the routed experts; the tiles of the second problem come first
     constexpr int MT = 4, WN = 4;
     constexpr int NT = 128 * WN;
@@ -1918,7 +1926,7 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmPair p
 
     // M-tile prefix over experts; the experts' row offsets and matrix pointers go to LDS tables on the way
     ExpertOfThread mine;
-    const int run = mtile_prefix_scan<NT>(g, tid, s_pref, s_wtot, mine, [&](int c) { return persistent_tiles(g, c); }, [&](int e, int o0, int o1) {
+    const int run = mtile_prefix_scan<NT>(g, tid, s_pref, s_wtot, mine, [&](int c) { return persistent_tiles(g, SPLIT ? min(c, split.n_rows) : c); }, [&](int e, int o0, int o1) {
         s_off[e] = o0;
         if (e == g.E - 1) s_off[g.E] = o1;
         s_ptr[0][e] = (unsigned long long)(uintptr_t)g.b0[e];
@@ -1941,7 +1949,8 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmPair p
     const SharedTiles second_tiles = PAIRED ? shared_tiles_of<W8>(pair_of.p[1], uni(s_off1[0]), uni(s_off1[1])) : SharedTiles{0, 0, 0, 0};
     const int ptiles1 = second_tiles.persistent;
     const int own = g.tail_cus > 0 ? sum_over_experts<NT>(g, tid, s_wtot, [&](int c) { return own_tiles<W8>(g, c); }) * g.n_tiles_n + second_tiles.own : 0;
-    const int all = run * g.n_tiles_n + ptiles1, total = all - tail_tiles(g, all, own);
+    const int slice_tiles = run * g.n_tiles_n;   // SPLIT: tiles of one slice
+    const int all = SPLIT ? slice_tiles * split.plan.slices : slice_tiles + ptiles1, total = all - tail_tiles(g, all, own);
     const int xcd = blockIdx.x & 7, slots = gridDim.x >> 3;
     int slot = blockIdx.x >> 3;
     auto tile_of = [&](int sl) { return ((sl / slots) * 8 + xcd) * slots + (sl % slots); };
@@ -1971,7 +1980,7 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmPair p
     // bf16 weights: k starts at another stage for every N tile (k_rotation); stage_of is the stage that pipeline step
     // kt fetches.  The rotation is adopted with the tile's DMA coordinates.
     // (So are the stages of a tile and the length of its token rows: the two problems may differ in them.)
-    int rot = 0, rot_n = 0, nk_dma = 0, K_n = 0;
+    int rot = 0, rot_n = 0, nk_dma = 0, K_n = 0, nk_n = 0;
     auto stage_of = [&](int kt, int r) { const int kp = kt + r; return kp >= nk_dma ? kp - nk_dma : kp; };
     auto setup = [&](int v) {
         const int l = fresh_lane();
@@ -1981,7 +1990,15 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmPair p
         const GemmArgs& g1 = pair_of.p[1];
         const int K = second ? g1.K : g.K, N = second ? g1.N : g.N, nk = K / BK, tiles_n = second ? g1.n_tiles_n : g.n_tiles_n;
         const int32_t* const row_map = SWIGLU ? (second ? g1.row_map : g.row_map) : nullptr;
-        int m_tile, n_tile, e, first;
+        int m_tile, n_tile, e, first, kb0 = 0;  // kb0: first block of 128 k
+        nk_n = nk;
+        int slice = 0;
+        if (SPLIT) {
+            slice = v / slice_tiles;
+            v -= slice * slice_tiles;
+            kb0 = slice * split.plan.blocks;
+            nk_n = 2 * min(split.plan.blocks, (K >> 7) - kb0);
+        }
         if (second) {
             e = PE;
             first = uni(s_off1[0]);
@@ -1996,11 +2013,14 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmPair p
             const int mt_e = uni(s_pref[e + 1]) - pe;
             first = uni(s_off[e]);
             row_end = uni(s_off[e + 1]);
+            if (SPLIT) row_end = min(row_end, first + split.n_rows);
             tile_in_expert(v - pe * tiles_n, mt_e, tiles_n, m_tile, n_tile);
         }
         row0 = first + m_tile * BM;
         n0 = n_tile * NBLK;
-        c_out = second ? g1.c : g.c;
+        // (SPLIT: the slice's sums of row `first`, moved so that row numbers stay those of the sorted rows)
+        if (SPLIT) c_out = reinterpret_cast<uint16_t*>(split.part + ((ptrdiff_t)slice * split.n_rows - first) * N);
+        else c_out = second ? g1.c : g.c;
         N_out = N;
         K_n = K;
         rot_n = W8 ? 0 : k_rotation<false>(n_tile, nk);
@@ -2015,7 +2035,7 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmPair p
             const int r = min(row0 + rt, row_end - 1);
             a_row_n[i] = row_map ? ((gptr_i32)(uintptr_t)row_map)[r] : r - row0;   // (down: sorted rows)
         }
-        a_base_n = reinterpret_cast<const uint8_t*>(second ? g1.a : g.a) + (row_map ? (size_t)0 : (size_t)row0 * K * 2);
+        a_base_n = reinterpret_cast<const uint8_t*>(second ? g1.a : g.a) + (row_map ? (size_t)0 : (size_t)row0 * K * 2) + (SPLIT ? kb0 * 256 : 0);
         a_records_n = row_map ? (int)(uint32_t)(second ? g1.a_bytes : g.a_bytes) : -1;
         const uint8_t* bmat0 = uni_ptr(reinterpret_cast<const void*>((uintptr_t)s_ptr[0][e]));
         const uint8_t* bmat1 = SWIGLU ? uni_ptr(reinterpret_cast<const void*>((uintptr_t)s_ptr[1][e])) : bmat0;
@@ -2029,9 +2049,9 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmPair p
                 int n = SWIGLU ? (n0 + (r & 127)) : (n0 + r);
                 b8_voff[i] = (uint32_t)min(n, N - 1) * (uint32_t)K + (uint32_t)bcol_b;
             }
-            b8m0 = bmat0; b8m1 = bmat1;
+            b8m0 = bmat0 + (SPLIT ? kb0 * 128 : 0); b8m1 = bmat1 + (SPLIT ? kb0 * 128 : 0);
             if (SWIGLU) { srow0 = (n0 >> 7) * KB; srow1 = srow0; }
-            else        { srow0 = (n0 >> 7) * KB; srow1 = min((n0 >> 7) + 1, (N >> 7) - 1) * KB; }
+            else        { srow0 = (n0 >> 7) * KB + kb0; srow1 = min((n0 >> 7) + 1, (N >> 7) - 1) * KB + kb0; }
         } else {
             bm0_n = bmat0; bm1_n = bmat1;
 #pragma unroll
@@ -2056,7 +2076,7 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmPair p
         }
         a_base = a_base_n;
         a_records = a_records_n;
-        nk_dma = K_n / BK;
+        nk_dma = SPLIT ? nk_n : K_n / BK;
         rot = rot_n;
     };
     auto dma_a = [&](int st, int kt, int i) __attribute__((always_inline)) {
@@ -2246,7 +2266,7 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmPair p
         // columns, 64 bytes of a row; neighbouring lane groups exchange halves and store them from the registers.  Down: 64
         // columns, a whole 128-byte line of a row, put together in LDS, 16 rows at a time, in the wave's 2 KiB of the one piece
         // of a stage that no DMA writes before the next tile's first barrier.
-        if (!SWIGLU) {
+        if (!SWIGLU && !SPLIT) {
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // every wave has read that piece
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
@@ -2259,11 +2279,17 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmPair p
             const int l = fresh_lane();
             const int fr = l & 15, q = l >> 4;
             const int rows_here = min(BM, out_row_end - out_row0) - wm * 128, ncol0 = out_n0 + wn * CW;
-            const uint8_t* out = uni_ptr(c + (size_t)(out_row0 + wm * 128) * N + ncol0);
+            const uint8_t* out = uni_ptr(SPLIT ? c + 2 * ((ptrdiff_t)(out_row0 + wm * 128) * N + ncol0) : c + (size_t)(out_row0 + wm * 128) * N + ncol0);
             uint8_t* ep = sA1b + wave_s * 2048;
 #pragma unroll
             for (int mi = 0; mi < TM; ++mi) {
-                if (SWIGLU) {
+                if (SPLIT) {                     // sums: 16 bytes of a row per lane and fragment
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) {
+                        const int r = 16 * mi + fr, col = 16 * j + 4 * q;
+                        store16<0>(__builtin_bit_cast(u32x4, acc[mi][j]), out, r < rows_here && ncol0 + col < N ? (uint32_t)(r * N + col) * 4u : 0x80000000u);
+                    }
+                } else if (SWIGLU) {
                     const u32x4 o = pair_columns(epilogue_pack<true>(acc[mi][0], acc[mi][2]), epilogue_pack<true>(acc[mi][1], acc[mi][3]));
                     const int r = 16 * mi + fr, col = 16 * (q & 1) + 8 * (q >> 1);
                     store16<0>(o, out, r < rows_here && ncol0 + col < N ? (uint32_t)(r * N + col) * 2u : 0x80000000u);
@@ -2346,8 +2372,8 @@ int launch_persistent(const GemmPair& pair, int n_rows, hipStream_t st) {
     long grid = ((max_mtiles * g.n_tiles_n + shared + 7) / 8) * 8;
     const long ncu = (cu_count() / 8) * 8;
     if (grid > ncu) grid = ncu;
-    if (pair.shared_rows > 0) hipLaunchKernelGGL((grouped_gemm_persistent_kernel<SWIGLU, W8, true>), dim3((unsigned)grid), dim3(512), 0, st, pair);
-    else hipLaunchKernelGGL((grouped_gemm_persistent_kernel<SWIGLU, W8, false>), dim3((unsigned)grid), dim3(512), 0, st, pair);
+    if (pair.shared_rows > 0) hipLaunchKernelGGL((grouped_gemm_persistent_kernel<SWIGLU, W8, true, false>), dim3((unsigned)grid), dim3(512), 0, st, pair, SplitArgs{});
+    else hipLaunchKernelGGL((grouped_gemm_persistent_kernel<SWIGLU, W8, false, false>), dim3((unsigned)grid), dim3(512), 0, st, pair, SplitArgs{});
     MOE_HIP_CHECK(hipGetLastError());
     return MOE_OK;
 }
@@ -2355,17 +2381,43 @@ int launch_persistent(const GemmPair& pair, int n_rows, hipStream_t st) {
 // 4 GiB of gathered rows or more: only the register-staged body addresses them
 inline bool gather_fits(const GemmArgs& g) { return !g.row_map || g.a_bytes < (1ull << 32); }
 
-// The split kernel's plan, slices == 0 where it does not pay: as many slices as fill the CUs once, of 8 blocks or more (a
-// shorter k loop is mostly its own start), at most 16; and only where k is long: 32 blocks (4096), so that what the slices save
-// outweighs their sums' way through memory.  (A long k without two tiles' worth of idle CUs, from 513 rows of DeepSeek-V3:
-// the persistent kernel.)
+// How the down projection of one MLP is cut in k, slices == 0 where that does not pay: only where k is long (32 blocks, 4096), so
+// that what the slices save outweighs their sums' way through memory, and where its own tiles leave CUs idle.
+//  * up to 256 rows on the split kernel: as many slices as fill the CUs once, of 8 blocks or more (a shorter k loop is mostly
+//    its own start), at most 16.
+//  * above, up to a round of 256-row tiles, on the persistent kernel: the number of slices whose rounds and sums cost least, a
+//    round of one block counted 3.0 us and the sums 6 us and 0.45 us per MB, if that is less than what the call takes
+//    uncut (0.6 of a round of whole tiles where half tiles go round once, else 0.88).
+// DeepSeek-V3's dense MLP (28 column tiles, 144 blocks), down projection, us, uncut or on the split kernel (up to 512 rows) -> this:
+// 300 rows 154 -> 129, 512: 146 -> 130, 520: 227 -> 171, 768: 232 -> 181, 800: 243 -> 245, 1000: 264 -> 248, 1300: 365 -> 351, 1536:
+// 383 -> 352; 2 rounds of whole tiles and more gain 6 % at most (3000 rows 724 -> 683, 2600: 652 -> 647, 4000: 871 -> 922).
 SplitPlan split_plan(int n_rows, int K, int n_tiles_n) {
-    const int nblk = K / 128;
+    const int nblk = K / 128, cus = cu_count();
+    if (nblk < 32 || n_rows < 1 || cus < 8) return SplitPlan{};
+    if (n_rows > 256) {
+        const int m = (n_rows + 255) / 256, left = n_rows & 255;
+        const long tiles = (long)m * n_tiles_n;
+        if (tiles > cus) return SplitPlan{};
+        const bool own = left > 0 && left <= 192;                    // (uncut, these rows are tiles of the other kernel)
+        const long pieces = (2 * (m - (own ? 1 : 0)) + (own ? 1 : 0)) * (long)n_tiles_n;
+        double best = nblk * 3.0 * (pieces <= cus ? 0.6 : 0.88);
+        SplitPlan plan{};
+        for (int s = 2; s <= 16 && nblk / s >= 8; ++s) {
+            const int blocks = (nblk + s - 1) / s, slices = (nblk + blocks - 1) / blocks;
+            const double rounds = (double)((tiles * slices + cus - 1) / cus);
+            const double us = rounds * blocks * 3.0 + 6.0 + 0.45e-6 * slices * n_rows * (double)n_tiles_n * 1024;
+            if (us < best) {
+                best = us;
+                plan = SplitPlan{m, 256, slices, blocks};
+            }
+        }
+        return plan;
+    }
     int m = (n_rows + 127) / 128;
     const int rows = m <= 1 ? n_rows : ((n_rows + m - 1) / m + 15) / 16 * 16;
-    if (nblk < 32 || n_rows < 1 || (long)m * n_tiles_n * 2 > cu_count()) return SplitPlan{};
+    if ((long)m * n_tiles_n * 2 > cus) return SplitPlan{};
     m = (n_rows + rows - 1) / rows;
-    int s = cu_count() / (m * n_tiles_n);
+    int s = cus / (m * n_tiles_n);
     s = s < nblk / 8 ? s : nblk / 8;
     s = s < 16 ? s : 16;
     const int blocks = (nblk + s - 1) / s;
@@ -2374,7 +2426,16 @@ SplitPlan split_plan(int n_rows, int K, int n_tiles_n) {
 
 int launch_split(const GemmArgs& g, int n_rows, const SplitPlan& plan, float* part, hipStream_t st) {
     const int pieces = plan.slices * g.n_tiles_n;
-    hipLaunchKernelGGL(grouped_gemm_split_kernel, dim3((pieces + 7) / 8 * 8 * plan.m_tiles), dim3(512), 0, st, g, n_rows, plan, part);
+    if (plan.rows == 256) {
+        GemmPair pair{};
+        pair.p[0] = g;
+        pair.p[0].rem_split = 1;                 // every row on this kernel's tiles, the last one padded
+        const long tiles = (long)pieces * plan.m_tiles, ncu = (cu_count() / 8) * 8, grid = (tiles + 7) / 8 * 8;
+        hipLaunchKernelGGL((grouped_gemm_persistent_kernel<false, true, false, true>), dim3((unsigned)(grid < ncu ? grid : ncu)), dim3(512), 0, st,
+                           pair, SplitArgs{plan, n_rows, part});
+    } else {
+        hipLaunchKernelGGL(grouped_gemm_split_kernel, dim3((pieces + 7) / 8 * 8 * plan.m_tiles), dim3(512), 0, st, g, n_rows, plan, part);
+    }
     hipLaunchKernelGGL(add_slices_kernel, dim3((unsigned)(((size_t)n_rows * g.N / 4 + 255) / 256)), dim3(256), 0, st, part, g.offsets, g.c,
                        n_rows, g.N, plan.slices);
     MOE_HIP_CHECK(hipGetLastError());

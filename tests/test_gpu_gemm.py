@@ -1066,6 +1066,48 @@ def test_dense_fp8_down_projection_in_slices_of_k(h, I):
         assert torch.equal(down(act[perm].contiguous(), need), y[perm])
 
 
+@pytest.mark.parametrize("n,first,rows", [
+    (1300, 0, 1300),        # slices of more than a round of tiles
+    (1000, 40, 700),        # fewer rows than the host allows for, behind other rows: fewer row tiles, the last one ragged
+    (600, 0, 0)])
+def test_dense_fp8_slices_of_k_on_whole_tiles(n, first, rows):
+    """The down projection of DeepSeek-V3's dense MLP, 256-row tiles of the persistent kernel once per slice of k: against float64 on the
+    dequantised weights, no other row written, nothing past the scratch, and a row's bits independent of its place."""
+    import ctypes
+    from moe_gen_amd import _native as N, ops
+    from moe_gen_amd.synthetic import quantize_fp8_block128
+    h, I = 7168, 18432
+    print(f"slices on whole tiles n={n} first={first} rows={rows}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    q, sc = quantize_fp8_block128(torch.randn(h, I, generator=g, device="cuda") * 0.02)
+    qi, si = torch.zeros(I, h, device="cuda").to(torch.float8_e4m3fn), torch.ones(I // 128, h // 128, device="cuda")
+    ptrs = ops.expert_pointers([qi], [qi], [q], [si], [si], [sc])
+    off = torch.tensor([first, first + rows], dtype=torch.int32, device="cuda")
+    act = torch.randn(n, I, generator=g, device="cuda").to(torch.bfloat16)
+
+    def down(a):
+        y = torch.full((n, h), 3.0, dtype=torch.bfloat16, device="cuda")
+        m, _, _ = ops.mlp_group(torch.zeros(n, h, dtype=torch.bfloat16, device="cuda"), None, ptrs, off, n, n, act=a, y=y)
+        need = N.lib().moe_mlp_workspace_bytes(ctypes.byref(m), h)
+        assert need > 4 * n * h and need % (4 * n * h) == 0
+        ws = torch.full((need // 4 + 64,), 7.0, device="cuda")
+        m.workspace, m.workspace_bytes = ws.data_ptr(), need
+        ops.grouped_swiglu_joint(m, None, h, True, ops.PHASE_DOWN)
+        assert (ws[need // 4:] == 7.0).all() and (y[:first] == 3.0).all() and (y[first + rows:] == 3.0).all()
+        return y[first:first + rows]
+    y = down(act)
+    if rows == 0:
+        return
+    wd = q.double() * sc.double().repeat_interleave(128, 0).repeat_interleave(128, 1)
+    ref = act[first:first + rows].double() @ wd.t()
+    # weights and result are each rounded to bf16: relative 2^-9 at most, independent per element
+    assert (y.double() - ref).norm() <= 2.0 ** -8 * ref.norm()
+    perm = torch.randperm(rows, generator=torch.Generator().manual_seed(n)).cuda()
+    moved = act.clone()
+    moved[first:first + rows] = act[first:first + rows][perm]
+    assert torch.equal(down(moved), y[perm])
+
+
 @pytest.mark.parametrize("n,inter", [(1, 256), (16, 256), (17, 256), (64, 256), (65, 256), (128, 256), (192, 256), (193, 256), (256, 256),
                                      (1, 4096), (16, 4096), (64, 4096), (65, 4096), (128, 4096)])
 def test_fp8_weights_are_dequantised_to_bf16_at_every_row_count(n, inter):
