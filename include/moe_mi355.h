@@ -371,7 +371,7 @@ int moe_combine_residual(const void* y, const int32_t* pos, const int32_t* topk_
 
 /*
  * Slot pool + cyclic prefetch of whole expert modules from pinned host memory
- * into HBM slots on a private copy stream.  Replaces, for the weights half,
+ * into HBM slots on two private copy streams (a slot stays with one of them).  Replaces, for the weights half,
  * HtoD_Engine::HtoD_Worker (core/HtoD_Engine/HtoD_Engine.cpp:201-268),
  * GPU_Weight_Buffer::{acquireEmptyBuffer, get_weights, releaseBuffer,
  * weights_copy_complete, clear_expert_buffer, resize_buffer, reset_prefill_buffer}
@@ -432,7 +432,7 @@ int moe_stage_acquire(moe_stager* s, int32_t id, void* stream, int32_t* slot);
  * The event that says so is recorded on `stream` by the next call that copies into a released slot, one event for
  * all slots released on that stream since the last such call (so `stream` must still exist then; moe_stage_sync
  * records what is pending, for a caller that is about to destroy a stream); a copy enqueued
- * behind a wait that is still pending costs the copy stream about 0.2 ms, and ten experts released and refilled
+ * behind a wait that is still pending costs its copy stream about 0.2 ms, and ten experts released and refilled
  * one by one paid it ten times.  The release that leaves the caller holding no module refills the freed slots at
  * once (the reference's worker refills a slot as soon as it is free, HtoD_Engine.cpp:201-268); while other modules
  * stay held the refill happens at the next moe_stage_acquire / moe_stage_fetch / moe_stage_pump. */
@@ -482,14 +482,14 @@ int moe_stage_set_phase_slots(moe_stager* s, int32_t type, int32_t n_prefill, in
  * decoding size (resize_buffer, GPU_Weight_Buffer.cpp:103-142); "prefill" only records the phase. */
 int moe_stage_set_phase(moe_stager* s, const char* phase);
 /* reset_prefill_buffer (GPU_Weight_Buffer.cpp:310-379): every pool back to its prefill size with
- * all residency dropped.  Drains the copy stream (host wait); MOE_ERR_STATE while a module is
+ * all residency dropped.  Drains the copy streams (host wait); MOE_ERR_STATE while a module is
  * acquired and not released. */
 int moe_stage_reset_prefill_buffer(moe_stager* s);
 /* reset_weight_copy_queue (HtoD_Engine.cpp:295-311): every cyclic queue back to registration order. */
 int moe_stage_reset_weight_copy_queue(moe_stager* s);
 /* Counters: copies issued, bytes issued. */
 int moe_stage_stats(moe_stager* s, int64_t* n_copies, int64_t* n_bytes);
-/* Host-blocking drain of the copy stream (teardown, tests). */
+/* Host-blocking drain of the copy streams (teardown, tests). */
 int moe_stage_sync(moe_stager* s);
 int moe_stage_destroy(moe_stager* s);
 

@@ -73,15 +73,23 @@ struct Type {
     int n_prefill = 0, n_decoding = 0;  // slots per phase (0: the phase verbs leave this type alone)
 };
 
+// Copy streams of a stager, and the one that every copy into slot `slot` goes to: copies into a slot then follow one another
+// without an event between them (a slot may be refilled before anyone has acquired what it held).  On one stream the link
+// idles between two copies: 5.8 MB copies from pinned memory 52.3 GB/s on one stream, 57.1 on two, 57.2 on three or four, one
+// copy of 346 MB 57.2.  DeepSeek-V2-Lite, 2048 tokens, three layers of 195 modules each staged: 67.5 -> 63.0 ms (61.1 in a plain loop).
+constexpr int kCopyStreams = 2;
+inline int stream_of_slot(int slot) { return slot % kCopyStreams; }
+
 // Copies out of PAGEABLE host memory (a mapped weight segment that was not allocated pinned): a worker thread
 // moves each module through a ring of pinned chunks -- host memcpy into the next chunk (split over a few helper
-// threads), then hipMemcpyAsync out of it on the copy stream -- so the segment is never copied whole and the
+// threads), then hipMemcpyAsync out of it on the slot's copy stream -- so the segment is never copied whole and the
 // pinned memory is n_chunks x chunk_bytes.  A chunk is refilled once the event recorded behind its last
 // hipMemcpyAsync has completed; the memcpy into one chunk overlaps the DMA out of the others.
 struct BounceJob {
     uint64_t seq = 0;
     uint8_t* dst = nullptr;
     std::vector<Piece> pieces;
+    hipStream_t stream = nullptr;
     hipEvent_t wait_for = nullptr;   // release event of the slot's previous user (device backend), or null
     hipEvent_t ready = nullptr;
 };
@@ -89,7 +97,6 @@ struct BounceJob {
 struct Bounce {
     int n_chunks = 0, n_threads = 1, device = 0, backend = MOE_STAGE_DEVICE;
     size_t chunk_bytes = 0;
-    hipStream_t stream = nullptr;
     std::vector<uint8_t*> chunk;
     std::vector<hipEvent_t> done;
     std::vector<char> busy;
@@ -118,7 +125,7 @@ struct Bounce {
     }
     int run_job(const BounceJob& j) {
         const bool dev = backend == MOE_STAGE_DEVICE;
-        if (dev && j.wait_for) MOE_HIP_CHECK(hipStreamWaitEvent(stream, j.wait_for, 0));
+        if (dev && j.wait_for) MOE_HIP_CHECK(hipStreamWaitEvent(j.stream, j.wait_for, 0));
         for (const Piece& p : j.pieces)
             for (size_t off = 0; off < p.bytes; off += chunk_bytes) {
                 const size_t len = std::min(chunk_bytes, p.bytes - off);
@@ -127,14 +134,14 @@ struct Bounce {
                 if (dev && busy[c]) MOE_HIP_CHECK(hipEventSynchronize(done[c]));
                 copy_in(chunk[c], static_cast<const uint8_t*>(p.src) + off, len);
                 if (dev) {
-                    MOE_HIP_CHECK(hipMemcpyAsync(j.dst + p.dst_off + off, chunk[c], len, hipMemcpyHostToDevice, stream));
-                    MOE_HIP_CHECK(hipEventRecord(done[c], stream));
+                    MOE_HIP_CHECK(hipMemcpyAsync(j.dst + p.dst_off + off, chunk[c], len, hipMemcpyHostToDevice, j.stream));
+                    MOE_HIP_CHECK(hipEventRecord(done[c], j.stream));
                     busy[c] = 1;
                 } else {
                     std::memcpy(j.dst + p.dst_off + off, chunk[c], len);
                 }
             }
-        if (dev) MOE_HIP_CHECK(hipEventRecord(j.ready, stream));
+        if (dev) MOE_HIP_CHECK(hipEventRecord(j.ready, j.stream));
         return MOE_OK;
     }
     void loop() {
@@ -157,7 +164,7 @@ struct Bounce {
             cv_done.notify_all();
         }
     }
-    // blocks until the copies of job `seq` have been enqueued on the copy stream
+    // blocks until the copies of job `seq` have been enqueued on its copy stream
     int wait_issued(uint64_t seq) {
         std::unique_lock<std::mutex> lk(mu);
         cv_done.wait(lk, [&] { return issued >= seq; });
@@ -184,7 +191,7 @@ struct Bounce {
 struct moe_stager {
     int backend = MOE_STAGE_DEVICE;
     Bounce bounce;
-    hipStream_t copy_stream = nullptr;
+    hipStream_t copy_stream[kCopyStreams] = {};
     std::vector<Type> types;
     std::vector<Module> modules;
     int64_t n_copies = 0, n_bytes = 0;
@@ -193,14 +200,19 @@ struct moe_stager {
     int decoding = 0;
     int n_held = 0;              // modules acquired and not yet released
     // Events of one consumer stream are recorded in ticket order, so a wait for ticket T covers every smaller one.
-    // Which ticket the copy stream already waits for, per consumer stream: for copies enqueued by the caller's
+    // Which ticket each copy stream already waits for, per consumer stream: for copies enqueued by the caller's
     // thread, and for the bounce worker's jobs (enqueued later, in job order).
     uint64_t ticket = 0;
-    std::vector<std::pair<hipStream_t, uint64_t>> waited_direct, waited_jobs;
+    std::vector<std::pair<hipStream_t, uint64_t>> waited_direct[kCopyStreams], waited_jobs[kCopyStreams];
     std::mutex mu;
 };
 
 namespace {
+
+int sync_copies(moe_stager* st) {
+    for (hipStream_t s : st->copy_stream) MOE_HIP_CHECK(hipStreamSynchronize(s));
+    return MOE_OK;
+}
 
 int find_free(const Type& t) {
     for (int s = 0; s < t.n_active; ++s)
@@ -254,6 +266,8 @@ int copy_into(moe_stager* st, int id, int slot) {
     Module& m = st->modules[id];
     Type& t = st->types[m.type];
     uint8_t* dst = t.mem + (size_t)slot * t.slot_bytes;
+    const int si = stream_of_slot(slot);
+    const hipStream_t stream = st->copy_stream[si];
     if (st->backend == MOE_STAGE_DEVICE && t.freed_pending[slot]) {
         int rc = flush_released(st);
         if (rc != MOE_OK) return rc;
@@ -266,10 +280,11 @@ int copy_into(moe_stager* st, int id, int slot) {
         }
         BounceJob j;
         j.dst = dst;
+        j.stream = stream;
         j.pieces = m.pieces;
         j.ready = m.ready;
         if (st->backend == MOE_STAGE_DEVICE && t.freed_valid[slot]) {
-            if (need_wait(st->waited_jobs, t.freed_strm[slot], t.freed_ticket[slot])) j.wait_for = t.freed_ev[slot];
+            if (need_wait(st->waited_jobs[si], t.freed_strm[slot], t.freed_ticket[slot])) j.wait_for = t.freed_ev[slot];
             t.freed_valid[slot] = 0;
         }
         {
@@ -281,13 +296,13 @@ int copy_into(moe_stager* st, int id, int slot) {
         b.cv_job.notify_one();
     } else if (st->backend == MOE_STAGE_DEVICE) {
         if (t.freed_valid[slot]) {
-            if (need_wait(st->waited_direct, t.freed_strm[slot], t.freed_ticket[slot]))
-                MOE_HIP_CHECK(hipStreamWaitEvent(st->copy_stream, t.freed_ev[slot], 0));
+            if (need_wait(st->waited_direct[si], t.freed_strm[slot], t.freed_ticket[slot]))
+                MOE_HIP_CHECK(hipStreamWaitEvent(stream, t.freed_ev[slot], 0));
             t.freed_valid[slot] = 0;
         }
         for (const Piece& p : m.pieces)
-            MOE_HIP_CHECK(hipMemcpyAsync(dst + p.dst_off, p.src, p.bytes, hipMemcpyHostToDevice, st->copy_stream));
-        MOE_HIP_CHECK(hipEventRecord(m.ready, st->copy_stream));
+            MOE_HIP_CHECK(hipMemcpyAsync(dst + p.dst_off, p.src, p.bytes, hipMemcpyHostToDevice, stream));
+        MOE_HIP_CHECK(hipEventRecord(m.ready, stream));
     } else {
         for (const Piece& p : m.pieces) std::memcpy(dst + p.dst_off, p.src, p.bytes);
     }
@@ -339,7 +354,7 @@ int fetch_one(moe_stager* st, int id) {
     if (slot < 0) {
         // A slot whose module nobody has acquired and no fetch has named -- left there by the cyclic prefetch before
         // the type was switched to on-demand, or by an earlier call's surplus -- is taken over: no consumer reads
-        // it, and the new copy follows the old one on the copy stream.
+        // it, and the new copy follows the old one on the slot's copy stream.
         for (int s = 0; s < t.n_active && slot < 0; ++s) {
             Module& o = st->modules[t.owner[s]];
             if (!o.held && !o.wanted) {
@@ -393,7 +408,8 @@ int drop_residency(moe_stager* st, int ti, const char* who) {
     if (st->backend == MOE_STAGE_DEVICE) {
         int rc = flush_released(st);        // (the consumers' streams are named now, while they certainly exist)
         if (rc != MOE_OK) return rc;
-        MOE_HIP_CHECK(hipStreamSynchronize(st->copy_stream));
+        rc = sync_copies(st);
+        if (rc != MOE_OK) return rc;
     }
     for (int s = 0; s < t.n_total; ++s) {
         if (t.owner[s] >= 0) {
@@ -448,18 +464,22 @@ extern "C" int moe_stage_create(moe_stager** out, int32_t n_types, const size_t*
         t.freed_valid.assign(t.n_total, 0);
     }
     if (backend == MOE_STAGE_DEVICE) {
-        hipError_t e = hipStreamCreateWithFlags(&st->copy_stream, hipStreamNonBlocking);
-        if (e != hipSuccess) {
-            moe::set_error("moe_stage_create: hipStreamCreateWithFlags: %s", hipGetErrorString(e));
-            delete st;
-            return MOE_ERR_HIP;
+        hipError_t e = hipSuccess;
+        for (hipStream_t& s : st->copy_stream) {
+            e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
+            if (e != hipSuccess) {
+                s = nullptr;
+                moe::set_error("moe_stage_create: hipStreamCreateWithFlags: %s", hipGetErrorString(e));
+                moe_stage_destroy(st);
+                return MOE_ERR_HIP;
+            }
         }
         for (Type& t : st->types)
             for (int s = 0; s < t.n_total; ++s) {
                 e = hipEventCreateWithFlags(&t.freed[s], hipEventDisableTiming);
                 if (e != hipSuccess) {
                     moe::set_error("moe_stage_create: hipEventCreateWithFlags: %s", hipGetErrorString(e));
-                    moe_stage_destroy(st);   // releases the stream and the events made so far
+                    moe_stage_destroy(st);   // releases the streams and the events made so far
                     return MOE_ERR_HIP;
                 }
             }
@@ -502,7 +522,6 @@ extern "C" int moe_stage_set_bounce(moe_stager* st, int32_t n_chunks, size_t chu
     Bounce& b = st->bounce;
     MOE_REQUIRE(b.n_chunks == 0, "moe_stage_set_bounce: the bounce ring is already configured");
     b.backend = st->backend;
-    b.stream = st->copy_stream;
     b.chunk_bytes = chunk_bytes;
     b.n_threads = n_threads;
     if (st->backend == MOE_STAGE_DEVICE) MOE_HIP_CHECK(hipGetDevice(&b.device));
@@ -770,7 +789,7 @@ extern "C" int moe_stage_sync(moe_stager* st) {
     if (st->backend == MOE_STAGE_DEVICE) {
         int rc = flush_released(st);
         if (rc != MOE_OK) return rc;
-        MOE_HIP_CHECK(hipStreamSynchronize(st->copy_stream));
+        return sync_copies(st);
     }
     return MOE_OK;
 }
@@ -779,13 +798,15 @@ extern "C" int moe_stage_destroy(moe_stager* st) {
     if (!st) return MOE_OK;
     st->bounce.shutdown();   // (joins the worker: queued jobs are finished first)
     if (st->backend == MOE_STAGE_DEVICE) {
-        (void)hipStreamSynchronize(st->copy_stream);
+        for (hipStream_t s : st->copy_stream)
+            if (s) (void)hipStreamSynchronize(s);
         for (Module& m : st->modules)
             if (m.ready) (void)hipEventDestroy(m.ready);
         for (Type& t : st->types)
             for (hipEvent_t ev : t.freed)
                 if (ev) (void)hipEventDestroy(ev);
-        (void)hipStreamDestroy(st->copy_stream);
+        for (hipStream_t s : st->copy_stream)
+            if (s) (void)hipStreamDestroy(s);
     }
     delete st;
     return MOE_OK;

@@ -1,4 +1,4 @@
-"""Weight staging on the device: pinned host -> HBM slots on the copy stream, event hand-off."""
+"""Weight staging on the device: pinned host -> HBM slots on the copy streams, event hand-off."""
 import pytest
 import torch
 
@@ -50,6 +50,34 @@ def test_stager_overlaps_with_compute():
         st.free_weights_buffer(f"routed_expert_0_{i}")
         assert torch.isfinite(s) and same
     torch.cuda.synchronize()
+    st.close()
+
+
+@pytest.mark.parametrize("pool", [1, 2, 3, 5])
+def test_slots_refilled_before_anyone_read_them(pool):
+    """Copies run on several streams, those into one slot one after the other: a slot whose module is let go unread is
+    refilled while its copy may still run, and what a consumer then gets is the later one."""
+    from moe_gen_amd import Stager
+    st = Stager({"routed_expert": {"a": ((1024, 2048), torch.bfloat16), "b": ((512, 1024), torch.bfloat16)}}, {"routed_expert": pool})
+    src = [{"a": torch.full((1024, 2048), float(i), dtype=torch.bfloat16).pin_memory(),
+            "b": torch.full((512, 1024), float(i) + 0.5, dtype=torch.bfloat16).pin_memory()} for i in range(7)]
+    for i, t in enumerate(src):
+        st.add_module(f"routed_expert_0_{i}", "routed_expert", t)
+    streams, seen = [torch.cuda.Stream(), torch.cuda.Stream()], []
+    st.pump()
+    for n in range(42):
+        key = f"routed_expert_0_{n % 7}"
+        if n % 3:
+            st.free_weights_buffer(key)                  # prefetched and dropped
+            continue
+        with torch.cuda.stream(streams[n & 1]):
+            w = st.get_weights(key)
+            seen.append((n % 7, w["a"].clone(), w["b"].clone()))
+            st.free_weights_buffer(key)
+    torch.cuda.synchronize()
+    st.sync()
+    for i, a, b in seen:
+        assert torch.equal(a.cpu(), src[i]["a"]) and torch.equal(b.cpu(), src[i]["b"]), i
     st.close()
 
 
