@@ -13,12 +13,13 @@
 //
 // One block per token; a lane handles 8 consecutive bf16 (16 bytes) of the row, so
 // every global access is a full 16-byte vector and a wave covers 1 KiB contiguous.
+#include "combine_math.h"
 #include "common.h"
 
 namespace moe {
 namespace {
 
-constexpr int MAX_K = 16;
+constexpr int MAX_K = kCombineMaxK;
 
 // KB: source rows whose 16-byte chunks a lane requests back to back before it starts adding (the
 // sum itself stays in slot order).  The kernel is bound by HBM latency x bytes in flight, and one
@@ -46,7 +47,7 @@ __global__ __launch_bounds__(1024) void combine_kernel(const u32x4* __restrict__
         }
         s_row[a] = pos[(size_t)t * k + j];
         const float w = topk_w[(size_t)t * k + j];
-        s_w[a] = (MODE == MOE_COMBINE_F32) ? w : round_to_bf16(w);
+        s_w[a] = combine_weight<MODE>(w);
     }
     __syncthreads();
     for (int c = threadIdx.x; c < chunks; c += blockDim.x) {
@@ -67,44 +68,10 @@ __global__ __launch_bounds__(1024) void combine_kernel(const u32x4* __restrict__
         for (int b = 0; b < KB; ++b) {
             if (a0 + b >= k) break;
             if (s_row[a0 + b] < 0) continue;
-            const u32x4 v = vb[b];
-            const float w = s_w[a0 + b];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                float lo = __uint_as_float(v[i] << 16), hi = __uint_as_float(v[i] & 0xffff0000u);
-                if (MODE == MOE_COMBINE_F32) {
-                    acc[2 * i] = acc[2 * i] + lo * w;
-                    acc[2 * i + 1] = acc[2 * i + 1] + hi * w;
-                } else {
-                    acc[2 * i] = acc[2 * i] + round_to_bf16(lo * w);
-                    acc[2 * i + 1] = acc[2 * i + 1] + round_to_bf16(hi * w);
-                    if (MODE == MOE_COMBINE_BF16_SEQ) {
-                        acc[2 * i] = round_to_bf16(acc[2 * i]);
-                        acc[2 * i + 1] = round_to_bf16(acc[2 * i + 1]);
-                    }
-                }
-            }
+            combine_add<MODE>(acc, vb[b], s_w[a0 + b]);
         }
         }
-        u32x4 o;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            uint32_t lo = f32_to_bf16_bits(acc[2 * i]), hi = f32_to_bf16_bits(acc[2 * i + 1]);
-            if (shared) {  // bf16 + bf16 -> bf16, as torch adds two bf16 tensors
-                lo = f32_to_bf16_bits(bf16_bits_to_f32(lo) + __uint_as_float(sh[i] << 16));
-                hi = f32_to_bf16_bits(bf16_bits_to_f32(hi) + __uint_as_float(sh[i] & 0xffff0000u));
-            }
-            o[i] = lo | (hi << 16);
-        }
-        if (residual) {
-            const u32x4 r = res;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t lo = f32_to_bf16_bits(__uint_as_float(r[i] << 16) + __uint_as_float(o[i] << 16));
-                const uint32_t hi = f32_to_bf16_bits(__uint_as_float(r[i] & 0xffff0000u) + __uint_as_float(o[i] & 0xffff0000u));
-                o[i] = lo | (hi << 16);
-            }
-        }
+        const u32x4 o = combine_finish(acc, shared != nullptr, sh, residual != nullptr, res);
         __builtin_nontemporal_store(o, &out[(size_t)t * chunks + c]);
     }
 }

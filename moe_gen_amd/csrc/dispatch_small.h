@@ -13,25 +13,29 @@ struct DispatchOut {
     int32_t *counts, *offsets, *perm, *pos;
     int32_t* row_map;        // perm / k, may be NULL
     int32_t* one_group;      // [2]: {0, tokens}, the row range of a group that holds every token (the shared expert); may be NULL
+    // [n_arrivals]: set to minus the experts that have rows and the one of one_group (CombineTail; one workgroup's form only)
+    int32_t* arrivals = nullptr;
+    int n_arrivals = 0;
 };
 
-// Wave w owns the w-th slice of the list (a multiple of 64 entries, at most IT of them): counts it, the first 256 threads
+// (NW waves.)  Wave w owns the w-th slice of the list (a multiple of 64 entries, at most IT of them): counts it, the first 256 threads
 // turn the 16 x E counts into counts[], offsets[] and one cursor per (wave, expert) -- offsets[e] + entries of e in
 // earlier slices -- and every wave ranks its slice 64 entries at a time.  The sorted position of an entry is the same
 // pure function of the list as in the three-kernel form.  get(i): entry i of the list, i < nk.
-template <int IT, typename F>
+template <int IT, int NW = SMALL_WAVES, typename F>
 __device__ __forceinline__ void dispatch_one_workgroup(int nk, int E, const DispatchOut& out, int k, F get) {
-    __shared__ int whist[SMALL_WAVES][kDispatchMaxE];
+    static_assert(64 * NW >= kDispatchMaxE, "a thread per expert");
+    __shared__ int whist[NW][kDispatchMaxE];
     __shared__ int wtot[4];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int slice = (nk + SMALL_WAVES * 64 - 1) / (SMALL_WAVES * 64) * 64;
+    const int slice = (nk + NW * 64 - 1) / (NW * 64) * 64;
     const int wbase = wave * slice;
     // the lane's entries of the slice, all requested at once (both passes use them: a load per step would put the
     // memory latency into every step); -1 marks an entry past the list or an id outside [0, E)
     int ev[IT];
 #pragma unroll
     for (int it = 0; it < IT; ++it) ev[it] = get(min(wbase + 64 * it + lane, nk - 1));
-    for (int e = tid; e < SMALL_WAVES * kDispatchMaxE; e += 64 * SMALL_WAVES) (&whist[0][0])[e] = 0;
+    for (int e = tid; e < NW * kDispatchMaxE; e += 64 * NW) (&whist[0][0])[e] = 0;
     __syncthreads();
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
@@ -44,7 +48,7 @@ __device__ __forceinline__ void dispatch_one_workgroup(int nk, int E, const Disp
     if (tid < kDispatchMaxE) {                 // waves 0 .. 3, whole waves
         if (tid < E) {
 #pragma unroll
-            for (int w = 0; w < SMALL_WAVES; ++w) cv += whist[w][tid];
+            for (int w = 0; w < NW; ++w) cv += whist[w][tid];
         }
         inc = cv;
 #pragma unroll
@@ -62,14 +66,15 @@ __device__ __forceinline__ void dispatch_one_workgroup(int nk, int E, const Disp
         out.offsets[tid] = run;
         if (tid == E - 1) out.offsets[E] = run + cv;
 #pragma unroll
-        for (int w = 0; w < SMALL_WAVES; ++w) {
+        for (int w = 0; w < NW; ++w) {
             const int c = whist[w][tid];
             whist[w][tid] = run;
             run += c;
         }
     }
     if (out.one_group && tid < 2) out.one_group[tid] = tid ? nk / k : 0;
-    __syncthreads();
+    const int busy = __syncthreads_count(tid < E && cv > 0);
+    for (int i = tid; i < out.n_arrivals; i += 64 * NW) out.arrivals[i] = -(busy + (out.one_group ? 1 : 0));
     int* cur = whist[wave];
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
@@ -107,6 +112,11 @@ int router_select(const float* bias, const moe_router_params& p, int32_t* topk_i
 // launches 10.)
 constexpr int select_dispatch_tokens(int E) { return SMALL_WAVES * (E <= 16 ? 4 : E <= 32 ? 2 : 1); }
 constexpr int kSelectDispatchTokens = 64;
+// logits, routing and dispatch in one launch of one workgroup, where that has every expert in one block and its 4 waves
+// route the tokens in one pass
+constexpr int router_dispatch_tokens(int E) { return E <= 16 ? 16 : E <= 32 ? 8 : E <= 64 ? 4 : 0; }
+int router_dispatch(const void* x, const void* w_gate, const float* bias, const moe_router_params& p, int32_t* topk_idx, float* topk_w,
+                    uint16_t* logits_bf16, const DispatchOut& out, hipStream_t st);
 int router_select_dispatch(const float* bias, const moe_router_params& p, int32_t* topk_idx, float* topk_w, float* logits,
                            uint16_t* logits_bf16, const DispatchOut& out, hipStream_t st);
 int check_router(const void* x, const void* w_gate, const moe_router_params* params, const int32_t* topk_idx, const float* topk_w);

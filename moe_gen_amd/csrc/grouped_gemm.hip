@@ -50,7 +50,9 @@
 #include <cmath>
 #include <type_traits>
 
+#include "combine_math.h"
 #include "common.h"
+#include "layer.h"
 
 namespace moe {
 namespace {
@@ -1622,11 +1624,89 @@ __global__ __launch_bounds__(128 * WN) void grouped_gemm_kernel(GemmPair pair_of
     }
 }
 
+// ---- the combine of a few tokens at the end of their down projection ----
+//
+// tail.arrivals: a counter per column tile, minus the waves that will write its columns (an expert with rows each, and the
+// shared expert); the dispatch of the call sets them.  The wave that brings a counter to zero finds every expert's columns
+// written and adds them up: no wave waits for another.  What waves on other XCDs read leaves and arrives past the L2 of an XCD
+// (relaxed atomics at agent scope), a wave's stores being complete before it counts itself.
+__device__ __forceinline__ void store_shared_8(uint16_t* p, const u32x2& v) {
+    __hip_atomic_store(reinterpret_cast<uint64_t*>(p), __builtin_bit_cast(uint64_t, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ u32x4 load_shared_16(const uint16_t* p) {
+    const uint64_t* q = reinterpret_cast<const uint64_t*>(p);
+    const u32x2 a = __builtin_bit_cast(u32x2, __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    const u32x2 b = __builtin_bit_cast(u32x2, __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    return u32x4{a[0], a[1], b[0], b[1]};
+}
+
+// A wave's share of the call's slots (up to kTailTokens * kCombineMaxK of them), requested before its products: what is left
+// behind the last arrival is a trip to memory for the rows
+struct TailSlots {
+    static constexpr int N = kTailTokens * kCombineMaxK / 64;
+    int id[N], row[N];
+    float w[N];
+    __device__ __forceinline__ TailSlots(const CombineTail& tail) {
+#pragma unroll
+        for (int u = 0; u < N; ++u) {
+            const int i = min((int)threadIdx.x + 64 * u, tail.n * tail.k - 1);
+            id[u] = tail.topk_idx[i];
+            row[u] = tail.pos[i];
+            w[u] = tail.topk_w[i];
+        }
+    }
+};
+
+// NCOL columns from n0 on of every token (at most kTailTokens), by one wave; a lane has 8 columns of a token.  lds: idle, 3 KiB
+template <int MODE, int NCOL>
+__device__ __forceinline__ void combine_columns(const CombineTail& tail, const TailSlots& slots, const uint16_t* y, const uint16_t* shared,
+                                                int h, int n0, uint8_t* lds) {
+    static_assert(kTailTokens * NCOL / 8 <= 64, "a chunk of 8 columns per lane");
+    const int lane = threadIdx.x, k = tail.k, nk = tail.n * k;
+    int* const rows = reinterpret_cast<int*>(lds);                    // [token][place in the summation order]
+    float* const weights = reinterpret_cast<float*>(lds + kTailTokens * kCombineMaxK * 4);
+    int* const ids = reinterpret_cast<int*>(lds + 2 * kTailTokens * kCombineMaxK * 4);
+    if (MODE == MOE_COMBINE_BF16_SEQ) {
+#pragma unroll
+        for (int u = 0; u < TailSlots::N; ++u) ids[lane + 64 * u] = slots.id[u];
+        __syncthreads();
+    }
+#pragma unroll
+    for (int u = 0; u < TailSlots::N; ++u) {
+        const int i = lane + 64 * u;
+        if (i >= nk) break;
+        const int t = i / k;
+        int a = i - t * k;
+        if (MODE == MOE_COMBINE_BF16_SEQ) {
+            a = 0;
+            for (int v = 0; v < k; ++v) a += ids[t * k + v] < slots.id[u] ? 1 : 0;
+        }
+        rows[t * kCombineMaxK + a] = slots.row[u];
+        weights[t * kCombineMaxK + a] = combine_weight<MODE>(slots.w[u]);
+    }
+    __syncthreads();
+    const int t = lane / (NCOL / 8), col = n0 + 8 * (lane % (NCOL / 8));
+    if (t >= tail.n || col >= h) return;
+    float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    u32x4 sh = {0, 0, 0, 0}, res = {0, 0, 0, 0};
+    if (shared) sh = load_shared_16(shared + (size_t)t * h + col);
+    if (tail.residual) res = *reinterpret_cast<const u32x4*>(tail.residual + (size_t)t * h + col);
+    for (int a0 = 0; a0 < k; a0 += 8) {
+        u32x4 v[8];
+#pragma unroll
+        for (int b = 0; b < 8; ++b) v[b] = load_shared_16(y + (size_t)max(rows[t * kCombineMaxK + min(a0 + b, k - 1)], 0) * h + col);
+#pragma unroll
+        for (int b = 0; b < 8; ++b)
+            if (a0 + b < k && rows[t * kCombineMaxK + a0 + b] >= 0) combine_add<MODE>(acc, v[b], weights[t * kCombineMaxK + a0 + b]);
+    }
+    *reinterpret_cast<u32x4*>(tail.out + (size_t)t * h + col) = combine_finish(acc, shared != nullptr, sh, tail.residual != nullptr, res);
+}
+
 // ---- thin kernel: calls in which no expert has more than 16 rows (decoding a few sequences), where thin_pays ----
 //
 // Such a call touches a few experts, and cut into tiles of 256 weight rows it has fewer tiles than the chip has CUs
 // (one token of DeepSeek-V2-Lite: 66) or two and a half rounds of them.  Here the unit is a WAVE with 32 weight rows --
-// 16 gate rows and the matching up rows, or 32 down rows -- and the whole K, each wave a workgroup of its own: no
+// 16 gate rows and the matching up rows, or 32 down rows (16 where that leaves most of the chip idle, thin_down_narrow) -- and the whole K, each wave a workgroup of its own: no
 // barrier, six of them per CU, and nothing to wait for but its own DMA.  A stage is 128 bytes of each weight row (64 k of
 // bf16, 128 of fp8: whole lines) and the same k of 16 token rows (rows that do not exist cost no request), NB stages in
 // a ring.  Every matrix instruction gets the k values that the streamers above give it, in the same lanes and the same
@@ -1634,13 +1714,16 @@ __global__ __launch_bounds__(128 * WN) void grouped_gemm_kernel(GemmPair pair_of
 // Measured (us, tile kernel -> this): DeepSeek-V2-Lite, one token (8 x 1408 of 2048) 25 + 25 and 19 + 33 -> 17 and 14;
 // DeepSeek-V3, 5 tokens (39 experts, fp8) 190 and 115 -> 187 and 92 = 6.0 TB/s.  Weights loaded into registers instead
 // reach 4 ... 5 TB/s: a fragment load then takes half a line from each of 16 rows.
-template <bool SWIGLU, bool W8>
-__global__ __launch_bounds__(64) void grouped_gemm_thin_kernel(GemmPair pair_of) {
-    constexpr int TBYTES = W8 ? 4096 : 2048;      // 16 token rows of a stage
-    constexpr int NB = W8 ? 3 : 4;                // stages in LDS
-    constexpr int NDT = TBYTES / 1024, NI = 4 + NDT;   // DMA instructions per stage: 4 for the weights
-    constexpr int NCOL = SWIGLU ? 16 : 32;        // output columns of a wave
-    constexpr int SB = 4096 + TBYTES;
+template <bool SWIGLU, bool W8, int NF, bool TAIL>
+__global__ __launch_bounds__(64) void grouped_gemm_thin_kernel(GemmPair pair_of, CombineTail tail) {
+    static_assert(!SWIGLU || NF == 2, "gate and up: a fragment of either");
+    static_assert(!TAIL || NF == 1, "the combine's rule");
+    constexpr int WBYTES = NF * 2048, TBYTES = W8 ? 4096 : 2048;       // weights and 16 token rows of a stage
+    constexpr int NDW = 2 * NF, NDT = TBYTES / 1024, NI = NDW + NDT;   // DMA instructions per stage
+    constexpr int NCOL = SWIGLU ? 16 : 16 * NF;   // output columns of a wave
+    constexpr int SB = WBYTES + TBYTES;
+    constexpr int NB = 24576 / SB;                // stages in LDS
+    static_assert(NB >= 3 && (NB - 1) * NI < 64, "stages");
     __shared__ __attribute__((aligned(1024))) uint8_t lds[NB * SB];
     const int lane = threadIdx.x;
     const bool of_shared = (int)blockIdx.x < pair_of.shared_tiles;
@@ -1682,6 +1765,7 @@ __global__ __launch_bounds__(64) void grouped_gemm_thin_kernel(GemmPair pair_of)
         left -= tot;
     }
     if (e < 0) return;
+    [[maybe_unused]] const auto slots = [&] { if constexpr (TAIL) return TailSlots(tail); else return 0; }();
     const int n0 = (unit % tiles) * NCOL;
     const int nk = K / (W8 ? 128 : 64);
     const int rot = (n0 / (SWIGLU ? 128 : 256)) % nk;      // the k rotation of the N tile these columns belong to
@@ -1698,16 +1782,16 @@ __global__ __launch_bounds__(64) void grouped_gemm_thin_kernel(GemmPair pair_of)
     // lane / 8; tokens, instruction i: 8 (fp8: 4) rows; chunks swizzled as in the streamers
     const int lr = lane >> 3, pp = lane & 7;
     const uint32_t row_bytes = (uint32_t)K * (W8 ? 1 : 2);
-    uint32_t w_voff[4], t_voff[4];                         // (NDT of the latter are used)
+    uint32_t w_voff[4], t_voff[4];                         // (NDW and NDT are used)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < NDW; ++i) {
         const int fr = 8 * (i & 1) + lr;
         w_voff[i] = (uint32_t)min(n0 + (SWIGLU ? 0 : 16 * (i >> 1)) + fr, N - 1) * row_bytes + (uint32_t)((pp ^ (W8 ? wsw(fr) : swz(fr))) << 4);
     }
     const int frow = lane & 15, q = lane >> 4;
     const int fq = ((q & 1) << 1) | (q >> 1);
     const uint32_t w_rd = (uint32_t)(frow * 128), wkey = (uint32_t)(W8 ? wsw(frow) : swz(frow));
-    const uint32_t t_rd = 4096u + (uint32_t)(frow * (W8 ? 256 : 128)), tkey = (uint32_t)(W8 ? tsw(frow) : swz(frow));
+    const uint32_t t_rd = (uint32_t)WBYTES + (uint32_t)(frow * (W8 ? 256 : 128)), tkey = (uint32_t)(W8 ? tsw(frow) : swz(frow));
 
     for (int r0 = row0; r0 < row_end; r0 += 16) {          // (more than once only if a caller's row bound was wrong)
         const uint8_t* a_base = reinterpret_cast<const uint8_t*>(g.a) + (g.row_map ? (size_t)0 : (size_t)r0 * K * 2);
@@ -1729,13 +1813,17 @@ __global__ __launch_bounds__(64) void grouped_gemm_thin_kernel(GemmPair pair_of)
             const __amdgpu_buffer_rsrc_t rad = __builtin_amdgcn_make_buffer_rsrc((void*)a_base, 0, live & a_records, 0x00020000);
             __builtin_amdgcn_raw_ptr_buffer_load_lds(r0d, (lds_u8)d, 16, w_voff[0], so, 0, 2);
             __builtin_amdgcn_raw_ptr_buffer_load_lds(r0d, (lds_u8)(d + 1024), 16, w_voff[1], so, 0, 2);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(r1d, (lds_u8)(d + 2048), 16, w_voff[2], so, 0, 2);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(r1d, (lds_u8)(d + 3072), 16, w_voff[3], so, 0, 2);
+            if constexpr (NF == 2) {
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(r1d, (lds_u8)(d + 2048), 16, w_voff[2], so, 0, 2);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(r1d, (lds_u8)(d + 3072), 16, w_voff[3], so, 0, 2);
+            }
 #pragma unroll
             for (int i = 0; i < NDT; ++i)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(rad, (lds_u8)(d + 4096 + i * 1024), 16, t_voff[i], W8 ? 2 * so : so, 0, 0);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rad, (lds_u8)(d + WBYTES + i * 1024), 16, t_voff[i], W8 ? 2 * so : so, 0, 0);
         };
-        f32x4 acc[2] = {f32x4{0}, f32x4{0}};
+        f32x4 acc[NF];
+#pragma unroll
+        for (int j = 0; j < NF; ++j) acc[j] = f32x4{0};
         float v0 = 0.0f, v1 = 0.0f;                        // fp8: lane l holds the scales of stage 64 i + l
         if (W8) { v0 = sc0[stage_at(lane)]; v1 = sc1[stage_at(lane)]; }
         for (int i = 0; i < NB - 1; ++i) dma(i, i);
@@ -1758,14 +1846,14 @@ __global__ __launch_bounds__(64) void grouped_gemm_thin_kernel(GemmPair pair_of)
                                     __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v1), k & 63))};
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
-                    u32x4 raw[2];
+                    u32x4 raw[NF];
 #pragma unroll
-                    for (int j = 0; j < 2; ++j) raw[j] = *reinterpret_cast<const u32x4*>(b + j * 2048 + w_rd + (((4 * h + fq) ^ wkey) << 4));
+                    for (int j = 0; j < NF; ++j) raw[j] = *reinterpret_cast<const u32x4*>(b + j * 2048 + w_rd + (((4 * h + fq) ^ wkey) << 4));
 #pragma unroll
                     for (int s2 = 0; s2 < 2; ++s2) {
                         const bf16x8 tf = *reinterpret_cast<const bf16x8*>(b + t_rd + (((8 * h + 2 * fq + s2) ^ tkey) << 4));
 #pragma unroll
-                        for (int j = 0; j < 2; ++j)
+                        for (int j = 0; j < NF; ++j)
                             acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
                                 __builtin_bit_cast(bf16x8, dequant8(raw[j][2 * s2], raw[j][2 * s2 + 1], c[j])), tf, acc[j], 0, 0, 0);
                     }
@@ -1776,7 +1864,7 @@ __global__ __launch_bounds__(64) void grouped_gemm_thin_kernel(GemmPair pair_of)
                     const uint32_t coff = (uint32_t)((4 * s + fq) ^ wkey) << 4;      // (wkey == tkey)
                     const bf16x8 tf = *reinterpret_cast<const bf16x8*>(b + t_rd + coff);
 #pragma unroll
-                    for (int j = 0; j < 2; ++j)
+                    for (int j = 0; j < NF; ++j)
                         acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(b + j * 2048 + w_rd + coff), tf, acc[j], 0, 0, 0);
                 }
             }
@@ -1786,13 +1874,29 @@ __global__ __launch_bounds__(64) void grouped_gemm_thin_kernel(GemmPair pair_of)
         const int r = r0 + frow;
         if (r < row_end) {
 #pragma unroll
-            for (int j = 0; j < (SWIGLU ? 1 : 2); ++j) {
+            for (int j = 0; j < (SWIGLU ? 1 : NF); ++j) {
                 const int col = n0 + 16 * j + 4 * q;
-                if (col < N) *reinterpret_cast<u32x2*>(g.c + (size_t)r * N + col) = epilogue_pack<SWIGLU>(acc[j], acc[SWIGLU ? 1 : j]);
+                if (col >= N) continue;
+                const u32x2 o = epilogue_pack<SWIGLU>(acc[j], acc[SWIGLU ? 1 : j]);
+                if constexpr (TAIL) store_shared_8(g.c + (size_t)r * N + col, o);
+                else *reinterpret_cast<u32x2*>(g.c + (size_t)r * N + col) = o;
             }
         }
     }
+    if constexpr (TAIL) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's columns are where every XCD finds them
+        int left_out = 0;
+        if (lane == 0) left_out = __hip_atomic_fetch_add(tail.arrivals + unit % tiles, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (__builtin_amdgcn_readfirstlane(left_out) != -1) return;
+        asm volatile("" ::: "memory");
+        const uint16_t* const y = pair_of.p[0].c;
+        const uint16_t* const sh = pair_of.shared_tiles > 0 ? pair_of.p[1].c : nullptr;
+        if (tail.mode == MOE_COMBINE_F32) combine_columns<MOE_COMBINE_F32, NCOL>(tail, slots, y, sh, N, n0, lds);
+        else if (tail.mode == MOE_COMBINE_BF16_PROD) combine_columns<MOE_COMBINE_BF16_PROD, NCOL>(tail, slots, y, sh, N, n0, lds);
+        else combine_columns<MOE_COMBINE_BF16_SEQ, NCOL>(tail, slots, y, sh, N, n0, lds);
+    }
 }
+
 
 // ---- split kernel: the down projection of a dense fp8 MLP at few rows ----
 //
@@ -2332,25 +2436,6 @@ int launch_tiles(const GemmPair& pair, int n_rows, hipStream_t st) {
     return MOE_OK;
 }
 
-template <bool SWIGLU, bool W8>
-int launch_thin(const GemmArgs& g, int n_rows, const GemmArgs* shared, hipStream_t st) {
-    constexpr int NCOL = SWIGLU ? 16 : 32;
-    GemmPair pair{};
-    pair.p[0] = g;
-    if (shared) {
-        pair.p[1] = *shared;
-        pair.shared_tiles = (shared->N + NCOL - 1) / NCOL;
-    }
-    const long grid = (long)(g.E < n_rows ? g.E : n_rows) * ((g.N + NCOL - 1) / NCOL) + pair.shared_tiles;
-    if (grid > 0x7fffffffL) {
-        set_error("grouped gemm: %ld workgroups exceed the grid limit", grid);
-        return MOE_ERR_INVALID;
-    }
-    hipLaunchKernelGGL((grouped_gemm_thin_kernel<SWIGLU, W8>), dim3((unsigned)grid), dim3(64), 0, st, pair);
-    MOE_HIP_CHECK(hipGetLastError());
-    return MOE_OK;
-}
-
 // CUs of the current device (the persistent kernel runs one workgroup on each)
 inline int cu_count() {
     static int cached[64] = {0};
@@ -2362,6 +2447,50 @@ inline int cu_count() {
         cached[dev] = n;
     }
     return cached[dev];
+}
+
+// The combine that the down projection of a layer call may take over: `done` then says so
+struct TailOf {
+    const CombineTail* args = nullptr;
+    bool* done = nullptr;
+};
+
+// waves of 32 columns that the thin kernel's down projection has at most
+inline long thin_down_waves(int E, int n_rows, bool shared, int N) { return ((E < n_rows ? E : n_rows) + (shared ? 1L : 0L)) * ((N + 31) / 32); }
+// Up to two waves per CU: 16 columns each instead of 32, so that twice as many stages are on their way, and the waves combine
+// too, which saves a launch where the host takes as long as the GPU.  Down projection and combine, us, in two launches -> this
+// (16 columns): DeepSeek-V2-Lite, 1 token (448 waves) 13.5 + 4.7 -> 16.3, the call, with the router's launches joined, 52.1 -> 47.3 on
+// weights that are in the caches and 51.1 -> 49.3 on others;
+// Mixtral-8x7B, 1 token (256) 56.1 + 5.7 -> 45.1, the call 161 -> 144.  Beyond, nothing is gained: DeepSeek-V2-Lite, 3 tokens (1216) 17.0 + 5.0 -> 22.8 with
+// 32 columns, Mixtral-8x22B, 2 tokens (768), the call 405 -> 408.
+inline bool thin_down_narrow(long waves) { return waves <= 2L * cu_count(); }
+
+template <bool SWIGLU, bool W8>
+int launch_thin(const GemmArgs& g, int n_rows, const GemmArgs* shared, TailOf tail, hipStream_t st) {
+    GemmPair pair{};
+    pair.p[0] = g;
+    if (shared) pair.p[1] = *shared;
+    const long experts = g.E < n_rows ? g.E : n_rows;
+    auto launch = [&](auto kernel, int ncol, const CombineTail& t) -> int {
+        pair.shared_tiles = shared ? (shared->N + ncol - 1) / ncol : 0;
+        const long grid = experts * ((g.N + ncol - 1) / ncol) + pair.shared_tiles;
+        if (grid > 0x7fffffffL) {
+            set_error("grouped gemm: %ld workgroups exceed the grid limit", grid);
+            return MOE_ERR_INVALID;
+        }
+        hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(64), 0, st, pair, t);
+        MOE_HIP_CHECK(hipGetLastError());
+        return MOE_OK;
+    };
+    if constexpr (SWIGLU) {
+        return launch(grouped_gemm_thin_kernel<true, W8, 2, false>, 16, CombineTail{});
+    } else {
+        const long waves = thin_down_waves(g.E, n_rows, shared != nullptr, g.N);
+        if (!thin_down_narrow(waves)) return launch(grouped_gemm_thin_kernel<false, W8, 2, false>, 32, CombineTail{});
+        if (!tail.args) return launch(grouped_gemm_thin_kernel<false, W8, 1, false>, 16, CombineTail{});
+        *tail.done = true;
+        return launch(grouped_gemm_thin_kernel<false, W8, 1, true>, 16, *tail.args);
+    }
 }
 
 template <bool SWIGLU, bool W8>
@@ -2486,7 +2615,7 @@ int launch_both(const GemmPair& pair, int n_rows, hipStream_t st) {
 
 // max_rows: no expert has more rows (callers that do not know pass n_rows)
 template <bool SWIGLU, bool W8>
-int launch_mt(const GemmArgs& g0, int n_rows, int max_rows, void* workspace, size_t workspace_bytes, hipStream_t st) {
+int launch_mt(const GemmArgs& g0, int n_rows, int max_rows, void* workspace, size_t workspace_bytes, TailOf tail, hipStream_t st) {
     GemmArgs g = g0;
     const long mean = g.E > 0 ? (long)n_rows / g.E : 0;
     if constexpr (W8 && !SWIGLU) {
@@ -2494,7 +2623,7 @@ int launch_mt(const GemmArgs& g0, int n_rows, int max_rows, void* workspace, siz
         if (plan.slices > 1 && workspace_bytes >= (size_t)plan.slices * n_rows * g.N * 4)
             return launch_split(g, n_rows, plan, static_cast<float*>(workspace), st);
     }
-    if (max_rows <= 16 && gather_fits(g) && thin_pays(g, n_rows, nullptr)) return launch_thin<SWIGLU, W8>(g, n_rows, nullptr, st);
+    if (max_rows <= 16 && gather_fits(g) && thin_pays(g, n_rows, nullptr)) return launch_thin<SWIGLU, W8>(g, n_rows, nullptr, tail, st);
     GemmPair pair{};
     if (mean < 128 || !persistent_fits(g)) {
         g.cold_max = 0x7fffffff;
@@ -2542,8 +2671,8 @@ int launch_mt(const GemmArgs& g0, int n_rows, int max_rows, void* workspace, siz
 
 // The shared expert's tiles in the routed experts' launches.  shared.alone: see joint_alone.
 template <bool SWIGLU, bool W8>
-int launch_joint(const GemmArgs& routed, int n_rows, int max_rows, const GemmArgs& shared, int n_shared, hipStream_t st) {
-    if (max_rows <= 16 && n_shared <= 16 && thin_pays(routed, n_rows, &shared)) return launch_thin<SWIGLU, W8>(routed, n_rows, &shared, st);
+int launch_joint(const GemmArgs& routed, int n_rows, int max_rows, const GemmArgs& shared, int n_shared, TailOf tail, hipStream_t st) {
+    if (max_rows <= 16 && n_shared <= 16 && thin_pays(routed, n_rows, &shared)) return launch_thin<SWIGLU, W8>(routed, n_rows, &shared, tail, st);
     GemmPair pair{{routed, shared}, 0, 0};
     if (n_rows / routed.E < 128) {
         pair.p[0].cold_max = pair.p[1].cold_max = 0x7fffffff;
@@ -2636,35 +2765,34 @@ bool joins(const moe_mlp_group& routed, const moe_mlp_group& shared, int32_t hid
 int joint_alone(const moe_mlp_group& shared) { return shared.n_rows < 128 || few_tiles(shared, cu_count()); }
 
 template <bool W8>
-int grouped_swiglu(const moe_mlp_group& m, int32_t hidden, int32_t phases, void* stream, const char* who) {
+int grouped_swiglu(const moe_mlp_group& m, int32_t hidden, int32_t phases, TailOf tail, void* stream, const char* who) {
     MOE_REQUIRE(phases >= MOE_PHASE_GATE_UP && phases <= MOE_PHASE_BOTH, "%s: bad phases %d", who, phases);
     int rc = check_group(m, hidden, W8, who);
     if (rc != MOE_OK || m.n_rows == 0) return rc;
     hipStream_t st = as_stream(stream);
-    if (phases & MOE_PHASE_GATE_UP) rc = launch_mt<true, W8>(gate_up_args(m, hidden), m.n_rows, row_bound(m), nullptr, 0, st);
+    if (phases & MOE_PHASE_GATE_UP) rc = launch_mt<true, W8>(gate_up_args(m, hidden), m.n_rows, row_bound(m), nullptr, 0, TailOf{}, st);
     if (rc == MOE_OK && (phases & MOE_PHASE_DOWN)) 
-        rc = launch_mt<false, W8>(down_args(m, hidden), m.n_rows, row_bound(m), m.workspace, m.workspace_bytes, st);
+        rc = launch_mt<false, W8>(down_args(m, hidden), m.n_rows, row_bound(m), m.workspace, m.workspace_bytes, tail, st);
     return rc;
 }
 
 template <bool W8>
-int grouped_swiglu_joint(const moe_mlp_group& r, const moe_mlp_group& s, int32_t hidden, int32_t phases, void* stream) {
-    const char* who = "moe_grouped_swiglu_joint";
+int grouped_swiglu_joint(const moe_mlp_group& r, const moe_mlp_group& s, int32_t hidden, int32_t phases, TailOf tail, void* stream, const char* who) {
     MOE_REQUIRE(phases >= MOE_PHASE_GATE_UP && phases <= MOE_PHASE_BOTH, "%s: bad phases %d", who, phases);
     int rc = check_group(r, hidden, W8, who);
     if (rc == MOE_OK) rc = check_group(s, hidden, W8, who);
     if (rc != MOE_OK) return rc;
     if (!joins(r, s, hidden)) {
-        rc = grouped_swiglu<W8>(r, hidden, phases, stream, who);
-        return rc != MOE_OK ? rc : grouped_swiglu<W8>(s, hidden, phases, stream, who);
+        rc = grouped_swiglu<W8>(r, hidden, phases, TailOf{}, stream, who);
+        return rc != MOE_OK ? rc : grouped_swiglu<W8>(s, hidden, phases, TailOf{}, stream, who);
     }
     hipStream_t st = as_stream(stream);
     GemmArgs gate_up = gate_up_args(s, hidden), down = down_args(s, hidden);
     if (W8) gate_up.alone = down.alone = joint_alone(s);
     if (phases & MOE_PHASE_GATE_UP)
-        rc = launch_joint<true, W8>(gate_up_args(r, hidden), r.n_rows, row_bound(r), gate_up, s.n_rows, st);
+        rc = launch_joint<true, W8>(gate_up_args(r, hidden), r.n_rows, row_bound(r), gate_up, s.n_rows, TailOf{}, st);
     if (rc == MOE_OK && (phases & MOE_PHASE_DOWN))
-        rc = launch_joint<false, W8>(down_args(r, hidden), r.n_rows, row_bound(r), down, s.n_rows, st);
+        rc = launch_joint<false, W8>(down_args(r, hidden), r.n_rows, row_bound(r), down, s.n_rows, tail, st);
     return rc;
 }
 
@@ -2691,7 +2819,27 @@ __global__ __launch_bounds__(256) void dequant_kernel(const uint8_t* __restrict_
     }
 }
 
+int swiglu_groups(const moe_mlp_group& routed, const moe_mlp_group* shared, int32_t hidden, int32_t fp8, int32_t phases, TailOf tail,
+                  void* stream) {
+    const char* who = "moe_grouped_swiglu_joint";
+    if (shared == nullptr)
+        return fp8 ? grouped_swiglu<true>(routed, hidden, phases, tail, stream, who) : grouped_swiglu<false>(routed, hidden, phases, tail, stream, who);
+    return fp8 ? grouped_swiglu_joint<true>(routed, *shared, hidden, phases, tail, stream, who)
+               : grouped_swiglu_joint<false>(routed, *shared, hidden, phases, tail, stream, who);
+}
+
 }  // namespace
+
+bool layer_may_combine(int32_t n_experts, int32_t n_rows, bool shared, int32_t hidden) {
+    return thin_down_narrow(thin_down_waves(n_experts, n_rows, shared, hidden));
+}
+
+int layer_experts(const moe_mlp_group& routed, const moe_mlp_group* shared, int32_t hidden, int32_t fp8, const CombineTail* tail,
+                  bool* combined, void* stream) {
+    *combined = false;
+    return swiglu_groups(routed, shared, hidden, fp8, MOE_PHASE_BOTH, TailOf{tail, combined}, stream);
+}
+
 }  // namespace moe
 
 extern "C" size_t moe_grouped_workspace_bytes(int32_t, int32_t) { return 256; }
@@ -2701,7 +2849,7 @@ extern "C" int moe_grouped_swiglu_bf16(const void* x, int32_t x_rows, const int3
                                        int32_t n_rows, int32_t n_experts, int32_t hidden, int32_t inter, void* act,
                                        void* y, int32_t phases, void*, size_t, void* stream) {
     const moe_mlp_group m{x, x_rows, n_rows, row_map, w_gate, w_up, w_down, nullptr, nullptr, nullptr, offsets, n_experts, inter, 0, 0, act, y, nullptr, 0};
-    return moe::grouped_swiglu<false>(m, hidden, phases, stream, "moe_grouped_swiglu_bf16");
+    return moe::grouped_swiglu<false>(m, hidden, phases, {}, stream, "moe_grouped_swiglu_bf16");
 }
 
 extern "C" int moe_grouped_swiglu_w8a16(const void* x, int32_t x_rows, const int32_t* row_map, const void* const* w_gate,
@@ -2711,18 +2859,14 @@ extern "C" int moe_grouped_swiglu_w8a16(const void* x, int32_t x_rows, const int
                                         int32_t n_experts, int32_t hidden, int32_t inter, void* act, void* y,
                                         int32_t phases, void*, size_t, void* stream) {
     const moe_mlp_group m{x, x_rows, n_rows, row_map, w_gate, w_up, w_down, s_gate, s_up, s_down, offsets, n_experts, inter, 0, 0, act, y, nullptr, 0};
-    return moe::grouped_swiglu<true>(m, hidden, phases, stream, "moe_grouped_swiglu_w8a16");
+    return moe::grouped_swiglu<true>(m, hidden, phases, {}, stream, "moe_grouped_swiglu_w8a16");
 }
 
 extern "C" int moe_grouped_swiglu_joint(const moe_mlp_group* routed, const moe_mlp_group* shared, int32_t hidden, int32_t fp8,
                                         int32_t phases, void* stream) {
     using namespace moe;
     MOE_REQUIRE(routed != nullptr, "moe_grouped_swiglu_joint: NULL group");
-    if (shared == nullptr)
-        return fp8 ? grouped_swiglu<true>(*routed, hidden, phases, stream, "moe_grouped_swiglu_joint")
-                   : grouped_swiglu<false>(*routed, hidden, phases, stream, "moe_grouped_swiglu_joint");
-    return fp8 ? grouped_swiglu_joint<true>(*routed, *shared, hidden, phases, stream)
-               : grouped_swiglu_joint<false>(*routed, *shared, hidden, phases, stream);
+    return swiglu_groups(*routed, shared, hidden, fp8, phases, {}, stream);
 }
 
 extern "C" size_t moe_mlp_workspace_bytes(const moe_mlp_group* m, int32_t hidden) {

@@ -3,13 +3,14 @@
 // 15 us of host time each, more than a decode-sized step runs on the GPU.
 #include "common.h"
 #include "dispatch_small.h"
+#include "layer.h"
 
 namespace moe {
 namespace {
 
 // byte offsets of the intermediate buffers in the workspace
 struct Layout {
-    size_t logits, x_norm, offsets, one_group, perm, pos, row_map, segments, act, y, act_shared, y_shared, total;
+    size_t logits, x_norm, offsets, one_group, perm, pos, row_map, segments, arrivals, act, y, act_shared, y_shared, total;
 };
 
 Layout layout_of(const moe_layer_args& a) {
@@ -30,6 +31,7 @@ Layout layout_of(const moe_layer_args& a) {
     l.pos = take(nk * 4);
     l.row_map = take(nk * 4);
     l.segments = take(moe_dispatch_workspace_bytes(p.n_tokens, p.top_k, p.n_experts));
+    l.arrivals = take(n <= kTailTokens ? tail_arrivals(p.hidden) * 4 : 0);
     l.act = take(nk * (size_t)a.routed->inter * 2);
     l.y = take(nk * h * 2);
     if (a.shared) {
@@ -87,15 +89,30 @@ extern "C" int moe_layer_forward(const moe_layer_args* args, void* stream) {
     }
     float* logits = reinterpret_cast<float*>(ws + l.logits);
     auto ints = [&](size_t off) { return reinterpret_cast<int32_t*>(ws + off); };
-    const DispatchOut d{a.counts, ints(l.offsets), ints(l.perm), ints(l.pos), ints(l.row_map), a.shared ? ints(l.one_group) : nullptr};
-    rc = router_logits(x, a.w_gate, p, logits, st);
-    if (rc != MOE_OK) return rc;
+    DispatchOut d{a.counts, ints(l.offsets), ints(l.perm), ints(l.pos), ints(l.row_map), a.shared ? ints(l.one_group) : nullptr};
+    // Of a few tokens the down projection may combine too (what a separate call would refuse is left to it)
+    const void* const y_shared = a.shared ? ws + l.y_shared : nullptr;
+    const CombineTail tail{d.pos, a.topk_idx, a.topk_w, static_cast<const uint16_t*>(a.norm_weight ? a.x : nullptr),
+                           static_cast<uint16_t*>(a.out), ints(l.arrivals), n, k, a.combine_mode};
+    const bool may_combine = n <= kTailTokens && n <= select_dispatch_tokens(E) && a.combine_mode >= MOE_COMBINE_F32 &&
+                             a.combine_mode <= MOE_COMBINE_BF16_SEQ && a.out != ws + l.y && a.out != y_shared &&
+                             layer_may_combine(E, n * k, a.shared != nullptr, h);
+    if (may_combine) {
+        d.arrivals = tail.arrivals;
+        d.n_arrivals = tail_arrivals(h);
+    }
+    bool combined = false;
     uint16_t* logits_bf16 = static_cast<uint16_t*>(a.logits_bf16);
-    if (n <= select_dispatch_tokens(E)) {
-        rc = router_select_dispatch(a.bias, p, a.topk_idx, a.topk_w, logits, logits_bf16, d, st);
+    if (n <= router_dispatch_tokens(E)) {
+        rc = router_dispatch(x, a.w_gate, a.bias, p, a.topk_idx, a.topk_w, logits_bf16, d, st);
     } else {
-        rc = router_select(a.bias, p, a.topk_idx, a.topk_w, logits, logits_bf16, st);
-        if (rc == MOE_OK) rc = dispatch_on_stream(a.topk_idx, n, k, E, d, ws + l.segments, st);
+        rc = router_logits(x, a.w_gate, p, logits, st);
+        if (rc == MOE_OK && n <= select_dispatch_tokens(E)) {
+            rc = router_select_dispatch(a.bias, p, a.topk_idx, a.topk_w, logits, logits_bf16, d, st);
+        } else if (rc == MOE_OK) {
+            rc = router_select(a.bias, p, a.topk_idx, a.topk_w, logits, logits_bf16, st);
+            if (rc == MOE_OK) rc = dispatch_on_stream(a.topk_idx, n, k, E, d, ws + l.segments, st);
+        }
     }
     if (rc != MOE_OK) return rc;
 
@@ -104,23 +121,21 @@ extern "C" int moe_layer_forward(const moe_layer_args* args, void* stream) {
     routed.max_rows = n;
     routed.act = ws + l.act; routed.y = ws + l.y;
     routed.workspace = nullptr; routed.workspace_bytes = 0;       // (the caller's fields may hold anything)
-    const void* y_shared = nullptr;
     if (a.shared) {
         moe_mlp_group shared = *a.shared;
         shared.x = x; shared.x_rows = shared.n_rows = shared.max_rows = n; shared.row_map = nullptr; shared.offsets = d.one_group;
         shared.act = ws + l.act_shared; shared.y = ws + l.y_shared;
         shared.workspace = nullptr; shared.workspace_bytes = 0;
-        y_shared = shared.y;
         if (a.join_shared && shared.fp8 == routed.fp8) {
-            rc = moe_grouped_swiglu_joint(&routed, &shared, h, routed.fp8, MOE_PHASE_BOTH, stream);
+            rc = layer_experts(routed, &shared, h, routed.fp8, may_combine ? &tail : nullptr, &combined, stream);
         } else {
             rc = moe_grouped_swiglu_joint(&routed, nullptr, h, routed.fp8, MOE_PHASE_BOTH, stream);
             if (rc == MOE_OK) rc = moe_grouped_swiglu_joint(&shared, nullptr, h, shared.fp8, MOE_PHASE_BOTH, stream);
         }
     } else {
-        rc = moe_grouped_swiglu_joint(&routed, nullptr, h, routed.fp8, MOE_PHASE_BOTH, stream);
+        rc = layer_experts(routed, nullptr, h, routed.fp8, may_combine ? &tail : nullptr, &combined, stream);
     }
-    if (rc != MOE_OK) return rc;
+    if (rc != MOE_OK || combined) return rc;
     if (a.norm_weight)
         return moe_combine_residual(ws + l.y, d.pos, a.topk_idx, a.topk_w, y_shared, a.x, n, k, h, a.combine_mode, a.out, stream);
     return moe_combine(ws + l.y, d.pos, a.topk_idx, a.topk_w, y_shared, n, k, h, a.combine_mode, a.out, stream);

@@ -223,6 +223,50 @@ def test_layer_call_equals_the_separate_calls(name, E):
 
 
 @pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("name,E,k,h", [("deepseek_v2_lite", 64, 6, 1024), ("deepseek_v2_lite", 17, 3, 576), ("deepseek_v3_w8a16", 256, 8, 384),
+                                        ("mixtral_8x7b", 8, 2, 512), ("mixtral_8x7b", 8, 8, 256), ("deepseek_v2_lite", 33, 16, 256),
+                                        ("mixtral_8x22b", 32, 16, 192)])
+def test_few_tokens_in_fewer_launches(name, E, k, h, fp8):
+    """Calls whose router also sorts, whose down projection has 16 columns a wave and also combines (a counter per column
+    tile, set anew by every call), and their neighbours in tokens and columns, h no multiple of 128 and E no power of two
+    among them: bit for bit the stage-by-stage path; again on the same buffers, and replayed from a graph."""
+    from moe_gen_amd import norm_moe_residual, synthetic
+    from moe_gen_amd.block import StageTimer
+    group = dict(n_group=1, topk_group=1) if name == "deepseek_v2_lite" else dict(n_group=4, topk_group=2) if name == "deepseek_v3_w8a16" else {}
+    w = synthetic.WORKLOADS[name].scaled(n=17, h=h, I=256, seq=17, E=E, k=k, fp8=fp8, **group)
+    if fp8 and h % 128:
+        pytest.skip("fp8 weights come in blocks of 128")
+    blk = synthetic.build_block(w, device="cuda", gen_device="cpu")
+    xs = synthetic.hidden_states(w, "cpu").cuda()
+    nw = (1 + 0.1 * torch.randn(h, generator=torch.Generator().manual_seed(1))).to(torch.bfloat16).cuda()
+    for n in (1, 2, 4, 5, 8, 9, 16, 17):
+        x = xs[:, :n].contiguous()
+        for norm in (False, True):
+            print(f"few tokens {name} E={E} k={k} h={h} fp8={fp8} n={n} norm={norm}", flush=True)
+            def run():
+                res = norm_moe_residual(blk, x, nw) if norm else blk(x)
+                res = res if isinstance(res, tuple) else (res,)
+                return [*res, blk.last_topk_idx, blk.last_topk_weight, blk.last_counts]
+            blk.stage_timer = StageTimer()
+            want = [t.clone() for t in run()]
+            blk.stage_timer = None
+            for _ in range(3):
+                for a, b in zip(run(), want):
+                    assert a.dtype == b.dtype and torch.equal(a, b), (n, norm)
+            if n != 1:
+                continue
+            torch.cuda.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph):
+                got = run()
+            for _ in range(3):
+                graph.replay()
+                torch.cuda.synchronize()
+                for a, b in zip(got, want):
+                    assert torch.equal(a, b), norm
+
+
+@pytest.mark.parametrize("fp8", [False, True])
 def test_dense_mlp_sees_replaced_weights_and_a_copied_block_its_own(fp8):
     """A dense MLP whose up projection (fp8: or its block scales) is replaced between two calls computes with the new one,
     and a deep copy of a block that has run gives the block's results after the block's weights are gone."""
