@@ -3,6 +3,7 @@
 // selection kernel for few tokens, which runs it on the indices it has just chosen.
 #pragma once
 #include "common.h"
+#include "layer.h"
 
 namespace moe {
 
@@ -102,8 +103,9 @@ __device__ __forceinline__ void dispatch_one_workgroup(int nk, int E, const Disp
 }
 
 // ---- launches behind the layer call (each checks its arguments as the entry point of the same name does) ----
-// logits into memory
-int router_logits(const void* x, const void* w_gate, const moe_router_params& p, float* logits, hipStream_t st);
+// logits into memory; shared: also its gate and up projection, may be NULL (for kRouterSharedE < E and up to kTailTokens tokens)
+constexpr int kRouterSharedE = 32;
+int router_logits(const void* x, const void* w_gate, const moe_router_params& p, float* logits, const SharedFirst* shared, hipStream_t st);
 // routes from them; logits_bf16: also written as bf16 (Mixtral's second result), may be NULL
 int router_select(const float* bias, const moe_router_params& p, int32_t* topk_idx, float* topk_w, float* logits,
                   uint16_t* logits_bf16, hipStream_t st);
@@ -112,9 +114,9 @@ int router_select(const float* bias, const moe_router_params& p, int32_t* topk_i
 // launches 10.)
 constexpr int select_dispatch_tokens(int E) { return SMALL_WAVES * (E <= 16 ? 4 : E <= 32 ? 2 : 1); }
 constexpr int kSelectDispatchTokens = 64;
-// logits, routing and dispatch in one launch of one workgroup, where that has every expert in one block and its 4 waves
-// route the tokens in one pass
-constexpr int router_dispatch_tokens(int E) { return E <= 16 ? 16 : E <= 32 ? 8 : E <= 64 ? 4 : 0; }
+// logits, routing and dispatch in one launch of one workgroup, where its 4 waves route the tokens in one pass (with 64 experts one
+// CU fetches the gate no sooner than two launches are done: DeepSeek-V2-Lite, 1 token, 9.7 + 4.4 us and 14.3)
+constexpr int router_dispatch_tokens(int E) { return E <= 16 ? 16 : E <= 32 ? 8 : 0; }
 int router_dispatch(const void* x, const void* w_gate, const float* bias, const moe_router_params& p, int32_t* topk_idx, float* topk_w,
                     uint16_t* logits_bf16, const DispatchOut& out, hipStream_t st);
 int router_select_dispatch(const float* bias, const moe_router_params& p, int32_t* topk_idx, float* topk_w, float* logits,

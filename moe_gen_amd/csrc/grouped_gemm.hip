@@ -53,6 +53,7 @@
 #include "combine_math.h"
 #include "common.h"
 #include "layer.h"
+#include "thin_gemm.h"
 
 namespace moe {
 namespace {
@@ -62,8 +63,6 @@ constexpr int ROW_B = 128;       // bytes per LDS row
 constexpr int BN_ROWS = 256;     // weight rows per workgroup (128 gate + 128 up when SWIGLU)
 constexpr int MAX_E = 1024;
 constexpr int PAIR_LO = 257, PAIR_HI = 384;   // bf16: rows of an expert that runs as two tiles of the 192-row body
-
-__device__ __forceinline__ float bf16r(float a) { return __uint_as_float(pack_bf16(a, 0.0f) << 16); }
 
 // 16 fp8 bytes -> 16 bf16 (two 16-byte chunks): bf16(f32(q) * s)
 __device__ __forceinline__ void dequant16(u32x4 q, float s, u32x4& lo, u32x4& hi) {
@@ -115,12 +114,6 @@ struct GemmPair {
     int shared_tiles, shared_rows;
 };
 
-// LDS rows are 128 bytes = 8 chunks of 16 bytes; chunk c of row r is stored at chunk c ^ swz(r).
-// swz makes any 8 consecutive rows hit 8 different chunks (32 banks x 4 B = one 128-byte row per
-// cycle) AND any 16 consecutive rows hit 16 different (row parity, chunk) slots (64 banks =
-// two rows per cycle), so 16-byte operand reads by 32 consecutive rows never collide.
-__device__ __forceinline__ int swz(int row) { return (row & 7) ^ ((row >> 3) & 1); }
-
 // Stage at which a tile of N tile n_tile starts its walk over k.  Workgroups that run side by side mostly differ in
 // their N tile; started at the same stage, their requests in flight would share the low address bits (rows of the weight
 // matrices are K elements apart) and crowd the same memory channels: with the start spread over the stages a launch
@@ -134,14 +127,6 @@ __device__ __forceinline__ int swz(int row) { return (row & 7) ^ ((row >> 3) & 1
 template <bool W8>
 __device__ __forceinline__ int k_rotation(int n_tile, int nk) { return (W8 ? 2 * n_tile : n_tile) % nk; }
 
-// global-address-space views: expert pointers come out of a pointer table in memory, and
-// without the address space the compiler must emit flat loads, whose completion is tracked
-// by the same counter as the LDS reads of the MFMA operands
-typedef const __attribute__((address_space(1))) u32x4* gptr_u32x4;
-typedef const __attribute__((address_space(1))) float* gptr_f32;
-typedef const __attribute__((address_space(1))) int32_t* gptr_i32;
-typedef __attribute__((address_space(3))) uint8_t* lds_u8;
-
 __device__ __forceinline__ u32x4 gload16(const void* p) { return *(gptr_u32x4)(uintptr_t)p; }
 // Weights under the one-workgroup-per-tile kernel are streamed: a tile of them is used by one workgroup (two
 // or more for an expert above 256 rows) and never again in the launch, so those loads are non-temporal
@@ -150,12 +135,6 @@ __device__ __forceinline__ u32x4 gload16(const void* p) { return *(gptr_u32x4)(u
 template <bool STREAM>
 __device__ __forceinline__ u32x4 gload16_w(const void* p) {
     return STREAM ? __builtin_nontemporal_load((gptr_u32x4)(uintptr_t)p) : *(gptr_u32x4)(uintptr_t)p;
-}
-__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
-__device__ __forceinline__ const uint8_t* uni_ptr(const void* p) {
-    uint64_t u = (uint64_t)(uintptr_t)p;
-    uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)u), hi = __builtin_amdgcn_readfirstlane((uint32_t)(u >> 32));
-    return reinterpret_cast<const uint8_t*>((uintptr_t)(((uint64_t)hi << 32) | lo));
 }
 
 
@@ -182,33 +161,6 @@ __device__ __forceinline__ void tile_in_expert(int local, int mt_e, int n_tiles_
     }
     n_tile = rem / gm;
     m_tile = m0 + (rem - n_tile * gm);
-}
-
-// 8 fp8 weights (two dwords) -> 8 bf16: bf16(f32(q) * s), the reference's dequantisation
-__device__ __forceinline__ u32x4 dequant8(uint32_t q0, uint32_t q1, float sc) {
-    const f32x2 c0 = __builtin_amdgcn_cvt_pk_f32_fp8(q0, false), c1 = __builtin_amdgcn_cvt_pk_f32_fp8(q0, true);
-    const f32x2 c2 = __builtin_amdgcn_cvt_pk_f32_fp8(q1, false), c3 = __builtin_amdgcn_cvt_pk_f32_fp8(q1, true);
-    return u32x4{pack_bf16(c0[0] * sc, c0[1] * sc), pack_bf16(c1[0] * sc, c1[1] * sc),
-                 pack_bf16(c2[0] * sc, c2[1] * sc), pack_bf16(c3[0] * sc, c3[1] * sc)};
-}
-
-// Epilogue values of one lane for one pair of accumulators: 4 consecutive output columns of one row.
-// SWIGLU: act = bf16(bf16(silu(bf16(g))) * bf16(u)), the rounding points of the reference's bf16
-// Linear / SiLU / mul modules (silu through the hardware exp and reciprocal); else bf16(acc).
-template <bool SWIGLU>
-__device__ __forceinline__ u32x2 epilogue_pack(const f32x4& a, const f32x4& up) {
-    if (SWIGLU) {
-        float o[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float gv = bf16r(a[i]);
-            const float uv = bf16r(up[i]);
-            const float sg = bf16r(gv * __builtin_amdgcn_rcpf(1.0f + __expf(-gv)));
-            o[i] = sg * uv;
-        }
-        return u32x2{pack_bf16(o[0], o[1]), pack_bf16(o[2], o[3])};
-    }
-    return u32x2{pack_bf16(a[0], a[1]), pack_bf16(a[2], a[3])};
 }
 
 // A lane's 4 columns (8 bytes) of two neighbouring 16-column fragments of one row -> 16 consecutive bytes of that row: lane
@@ -691,9 +643,6 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, Stage st0, Stage st
 //  rows, lane groups q and q + 2, whose chunks f(q) and f(q + 2) = f(q) + 1 are neighbours): with these keys their 16
 //  reads fall on 16 different bank groups.  (Measured with 8 waves reading back to back: 32 cycles per wave and
 //  ds_read_b128 for both layouts, 55 with lane group q on chunk q.)
-__device__ __forceinline__ int wsw(int r) { return ((r >> 1) & 1) | (((r >> 2) & 1) << 2); }
-__device__ __forceinline__ int tsw(int r) { return (r & 3) | ((r & 4) << 1); }
-
 constexpr int S8_WBYTES = 32 * 1024;              // weight region of a buffer: 8 waves x 32 rows x 128 fp8
 constexpr int S8_TROWS = 64;                      // token rows staged
 
@@ -1630,9 +1579,6 @@ __global__ __launch_bounds__(128 * WN) void grouped_gemm_kernel(GemmPair pair_of
 // shared expert); the dispatch of the call sets them.  The wave that brings a counter to zero finds every expert's columns
 // written and adds them up: no wave waits for another.  What waves on other XCDs read leaves and arrives past the L2 of an XCD
 // (relaxed atomics at agent scope), a wave's stores being complete before it counts itself.
-__device__ __forceinline__ void store_shared_8(uint16_t* p, const u32x2& v) {
-    __hip_atomic_store(reinterpret_cast<uint64_t*>(p), __builtin_bit_cast(uint64_t, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 __device__ __forceinline__ u32x4 load_shared_16(const uint16_t* p) {
     const uint64_t* q = reinterpret_cast<const uint64_t*>(p);
     const u32x2 a = __builtin_bit_cast(u32x2, __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
@@ -1706,30 +1652,26 @@ __device__ __forceinline__ void combine_columns(const CombineTail& tail, const T
 //
 // Such a call touches a few experts, and cut into tiles of 256 weight rows it has fewer tiles than the chip has CUs
 // (one token of DeepSeek-V2-Lite: 66) or two and a half rounds of them.  Here the unit is a WAVE with 32 weight rows --
-// 16 gate rows and the matching up rows, or 32 down rows (16 where that leaves most of the chip idle, thin_down_narrow) -- and the whole K, each wave a workgroup of its own: no
-// barrier, six of them per CU, and nothing to wait for but its own DMA.  A stage is 128 bytes of each weight row (64 k of
-// bf16, 128 of fp8: whole lines) and the same k of 16 token rows (rows that do not exist cost no request), NB stages in
-// a ring.  Every matrix instruction gets the k values that the streamers above give it, in the same lanes and the same
-// order, so a row's bits are those of a larger call (fp8: of a larger call whose experts have up to 64 rows).
+// 16 gate rows and the matching up rows, or 32 down rows (16 where that leaves most of the chip idle, thin_down_narrow) -- and
+// the whole K, each wave a workgroup of its own: no barrier, six of them per CU, and nothing to wait for but its own DMA.  A
+// stage is 128 bytes of each weight row (64 k of bf16, 128 of fp8: whole lines) and the same k of 16 token rows (rows that do not
+// exist cost no request), NB stages in a ring.  Every matrix instruction gets the k values that the streamers above give it, in
+// the same lanes and the same order, so a row's bits are those of a larger call (fp8: of a larger call whose experts have up
+// to 64 rows).  The body is thin_columns (thin_gemm.h).
 // Measured (us, tile kernel -> this): DeepSeek-V2-Lite, one token (8 x 1408 of 2048) 25 + 25 and 19 + 33 -> 17 and 14;
 // DeepSeek-V3, 5 tokens (39 experts, fp8) 190 and 115 -> 187 and 92 = 6.0 TB/s.  Weights loaded into registers instead
 // reach 4 ... 5 TB/s: a fragment load then takes half a line from each of 16 rows.
 template <bool SWIGLU, bool W8, int NF, bool TAIL>
 __global__ __launch_bounds__(64) void grouped_gemm_thin_kernel(GemmPair pair_of, CombineTail tail) {
-    static_assert(!SWIGLU || NF == 2, "gate and up: a fragment of either");
     static_assert(!TAIL || NF == 1, "the combine's rule");
-    constexpr int WBYTES = NF * 2048, TBYTES = W8 ? 4096 : 2048;       // weights and 16 token rows of a stage
-    constexpr int NDW = 2 * NF, NDT = TBYTES / 1024, NI = NDW + NDT;   // DMA instructions per stage
     constexpr int NCOL = SWIGLU ? 16 : 16 * NF;   // output columns of a wave
-    constexpr int SB = WBYTES + TBYTES;
-    constexpr int NB = 24576 / SB;                // stages in LDS
-    static_assert(NB >= 3 && (NB - 1) * NI < 64, "stages");
-    __shared__ __attribute__((aligned(1024))) uint8_t lds[NB * SB];
+    constexpr int NB = 24576 / thin_stage_bytes<W8, NF>;               // stages in LDS
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[NB * thin_stage_bytes<W8, NF>];
     const int lane = threadIdx.x;
     const bool of_shared = (int)blockIdx.x < pair_of.shared_tiles;
     const GemmArgs& g = pair_of.p[of_shared ? 1 : 0];
     const int unit = (int)blockIdx.x - (of_shared ? 0 : pair_of.shared_tiles);
-    const int K = g.K, N = g.N;
+    const int N = g.N;
     const int tiles = (N + NCOL - 1) / NCOL;
 
     // the (unit / tiles)-th expert that has rows: 256 experts at a time, 4 per lane
@@ -1767,122 +1709,8 @@ __global__ __launch_bounds__(64) void grouped_gemm_thin_kernel(GemmPair pair_of,
     if (e < 0) return;
     [[maybe_unused]] const auto slots = [&] { if constexpr (TAIL) return TailSlots(tail); else return 0; }();
     const int n0 = (unit % tiles) * NCOL;
-    const int nk = K / (W8 ? 128 : 64);
-    const int rot = (n0 / (SWIGLU ? 128 : 256)) % nk;      // the k rotation of the N tile these columns belong to
-    auto stage_at = [&](int k) { const int s = min(k, nk - 1) + rot; return s >= nk ? s - nk : s; };
-
-    const uint8_t* bm0 = uni_ptr(g.b0[e]);
-    const uint8_t* bm1 = SWIGLU ? uni_ptr(g.b1[e]) : bm0;
-    gptr_f32 sc0 = nullptr, sc1 = nullptr;                 // scales of the 128 rows the wave's columns lie in
-    if (W8) {
-        sc0 = (gptr_f32)(uintptr_t)uni_ptr(g.s0[e]) + (n0 >> 7) * nk;
-        sc1 = SWIGLU ? (gptr_f32)(uintptr_t)uni_ptr(g.s1[e]) + (n0 >> 7) * nk : sc0;
-    }
-    // DMA: weights, instruction i: fragment i / 2 (gate / up, or the two halves of the 32 down rows), rows 8 (i & 1) +
-    // lane / 8; tokens, instruction i: 8 (fp8: 4) rows; chunks swizzled as in the streamers
-    const int lr = lane >> 3, pp = lane & 7;
-    const uint32_t row_bytes = (uint32_t)K * (W8 ? 1 : 2);
-    uint32_t w_voff[4], t_voff[4];                         // (NDW and NDT are used)
-#pragma unroll
-    for (int i = 0; i < NDW; ++i) {
-        const int fr = 8 * (i & 1) + lr;
-        w_voff[i] = (uint32_t)min(n0 + (SWIGLU ? 0 : 16 * (i >> 1)) + fr, N - 1) * row_bytes + (uint32_t)((pp ^ (W8 ? wsw(fr) : swz(fr))) << 4);
-    }
-    const int frow = lane & 15, q = lane >> 4;
-    const int fq = ((q & 1) << 1) | (q >> 1);
-    const uint32_t w_rd = (uint32_t)(frow * 128), wkey = (uint32_t)(W8 ? wsw(frow) : swz(frow));
-    const uint32_t t_rd = (uint32_t)WBYTES + (uint32_t)(frow * (W8 ? 256 : 128)), tkey = (uint32_t)(W8 ? tsw(frow) : swz(frow));
-
-    for (int r0 = row0; r0 < row_end; r0 += 16) {          // (more than once only if a caller's row bound was wrong)
-        const uint8_t* a_base = reinterpret_cast<const uint8_t*>(g.a) + (g.row_map ? (size_t)0 : (size_t)r0 * K * 2);
-        const int a_records = g.row_map ? (int)(uint32_t)g.a_bytes : min(16, row_end - r0) * K * 2;
-#pragma unroll
-        for (int i = 0; i < NDT; ++i) {
-            const int tr = W8 ? 4 * i + (lane >> 4) : 8 * i + lr;
-            const int r = min(r0 + tr, row_end - 1);
-            const int src = g.row_map ? ((gptr_i32)(uintptr_t)g.row_map)[r] : r - r0;
-            t_voff[i] = (uint32_t)src * (uint32_t)(K * 2) + (uint32_t)((W8 ? (lane & 15) ^ tsw(tr) : pp ^ swz(tr)) << 4);
-            if (r0 + tr >= row_end || (g.row_map && (unsigned)src >= (unsigned)g.a_rows)) t_voff[i] = 0xfffffff0u;
-        }
-        auto dma = [&](int k, int buf) __attribute__((always_inline)) {
-            const int live = uni(k < nk ? -1 : 0);         // past the end: empty descriptors, the instructions still count
-            uint8_t* d = lds + buf * SB;
-            const uint32_t so = (uint32_t)stage_at(k) * 128u;
-            const __amdgpu_buffer_rsrc_t r0d = __builtin_amdgcn_make_buffer_rsrc((void*)bm0, 0, live, 0x00020000);
-            const __amdgpu_buffer_rsrc_t r1d = __builtin_amdgcn_make_buffer_rsrc((void*)bm1, 0, live, 0x00020000);
-            const __amdgpu_buffer_rsrc_t rad = __builtin_amdgcn_make_buffer_rsrc((void*)a_base, 0, live & a_records, 0x00020000);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(r0d, (lds_u8)d, 16, w_voff[0], so, 0, 2);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(r0d, (lds_u8)(d + 1024), 16, w_voff[1], so, 0, 2);
-            if constexpr (NF == 2) {
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(r1d, (lds_u8)(d + 2048), 16, w_voff[2], so, 0, 2);
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(r1d, (lds_u8)(d + 3072), 16, w_voff[3], so, 0, 2);
-            }
-#pragma unroll
-            for (int i = 0; i < NDT; ++i)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(rad, (lds_u8)(d + WBYTES + i * 1024), 16, t_voff[i], W8 ? 2 * so : so, 0, 0);
-        };
-        f32x4 acc[NF];
-#pragma unroll
-        for (int j = 0; j < NF; ++j) acc[j] = f32x4{0};
-        float v0 = 0.0f, v1 = 0.0f;                        // fp8: lane l holds the scales of stage 64 i + l
-        if (W8) { v0 = sc0[stage_at(lane)]; v1 = sc1[stage_at(lane)]; }
-        for (int i = 0; i < NB - 1; ++i) dma(i, i);
-        // (waits by hand: the compiler's own, in front of the readlane below, would cover the DMA of the next stage too.  The
-        // scales were requested before the DMA; where the compiler moves them behind some of it, it waits for them here itself)
-        if (W8) asm volatile("s_waitcnt vmcnt(%2)" : "+v"(v0), "+v"(v1) : "n"((NB - 1) * NI));
-        int buf = 0;
-        for (int k = 0; k < nk; ++k) {
-            // this wave's DMA of stage k has landed and its reads of stage k - 1, whose buffer is refilled, have returned
-            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"((NB - 2) * NI) : "memory");
-            if (W8 && (k & 63) == 0 && k > 0) {
-                v0 = sc0[stage_at(k + lane)];
-                v1 = sc1[stage_at(k + lane)];
-                asm volatile("s_waitcnt vmcnt(0)" : "+v"(v0), "+v"(v1));
-            }
-            dma(k + NB - 1, buf == 0 ? NB - 1 : buf - 1);
-            const uint8_t* b = lds + buf * SB;
-            if (W8) {
-                const float c[2] = {__builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v0), k & 63)),
-                                    __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v1), k & 63))};
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    u32x4 raw[NF];
-#pragma unroll
-                    for (int j = 0; j < NF; ++j) raw[j] = *reinterpret_cast<const u32x4*>(b + j * 2048 + w_rd + (((4 * h + fq) ^ wkey) << 4));
-#pragma unroll
-                    for (int s2 = 0; s2 < 2; ++s2) {
-                        const bf16x8 tf = *reinterpret_cast<const bf16x8*>(b + t_rd + (((8 * h + 2 * fq + s2) ^ tkey) << 4));
-#pragma unroll
-                        for (int j = 0; j < NF; ++j)
-                            acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                                __builtin_bit_cast(bf16x8, dequant8(raw[j][2 * s2], raw[j][2 * s2 + 1], c[j])), tf, acc[j], 0, 0, 0);
-                    }
-                }
-            } else {
-#pragma unroll
-                for (int s = 0; s < 2; ++s) {
-                    const uint32_t coff = (uint32_t)((4 * s + fq) ^ wkey) << 4;      // (wkey == tkey)
-                    const bf16x8 tf = *reinterpret_cast<const bf16x8*>(b + t_rd + coff);
-#pragma unroll
-                    for (int j = 0; j < NF; ++j)
-                        acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(b + j * 2048 + w_rd + coff), tf, acc[j], 0, 0, 0);
-                }
-            }
-            buf = buf + 1 == NB ? 0 : buf + 1;
-        }
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");   // no DMA may land in LDS after the workgroup has gone
-        const int r = r0 + frow;
-        if (r < row_end) {
-#pragma unroll
-            for (int j = 0; j < (SWIGLU ? 1 : NF); ++j) {
-                const int col = n0 + 16 * j + 4 * q;
-                if (col >= N) continue;
-                const u32x2 o = epilogue_pack<SWIGLU>(acc[j], acc[SWIGLU ? 1 : j]);
-                if constexpr (TAIL) store_shared_8(g.c + (size_t)r * N + col, o);
-                else *reinterpret_cast<u32x2*>(g.c + (size_t)r * N + col) = o;
-            }
-        }
-    }
+    thin_columns<SWIGLU, W8, NF, TAIL, NB>(ThinUnit{g.b0[e], SWIGLU ? g.b1[e] : nullptr, W8 ? g.s0[e] : nullptr, W8 && SWIGLU ? g.s1[e] : nullptr, g.a,
+                                                    g.row_map, g.a_bytes, g.a_rows, g.c, g.K, N, row0, row_end}, n0, lds);
     if constexpr (TAIL) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's columns are where every XCD finds them
         int left_out = 0;
@@ -2449,24 +2277,17 @@ inline int cu_count() {
     return cached[dev];
 }
 
-// The combine that the down projection of a layer call may take over: `done` then says so
-struct TailOf {
-    const CombineTail* args = nullptr;
-    bool* done = nullptr;
-};
-
 // waves of 32 columns that the thin kernel's down projection has at most
 inline long thin_down_waves(int E, int n_rows, bool shared, int N) { return ((E < n_rows ? E : n_rows) + (shared ? 1L : 0L)) * ((N + 31) / 32); }
 // Up to two waves per CU: 16 columns each instead of 32, so that twice as many stages are on their way, and the waves combine
 // too, which saves a launch where the host takes as long as the GPU.  Down projection and combine, us, in two launches -> this
-// (16 columns): DeepSeek-V2-Lite, 1 token (448 waves) 13.5 + 4.7 -> 16.3, the call, with the router's launches joined, 52.1 -> 47.3 on
-// weights that are in the caches and 51.1 -> 49.3 on others;
-// Mixtral-8x7B, 1 token (256) 56.1 + 5.7 -> 45.1, the call 161 -> 144.  Beyond, nothing is gained: DeepSeek-V2-Lite, 3 tokens (1216) 17.0 + 5.0 -> 22.8 with
-// 32 columns, Mixtral-8x22B, 2 tokens (768), the call 405 -> 408.
+// (16 columns): DeepSeek-V2-Lite, 1 token (448 waves) 13.5 + 4.7 -> 16.3; Mixtral-8x7B, 1 token (256) 56.1 + 5.7 -> 45.1, the call 161 ->
+// 144.  Beyond, nothing is gained: DeepSeek-V2-Lite, 3 tokens (1216) 17.0 + 5.0 -> 22.8 with 32 columns, Mixtral-8x22B, 2 tokens (768),
+// the call 405 -> 408.
 inline bool thin_down_narrow(long waves) { return waves <= 2L * cu_count(); }
 
 template <bool SWIGLU, bool W8>
-int launch_thin(const GemmArgs& g, int n_rows, const GemmArgs* shared, TailOf tail, hipStream_t st) {
+int launch_thin(const GemmArgs& g, int n_rows, const GemmArgs* shared, LayerCall* call, hipStream_t st) {
     GemmPair pair{};
     pair.p[0] = g;
     if (shared) pair.p[1] = *shared;
@@ -2487,9 +2308,9 @@ int launch_thin(const GemmArgs& g, int n_rows, const GemmArgs* shared, TailOf ta
     } else {
         const long waves = thin_down_waves(g.E, n_rows, shared != nullptr, g.N);
         if (!thin_down_narrow(waves)) return launch(grouped_gemm_thin_kernel<false, W8, 2, false>, 32, CombineTail{});
-        if (!tail.args) return launch(grouped_gemm_thin_kernel<false, W8, 1, false>, 16, CombineTail{});
-        *tail.done = true;
-        return launch(grouped_gemm_thin_kernel<false, W8, 1, true>, 16, *tail.args);
+        if (!call || !call->tail) return launch(grouped_gemm_thin_kernel<false, W8, 1, false>, 16, CombineTail{});
+        call->combined = true;
+        return launch(grouped_gemm_thin_kernel<false, W8, 1, true>, 16, *call->tail);
     }
 }
 
@@ -2615,7 +2436,7 @@ int launch_both(const GemmPair& pair, int n_rows, hipStream_t st) {
 
 // max_rows: no expert has more rows (callers that do not know pass n_rows)
 template <bool SWIGLU, bool W8>
-int launch_mt(const GemmArgs& g0, int n_rows, int max_rows, void* workspace, size_t workspace_bytes, TailOf tail, hipStream_t st) {
+int launch_mt(const GemmArgs& g0, int n_rows, int max_rows, void* workspace, size_t workspace_bytes, LayerCall* call, hipStream_t st) {
     GemmArgs g = g0;
     const long mean = g.E > 0 ? (long)n_rows / g.E : 0;
     if constexpr (W8 && !SWIGLU) {
@@ -2623,7 +2444,7 @@ int launch_mt(const GemmArgs& g0, int n_rows, int max_rows, void* workspace, siz
         if (plan.slices > 1 && workspace_bytes >= (size_t)plan.slices * n_rows * g.N * 4)
             return launch_split(g, n_rows, plan, static_cast<float*>(workspace), st);
     }
-    if (max_rows <= 16 && gather_fits(g) && thin_pays(g, n_rows, nullptr)) return launch_thin<SWIGLU, W8>(g, n_rows, nullptr, tail, st);
+    if (max_rows <= 16 && gather_fits(g) && thin_pays(g, n_rows, nullptr)) return launch_thin<SWIGLU, W8>(g, n_rows, nullptr, call, st);
     GemmPair pair{};
     if (mean < 128 || !persistent_fits(g)) {
         g.cold_max = 0x7fffffff;
@@ -2669,10 +2490,15 @@ int launch_mt(const GemmArgs& g0, int n_rows, int max_rows, void* workspace, siz
     return launch_both<SWIGLU, W8>(pair, n_rows, st);
 }
 
+inline bool joint_thin(const GemmArgs& routed, int n_rows, int max_rows, const GemmArgs& shared, int n_shared) {
+    return max_rows <= 16 && n_shared <= 16 && thin_pays(routed, n_rows, &shared);
+}
+
 // The shared expert's tiles in the routed experts' launches.  shared.alone: see joint_alone.
 template <bool SWIGLU, bool W8>
-int launch_joint(const GemmArgs& routed, int n_rows, int max_rows, const GemmArgs& shared, int n_shared, TailOf tail, hipStream_t st) {
-    if (max_rows <= 16 && n_shared <= 16 && thin_pays(routed, n_rows, &shared)) return launch_thin<SWIGLU, W8>(routed, n_rows, &shared, tail, st);
+int launch_joint(const GemmArgs& routed, int n_rows, int max_rows, const GemmArgs& shared, int n_shared, LayerCall* call, hipStream_t st) {
+    if (joint_thin(routed, n_rows, max_rows, shared, n_shared))
+        return launch_thin<SWIGLU, W8>(routed, n_rows, SWIGLU && call && call->shared_gate_up_done ? nullptr : &shared, call, st);
     GemmPair pair{{routed, shared}, 0, 0};
     if (n_rows / routed.E < 128) {
         pair.p[0].cold_max = pair.p[1].cold_max = 0x7fffffff;
@@ -2765,34 +2591,34 @@ bool joins(const moe_mlp_group& routed, const moe_mlp_group& shared, int32_t hid
 int joint_alone(const moe_mlp_group& shared) { return shared.n_rows < 128 || few_tiles(shared, cu_count()); }
 
 template <bool W8>
-int grouped_swiglu(const moe_mlp_group& m, int32_t hidden, int32_t phases, TailOf tail, void* stream, const char* who) {
+int grouped_swiglu(const moe_mlp_group& m, int32_t hidden, int32_t phases, LayerCall* call, void* stream, const char* who) {
     MOE_REQUIRE(phases >= MOE_PHASE_GATE_UP && phases <= MOE_PHASE_BOTH, "%s: bad phases %d", who, phases);
     int rc = check_group(m, hidden, W8, who);
     if (rc != MOE_OK || m.n_rows == 0) return rc;
     hipStream_t st = as_stream(stream);
-    if (phases & MOE_PHASE_GATE_UP) rc = launch_mt<true, W8>(gate_up_args(m, hidden), m.n_rows, row_bound(m), nullptr, 0, TailOf{}, st);
+    if (phases & MOE_PHASE_GATE_UP) rc = launch_mt<true, W8>(gate_up_args(m, hidden), m.n_rows, row_bound(m), nullptr, 0, nullptr, st);
     if (rc == MOE_OK && (phases & MOE_PHASE_DOWN)) 
-        rc = launch_mt<false, W8>(down_args(m, hidden), m.n_rows, row_bound(m), m.workspace, m.workspace_bytes, tail, st);
+        rc = launch_mt<false, W8>(down_args(m, hidden), m.n_rows, row_bound(m), m.workspace, m.workspace_bytes, call, st);
     return rc;
 }
 
 template <bool W8>
-int grouped_swiglu_joint(const moe_mlp_group& r, const moe_mlp_group& s, int32_t hidden, int32_t phases, TailOf tail, void* stream, const char* who) {
+int grouped_swiglu_joint(const moe_mlp_group& r, const moe_mlp_group& s, int32_t hidden, int32_t phases, LayerCall* call, void* stream, const char* who) {
     MOE_REQUIRE(phases >= MOE_PHASE_GATE_UP && phases <= MOE_PHASE_BOTH, "%s: bad phases %d", who, phases);
     int rc = check_group(r, hidden, W8, who);
     if (rc == MOE_OK) rc = check_group(s, hidden, W8, who);
     if (rc != MOE_OK) return rc;
     if (!joins(r, s, hidden)) {
-        rc = grouped_swiglu<W8>(r, hidden, phases, TailOf{}, stream, who);
-        return rc != MOE_OK ? rc : grouped_swiglu<W8>(s, hidden, phases, TailOf{}, stream, who);
+        rc = grouped_swiglu<W8>(r, hidden, phases, nullptr, stream, who);
+        return rc != MOE_OK ? rc : grouped_swiglu<W8>(s, hidden, phases, nullptr, stream, who);
     }
     hipStream_t st = as_stream(stream);
     GemmArgs gate_up = gate_up_args(s, hidden), down = down_args(s, hidden);
     if (W8) gate_up.alone = down.alone = joint_alone(s);
     if (phases & MOE_PHASE_GATE_UP)
-        rc = launch_joint<true, W8>(gate_up_args(r, hidden), r.n_rows, row_bound(r), gate_up, s.n_rows, TailOf{}, st);
+        rc = launch_joint<true, W8>(gate_up_args(r, hidden), r.n_rows, row_bound(r), gate_up, s.n_rows, call, st);
     if (rc == MOE_OK && (phases & MOE_PHASE_DOWN))
-        rc = launch_joint<false, W8>(down_args(r, hidden), r.n_rows, row_bound(r), down, s.n_rows, tail, st);
+        rc = launch_joint<false, W8>(down_args(r, hidden), r.n_rows, row_bound(r), down, s.n_rows, call, st);
     return rc;
 }
 
@@ -2819,13 +2645,13 @@ __global__ __launch_bounds__(256) void dequant_kernel(const uint8_t* __restrict_
     }
 }
 
-int swiglu_groups(const moe_mlp_group& routed, const moe_mlp_group* shared, int32_t hidden, int32_t fp8, int32_t phases, TailOf tail,
+int swiglu_groups(const moe_mlp_group& routed, const moe_mlp_group* shared, int32_t hidden, int32_t fp8, int32_t phases, LayerCall* call,
                   void* stream) {
     const char* who = "moe_grouped_swiglu_joint";
     if (shared == nullptr)
-        return fp8 ? grouped_swiglu<true>(routed, hidden, phases, tail, stream, who) : grouped_swiglu<false>(routed, hidden, phases, tail, stream, who);
-    return fp8 ? grouped_swiglu_joint<true>(routed, *shared, hidden, phases, tail, stream, who)
-               : grouped_swiglu_joint<false>(routed, *shared, hidden, phases, tail, stream, who);
+        return fp8 ? grouped_swiglu<true>(routed, hidden, phases, call, stream, who) : grouped_swiglu<false>(routed, hidden, phases, call, stream, who);
+    return fp8 ? grouped_swiglu_joint<true>(routed, *shared, hidden, phases, call, stream, who)
+               : grouped_swiglu_joint<false>(routed, *shared, hidden, phases, call, stream, who);
 }
 
 }  // namespace
@@ -2834,10 +2660,14 @@ bool layer_may_combine(int32_t n_experts, int32_t n_rows, bool shared, int32_t h
     return thin_down_narrow(thin_down_waves(n_experts, n_rows, shared, hidden));
 }
 
-int layer_experts(const moe_mlp_group& routed, const moe_mlp_group* shared, int32_t hidden, int32_t fp8, const CombineTail* tail,
-                  bool* combined, void* stream) {
-    *combined = false;
-    return swiglu_groups(routed, shared, hidden, fp8, MOE_PHASE_BOTH, TailOf{tail, combined}, stream);
+bool layer_shared_first(const moe_mlp_group& routed, const moe_mlp_group& shared, int32_t hidden) {
+    return shared.n_rows > 0 && check_group(routed, hidden, routed.fp8, "moe_layer_forward") == MOE_OK &&
+           check_group(shared, hidden, shared.fp8, "moe_layer_forward") == MOE_OK && joins(routed, shared, hidden) &&
+           joint_thin(gate_up_args(routed, hidden), routed.n_rows, row_bound(routed), gate_up_args(shared, hidden), shared.n_rows);
+}
+
+int layer_experts(const moe_mlp_group& routed, const moe_mlp_group* shared, int32_t hidden, int32_t fp8, LayerCall* call, void* stream) {
+    return swiglu_groups(routed, shared, hidden, fp8, MOE_PHASE_BOTH, call, stream);
 }
 
 }  // namespace moe
@@ -2849,7 +2679,7 @@ extern "C" int moe_grouped_swiglu_bf16(const void* x, int32_t x_rows, const int3
                                        int32_t n_rows, int32_t n_experts, int32_t hidden, int32_t inter, void* act,
                                        void* y, int32_t phases, void*, size_t, void* stream) {
     const moe_mlp_group m{x, x_rows, n_rows, row_map, w_gate, w_up, w_down, nullptr, nullptr, nullptr, offsets, n_experts, inter, 0, 0, act, y, nullptr, 0};
-    return moe::grouped_swiglu<false>(m, hidden, phases, {}, stream, "moe_grouped_swiglu_bf16");
+    return moe::grouped_swiglu<false>(m, hidden, phases, nullptr, stream, "moe_grouped_swiglu_bf16");
 }
 
 extern "C" int moe_grouped_swiglu_w8a16(const void* x, int32_t x_rows, const int32_t* row_map, const void* const* w_gate,
@@ -2859,14 +2689,14 @@ extern "C" int moe_grouped_swiglu_w8a16(const void* x, int32_t x_rows, const int
                                         int32_t n_experts, int32_t hidden, int32_t inter, void* act, void* y,
                                         int32_t phases, void*, size_t, void* stream) {
     const moe_mlp_group m{x, x_rows, n_rows, row_map, w_gate, w_up, w_down, s_gate, s_up, s_down, offsets, n_experts, inter, 0, 0, act, y, nullptr, 0};
-    return moe::grouped_swiglu<true>(m, hidden, phases, {}, stream, "moe_grouped_swiglu_w8a16");
+    return moe::grouped_swiglu<true>(m, hidden, phases, nullptr, stream, "moe_grouped_swiglu_w8a16");
 }
 
 extern "C" int moe_grouped_swiglu_joint(const moe_mlp_group* routed, const moe_mlp_group* shared, int32_t hidden, int32_t fp8,
                                         int32_t phases, void* stream) {
     using namespace moe;
     MOE_REQUIRE(routed != nullptr, "moe_grouped_swiglu_joint: NULL group");
-    return swiglu_groups(*routed, shared, hidden, fp8, phases, {}, stream);
+    return swiglu_groups(*routed, shared, hidden, fp8, phases, nullptr, stream);
 }
 
 extern "C" size_t moe_mlp_workspace_bytes(const moe_mlp_group* m, int32_t hidden) {

@@ -101,12 +101,35 @@ extern "C" int moe_layer_forward(const moe_layer_args* args, void* stream) {
         d.arrivals = tail.arrivals;
         d.n_arrivals = tail_arrivals(h);
     }
-    bool combined = false;
+    LayerCall call;
+    call.tail = may_combine ? &tail : nullptr;
+
+    moe_mlp_group routed = *a.routed;
+    routed.x = x; routed.x_rows = n; routed.n_rows = n * k; routed.row_map = d.row_map; routed.offsets = d.offsets;
+    routed.max_rows = n;
+    routed.act = ws + l.act; routed.y = ws + l.y;
+    routed.workspace = nullptr; routed.workspace_bytes = 0;       // (the caller's fields may hold anything)
+    moe_mlp_group shared{};
+    if (a.shared) {
+        shared = *a.shared;
+        shared.x = x; shared.x_rows = shared.n_rows = shared.max_rows = n; shared.row_map = nullptr; shared.offsets = d.one_group;
+        shared.act = ws + l.act_shared; shared.y = ws + l.y_shared;
+        shared.workspace = nullptr; shared.workspace_bytes = 0;
+    }
+    const bool join = a.shared && a.join_shared && shared.fp8 == routed.fp8;
+    SharedFirst first{};
+    if (join && n <= kTailTokens && E > kRouterSharedE && layer_shared_first(routed, shared, h)) {
+        first = SharedFirst{shared.w_gate, shared.w_up, shared.s_gate, shared.s_up, static_cast<const uint16_t*>(x),
+                            static_cast<uint16_t*>(shared.act), n, h, shared.inter, shared.fp8, 0};
+        call.shared_gate_up_done = true;
+    }
+    const SharedFirst* const with = call.shared_gate_up_done ? &first : nullptr;
+
     uint16_t* logits_bf16 = static_cast<uint16_t*>(a.logits_bf16);
-    if (n <= router_dispatch_tokens(E)) {
+    if (!with && n <= router_dispatch_tokens(E)) {
         rc = router_dispatch(x, a.w_gate, a.bias, p, a.topk_idx, a.topk_w, logits_bf16, d, st);
     } else {
-        rc = router_logits(x, a.w_gate, p, logits, st);
+        rc = router_logits(x, a.w_gate, p, logits, with, st);
         if (rc == MOE_OK && n <= select_dispatch_tokens(E)) {
             rc = router_select_dispatch(a.bias, p, a.topk_idx, a.topk_w, logits, logits_bf16, d, st);
         } else if (rc == MOE_OK) {
@@ -116,26 +139,13 @@ extern "C" int moe_layer_forward(const moe_layer_args* args, void* stream) {
     }
     if (rc != MOE_OK) return rc;
 
-    moe_mlp_group routed = *a.routed;
-    routed.x = x; routed.x_rows = n; routed.n_rows = n * k; routed.row_map = d.row_map; routed.offsets = d.offsets;
-    routed.max_rows = n;
-    routed.act = ws + l.act; routed.y = ws + l.y;
-    routed.workspace = nullptr; routed.workspace_bytes = 0;       // (the caller's fields may hold anything)
-    if (a.shared) {
-        moe_mlp_group shared = *a.shared;
-        shared.x = x; shared.x_rows = shared.n_rows = shared.max_rows = n; shared.row_map = nullptr; shared.offsets = d.one_group;
-        shared.act = ws + l.act_shared; shared.y = ws + l.y_shared;
-        shared.workspace = nullptr; shared.workspace_bytes = 0;
-        if (a.join_shared && shared.fp8 == routed.fp8) {
-            rc = layer_experts(routed, &shared, h, routed.fp8, may_combine ? &tail : nullptr, &combined, stream);
-        } else {
-            rc = moe_grouped_swiglu_joint(&routed, nullptr, h, routed.fp8, MOE_PHASE_BOTH, stream);
-            if (rc == MOE_OK) rc = moe_grouped_swiglu_joint(&shared, nullptr, h, shared.fp8, MOE_PHASE_BOTH, stream);
-        }
+    if (join || !a.shared) {
+        rc = layer_experts(routed, join ? &shared : nullptr, h, routed.fp8, &call, stream);
     } else {
-        rc = layer_experts(routed, nullptr, h, routed.fp8, may_combine ? &tail : nullptr, &combined, stream);
+        rc = moe_grouped_swiglu_joint(&routed, nullptr, h, routed.fp8, MOE_PHASE_BOTH, stream);
+        if (rc == MOE_OK) rc = moe_grouped_swiglu_joint(&shared, nullptr, h, shared.fp8, MOE_PHASE_BOTH, stream);
     }
-    if (rc != MOE_OK || combined) return rc;
+    if (rc != MOE_OK || call.combined) return rc;
     if (a.norm_weight)
         return moe_combine_residual(ws + l.y, d.pos, a.topk_idx, a.topk_w, y_shared, a.x, n, k, h, a.combine_mode, a.out, stream);
     return moe_combine(ws + l.y, d.pos, a.topk_idx, a.topk_w, y_shared, n, k, h, a.combine_mode, a.out, stream);

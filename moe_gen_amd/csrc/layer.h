@@ -20,8 +20,29 @@ constexpr int tail_arrivals(int hidden) { return (hidden + 15) / 16; }
 // Whether a down projection of n_rows rows (and of a shared expert) in layer_experts may combine: no call for which this is false does
 bool layer_may_combine(int32_t n_experts, int32_t n_rows, bool shared, int32_t hidden);
 
-// moe_grouped_swiglu_joint, both phases (shared may be NULL); combined: the down projection has also done what `tail` says
-int layer_experts(const moe_mlp_group& routed, const moe_mlp_group* shared, int32_t hidden, int32_t fp8, const CombineTail* tail,
-                  bool* combined, void* stream);
+// The shared expert's gate and up projection of a few tokens, which needs nothing of the router: its waves run in the router's
+// launch, which leaves most of the chip and all of the memory's rate idle (layer_shared_first).  Layers, us, in the routed experts' launch
+// -> here: DeepSeek-V2-Lite 1 / 3 / 8 / 16 tokens 49.3 / 64.2 / 79.9 / 92.3 -> 48.1 / 62.8 / 77.2 / 91.8, DeepSeek-V2-236B 2 / 8 / 16 139.4 /
+// 245.8 / 338.5 -> 131.7 / 241.5 / 330.0, DeepSeek-V3 1 / 5 / 14 123.0 / 328.6 / 655.1 -> 121.7 / 327.9 / 652.3.
+struct SharedFirst {
+    const void *const *w_gate, *const *w_up;
+    const float *const *s_gate, *const *s_up;
+    const uint16_t* x;
+    uint16_t* act;
+    int rows, hidden, inter, fp8;
+    int first_block;                     // of the launch
+};
+constexpr int shared_first_blocks(int inter) { return (inter + 15) / 16; }
+
+// Whether it may run there: the thin kernel then serves the call, whose gate and up launch leaves it out
+bool layer_shared_first(const moe_mlp_group& routed, const moe_mlp_group& shared, int32_t hidden);
+
+// moe_grouped_swiglu_joint, both phases (shared may be NULL), as a part of a layer call
+struct LayerCall {
+    const CombineTail* tail = nullptr;   // the combine, for a down projection that can end with it
+    bool combined = false;               // (result) it did
+    bool shared_gate_up_done = false;
+};
+int layer_experts(const moe_mlp_group& routed, const moe_mlp_group* shared, int32_t hidden, int32_t fp8, LayerCall* call, void* stream);
 
 }  // namespace moe

@@ -17,6 +17,7 @@
 #include "common.h"
 #include "dispatch_small.h"
 #include "moe_math.h"
+#include "thin_gemm.h"
 
 namespace moe {
 namespace {
@@ -276,10 +277,9 @@ __device__ void route_token(const float* row, const float* __restrict__ bias, co
 // FUSED == true (a caller without a logits buffer): the workgroup walks the expert blocks of its tokens one after the
 // other, keeps the logits in LDS and routes the tokens itself.  Where that leaves most CUs without tokens
 // router_tokens_kernel takes the call.
-// DISPATCH (with FUSED, one workgroup): it sorts the token's experts too, for a few tokens of up to 64 experts.
-// us, in two launches -> this: DeepSeek-V2-Lite,
-// 1 token 9.7 + 4.4 -> 14.3 and a launch less for the host; Mixtral-8x7B 17.4 + 4.9 -> 20.9.
-typedef __attribute__((address_space(3))) uint8_t* lds_u8;
+// DISPATCH (with FUSED, one workgroup): it sorts the tokens' experts too, for a few tokens of up to 32 experts.
+// Mixtral-8x7B, 1 token, us: two launches 17.4 + 4.9, this 20.9.
+// SHARED (1 bf16, 2 fp8 weights): workgroups behind the router's bring the shared expert's gate and up projection (SharedFirst).
 
 constexpr int kStageBytes = 256, kStepsPerStage = 32;    // 128 k of a row per stage, 4 k per step
 constexpr int kBlock = 1024 + 64;                        // four rows of a stage in LDS
@@ -301,11 +301,11 @@ __device__ __forceinline__ void read_bf16_as_f32(float& v, uint32_t addr) {
     asm volatile("ds_read_u16_d16_hi %0, %1 offset:%2" : "+v"(v) : "v"(addr), "n"(OFF));
 }
 
-template <int WT, int WE, int TT, int TE, int S, bool FUSED, int GW, int EJ, bool DISPATCH = false>   // (GW, EJ: route_token; read where FUSED)
+template <int WT, int WE, int TT, int TE, int S, bool FUSED, int GW, int EJ, bool DISPATCH = false, int SHARED = 0>   // (GW, EJ: route_token; read where FUSED)
 __global__ __launch_bounds__(64 * WT * WE, 1) void router_logits_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ wg, const float* __restrict__ bias,
     moe_router_params p, int32_t* topk_idx, float* __restrict__ topk_w, float* __restrict__ logits, uint16_t* __restrict__ logits_bf16,
-    DispatchOut out) {
+    DispatchOut out, SharedFirst shared) {
     static_assert(FUSED || !DISPATCH, "the tokens of one workgroup");
     static_assert(TT == TE && TT <= 2, "one tile per wave or 2 x 2");
     constexpr int NW = WT * WE, BT = 16 * TT * WT, BE = 16 * TE * WE;
@@ -320,6 +320,19 @@ __global__ __launch_bounds__(64 * WT * WE, 1) void router_logits_kernel(
     constexpr bool VAL_IN_STAGES = S == 3;                      // the selection's values in the stage buffers: two workgroups per CU then fit
     static_assert(NW * 64 * EJ * 4 <= S * SB, "selection");
     __shared__ float val_own[FUSED && !VAL_IN_STAGES ? NW * 64 * EJ : 1];
+    if constexpr (SHARED != 0) {
+        // one wave of the workgroup: the launch has more CUs than such waves, and the workgroup's LDS is its ring
+        constexpr bool W8 = SHARED == 2;
+        constexpr int STAGES = W8 ? 8 : 11;                     // as many as the counter of outstanding loads allows
+        static_assert(STAGES * thin_stage_bytes<W8, 2> <= S * SB, "ring");
+        if ((int)blockIdx.x >= shared.first_block) {
+            if (threadIdx.x < 64)
+                thin_columns<true, W8, 2, false, STAGES>(ThinUnit{shared.w_gate[0], shared.w_up[0], W8 ? shared.s_gate[0] : nullptr,
+                                                                  W8 ? shared.s_up[0] : nullptr, shared.x, nullptr, 0, 0, shared.act, shared.hidden,
+                                                                  shared.inter, 0, shared.rows}, 16 * ((int)blockIdx.x - shared.first_block), lds);
+            return;
+        }
+    }
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -671,12 +684,21 @@ __global__ __launch_bounds__(64 * SMALL_WAVES) void router_select_dispatch_kerne
     dispatch_one_workgroup<IT>(p.n_tokens * p.top_k, p.n_experts, out, p.top_k, [&](int i) { return idx[i]; });
 }
 
-template <int WT, int WE, int TT, int TE, int S>
-void launch_logits(const void* x, const void* w, const moe_router_params& p, float* logits, hipStream_t st) {
+// The launch's workgroups for the shared expert, if there is one, follow the router's
+SharedFirst behind(const SharedFirst* shared, int blocks) {
+    SharedFirst s = shared ? *shared : SharedFirst{};
+    s.first_block = blocks;
+    return s;
+}
+int more_blocks(const SharedFirst* shared) { return shared ? shared_first_blocks(shared->inter) : 0; }
+
+template <int WT, int WE, int TT, int TE, int S, int SHARED = 0>
+void launch_logits(const void* x, const void* w, const moe_router_params& p, float* logits, const SharedFirst* shared, hipStream_t st) {
     constexpr int BT = 16 * TT * WT, BE = 16 * TE * WE;
-    const int ntb = (p.n_tokens + BT - 1) / BT, neb = (p.n_experts + BE - 1) / BE;
-    hipLaunchKernelGGL((router_logits_kernel<WT, WE, TT, TE, S, false, 64, 2>), dim3((ntb + 7) / 8 * 8 * neb), dim3(64 * WT * WE), 0, st,
-                       (const uint16_t*)x, (const uint16_t*)w, nullptr, p, nullptr, nullptr, logits, nullptr, DispatchOut{});
+    const int ntb = (p.n_tokens + BT - 1) / BT, neb = (p.n_experts + BE - 1) / BE, blocks = (ntb + 7) / 8 * 8 * neb;
+    hipLaunchKernelGGL((router_logits_kernel<WT, WE, TT, TE, S, false, 64, 2, false, SHARED>), dim3(blocks + more_blocks(shared)),
+                       dim3(64 * WT * WE), 0, st, (const uint16_t*)x, (const uint16_t*)w, nullptr, p, nullptr, nullptr, logits, nullptr,
+                       DispatchOut{}, behind(shared, blocks));
 }
 template <int WE>
 void launch_tokens(const void* x, const void* w, const float* bias, const moe_router_params& p, int32_t* idx, float* tw, hipStream_t st) {
@@ -687,7 +709,7 @@ template <int WT, int WE, int TT, int S, int GW, int EJ>
 void launch_fused(const void* x, const void* w, const float* bias, const moe_router_params& p, int32_t* idx, float* tw, hipStream_t st) {
     constexpr int BT = 16 * TT * WT;
     hipLaunchKernelGGL((router_logits_kernel<WT, WE, TT, TT, S, true, GW, EJ>), dim3((p.n_tokens + BT - 1) / BT), dim3(64 * WT * WE), 0, st,
-                       (const uint16_t*)x, (const uint16_t*)w, bias, p, idx, tw, nullptr, nullptr, DispatchOut{});
+                       (const uint16_t*)x, (const uint16_t*)w, bias, p, idx, tw, nullptr, nullptr, DispatchOut{}, SharedFirst{});
 }
 
 }  // namespace
@@ -731,16 +753,15 @@ int router_dispatch(const void* x, const void* w_gate, const float* bias, const 
     static_assert(router_dispatch_tokens(1) * 16 <= 256, "one pass of 4 waves over the indices");
     auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3(1), dim3(256), 0, st, (const uint16_t*)x, (const uint16_t*)w_gate, bias, p, topk_idx, topk_w, nullptr,
-                           logits_bf16, out);
+                           logits_bf16, out, SharedFirst{});
     };
     if (p.n_experts <= 16) launch(router_logits_kernel<4, 1, 1, 1, 6, true, 16, 1, true>);
-    else if (p.n_experts <= 32) launch(router_logits_kernel<1, 4, 1, 1, 6, true, 32, 1, true>);
-    else launch(router_logits_kernel<1, 4, 1, 1, 6, true, 64, 1, true>);
+    else launch(router_logits_kernel<1, 4, 1, 1, 6, true, 32, 1, true>);
     MOE_HIP_CHECK(hipGetLastError());
     return MOE_OK;
 }
 
-int router_logits(const void* x, const void* w_gate, const moe_router_params& p, float* logits, hipStream_t st) {
+int router_logits(const void* x, const void* w_gate, const moe_router_params& p, float* logits, const SharedFirst* shared, hipStream_t st) {
     const int E = p.n_experts, n = p.n_tokens;
     // One tile per wave up to 4096 tokens of 256 experts: the matrix cores of all CUs are then busy for less than about
     // four rounds of it, and smaller workgroups leave less of the last round idle; and where the last block of 64 experts
@@ -751,10 +772,12 @@ int router_logits(const void* x, const void* w_gate, const moe_router_params& p,
     //   160 experts  16384 tokens: one tile 264, 2 x 2 with 32-expert blocks 301
     //   8 experts    16384 tokens (h = 6144): 4 waves along the tokens 35, 2 waves 38
     const int64_t work = (int64_t)n * E;
-    if (E <= 16) launch_logits<4, 1, 1, 1, 4>(x, w_gate, p, logits, st);
-    else if (work < (1 << 20) || (E % 64 != 0 && E % 64 <= 32)) launch_logits<2, 2, 1, 1, 4>(x, w_gate, p, logits, st);
-    else if (work < (1 << 21) || (E % 128 != 0 && E % 128 <= 64)) launch_logits<2, 2, 2, 2, 4>(x, w_gate, p, logits, st);
-    else launch_logits<2, 4, 2, 2, 3>(x, w_gate, p, logits, st);
+    if (E <= 16) launch_logits<4, 1, 1, 1, 4>(x, w_gate, p, logits, nullptr, st);
+    else if (shared && shared->fp8) launch_logits<2, 2, 1, 1, 4, 2>(x, w_gate, p, logits, shared, st);
+    else if (shared) launch_logits<2, 2, 1, 1, 4, 1>(x, w_gate, p, logits, shared, st);
+    else if (work < (1 << 20) || (E % 64 != 0 && E % 64 <= 32)) launch_logits<2, 2, 1, 1, 4>(x, w_gate, p, logits, nullptr, st);
+    else if (work < (1 << 21) || (E % 128 != 0 && E % 128 <= 64)) launch_logits<2, 2, 2, 2, 4>(x, w_gate, p, logits, nullptr, st);
+    else launch_logits<2, 4, 2, 2, 3>(x, w_gate, p, logits, nullptr, st);
     MOE_HIP_CHECK(hipGetLastError());
     return MOE_OK;
 }
@@ -855,7 +878,7 @@ int route(const void* x, const void* w_gate, const float* bias, const moe_router
         MOE_HIP_CHECK(hipGetLastError());
         return MOE_OK;
     }
-    const int rc = router_logits(x, w_gate, p, logits_out, st);
+    const int rc = router_logits(x, w_gate, p, logits_out, nullptr, st);
     return rc != MOE_OK ? rc : router_select(bias, p, topk_idx, topk_w, logits_out, nullptr, st);
 }
 }  // namespace
