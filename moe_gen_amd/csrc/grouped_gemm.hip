@@ -89,8 +89,9 @@ struct GemmArgs {
     uint16_t* c;                // output, row stride N, sorted-row order
     int E, K, N;
     int n_tiles_n;              // ceil(N / (SWIGLU ? 128 : 256))
-    int cold_max;               // experts of up to this many rows belong to the one-workgroup-per-tile kernel, the
-                                // others to the persistent kernel (0: all to the latter, INT_MAX: all to the former)
+    // a call of both kinds of tiles (grouped_gemm_both_kernel):
+    int cold_max;               // experts of up to this many rows are tiles of one workgroup each, the others tiles of the
+                                // persistent workgroups (0: all are)
     int rem_split;              // 1: the rule applies to what an expert's full 256-row tiles leave over (count % 256)
                                 // instead of to its count: the persistent kernel takes the full tiles, and the
                                 // last, ragged one only if it holds more than cold_max rows
@@ -1161,15 +1162,15 @@ __host__ __device__ __forceinline__ int persistent_tiles(const GemmArgs& g, int 
     if (g.rem_split) return (count >> 8) + ((count & 255) > g.cold_max ? 1 : 0);
     return is_cold(g, count) ? 0 : (count + 255) >> 8;
 }
-// How many tiles at the end of that space the persistent kernel leaves to the other kernel.  One workgroup per CU
-// walks the space in rounds of tail_cus tiles, and a last round of a few tiles costs as much as a full one while
-// most CUs idle.  Cut into 128-row halves those tiles occupy twice as many CUs for about 0.7 of a tile's time
-// each, and they join the other kernel's `own` tiles in its rounds.  The last round moves if that makes the two
-// launches shorter, counting a round of the persistent kernel 1.0 and a round of the other 0.72: alone (own = 0)
-// that is a last round of at most half the CUs; next to other work also a longer one (Mixtral-8x22B, 1024 tokens,
-// down projection: 144 tiles here and 144 there are two half-empty launches in a row, 0.71 ms; as one launch of 432
-// tiles 0.56).  Both kernels evaluate this on the same offsets[].
-struct RoundCost { int keep, move; };       // the two launches with the last round in the persistent kernel / in the other
+// How many tiles at the end of that space the persistent workgroups leave to workgroups of one tile.  One persistent workgroup
+// per CU walks the space in rounds of tail_cus tiles, and a last round of a few tiles costs as much as a full one.  Cut into
+// 128-row halves those tiles occupy twice as many CUs for about 0.7 of a tile's time each, and they join the `own` tiles of
+// that kind in their rounds.  The last round moves if that makes the sum of both kinds' rounds shorter, a round of persistent tiles
+// counted 1.0 and one of the others 0.72: alone (own = 0) that is a last round of at most half the CUs; next to other work also
+// a longer one.  (That the two kinds share a launch is not in the count: with CU-time instead of rounds, DeepSeek-V2-236B, 4000
+// tokens, gains 1 %, Mixtral-8x7B, 700 and 2500, and Mixtral-8x22B, 1200, lose 6, 4 and 5 %.)  Every workgroup evaluates this on the same
+// offsets[].
+struct RoundCost { int keep, move; };       // the rounds of both kinds with the last one persistent / as halves
 __host__ __device__ __forceinline__ RoundCost round_cost(int total, int own, int cus) {
     return RoundCost{100 * ((total + cus - 1) / cus) + 72 * ((own + cus - 1) / cus),
                      100 * (total / cus) + 72 * ((own + 2 * (total % cus) + cus - 1) / cus)};
@@ -1443,48 +1444,12 @@ __global__ __launch_bounds__(128 * WN) void grouped_gemm_kernel(GemmPair pair_of
     int v = (((slot >> 2) << 3) + (blockIdx.x & 7)) * 4 + (slot & 3);
     const bool in_front = v < pair_of.shared_tiles;
     if (!in_front) v -= pair_of.shared_tiles;
-    int problem = in_front ? 1 : 0;
 
     // ---- M-tile prefix over experts ----
-    const GemmArgs& ga = pair_of.p[problem];
-    int shared_first = 0, shared_end = 0;    // (requested here, so that the answer comes with that to the scan's loads)
-    if (pair_of.shared_rows > 0) {
-        shared_first = pair_of.p[1].offsets[0];
-        shared_end = pair_of.p[1].offsets[1];
-    }
+    const GemmArgs& g = pair_of.p[in_front ? 1 : 0];
     ExpertOfThread mine;
-    int run = mtile_prefix_scan<NT>(ga, tid, s_pref, s_wtot, mine, [&](int c) { return own_tiles<W8>(ga, c); }, [](int, int, int) {});
-    const int total = run * ga.n_tiles_n;
-
-    // Past the routed experts' tiles, where the persistent kernel runs too: the shared expert's, and then the tiles that the
-    // persistent kernel leaves at the end of ITS tile space, two workgroups (128-row halves, neighbours on one XCD) per
-    // tile.  The prefix is rebuilt over that space.
-    int half = -1;
-    if (v >= total) {
-        if (in_front || ga.tail_cus <= 0 || ga.E > NT) return;
-        SharedTiles s{0, 0, 0, 0};
-        if (pair_of.shared_rows > 0) s = shared_tiles_of<W8>(pair_of.p[1], uni(shared_first), uni(shared_end));
-        v -= total;
-        int shared = s.own;                          // of the shared expert in the tile space that v counts in
-        if (v >= shared) {
-            const int t = v - shared;
-            __syncthreads();             // s_wtot of the first scan has been read by everyone
-            run = mtile_prefix_scan<NT>(ga, tid, s_pref, s_wtot, mine, [&](int c) { return persistent_tiles(ga, c); }, [](int, int, int) {});
-            shared = s.persistent;
-            const int total_p = run * ga.n_tiles_n + shared;
-            const int tail = tail_tiles(ga, total_p, total + s.own);
-            if (t >= 2 * tail) return;
-            v = total_p - tail + (t >> 1);
-            half = t & 1;
-        }
-        if (v < shared) {                            // its one expert belongs to thread 0
-            problem = 1;
-            mine = ExpertOfThread{0, tid == 0 ? shared / pair_of.p[1].n_tiles_n : 0, s.first, s.end};
-        } else {
-            v -= shared;
-        }
-    }
-    const GemmArgs& g = pair_of.p[problem];
+    const int run = mtile_prefix_scan<NT>(g, tid, s_pref, s_wtot, mine, [&](int c) { return tiles_of<!W8>(c); }, [](int, int, int) {});
+    if (v >= run * g.n_tiles_n) return;
     const bool s8_ok = !g.row_map || g.a_bytes < (1ull << 32);   // (the weight streamer addresses gathered rows with 32-bit offsets)
     const int q = v / g.n_tiles_n;  // global M-tile number
     // find e with prefix[e] <= q < prefix[e+1].  Up to NT experts every thread still holds its own
@@ -1514,17 +1479,8 @@ __global__ __launch_bounds__(128 * WN) void grouped_gemm_kernel(GemmPair pair_of
     const int mt_e = uni(s_sel[2]);
     int m_tile, n_tile;
     tile_in_expert(v - pe * g.n_tiles_n, mt_e, g.n_tiles_n, m_tile, n_tile);
-    if (half >= 0) {                     // half of a 256-row tile of the persistent kernel's space
-        const int r0 = uni(s_sel[3]) + m_tile * 256 + half * 128;
-        const int r1 = min(uni(s_sel[4]), uni(s_sel[3]) + (m_tile + 1) * 256);
-        if (r0 >= r1) return;
-        if (W8 && s8_ok) stream8x<SWIGLU>(g, lds, e, r0, min(r1, r0 + 128), n_tile, false);
-        else if (s8_ok) stream16<SWIGLU, true>(g, lw0, lw1, lw2, lt0, lt1, e, r0, min(r1, r0 + 128), n_tile);
-        else gemm_tile<2, WN, SWIGLU, W8, false>(g, stage(0), stage(1), e, r0, r1, n_tile);
-        return;
-    }
     const int row_end = uni(s_sel[4]);
-    const int first_row = uni(s_sel[3]) + (g.rem_split ? ((row_end - uni(s_sel[3])) & ~255) : 0);
+    const int first_row = uni(s_sel[3]);
     if (W8 && s8_ok) {
         // fp8 weights: the weight streamers.  Up to 64 rows where no other kernel's summation order has to be matched: the
         // form that reads a lane's 16 weights at once.  Everything else -- up to 192 rows; what an expert's full 256-row
@@ -1823,34 +1779,55 @@ __device__ __forceinline__ int fresh_lane() {
 // conversion, 64 vector instructions per 64 matrix instructions, is what is left (a tenth more with most of it taken out).
 // PAIRED: with a second problem.  (An instantiation of its own: the choice per tile costs DeepSeek-V3's 65536 tokens 0.4 %.)
 // SPLIT: the down projection of one MLP, its tiles once per slice of k, all of them here; the fp32 sums go to `split`.
+// LDS of its workgroup: the two stages' token rows in halves, their weights, and tables.  Every piece that a DMA writes while another
+// is read is an array of its own: as separate objects they provably do not alias (otherwise a read waits for every
+// outstanding DMA).  The fp8 path writes the weight stages with ordinary LDS stores.
+constexpr int PE = 512;                          // experts that the tables hold
+struct PersistentTables {                        // (read by read_pair and read_pointers once the DMA has begun)
+    unsigned long long ptr1[4];                  // the second problem's matrices and scales
+    int off1[2];                                 // and its rows
+    int wtot[8];
+    int pref[PE + 1], off[PE + 1];               // M tiles in front of an expert, and its first row
+};
+struct PersistentLds {
+    uint8_t *a0a, *a0b, *a1a, *a1b, *b0, *b1;
+    unsigned long long* ptr;                     // [4][PE] matrices and scales of the experts
+    PersistentTables* tables;
+};
+// Reads of tables that lie behind token rows in one array: as ordinary reads they would wait for every DMA into those rows.
+__device__ __forceinline__ void read_pair(const int* p, int& a, int& b) {       // p[0], p[1]
+    unsigned long long v;
+    asm volatile("ds_read2_b32 %0, %1 offset1:1\n\ts_waitcnt lgkmcnt(0)" : "=v"(v) : "v"((uint32_t)(uintptr_t)(lds_u8)const_cast<int*>(p)) : "memory");
+    a = uni((int)(uint32_t)v);
+    b = uni((int)(v >> 32));
+}
+// N words, `stride` bytes apart
+template <int N>
+__device__ __forceinline__ void read_pointers(const unsigned long long* table, uint32_t stride, unsigned long long (&v)[4]) {
+    const uint32_t at = (uint32_t)(uintptr_t)(lds_u8)const_cast<unsigned long long*>(table);
+    if constexpr (N == 4)
+        asm volatile("ds_read_b64 %0, %4\n\tds_read_b64 %1, %5\n\tds_read_b64 %2, %6\n\tds_read_b64 %3, %7\n\ts_waitcnt lgkmcnt(0)"
+                     : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]) : "v"(at), "v"(at + stride), "v"(at + 2 * stride), "v"(at + 3 * stride) : "memory");
+    else if constexpr (N == 2)
+        asm volatile("ds_read_b64 %0, %2\n\tds_read_b64 %1, %3\n\ts_waitcnt lgkmcnt(0)" : "=&v"(v[0]), "=&v"(v[1]) : "v"(at), "v"(at + stride) : "memory");
+    else
+        asm volatile("ds_read_b64 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(v[0]) : "v"(at) : "memory");
+}
 template <bool SWIGLU, bool W8, bool PAIRED, bool SPLIT>
-__global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmPair pair_of, SplitArgs split) {
+__device__ __forceinline__ void persistent_body(const GemmPair& pair_of, const SplitArgs& split, const PersistentLds& L, int grid) {
     static_assert(!SPLIT || (!SWIGLU && W8 && !PAIRED), "slices of k: the down projection of one fp8 MLP");
     const GemmArgs& g = pair_of.p[0];            // the routed experts; the tiles of the second problem come first
     constexpr int MT = 4, WN = 4;
     constexpr int NT = 128 * WN;
     constexpr int BM = 64 * MT;
-    constexpr int A_HALF = BM / 2 * ROW_B;      // half of a token stage: the first or the last 64 rows of either wave row
-    constexpr int B_STAGE = BN_ROWS * ROW_B;
     constexpr int RB = NT / 4;                  // fp8: B rows per pass (rows are 4 chunks of 16 weights)
     constexpr int NB = BN_ROWS / RB;            // fp8: 16-byte global B chunks per thread per stage (2)
     constexpr int NBLK = SWIGLU ? 128 : 256;
     constexpr int ND = 4;                       // DMA instructions per wave and tile half (32 rows of 128 bytes = 4 x 1 KiB)
-    // Every piece that a DMA writes while another is read is an array of its own: as separate objects they provably do
-    // not alias (otherwise a read waits for every outstanding DMA).  The fp8 path writes the weight stages with
-    // ordinary LDS stores.
-    __shared__ __attribute__((aligned(1024))) uint8_t sA0a[A_HALF];
-    __shared__ __attribute__((aligned(1024))) uint8_t sA0b[A_HALF];
-    __shared__ __attribute__((aligned(1024))) uint8_t sA1a[A_HALF];
-    __shared__ __attribute__((aligned(1024))) uint8_t sA1b[A_HALF];
-    __shared__ __attribute__((aligned(1024))) uint8_t sB0[B_STAGE];
-    __shared__ __attribute__((aligned(1024))) uint8_t sB1[B_STAGE];
-    __shared__ int s_pref[MAX_E + 1];
-    __shared__ int s_wtot[NT / 64];
-    constexpr int PE = 512;
-    __shared__ int s_off[PE + 1];
-    __shared__ unsigned long long s_ptr[4][PE + 1];        // (the last column: the second problem's)
-    __shared__ int s_off1[2];
+    uint8_t *const sA0a = L.a0a, *const sA0b = L.a0b, *const sA1a = L.a1a, *const sA1b = L.a1b, *const sB0 = L.b0, *const sB1 = L.b1;
+    int *const s_pref = L.tables->pref, *const s_wtot = L.tables->wtot, *const s_off = L.tables->off, *const s_off1 = L.tables->off1;
+    unsigned long long* const s_ptr1 = L.tables->ptr1;
+    constexpr int NM = (SWIGLU ? 2 : 1) * (W8 ? 2 : 1);       // pointers of a tile: gate (down), up, then their scales
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wave_s = uni(wave);
@@ -1861,20 +1838,20 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmPair p
     const int run = mtile_prefix_scan<NT>(g, tid, s_pref, s_wtot, mine, [&](int c) { return persistent_tiles(g, SPLIT ? min(c, split.n_rows) : c); }, [&](int e, int o0, int o1) {
         s_off[e] = o0;
         if (e == g.E - 1) s_off[g.E] = o1;
-        s_ptr[0][e] = (unsigned long long)(uintptr_t)g.b0[e];
-        s_ptr[1][e] = SWIGLU ? (unsigned long long)(uintptr_t)g.b1[e] : 0ull;
-        s_ptr[2][e] = W8 ? (unsigned long long)(uintptr_t)g.s0[e] : 0ull;
-        s_ptr[3][e] = (W8 && SWIGLU) ? (unsigned long long)(uintptr_t)g.s1[e] : 0ull;
+        L.ptr[e] = (unsigned long long)(uintptr_t)g.b0[e];
+        if (SWIGLU) L.ptr[PE + e] = (unsigned long long)(uintptr_t)g.b1[e];
+        if (W8) L.ptr[NM / 2 * PE + e] = (unsigned long long)(uintptr_t)g.s0[e];
+        if (W8 && SWIGLU) L.ptr[3 * PE + e] = (unsigned long long)(uintptr_t)g.s1[e];
     });
     if (tid == 0) s_pref[g.E] = run;
     if (PAIRED && tid == 0) {
         const GemmArgs& s = pair_of.p[1];
         s_off1[0] = s.offsets[0];
         s_off1[1] = s.offsets[1];
-        s_ptr[0][PE] = (unsigned long long)(uintptr_t)s.b0[0];
-        s_ptr[1][PE] = SWIGLU ? (unsigned long long)(uintptr_t)s.b1[0] : 0ull;
-        s_ptr[2][PE] = W8 ? (unsigned long long)(uintptr_t)s.s0[0] : 0ull;
-        s_ptr[3][PE] = (W8 && SWIGLU) ? (unsigned long long)(uintptr_t)s.s1[0] : 0ull;
+        s_ptr1[0] = (unsigned long long)(uintptr_t)s.b0[0];
+        if (SWIGLU) s_ptr1[1] = (unsigned long long)(uintptr_t)s.b1[0];
+        if (W8) s_ptr1[NM / 2] = (unsigned long long)(uintptr_t)s.s0[0];
+        if (W8 && SWIGLU) s_ptr1[3] = (unsigned long long)(uintptr_t)s.s1[0];
     }
     __syncthreads();
     // whole rounds, and the last one unless it is better off with the other kernel, whose own tiles are counted for that
@@ -1883,7 +1860,7 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmPair p
     const int own = g.tail_cus > 0 ? sum_over_experts<NT>(g, tid, s_wtot, [&](int c) { return own_tiles<W8>(g, c); }) * g.n_tiles_n + second_tiles.own : 0;
     const int slice_tiles = run * g.n_tiles_n;   // SPLIT: tiles of one slice
     const int all = SPLIT ? slice_tiles * split.plan.slices : slice_tiles + ptiles1, total = all - tail_tiles(g, all, own);
-    const int xcd = blockIdx.x & 7, slots = gridDim.x >> 3;
+    const int xcd = blockIdx.x & 7, slots = grid >> 3;
     int slot = blockIdx.x >> 3;
     auto tile_of = [&](int sl) { return ((sl / slots) * 8 + xcd) * slots + (sl % slots); };
     if (tile_of(slot) >= total) return;
@@ -1932,19 +1909,18 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmPair p
             nk_n = 2 * min(split.plan.blocks, (K >> 7) - kb0);
         }
         if (second) {
-            e = PE;
-            first = uni(s_off1[0]);
-            row_end = uni(s_off1[1]);
+            e = 0;
+            read_pair(s_off1, first, row_end);
             tile_in_expert(v, ptiles1 / tiles_n, tiles_n, m_tile, n_tile);
         } else {
             v -= ptiles1;
             const int q = v / tiles_n;
-            while (uni(s_pref[cur_e + 1]) <= q) ++cur_e;
+            int pe, pe_end;
+            read_pair(s_pref + cur_e, pe, pe_end);
+            while (pe_end <= q) read_pair(s_pref + ++cur_e, pe, pe_end);
             e = cur_e;
-            const int pe = uni(s_pref[e]);
-            const int mt_e = uni(s_pref[e + 1]) - pe;
-            first = uni(s_off[e]);
-            row_end = uni(s_off[e + 1]);
+            const int mt_e = pe_end - pe;
+            read_pair(s_off + e, first, row_end);
             if (SPLIT) row_end = min(row_end, first + split.n_rows);
             tile_in_expert(v - pe * tiles_n, mt_e, tiles_n, m_tile, n_tile);
         }
@@ -1969,11 +1945,13 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmPair p
         }
         a_base_n = reinterpret_cast<const uint8_t*>(second ? g1.a : g.a) + (row_map ? (size_t)0 : (size_t)row0 * K * 2) + (SPLIT ? kb0 * 256 : 0);
         a_records_n = row_map ? (int)(uint32_t)(second ? g1.a_bytes : g.a_bytes) : -1;
-        const uint8_t* bmat0 = uni_ptr(reinterpret_cast<const void*>((uintptr_t)s_ptr[0][e]));
-        const uint8_t* bmat1 = SWIGLU ? uni_ptr(reinterpret_cast<const void*>((uintptr_t)s_ptr[1][e])) : bmat0;
+        unsigned long long ptr[4] = {};
+        read_pointers<NM>(second ? s_ptr1 : L.ptr + e, second ? 8u : PE * 8u, ptr);
+        const uint8_t* bmat0 = uni_ptr(reinterpret_cast<const void*>((uintptr_t)ptr[0]));
+        const uint8_t* bmat1 = SWIGLU ? uni_ptr(reinterpret_cast<const void*>((uintptr_t)ptr[1])) : bmat0;
         if (W8) {
-            sc0 = (gptr_f32)(uintptr_t)uni_ptr(reinterpret_cast<const void*>((uintptr_t)s_ptr[2][e]));
-            sc1 = SWIGLU ? (gptr_f32)(uintptr_t)uni_ptr(reinterpret_cast<const void*>((uintptr_t)s_ptr[3][e])) : sc0;
+            sc0 = (gptr_f32)(uintptr_t)uni_ptr(reinterpret_cast<const void*>((uintptr_t)ptr[NM / 2]));
+            sc1 = SWIGLU ? (gptr_f32)(uintptr_t)uni_ptr(reinterpret_cast<const void*>((uintptr_t)ptr[3])) : sc0;
             const int brow = t >> 2, bcol_b = (t & 3) << 4, KB = K >> 7;
 #pragma unroll
             for (int i = 0; i < NB; ++i) {
@@ -2246,15 +2224,132 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_kernel(GemmPair p
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no DMA may land in LDS after the workgroup has gone
 }
 
+// ---- both kinds of tiles in one launch: calls of a mean of 128 rows per expert or more ----
+//
+// One persistent workgroup per CU comes first; the workgroups of one tile behind them start as CUs fall free, so that the
+// rounds of the two kinds overlap and the launch drains once.  As two launches, one behind the other, the second's workgroups waited
+// for the first's last tile (a second stream costs more than it gains).  Layers, us, two launches -> this: DeepSeek-V2-Lite, 1500 / 2200 /
+// 3000 / 4096 tokens 423 / 514 / 589 / 701 -> 411 / 493 / 577 / 689, DeepSeek-V3 4500 / 9000 4385 / 7907 -> 4276 / 7840, DeepSeek-V2-236B
+// 4000 / 9000 2286 / 3743 -> 2276 / 3735, Mixtral-8x7B 700 / 2500 714 / 1694 -> 692 / 1687; 16384 tokens and more the same.
+// The two bodies take the call's arguments from two copies of them: loads that both need would move in front of the branch, and so
+// many scalar registers alive there cost the down projection 320 to 376 bytes of spills (236 -> 308 us, DeepSeek-V2-Lite, 4096 tokens).
+//
+// A workgroup of one tile: the routed experts' own tiles, the shared expert's, then the halves of the tiles that the persistent
+// workgroups leave at the end of THEIR tile space, neighbours on one XCD (the prefix is rebuilt over that space).
+struct TileTables {
+    int pref[PE + 1], wtot[8], sel[5];
+};
+template <bool SWIGLU, bool W8>
+__device__ __forceinline__ void tile_body(const GemmPair& pair_of, const TileLds& lds, int* s_pref, int* s_wtot, int* s_sel, int block) {
+    constexpr int NT = 512;
+    const int tid = threadIdx.x;
+    const int slot = block >> 3;
+    int v = (((slot >> 2) << 3) + (block & 7)) * 4 + (slot & 3);
+    int problem = 0;
+    const GemmArgs& ga = pair_of.p[0];
+    int shared_first = 0, shared_end = 0;    // (requested here, so that the answer comes with that to the scan's loads)
+    if (pair_of.shared_rows > 0) {
+        shared_first = pair_of.p[1].offsets[0];
+        shared_end = pair_of.p[1].offsets[1];
+    }
+    ExpertOfThread mine;
+    int run = mtile_prefix_scan<NT>(ga, tid, s_pref, s_wtot, mine, [&](int c) { return own_tiles<W8>(ga, c); }, [](int, int, int) {});
+    const int total = run * ga.n_tiles_n;
+    int half = -1;
+    if (v >= total) {
+        SharedTiles s{0, 0, 0, 0};
+        if (pair_of.shared_rows > 0) s = shared_tiles_of<W8>(pair_of.p[1], uni(shared_first), uni(shared_end));
+        v -= total;
+        int shared = s.own;                          // of the shared expert in the tile space that v counts in
+        if (v >= shared) {
+            const int t = v - shared;
+            __syncthreads();             // s_wtot of the first scan has been read by everyone
+            run = mtile_prefix_scan<NT>(ga, tid, s_pref, s_wtot, mine, [&](int c) { return persistent_tiles(ga, c); }, [](int, int, int) {});
+            shared = s.persistent;
+            const int total_p = run * ga.n_tiles_n + shared;
+            const int tail = tail_tiles(ga, total_p, total + s.own);
+            if (t >= 2 * tail) return;
+            v = total_p - tail + (t >> 1);
+            half = t & 1;
+        }
+        if (v < shared) {                            // its one expert belongs to thread 0
+            problem = 1;
+            mine = ExpertOfThread{0, tid == 0 ? shared / pair_of.p[1].n_tiles_n : 0, s.first, s.end};
+        } else {
+            v -= shared;
+        }
+    }
+    const GemmArgs& g = pair_of.p[problem];
+    const int q = v / g.n_tiles_n;
+    if (tid < g.E && mine.start <= q && q < mine.start + mine.mt) {
+        s_sel[0] = tid; s_sel[1] = mine.start; s_sel[2] = mine.mt; s_sel[3] = mine.o0; s_sel[4] = mine.o1;
+    }
+    __syncthreads();
+    const int e = uni(s_sel[0]), pe = uni(s_sel[1]), mt_e = uni(s_sel[2]), o0 = uni(s_sel[3]), row_end = uni(s_sel[4]);
+    int m_tile, n_tile;
+    tile_in_expert(v - pe * g.n_tiles_n, mt_e, g.n_tiles_n, m_tile, n_tile);
+    int r0, r1;
+    bool neighbours = true;
+    if (half >= 0) {                     // half of a 256-row tile of the persistent kernel's space
+        r0 = o0 + m_tile * 256 + half * 128;
+        r1 = min(min(row_end, o0 + (m_tile + 1) * 256), r0 + 128);
+        if (r0 >= r1) return;
+    } else {
+        const int first_row = o0 + (g.rem_split ? ((row_end - o0) & ~255) : 0), rows_e = row_end - first_row;
+        const int slice = !W8 && rows_e >= PAIR_LO ? half_rows(rows_e) : 128;
+        r0 = mt_e > 1 ? first_row + m_tile * slice : first_row;
+        r1 = mt_e > 1 ? min(row_end, r0 + slice) : row_end;
+        neighbours = mt_e > 1;
+    }
+    if (W8) stream8x<SWIGLU>(g, lds, e, r0, r1, n_tile, false);
+    else if (neighbours) stream16<SWIGLU, true>(g, lds.w0, lds.w1, lds.w2, lds.t0, lds.t1, e, r0, r1, n_tile);
+    else stream16<SWIGLU, false>(g, lds.w0, lds.w1, lds.w2, lds.t0, lds.t1, e, r0, r1, n_tile);
+}
+template <bool SWIGLU, bool W8, bool PAIRED>
+__global__ __launch_bounds__(512) void grouped_gemm_both_kernel(GemmPair persistent_of, GemmPair tiles_of, int persistent_grid) {
+    // The streamers' three weight buffers and token buffers.  The persistent kernel has its weights in the first two and its token
+    // rows in the lower 16 KiB of the others, with its tables behind two of those.  (bf16: the whole LDS of a CU.)
+    constexpr int TOKENS = 128 * ROW_B;
+    __shared__ __attribute__((aligned(1024))) uint8_t lw0[S8_WBYTES];
+    __shared__ __attribute__((aligned(1024))) uint8_t lw1[S8_WBYTES];
+    __shared__ __attribute__((aligned(1024))) uint8_t lw2[S8_WBYTES];
+    __shared__ __attribute__((aligned(1024))) uint8_t lt0[W8 ? TOKENS : 192 * ROW_B];
+    __shared__ __attribute__((aligned(1024))) uint8_t lt1[192 * ROW_B];
+    __shared__ __attribute__((aligned(1024))) uint8_t lt2[TOKENS];
+    __shared__ __attribute__((aligned(16))) uint8_t tile_tables[W8 ? sizeof(TileTables) : 16];
+    static_assert(TOKENS + 4 * PE * 8 <= S8_WBYTES && TOKENS + sizeof(PersistentTables) <= 192 * ROW_B && sizeof(TileTables) <= TOKENS, "tables");
+    if ((int)blockIdx.x < persistent_grid) {
+        persistent_body<SWIGLU, W8, PAIRED, false>(persistent_of, SplitArgs{}, PersistentLds{lt0, lt1, lt2, lw2, lw0, lw1,
+                                                   reinterpret_cast<unsigned long long*>(lw2 + TOKENS),
+                                                   reinterpret_cast<PersistentTables*>(lt1 + TOKENS)}, persistent_grid);
+    } else {
+        TileTables& t = *reinterpret_cast<TileTables*>(W8 ? tile_tables : lt2);      // (the bf16 streamer has two token buffers)
+        tile_body<SWIGLU, W8>(tiles_of, TileLds{lw0, lw1, lw2, lt0, lt1, lt2}, t.pref, t.wtot, t.sel, (int)blockIdx.x - persistent_grid);
+    }
+}
+
+// The persistent kernel alone: one MLP's down projection in slices of k
+__global__ __launch_bounds__(512) void grouped_gemm_persistent_split_kernel(GemmPair pair_of, SplitArgs split) {
+    __shared__ __attribute__((aligned(1024))) uint8_t a0a[128 * ROW_B];
+    __shared__ __attribute__((aligned(1024))) uint8_t a0b[128 * ROW_B];
+    __shared__ __attribute__((aligned(1024))) uint8_t a1a[128 * ROW_B];
+    __shared__ __attribute__((aligned(1024))) uint8_t a1b[128 * ROW_B];
+    __shared__ __attribute__((aligned(1024))) uint8_t b0[BN_ROWS * ROW_B];
+    __shared__ __attribute__((aligned(1024))) uint8_t b1[BN_ROWS * ROW_B];
+    __shared__ unsigned long long ptr[4 * PE];
+    __shared__ PersistentTables tables;
+    persistent_body<false, true, false, true>(pair_of, split, PersistentLds{a0a, a0b, a1a, a1b, b0, b1, ptr, &tables}, (int)gridDim.x);
+}
+
+// tiles of one workgroup each, whole rounds of 8 groups of 4
+inline long tile_grid(long tiles) { return (tiles + 31) / 32 * 32; }
+
 template <int WN, bool SWIGLU, bool W8>
 int launch_tiles(const GemmPair& pair, int n_rows, hipStream_t st) {
     auto kern = grouped_gemm_kernel<WN, SWIGLU, W8>;
     const GemmArgs& g = pair.p[0];
-    // sum_e tiles_of(c_e) <= sum_e (c_e / 128 + 1); with the larger experts elsewhere, one tile per expert that has rows
-    const long max_mtiles = g.cold_max <= 192 ? (g.pair_rows ? 2 : 1) * (long)(g.E < n_rows ? g.E : n_rows) : (long)n_rows / 128 + g.E;
-    // (+ the persistent kernel's last tiles, less than a round of them, as two half tiles each)
-    const int shared = pair.shared_rows > 0 ? shared_tiles_bound<W8>(pair.p[1], pair.shared_rows).own : pair.shared_tiles;
-    const long grid = ((max_mtiles * g.n_tiles_n + shared + 2 * g.tail_cus + 31) / 32) * 32;   // whole rounds of 8 groups of 4 tiles
+    const long tiles = ((long)n_rows / 128 + g.E) * g.n_tiles_n;       // sum_e tiles_of(c_e) <= sum_e (c_e / 128 + 1)
+    const long grid = tile_grid(tiles + pair.shared_tiles);
     if (grid > 0x7fffffffL) {
         set_error("grouped gemm: %ld workgroups exceed the grid limit", grid);
         return MOE_ERR_INVALID;
@@ -2314,20 +2409,6 @@ int launch_thin(const GemmArgs& g, int n_rows, const GemmArgs* shared, LayerCall
     }
 }
 
-template <bool SWIGLU, bool W8>
-int launch_persistent(const GemmPair& pair, int n_rows, hipStream_t st) {
-    const GemmArgs& g = pair.p[0];
-    const long max_mtiles = (long)n_rows / 256 + g.E;
-    const int shared = pair.shared_rows > 0 ? shared_tiles_bound<W8>(pair.p[1], pair.shared_rows).persistent : 0;
-    long grid = ((max_mtiles * g.n_tiles_n + shared + 7) / 8) * 8;
-    const long ncu = (cu_count() / 8) * 8;
-    if (grid > ncu) grid = ncu;
-    if (pair.shared_rows > 0) hipLaunchKernelGGL((grouped_gemm_persistent_kernel<SWIGLU, W8, true, false>), dim3((unsigned)grid), dim3(512), 0, st, pair, SplitArgs{});
-    else hipLaunchKernelGGL((grouped_gemm_persistent_kernel<SWIGLU, W8, false, false>), dim3((unsigned)grid), dim3(512), 0, st, pair, SplitArgs{});
-    MOE_HIP_CHECK(hipGetLastError());
-    return MOE_OK;
-}
-
 // 4 GiB of gathered rows or more: only the register-staged body addresses them
 inline bool gather_fits(const GemmArgs& g) { return !g.row_map || g.a_bytes < (1ull << 32); }
 
@@ -2381,8 +2462,8 @@ int launch_split(const GemmArgs& g, int n_rows, const SplitPlan& plan, float* pa
         pair.p[0] = g;
         pair.p[0].rem_split = 1;                 // every row on this kernel's tiles, the last one padded
         const long tiles = (long)pieces * plan.m_tiles, ncu = (cu_count() / 8) * 8, grid = (tiles + 7) / 8 * 8;
-        hipLaunchKernelGGL((grouped_gemm_persistent_kernel<false, true, false, true>), dim3((unsigned)(grid < ncu ? grid : ncu)), dim3(512), 0, st,
-                           pair, SplitArgs{plan, n_rows, part});
+        hipLaunchKernelGGL(grouped_gemm_persistent_split_kernel, dim3((unsigned)(grid < ncu ? grid : ncu)), dim3(512), 0, st, pair,
+                           SplitArgs{plan, n_rows, part});
     } else {
         hipLaunchKernelGGL(grouped_gemm_split_kernel, dim3((pieces + 7) / 8 * 8 * plan.m_tiles), dim3(512), 0, st, g, n_rows, plan, part);
     }
@@ -2417,21 +2498,33 @@ bool thin_pays(const GemmArgs& g, int n_rows, const GemmArgs* shared) {
 // tables for up to 512 experts and addresses gathered rows with 32-bit offsets.
 inline bool persistent_fits(const GemmArgs& g) { return g.K % 128 == 0 && g.E <= 512 && gather_fits(g) && cu_count() >= 8; }
 
-// the rules by which a call's tiles fall to the two kernels (reasons in launch_mt)
+// the rules by which a call's tiles fall to the two kinds of workgroups (reasons in launch_mt)
 template <bool W8>
 GemmArgs both_kernels(GemmArgs g) {
     g.alone = 0;
     g.cold_max = 192;
     g.rem_split = W8 ? 1 : 0;
     g.pair_rows = W8 ? 0 : 1;
-    g.tail_cus = (cu_count() / 8) * 8;     // the persistent launch's grid when there is a round of tiles or more
+    g.tail_cus = (cu_count() / 8) * 8;     // the persistent workgroups when there is a round of tiles or more
     return g;
 }
 
 template <bool SWIGLU, bool W8>
 int launch_both(const GemmPair& pair, int n_rows, hipStream_t st) {
-    const int rc = launch_persistent<SWIGLU, W8>(pair, n_rows, st);
-    return rc != MOE_OK ? rc : launch_tiles<4, SWIGLU, W8>(pair, n_rows, st);
+    const GemmArgs& g = pair.p[0];
+    const SharedTiles shared = pair.shared_rows > 0 ? shared_tiles_bound<W8>(pair.p[1], pair.shared_rows) : SharedTiles{};
+    const long ncu = (cu_count() / 8) * 8, own = ((long)n_rows / 256 + g.E) * g.n_tiles_n + shared.persistent;
+    const long persistent = own < ncu ? (own + 7) / 8 * 8 : ncu;
+    // one tile per expert that has rows (bf16 weights: two), the shared expert's, and a last round's halves
+    const long grid = persistent + tile_grid((W8 ? 1 : 2) * (long)(g.E < n_rows ? g.E : n_rows) * g.n_tiles_n + shared.own + 2 * g.tail_cus);
+    if (grid > 0x7fffffffL) {
+        set_error("grouped gemm: %ld workgroups exceed the grid limit", grid);
+        return MOE_ERR_INVALID;
+    }
+    if (pair.shared_rows > 0) hipLaunchKernelGGL((grouped_gemm_both_kernel<SWIGLU, W8, true>), dim3((unsigned)grid), dim3(512), 0, st, pair, pair, (int)persistent);
+    else hipLaunchKernelGGL((grouped_gemm_both_kernel<SWIGLU, W8, false>), dim3((unsigned)grid), dim3(512), 0, st, pair, pair, (int)persistent);
+    MOE_HIP_CHECK(hipGetLastError());
+    return MOE_OK;
 }
 
 // max_rows: no expert has more rows (callers that do not know pass n_rows)
@@ -2447,19 +2540,15 @@ int launch_mt(const GemmArgs& g0, int n_rows, int max_rows, void* workspace, siz
     if (max_rows <= 16 && gather_fits(g) && thin_pays(g, n_rows, nullptr)) return launch_thin<SWIGLU, W8>(g, n_rows, nullptr, call, st);
     GemmPair pair{};
     if (mean < 128 || !persistent_fits(g)) {
-        g.cold_max = 0x7fffffff;
         g.alone = 1;
         pair.p[0] = g;
         return launch_tiles<4, SWIGLU, W8>(pair, n_rows, st);
     }
-    // The counts themselves live on the device; only their mean is known here.  Both kernels are launched and every
-    // expert goes by its own count: what fits one tile of the one-workgroup-per-tile kernel runs there, at its own
-    // height and without 256-row padding, the rest on the persistent kernel's 256-row tiles.  A launch that finds
-    // nothing of its kind costs a prefix scan per workgroup.  DeepSeek-V2-Lite, 4096 tokens (64 experts of
+    // The counts themselves live on the device; only their mean is known here.  Every expert goes by its own count: what
+    // fits one tile of a workgroup of its own runs there, at its own height and without 256-row padding, the rest on the
+    // persistent workgroups' 256-row tiles.  (As two launches:) DeepSeek-V2-Lite, 4096 tokens (64 experts of
     // 0 ... 3989 rows, 47 of them below 193, whose 256-row tiles were 49 % padding): block step 0.923 -> 0.847 ms,
     // routed gate/up 0.395 -> 0.355 ms; DeepSeek-V2-236B, 32768 tokens: 11.48 -> 11.39 ms.
-    // (The two launches on two streams, so that the second fills the CUs that the persistent kernel's last round
-    // leaves idle, measured the same 0.36 ms: the launches stay on the caller's stream.)
     // fp8 weights: the rule is applied to what an expert's full 256-row tiles leave over.  A ragged
     // last tile costs the persistent kernel a full tile of MFMA time; the other kernel streams the expert's weights
     // once more for it, and fp8 weights are half the bytes.  DeepSeek-V3, 65536 tokens (256 experts of 581 ... 3941
@@ -2469,16 +2558,14 @@ int launch_mt(const GemmArgs& g0, int n_rows, int max_rows, void* workspace, siz
     // 3584 / 4096 / 8192 tokens 4.53 -> 3.99, 4.64 -> 4.31, 7.50 -> 7.41 ms (at 4096 tokens 109 of the 256 experts hold
     // 129 to 192 rows, which were padded 256-row tiles).  With bf16
     // weights it is break-even (Mixtral-8x7B 9.28 -> 9.23 ms, DeepSeek-V2-236B 11.34 -> 11.42) and not done.
-    // (Both launches at every mean: from 1536 rows per expert a small expert is rare, but the second launch is there
-    // for the persistent kernel's last round anyway.)
     // Last round of the persistent kernel (tail_tiles above): Mixtral-8x22B, 8192 tokens, down projection (6.4 rounds
     // of 0.4 ms) 2.82 -> 2.66 ms, step 8.31 -> 8.13; Mixtral-8x7B 9.39 -> 9.27 ms; DeepSeek-V2-Lite 0.855 -> 0.821 ms
     // (its shared expert's 128 down tiles become 256 half tiles: 0.071 -> 0.055 ms); DeepSeek-V2-236B 11.43 -> 11.46,
     // DeepSeek-V3 46.56 -> 46.54: short rounds gain nothing, a partial round of few CUs runs at a higher clock anyway.
     pair.p[0] = both_kernels<W8>(g);
     // One fp8 expert (a dense MLP): the rows are known here.  What its full tiles leave over goes to the persistent kernel too,
-    // as a padded tile, where that shortens the two launches by the same count: the last round has room, or the other launch
-    // is saved.  DeepSeek-V3's dense MLP, us: 1300 / 1800 / 2200 / 4000 / 6000 tokens (leftovers of 20, 8, 152, 160 and 112 rows) 1129 /
+    // as a padded tile, where that shortens the rounds by the same count: the last one has room, or the other kind is
+    // saved.  DeepSeek-V3's dense MLP, us: 1300 / 1800 / 2200 / 4000 / 6000 tokens (leftovers of 20, 8, 152, 160 and 112 rows) 1129 /
     // 1352 / 1567 / 2726 / 3998 -> 1015 / 1263 / 1465 / 2606 / 3887; done always, 600 / 1100 / 3500 tokens would be 616 / 931 / 2370
     // instead of 534 / 816 / 2265.
     if (W8 && g.E == 1 && own_tiles<W8>(pair.p[0], n_rows) > 0) {
@@ -2501,7 +2588,6 @@ int launch_joint(const GemmArgs& routed, int n_rows, int max_rows, const GemmArg
         return launch_thin<SWIGLU, W8>(routed, n_rows, SWIGLU && call && call->shared_gate_up_done ? nullptr : &shared, call, st);
     GemmPair pair{{routed, shared}, 0, 0};
     if (n_rows / routed.E < 128) {
-        pair.p[0].cold_max = pair.p[1].cold_max = 0x7fffffff;
         pair.p[0].alone = 1;
         pair.shared_tiles = tiles_of<!W8>(n_shared) * shared.n_tiles_n;
         return launch_tiles<4, SWIGLU, W8>(pair, n_rows, st);
