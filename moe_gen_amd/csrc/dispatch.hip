@@ -9,10 +9,11 @@
 //     offsets[e] + #{i' < i : idx[i'] == e}
 // which is a pure function of the index list, hence identical on every run.
 //
-// Three small kernels over the n*k index list (a few MB at most):
+// Small kernels over the n*k index list (a few MB at most):
 //   1. block_histogram : each block counts its 2048-entry segment per expert (LDS atomics)
 //   2. scan_segments   : one wave per expert turns the per-segment counts into exclusive
-//                        bases across segments and writes counts[e]
+//                        bases across segments and writes counts[e]; up to SUM_SEGMENTS segments every block of
+//                        the next kernel adds up the counts itself instead, a launch less
 //   3. rank_scatter    : each block rebuilds offsets[] in LDS, ranks its entries with
 //                        wave-level match masks and writes perm / pos (and row_map = perm / k,
 //                        the token row behind each sorted row, for the GEMM's fused gather)
@@ -76,50 +77,76 @@ __global__ __launch_bounds__(256) void scan_segments(int32_t* __restrict__ seg_c
     if (lane == 0) counts[e] = carry;
 }
 
+// SCANNED: seg_base holds the segments' exclusive bases and counts[] their sums; else the segments' counts, which every block adds
+// up for itself (a thread per expert, its loads all on their way at once), and counts[] is written here.
+template <bool SCANNED>
 __global__ __launch_bounds__(256) void rank_scatter(const int32_t* __restrict__ idx, int64_t nk, int E,
-                                                    const int32_t* __restrict__ seg_base,
-                                                    const int32_t* __restrict__ counts,
+                                                    const int32_t* __restrict__ seg_base, int nseg,
+                                                    int32_t* __restrict__ counts,
                                                     int32_t* __restrict__ offsets, int32_t* __restrict__ perm,
                                                     int32_t* __restrict__ pos, int32_t* __restrict__ row_map, int k,
                                                     int32_t* __restrict__ one_group) {
-    __shared__ int off[MAX_E];                 // exclusive prefix sum of counts
     __shared__ int whist[SEG_WAVES][MAX_E];    // per-wave counts, then per-wave running cursors
+    __shared__ int wtot[4];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 
+    // the lane's entries of the wave's 512-entry slice, requested at once; -1: past the list or an id outside [0, E)
+    constexpr int IT = SEG_PER_WAVE / 64;
+    const int64_t wbase = (int64_t)blockIdx.x * SEG + (int64_t)wave * SEG_PER_WAVE;
+    int ev[IT];
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+        const int64_t g = wbase + 64 * it + lane;
+        ev[it] = idx[g < nk ? g : nk - 1];
+    }
+    int cv = 0, base = 0;                      // entries of expert tid, and those in earlier segments
+    if (SCANNED) {
+        if (tid < E) {
+            cv = counts[tid];
+            base = seg_base[(size_t)blockIdx.x * E + tid];
+        }
+    } else if (tid < E) {
+        for (int b0 = 0; b0 < nseg; b0 += 16) {
+            int c[16];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) c[i] = seg_base[(size_t)min(b0 + i, nseg - 1) * E + tid];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const int v = b0 + i < nseg ? c[i] : 0;
+                cv += v;
+                base += b0 + i < (int)blockIdx.x ? v : 0;
+            }
+        }
+        if (blockIdx.x == 0) counts[tid] = cv;
+    }
     // offsets[e] = sum_{e' < e} counts[e'] : 256-wide scan by the whole block
-    int cv = tid < E ? counts[tid] : 0;
     int inc = cv;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
         int o = __shfl_up(inc, d);
         if (lane >= d) inc += o;
     }
-    __shared__ int wtot[4];
     if (lane == 63) wtot[wave] = inc;
     for (int e = tid; e < SEG_WAVES * MAX_E; e += 256) (&whist[0][0])[e] = 0;
     __syncthreads();
-    int wpre = 0;
-    for (int w = 0; w < wave; ++w) wpre += wtot[w];
-    off[tid] = wpre + inc - cv;
+    int off = inc - cv;
+    for (int w = 0; w < wave; ++w) off += wtot[w];
     if (blockIdx.x == 0) {
-        if (tid < E) offsets[tid] = wpre + inc - cv;
-        if (tid == E - 1) offsets[E] = wpre + inc;
+        if (tid < E) offsets[tid] = off;
+        if (tid == E - 1) offsets[E] = off + cv;
         if (one_group && tid < 2) one_group[tid] = tid ? (int32_t)(nk / k) : 0;
     }
 
-    // pass 1: counts of this wave's 512-entry slice
-    const int64_t wbase = (int64_t)blockIdx.x * SEG + (int64_t)wave * SEG_PER_WAVE;
-    for (int i = lane; i < SEG_PER_WAVE; i += 64) {
-        int64_t g = wbase + i;
-        if (g < nk) {
-            int e = idx[g];
-            if ((unsigned)e < (unsigned)E) atomicAdd(&whist[wave][e], 1);
-        }
+    // pass 1: counts of this wave's slice
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+        if (wbase + 64 * it + lane >= nk || (unsigned)ev[it] >= (unsigned)E) ev[it] = -1;
+        if (ev[it] >= 0) atomicAdd(&whist[wave][ev[it]], 1);
     }
     __syncthreads();
     // cursor of wave w for expert e = offsets[e] + base of this segment + counts of earlier waves
     if (tid < E) {
-        int run = off[tid] + seg_base[(size_t)blockIdx.x * E + tid];
+        int run = off + base;
 #pragma unroll
         for (int w = 0; w < SEG_WAVES; ++w) {
             int c = whist[w][tid];
@@ -131,14 +158,14 @@ __global__ __launch_bounds__(256) void rank_scatter(const int32_t* __restrict__ 
 
     // pass 2: stable rank inside the wave slice, 64 entries at a time in index order
     int* cur = whist[wave];
-    for (int i0 = 0; i0 < SEG_PER_WAVE; i0 += 64) {
-        int64_t g = wbase + i0 + lane;
-        const bool in_list = g < nk;
-        int e = in_list ? idx[g] : 0;
-        const bool ok = in_list && (unsigned)e < (unsigned)E;
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+        const int64_t g = wbase + 64 * it + lane;
+        const int e = ev[it];
+        const bool ok = e >= 0;
         // an expert id outside [0, E) owns no sorted row: its slot gets -1, which the combine
         // skips (no row read, nothing added)
-        if (in_list && !ok) pos[g] = -1;
+        if (g < nk && !ok) pos[g] = -1;
         uint64_t peers = __ballot(ok);
 #pragma unroll
         for (int b = 0; b < 8; ++b) {
@@ -146,23 +173,30 @@ __global__ __launch_bounds__(256) void rank_scatter(const int32_t* __restrict__ 
             uint64_t bal = __ballot(bit);
             peers &= bit ? bal : ~bal;
         }
+        const uint64_t below = peers & ((1ull << lane) - 1ull);
         if (ok) {
-            uint64_t below = peers & ((1ull << lane) - 1ull);
             int r = cur[e] + __popcll(below);
             perm[r] = (int32_t)g;
             pos[g] = r;
             if (row_map) row_map[r] = (int32_t)(g / k);
         }
         // every read of cur[] above precedes this update in the wave's LDS order
-        if (ok && (peers & ((1ull << lane) - 1ull)) == 0) cur[e] += __popcll(peers);
+        if (ok && below == 0) cur[e] += __popcll(peers);
     }
 }
 
-constexpr int SMALL_MAX = 12288;   // one launch of 18.6 us against three of 21.7 (16384 entries: 23.7)
+// Launches of a list, us, 64 and 256 experts.  One of one workgroup, a pass of its 1024 threads per 1024 entries: 1024 entries 3.6 and
+// 3.7 (with room for all passes 4.2 and 4.4), 4096 6.5 and 7.1, 6144 8.3 and 9.1, 8192 10.4 and 11.7, 12288 13.7 and 16.2.  Two (histogram,
+// ranks): 4096 8.9 and 9.2, 8192 9.0 and 9.3, 24576 9.1 and 9.5, 131072 11.2 and 11.9; with the scan between them, and every entry loaded
+// twice, 24576 13.5 and 14.3, 131072 14.0 and 14.9.  Three: 196608 11.9 and 12.6, 524288 14.5 and 16.8 (every entry loaded twice 14.7 and
+// 15.9, 17.9 and 19.8).
+constexpr int SMALL_MAX = 6144;
+constexpr int SUM_SEGMENTS = 64;
 
+template <int IT>                            // passes over the list
 __global__ __launch_bounds__(64 * SMALL_WAVES) void dispatch_small(const int32_t* __restrict__ idx, int nk, int E, DispatchOut out,
                                                                    int k) {
-    dispatch_one_workgroup<SMALL_MAX / (SMALL_WAVES * 64)>(nk, E, out, k, [&](int i) { return idx[i]; });
+    dispatch_one_workgroup<IT>(nk, E, out, k, [&](int i) { return idx[i]; });
 }
 
 __global__ __launch_bounds__(256) void gather_rows(const u32x4* __restrict__ x, const int32_t* __restrict__ perm,
@@ -193,13 +227,16 @@ namespace {
 int dispatch_launch(const int32_t* topk_idx, int64_t nk, int32_t top_k, int32_t n_experts, const DispatchOut& out, const void* x,
                     int32_t hidden, void* xs, int32_t* seg, hipStream_t st) {
     if (nk <= SMALL_MAX) {
-        hipLaunchKernelGGL(dispatch_small, dim3(1), dim3(64 * SMALL_WAVES), 0, st, topk_idx, (int)nk, n_experts, out, top_k);
+        constexpr int PASS = 64 * SMALL_WAVES;
+        hipLaunchKernelGGL(nk <= PASS ? dispatch_small<1> : dispatch_small<SMALL_MAX / PASS>, dim3(1), dim3(PASS), 0, st, topk_idx, (int)nk,
+                           n_experts, out, top_k);
     } else {
         const int nseg = (int)((nk + SEG - 1) / SEG);
         hipLaunchKernelGGL(block_histogram, dim3(nseg), dim3(256), 0, st, topk_idx, nk, n_experts, seg);
-        hipLaunchKernelGGL(scan_segments, dim3((n_experts + 3) / 4), dim3(256), 0, st, seg, nseg, n_experts, out.counts);
-        hipLaunchKernelGGL(rank_scatter, dim3(nseg), dim3(256), 0, st, topk_idx, nk, n_experts, seg, out.counts, out.offsets,
-                           out.perm, out.pos, out.row_map, top_k, out.one_group);
+        if (nseg > SUM_SEGMENTS)
+            hipLaunchKernelGGL(scan_segments, dim3((n_experts + 3) / 4), dim3(256), 0, st, seg, nseg, n_experts, out.counts);
+        hipLaunchKernelGGL(nseg > SUM_SEGMENTS ? rank_scatter<true> : rank_scatter<false>, dim3(nseg), dim3(256), 0, st, topk_idx, nk, n_experts,
+                           seg, nseg, out.counts, out.offsets, out.perm, out.pos, out.row_map, top_k, out.one_group);
     }
     if (x) {
         hipLaunchKernelGGL(gather_rows, dim3((unsigned)((nk + 3) / 4)), dim3(256), 0, st,

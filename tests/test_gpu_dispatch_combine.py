@@ -21,7 +21,7 @@ def rand_idx(n, k, E, seed, skew=False):
 
 @pytest.mark.parametrize("n,k,E", [(1, 1, 1), (7, 2, 8), (300, 6, 64), (2048, 8, 256), (5000, 6, 160),
                                    (4097, 2, 8), (33, 8, 256),
-                                   (1536, 8, 256), (1537, 8, 256), (767, 16, 200)])   # either side of the one-workgroup form's 12288 entries
+                                   (1536, 8, 256), (1537, 8, 256), (767, 16, 200)])   # 12288 entries and a few more
 @pytest.mark.parametrize("skew", [False, True])
 def test_dispatch_bit_exact(n, k, E, skew):
     from moe_gen_amd import ops
@@ -102,6 +102,29 @@ def test_dispatch_ignores_out_of_range_ids():
         torch.cuda.synchronize()
         ref = O.combine(bits(ys_ref), pos_ref, idx_ref, w_ref, None, mode)
         assert np.array_equal(bits(out), ref), mode
+
+
+@pytest.mark.parametrize("n,k,E", [(1024, 1, 64), (1025, 1, 64), (2048, 3, 256), (6145, 1, 256), (16384, 8, 200), (16385, 8, 256), (33000, 8, 17)])
+def test_dispatch_at_the_limits_of_its_forms(n, k, E):
+    """One workgroup with one pass over the list (up to 1024 entries) and with several (6144), two launches (64 segments of 2048
+    entries, counts that every block adds up) and three: against a stable sort, ids outside [0, E) included."""
+    from moe_gen_amd import ops
+    print(f"dispatch forms n={n} k={k} E={E}", flush=True)
+    g = torch.Generator().manual_seed(n + E)
+    idx = (torch.rand(n * k, generator=g) ** 3 * E).to(torch.int32)         # skewed to the low ids
+    bad = torch.randint(0, n * k, (5,), generator=g)
+    idx[bad] = torch.tensor([-1, E, E + 7, -5, 1 << 20], dtype=torch.int32)
+    d = ops.dispatch(idx.view(n, k).cuda(), E, None, want_row_map=True)
+    torch.cuda.synchronize()
+    ok = (idx >= 0) & (idx < E)
+    order = torch.where(ok, idx, E).argsort(stable=True)[:int(ok.sum())]
+    pos = torch.full((n * k,), -1, dtype=torch.int64)
+    pos[order] = torch.arange(len(order))
+    counts = torch.bincount(idx[ok], minlength=E)
+    assert torch.equal(d.counts.cpu().long(), counts)
+    assert torch.equal(d.offsets.cpu().long(), torch.cat([torch.zeros(1, dtype=torch.int64), counts.cumsum(0)]))
+    assert torch.equal(d.pos.cpu().long(), pos)
+    assert torch.equal(d.perm.cpu().long()[:len(order)], order) and torch.equal(d.row_map.cpu().long()[:len(order)], order // k)
 
 
 @pytest.mark.parametrize("mode", [0, 1, 2])
