@@ -26,7 +26,8 @@ constexpr int MAX_K = kCombineMaxK;
 // outstanding load per lane is too few.  The block has one lane per chunk of the row where that
 // fits (up to 1024 threads), so a token's loads all leave at once.  Expert outputs are read once and
 // the result is not read again here: both go past the caches non-temporally (measured on 65536 x 8
-// rows of 7168: 1.90 -> 1.70 ms; 32768 x 6 of 5120: 0.54 -> 0.46 ms).
+// rows of 7168: 1.90 -> 1.70 ms; 32768 x 6 of 5120: 0.54 -> 0.46 ms).  KB is the next of 2, 4, 6 and 8 above k: what is past k
+// requests the last row again (six rows with KB of 8, 32768 x 6 of 5120 between the kernels of the layer: 508 us, of 6: 471).
 template <int MODE, int KB>
 __global__ __launch_bounds__(1024) void combine_kernel(const u32x4* __restrict__ y, const int32_t* __restrict__ pos,
                                                       const int32_t* __restrict__ topk_idx,
@@ -110,6 +111,7 @@ int combine_impl(const void* y, const int32_t* pos, const int32_t* topk_idx, con
     do {                                                 \
         if (top_k <= 2) MOE_LAUNCH_COMBINE(M, 2);        \
         else if (top_k <= 4) MOE_LAUNCH_COMBINE(M, 4);   \
+        else if (top_k <= 6) MOE_LAUNCH_COMBINE(M, 6);   \
         else MOE_LAUNCH_COMBINE(M, 8);                   \
     } while (0)
     if (mode == MOE_COMBINE_F32) MOE_LAUNCH_COMBINE_K(MOE_COMBINE_F32);

@@ -146,3 +146,10 @@ def test_combine_bit_exact(mode, n, k, h, shared):
     torch.cuda.synchronize()
     ref = O.combine(bits(ys), pos, idx, w.numpy(), None if sh is None else bits(sh), mode)
     assert np.array_equal(bits(out), ref), f"max abs diff {np.abs(O.bf16_to_f32(bits(out)) - O.bf16_to_f32(ref)).max()}"
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2])
+@pytest.mark.parametrize("n,k,h,shared", [(9, 5, 1024, True), (9, 6, 576, False), (9, 7, 1024, True), (3, 16, 64, True), (3, 13, 8200, False)])
+def test_combine_of_any_number_of_rows(mode, n, k, h, shared):
+    """Row counts on either side of those that a lane requests at once."""
+    test_combine_bit_exact(mode, n, k, h, shared)
