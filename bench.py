@@ -428,16 +428,13 @@ def run_workload(name: str, args, with_cpu: bool):
     gemm_ms = sum(st.get(k, 0.0) for k in ("routed_gate_up", "routed_down", "shared_gate_up", "shared_down"))
     gemm_tflops = (w.routed_flop + w.shared_flop) / (gemm_ms * 1e-3) / 1e12
     disp_bytes = w.dispatch_bytes if args.materialize else 4.0 * w.n * w.k
-    pair = persistent
     wbytes = 3.0 * w.E * w.h * w.I * (1 if w.fp8 else 2)
     w8 = "true" if w.fp8 else "false"
     if persistent:
         roofline = {"bound": "mfma",
-                    "kernel": f"grouped_gemm_persistent_kernel<SWIGLU=true,W8={w8}> (gate/up + SiLU*mul)"
-                              + (f" + grouped_gemm_kernel<WN=4,SWIGLU=true,W8={w8}> for the "
-                                 + ("rows past an expert's full 256-row tiles" if w.fp8 else "experts of one small tile")
-                                 + " and a short last round of the persistent kernel: a call is this pair of launches, timed as one"
-                                 if pair else ""),
+                    "kernel": f"grouped_gemm_both_kernel<SWIGLU=true,W8={w8}> (gate/up + SiLU*mul): persistent workgroups and, for "
+                              + ("the rows past an expert's full 256-row tiles" if w.fp8 else "experts of one small tile")
+                              + " and a short last round, workgroups of one tile in the same launch",
                     "achieved": achieved, "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
                     "frac": achieved / PEAK_BF16_TFLOPS, "traffic": MEASURED_TRAFFIC.get(name, (None, None))[0],
                     "traffic_source": (f"recorded from {MEASURED_TRAFFIC[name][1]} (rocprofv3 --pmc), not measured by this run"
