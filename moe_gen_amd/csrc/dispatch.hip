@@ -191,6 +191,7 @@ __global__ __launch_bounds__(256) void rank_scatter(const int32_t* __restrict__ 
 // twice, 24576 13.5 and 14.3, 131072 14.0 and 14.9.  Three: 196608 11.9 and 12.6, 524288 14.5 and 16.8 (every entry loaded twice 14.7 and
 // 15.9, 17.9 and 19.8).
 constexpr int SMALL_MAX = 6144;
+constexpr int STATIC_SMALL_MAX = 12288;       // moe_dispatch_static: calls of one workgroup need no scratch and so may overlap
 constexpr int SUM_SEGMENTS = 64;
 
 template <int IT>                            // passes over the list
@@ -225,11 +226,11 @@ namespace {
 
 // The launches behind both entry points; `seg` holds nseg * n_experts per-segment counts.
 int dispatch_launch(const int32_t* topk_idx, int64_t nk, int32_t top_k, int32_t n_experts, const DispatchOut& out, const void* x,
-                    int32_t hidden, void* xs, int32_t* seg, hipStream_t st) {
-    if (nk <= SMALL_MAX) {
+                    int32_t hidden, void* xs, int32_t* seg, int small_max, hipStream_t st) {
+    if (nk <= small_max) {
         constexpr int PASS = 64 * SMALL_WAVES;
-        hipLaunchKernelGGL(nk <= PASS ? dispatch_small<1> : dispatch_small<SMALL_MAX / PASS>, dim3(1), dim3(PASS), 0, st, topk_idx, (int)nk,
-                           n_experts, out, top_k);
+        const auto kernel = nk <= PASS ? dispatch_small<1> : nk <= SMALL_MAX ? dispatch_small<SMALL_MAX / PASS> : dispatch_small<STATIC_SMALL_MAX / PASS>;
+        hipLaunchKernelGGL(kernel, dim3(1), dim3(PASS), 0, st, topk_idx, (int)nk, n_experts, out, top_k);
     } else {
         const int nseg = (int)((nk + SEG - 1) / SEG);
         hipLaunchKernelGGL(block_histogram, dim3(nseg), dim3(256), 0, st, topk_idx, nk, n_experts, seg);
@@ -288,14 +289,14 @@ extern "C" int moe_dispatch(const int32_t* topk_idx, int32_t n_tokens, int32_t t
         return MOE_ERR_WORKSPACE;
     }
     return dispatch_launch(topk_idx, nk, top_k, n_experts, DispatchOut{counts, offsets, perm, pos, row_map, nullptr}, x, hidden, xs,
-                           static_cast<int32_t*>(workspace), st);
+                           static_cast<int32_t*>(workspace), SMALL_MAX, st);
 }
 
 namespace moe {
 int dispatch_on_stream(const int32_t* topk_idx, int32_t n_tokens, int32_t top_k, int32_t n_experts, const DispatchOut& out,
                        void* workspace, hipStream_t st) {
     return dispatch_launch(topk_idx, (int64_t)n_tokens * top_k, top_k, n_experts, out, nullptr, 0, nullptr,
-                           static_cast<int32_t*>(workspace), st);
+                           static_cast<int32_t*>(workspace), SMALL_MAX, st);
 }
 }  // namespace moe
 
@@ -359,7 +360,7 @@ extern "C" int moe_dispatch_static(const int32_t* topk_idx, int32_t n_tokens, in
     rc = static_scratch(&seg);
     if (rc != MOE_OK) return rc;
     return dispatch_launch(topk_idx, nk, top_k, n_experts, DispatchOut{counts, offsets, perm, pos, row_map, nullptr}, x, hidden, xs,
-                           seg, st);
+                           seg, STATIC_SMALL_MAX, st);
 }
 
 // ---- 64-bit words from the host into device memory inside kernel arguments ----
