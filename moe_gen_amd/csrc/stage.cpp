@@ -23,6 +23,7 @@
 //   GPU_Weight_Buffer::clear_expert_buffer    GPU_Weight_Buffer.cpp:261-308  (moe_stage_clear_expert_buffer)
 //   MoE_Gen::set_phase -> resize_buffer       MoE_Gen.cpp:128-134            (moe_stage_set_phase)
 //   MoE_Gen::reset_prefill_buffer / reset_weight_copy_queue   MoE_Gen.cpp:205-211
+#include <atomic>
 #include <condition_variable>
 #include <cstdlib>
 #include <cstring>
@@ -53,6 +54,13 @@ struct Module {
     uint64_t job_seq = 0;        // sequence number of this module's latest bounce job
 };
 
+// Recorded behind what consumers do with the slots they let go (flush_released).  Not recorded again while anyone still has to
+// wait for that record: a wait sees the last one, and another consumer's says nothing about this one's reads.
+struct ReleaseEvent {
+    hipEvent_t ev = nullptr;
+    std::atomic<int> users{0};          // slots and bounce jobs that refer to its last record
+};
+
 struct Type {
     size_t slot_bytes = 0;
     int n_total = 0, n_active = 0;
@@ -61,12 +69,10 @@ struct Type {
     // Hand-back of a slot (device backend).  A release only notes the consumer's stream (freed_pending); the next
     // copy that wants any such slot records ONE event per stream for all slots released since, and each of them then
     // refers to that event (freed_ev) under a ticket that grows with every record.
-    std::vector<hipEvent_t> freed;      // one event object per slot
     std::vector<char> freed_pending;    // released, no event recorded yet
     std::vector<hipStream_t> freed_strm;
-    std::vector<hipEvent_t> freed_ev;   // the event the next copy into the slot waits for (some slot's object)
+    std::vector<ReleaseEvent*> freed_ev;   // the event the next copy into the slot waits for, or null
     std::vector<uint64_t> freed_ticket;
-    std::vector<char> freed_valid;
     std::vector<int> order;             // registration order
     std::deque<int> fifo;               // cyclic copy queue
     int policy = MOE_STAGE_CYCLIC;
@@ -90,7 +96,7 @@ struct BounceJob {
     uint8_t* dst = nullptr;
     std::vector<Piece> pieces;
     hipStream_t stream = nullptr;
-    hipEvent_t wait_for = nullptr;   // release event of the slot's previous user (device backend), or null
+    ReleaseEvent* wait_for = nullptr;   // of the slot's previous user (device backend), or null
     hipEvent_t ready = nullptr;
 };
 
@@ -125,7 +131,11 @@ struct Bounce {
     }
     int run_job(const BounceJob& j) {
         const bool dev = backend == MOE_STAGE_DEVICE;
-        if (dev && j.wait_for) MOE_HIP_CHECK(hipStreamWaitEvent(j.stream, j.wait_for, 0));
+        if (dev && j.wait_for) {
+            const hipError_t e = hipStreamWaitEvent(j.stream, j.wait_for->ev, 0);
+            j.wait_for->users.fetch_sub(1, std::memory_order_release);
+            MOE_HIP_CHECK(e);
+        }
         for (const Piece& p : j.pieces)
             for (size_t off = 0; off < p.bytes; off += chunk_bytes) {
                 const size_t len = std::min(chunk_bytes, p.bytes - off);
@@ -194,6 +204,7 @@ struct moe_stager {
     hipStream_t copy_stream[kCopyStreams] = {};
     std::vector<Type> types;
     std::vector<Module> modules;
+    std::deque<ReleaseEvent> release_events;   // one per slot
     int64_t n_copies = 0, n_bytes = 0;
     int wrap_layers = 0;         // layers [0, wrap_layers) take the last layer as their "previous" one
     int num_hidden_layers = 0, num_local_experts = 0;
@@ -220,6 +231,27 @@ int find_free(const Type& t) {
     return -1;
 }
 
+void drop_event(Type& t, int slot) {
+    if (t.freed_ev[slot]) t.freed_ev[slot]->users.fetch_sub(1, std::memory_order_relaxed);
+    t.freed_ev[slot] = nullptr;
+}
+
+// An event that nobody refers to.  There are as many as slots and a slot that is let go refers to none, so only jobs that the
+// worker has not come to can hold them all.
+int unused_event(moe_stager* st, ReleaseEvent** ev) {
+    for (int pass = 0; pass < 2; ++pass) {
+        for (ReleaseEvent& r : st->release_events)
+            if (r.users.load(std::memory_order_acquire) == 0) {
+                *ev = &r;
+                return MOE_OK;
+            }
+        int rc = st->bounce.wait_issued(st->bounce.enqueued);
+        if (rc != MOE_OK) return rc;
+    }
+    moe::set_error("no release event is free");
+    return MOE_ERR_STATE;
+}
+
 // One event per consumer stream for every slot released since the last call.  A wait that is still pending when a
 // copy is enqueued costs the copy stream about 0.2 ms on this runtime: a wave of ten experts released one by one and
 // refilled one by one, each behind its own event, lost 2.3 ms per wave (272 instead of 211 ms per DeepSeek-V3 layer
@@ -228,14 +260,15 @@ int find_free(const Type& t) {
 int flush_released(moe_stager* st) {
     for (;;) {
         hipStream_t strm = nullptr;
-        hipEvent_t ev = nullptr;
+        ReleaseEvent* ev = nullptr;
         for (Type& t : st->types)
             for (int s = 0; s < t.n_total; ++s) {
                 if (!t.freed_pending[s]) continue;
                 if (!ev) {
                     strm = t.freed_strm[s];
-                    ev = t.freed[s];
-                    MOE_HIP_CHECK(hipEventRecord(ev, strm));
+                    int rc = unused_event(st, &ev);
+                    if (rc != MOE_OK) return rc;
+                    MOE_HIP_CHECK(hipEventRecord(ev->ev, strm));
                     ++st->ticket;
                 } else if (t.freed_strm[s] != strm) {
                     continue;                 // another consumer stream: the next round
@@ -243,7 +276,7 @@ int flush_released(moe_stager* st) {
                 t.freed_pending[s] = 0;
                 t.freed_ev[s] = ev;
                 t.freed_ticket[s] = st->ticket;
-                t.freed_valid[s] = 1;
+                ev->users.fetch_add(1, std::memory_order_relaxed);
             }
         if (!ev) return MOE_OK;
     }
@@ -283,9 +316,9 @@ int copy_into(moe_stager* st, int id, int slot) {
         j.stream = stream;
         j.pieces = m.pieces;
         j.ready = m.ready;
-        if (st->backend == MOE_STAGE_DEVICE && t.freed_valid[slot]) {
-            if (need_wait(st->waited_jobs[si], t.freed_strm[slot], t.freed_ticket[slot])) j.wait_for = t.freed_ev[slot];
-            t.freed_valid[slot] = 0;
+        if (t.freed_ev[slot]) {
+            if (need_wait(st->waited_jobs[si], t.freed_strm[slot], t.freed_ticket[slot])) std::swap(j.wait_for, t.freed_ev[slot]);
+            else drop_event(t, slot);
         }
         {
             std::lock_guard<std::mutex> lk(b.mu);
@@ -295,10 +328,10 @@ int copy_into(moe_stager* st, int id, int slot) {
         }
         b.cv_job.notify_one();
     } else if (st->backend == MOE_STAGE_DEVICE) {
-        if (t.freed_valid[slot]) {
+        if (t.freed_ev[slot]) {
             if (need_wait(st->waited_direct[si], t.freed_strm[slot], t.freed_ticket[slot]))
-                MOE_HIP_CHECK(hipStreamWaitEvent(stream, t.freed_ev[slot], 0));
-            t.freed_valid[slot] = 0;
+                MOE_HIP_CHECK(hipStreamWaitEvent(stream, t.freed_ev[slot]->ev, 0));
+            drop_event(t, slot);
         }
         for (const Piece& p : m.pieces)
             MOE_HIP_CHECK(hipMemcpyAsync(dst + p.dst_off, p.src, p.bytes, hipMemcpyHostToDevice, stream));
@@ -382,7 +415,7 @@ int release_one(moe_stager* st, int id, hipStream_t stream) {
     if (st->backend == MOE_STAGE_DEVICE) {
         t.freed_pending[m.slot] = 1;
         t.freed_strm[m.slot] = stream;
-        t.freed_valid[m.slot] = 0;
+        drop_event(t, m.slot);
     }
     t.owner[m.slot] = -1;
     m.slot = -1;
@@ -456,12 +489,10 @@ extern "C" int moe_stage_create(moe_stager** out, int32_t n_types, const size_t*
         t.n_total = t.n_active = n_slots[i];
         t.mem = static_cast<uint8_t*>(slot_mem[i]);
         t.owner.assign(t.n_total, -1);
-        t.freed.assign(t.n_total, nullptr);
         t.freed_pending.assign(t.n_total, 0);
         t.freed_strm.assign(t.n_total, nullptr);
         t.freed_ev.assign(t.n_total, nullptr);
         t.freed_ticket.assign(t.n_total, 0);
-        t.freed_valid.assign(t.n_total, 0);
     }
     if (backend == MOE_STAGE_DEVICE) {
         hipError_t e = hipSuccess;
@@ -476,7 +507,7 @@ extern "C" int moe_stage_create(moe_stager** out, int32_t n_types, const size_t*
         }
         for (Type& t : st->types)
             for (int s = 0; s < t.n_total; ++s) {
-                e = hipEventCreateWithFlags(&t.freed[s], hipEventDisableTiming);
+                e = hipEventCreateWithFlags(&st->release_events.emplace_back().ev, hipEventDisableTiming);
                 if (e != hipSuccess) {
                     moe::set_error("moe_stage_create: hipEventCreateWithFlags: %s", hipGetErrorString(e));
                     moe_stage_destroy(st);   // releases the streams and the events made so far
@@ -802,9 +833,8 @@ extern "C" int moe_stage_destroy(moe_stager* st) {
             if (s) (void)hipStreamSynchronize(s);
         for (Module& m : st->modules)
             if (m.ready) (void)hipEventDestroy(m.ready);
-        for (Type& t : st->types)
-            for (hipEvent_t ev : t.freed)
-                if (ev) (void)hipEventDestroy(ev);
+        for (ReleaseEvent& r : st->release_events)
+            if (r.ev) (void)hipEventDestroy(r.ev);
         for (hipStream_t s : st->copy_stream)
             if (s) (void)hipStreamDestroy(s);
     }
