@@ -73,6 +73,7 @@ struct Type {
     std::vector<hipStream_t> freed_strm;
     std::vector<ReleaseEvent*> freed_ev;   // the event the next copy into the slot waits for, or null
     std::vector<uint64_t> freed_ticket;
+    std::vector<uint64_t> last_job;     // the latest bounce job into the slot
     std::vector<int> order;             // registration order
     std::deque<int> fifo;               // cyclic copy queue
     int policy = MOE_STAGE_CYCLIC;
@@ -305,6 +306,12 @@ int copy_into(moe_stager* st, int id, int slot) {
         int rc = flush_released(st);
         if (rc != MOE_OK) return rc;
     }
+    if (!m.pageable && t.last_job[slot] > 0) {
+        // a bounce job whose module was let go unread, or taken over, may still be queued: it is not to land on this copy
+        int rc = st->bounce.wait_issued(t.last_job[slot]);
+        if (rc != MOE_OK) return rc;
+        t.last_job[slot] = 0;
+    }
     if (m.pageable) {
         Bounce& b = st->bounce;
         if (b.n_chunks == 0) {
@@ -323,7 +330,7 @@ int copy_into(moe_stager* st, int id, int slot) {
         {
             std::lock_guard<std::mutex> lk(b.mu);
             j.seq = ++b.enqueued;
-            m.job_seq = j.seq;
+            m.job_seq = t.last_job[slot] = j.seq;
             b.jobs.push_back(std::move(j));
         }
         b.cv_job.notify_one();
@@ -493,6 +500,7 @@ extern "C" int moe_stage_create(moe_stager** out, int32_t n_types, const size_t*
         t.freed_strm.assign(t.n_total, nullptr);
         t.freed_ev.assign(t.n_total, nullptr);
         t.freed_ticket.assign(t.n_total, 0);
+        t.last_job.assign(t.n_total, 0);
     }
     if (backend == MOE_STAGE_DEVICE) {
         hipError_t e = hipSuccess;

@@ -26,13 +26,11 @@ def library(tmp_path_factory):
     return so
 
 
-SLOT = 64
-
-
 class Pool:
     """One module type of `slots` slots over the model; a module's bytes are its id.  Notes what every consumer stream read."""
 
-    def __init__(self, library, slots, modules, pageable=(), on_demand=True):
+    def __init__(self, library, slots, modules, pageable=(), on_demand=True, slot_bytes=64):
+        SLOT = self.slot_bytes = slot_bytes
         # a library of its own per pool: the model's streams and log are global
         so = f"{library}.{Pool.count}"
         Pool.count += 1
@@ -70,7 +68,7 @@ class Pool:
         for line in self.L.fake_copies().decode().splitlines():
             head, clock = line.split("|")
             dst, _, stream, number = map(int, head.split())
-            out.append(((dst - self.base) // SLOT, stream, number, dict(map(int, c.split(":")) for c in clock.split())))
+            out.append(((dst - self.base) // self.slot_bytes, stream, number, dict(map(int, c.split(":")) for c in clock.split())))
         return out
 
     def fetch(self, *ids):
@@ -85,7 +83,7 @@ class Pool:
         into = [c for c in self.copies() if c[0] == s]
         clock = dict(map(int, c.split(":")) for c in self.L.fake_clock(stream).decode().split())
         assert all(clock.get(st, 0) >= number for _, st, number, _ in into), f"module {m}: read in front of its copy"
-        assert bytes(self.mem[s * SLOT:(s + 1) * SLOT]) == bytes([m] * SLOT), f"module {m}: slot {s} holds other weights"
+        assert bytes(self.mem[s * self.slot_bytes:(s + 1) * self.slot_bytes]) == bytes([m] * self.slot_bytes), f"module {m}: slot {s} holds other weights"
         self.held[m] = (s, stream, len(into))
         return True
 
@@ -134,12 +132,26 @@ def test_a_shared_release_event_outlives_the_next_release(library, pageable):
     p.close()
 
 
+def test_a_pinned_module_follows_a_queued_copy_into_its_slot(library):
+    """A module of ordinary memory is dropped, or taken over, while the worker has still to copy it: a pinned module that gets its slot
+    is copied behind it, not under it."""
+    p = Pool(library, 1, 2, pageable=(0,), slot_bytes=1 << 18)               # (64 chunks: the worker is still at it)
+    for i in range(6):
+        assert p.fetch(0) == 0
+        p.release(0, B)
+        assert p.acquire(1, A)
+        p.release(1)
+    p.ok(p.L.moe_stage_sync(p.st))
+    p.check()
+    p.close()
+
+
 @pytest.mark.parametrize("seed", range(24))
 def test_random_calls_of_several_consumer_streams(library, seed):
     rng = random.Random(seed)
     modules = 9
-    pageable = {0: (), 1: range(modules)}.get(seed % 2)
-    p = Pool(library, rng.choice([1, 2, 3, 5]), modules, pageable, on_demand=seed % 3 != 0)
+    pageable = ((), range(modules), range(0, modules, 2))[seed % 3]
+    p = Pool(library, rng.choice([1, 2, 3, 5]), modules, pageable, on_demand=seed % 4 != 0)
     for _ in range(120):
         what, m = rng.random(), rng.randrange(modules)
         if what < 0.35 and p.held:
