@@ -30,7 +30,7 @@ class Pool:
     """One module type of `slots` slots over the model; a module's bytes are its id.  Notes what every consumer stream read."""
 
     def __init__(self, library, slots, modules, pageable=(), on_demand=True, slot_bytes=64):
-        SLOT = self.slot_bytes = slot_bytes
+        self.slot_bytes = slot_bytes
         # a library of its own per pool: the model's streams and log are global
         so = f"{library}.{Pool.count}"
         Pool.count += 1
@@ -41,17 +41,17 @@ class Pool:
         L.fake_kernel.restype = ctypes.c_uint64
         for f in ("fake_kernel", "fake_clock"):
             getattr(L, f).argtypes = [ctypes.c_void_p]
-        self.mem = (ctypes.c_uint8 * (slots * SLOT))()
+        self.mem = (ctypes.c_uint8 * (slots * slot_bytes))()
         self.base = ctypes.addressof(self.mem)
         self.st = ctypes.c_void_p()
-        self.ok(L.moe_stage_create(ctypes.byref(self.st), 1, (ctypes.c_size_t * 1)(SLOT), (ctypes.c_int32 * 1)(slots),
+        self.ok(L.moe_stage_create(ctypes.byref(self.st), 1, (ctypes.c_size_t * 1)(slot_bytes), (ctypes.c_int32 * 1)(slots),
                                    (ctypes.c_void_p * 1)(self.base), 0))
         if pageable:
             self.ok(L.moe_stage_set_bounce(self.st, 2, ctypes.c_size_t(4096), 1))
-        self.src = [(ctypes.c_uint8 * SLOT)(*([m] * SLOT)) for m in range(modules)]
+        self.src = [(ctypes.c_uint8 * slot_bytes)(*([m] * slot_bytes)) for m in range(modules)]
         for m in range(modules):
             add = L.moe_stage_add_module_pageable if m in pageable else L.moe_stage_add_module
-            assert add(self.st, 0, 1, (ctypes.c_void_p * 1)(ctypes.addressof(self.src[m])), (ctypes.c_size_t * 1)(SLOT),
+            assert add(self.st, 0, 1, (ctypes.c_void_p * 1)(ctypes.addressof(self.src[m])), (ctypes.c_size_t * 1)(slot_bytes),
                        (ctypes.c_size_t * 1)(0)) == m
         if on_demand:
             self.ok(L.moe_stage_set_policy(self.st, 0, 1))
