@@ -105,6 +105,9 @@ __device__ __forceinline__ void dispatch_one_workgroup(int nk, int E, const Disp
 // ---- launches behind the layer call (each checks its arguments as the entry point of the same name does) ----
 // logits into memory; shared: also its gate and up projection, may be NULL (for kRouterSharedE < E and up to kTailTokens tokens)
 constexpr int kRouterSharedE = 32;
+// workgroups of the logits launch in front of the shared expert's: a block of 32 experts each, for the one block of tokens and seven
+// that find none (workgroups go to the XCDs round robin)
+constexpr int router_shared_front(int E) { return 8 * ((E + 31) / 32); }
 int router_logits(const void* x, const void* w_gate, const moe_router_params& p, float* logits, const SharedFirst* shared, hipStream_t st);
 // routes from them; logits_bf16: also written as bf16 (Mixtral's second result), may be NULL
 int router_select(const float* bias, const moe_router_params& p, int32_t* topk_idx, float* topk_w, float* logits,

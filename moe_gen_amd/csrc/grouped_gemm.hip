@@ -52,6 +52,7 @@
 
 #include "combine_math.h"
 #include "common.h"
+#include "dispatch_small.h"
 #include "layer.h"
 #include "thin_gemm.h"
 
@@ -2747,6 +2748,7 @@ bool layer_may_combine(int32_t n_experts, int32_t n_rows, bool shared, int32_t h
 }
 
 bool layer_shared_first(const moe_mlp_group& routed, const moe_mlp_group& shared, int32_t hidden) {
+    if (router_shared_front(routed.n_experts) + shared_first_blocks(shared.inter) > cu_count()) return false;
     return shared.n_rows > 0 && check_group(routed, hidden, routed.fp8, "moe_layer_forward") == MOE_OK &&
            check_group(shared, hidden, shared.fp8, "moe_layer_forward") == MOE_OK && joins(routed, shared, hidden) &&
            joint_thin(gate_up_args(routed, hidden), routed.n_rows, row_bound(routed), gate_up_args(shared, hidden), shared.n_rows);

@@ -321,7 +321,7 @@ __global__ __launch_bounds__(64 * WT * WE, 1) void router_logits_kernel(
     static_assert(NW * 64 * EJ * 4 <= S * SB, "selection");
     __shared__ float val_own[FUSED && !VAL_IN_STAGES ? NW * 64 * EJ : 1];
     if constexpr (SHARED != 0) {
-        // one wave of the workgroup: the launch has more CUs than such waves, and the workgroup's LDS is its ring
+        // one wave of the workgroup, whose LDS is its ring: the launch has no more workgroups than CUs (layer_shared_first)
         constexpr bool W8 = SHARED == 2;
         constexpr int STAGES = W8 ? 8 : 11;                     // as many as the counter of outstanding loads allows
         static_assert(STAGES * thin_stage_bytes<W8, 2> <= S * SB, "ring");

@@ -222,6 +222,37 @@ def test_layer_call_equals_the_separate_calls(name, E):
                 assert a.dtype == b.dtype and torch.equal(a, b), (n, norm)
 
 
+@pytest.mark.parametrize("E,I,S,fits", [(64, 128, 30, True), (64, 128, 31, False), (64, 256, 32, False), (33, 128, 30, True), (256, 128, 24, True),
+                                        (256, 128, 25, False), (65, 128, 29, True), (65, 128, 30, False)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_wide_shared_expert_next_to_the_router(E, I, S, fits, fp8):
+    """The shared expert's gate and up projection runs in the router's launch while that has at most one workgroup per CU (256): 16 columns
+    each, behind 8 per 32 experts.  On both sides of the line the bits are those of the stage-by-stage path."""
+    import ctypes
+    from moe_gen_amd import _native as N, synthetic
+    from moe_gen_amd.block import StageTimer
+    inter = S * I
+    print(f"wide shared expert E={E} shared={inter} fp8={fp8}", flush=True)
+    first = ctypes.CDLL(N.LIB_PATH)["_ZN3moe18layer_shared_firstERK13moe_mlp_groupS2_i"]
+    first.restype = ctypes.c_bool
+
+    def group(n_experts, width, rows):                       # (the rule reads no memory)
+        g = N.MlpGroup()
+        for f in ("x", "w_gate", "w_up", "w_down", "s_gate", "s_up", "s_down", "offsets", "act", "y"):
+            setattr(g, f, 256)
+        g.x_rows, g.n_rows, g.n_experts, g.inter, g.fp8, g.max_rows = 2, rows, n_experts, width, int(fp8), 2
+        return g
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert first(ctypes.byref(group(E, I, 4)), ctypes.byref(group(1, inter, 2)), 512) == fits
+    w = synthetic.WORKLOADS["deepseek_v2_lite"].scaled(n=2, h=512, I=I, S=S, seq=2, E=E, k=2, n_group=1, topk_group=1, fp8=fp8)
+    blk = synthetic.build_block(w, device="cuda", gen_device="cpu")
+    x = synthetic.hidden_states(w, "cpu").cuda()
+    blk.stage_timer = StageTimer()
+    want = blk(x).clone()
+    blk.stage_timer = None
+    assert torch.equal(blk(x), want)
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("name,E,k,h", [("deepseek_v2_lite", 64, 6, 1024), ("deepseek_v2_lite", 17, 3, 576), ("deepseek_v3_w8a16", 256, 8, 384),
                                         ("mixtral_8x7b", 8, 2, 512), ("mixtral_8x7b", 8, 8, 256), ("deepseek_v2_lite", 33, 16, 256),
