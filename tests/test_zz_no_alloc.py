@@ -59,9 +59,32 @@ def test_static_dispatch_matches_dispatch_on_consecutive_calls():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("nk", [1024, 1025, 6144, 6145, 12288, 12289])
+@pytest.mark.parametrize("E", [1, 64, 256])
+def test_static_dispatch_where_its_forms_change(nk, E):
+    """One workgroup with one, six and twelve passes over the list, and two launches, on both sides of each limit, ids outside [0, E) among
+    them, against a stable sort."""
+    print(f"no-alloc dispatch {nk}/{E}", flush=True)
+    rng = np.random.default_rng(nk + E)
+    ids = rng.integers(0, E, nk).astype(np.int32)
+    bad = rng.random(nk) < 0.02
+    ids[bad] = rng.choice(np.array([-1, E, E + 7, 2 ** 31 - 1, -2 ** 31], dtype=np.int64), bad.sum()).astype(np.int32)
+    counts, offsets, perm, pos, row_map, _ = (None if t is None else t.cpu().numpy() for t in
+                                              _run("moe_dispatch_static", torch.from_numpy(ids.reshape(nk, 1)).cuda(), E))
+    good = np.flatnonzero(~bad)
+    order = good[np.argsort(ids[good], kind="stable")]
+    want = np.bincount(ids[good], minlength=E)
+    assert np.array_equal(counts, want) and np.array_equal(offsets, np.concatenate([[0], np.cumsum(want)]))
+    assert np.array_equal(perm[:len(order)], order) and np.array_equal(row_map[:len(order)], order)
+    where = np.full(nk, -1, dtype=np.int32)
+    where[order] = np.arange(len(order))
+    assert np.array_equal(pos, where)
+
+
+@pytest.mark.gpu
 def test_static_dispatch_captured_in_a_graph():
     """The use the entry point is documented for: after one eager call on the device (which looks the array's
-    address up), further calls are captured into a HIP graph -- three kernel launches, no allocation, no memset --
+    address up), further calls are captured into a HIP graph -- two kernel launches, no allocation, no memset --
     and every replay, with the program's own eager work and synchronisations in between and with new routing in the
     same buffers, gives what moe_dispatch gives eagerly."""
     n, k, E = 5000, 6, 160
