@@ -2748,6 +2748,7 @@ bool layer_may_combine(int32_t n_experts, int32_t n_rows, bool shared, int32_t h
 }
 
 bool layer_shared_first(const moe_mlp_group& routed, const moe_mlp_group& shared, int32_t hidden) {
+    if (hidden < (routed.fp8 ? 6144 : 2048)) return false;
     if (router_shared_front(routed.n_experts) + shared_first_blocks(shared.inter) > cu_count()) return false;
     return shared.n_rows > 0 && check_group(routed, hidden, routed.fp8, "moe_layer_forward") == MOE_OK &&
            check_group(shared, hidden, shared.fp8, "moe_layer_forward") == MOE_OK && joins(routed, shared, hidden) &&

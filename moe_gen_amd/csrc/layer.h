@@ -34,12 +34,15 @@ struct SharedFirst {
 };
 constexpr int shared_first_blocks(int inter) { return (inter + 15) / 16; }
 
-// Whether it may run there: the thin kernel then serves the call, whose gate and up launch leaves it out.  One workgroup per CU is the
-// line, those of the router that find no tokens counted: a workgroup is one wave that streams, in an LDS of 70 KiB, and past it a
-// CU has a second one to wait for, where the thin kernel runs six.  Layers, us, in the routed experts' launch -> here, 1 and 8 tokens: 64 fp8
-// experts (16 workgroups in front), shared 3840 wide 89 / 122 -> 90 / 112, 3968 90 / 114 -> 114 / 129, 16384 204 / 394 -> 219 / 419; 256
-// (64), 3072 90 / 138 -> 91 / 136, 3584 92 / 140 -> 116 / 160; DeepSeek-V2-236B's router (40) and bf16, 3072 73 / 97 -> 70 / 86, 3584 74 / 98 ->
-// 86 / 100.
+// Whether it may run there: the thin kernel then serves the call, whose gate and up launch leaves it out.
+//  * One workgroup per CU is the line, those of the router that find no tokens counted: a workgroup is one wave that streams, in an LDS of
+//    70 KiB, and past it a CU has a second one to wait for, where the thin kernel runs six.  Layers, us, in the routed experts' launch ->
+//    here, 1 and 8 tokens: 64 fp8 experts (16 workgroups in front), shared 3840 wide 89 / 122 -> 90 / 112, 3968 90 / 114 -> 114 / 129, 16384
+//    204 / 394 -> 219 / 419; 256 (64), 3072 90 / 138 -> 91 / 136, 3584 92 / 140 -> 116 / 160; DeepSeek-V2-236B's router (40) and bf16,
+//    3072 73 / 97 -> 70 / 86, 3584 74 / 98 -> 86 / 100.
+//  * And the router has to take long enough: its chain grows with the hidden size, a shared wave of few stages is mostly its own start.
+//    Graph replays of 9 layers of 1 to 16 tokens each, ratio: bf16, hidden size 512 1.037, 1024 1.016, 1536 0.992, 2048 0.983, 4096 and more
+//    0.97; fp8 512 1.049, 2048 1.027, 4096 1.015, 5120 1.000, 7168 0.992.
 bool layer_shared_first(const moe_mlp_group& routed, const moe_mlp_group& shared, int32_t hidden);
 
 // moe_grouped_swiglu_joint, both phases (shared may be NULL), as a part of a layer call

@@ -223,16 +223,16 @@ def test_layer_call_equals_the_separate_calls(name, E):
 
 
 @pytest.mark.parametrize("E,I,S,fits", [(64, 128, 30, True), (64, 128, 31, False), (64, 256, 32, False), (33, 128, 30, True), (256, 128, 24, True),
-                                        (256, 128, 25, False), (65, 128, 29, True), (65, 128, 30, False)])
+                                        (256, 128, 25, False), (65, 128, 29, True), (65, 128, 30, False), (40, 128, 1, True)])
 @pytest.mark.parametrize("fp8", [False, True])
-def test_wide_shared_expert_next_to_the_router(E, I, S, fits, fp8):
+def test_shared_expert_next_to_the_router(E, I, S, fits, fp8):
     """The shared expert's gate and up projection runs in the router's launch while that has at most one workgroup per CU (256): 16 columns
-    each, behind 8 per 32 experts.  On both sides of the line the bits are those of the stage-by-stage path."""
+    each, behind 8 per 32 experts; and from a hidden size of 2048 on, 6144 with fp8 weights.  On both sides of these lines the bits are those
+    of the stage-by-stage path, also from a graph."""
     import ctypes
     from moe_gen_amd import _native as N, synthetic
     from moe_gen_amd.block import StageTimer
-    inter = S * I
-    print(f"wide shared expert E={E} shared={inter} fp8={fp8}", flush=True)
+    inter, line = S * I, 6144 if fp8 else 2048
     first = ctypes.CDLL(N.LIB_PATH)["_ZN3moe18layer_shared_firstERK13moe_mlp_groupS2_i"]
     first.restype = ctypes.c_bool
 
@@ -243,14 +243,29 @@ def test_wide_shared_expert_next_to_the_router(E, I, S, fits, fp8):
         g.x_rows, g.n_rows, g.n_experts, g.inter, g.fp8, g.max_rows = 2, rows, n_experts, width, int(fp8), 2
         return g
     if torch.cuda.get_device_properties(0).multi_processor_count == 256:
-        assert first(ctypes.byref(group(E, I, 4)), ctypes.byref(group(1, inter, 2)), 512) == fits
-    w = synthetic.WORKLOADS["deepseek_v2_lite"].scaled(n=2, h=512, I=I, S=S, seq=2, E=E, k=2, n_group=1, topk_group=1, fp8=fp8)
-    blk = synthetic.build_block(w, device="cuda", gen_device="cpu")
-    x = synthetic.hidden_states(w, "cpu").cuda()
-    blk.stage_timer = StageTimer()
-    want = blk(x).clone()
-    blk.stage_timer = None
-    assert torch.equal(blk(x), want)
+        for h, pays in ((line, True), (line - 128, False), (2 * line, True)):
+            assert first(ctypes.byref(group(E, I, 4)), ctypes.byref(group(1, inter, 2)), h) == (fits and pays), h
+    w = synthetic.WORKLOADS["deepseek_v2_lite"].scaled(n=17, h=line, I=I, S=S, seq=17, E=E, k=2, n_group=1, topk_group=1, fp8=fp8)
+    blk = synthetic.build_block(w, device="cuda")
+    xs = synthetic.hidden_states(w, "cpu").cuda()
+    for n in (1, 2, 16, 17):
+        print(f"shared expert next to the router E={E} shared={inter} fp8={fp8} n={n}", flush=True)
+        x = xs[:, :n].contiguous()
+        blk.stage_timer = StageTimer()
+        want = blk(x).clone()
+        blk.stage_timer = None
+        assert torch.equal(blk(x), want)
+        if n != 2:
+            continue
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            got = blk(x)
+        for _ in range(3):
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(got, want)
+            assert torch.equal(blk(x), want)
 
 
 @pytest.mark.parametrize("fp8", [False, True])
