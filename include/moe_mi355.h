@@ -231,9 +231,9 @@ typedef struct moe_mlp_group {
 
 /*
  * Device scratch with which a group runs faster, 0 if none does: ONE fp8 MLP (n_experts 1) with a long intermediate size whose
- * down projection has too few tiles for the chip (DeepSeek-V3's dense layers, up to 1536 rows) gives every tile of it to several
- * workgroups, which leave their fp32 sums here.  Without it, or with less, the call runs as the two above.  A row's bits may differ
- * between the two by the order of its sums.
+ * down projection has too few tiles for the chip (DeepSeek-V3's dense layers: up to 1024 rows and from 1217 to 1536) gives every tile
+ * of it to several workgroups, which leave their fp32 sums here.  Without it, or with less, the call runs as the two above.  A row's
+ * bits may differ between the two by the order of its sums.
  */
 size_t moe_mlp_workspace_bytes(const moe_mlp_group* group, int32_t hidden);
 

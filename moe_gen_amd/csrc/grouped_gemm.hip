@@ -1690,7 +1690,7 @@ __global__ __launch_bounds__(64) void grouped_gemm_thin_kernel(GemmPair pair_of,
 // workgroup each, so that tiles x slices fill the CUs once; the fp32 sums of the slices go to the workspace and
 // add_slices_kernel adds them, in order, and rounds once.  Rows past 128 are cut into tiles of equal height; all tiles of a
 // call run the same body, chosen by that height, so a row's bits do not depend on its place.  The M tiles of one piece of
-// the weights are neighbours on one XCD.  (From 257 rows on the slices run as 256-row tiles of the persistent kernel, split_plan.)
+// the weights are neighbours on one XCD.  (From 257 rows on they may run as 256-row tiles of the persistent kernel instead, split_plan.)
 // Measured (DeepSeek-V3's dense MLP, both launches, us, without scratch -> with it): 1 token 119 -> 75, 17: 185 -> 87,
 // 64: 231 -> 115, 128: 356 -> 161, 192: 516 -> 220, 256: 426 -> 273; of those the gate and up products take 49, 58, 76, 104, 150
 // and 186.
@@ -2417,43 +2417,51 @@ inline bool gather_fits(const GemmArgs& g) { return !g.row_map || g.a_bytes < (1
 // that what the slices save outweighs their sums' way through memory, and where its own tiles leave CUs idle.
 //  * up to 256 rows on the split kernel: as many slices as fill the CUs once, of 8 blocks or more (a shorter k loop is mostly
 //    its own start), at most 16.
-//  * above, up to a round of 256-row tiles, on the persistent kernel: the number of slices whose rounds and sums cost least, a
-//    round of one block counted 3.0 us and the sums 6 us and 0.45 us per MB, if that is less than what the call takes
-//    uncut (0.6 of a round of whole tiles where half tiles go round once, else 0.88).
-// DeepSeek-V3's dense MLP (28 column tiles, 144 blocks), down projection, us, uncut or on the split kernel (up to 512 rows) -> this:
-// 300 rows 154 -> 129, 512: 146 -> 130, 520: 227 -> 171, 768: 232 -> 181, 800: 243 -> 245, 1000: 264 -> 248, 1300: 365 -> 351, 1536:
-// 383 -> 352; 2 rounds of whole tiles and more gain 6 % at most (3000 rows 724 -> 683, 2600: 652 -> 647, 4000: 871 -> 922).
+//  * above, up to a round of 256-row tiles, whichever of three takes least by these counts (us), each at its best number of slices: uncut,
+//    1.55 a block of k while the pieces leave a third of the CUs idle, 15 % more up to a round of them and 60 % beyond; the split
+//    kernel, one round, 0.9 + 0.0055 a row of its tiles a block and 0.37 per MB of sums; the persistent kernel's 256-row tiles, 2.8
+//    a block, 20 a further round and 0.16 per MB.  The split kernel's lower tiles win where slices are short or tiles few.
+// Measured: h of 1024 to 8192, k of 4096 to 18432, 257 to 3000 rows, all three at every number of slices: the counts are within 12 %
+// and the choice 0.5 % behind the best of them in the mean, 5 % at most.  Down projection, us, uncut / split kernel / 256-row tiles:
+// h 7168, k 18432, 257 rows 212 / 112 / 121, 400: 238 / 133 / 125, 640: 216 / - / 170, 1000: 264 / - / 231, 1300: 360 / - / 340;
+// 4096, 14336, 257: 164 / 50 / 63, 768: 167 / 102 / 91; 2048, 5632, 257: 72 / 24 / 40, 1000: 71 / 37 / 44; 1024, 4096, 1000: 55 / 26 / 40.
 SplitPlan split_plan(int n_rows, int K, int n_tiles_n) {
     const int nblk = K / 128, cus = cu_count();
     if (nblk < 32 || n_rows < 1 || cus < 8) return SplitPlan{};
-    if (n_rows > 256) {
-        const int m = (n_rows + 255) / 256, left = n_rows & 255;
-        const long tiles = (long)m * n_tiles_n;
-        if (tiles > cus) return SplitPlan{};
-        const bool own = left > 0 && left <= 192;                    // (uncut, these rows are tiles of the other kernel)
-        const long pieces = (2 * (m - (own ? 1 : 0)) + (own ? 1 : 0)) * (long)n_tiles_n;
-        double best = nblk * 3.0 * (pieces <= cus ? 0.6 : 0.88);
-        SplitPlan plan{};
-        for (int s = 2; s <= 16 && nblk / s >= 8; ++s) {
-            const int blocks = (nblk + s - 1) / s, slices = (nblk + blocks - 1) / blocks;
-            const double rounds = (double)((tiles * slices + cus - 1) / cus);
-            const double us = rounds * blocks * 3.0 + 6.0 + 0.45e-6 * slices * n_rows * (double)n_tiles_n * 1024;
-            if (us < best) {
-                best = us;
-                plan = SplitPlan{m, 256, slices, blocks};
-            }
-        }
-        return plan;
-    }
     int m = (n_rows + 127) / 128;
     const int rows = m <= 1 ? n_rows : ((n_rows + m - 1) / m + 15) / 16 * 16;
-    if ((long)m * n_tiles_n * 2 > cus) return SplitPlan{};
+    if (n_rows <= 256) {
+        if ((long)m * n_tiles_n * 2 > cus) return SplitPlan{};
+        m = (n_rows + rows - 1) / rows;
+        int s = cus / (m * n_tiles_n);
+        s = s < nblk / 8 ? s : nblk / 8;
+        s = s < 16 ? s : 16;
+        const int blocks = (nblk + s - 1) / s;
+        return SplitPlan{m, rows, (nblk + blocks - 1) / blocks, blocks};
+    }
     m = (n_rows + rows - 1) / rows;
-    int s = cus / (m * n_tiles_n);
-    s = s < nblk / 8 ? s : nblk / 8;
-    s = s < 16 ? s : 16;
-    const int blocks = (nblk + s - 1) / s;
-    return SplitPlan{m, rows, (nblk + blocks - 1) / blocks, blocks};
+    const int m256 = (n_rows + 255) / 256, left = n_rows & 255;
+    const long tiles = (long)m256 * n_tiles_n;
+    if (tiles > cus) return SplitPlan{};
+    const bool own = left > 0 && left <= 192;                        // (uncut, these rows are a tile of a workgroup of its own)
+    const long pieces = (2 * (m256 - (own ? 1 : 0)) + (own ? 1 : 0)) * (long)n_tiles_n;
+    double best = 4.0 + 1.55 * nblk * (3 * pieces <= 2 * cus ? 1.0 : pieces <= cus ? 1.15 : 1.6);
+    SplitPlan plan{};
+    auto consider = [&](double us, const SplitPlan& p) {
+        if (us < best) {
+            best = us;
+            plan = p;
+        }
+    };
+    for (int s = 2; s <= 16 && nblk / s >= 8; ++s) {
+        const int blocks = (nblk + s - 1) / s, slices = (nblk + blocks - 1) / blocks;
+        const double mb = 1e-6 * slices * n_rows * (double)n_tiles_n * 1024;
+        if (((long)slices * n_tiles_n + 7) / 8 * 8 * m <= cus)
+            consider(8.0 + blocks * (0.9 + 0.0055 * rows) + 0.37 * mb, SplitPlan{m, rows, slices, blocks});
+        const long rounds = (tiles * slices + cus - 1) / cus;
+        consider(16.0 + 20.0 * (rounds - 1) + 2.8 * rounds * blocks + 0.16 * mb, SplitPlan{m256, 256, slices, blocks});
+    }
+    return plan;
 }
 
 int launch_split(const GemmArgs& g, int n_rows, const SplitPlan& plan, float* part, hipStream_t st) {

@@ -1066,6 +1066,47 @@ def test_dense_fp8_down_projection_in_slices_of_k(h, I):
         assert torch.equal(down(act[perm].contiguous(), need), y[perm])
 
 
+@pytest.mark.parametrize("h,I,n,slices", [
+    (1024, 4224, 257, 4),       # the split kernel past 256 rows, its last slice 6 of 9 blocks
+    (1024, 4096, 2000, 4),      # sixteen row tiles of it
+    (2048, 5632, 900, 4), (4096, 14336, 257, 5), (7168, 18432, 257, 2),
+    (7168, 5248, 640, 3),       # 256-row tiles, slices of 14, 14 and 13 blocks
+    (4096, 14336, 768, 5), (7168, 18432, 400, 4)])
+def test_dense_fp8_slices_past_256_rows(h, I, n, slices):
+    """Past 256 rows the down projection of an fp8 MLP is cut on the kernel and into the slices that take least (the number of slices
+    is what the scratch is asked for): against float64 on the dequantised weights, nothing past the scratch, and a row's bits
+    independent of its place."""
+    import ctypes
+    from moe_gen_amd import _native as N, ops
+    from moe_gen_amd.synthetic import quantize_fp8_block128
+    print(f"slices past 256 rows h={h} I={I} n={n}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(n + h)
+    q, sc = quantize_fp8_block128(torch.randn(h, I, generator=g, device="cuda") * 0.02)
+    qi, si = torch.zeros(I, h, device="cuda").to(torch.float8_e4m3fn), torch.ones(I // 128, h // 128, device="cuda")
+    ptrs = ops.expert_pointers([qi], [qi], [q], [si], [si], [sc])
+    off = torch.tensor([0, n], dtype=torch.int32, device="cuda")
+    act = torch.randn(n, I, generator=g, device="cuda").to(torch.bfloat16)
+
+    def down(a):
+        y = torch.full((n, h), 3.0, dtype=torch.bfloat16, device="cuda")
+        m, _, _ = ops.mlp_group(torch.zeros(n, h, dtype=torch.bfloat16, device="cuda"), None, ptrs, off, n, n, act=a, y=y)
+        need = N.lib().moe_mlp_workspace_bytes(ctypes.byref(m), h)
+        if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+            assert need == 4 * slices * n * h
+        ws = torch.full((need // 4 + 64,), 7.0, device="cuda")
+        m.workspace, m.workspace_bytes = ws.data_ptr(), need
+        ops.grouped_swiglu_joint(m, None, h, True, ops.PHASE_DOWN)
+        assert (ws[need // 4:] == 7.0).all()
+        return y
+    y = down(act)
+    wd = q.double() * sc.double().repeat_interleave(128, 0).repeat_interleave(128, 1)
+    ref = act.double() @ wd.t()
+    # weights and result are each rounded to bf16: relative 2^-9 at most, independent per element
+    assert (y.double() - ref).norm() <= 2.0 ** -8 * ref.norm()
+    perm = torch.randperm(n, generator=torch.Generator().manual_seed(n)).cuda()
+    assert torch.equal(down(act[perm].contiguous()), y[perm])
+
+
 @pytest.mark.parametrize("n,first,rows", [
     (1300, 0, 1300),        # slices of more than a round of tiles
     (1000, 40, 700),        # fewer rows than the host allows for, behind other rows: fewer row tiles, the last one ragged
