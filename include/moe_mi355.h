@@ -145,7 +145,7 @@ int moe_dispatch_static(const int32_t* topk_idx, int32_t n_tokens, int32_t top_k
  *             row_map != NULL, the unsorted matrix, row r being x[row_map[r]]
  *   x_rows    rows of x (>= 1).  It bounds the gather: a row_map entry outside [0, x_rows) stands for a
  *             row of zeros (where rows are fetched through a buffer descriptor with 32-bit offsets -- the
- *             persistent kernel, below -- an entry whose byte offset wraps 32 bits reads some row of x
+ *             persistent workgroups, below -- an entry whose byte offset wraps 32 bits reads some row of x
  *             instead), never memory outside x.  Without row_map it only has to cover the rows the
  *             call reads
  *   row_map   device int32 [n_rows] or NULL
@@ -162,20 +162,20 @@ int moe_dispatch_static(const int32_t* topk_idx, int32_t n_tokens, int32_t top_k
  *             scratch; NULL / 0 is accepted (moe_grouped_workspace_bytes reports the reserve)
  *   phases    MOE_PHASE_GATE_UP (writes act), MOE_PHASE_DOWN (reads act, writes y) or
  *             MOE_PHASE_BOTH; the two launches can be issued (and timed) separately
- * Requires h % 64 == 0 and I % 64 == 0, 1 <= E <= 1024.  Two kernels share a call: experts that fit one tile of
+ * Requires h % 64 == 0 and I % 64 == 0, 1 <= E <= 1024.  Two kinds of tiles share a launch: experts that fit one tile of
  * up to 192 rows run one workgroup per tile, at a tile height chosen per expert on the device in steps of 16 rows
  * (bf16 weights: also experts of 257 to 384 rows, as two such tiles);
  * larger experts run on 256-row tiles of persistent workgroups (with fp8 weights: their full 256-row tiles, and the
  * rows these leave over as one tile of the first kind if they are at most 192; those of a single expert, E = 1, as a padded tile
  * of the second kind where that shortens the call).  The persistent workgroups,
- * one per CU, take whole rounds of tiles; a last, partial round is cut into 128-row halves and runs with the first
- * kind when that shortens the two launches (alone: if it is at most half the CUs' worth of tiles).  Below a mean of 128 rows per expert (n_rows / E), with K not a multiple of
- * 128, with more than 512 experts or with 4 GiB or more of gathered x, the one-workgroup-per-tile kernel serves the
- * call alone (larger experts cut into 128-row tiles).  With bf16 weights an output row's bits depend on the row and its
+ * one per CU, take whole rounds of tiles; a last, partial round is cut into 128-row halves, which join the first kind, when that
+ * shortens the rounds of both (alone: if it is at most half the CUs' worth of tiles).  Below a mean of 128 rows per expert
+ * (n_rows / E), with K not a multiple of 128, with more than 512 experts or with 4 GiB or more of gathered x, all tiles are of the
+ * first kind (larger experts cut into 128-row tiles).  With bf16 weights an output row's bits depend on the row and its
  * expert's weights alone, never on the row's place among its expert's rows, on any expert's count, on the kernel that
- * computes it or on the call.  With fp8 weights that holds inside a call that launches both kernels, and two things
- * change the order in which a row's products are added, and with it the last bit: a call that the
- * one-workgroup-per-tile kernel serves alone starts its k loops at other stages, and there an expert of up to 64 rows
+ * computes it or on the call.  With fp8 weights that holds inside a call with both kinds of tiles, and two things
+ * change the order in which a row's products are added, and with it the last bit: a call of the first kind
+ * alone starts its k loops at other stages, and there an expert of up to 64 rows
  * adds the products of a stage in another order than one of more.  (The scratch of moe_mlp_workspace_bytes changes it too.)
  * Calls in which no expert has more than 16 rows run on a kernel of one wave per 32 weight rows where that is the faster one.
  */

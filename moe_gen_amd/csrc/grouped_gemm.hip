@@ -15,32 +15,31 @@
 // expert is cut into M tiles (the last one partial); an M tile times an N tile of the
 // weight matrix is one unit of work.  Every workgroup rebuilds the (tiny) M-tile prefix
 // over experts in LDS from offsets[], so a launch needs neither a host sync nor a tile table.
-// Two kernels, and a call usually launches both (launch_mt): every expert goes by its own count, which both
-// kernels read from offsets[]; each builds the prefix over its own share of the tiles.
-//  * grouped_gemm_persistent_kernel (experts above one small tile; with fp8 weights the full 256-row
-//    tiles of every expert): 256-row tiles, one
-//    workgroup per CU, groups of 32 consecutive tiles go round-robin to the XCDs (workgroup
-//    ids are dealt to the 8 XCDs one by one by the hardware; the tiles of a group share their
-//    A and B panels through that XCD's L2), and a workgroup's k pipeline runs on from one of
-//    its tiles into the next.
-//  * grouped_gemm_kernel (experts of up to 192 rows, and with fp8 weights what an expert's full 256-row tiles
-//    leave over if that is at most 192 rows, a single MLP's where a padded tile of the other kernel is not the
-//    shorter way; work that mostly streams weights): one workgroup per tile, grid = upper bound on the tile count,
-//    surplus workgroups exit at once;
-//    the tile height (16 ... 192 rows in steps of 16) follows the expert, groups of 4 tiles go round-robin
-//    to the XCDs.  Its tiles run through the weight streamers (stream16_tile, stream8x_tile, stream8_tile):
-//    weights AND token rows reach LDS by DMA, three weight buffers, one barrier per stage.
+// Two kinds of tiles; which kind an expert's rows are follows its own count, which every workgroup reads from offsets[]
+// (both_kernels, launch_mt):
+//  * persistent tiles (persistent_body): experts above one small tile, with fp8 weights the full 256-row tiles of every expert.  256
+//    rows, one workgroup per CU; groups of 32 consecutive tiles go round-robin to the XCDs (workgroup ids are dealt to the 8 XCDs
+//    one by one by the hardware; the tiles of a group share their A and B panels through that XCD's L2), and a workgroup's k
+//    pipeline runs on from one of its tiles into the next.
+//  * tiles of one workgroup each: experts of up to 192 rows, and with fp8 weights what an expert's full 256-row tiles leave over if that
+//    is at most 192 rows, a single MLP's where a padded persistent tile is not the shorter way; work that mostly streams weights.  The
+//    grid is an upper bound on the tile count, surplus workgroups exit at once; the tile height (16 ... 192 rows in steps of 16)
+//    follows the expert.  They run through the weight streamers (stream16_tile, stream8x_tile, stream8_tile): weights AND token
+//    rows reach LDS by DMA, three weight buffers, one barrier per stage.
+// Kernels: grouped_gemm_both_kernel has both kinds in one launch, the persistent workgroups first (calls of a mean of 128 rows per
+// expert or more); grouped_gemm_kernel one-workgroup tiles alone (fewer rows, and what the persistent body cannot address);
+// grouped_gemm_thin_kernel waves of 16 columns (up to 16 rows per expert); the split kernels slices of k of one fp8 MLP.
 //
 // Workgroup = 8 waves, two per SIMD.  v_mfma_f32_16x16x32_bf16 throughout: on real (non-zero) data this
 // chip is power-limited under MFMA load; the 16x16x32 shape moves a third less accumulator data per flop
 // than 32x32x16 and sustains ~13 % more (1.95 vs 1.73 PFLOP/s in a registers-only loop with random
-// operands), which is worth ~6 % here.  The persistent kernel's waves are 2 along M x 4 along N, 8 x 4 MFMA
+// operands), which is worth ~6 % here.  The persistent body's waves are 2 along M x 4 along N, 8 x 4 MFMA
 // tiles each (128x64 outputs, 128 fp32 accumulators).  K advances 64 at a time through two LDS stages; rows
 // are 128 bytes with a 16-byte-chunk XOR swizzle so that both the 16-byte stores and the 16-byte MFMA
 // operand reads are bank-conflict free.  Token rows and bf16 weights come into LDS by DMA
-// (buffer_load ... lds); fp8 weights of the persistent kernel go through registers, converted on the way,
+// (buffer_load ... lds); fp8 weights of the persistent body go through registers, converted on the way,
 // two k-stages ahead, every wave interleaving its share of that with its MFMAs, one piece per group of
-// MFMAs, between the two barriers per k-stage.  gemm_tile, the register-staged body of the other kernel,
+// MFMAs, between the two barriers per k-stage.  gemm_tile, the register-staged body of one-workgroup tiles,
 // remains for calls that gather from 4 GiB of rows or more (the DMA paths address them with 32 bits).
 //
 // The MFMA is issued with the WEIGHT fragment as srcA and the TOKEN fragment as srcB, so
@@ -94,23 +93,23 @@ struct GemmArgs {
     int cold_max;               // experts of up to this many rows are tiles of one workgroup each, the others tiles of the
                                 // persistent workgroups (0: all are)
     int rem_split;              // 1: the rule applies to what an expert's full 256-row tiles leave over (count % 256)
-                                // instead of to its count: the persistent kernel takes the full tiles, and the
-                                // last, ragged one only if it holds more than cold_max rows
-    int pair_rows;              // 1: experts of PAIR_LO .. PAIR_HI rows also belong to the one-workgroup-per-tile kernel
-    int alone;                  // 1 (fp8): no other kernel's sums have to be matched: k_rotation, and the stage order of
+                                // instead of to its count: the full tiles are persistent ones, and so is the
+                                // last, ragged one if it holds more than cold_max rows
+    int pair_rows;              // 1: experts of PAIR_LO .. PAIR_HI rows are tiles of one workgroup each too
+    int alone;                  // 1 (fp8): no persistent tile's sums have to be matched: k_rotation, and the stage order of
                                 // stream8_tile for tiles of up to 64 rows
-    int tail_cus;               // > 0: the persistent kernel runs whole rounds of this many tiles (one per CU); what
-                                // is left goes to the other kernel as 128-row half tiles if that pays (tail_tiles)
+    int tail_cus;               // > 0: the persistent workgroups run whole rounds of this many tiles (one per CU); what
+                                // is left goes to workgroups of 128-row half tiles if that pays (tail_tiles)
 };
 
 // What a launch works on: the routed experts and a second problem of one expert with matrices, sizes and buffers of its own,
 // the layer's shared expert.  A launch pair for the shared expert alone has a tile for a fraction of the CUs at small batches
 // (DeepSeek-V2-236B, 64 tokens: 24 and 20 tiles, 70 + 44 us for 94 MB) and rounds of its own that end part-filled at larger ones.
 // The host knows a bound of its rows, the kernels its rows (offsets[], like every expert's):
-//  * one kernel serves the call: `shared_tiles` workgroups in front of the routed experts' are the shared expert's; those past
+//  * a call of one kind of tiles: `shared_tiles` workgroups in front of the routed experts' are the shared expert's; those past
 //    its rows return at once.
-//  * both kernels do: `shared_rows` > 0 bounds its rows, and each kernel counts its tiles as it does any expert's (persistent
-//    kernel: in front of the routed experts'; the other one: behind them, in front of the half tiles).
+//  * a call of both: `shared_rows` > 0 bounds its rows, and its tiles are counted as any expert's (persistent ones in front of the
+//    routed experts'; one-workgroup tiles behind them, in front of the half tiles).
 struct GemmPair {
     GemmArgs p[2];              // routed, shared
     int shared_tiles, shared_rows;
@@ -120,19 +119,18 @@ struct GemmPair {
 // their N tile; started at the same stage, their requests in flight would share the low address bits (rows of the weight
 // matrices are K elements apart) and crowd the same memory channels: with the start spread over the stages a launch
 // that streams weights gains about a tenth (Mixtral-8x22B shapes, 8 experts x 16 ... 120 rows: 6.1 -> 6.8, 5.4 -> 6.1
-// TB/s; 128 / 160 / 192 rows next to the persistent kernel: gate/up 0.63 / 0.64 / 0.66 -> 0.55 / 0.58 / 0.62 ms).
-// bf16 weights: every path of both kernels uses this rule, so which kernel or tile computes a row does not change the
-// order its products are added in (the persistent kernel itself runs within 0.5 % either way).  fp8 weights (a scale
-// per 128 k: pairs of stages stay together): only in calls that the one-workgroup-per-tile kernel serves alone (and not for
-// a large shared expert in them, joint_alone); the persistent kernel loses 1.6 % of the DeepSeek-V3 step to a rotated
-// walk, so calls that launch it start every tile at stage 0, in both kernels.
+// TB/s; 128 / 160 / 192 rows next to persistent tiles: gate/up 0.63 / 0.64 / 0.66 -> 0.55 / 0.58 / 0.62 ms).
+// bf16 weights: every path uses this rule, so which kernel or tile computes a row does not change the order its products are
+// added in (the persistent body itself runs within 0.5 % either way).  fp8 weights (a scale per 128 k: pairs of stages stay
+// together): only in calls of one-workgroup tiles alone (and not for a large shared expert in them, joint_alone); the persistent
+// body loses 1.6 % of the DeepSeek-V3 step to a rotated walk, so calls with persistent tiles start every tile at stage 0.
 template <bool W8>
 __device__ __forceinline__ int k_rotation(int n_tile, int nk) { return (W8 ? 2 * n_tile : n_tile) % nk; }
 
 __device__ __forceinline__ u32x4 gload16(const void* p) { return *(gptr_u32x4)(uintptr_t)p; }
-// Weights under the one-workgroup-per-tile kernel are streamed: a tile of them is used by one workgroup (two
+// Weights of one-workgroup tiles are streamed: a tile of them is used by one workgroup (two
 // or more for an expert above 256 rows) and never again in the launch, so those loads are non-temporal
-// (Mixtral-8x22B, 256 tokens: down projection 0.325 -> 0.302 ms).  In the persistent kernel the panels are
+// (Mixtral-8x22B, 256 tokens: down projection 0.325 -> 0.302 ms).  In the persistent body the panels are
 // shared through L2 and stay plain.
 template <bool STREAM>
 __device__ __forceinline__ u32x4 gload16_w(const void* p) {
@@ -140,7 +138,7 @@ __device__ __forceinline__ u32x4 gload16_w(const void* p) {
 }
 
 
-// ---- pieces shared by the one-workgroup-per-tile kernel and the persistent kernel ----
+// ---- pieces shared by one-workgroup tiles and the persistent body ----
 
 // Position of the expert's `local`-th tile.  Inside an expert, tiles are visited in groups of about
 // GM consecutive M tiles (the expert's M tiles split as evenly as possible); within a group the M
@@ -280,7 +278,7 @@ __device__ __forceinline__ void store_wave_outputs(const f32x4 (&acc)[2 * MT][TN
     }
 }
 
-// One tile of the one-workgroup-per-tile kernel: rows [row0, min(row0 + 64 MT, row_end)) of expert e times N tile n_tile.
+// One one-workgroup tile: rows [row0, min(row0 + 64 MT, row_end)) of expert e times N tile n_tile.
 // MT: 32-row units per wave along M (tile rows BM = 64*MT, 2 waves along M)
 // WN: waves along N; 4 -> 8 waves of up to 128x64 outputs, two per SIMD; every wave interleaves
 //     its share of the load / dequantise / LDS-store work with its MFMAs, a piece per MFMA group
@@ -623,7 +621,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, Stage st0, Stage st
                                                        min(BM, row_end - row0) - wm * 32 * MT, N - ncol0);
 }
 
-// ---- fp8 weight streamer: experts of up to 64 rows in calls that the one-workgroup-per-tile kernel serves alone ----
+// ---- fp8 weight streamer: experts of up to 64 rows in calls of one-workgroup tiles alone ----
 //
 // With a handful of rows per expert a launch reads every weight once (Expert_Wrapper.forward in its decoding use,
 // Wrapper.py:470-530) and is bound by how fast a CU can take fp8 weights in.  Through gemm_tile a 64-k stage of 256
@@ -660,7 +658,7 @@ struct TileLds {
     uint8_t *w0, *w1, *w2, *t0, *t1, *t2;
 };
 
-// How the down projection of one MLP is cut when its k is: row tiles of `rows` (256: on the persistent kernel, else on the split
+// How the down projection of one MLP is cut when its k is: row tiles of `rows` (256: on the persistent body, else on the split
 // kernel), k into `slices` of up to `blocks` blocks of 128.  part: where the fp32 sums go, [slices][n_rows][N].
 struct SplitPlan {
     int m_tiles, rows, slices, blocks;
@@ -855,13 +853,13 @@ __device__ __forceinline__ void stream8_tile(const GemmArgs& g, SBuf buf0, SBuf 
 }
 
 
-// ---- fp8 weight streamer in the persistent kernel's summation order: tiles of up to 192 rows ----
+// ---- fp8 weight streamer in the persistent body's summation order: tiles of up to 192 rows ----
 //
 // The same division of labour as stream8_tile (8 waves x 32 weight rows, fp8 weights by DMA in whole lines, every wave
 // multiplies all token rows, a weight is converted once, by the wave that multiplies it), for tiles whose rows another
-// kernel might have computed: what an fp8 expert's full 256-row tiles leave over, the halves of the persistent kernel's last
+// kernel might have computed: what an fp8 expert's full 256-row tiles leave over, the halves of the persistent body's last
 // tiles, and in calls that this kernel serves alone the experts (or 128-row slices of experts) above 64 rows.  A row's bits
-// must then not depend on who computes it, so every matrix instruction gets the k values the persistent kernel gives it,
+// must then not depend on who computes it, so every matrix instruction gets the k values the persistent body gives it,
 // in the same lanes: lane group q holds k = 32 s + 8 f(q) + (0..7) of k-step s, f = 0, 2, 1, 3.  Those are the 16-byte token
 // chunk 4 s + f(q) of a 64-k half, and 8 consecutive fp8 weights, one half of the 16-byte part 2 s + (q & 1): lane groups q and
 // q + 2 use the two halves of one part.  So lane group q reads part q, the lower half of the wave those of step 0 and the upper
@@ -900,7 +898,7 @@ __device__ __forceinline__ void stream8x_tile(const GemmArgs& g, const TileLds& 
     // Order of issue in half h of block p: the tokens two halves ahead (above 128 rows: one), h = 0: the scales of block p + 1, and
     // the weights of block p + 2 (all four instructions in h = 0; above 128 rows two in either half).  VM: DMA operations that may
     // stay in flight at the barrier of a half, those issued after its tokens.  (The scales do not count: nothing holds their
-    // place among the DMA, see the persistent kernel)
+    // place among the DMA, see the persistent body)
     constexpr int VM = WIDE ? 2 : 4 + NDT;
     static_assert(!(SPLIT && SWIGLU), "slices of k: the down projection");
     static_assert(TG >= 1 && TG <= 12, "token rows staged");
@@ -1148,14 +1146,14 @@ __device__ __forceinline__ void stream8x_tile(const GemmArgs& g, const TileLds& 
     }
 }
 
-// M tiles of an expert with `count` rows in the one-workgroup-per-tile kernel: one tile of up to 192 rows if that
+// One-workgroup tiles of an expert with `count` rows: one tile of up to 192 rows if that
 // holds them all, else tiles of 128.  The height follows the EXPERT, not the launch: a tile taller
 // than its expert stages and multiplies rows that do not exist, and an expert cut into several tiles reads its
 // weights once per tile and adds workgroups (the hot expert of a skewed decode batch: 9 x 128 tiles are 4.5 rounds
 // of 256 CUs and cost 5).  The tiles of an expert that is cut (above 192 rows) run side by side on one XCD and take
 // the weights with plain loads, so that all but the first read of a line come out of that XCD's L2.
-// 256-row tiles of an expert with `count` rows in the persistent kernel's tile space
-// whether an expert of `count` rows belongs to the one-workgroup-per-tile kernel (no rem_split)
+// (tiles_of, own_tiles; persistent_tiles: 256-row tiles of such an expert.)  is_cold: whether all its rows are one-workgroup tiles (no
+// rem_split)
 __host__ __device__ __forceinline__ bool is_cold(const GemmArgs& g, int count) {
     return count <= g.cold_max || (g.pair_rows && count >= PAIR_LO && count <= PAIR_HI);
 }
@@ -1190,9 +1188,9 @@ __host__ __device__ __forceinline__ int tiles_of(int count) {
     if (count <= SINGLE) return count > 0 ? 1 : 0;
     // bf16 weights: an expert of 257 to 384 rows is cut in the middle, into two tiles of the 192-row body that run
     // side by side on one XCD and share the weights through its L2: 320 rows are 2 x 160 rows of MFMA work, where
-    // two 256-row tiles of the persistent kernel multiply 512 and three 128-row tiles read the weights three times.
+    // two 256-row tiles of the persistent body multiply 512 and three 128-row tiles read the weights three times.
     // Mixtral-8x22B shapes, 8 experts of 288 / 320 / 384 rows: gate/up 1.31 / 1.29 / 1.30 -> 1.07 / 1.13 / 1.17 ms,
-    // down projection within 4 % either way; up to 256 rows one tile of the persistent kernel stays better (224
+    // down projection within 4 % either way; up to 256 rows one tile of the persistent body stays better (224
     // rows: 0.82 against 1.01 ms).
     if (PAIR && count > PAIR_LO - 1 && count <= PAIR_HI) return 2;
     return (count + 127) >> 7;
@@ -1200,14 +1198,14 @@ __host__ __device__ __forceinline__ int tiles_of(int count) {
 // rows of either tile of such a pair (the first tile holds whole 16-row groups)
 __device__ __forceinline__ int half_rows(int count) { return ((count + 1) / 2 + 15) & ~15; }
 
-// M tiles of an expert with `count` rows in the one-workgroup-per-tile kernel's own tile space
+// One-workgroup tiles of an expert with `count` rows in a call of both kinds
 template <bool W8>
 __host__ __device__ __forceinline__ int own_tiles(const GemmArgs& g, int c) {
-    if (g.rem_split) c &= 255;      // the rows the persistent kernel's full tiles leave over
+    if (g.rem_split) c &= 255;      // the rows the persistent body's full tiles leave over
     return (g.rem_split ? c > g.cold_max : !is_cold(g, c)) ? 0 : tiles_of<!W8>(c);
 }
 
-// The shared expert's rows and its tiles in the spaces of the two kernels when both run, all 0 without one
+// The shared expert's rows and its tiles of either kind in a call of both, all 0 without one
 struct SharedTiles { int first, end, own, persistent; };
 template <bool W8>
 __host__ __device__ __forceinline__ SharedTiles shared_tiles_of(const GemmArgs& g, int first, int end) {
@@ -1235,11 +1233,11 @@ __device__ __forceinline__ int sum_over_experts(const GemmArgs& g, int tid, int*
     return tot;
 }
 
-// ---- bf16 weight streamer in the persistent kernel's summation order: tiles of up to 192 rows ----
+// ---- bf16 weight streamer in the persistent body's summation order: tiles of up to 192 rows ----
 //
 // The fp8 streamers' way of moving data for bf16 weights: weights and token rows reach LDS by DMA in the persistent
 // kernel's layout of a 64-k stage (128-byte rows, chunk c of row r at c ^ swz(r)), and every matrix instruction gets
-// the k values the persistent kernel gives it, in the same lanes, so a row's bits do not depend on who computes it.
+// the k values the persistent body gives it, in the same lanes, so a row's bits do not depend on who computes it.
 // No staging registers and no LDS stores, so every operand of a stage can be requested up front.  Up to 64 rows the 8
 // waves split the tile's 256 weight rows and each multiplies all token rows; above, two sets of 4 waves take half of
 // the token groups each (4 + TG / 2 operand reads per k-step for 2 TG matrix instructions, where 8 x 1 waves need
@@ -1412,7 +1410,8 @@ __device__ __forceinline__ void stream8x(const GemmArgs& g, const TileLds& lds, 
     }
 }
 
-// One workgroup per (M tile, N tile); serves what the persistent kernel does not take (few rows per expert, odd K).
+// One workgroup per (M tile, N tile), in calls without persistent tiles (few rows per expert, odd K).  (tile_body is its counterpart in calls
+// of both kinds: which rows a tile has, and which streamer computes them, is the same there, since a row's bits follow from it.)
 template <int WN, bool SWIGLU, bool W8>
 __global__ __launch_bounds__(128 * WN) void grouped_gemm_kernel(GemmPair pair_of) {
     constexpr int NT = 128 * WN;
@@ -1483,10 +1482,10 @@ __global__ __launch_bounds__(128 * WN) void grouped_gemm_kernel(GemmPair pair_of
     const int row_end = uni(s_sel[4]);
     const int first_row = uni(s_sel[3]);
     if (W8 && s8_ok) {
-        // fp8 weights: the weight streamers.  Up to 64 rows where no other kernel's summation order has to be matched: the
+        // fp8 weights: the weight streamers.  Up to 64 rows where no persistent tile's summation order has to be matched: the
         // form that reads a lane's 16 weights at once.  Everything else -- up to 192 rows; what an expert's full 256-row
-        // tiles leave over; 128-row slices of larger experts when the kernel serves the call by itself -- in the
-        // persistent kernel's order.
+        // tiles leave over; 128-row slices of larger experts when the kernel serves the call by itself -- in the order of
+        // persistent tiles.
         const int r0 = first_row + (mt_e > 1 ? m_tile * 128 : 0), r1 = mt_e > 1 ? min(row_end, r0 + 128) : row_end;
         const int rows = r1 - r0;
         if (g.alone && mt_e == 1 && rows <= 64) {
@@ -1506,7 +1505,7 @@ __global__ __launch_bounds__(128 * WN) void grouped_gemm_kernel(GemmPair pair_of
     const int slice = pair ? half_rows(rows_e) : 128;
     const int t0 = mt_e > 1 ? first_row + m_tile * slice : first_row, t1 = mt_e > 1 ? min(row_end, t0 + slice) : row_end;
     if (!W8 && s8_ok) {
-        // bf16 weights: the weight streamer in the persistent kernel's order
+        // bf16 weights: the weight streamer in the persistent body's order
         if (mt_e == 1) stream16<SWIGLU, false>(g, lw0, lw1, lw2, lt0, lt1, e, t0, t1, n_tile);
         else stream16<SWIGLU, true>(g, lw0, lw1, lw2, lt0, lt1, e, t0, t1, n_tile);
         return;
@@ -1690,7 +1689,7 @@ __global__ __launch_bounds__(64) void grouped_gemm_thin_kernel(GemmPair pair_of,
 // workgroup each, so that tiles x slices fill the CUs once; the fp32 sums of the slices go to the workspace and
 // add_slices_kernel adds them, in order, and rounds once.  Rows past 128 are cut into tiles of equal height; all tiles of a
 // call run the same body, chosen by that height, so a row's bits do not depend on its place.  The M tiles of one piece of
-// the weights are neighbours on one XCD.  (From 257 rows on they may run as 256-row tiles of the persistent kernel instead, split_plan.)
+// the weights are neighbours on one XCD.  (From 257 rows on they may run as 256-row tiles of the persistent body instead, split_plan.)
 // Measured (DeepSeek-V3's dense MLP, both launches, us, without scratch -> with it): 1 token 119 -> 75, 17: 185 -> 87,
 // 64: 231 -> 115, 128: 356 -> 161, 192: 516 -> 220, 256: 426 -> 273; of those the gate and up products take 49, 58, 76, 104, 150
 // and 186.
@@ -1750,7 +1749,7 @@ __device__ __forceinline__ int fresh_lane() {
     return l;
 }
 
-// Persistent kernel for BM = 256: one workgroup per CU walks its share of the tiles, and the software
+// Persistent body for BM = 256: one workgroup per CU walks its share of the tiles, and the software
 // pipeline runs on across the tile boundary (a tile's last k-iterations already fetch the next tile's
 // first stages, and the epilogue runs beside them).  What a fresh workgroup pays per tile -- launch,
 // tile-prefix scan, pointer chase, first fetch, store drain: 6-8 us against 57 us of k loop for K = 2048 --
@@ -1855,7 +1854,7 @@ __device__ __forceinline__ void persistent_body(const GemmPair& pair_of, const S
         if (W8 && SWIGLU) s_ptr1[3] = (unsigned long long)(uintptr_t)s.s1[0];
     }
     __syncthreads();
-    // whole rounds, and the last one unless it is better off with the other kernel, whose own tiles are counted for that
+    // whole rounds, and the last one unless it is better off as half tiles: one-workgroup tiles, whose own are counted for that
     const SharedTiles second_tiles = PAIRED ? shared_tiles_of<W8>(pair_of.p[1], uni(s_off1[0]), uni(s_off1[1])) : SharedTiles{0, 0, 0, 0};
     const int ptiles1 = second_tiles.persistent;
     const int own = g.tail_cus > 0 ? sum_over_experts<NT>(g, tid, s_wtot, [&](int c) { return own_tiles<W8>(g, c); }) * g.n_tiles_n + second_tiles.own : 0;
@@ -2291,7 +2290,7 @@ __device__ __forceinline__ void tile_body(const GemmPair& pair_of, const TileLds
     tile_in_expert(v - pe * g.n_tiles_n, mt_e, g.n_tiles_n, m_tile, n_tile);
     int r0, r1;
     bool neighbours = true;
-    if (half >= 0) {                     // half of a 256-row tile of the persistent kernel's space
+    if (half >= 0) {                     // half of a 256-row tile of the persistent body's space
         r0 = o0 + m_tile * 256 + half * 128;
         r1 = min(min(row_end, o0 + (m_tile + 1) * 256), r0 + 128);
         if (r0 >= r1) return;
@@ -2308,7 +2307,7 @@ __device__ __forceinline__ void tile_body(const GemmPair& pair_of, const TileLds
 }
 template <bool SWIGLU, bool W8, bool PAIRED>
 __global__ __launch_bounds__(512) void grouped_gemm_both_kernel(GemmPair persistent_of, GemmPair tiles_of, int persistent_grid) {
-    // The streamers' three weight buffers and token buffers.  The persistent kernel has its weights in the first two and its token
+    // The streamers' three weight buffers and token buffers.  The persistent body has its weights in the first two and its token
     // rows in the lower 16 KiB of the others, with its tables behind two of those.  (bf16: the whole LDS of a CU.)
     constexpr int TOKENS = 128 * ROW_B;
     __shared__ __attribute__((aligned(1024))) uint8_t lw0[S8_WBYTES];
@@ -2329,7 +2328,7 @@ __global__ __launch_bounds__(512) void grouped_gemm_both_kernel(GemmPair persist
     }
 }
 
-// The persistent kernel alone: one MLP's down projection in slices of k
+// The persistent body alone: one MLP's down projection in slices of k
 __global__ __launch_bounds__(512) void grouped_gemm_persistent_split_kernel(GemmPair pair_of, SplitArgs split) {
     __shared__ __attribute__((aligned(1024))) uint8_t a0a[128 * ROW_B];
     __shared__ __attribute__((aligned(1024))) uint8_t a0b[128 * ROW_B];
@@ -2360,7 +2359,7 @@ int launch_tiles(const GemmPair& pair, int n_rows, hipStream_t st) {
     return MOE_OK;
 }
 
-// CUs of the current device (the persistent kernel runs one workgroup on each)
+// CUs of the current device (one persistent workgroup on each)
 inline int cu_count() {
     static int cached[64] = {0};
     int dev = 0;
@@ -2419,7 +2418,7 @@ inline bool gather_fits(const GemmArgs& g) { return !g.row_map || g.a_bytes < (1
 //    its own start), at most 16.
 //  * above, up to a round of 256-row tiles, whichever of three takes least by these counts (us), each at its best number of slices: uncut,
 //    1.55 a block of k while the pieces leave a third of the CUs idle, 15 % more up to a round of them and 60 % beyond; the split
-//    kernel, one round, 0.9 + 0.0055 a row of its tiles a block and 0.37 per MB of sums; the persistent kernel's 256-row tiles, 2.8
+//    kernel, one round, 0.9 + 0.0055 a row of its tiles a block and 0.37 per MB of sums; the persistent body's 256-row tiles, 2.8
 //    a block, 20 a further round and 0.16 per MB.  The split kernel's lower tiles win where slices are short or tiles few.
 // Measured: h of 1024 to 8192, k of 4096 to 18432, 257 to 3000 rows, all three at every number of slices: the counts are within 12 %
 // and the choice 0.5 % behind the best of them in the mean, 5 % at most.  Down projection, us, uncut / split kernel / 256-row tiles:
@@ -2443,7 +2442,7 @@ SplitPlan split_plan(int n_rows, int K, int n_tiles_n) {
     const int m256 = (n_rows + 255) / 256, left = n_rows & 255;
     const long tiles = (long)m256 * n_tiles_n;
     if (tiles > cus) return SplitPlan{};
-    const bool own = left > 0 && left <= 192;                        // (uncut, these rows are a tile of a workgroup of its own)
+    const bool own = left > 0 && left <= 192;                        // (uncut, these rows are a one-workgroup tile)
     const long pieces = (2 * (m256 - (own ? 1 : 0)) + (own ? 1 : 0)) * (long)n_tiles_n;
     double best = 4.0 + 1.55 * nblk * (3 * pieces <= 2 * cus ? 1.0 : pieces <= cus ? 1.15 : 1.6);
     SplitPlan plan{};
@@ -2503,7 +2502,7 @@ bool thin_pays(const GemmArgs& g, int n_rows, const GemmArgs* shared) {
     return thin < std::ceil(tiles / cus) * cus * (g.K <= 2048 ? 1.07 : 1.0);
 }
 
-// The persistent kernel needs an even number of k-stages for its hand-over (fp8 sizes always have one), keeps per-expert
+// The persistent body needs an even number of k-stages for its hand-over (fp8 sizes always have one), keeps per-expert
 // tables for up to 512 experts and addresses gathered rows with 32-bit offsets.
 inline bool persistent_fits(const GemmArgs& g) { return g.K % 128 == 0 && g.E <= 512 && gather_fits(g) && cu_count() >= 8; }
 
@@ -2559,7 +2558,7 @@ int launch_mt(const GemmArgs& g0, int n_rows, int max_rows, void* workspace, siz
     // 0 ... 3989 rows, 47 of them below 193, whose 256-row tiles were 49 % padding): block step 0.923 -> 0.847 ms,
     // routed gate/up 0.395 -> 0.355 ms; DeepSeek-V2-236B, 32768 tokens: 11.48 -> 11.39 ms.
     // fp8 weights: the rule is applied to what an expert's full 256-row tiles leave over.  A ragged
-    // last tile costs the persistent kernel a full tile of MFMA time; the other kernel streams the expert's weights
+    // last tile costs a persistent workgroup a full tile of MFMA time; a one-workgroup tile streams the expert's weights
     // once more for it, and fp8 weights are half the bytes.  DeepSeek-V3, 65536 tokens (256 experts of 581 ... 3941
     // rows, every second one with at most 128 rows over): block step 46.3 -> 45.8 ms, routed gate/up 25.2 -> 24.8,
     // down 12.9 -> 12.7 (with up to 64 or 96 rows over 46.2 - 46.3; with all, as two 128-row tiles, 47.1).  Up to 192
@@ -2567,12 +2566,12 @@ int launch_mt(const GemmArgs& g0, int n_rows, int max_rows, void* workspace, siz
     // 3584 / 4096 / 8192 tokens 4.53 -> 3.99, 4.64 -> 4.31, 7.50 -> 7.41 ms (at 4096 tokens 109 of the 256 experts hold
     // 129 to 192 rows, which were padded 256-row tiles).  With bf16
     // weights it is break-even (Mixtral-8x7B 9.28 -> 9.23 ms, DeepSeek-V2-236B 11.34 -> 11.42) and not done.
-    // Last round of the persistent kernel (tail_tiles above): Mixtral-8x22B, 8192 tokens, down projection (6.4 rounds
+    // Last round of the persistent body (tail_tiles above): Mixtral-8x22B, 8192 tokens, down projection (6.4 rounds
     // of 0.4 ms) 2.82 -> 2.66 ms, step 8.31 -> 8.13; Mixtral-8x7B 9.39 -> 9.27 ms; DeepSeek-V2-Lite 0.855 -> 0.821 ms
     // (its shared expert's 128 down tiles become 256 half tiles: 0.071 -> 0.055 ms); DeepSeek-V2-236B 11.43 -> 11.46,
     // DeepSeek-V3 46.56 -> 46.54: short rounds gain nothing, a partial round of few CUs runs at a higher clock anyway.
     pair.p[0] = both_kernels<W8>(g);
-    // One fp8 expert (a dense MLP): the rows are known here.  What its full tiles leave over goes to the persistent kernel too,
+    // One fp8 expert (a dense MLP): the rows are known here.  What its full tiles leave over goes to the persistent body too,
     // as a padded tile, where that shortens the rounds by the same count: the last one has room, or the other kind is
     // saved.  DeepSeek-V3's dense MLP, us: 1300 / 1800 / 2200 / 4000 / 6000 tokens (leftovers of 20, 8, 152, 160 and 112 rows) 1129 /
     // 1352 / 1567 / 2726 / 3998 -> 1015 / 1263 / 1465 / 2606 / 3887; done always, 600 / 1100 / 3500 tokens would be 616 / 931 / 2370
@@ -2658,13 +2657,13 @@ bool sliced(const moe_mlp_group& m, int32_t hidden) {
 // Whether 256-row tiles of the group (its gate and up projection) are fewer than 3/8 of the CUs
 bool few_tiles(const moe_mlp_group& m, long cus) { return (long)(m.n_rows / 256 + 1) * ((m.inter + 127) / 128) * 8 < 3 * cus; }
 
-// Whether the shared expert's tiles join the routed experts' launches.  Where the routed call goes to both kernels they do if a
-// call of its own would go to both as well (128 rows, no slices of k), up to four rounds of tiles of its own (beyond, the same
-// within 0.2 %): the two then fill their last rounds together.  Where the routed call is one that the one-workgroup-per-tile
-// kernel (or the thin one) serves alone, a few tiles always do; more of them up to two of that kernel's 128-row tiles, all that
+// Whether the shared expert's tiles join the routed experts' launches.  Where the routed call has both kinds of tiles they do if a
+// call of its own would have both as well (128 rows, no slices of k), up to four rounds of tiles of its own (beyond, the same
+// within 0.2 %): the two then fill their last rounds together.  Where the routed call has one-workgroup tiles (or the
+// thin kernel's waves) alone, a few tiles always do; more of them up to two of that kernel's 128-row tiles, all that
 // the shared expert gets there, per CU, unless its own call is in slices.
-// Layers, us, apart -> joined.  Both kernels: DeepSeek-V2-Lite 1400 / 2000 / 2777 / 4096 tokens 439 / 514 / 585 / 725 -> 397 / 470 /
-// 563 / 699; DeepSeek-V3 4096 / 6000 4046 / 5498 -> 4004 / 5367, 16384 the same.  One kernel: DeepSeek-V2-Lite 1024 / 1300 366 /
+// Layers, us, apart -> joined.  Both kinds: DeepSeek-V2-Lite 1400 / 2000 / 2777 / 4096 tokens 439 / 514 / 585 / 725 -> 397 / 470 /
+// 563 / 699; DeepSeek-V3 4096 / 6000 4046 / 5498 -> 4004 / 5367, 16384 the same.  One kind: DeepSeek-V2-Lite 1024 / 1300 366 /
 // 409 -> 322 / 351; DeepSeek-V2-236B 1024 / 1500 1463 / 1641 -> 1416 / 1615, 2048 the same, 3000 2074 -> 2090 (not joined: 576 tiles);
 // DeepSeek-V3 1500 / 2997 / 4000 2507 / 3437 / 4139 -> 2470 / 3382 / 4120.
 bool joins(const moe_mlp_group& routed, const moe_mlp_group& shared, int32_t hidden) {

@@ -78,7 +78,7 @@ __device__ __forceinline__ void store_shared_8(uint16_t* p, const u32x2& v) {
     __hip_atomic_store(reinterpret_cast<uint64_t*>(p), __builtin_bit_cast(uint64_t, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Bytes of LDS for NB stages, and the columns a wave has
+// Bytes of LDS of a stage
 template <bool W8, int NF>
 constexpr int thin_stage_bytes = NF * 2048 + (W8 ? 4096 : 2048);
 

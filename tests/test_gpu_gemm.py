@@ -141,14 +141,14 @@ def test_tile_height_follows_the_expert(fp8):
 
 @pytest.mark.parametrize("fp8", [False, True])
 def test_experts_split_between_the_two_kernels(fp8):
-    """From a mean of 128 rows per expert a call launches both kernels and every expert goes by its own count.  bf16
-    weights: up to 192 rows one tile of the one-workgroup-per-tile kernel, more the persistent kernel's 256-row tiles.
-    fp8 weights: the persistent kernel's tile space holds an expert's full 256-row tiles, and what they leave over goes
-    to the other kernel if it is at most 192 rows (300 = 256 + 44, 640 = 512 + 128, 700 = 512 + 188, 512 leaves nothing,
-    2000 = 1792 + 208 stays whole).  (At this size the tile space is a short last round, which the other kernel runs as half tiles.)
+    """From a mean of 128 rows per expert a launch has both kinds of tiles and every expert goes by its own count.  bf16
+    weights: up to 192 rows one tile of a workgroup of its own, more 256-row tiles of the persistent workgroups.
+    fp8 weights: the persistent tile space holds an expert's full 256-row tiles, and what they leave over is a tile
+    of one workgroup if it is at most 192 rows (300 = 256 + 44, 640 = 512 + 128, 700 = 512 + 188, 512 leaves nothing,
+    2000 = 1792 + 208 stays whole).  (At this size the tile space is a short last round, which runs as half tiles of one workgroup.)
     Against the oracle, and every expert's rows bit-for-bit against a call that holds this expert alone, whichever
-    kernel and tile its rows fall to there.  (A lone call below a mean of 128 is served by the one-workgroup-per-tile
-    kernel alone, which then walks k from other stages than a call of both kernels, and is left out.)"""
+    kernel and tile its rows fall to there.  (A lone call below a mean of 128 has one-workgroup tiles
+    alone, which then walk k from other stages than a call of both kinds, and is left out.)"""
     from moe_gen_amd import ops
     E, h, I = 13, 256, 384
     counts = [700, 3, 192, 193, 64, 0, 129, 2000, 128, 300, 512, 640, 1600]
@@ -176,14 +176,14 @@ def test_experts_split_between_the_two_kernels(fp8):
 
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("I,counts", [(1280, [700, 520, 300, 1300, 90]),      # gate/up: less than half a round
-                                      (2048, [700, 520, 300, 1300, 90]),      # gate/up: 192 tiles next to 48 of the other kernel
+                                      (2048, [700, 520, 300, 1300, 90]),      # gate/up: 192 tiles next to 48 of one workgroup each
                                       (2560, [700, 520, 300, 1300, 90]),      # gate/up: a round and a few tiles
                                       (1664, [2100, 2300, 2500, 1500, 10])])  # gate/up: 442 tiles, a round + 186, next to 13
 def test_rounds_of_the_persistent_kernel_and_its_last_tiles(fp8, I, counts):
-    """The persistent kernel (one workgroup per CU) takes whole rounds of 256 tiles; its last, partial round goes to
-    the other kernel as 128-row halves when that shortens the two launches: alone, a round of at most 128 tiles;
-    next to the other kernel's own tiles also a longer one (192 + 48 tiles: one launch of 432 half and whole tiles
-    instead of two launches; 186 of 442 likewise).  Tile counts in the comments are for bf16 weights (with fp8
+    """The persistent workgroups (one per CU) take whole rounds of 256 tiles; their last, partial round becomes
+    128-row halves of one workgroup each when that shortens the rounds of both kinds: alone, a round of at most 128 tiles;
+    next to one-workgroup tiles also a longer one (192 + 48 tiles: 432 half and whole tiles
+    of one workgroup; 186 of 442 likewise).  Tile counts in the comments are for bf16 weights (with fp8
     weights only an expert's full tiles and ragged tiles above 128 rows count).  The down projections of these cases
     have a few dozen tiles, all of them half tiles.  Against the oracle."""
     from moe_gen_amd import ops
@@ -270,7 +270,7 @@ def test_fp8_weight_streamer_rows_do_not_depend_on_the_tile(h, I):
 
 @pytest.mark.parametrize("counts", [
     [5, 16, 17, 32, 33, 64, 65, 80, 81, 96, 112, 128, 129, 144, 160, 176, 192] + [5] * 12,     # mean 59: one kernel
-    [192, 181, 170, 160, 150, 140, 130, 129, 257, 300, 384, 600, 5]])                          # mean 215: both kernels
+    [192, 181, 170, 160, 150, 140, 130, 129, 257, 300, 384, 600, 5]])                          # mean 215: both kinds of tiles
 def test_bf16_weight_streamer_rows_do_not_depend_on_the_tile(counts):
     """bf16 experts of up to 192 rows (and the halves of one of 257 ... 384) go through the bf16 weight streamer: one
     body per number of 16-row groups, two wave layouts (up to 64 rows, above), weights and token rows by DMA.
@@ -304,9 +304,9 @@ def test_bf16_weight_streamer_rows_do_not_depend_on_the_tile(counts):
 
 
 def test_bf16_rows_do_not_depend_on_the_call():
-    """With bf16 weights every path of both kernels adds a column's products in one order, in every call: the same 40
+    """With bf16 weights every path adds a column's products in one order, in every call: the same 40
     rows come out bit-identical from a call that the one-workgroup-per-tile kernel serves alone (one expert of 40
-    rows) and from a call that launches both kernels, where they open an expert of 600 rows (persistent kernel), one
+    rows) and from a call with both kinds of tiles, where they open an expert of 600 rows (persistent kernel), one
     of 150 (a single tile) and one of 300 (the first of two tiles side by side)."""
     from moe_gen_amd import ops
     h, I, r = 512, 768, 40
@@ -343,7 +343,7 @@ def test_bf16_weight_streamer_shapes_and_gather(h, I):
 
 
 @pytest.mark.parametrize("counts", [
-    [129, 144, 145, 160, 176, 177, 192, 400, 600, 320, 449, 70],     # mean 255: both kernels; 400 = 256 + 144 left over
+    [129, 144, 145, 160, 176, 177, 192, 400, 600, 320, 449, 70],     # mean 255: both kinds of tiles; 400 = 256 + 144 left over
     [129, 150, 192, 170, 64, 65] + [5] * 20])                         # mean 35: the one-workgroup-per-tile kernel alone
 @pytest.mark.parametrize("h,I", [(640, 384), (1024, 896)])            # 5 / 3 and 8 / 7 blocks of 128 k (odd and even counts)
 def test_fp8_weight_streamer_tiles_of_129_to_192_rows(counts, h, I):
@@ -871,7 +871,7 @@ def test_shared_expert_in_the_launches_of_both_kernels(fp8, n, E, I, shared_inte
     the other one.  Bit for bit what the calls give apart, with fp8 weights too (both start every tile at k 0 there)."""
     from moe_gen_amd import ops
     k, h = 2, 384
-    print(f"joint, both kernels fp8={fp8} n={n} E={E} I={I} shared_inter={shared_inter}", flush=True)
+    print(f"joint, both kinds of tiles fp8={fp8} n={n} E={E} I={I} shared_inter={shared_inter}", flush=True)
     g = torch.Generator().manual_seed(n)
     dev = lambda m: tuple(t.cuda() for t in m) if isinstance(m, tuple) else m.cuda()
     tables = []
@@ -897,7 +897,7 @@ def test_shared_expert_in_the_launches_of_both_kernels(fp8, n, E, I, shared_inte
 
 
 @pytest.mark.parametrize("fp8", [False, True])
-@pytest.mark.parametrize("E", [2, 16])          # routed experts of 256 rows (both kernels) and of 32 (one kernel)
+@pytest.mark.parametrize("E", [2, 16])          # routed experts of 256 rows (both kinds of tiles) and of 32 (one kind)
 @pytest.mark.parametrize("n_rows,rows", [
     (192, 150), (300, 150), (300, 200), (384, 200), (384, 260), (600, 0), (600, 150), (600, 200), (600, 300), (600, 384), (600, 500),
     (1100, 513)])
@@ -944,7 +944,7 @@ def test_joint_call_with_fewer_shared_rows_than_its_bound(fp8, E, n_rows, rows):
 @pytest.mark.parametrize("n,shared_inter", [(280, 6144), (500, 6144), (700, 4096)])     # the least sizes of the rule
 def test_large_fp8_shared_expert_in_a_one_kernel_call_has_the_bits_of_its_own_call(n, shared_inter):
     """Below a mean of 128 rows per routed expert a shared expert of 3/8 of the CUs' worth of 256-row tiles or more is summed as in a
-    call of its own, where both kernels run.  Last tiles of 24, 116 and 60 rows."""
+    call of its own, which has both kinds of tiles.  Last tiles of 24, 116 and 60 rows."""
     from moe_gen_amd import ops
     E, k, h, I = 12, 2, 256, 128
     print(f"large shared expert n={n} shared_inter={shared_inter}", flush=True)
@@ -972,8 +972,8 @@ def test_large_fp8_shared_expert_in_a_one_kernel_call_has_the_bits_of_its_own_ca
 
 @pytest.mark.parametrize("E,rows,shared_inter,scratch", [
     (12, 17, 12288, True),     # one kernel for the routed experts, slices of k for the shared one
-    (2, 300, 4096, True),      # both kernels
-    (2, 100, 640, False)])     # both kernels, and one that would start its sums elsewhere
+    (2, 300, 4096, True),      # both kinds of tiles
+    (2, 100, 640, False)])     # both kinds of tiles, and one that would start its sums elsewhere
 def test_joint_call_leaves_apart_what_its_own_call_sums_in_another_way(E, rows, shared_inter, scratch):
     """fp8.  Bit for bit two separate calls on the same groups, scratch included."""
     from moe_gen_amd import _native as N
