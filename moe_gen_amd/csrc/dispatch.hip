@@ -85,7 +85,7 @@ __global__ __launch_bounds__(256) void rank_scatter(const int32_t* __restrict__ 
                                                     int32_t* __restrict__ counts,
                                                     int32_t* __restrict__ offsets, int32_t* __restrict__ perm,
                                                     int32_t* __restrict__ pos, int32_t* __restrict__ row_map, int k,
-                                                    int32_t* __restrict__ one_group) {
+                                                    int32_t* __restrict__ one_group, int32_t* __restrict__ claims, int n_claims) {
     __shared__ int whist[SEG_WAVES][MAX_E];    // per-wave counts, then per-wave running cursors
     __shared__ int wtot[4];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -135,6 +135,7 @@ __global__ __launch_bounds__(256) void rank_scatter(const int32_t* __restrict__ 
         if (tid < E) offsets[tid] = off;
         if (tid == E - 1) offsets[E] = off + cv;
         if (one_group && tid < 2) one_group[tid] = tid ? (int32_t)(nk / k) : 0;
+        for (int i = tid; i < n_claims; i += 256) claims[i] = 0;
     }
 
     // pass 1: counts of this wave's slice
@@ -237,7 +238,7 @@ int dispatch_launch(const int32_t* topk_idx, int64_t nk, int32_t top_k, int32_t 
         if (nseg > SUM_SEGMENTS)
             hipLaunchKernelGGL(scan_segments, dim3((n_experts + 3) / 4), dim3(256), 0, st, seg, nseg, n_experts, out.counts);
         hipLaunchKernelGGL(nseg > SUM_SEGMENTS ? rank_scatter<true> : rank_scatter<false>, dim3(nseg), dim3(256), 0, st, topk_idx, nk, n_experts,
-                           seg, nseg, out.counts, out.offsets, out.perm, out.pos, out.row_map, top_k, out.one_group);
+                           seg, nseg, out.counts, out.offsets, out.perm, out.pos, out.row_map, top_k, out.one_group, out.claims, out.n_claims);
     }
     if (x) {
         hipLaunchKernelGGL(gather_rows, dim3((unsigned)((nk + 3) / 4)), dim3(256), 0, st,

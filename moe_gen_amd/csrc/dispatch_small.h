@@ -17,6 +17,8 @@ struct DispatchOut {
     // [n_arrivals]: set to minus the experts that have rows and the one of one_group (CombineTail; one workgroup's form only)
     int32_t* arrivals = nullptr;
     int n_arrivals = 0;
+    int32_t* claims = nullptr;   // [n_claims]: set to 0 (LayerCall)
+    int n_claims = 0;
 };
 
 // (NW waves.)  Wave w owns the w-th slice of the list (a multiple of 64 entries, at most IT of them): counts it, the first 256 threads
@@ -76,6 +78,7 @@ __device__ __forceinline__ void dispatch_one_workgroup(int nk, int E, const Disp
     if (out.one_group && tid < 2) out.one_group[tid] = tid ? nk / k : 0;
     const int busy = __syncthreads_count(tid < E && cv > 0);
     for (int i = tid; i < out.n_arrivals; i += 64 * NW) out.arrivals[i] = -(busy + (out.one_group ? 1 : 0));
+    for (int i = tid; i < out.n_claims; i += 64 * NW) out.claims[i] = 0;
     int* cur = whist[wave];
 #pragma unroll
     for (int it = 0; it < IT; ++it) {

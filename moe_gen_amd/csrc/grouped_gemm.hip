@@ -113,6 +113,7 @@ struct GemmArgs {
 struct GemmPair {
     GemmArgs p[2];              // routed, shared
     int shared_tiles, shared_rows;
+    int32_t* claims;            // kClaimInts zeros, or NULL (see Claims)
 };
 
 // Stage at which a tile of N tile n_tile starts its walk over k.  Workgroups that run side by side mostly differ in
@@ -137,6 +138,75 @@ __device__ __forceinline__ u32x4 gload16_w(const void* p) {
     return STREAM ? __builtin_nontemporal_load((gptr_u32x4)(uintptr_t)p) : *(gptr_u32x4)(uintptr_t)p;
 }
 
+
+// A barrier behind this wave's LDS operations that leaves loads and stores to memory in flight
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// ---- which workgroup computes which tile of one workgroup ----
+//
+// Tiles are dealt to the XCDs in groups of 4 consecutive ones (the M tiles of one N tile first), round robin: those that read the
+// same weights share them through one XCD's L2, and small groups keep the XCDs even whatever the number of tiles and however much
+// one expert's tiles cost more than another's.  (Workgroup ids are dealt to the XCDs one by one by the hardware.)
+__device__ __forceinline__ int dealt_tile(int xcd, int i) { return (((i >> 2) << 3) + xcd) * 4 + (i & 3); }
+// The i-th tile of an XCD goes to the i-th workgroup of the XCD, in a grid that the host bounds without knowing the counts (OneTile);
+// or, in calls of both kinds that bring counters (zeros: a layer call, whose dispatch sets them), to its i-th claim: a workgroup per
+// CU, the persistent ones among them when they are done, claims tiles until none is left, and an XCD that is done goes on with
+// the others'.  That spares a tile its launch and the scan over the experts, and the CUs the surplus workgroups of such a grid, which
+// take 3 us each: DeepSeek-V2-236B, 4000 tokens, 4100 of them in the down projection, the layer 2165 -> 2108 us.  (Calls of tiles of one
+// workgroup alone stay with the launches: with claims 1 % faster where many experts have no rows, DeepSeek-V2-236B 32 and 64 tokens,
+// 2 to 3 % slower at few tiles a CU, DeepSeek-V2-Lite 32 ... 256 and DeepSeek-V3 1000.)
+struct OneTile {
+    __device__ __forceinline__ int thread() const { return threadIdx.x; }
+    __device__ __forceinline__ void ask() {}
+};
+struct Claims {
+    int32_t* counters;           // one per XCD, kClaimStride apart; NULL: the workgroup has one tile
+    int xcd, limit;              // the tiles are those below limit
+    int next;                    // what ask() found (the first lane's)
+    // the thread's number, produced where it is used: what every form of a tile derives from it is not computed in front of the loop
+    // over the tiles and kept, or spilled, through it
+    __device__ __forceinline__ int thread() const {
+        int t = threadIdx.x;
+        asm volatile("" : "+v"(t));
+        __builtin_assume(t >= 0 && t < 512);
+        return t;
+    }
+    __device__ __forceinline__ int count(int from) const {
+        return __hip_atomic_fetch_add(counters + from * kClaimStride, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    // in front of a tile's epilogue: the answer takes about 2 us
+    __device__ __forceinline__ void ask() {
+        if (counters && threadIdx.x == 0) next = count(xcd);
+    }
+    // The workgroup's next tile, -1 if there is none.  All threads; told: LDS.  (Bare barriers: a fence would wait for the stores of
+    // the epilogue.)
+    __device__ __forceinline__ int take(int* told) const {
+        if (!counters) return -1;
+        int v = -1;
+        if (threadIdx.x < 64) {
+            const int lane = threadIdx.x;
+            v = dealt_tile(xcd, uni(next));
+            while (v >= limit) {
+                v = -1;
+                const int seen = lane < 8 ? __hip_atomic_load(counters + lane * kClaimStride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+                const uint64_t left = __ballot(lane < 8 && dealt_tile(lane, seen) < limit);
+                if (left == 0) break;
+                const int from = (int)__builtin_ctzll(left);
+                int i = 0;
+                if (lane == 0) i = count(from);
+                v = dealt_tile(from, uni(i));
+            }
+        }
+        lds_barrier();                           // every wave has left the tile before, and read its number
+        if (threadIdx.x == 0) *told = v;
+        lds_barrier();
+        return uni(*told);
+    }
+};
 
 // ---- pieces shared by one-workgroup tiles and the persistent body ----
 
@@ -676,9 +746,9 @@ struct KSlice {
     float* part;
 };
 
-template <int TG, bool SWIGLU, bool SPLIT = false>   // TG: 16-row token groups multiplied (the expert has at most 16 TG <= 64 rows)
+template <int TG, bool SWIGLU, bool SPLIT = false, typename C>   // TG: 16-row token groups multiplied (the expert has at most 16 TG <= 64 rows)
 __device__ __forceinline__ void stream8_tile(const GemmArgs& g, SBuf buf0, SBuf buf1, SBuf buf2, int e, int row0,
-                                             int row_end, int n_tile, KSlice ks = {}) {
+                                             int row_end, int n_tile, C& claims, KSlice ks = {}) {
     constexpr int NBLK = SWIGLU ? 128 : 256;
     constexpr int NDW = 4, NDT = 2;               // DMA instructions per wave and 128-k block: weights, tokens
     // Operations that may stay in flight at the wait for a block: the DMA of the next block, NDW + NDT instructions
@@ -688,7 +758,7 @@ __device__ __forceinline__ void stream8_tile(const GemmArgs& g, SBuf buf0, SBuf 
     constexpr int VM_BLOCK = NDW + NDT;
     static_assert(!(SPLIT && SWIGLU), "slices of k: the down projection");
     static_assert(TG >= 1 && 16 * TG <= S8_TROWS, "token rows staged");
-    const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
+    const int tid = claims.thread(), lane = tid & 63, wave = uni(tid >> 6);
     const int n0 = n_tile * NBLK;
     const int K = g.K, N = g.N;
     const int npair = SPLIT ? ks.count : K >> 7;             // blocks of 128 k multiplied
@@ -831,6 +901,7 @@ __device__ __forceinline__ void stream8_tile(const GemmArgs& g, SBuf buf0, SBuf 
         if (p + 1 < npair) iteration(p + 1, buf1, buf0, 1);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no DMA may land in LDS after the workgroup has gone
+    claims.ask();
 
     // ---- epilogue: a lane holds 4 consecutive columns of one row per accumulator and stores them itself ----
 #pragma unroll
@@ -886,9 +957,9 @@ __device__ __forceinline__ void stream8_tile(const GemmArgs& g, SBuf buf0, SBuf 
 // 4-11, 16-19, 28-31, and the same of the upper half-wave: with lane group q on part q their 16 reads fall on 16 different bank
 // groups (wsw gives two on each)
 __device__ __forceinline__ int wsx(int r) { return (r & 2) | ((r >> 1) & 4); }
-template <int TG, bool SWIGLU, bool SPLIT = false>   // TG: 16-row token groups multiplied (1 .. 12)
+template <int TG, bool SWIGLU, bool SPLIT = false, typename C>   // TG: 16-row token groups multiplied (1 .. 12)
 __device__ __forceinline__ void stream8x_tile(const GemmArgs& g, const TileLds& lds, int e, int row0, int row_end, int n_tile,
-                                              bool rotate, KSlice ks = {}) {
+                                              bool rotate, C& claims, KSlice ks = {}) {
     constexpr int NBLK = SWIGLU ? 128 : 256;
     constexpr bool WIDE = TG > 8;                 // two token buffers
     constexpr int NP = (TG + 3) / 4;              // parts of a k-step
@@ -902,7 +973,7 @@ __device__ __forceinline__ void stream8x_tile(const GemmArgs& g, const TileLds& 
     constexpr int VM = WIDE ? 2 : 4 + NDT;
     static_assert(!(SPLIT && SWIGLU), "slices of k: the down projection");
     static_assert(TG >= 1 && TG <= 12, "token rows staged");
-    const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
+    const int tid = claims.thread(), lane = tid & 63, wave = uni(tid >> 6);
     const int n0 = n_tile * NBLK;
     const int K = g.K, N = g.N;
     const int npair = SPLIT ? ks.count : K >> 7;             // blocks of 128 k multiplied
@@ -1125,6 +1196,7 @@ __device__ __forceinline__ void stream8x_tile(const GemmArgs& g, const TileLds& 
     }
     multiply(V - 1);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no DMA may land in LDS after the workgroup has gone
+    claims.ask();
 
     // ---- epilogue: a lane holds 4 consecutive columns of one row per accumulator and stores them itself ----
 #pragma unroll
@@ -1161,18 +1233,28 @@ __host__ __device__ __forceinline__ int persistent_tiles(const GemmArgs& g, int 
     if (g.rem_split) return (count >> 8) + ((count & 255) > g.cold_max ? 1 : 0);
     return is_cold(g, count) ? 0 : (count + 255) >> 8;
 }
-// How many tiles at the end of that space the persistent workgroups leave to workgroups of one tile.  One persistent workgroup
-// per CU walks the space in rounds of tail_cus tiles, and a last round of a few tiles costs as much as a full one.  Cut into
-// 128-row halves those tiles occupy twice as many CUs for about 0.7 of a tile's time each, and they join the `own` tiles of
-// that kind in their rounds.  The last round moves if that makes the sum of both kinds' rounds shorter, a round of persistent tiles
-// counted 1.0 and one of the others 0.72: alone (own = 0) that is a last round of at most half the CUs; next to other work also
-// a longer one.  (That the two kinds share a launch is not in the count: with CU-time instead of rounds, DeepSeek-V2-236B, 4000
-// tokens, gains 1 %, Mixtral-8x7B, 700 and 2500, and Mixtral-8x22B, 1200, lose 6, 4 and 5 %.)  Every workgroup evaluates this on the same
-// offsets[].
-struct RoundCost { int keep, move; };       // the rounds of both kinds with the last one persistent / as halves
+// How the CUs are shared between the two kinds of tiles.  Persistent workgroups are bound by the matrix cores, tiles of one workgroup
+// mostly by the weights they stream: with every CU at the one kind and then at the other, the memory idles first and the matrix
+// cores behind it.  So `full` rounds run on every persistent workgroup, and in the rounds behind those `width` of them go on while
+// the CUs of the others fall to the tiles of one workgroup (persistent_plan).  Rounds: as many as the tiles of both kinds take
+// together, one of the others counted kStreamCost hundredths (of 36 us beside persistent tiles and 50 among its like, where a persistent
+// one takes 60: DeepSeek-V2-Lite, 4096 tokens, gate and up), rounded down: what is left of the others then runs on every CU, in
+// small pieces.  The places that the persistent tiles leave free in those rounds are taken in the longest stretch of the narrowest
+// strip that holds nearly all of them, of whole 32 CUs: the tiles that an XCD has at a time then stay whole blocks of 4 M tiles,
+// which share their panels (strips of any 8 CUs: DeepSeek-V2-236B, 32768 tokens, and DeepSeek-V3, 65536, 1 and 2 % slower
+// than without any).
+// A last round of a few tiles costs as much as a full one.  Where the others do not fill the CUs that it leaves over, and cut into
+// 128-row halves its tiles make the sum of both kinds' rounds shorter (a round of halves and others counted kHalfCost), it goes
+// to workgroups of one tile.  Every workgroup evaluates all this on the same offsets[].
+// Layers, us, every CU at the persistent tiles first and one workgroup launched per tile of the others -> this (and Claims): DeepSeek-V2-Lite
+// 1400 / 2000 / 3000 / 4096 tokens 387 / 461 / 551 / 655 -> 339 / 411 / 499 / 623, DeepSeek-V2-236B 4000 / 8000 / 16000 / 32768 2223 / 3391 /
+// 5709 / 10523 -> 2054 / 3163 / 5540 / 10405, Mixtral-8x22B 700 / 2000 1172 / 2312 -> 1076 / 2220, Mixtral-8x7B 1500 1122 -> 1056,
+// DeepSeek-V3 4096 / 8000 / 65536 3906 / 6753 / 45436 -> 3824 / 6653 / 44486.  (Strips of up to 192 CUs instead of 128: the same to 0.6 % slower.)
+constexpr int kStreamCost = 50, kHalfCost = 72, kMostAside = 128;
+struct RoundCost { int keep, move; };       // hundredths of a round, with the last one persistent / as halves
 __host__ __device__ __forceinline__ RoundCost round_cost(int total, int own, int cus) {
-    return RoundCost{100 * ((total + cus - 1) / cus) + 72 * ((own + cus - 1) / cus),
-                     100 * (total / cus) + 72 * ((own + 2 * (total % cus) + cus - 1) / cus)};
+    const int whole = 100 * ((total + cus - 1) / cus), shared = (100 * total + kStreamCost * own) / cus;
+    return RoundCost{whole > shared ? whole : shared, 100 * (total / cus) + kHalfCost * ((own + 2 * (total % cus) + cus - 1) / cus)};
 }
 __device__ __forceinline__ int tail_tiles(const GemmArgs& g, int total, int own) {
     if (g.tail_cus <= 0) return 0;
@@ -1180,6 +1262,25 @@ __device__ __forceinline__ int tail_tiles(const GemmArgs& g, int total, int own)
     if (tail == 0) return 0;
     const RoundCost c = round_cost(total, own, g.tail_cus);
     return c.move < c.keep ? tail : 0;
+}
+struct PersistentPlan { int full, width; };
+// of `grid` persistent workgroups with `total` tiles.  (Less than a round of tiles: an eighth of them on each XCD; all of an XCD's places
+// in a row, as in whole rounds, left the memory paths of the others idle: Mixtral-8x22B, 512 tokens, 1012 us with that and 988 with this.)
+__device__ __forceinline__ PersistentPlan persistent_plan(const GemmArgs& g, int total, int own, int grid) {
+    if (total <= grid) return PersistentPlan{0, (total + 7) / 8 * 8};
+    PersistentPlan p{0, grid};
+    if (own == 0 || grid < g.tail_cus) return p;
+    const int rounds = max((total + grid - 1) / grid, (total + own * kStreamCost / 100) / grid), spare = rounds * grid - total;
+    int most = 0;
+#pragma unroll
+    for (int c = kMostAside; c >= 32; c -= 32) {
+        const int b = min(rounds, spare / c);
+        if (c * b >= max(most, 1) && c < grid) {
+            most = c * b;
+            p = PersistentPlan{rounds - b, grid - c};
+        }
+    }
+    return p;
 }
 
 template <bool PAIR>   // whether an expert of PAIR_LO .. PAIR_HI rows is cut in the middle (bf16 weights)
@@ -1246,9 +1347,9 @@ __device__ __forceinline__ int sum_over_experts(const GemmArgs& g, int tid, int*
 // before the next stage's barrier leaves only the 4 weight instructions behind them in flight.
 // Weight row R of a stage (LDS row R, brought by wave R / 32): column n0 + R; gate and up: gate column n0 + R,
 // R < 128, up column n0 + R - 128 above.  k starts at stage 0 unless the kernel has the call to itself.
-template <int TG, bool SWIGLU, bool SHARED>   // TG: 16-row token groups multiplied (1 .. 12); SHARED: another tile reads these weights
+template <int TG, bool SWIGLU, bool SHARED, typename C>   // TG: 16-row token groups multiplied (1 .. 12); SHARED: another tile reads these weights
 __device__ __forceinline__ void stream16_tile(const GemmArgs& g, uint8_t* w0, uint8_t* w1, uint8_t* w2, uint8_t* t0, uint8_t* t1,
-                                              int e, int row0, int row_end, int n_tile) {
+                                              int e, int row0, int row_end, int n_tile, C& claims) {
     constexpr int NBLK = SWIGLU ? 128 : 256;
     constexpr int WM = TG >= 5 ? 2 : 1;           // sets of waves across the token groups
     constexpr int TH = (TG + WM - 1) / WM;        // token groups per wave (an odd TG: the second set's last group is padding)
@@ -1256,7 +1357,7 @@ __device__ __forceinline__ void stream16_tile(const GemmArgs& g, uint8_t* w0, ui
     constexpr int NDW = 4;                        // weight DMA instructions per wave and stage
     constexpr int NDT = (2 * TG + 7) / 8;         // token DMA instructions per wave and stage (8 rows each; 64 rows per round of the waves)
     static_assert(TG >= 1 && TG <= 12, "token rows staged");
-    const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
+    const int tid = claims.thread(), lane = tid & 63, wave = uni(tid >> 6);
     const int wm = WM == 2 ? wave >> 2 : 0, wn = WM == 2 ? wave & 3 : wave;
     const int n0 = n_tile * NBLK;
     const int K = g.K, N = g.N;
@@ -1372,6 +1473,7 @@ __device__ __forceinline__ void stream16_tile(const GemmArgs& g, uint8_t* w0, ui
     if (kt + 3 < nk) stage(kt + 3, w0, t1, w2, t0);
     if (kt + 4 < nk) stage(kt + 4, w1, t0, w0, t1);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no DMA may land in LDS after the workgroup has gone
+    claims.ask();
 
     // ---- epilogue: a lane holds 4 consecutive columns of one row per accumulator and stores them itself ----
 #pragma unroll
@@ -1386,27 +1488,43 @@ __device__ __forceinline__ void stream16_tile(const GemmArgs& g, uint8_t* w0, ui
     }
 }
 
-template <bool SWIGLU, bool SHARED>
+template <bool SWIGLU, bool SHARED, typename C>
 __device__ __forceinline__ void stream16(const GemmArgs& g, uint8_t* w0, uint8_t* w1, uint8_t* w2, uint8_t* t0, uint8_t* t1, int e,
-                                         int row0, int row_end, int n_tile) {
+                                         int row0, int row_end, int n_tile, C& claims) {
     const int tg = (row_end - row0 + 15) >> 4;
     switch (tg) {
-#define MOE_S16_CASE(n) case n: stream16_tile<n, SWIGLU, SHARED>(g, w0, w1, w2, t0, t1, e, row0, row_end, n_tile); break;
+#define MOE_S16_CASE(n) case n: stream16_tile<n, SWIGLU, SHARED>(g, w0, w1, w2, t0, t1, e, row0, row_end, n_tile, claims); break;
     MOE_S16_CASE(1) MOE_S16_CASE(2) MOE_S16_CASE(3) MOE_S16_CASE(4) MOE_S16_CASE(5) MOE_S16_CASE(6)
     MOE_S16_CASE(7) MOE_S16_CASE(8) MOE_S16_CASE(9) MOE_S16_CASE(10) MOE_S16_CASE(11)
 #undef MOE_S16_CASE
-    default: stream16_tile<12, SWIGLU, SHARED>(g, w0, w1, w2, t0, t1, e, row0, row_end, n_tile); break;
+    default: stream16_tile<12, SWIGLU, SHARED>(g, w0, w1, w2, t0, t1, e, row0, row_end, n_tile, claims); break;
     }
 }
 
-template <bool SWIGLU>
-__device__ __forceinline__ void stream8x(const GemmArgs& g, const TileLds& lds, int e, int row0, int row_end, int n_tile, bool rotate) {
+template <bool SWIGLU, typename C>
+__device__ __forceinline__ void stream8x(const GemmArgs& g, const TileLds& lds, int e, int row0, int row_end, int n_tile, bool rotate,
+                                         C& claims) {
     switch ((row_end - row0 + 15) >> 4) {
-#define MOE_S8X_CASE(n) case n: stream8x_tile<n, SWIGLU>(g, lds, e, row0, row_end, n_tile, rotate); break;
+#define MOE_S8X_CASE(n) case n: stream8x_tile<n, SWIGLU>(g, lds, e, row0, row_end, n_tile, rotate, claims); break;
     MOE_S8X_CASE(1) MOE_S8X_CASE(2) MOE_S8X_CASE(3) MOE_S8X_CASE(4) MOE_S8X_CASE(5) MOE_S8X_CASE(6)
     MOE_S8X_CASE(7) MOE_S8X_CASE(8) MOE_S8X_CASE(9) MOE_S8X_CASE(10) MOE_S8X_CASE(11)
 #undef MOE_S8X_CASE
-    default: stream8x_tile<12, SWIGLU>(g, lds, e, row0, row_end, n_tile, rotate); break;
+    default: stream8x_tile<12, SWIGLU>(g, lds, e, row0, row_end, n_tile, rotate, claims); break;
+    }
+}
+
+// the expert that M tile q belongs to: pref[e] <= q < pref[e + 1]
+struct ExpertAt { int e, first, tiles; };
+__device__ __forceinline__ ExpertAt expert_at(const int* pref, int E, int q) {
+    const int lane = threadIdx.x & 63;
+    for (int e0 = 0;; e0 += 64) {
+        const int i = min(e0 + lane, E - 1), a = pref[i], b = pref[i + 1];
+        const uint64_t m = __ballot(a <= q && q < b);
+        if (m != 0 || e0 + 64 >= E) {
+            const int l = m != 0 ? (int)__builtin_ctzll(m) : 0;
+            const int first = __builtin_amdgcn_readlane(a, l), end = __builtin_amdgcn_readlane(b, l);
+            return ExpertAt{min(e0 + l, E - 1), first, end - first};
+        }
     }
 }
 
@@ -1436,12 +1554,8 @@ __global__ __launch_bounds__(128 * WN) void grouped_gemm_kernel(GemmPair pair_of
     __shared__ int s_sel[5];
     const int tid = threadIdx.x;
 
-    // ---- XCD-aware id: groups of 4 consecutive tiles (the M tiles of one N tile first) go round-robin to the XCDs
-    // (workgroup ids are dealt to the XCDs one by one).  The tiles of a multi-tile expert that read the same
-    // weights then share them through one XCD's L2, and dealing small groups round keeps the XCDs even whatever
-    // the number of tiles and however much one expert's tiles cost more than another's ----
-    const int slot = blockIdx.x >> 3;
-    int v = (((slot >> 2) << 3) + (blockIdx.x & 7)) * 4 + (slot & 3);
+    int v = dealt_tile(blockIdx.x & 7, blockIdx.x >> 3);
+    OneTile one;
     const bool in_front = v < pair_of.shared_tiles;
     if (!in_front) v -= pair_of.shared_tiles;
 
@@ -1489,12 +1603,12 @@ __global__ __launch_bounds__(128 * WN) void grouped_gemm_kernel(GemmPair pair_of
         const int r0 = first_row + (mt_e > 1 ? m_tile * 128 : 0), r1 = mt_e > 1 ? min(row_end, r0 + 128) : row_end;
         const int rows = r1 - r0;
         if (g.alone && mt_e == 1 && rows <= 64) {
-            if (rows <= 16) stream8_tile<1, SWIGLU>(g, sb0, sb1, sb2, e, r0, r1, n_tile);
-            else if (rows <= 32) stream8_tile<2, SWIGLU>(g, sb0, sb1, sb2, e, r0, r1, n_tile);
-            else if (rows <= 48) stream8_tile<3, SWIGLU>(g, sb0, sb1, sb2, e, r0, r1, n_tile);
-            else stream8_tile<4, SWIGLU>(g, sb0, sb1, sb2, e, r0, r1, n_tile);
+            if (rows <= 16) stream8_tile<1, SWIGLU>(g, sb0, sb1, sb2, e, r0, r1, n_tile, one);
+            else if (rows <= 32) stream8_tile<2, SWIGLU>(g, sb0, sb1, sb2, e, r0, r1, n_tile, one);
+            else if (rows <= 48) stream8_tile<3, SWIGLU>(g, sb0, sb1, sb2, e, r0, r1, n_tile, one);
+            else stream8_tile<4, SWIGLU>(g, sb0, sb1, sb2, e, r0, r1, n_tile, one);
         } else {
-            stream8x<SWIGLU>(g, lds, e, r0, r1, n_tile, g.alone);
+            stream8x<SWIGLU>(g, lds, e, r0, r1, n_tile, g.alone, one);
         }
         return;
     }
@@ -1506,8 +1620,8 @@ __global__ __launch_bounds__(128 * WN) void grouped_gemm_kernel(GemmPair pair_of
     const int t0 = mt_e > 1 ? first_row + m_tile * slice : first_row, t1 = mt_e > 1 ? min(row_end, t0 + slice) : row_end;
     if (!W8 && s8_ok) {
         // bf16 weights: the weight streamer in the persistent body's order
-        if (mt_e == 1) stream16<SWIGLU, false>(g, lw0, lw1, lw2, lt0, lt1, e, t0, t1, n_tile);
-        else stream16<SWIGLU, true>(g, lw0, lw1, lw2, lt0, lt1, e, t0, t1, n_tile);
+        if (mt_e == 1) stream16<SWIGLU, false>(g, lw0, lw1, lw2, lt0, lt1, e, t0, t1, n_tile, one);
+        else stream16<SWIGLU, true>(g, lw0, lw1, lw2, lt0, lt1, e, t0, t1, n_tile, one);
         return;
     }
     // 4 GiB of gathered rows or more: the register-staged body, which addresses them with 64-bit offsets, 128 rows
@@ -1712,16 +1826,17 @@ __global__ __launch_bounds__(512) void grouped_gemm_split_kernel(GemmArgs g, int
     const int first = slice * plan.blocks;
     const KSlice ks{first, min(plan.blocks, (g.K >> 7) - first), base, part + (size_t)slice * n_rows * g.N};
     const int groups = (r1 - r0 + 15) >> 4;
+    OneTile none;
     if (plan.rows <= 64) {
-        if (groups == 1) stream8_tile<1, false, true>(g, b0, b1, b2, 0, r0, r1, n_tile, ks);
-        else if (groups == 2) stream8_tile<2, false, true>(g, b0, b1, b2, 0, r0, r1, n_tile, ks);
-        else if (groups == 3) stream8_tile<3, false, true>(g, b0, b1, b2, 0, r0, r1, n_tile, ks);
-        else stream8_tile<4, false, true>(g, b0, b1, b2, 0, r0, r1, n_tile, ks);
+        if (groups == 1) stream8_tile<1, false, true>(g, b0, b1, b2, 0, r0, r1, n_tile, none, ks);
+        else if (groups == 2) stream8_tile<2, false, true>(g, b0, b1, b2, 0, r0, r1, n_tile, none, ks);
+        else if (groups == 3) stream8_tile<3, false, true>(g, b0, b1, b2, 0, r0, r1, n_tile, none, ks);
+        else stream8_tile<4, false, true>(g, b0, b1, b2, 0, r0, r1, n_tile, none, ks);
     } else {
-        if (groups <= 5) stream8x_tile<5, false, true>(g, lds, 0, r0, r1, n_tile, true, ks);
-        else if (groups == 6) stream8x_tile<6, false, true>(g, lds, 0, r0, r1, n_tile, true, ks);
-        else if (groups == 7) stream8x_tile<7, false, true>(g, lds, 0, r0, r1, n_tile, true, ks);
-        else stream8x_tile<8, false, true>(g, lds, 0, r0, r1, n_tile, true, ks);
+        if (groups <= 5) stream8x_tile<5, false, true>(g, lds, 0, r0, r1, n_tile, true, none, ks);
+        else if (groups == 6) stream8x_tile<6, false, true>(g, lds, 0, r0, r1, n_tile, true, none, ks);
+        else if (groups == 7) stream8x_tile<7, false, true>(g, lds, 0, r0, r1, n_tile, true, none, ks);
+        else stream8x_tile<8, false, true>(g, lds, 0, r0, r1, n_tile, true, none, ks);
     }
 }
 
@@ -1860,10 +1975,15 @@ __device__ __forceinline__ void persistent_body(const GemmPair& pair_of, const S
     const int own = g.tail_cus > 0 ? sum_over_experts<NT>(g, tid, s_wtot, [&](int c) { return own_tiles<W8>(g, c); }) * g.n_tiles_n + second_tiles.own : 0;
     const int slice_tiles = run * g.n_tiles_n;   // SPLIT: tiles of one slice
     const int all = SPLIT ? slice_tiles * split.plan.slices : slice_tiles + ptiles1, total = all - tail_tiles(g, all, own);
-    const int xcd = blockIdx.x & 7, slots = grid >> 3;
-    int slot = blockIdx.x >> 3;
-    auto tile_of = [&](int sl) { return ((sl / slots) * 8 + xcd) * slots + (sl % slots); };
-    if (tile_of(slot) >= total) return;
+    const PersistentPlan plan = SPLIT ? PersistentPlan{0, grid} : persistent_plan(g, total, own, grid);
+    const int xcd = blockIdx.x & 7, place = blockIdx.x >> 3;
+    // this workgroup's it-th tile, `total` or more past its last one
+    auto tile_of = [&](int it) {
+        if (it < plan.full) return (it * 8 + xcd) * (grid >> 3) + place;
+        return place < (plan.width >> 3) ? plan.full * grid + ((it - plan.full) * 8 + xcd) * (plan.width >> 3) + place : total;
+    };
+    int it = 0;
+    if (tile_of(0) >= total) return;
 
     // Token rows come through a buffer descriptor and 32-bit byte offsets.  Gathered rows (row_map): one
     // descriptor over all of x, whose size the launcher has checked against 4 GiB, so a row_map entry
@@ -2132,7 +2252,7 @@ __device__ __forceinline__ void persistent_body(const GemmPair& pair_of, const S
     };
     static_assert(ND == 4 && (!W8 || NB == 2), "slot plan");
     // ---- tiles ----
-    setup(tile_of(slot));
+    setup(tile_of(0));
     adopt();
     // prologue: what the iterations before the first would have issued, all of it landed (the scheduler orders it as it likes)
 #pragma unroll
@@ -2153,9 +2273,9 @@ __device__ __forceinline__ void persistent_body(const GemmPair& pair_of, const S
         uint16_t* const c = c_out;
         bool more = false;
         auto next_tile = [&]() {
-            slot += slots;
-            more = tile_of(slot) < total;
-            setup(tile_of(more ? slot : slot - slots));
+            const int v = tile_of(++it);
+            more = v < total;
+            setup(more ? v : tile_of(it - 1));
         };
         constexpr std::true_type yes{};
         constexpr std::false_type no{};
@@ -2226,8 +2346,8 @@ __device__ __forceinline__ void persistent_body(const GemmPair& pair_of, const S
 
 // ---- both kinds of tiles in one launch: calls of a mean of 128 rows per expert or more ----
 //
-// One persistent workgroup per CU comes first; the workgroups of one tile behind them start as CUs fall free, so that the
-// rounds of the two kinds overlap and the launch drains once.  As two launches, one behind the other, the second's workgroups waited
+// One persistent workgroup per CU comes first; the tiles of one workgroup run on CUs that the plan leaves to them or as CUs fall free,
+// claimed by the workgroups that are there or in workgroups of their own (Claims), so that the two kinds overlap and the launch drains once.  As two launches, one behind the other, the second's workgroups waited
 // for the first's last tile (a second stream costs more than it gains).  Layers, us, two launches -> this: DeepSeek-V2-Lite, 1500 / 2200 /
 // 3000 / 4096 tokens 423 / 514 / 589 / 701 -> 411 / 493 / 577 / 689, DeepSeek-V3 4500 / 9000 4385 / 7907 -> 4276 / 7840, DeepSeek-V2-236B
 // 4000 / 9000 2286 / 3743 -> 2276 / 3735, Mixtral-8x7B 700 / 2500 714 / 1694 -> 692 / 1687; 16384 tokens and more the same.
@@ -2237,15 +2357,13 @@ __device__ __forceinline__ void persistent_body(const GemmPair& pair_of, const S
 // A workgroup of one tile: the routed experts' own tiles, the shared expert's, then the halves of the tiles that the persistent
 // workgroups leave at the end of THEIR tile space, neighbours on one XCD (the prefix is rebuilt over that space).
 struct TileTables {
-    int pref[PE + 1], wtot[8], sel[5];
+    int own[PE + 1], persistent[PE + 1], off[PE + 1], wtot[8], claim;      // M tiles of either kind in front of an expert, its first row
 };
 template <bool SWIGLU, bool W8>
-__device__ __forceinline__ void tile_body(const GemmPair& pair_of, const TileLds& lds, int* s_pref, int* s_wtot, int* s_sel, int block) {
+__device__ __forceinline__ void tile_body(const GemmPair& pair_of, const TileLds& lds, TileTables& t, int block) {
     constexpr int NT = 512;
-    const int tid = threadIdx.x;
-    const int slot = block >> 3;
-    int v = (((slot >> 2) << 3) + (block & 7)) * 4 + (slot & 3);
-    int problem = 0;
+    const int tid = threadIdx.x, xcd = block & 7;
+    const bool claiming = pair_of.claims != nullptr;
     const GemmArgs& ga = pair_of.p[0];
     int shared_first = 0, shared_end = 0;    // (requested here, so that the answer comes with that to the scan's loads)
     if (pair_of.shared_rows > 0) {
@@ -2253,47 +2371,62 @@ __device__ __forceinline__ void tile_body(const GemmPair& pair_of, const TileLds
         shared_end = pair_of.p[1].offsets[1];
     }
     ExpertOfThread mine;
-    int run = mtile_prefix_scan<NT>(ga, tid, s_pref, s_wtot, mine, [&](int c) { return own_tiles<W8>(ga, c); }, [](int, int, int) {});
-    const int total = run * ga.n_tiles_n;
-    int half = -1;
-    if (v >= total) {
-        SharedTiles s{0, 0, 0, 0};
-        if (pair_of.shared_rows > 0) s = shared_tiles_of<W8>(pair_of.p[1], uni(shared_first), uni(shared_end));
-        v -= total;
-        int shared = s.own;                          // of the shared expert in the tile space that v counts in
-        if (v >= shared) {
-            const int t = v - shared;
-            __syncthreads();             // s_wtot of the first scan has been read by everyone
-            run = mtile_prefix_scan<NT>(ga, tid, s_pref, s_wtot, mine, [&](int c) { return persistent_tiles(ga, c); }, [](int, int, int) {});
-            shared = s.persistent;
-            const int total_p = run * ga.n_tiles_n + shared;
-            const int tail = tail_tiles(ga, total_p, total + s.own);
-            if (t >= 2 * tail) return;
-            v = total_p - tail + (t >> 1);
-            half = t & 1;
-        }
-        if (v < shared) {                            // its one expert belongs to thread 0
-            problem = 1;
-            mine = ExpertOfThread{0, tid == 0 ? shared / pair_of.p[1].n_tiles_n : 0, s.first, s.end};
-        } else {
-            v -= shared;
-        }
+    const int run = mtile_prefix_scan<NT>(ga, tid, t.own, t.wtot, mine, [&](int c) { return own_tiles<W8>(ga, c); }, [&](int e, int o0, int o1) {
+        t.off[e] = o0;
+        if (e == ga.E - 1) t.off[ga.E] = o1;
+    });
+    if (tid == 0) t.own[ga.E] = run;
+    SharedTiles s{0, 0, 0, 0};
+    if (pair_of.shared_rows > 0) s = shared_tiles_of<W8>(pair_of.p[1], uni(shared_first), uni(shared_end));
+    const int own = run * ga.n_tiles_n;
+    int v = dealt_tile(xcd, block >> 3), total_p = 0, tail = 0;
+    __syncthreads();                     // t.wtot has been read, t.own is whole
+    if (claiming || v >= own + s.own) {
+        const int run_p = mtile_prefix_scan<NT>(ga, tid, t.persistent, t.wtot, mine, [&](int c) { return persistent_tiles(ga, c); }, [](int, int, int) {});
+        if (tid == 0) t.persistent[ga.E] = run_p;
+        total_p = run_p * ga.n_tiles_n + s.persistent;
+        tail = tail_tiles(ga, total_p, own + s.own);
+        __syncthreads();
     }
-    const GemmArgs& g = pair_of.p[problem];
-    const int q = v / g.n_tiles_n;
-    if (tid < g.E && mine.start <= q && q < mine.start + mine.mt) {
-        s_sel[0] = tid; s_sel[1] = mine.start; s_sel[2] = mine.mt; s_sel[3] = mine.o0; s_sel[4] = mine.o1;
+    const int limit = own + s.own + 2 * tail;
+    Claims claims{pair_of.claims, xcd, limit, 0};
+    if (claiming) {
+        claims.ask();
+        v = claims.take(&t.claim);
+    } else if (v >= limit) {
+        return;
     }
-    __syncthreads();
-    const int e = uni(s_sel[0]), pe = uni(s_sel[1]), mt_e = uni(s_sel[2]), o0 = uni(s_sel[3]), row_end = uni(s_sel[4]);
+    for (; v >= 0; v = claims.take(&t.claim)) {
+    const int* pref = t.own;
+    int half = -1, shared = 0, at = v;   // shared: tiles of the shared expert in front of the routed experts' in the space `at` counts in
+    bool of_shared = false;
+    if (v >= own + s.own) {              // a half of one of the last persistent tiles
+        const int h = v - own - s.own;
+        at = total_p - tail + (h >> 1);
+        half = h & 1;
+        pref = t.persistent;
+        shared = s.persistent;
+        of_shared = at < shared;
+        if (!of_shared) at -= shared;
+    } else if (v >= own) {
+        at = v - own;
+        shared = s.own;
+        of_shared = true;
+    }
+    const GemmArgs& g = pair_of.p[of_shared ? 1 : 0];
+    const ExpertAt x = of_shared ? ExpertAt{0, 0, shared / g.n_tiles_n} : expert_at(pref, g.E, at / g.n_tiles_n);
+    const int e = x.e, o0 = of_shared ? s.first : uni(t.off[e]), row_end = of_shared ? s.end : uni(t.off[e + 1]), mt_e = x.tiles;
     int m_tile, n_tile;
-    tile_in_expert(v - pe * g.n_tiles_n, mt_e, g.n_tiles_n, m_tile, n_tile);
+    tile_in_expert(at - x.first * g.n_tiles_n, mt_e, g.n_tiles_n, m_tile, n_tile);
     int r0, r1;
     bool neighbours = true;
     if (half >= 0) {                     // half of a 256-row tile of the persistent body's space
         r0 = o0 + m_tile * 256 + half * 128;
         r1 = min(min(row_end, o0 + (m_tile + 1) * 256), r0 + 128);
-        if (r0 >= r1) return;
+        if (r0 >= r1) {
+            claims.ask();
+            continue;
+        }
     } else {
         const int first_row = o0 + (g.rem_split ? ((row_end - o0) & ~255) : 0), rows_e = row_end - first_row;
         const int slice = !W8 && rows_e >= PAIR_LO ? half_rows(rows_e) : 128;
@@ -2301,9 +2434,10 @@ __device__ __forceinline__ void tile_body(const GemmPair& pair_of, const TileLds
         r1 = mt_e > 1 ? min(row_end, r0 + slice) : row_end;
         neighbours = mt_e > 1;
     }
-    if (W8) stream8x<SWIGLU>(g, lds, e, r0, r1, n_tile, false);
-    else if (neighbours) stream16<SWIGLU, true>(g, lds.w0, lds.w1, lds.w2, lds.t0, lds.t1, e, r0, r1, n_tile);
-    else stream16<SWIGLU, false>(g, lds.w0, lds.w1, lds.w2, lds.t0, lds.t1, e, r0, r1, n_tile);
+    if (W8) stream8x<SWIGLU>(g, lds, e, r0, r1, n_tile, false, claims);
+    else if (neighbours) stream16<SWIGLU, true>(g, lds.w0, lds.w1, lds.w2, lds.t0, lds.t1, e, r0, r1, n_tile, claims);
+    else stream16<SWIGLU, false>(g, lds.w0, lds.w1, lds.w2, lds.t0, lds.t1, e, r0, r1, n_tile, claims);
+    }
 }
 template <bool SWIGLU, bool W8, bool PAIRED>
 __global__ __launch_bounds__(512) void grouped_gemm_both_kernel(GemmPair persistent_of, GemmPair tiles_of, int persistent_grid) {
@@ -2322,10 +2456,11 @@ __global__ __launch_bounds__(512) void grouped_gemm_both_kernel(GemmPair persist
         persistent_body<SWIGLU, W8, PAIRED, false>(persistent_of, SplitArgs{}, PersistentLds{lt0, lt1, lt2, lw2, lw0, lw1,
                                                    reinterpret_cast<unsigned long long*>(lw2 + TOKENS),
                                                    reinterpret_cast<PersistentTables*>(lt1 + TOKENS)}, persistent_grid);
-    } else {
-        TileTables& t = *reinterpret_cast<TileTables*>(W8 ? tile_tables : lt2);      // (the bf16 streamer has two token buffers)
-        tile_body<SWIGLU, W8>(tiles_of, TileLds{lw0, lw1, lw2, lt0, lt1, lt2}, t.pref, t.wtot, t.sel, (int)blockIdx.x - persistent_grid);
+        if (tiles_of.claims == nullptr) return;
+        __syncthreads();                 // every wave has left the persistent body's LDS
     }
+    TileTables& t = *reinterpret_cast<TileTables*>(W8 ? tile_tables : lt2);      // (the bf16 streamer has two token buffers)
+    tile_body<SWIGLU, W8>(tiles_of, TileLds{lw0, lw1, lw2, lt0, lt1, lt2}, t, (int)blockIdx.x - (tiles_of.claims ? 0 : persistent_grid));
 }
 
 // The persistent body alone: one MLP's down projection in slices of k
@@ -2524,7 +2659,8 @@ int launch_both(const GemmPair& pair, int n_rows, hipStream_t st) {
     const long ncu = (cu_count() / 8) * 8, own = ((long)n_rows / 256 + g.E) * g.n_tiles_n + shared.persistent;
     const long persistent = own < ncu ? (own + 7) / 8 * 8 : ncu;
     // one tile per expert that has rows (bf16 weights: two), the shared expert's, and a last round's halves
-    const long grid = persistent + tile_grid((W8 ? 1 : 2) * (long)(g.E < n_rows ? g.E : n_rows) * g.n_tiles_n + shared.own + 2 * g.tail_cus);
+    const long tiles = tile_grid((W8 ? 1 : 2) * (long)(g.E < n_rows ? g.E : n_rows) * g.n_tiles_n + shared.own + 2 * g.tail_cus);
+    const long grid = pair.claims ? ncu : persistent + tiles;
     if (grid > 0x7fffffffL) {
         set_error("grouped gemm: %ld workgroups exceed the grid limit", grid);
         return MOE_ERR_INVALID;
@@ -2533,6 +2669,14 @@ int launch_both(const GemmPair& pair, int n_rows, hipStream_t st) {
     else hipLaunchKernelGGL((grouped_gemm_both_kernel<SWIGLU, W8, false>), dim3((unsigned)grid), dim3(512), 0, st, pair, pair, (int)persistent);
     MOE_HIP_CHECK(hipGetLastError());
     return MOE_OK;
+}
+
+// counters for one launch of a layer call
+inline int32_t* next_claims(LayerCall* call) {
+    if (!call || !call->claims) return nullptr;
+    int32_t* const c = call->claims;
+    call->claims += kClaimInts;
+    return c;
 }
 
 // max_rows: no expert has more rows (callers that do not know pass n_rows)
@@ -2547,6 +2691,7 @@ int launch_mt(const GemmArgs& g0, int n_rows, int max_rows, void* workspace, siz
     }
     if (max_rows <= 16 && gather_fits(g) && thin_pays(g, n_rows, nullptr)) return launch_thin<SWIGLU, W8>(g, n_rows, nullptr, call, st);
     GemmPair pair{};
+    pair.claims = next_claims(call);
     if (mean < 128 || !persistent_fits(g)) {
         g.alone = 1;
         pair.p[0] = g;
@@ -2594,7 +2739,7 @@ template <bool SWIGLU, bool W8>
 int launch_joint(const GemmArgs& routed, int n_rows, int max_rows, const GemmArgs& shared, int n_shared, LayerCall* call, hipStream_t st) {
     if (joint_thin(routed, n_rows, max_rows, shared, n_shared))
         return launch_thin<SWIGLU, W8>(routed, n_rows, SWIGLU && call && call->shared_gate_up_done ? nullptr : &shared, call, st);
-    GemmPair pair{{routed, shared}, 0, 0};
+    GemmPair pair{{routed, shared}, 0, 0, next_claims(call)};
     if (n_rows / routed.E < 128) {
         pair.p[0].alone = 1;
         pair.shared_tiles = tiles_of<!W8>(n_shared) * shared.n_tiles_n;
@@ -2690,7 +2835,7 @@ int grouped_swiglu(const moe_mlp_group& m, int32_t hidden, int32_t phases, Layer
     int rc = check_group(m, hidden, W8, who);
     if (rc != MOE_OK || m.n_rows == 0) return rc;
     hipStream_t st = as_stream(stream);
-    if (phases & MOE_PHASE_GATE_UP) rc = launch_mt<true, W8>(gate_up_args(m, hidden), m.n_rows, row_bound(m), nullptr, 0, nullptr, st);
+    if (phases & MOE_PHASE_GATE_UP) rc = launch_mt<true, W8>(gate_up_args(m, hidden), m.n_rows, row_bound(m), nullptr, 0, call, st);
     if (rc == MOE_OK && (phases & MOE_PHASE_DOWN)) 
         rc = launch_mt<false, W8>(down_args(m, hidden), m.n_rows, row_bound(m), m.workspace, m.workspace_bytes, call, st);
     return rc;
@@ -2703,8 +2848,9 @@ int grouped_swiglu_joint(const moe_mlp_group& r, const moe_mlp_group& s, int32_t
     if (rc == MOE_OK) rc = check_group(s, hidden, W8, who);
     if (rc != MOE_OK) return rc;
     if (!joins(r, s, hidden)) {
-        rc = grouped_swiglu<W8>(r, hidden, phases, nullptr, stream, who);
-        return rc != MOE_OK ? rc : grouped_swiglu<W8>(s, hidden, phases, nullptr, stream, who);
+        if (call) call->tail = nullptr;              // (what the routed experts add up is not the whole layer)
+        rc = grouped_swiglu<W8>(r, hidden, phases, call, stream, who);
+        return rc != MOE_OK ? rc : grouped_swiglu<W8>(s, hidden, phases, call, stream, who);
     }
     hipStream_t st = as_stream(stream);
     GemmArgs gate_up = gate_up_args(s, hidden), down = down_args(s, hidden);

@@ -10,7 +10,7 @@ namespace {
 
 // byte offsets of the intermediate buffers in the workspace
 struct Layout {
-    size_t logits, x_norm, offsets, one_group, perm, pos, row_map, segments, arrivals, act, y, act_shared, y_shared, total;
+    size_t logits, x_norm, offsets, one_group, perm, pos, row_map, segments, arrivals, claims, act, y, act_shared, y_shared, total;
 };
 
 Layout layout_of(const moe_layer_args& a) {
@@ -32,6 +32,7 @@ Layout layout_of(const moe_layer_args& a) {
     l.row_map = take(nk * 4);
     l.segments = take(moe_dispatch_workspace_bytes(p.n_tokens, p.top_k, p.n_experts));
     l.arrivals = take(n <= kTailTokens ? tail_arrivals(p.hidden) * 4 : 0);
+    l.claims = take(kLayerClaims * 4);
     l.act = take(nk * (size_t)a.routed->inter * 2);
     l.y = take(nk * h * 2);
     if (a.shared) {
@@ -103,6 +104,8 @@ extern "C" int moe_layer_forward(const moe_layer_args* args, void* stream) {
     }
     LayerCall call;
     call.tail = may_combine ? &tail : nullptr;
+    call.claims = d.claims = ints(l.claims);
+    d.n_claims = kLayerClaims;
 
     moe_mlp_group routed = *a.routed;
     routed.x = x; routed.x_rows = n; routed.n_rows = n * k; routed.row_map = d.row_map; routed.offsets = d.offsets;
@@ -142,8 +145,9 @@ extern "C" int moe_layer_forward(const moe_layer_args* args, void* stream) {
     if (join || !a.shared) {
         rc = layer_experts(routed, join ? &shared : nullptr, h, routed.fp8, &call, stream);
     } else {
-        rc = moe_grouped_swiglu_joint(&routed, nullptr, h, routed.fp8, MOE_PHASE_BOTH, stream);
-        if (rc == MOE_OK) rc = moe_grouped_swiglu_joint(&shared, nullptr, h, shared.fp8, MOE_PHASE_BOTH, stream);
+        call.tail = nullptr;
+        rc = layer_experts(routed, nullptr, h, routed.fp8, &call, stream);
+        if (rc == MOE_OK) rc = layer_experts(shared, nullptr, h, shared.fp8, &call, stream);
     }
     if (rc != MOE_OK || call.combined) return rc;
     if (a.norm_weight)

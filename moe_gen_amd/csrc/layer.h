@@ -50,7 +50,10 @@ struct LayerCall {
     const CombineTail* tail = nullptr;   // the combine, for a down projection that can end with it
     bool combined = false;               // (result) it did
     bool shared_gate_up_done = false;
+    int32_t* claims = nullptr;           // counters that the dispatch sets to 0, kClaimInts for each launch of the call
 };
+constexpr int kClaimStride = 32, kClaimInts = 8 * kClaimStride;      // a line per XCD
+constexpr int kLayerClaims = 4 * kClaimInts;                         // two projections, the shared expert's apart
 int layer_experts(const moe_mlp_group& routed, const moe_mlp_group* shared, int32_t hidden, int32_t fp8, LayerCall* call, void* stream);
 
 }  // namespace moe

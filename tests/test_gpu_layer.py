@@ -417,3 +417,41 @@ def test_first_call_of_a_block_on_another_stream_finds_its_tables():
                 outs.append(blk(x))
         torch.cuda.synchronize()
         assert torch.equal(outs[0], want) and torch.equal(outs[1], want)
+
+
+@pytest.mark.parametrize("name,n,E", [("deepseek_v2_lite", 1500, 64), ("deepseek_v2_lite", 700, 16), ("deepseek_v2_236b", 2000, 40),
+                                      ("mixtral_8x7b", 600, 8), ("mixtral_8x22b", 1300, 8), ("deepseek_v3_w8a16", 1500, 64),
+                                      ("deepseek_v3_w8a16", 600, 16)])
+def test_claimed_tiles_give_the_bits_of_launched_ones(name, n, E):
+    """Calls of both kinds of tiles: the layer call's workgroups claim the tiles that are not persistent ones from counters that the
+    dispatch clears, the stage-by-stage path of an attached timer launches one for each.  Skewed counts, so that experts of every
+    kind, pairs and last rounds in halves occur; again on other tokens, and in replays of a graph between eager calls."""
+    from moe_gen_amd import synthetic
+    from moe_gen_amd.block import StageTimer
+    first = lambda r: r[0] if isinstance(r, tuple) else r
+    w = synthetic.WORKLOADS[name].scaled(n=n, h=768, I=640, seq=n, E=E)
+    print(f"claimed tiles {name} n={n} E={E}", flush=True)
+    blk = synthetic.build_block(w, device="cuda", gen_device="cpu")
+    x = synthetic.hidden_states(w, "cpu").cuda()
+    more = [x, x.flip(-1).contiguous(), (0.5 * x).contiguous()]
+    blk.stage_timer = StageTimer()
+    want = [first(blk(v)).clone() for v in more]
+    blk.stage_timer = None
+    for rep in range(2):
+        for v, y in zip(more, want):
+            assert torch.equal(first(blk(v)), y), rep
+    static = x.clone()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        blk(static)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = first(blk(static))
+    for v, y in zip(more + more, want + want):
+        static.copy_(v)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, y)
+        assert torch.equal(first(blk(v)), y)
