@@ -728,6 +728,16 @@ struct TileLds {
     uint8_t *w0, *w1, *w2, *t0, *t1, *t2;
 };
 
+// Whether a call of a group has tiles of both kinds (where the persistent body can address its rows), by the mean of its rows per expert.
+// fp8 weights: from 128 rows on; sums start elsewhere in calls of one kind (k_rotation).  bf16 weights, whose sums do not depend on it:
+// the more experts there are, the lower the mean at which some of them hold most of the rows (and would be 128-row tiles that
+// fetch their weights again and again).  Layers, us, one kind -> both: 160 experts, DeepSeek-V2-236B, 500 / 900 / 1500 / 2000 / 3000 tokens
+// (means of 18 to 112) 1189 / 1407 / 1607 / 1773 / 2075 -> 1189 / 1364 / 1496 / 1583 / 1850; 64 experts, DeepSeek-V2-Lite, 350 / 512 / 700 /
+// 1000 / 1300 (32 to 121) 196 / 218 / 271 / 301 / 344 -> 234 / 225 / 261 / 286 / 332; 8 experts, Mixtral-8x7B and 8x22B, 256 and 400 (64 and
+// 100) the same to 1 % slower.
+template <bool W8>
+inline bool both_kinds(long n_rows, int E) { return E > 0 && n_rows / E >= (W8 || E < 32 ? 128 : E < 128 ? 64 : 32); }
+
 // How the down projection of one MLP is cut when its k is: row tiles of `rows` (256: on the persistent body, else on the split
 // kernel), k into `slices` of up to `blocks` blocks of 128.  part: where the fp32 sums go, [slices][n_rows][N].
 struct SplitPlan {
@@ -1249,7 +1259,8 @@ __host__ __device__ __forceinline__ int persistent_tiles(const GemmArgs& g, int 
 // Layers, us, every CU at the persistent tiles first and one workgroup launched per tile of the others -> this (and Claims): DeepSeek-V2-Lite
 // 1400 / 2000 / 3000 / 4096 tokens 387 / 461 / 551 / 655 -> 339 / 411 / 499 / 623, DeepSeek-V2-236B 4000 / 8000 / 16000 / 32768 2223 / 3391 /
 // 5709 / 10523 -> 2054 / 3163 / 5540 / 10405, Mixtral-8x22B 700 / 2000 1172 / 2312 -> 1076 / 2220, Mixtral-8x7B 1500 1122 -> 1056,
-// DeepSeek-V3 4096 / 8000 / 65536 3906 / 6753 / 45436 -> 3824 / 6653 / 44486.  (Strips of up to 192 CUs instead of 128: the same to 0.6 % slower.)
+// DeepSeek-V3 4096 / 8000 / 65536 3906 / 6753 / 45436 -> 3824 / 6653 / 44486.  (Strips of up to 192 CUs instead of 128: the same
+// to 0.6 % slower.  kStreamCost 40 and 62: -0.2 ... +5.5 % and -3.6 ... +1.5 %, 0.5 % slower and 0.2 % faster in the mean of 22 calls.)
 constexpr int kStreamCost = 50, kHalfCost = 72, kMostAside = 128;
 struct RoundCost { int keep, move; };       // hundredths of a round, with the last one persistent / as halves
 __host__ __device__ __forceinline__ RoundCost round_cost(int total, int own, int cus) {
@@ -2683,7 +2694,6 @@ inline int32_t* next_claims(LayerCall* call) {
 template <bool SWIGLU, bool W8>
 int launch_mt(const GemmArgs& g0, int n_rows, int max_rows, void* workspace, size_t workspace_bytes, LayerCall* call, hipStream_t st) {
     GemmArgs g = g0;
-    const long mean = g.E > 0 ? (long)n_rows / g.E : 0;
     if constexpr (W8 && !SWIGLU) {
         const SplitPlan plan = g.E == 1 && workspace ? split_plan(n_rows, g.K, g.n_tiles_n) : SplitPlan{};
         if (plan.slices > 1 && workspace_bytes >= (size_t)plan.slices * n_rows * g.N * 4)
@@ -2692,7 +2702,7 @@ int launch_mt(const GemmArgs& g0, int n_rows, int max_rows, void* workspace, siz
     if (max_rows <= 16 && gather_fits(g) && thin_pays(g, n_rows, nullptr)) return launch_thin<SWIGLU, W8>(g, n_rows, nullptr, call, st);
     GemmPair pair{};
     pair.claims = next_claims(call);
-    if (mean < 128 || !persistent_fits(g)) {
+    if (!both_kinds<W8>(n_rows, g.E) || !persistent_fits(g)) {
         g.alone = 1;
         pair.p[0] = g;
         return launch_tiles<4, SWIGLU, W8>(pair, n_rows, st);
@@ -2740,7 +2750,7 @@ int launch_joint(const GemmArgs& routed, int n_rows, int max_rows, const GemmArg
     if (joint_thin(routed, n_rows, max_rows, shared, n_shared))
         return launch_thin<SWIGLU, W8>(routed, n_rows, SWIGLU && call && call->shared_gate_up_done ? nullptr : &shared, call, st);
     GemmPair pair{{routed, shared}, 0, 0, next_claims(call)};
-    if (n_rows / routed.E < 128) {
+    if (!both_kinds<W8>(n_rows, routed.E)) {
         pair.p[0].alone = 1;
         pair.shared_tiles = tiles_of<!W8>(n_shared) * shared.n_tiles_n;
         return launch_tiles<4, SWIGLU, W8>(pair, n_rows, st);
@@ -2816,7 +2826,7 @@ bool joins(const moe_mlp_group& routed, const moe_mlp_group& shared, int32_t hid
     if (routed.row_map && (size_t)routed.x_rows * (size_t)hidden * 2 >= (1ull << 32)) return false;
     if (shared.row_map && (size_t)shared.x_rows * (size_t)hidden * 2 >= (1ull << 32)) return false;
     const long cus = cu_count(), cols = (shared.inter + 127) / 128, rows = shared.n_rows;
-    if (routed.n_rows / routed.n_experts >= 128)
+    if (routed.fp8 ? both_kinds<true>(routed.n_rows, routed.n_experts) : both_kinds<false>(routed.n_rows, routed.n_experts))
         return rows >= 128 && (rows + 255) / 256 * cols <= 4 * cus && hidden % 128 == 0 && routed.inter % 128 == 0 &&
                shared.inter % 128 == 0 && routed.n_experts <= 512 && cus >= 8 && !sliced(shared, hidden);
     return few_tiles(shared, cus) || ((rows + 127) / 128 * cols <= 2 * cus && !sliced(shared, hidden));

@@ -1224,3 +1224,27 @@ def test_kernel_choice_for_few_rows_leaves_the_bits(fp8, E, h, I):
     assert want.float().abs().max() > 0
     for rows in (1, 2, 3, 4, 16):
         assert torch.equal(call(rows, 16), want[:, :rows]), rows
+
+
+@pytest.mark.parametrize("E,mean", [(8, 127), (8, 128), (40, 63), (40, 64), (130, 31), (130, 32)])     # both sides of the line of both_kinds
+def test_bf16_skewed_experts_around_the_line_between_one_and_both_kinds(E, mean):
+    """A few experts hold most of the rows: 256-row tiles, pairs and slices next to small ones.  Every expert's rows equal, bit
+    for bit, those of a call with that expert alone."""
+    from moe_gen_amd import ops
+    h, I = 384, 320
+    rows = E * mean
+    counts = np.full(E, 3, np.int64)
+    counts[[1, 3, 4]] = rows // 4, 300, 190
+    counts[6] += rows - counts.sum()
+    offsets = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    print(f"skewed experts E={E} mean={mean}", flush=True)
+    assert counts.min() > 0 and offsets[-1] == rows
+    g = torch.Generator().manual_seed(E + mean)
+    x = torch.randn(rows, h, generator=g).to(torch.bfloat16).cuda()
+    mats = [[m.cuda() for m in one] for one in make_experts(E, h, I, False, E)]
+    call = lambda xs, ms, off: ops.grouped_swiglu(xs, None, ops.expert_pointers(*([m[j] for m in ms] for j in range(3))),
+                                                  torch.tensor(off, dtype=torch.int32, device="cuda"), xs.shape[0])
+    y = call(x, mats, offsets.tolist())
+    for e in (0, 1, 3, 4, 5, 6, E - 1):
+        a, b = int(offsets[e]), int(offsets[e + 1])
+        assert torch.equal(y[a:b], call(x[a:b].contiguous(), [mats[e]], [0, b - a])), f"expert {e} ({b - a} rows)"
