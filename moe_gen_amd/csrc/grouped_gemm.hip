@@ -100,6 +100,7 @@ struct GemmArgs {
                                 // stream8_tile for tiles of up to 64 rows
     int tail_cus;               // > 0: the persistent workgroups run whole rounds of this many tiles (one per CU); what
                                 // is left goes to workgroups of 128-row half tiles if that pays (tail_tiles)
+    int cut_cus;                // > 0 (bf16, tiles of one workgroup alone): the CUs, see cut_rows
 };
 
 // What a launch works on: the routed experts and a second problem of one expert with matrices, sizes and buffers of its own,
@@ -1539,6 +1540,20 @@ __device__ __forceinline__ ExpertAt expert_at(const int* pref, int E, int q) {
     }
 }
 
+// Rows above which an expert is cut into tiles of equal height (neighbours on one XCD, which share its weights through the L2), 0: as
+// tiles_of says.  A call of few tiles, a down projection of a few experts, leaves CUs without any while its tallest tiles, bound
+// by the matrix cores above about 100 rows, take longest: cut as long as every tile has a CU.  Every workgroup finds the same.
+// Mixtral-8x22B, layers of 256 / 350 tokens (tallest experts 181 and 250 rows, 192 tiles for 256 CUs) 847 / 915 -> 831 / 899 us, of fewer tokens
+// and Mixtral-8x7B the same.
+template <int NT>
+__device__ __forceinline__ int cut_rows(const GemmArgs& g, int tid, int* s_wtot) {
+    if (g.cut_cus <= 0) return 0;
+    const int low = sum_over_experts<NT>(g, tid, s_wtot, [](int c) { return (c + 95) / 96; });
+    if ((long)low * g.n_tiles_n <= g.cut_cus) return 96;
+    const int high = sum_over_experts<NT>(g, tid, s_wtot, [](int c) { return (c + 127) / 128; });
+    return (long)high * g.n_tiles_n <= g.cut_cus ? 128 : 0;
+}
+
 // One workgroup per (M tile, N tile), in calls without persistent tiles (few rows per expert, odd K).  (tile_body is its counterpart in calls
 // of both kinds: which rows a tile has, and which streamer computes them, is the same there, since a row's bits follow from it.)
 template <int WN, bool SWIGLU, bool W8>
@@ -1573,7 +1588,8 @@ __global__ __launch_bounds__(128 * WN) void grouped_gemm_kernel(GemmPair pair_of
     // ---- M-tile prefix over experts ----
     const GemmArgs& g = pair_of.p[in_front ? 1 : 0];
     ExpertOfThread mine;
-    const int run = mtile_prefix_scan<NT>(g, tid, s_pref, s_wtot, mine, [&](int c) { return tiles_of<!W8>(c); }, [](int, int, int) {});
+    const int cut = W8 || in_front ? 0 : cut_rows<NT>(g, tid, s_wtot);
+    const int run = mtile_prefix_scan<NT>(g, tid, s_pref, s_wtot, mine, [&](int c) { return cut ? (c + cut - 1) / cut : tiles_of<!W8>(c); }, [](int, int, int) {});
     if (v >= run * g.n_tiles_n) return;
     const bool s8_ok = !g.row_map || g.a_bytes < (1ull << 32);   // (the weight streamer addresses gathered rows with 32-bit offsets)
     const int q = v / g.n_tiles_n;  // global M-tile number
@@ -1627,8 +1643,9 @@ __global__ __launch_bounds__(128 * WN) void grouped_gemm_kernel(GemmPair pair_of
     // expert of PAIR_LO .. PAIR_HI rows (bf16), or a 128-row slice.
     const int rows_e = row_end - first_row;
     const bool pair = !W8 && rows_e >= PAIR_LO && rows_e <= PAIR_HI;
-    const int slice = pair ? half_rows(rows_e) : 128;
+    const int slice = cut ? ((rows_e + mt_e - 1) / mt_e + 15) & ~15 : pair ? half_rows(rows_e) : 128;
     const int t0 = mt_e > 1 ? first_row + m_tile * slice : first_row, t1 = mt_e > 1 ? min(row_end, t0 + slice) : row_end;
+    if (t0 >= t1) return;           // (heights are whole groups of 16)
     if (!W8 && s8_ok) {
         // bf16 weights: the weight streamer in the persistent body's order
         if (mt_e == 1) stream16<SWIGLU, false>(g, lw0, lw1, lw2, lt0, lt1, e, t0, t1, n_tile, one);
@@ -2494,7 +2511,8 @@ template <int WN, bool SWIGLU, bool W8>
 int launch_tiles(const GemmPair& pair, int n_rows, hipStream_t st) {
     auto kern = grouped_gemm_kernel<WN, SWIGLU, W8>;
     const GemmArgs& g = pair.p[0];
-    const long tiles = ((long)n_rows / 128 + g.E) * g.n_tiles_n;       // sum_e tiles_of(c_e) <= sum_e (c_e / 128 + 1)
+    long tiles = ((long)n_rows / 128 + g.E) * g.n_tiles_n;             // sum_e tiles_of(c_e) <= sum_e (c_e / 128 + 1)
+    if (tiles < g.cut_cus) tiles = g.cut_cus;                          // (no more than that where rows are cut lower)
     const long grid = tile_grid(tiles + pair.shared_tiles);
     if (grid > 0x7fffffffL) {
         set_error("grouped gemm: %ld workgroups exceed the grid limit", grid);
@@ -2704,6 +2722,7 @@ int launch_mt(const GemmArgs& g0, int n_rows, int max_rows, void* workspace, siz
     pair.claims = next_claims(call);
     if (!both_kinds<W8>(n_rows, g.E) || !persistent_fits(g)) {
         g.alone = 1;
+        if (!W8 && (long)g.E * g.n_tiles_n <= cu_count()) g.cut_cus = cu_count();
         pair.p[0] = g;
         return launch_tiles<4, SWIGLU, W8>(pair, n_rows, st);
     }

@@ -1248,3 +1248,38 @@ def test_bf16_skewed_experts_around_the_line_between_one_and_both_kinds(E, mean)
     for e in (0, 1, 3, 4, 5, 6, E - 1):
         a, b = int(offsets[e]), int(offsets[e + 1])
         assert torch.equal(y[a:b], call(x[a:b].contiguous(), [mats[e]], [0, b - a])), f"expert {e} ({b - a} rows)"
+
+
+@pytest.mark.parametrize("h,E,counts", [(2048, 6, [192, 97, 96, 1, 200, 130]),      # 8 column tiles an expert, 88 tiles of up to 96 rows
+                                        (4096, 8, [97, 97, 97, 97, 97, 97, 97, 97]),   # 16: as many tiles as CUs
+                                        (4096, 16, [300, 20, 700, 60, 257]),        # 16: too many of 96 rows for 256 CUs, 14 of 128
+                                        (4096, 16, [900, 3, 1, 385, 384]),          # 16: too many of 128 as well
+                                        (256, 24, [1000, 161, 64, 17])])            # one column tile, rows in up to 11 tiles
+def test_bf16_down_projection_of_few_tiles_is_cut_in_rows(h, E, counts):
+    """Heights that the call's own counts choose: rows equal, bit for bit, those of calls with 64 rows of their expert alone."""
+    from moe_gen_amd import ops
+    I = 320
+    counts = counts + [0] * (E - len(counts))
+    offsets = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    print(f"few tiles h={h} {counts}", flush=True)
+    g = torch.Generator().manual_seed(h + E)
+    act = torch.randn(int(offsets[-1]), I, generator=g).to(torch.bfloat16).cuda()
+    downs = [(torch.randn(h, I, generator=g) * 0.05).to(torch.bfloat16).cuda() for _ in counts]
+    other = torch.zeros(I, h, dtype=torch.bfloat16, device="cuda")
+
+    def down(rows, mats, off):
+        ptrs = ops.expert_pointers([other] * len(mats), [other] * len(mats), mats)
+        y = torch.full((rows.shape[0], h), 7.0, dtype=torch.bfloat16, device="cuda")
+        x = torch.zeros(rows.shape[0], h, dtype=torch.bfloat16, device="cuda")
+        m, _, _ = ops.mlp_group(x, None, ptrs, torch.tensor(off, dtype=torch.int32, device="cuda"), rows.shape[0], rows.shape[0], act=rows, y=y)
+        ops.grouped_swiglu_joint(m, None, h, False, ops.PHASE_DOWN)
+        return y
+
+    assert offsets[-1] // E < 128                      # (tiles of one workgroup alone)
+    y = down(act, downs, offsets.tolist())
+    for e in range(E):
+        if counts[e] == 0:
+            continue
+        a, b = int(offsets[e]), int(offsets[e + 1])
+        parts = [down(act[i:min(i + 64, b)].contiguous(), [downs[e]], [0, min(i + 64, b) - i]) for i in range(a, b, 64)]
+        assert torch.equal(y[a:b], torch.cat(parts)), f"expert {e} ({b - a} rows)"
