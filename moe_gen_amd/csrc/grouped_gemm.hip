@@ -161,21 +161,12 @@ __device__ __forceinline__ int dealt_tile(int xcd, int i) { return (((i >> 2) <<
 // workgroup alone stay with the launches: with claims 1 % faster where many experts have no rows, DeepSeek-V2-236B 32 and 64 tokens,
 // 2 to 3 % slower at few tiles a CU, DeepSeek-V2-Lite 32 ... 256 and DeepSeek-V3 1000.)
 struct OneTile {
-    __device__ __forceinline__ int thread() const { return threadIdx.x; }
     __device__ __forceinline__ void ask() {}
 };
 struct Claims {
     int32_t* counters;           // one per XCD, kClaimStride apart; NULL: the workgroup has one tile
     int xcd, limit;              // the tiles are those below limit
     int next;                    // what ask() found (the first lane's)
-    // the thread's number, produced where it is used: what every form of a tile derives from it is not computed in front of the loop
-    // over the tiles and kept, or spilled, through it
-    __device__ __forceinline__ int thread() const {
-        int t = threadIdx.x;
-        asm volatile("" : "+v"(t));
-        __builtin_assume(t >= 0 && t < 512);
-        return t;
-    }
     __device__ __forceinline__ int count(int from) const {
         return __hip_atomic_fetch_add(counters + from * kClaimStride, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
@@ -769,7 +760,7 @@ __device__ __forceinline__ void stream8_tile(const GemmArgs& g, SBuf buf0, SBuf 
     constexpr int VM_BLOCK = NDW + NDT;
     static_assert(!(SPLIT && SWIGLU), "slices of k: the down projection");
     static_assert(TG >= 1 && 16 * TG <= S8_TROWS, "token rows staged");
-    const int tid = claims.thread(), lane = tid & 63, wave = uni(tid >> 6);
+    const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
     const int n0 = n_tile * NBLK;
     const int K = g.K, N = g.N;
     const int npair = SPLIT ? ks.count : K >> 7;             // blocks of 128 k multiplied
@@ -984,7 +975,7 @@ __device__ __forceinline__ void stream8x_tile(const GemmArgs& g, const TileLds& 
     constexpr int VM = WIDE ? 2 : 4 + NDT;
     static_assert(!(SPLIT && SWIGLU), "slices of k: the down projection");
     static_assert(TG >= 1 && TG <= 12, "token rows staged");
-    const int tid = claims.thread(), lane = tid & 63, wave = uni(tid >> 6);
+    const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
     const int n0 = n_tile * NBLK;
     const int K = g.K, N = g.N;
     const int npair = SPLIT ? ks.count : K >> 7;             // blocks of 128 k multiplied
@@ -1369,7 +1360,7 @@ __device__ __forceinline__ void stream16_tile(const GemmArgs& g, uint8_t* w0, ui
     constexpr int NDW = 4;                        // weight DMA instructions per wave and stage
     constexpr int NDT = (2 * TG + 7) / 8;         // token DMA instructions per wave and stage (8 rows each; 64 rows per round of the waves)
     static_assert(TG >= 1 && TG <= 12, "token rows staged");
-    const int tid = claims.thread(), lane = tid & 63, wave = uni(tid >> 6);
+    const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
     const int wm = WM == 2 ? wave >> 2 : 0, wn = WM == 2 ? wave & 3 : wave;
     const int n0 = n_tile * NBLK;
     const int K = g.K, N = g.N;
@@ -1823,6 +1814,141 @@ __global__ __launch_bounds__(64) void grouped_gemm_thin_kernel(GemmPair pair_of,
     }
 }
 
+
+// ---- the gate and up projection of one fp8 MLP at few rows ----
+//
+// One wide MLP (DeepSeek-V3: 18432 columns) has tiles of 128 columns for about half of the CUs, and each takes what a CU can
+// stream, 38 GB/s, or, from some 64 rows on, what its waves can multiply.  Here a wave has 8 columns, their gate rows and
+// their up rows in one fragment of 16, and a workgroup as many waves (8 to 10) as make one tile for every CU: 9 for 18432 columns and
+// 256 CUs.  Weights (whole lines, a wave's own) and token rows reach LDS by DMA, 128 k a stage, NB stages in a ring; a lane reads 16 weights
+// at once, as in stream8_tile, so every weight is converted once.  Every tile starts its walk over k at a block of its own.
+// What bounds it: up to 32 rows the weights' way from memory, above it LDS: every wave reads all token rows for its one fragment.
+// DeepSeek-V3's dense MLP, whole call, us, thin kernel (up to 16 rows) or tile kernel -> this: 1 / 4 / 16 / 32 / 64 / 96 tokens 82 / 81 / 91 /
+// 95 / 114 / 138 -> 77 / 75 / 77 / 85 / 107 / 132; 112 148 and 148, 128 156 and 161, so that it ends at 96 rows.
+constexpr int DM_WAVES = 10, DM_ROWS = 96;       // at most
+constexpr int dm_stages(int tg) { return tg == 1 ? 6 : tg == 2 ? 5 : tg <= 4 ? 4 : 3; }      // (what fits)
+constexpr int dm_stage_bytes(int tg) { return DM_WAVES * 2048 + tg * 4096; }
+template <int TG>                                // 16-row token groups (1 .. 6)
+__device__ __forceinline__ void gate_up_few_rows(const GemmArgs& g, int n_rows, uint8_t* lds) {
+    constexpr int NB = dm_stages(TG), SB = dm_stage_bytes(TG);
+    constexpr int NDT = (TG + 1) / 2, NI = 2 + NDT;        // token DMA instructions per wave (4 rows each), all of a stage
+    static_assert(TG >= 1 && 16 * TG <= DM_ROWS && (NB - 1) * NI < 64, "stages");
+    const int lane = threadIdx.x & 63, wave = uni(threadIdx.x >> 6), waves = (int)blockDim.x >> 6;
+    const int K = g.K, N = g.N, nk = K >> 7;
+    const int rot = (int)blockIdx.x % nk;
+    const int n0 = ((int)blockIdx.x * waves + wave) * 8;   // this wave's columns (N or more: none)
+    const int col0 = min(n0, N - 8);
+    const int row0 = uni(g.offsets[0]), row_end = min(uni(g.offsets[1]), row0 + n_rows);
+    if (row0 >= row_end) return;
+    auto block_of = [&](int p) { const int b = min(p, nk - 1) + rot; return b >= nk ? b - nk : b; };
+
+    const uint8_t *bm0 = uni_ptr(g.b0[0]), *bm1 = uni_ptr(g.b1[0]);
+    gptr_f32 sc0 = (gptr_f32)(uintptr_t)uni_ptr(g.s0[0]) + (col0 >> 7) * nk, sc1 = (gptr_f32)(uintptr_t)uni_ptr(g.s1[0]) + (col0 >> 7) * nk;
+    // DMA: weights, instruction 0 the gate rows, 1 the up rows (fragment rows 0 .. 7 and 8 .. 15): row lane / 8, part lane % 8
+    const int lr = lane >> 3, pp = lane & 7;
+    uint32_t w_voff[2], t_voff[NDT], t_dst[NDT];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) w_voff[i] = (uint32_t)(col0 + lr) * (uint32_t)K + (uint32_t)((pp ^ wsw(8 * i + lr)) << 4);
+    const uint8_t* a_base = reinterpret_cast<const uint8_t*>(g.a) + (g.row_map ? (size_t)0 : (size_t)row0 * K * 2);
+    const int a_records = g.row_map ? (int)(uint32_t)g.a_bytes : (row_end - row0) * K * 2;
+#pragma unroll
+    for (int i = 0; i < NDT; ++i) {               // token rows 4 (waves i + wave) + lane / 16, chunk lane % 16
+        const int at = waves * i + wave, tr = 4 * at + (lane >> 4);
+        const int r = min(row0 + tr, row_end - 1);
+        const int src = g.row_map ? ((gptr_i32)(uintptr_t)g.row_map)[r] : r - row0;
+        t_voff[i] = (uint32_t)src * (uint32_t)(K * 2) + (uint32_t)(((lane & 15) ^ tsw(tr)) << 4);
+        if (row0 + tr >= row_end || (g.row_map && (unsigned)src >= (unsigned)g.a_rows)) t_voff[i] = 0xfffffff0u;
+        t_dst[i] = (uint32_t)uni(at < 4 * TG ? DM_WAVES * 2048 + at * 1024 : -1);      // -1: past the staged rows
+    }
+    auto dma = [&](int p, int buf) __attribute__((always_inline)) {
+        const int live = uni(p < nk ? -1 : 0);    // past the end: empty descriptors, the instructions still count
+        uint8_t* d = lds + buf * SB;
+        const uint32_t so = (uint32_t)block_of(p) * 128u;
+        const __amdgpu_buffer_rsrc_t r0d = __builtin_amdgcn_make_buffer_rsrc((void*)bm0, 0, live, 0x00020000);
+        const __amdgpu_buffer_rsrc_t r1d = __builtin_amdgcn_make_buffer_rsrc((void*)bm1, 0, live, 0x00020000);
+        const __amdgpu_buffer_rsrc_t rad = __builtin_amdgcn_make_buffer_rsrc((void*)a_base, 0, live & a_records, 0x00020000);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(r0d, (lds_u8)(d + wave * 2048), 16, w_voff[0], so, 0, 2);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(r1d, (lds_u8)(d + wave * 2048 + 1024), 16, w_voff[1], so, 0, 2);
+#pragma unroll
+        for (int i = 0; i < NDT; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rad, (lds_u8)((int)t_dst[i] < 0 ? lds + NB * SB : d + t_dst[i]), 16, t_voff[i], 2 * so, 0, 0);
+    };
+
+    const int frow = lane & 15, q = lane >> 4;
+    const int fq = ((q & 1) << 1) | (q >> 1);
+    const uint32_t w_rd = (uint32_t)(wave * 2048 + frow * 128), wkey = (uint32_t)wsw(frow);
+    const uint32_t t_rd = (uint32_t)(DM_WAVES * 2048 + frow * 256), tkey = (uint32_t)tsw(frow);
+    f32x4 acc[TG];
+#pragma unroll
+    for (int t = 0; t < TG; ++t) acc[t] = f32x4{0};
+    // lane l holds the block scales of stage 64 i + l, requested before the DMA that the waits count
+    float v0 = sc0[block_of(lane)], v1 = sc1[block_of(lane)];
+#pragma unroll
+    for (int i = 0; i < NB - 1; ++i) dma(i, i);
+    asm volatile("s_waitcnt vmcnt(%2)" : "+v"(v0), "+v"(v1) : "n"((NB - 1) * NI));
+    int buf = 0;
+    for (int p = 0; p < nk; ++p) {
+        // this wave's DMA of block p has landed and its reads of block p - 1 have returned, then everybody's: behind the barrier
+        // that block's buffer takes block p + NB - 1
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"((NB - 2) * NI) : "memory");
+        if ((p & 63) == 0 && p > 0) {
+            v0 = sc0[block_of(p + lane)];
+            v1 = sc1[block_of(p + lane)];
+            asm volatile("s_waitcnt vmcnt(0)" : "+v"(v0), "+v"(v1));
+        }
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        const uint8_t* b = lds + buf * SB;
+        const float c0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v0), p & 63));
+        const float c1 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v1), p & 63));
+        const float scale = frow < 8 ? c0 : c1;
+        u32x4 raw[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) raw[h] = *reinterpret_cast<const u32x4*>(b + w_rd + (((4 * h + fq) ^ wkey) << 4));
+        dma(p + NB - 1, buf == 0 ? NB - 1 : buf - 1);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll
+            for (int s2 = 0; s2 < 2; ++s2) {
+                const uint32_t coff = (uint32_t)(((8 * h + 2 * fq + s2) ^ tkey) << 4);
+                const bf16x8 wa = __builtin_bit_cast(bf16x8, dequant8(raw[h][2 * s2], raw[h][2 * s2 + 1], scale));
+#pragma unroll
+                for (int t = 0; t < TG; ++t) {
+                    const bf16x8 tf = *reinterpret_cast<const bf16x8*>(b + t_rd + t * 16 * 256 + coff);
+                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa, tf, acc[t], 0, 0, 0);
+                }
+            }
+        }
+        buf = buf + 1 == NB ? 0 : buf + 1;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no DMA may land in LDS after the workgroup has gone
+
+    // A lane of the lower half-wave holds 4 gate columns of a row, the same lane of the upper half their up columns: the lower half
+    // takes columns 0 and 1, the upper one 2 and 3
+#pragma unroll
+    for (int t = 0; t < TG; ++t) {
+        f32x4 gate = {0, 0, 0, 0}, up = {0, 0, 0, 0};
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const float a = acc[t][i], b = acc[t][2 + i];
+            const auto x = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
+            uint32_t lo = x[0], hi = x[1];
+            asm volatile("" : "+v"(lo), "+v"(hi));            // (here, with every lane, not where the store needs it)
+            gate[i] = __builtin_bit_cast(float, lo);
+            up[i] = __builtin_bit_cast(float, hi);
+        }
+        const u32x2 o = epilogue_pack<true>(gate, up);
+        const int r = row0 + 16 * t + frow;
+        if (r < row_end && n0 < N) *reinterpret_cast<uint32_t*>(g.c + (size_t)r * N + n0 + 4 * (q & 1) + 2 * (q >> 1)) = o[0];
+    }
+}
+template <int TG>
+__global__ __launch_bounds__(64 * DM_WAVES) void gate_up_few_rows_kernel(GemmArgs g, int n_rows) {
+    // (1 KiB that nobody reads behind the stages)
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[dm_stages(TG) * dm_stage_bytes(TG) + 1024];
+    static_assert(sizeof(lds) <= 160 * 1024, "LDS");
+    gate_up_few_rows<TG>(g, n_rows, lds);
+}
 
 // ---- split kernel: the down projection of a dense fp8 MLP at few rows ----
 //
@@ -2627,6 +2753,27 @@ SplitPlan split_plan(int n_rows, int K, int n_tiles_n) {
     return plan;
 }
 
+// waves of a workgroup of gate_up_few_rows_kernel, 0 where the others serve the call: one MLP, up to 96 rows, of as many columns as
+// make a workgroup of 8 to 10 waves for every CU.  (Fewer columns: what its workgroups would have to share of the token rows grows.)
+int few_rows_waves(const GemmArgs& g, int n_rows) {
+    const int cus = cu_count();
+    if (g.E != 1 || n_rows > DM_ROWS || cus < 8) return 0;
+    const int waves = (g.N / 8 + cus - 1) / cus;
+    return waves >= 8 && waves <= DM_WAVES && g.K < 1 << 15 ? waves : 0;
+}
+int launch_few_rows(const GemmArgs& g, int n_rows, int waves, hipStream_t st) {
+    const dim3 grid((unsigned)((g.N / 8 + waves - 1) / waves)), block((unsigned)(64 * waves));
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, st, g, n_rows); };
+    switch ((n_rows + 15) / 16) {
+#define MOE_DM_CASE(n) case n: launch(gate_up_few_rows_kernel<n>); break;
+    MOE_DM_CASE(1) MOE_DM_CASE(2) MOE_DM_CASE(3) MOE_DM_CASE(4) MOE_DM_CASE(5)
+#undef MOE_DM_CASE
+    default: launch(gate_up_few_rows_kernel<6>); break;
+    }
+    MOE_HIP_CHECK(hipGetLastError());
+    return MOE_OK;
+}
+
 int launch_split(const GemmArgs& g, int n_rows, const SplitPlan& plan, float* part, hipStream_t st) {
     const int pieces = plan.slices * g.n_tiles_n;
     if (plan.rows == 256) {
@@ -2717,11 +2864,19 @@ int launch_mt(const GemmArgs& g0, int n_rows, int max_rows, void* workspace, siz
         if (plan.slices > 1 && workspace_bytes >= (size_t)plan.slices * n_rows * g.N * 4)
             return launch_split(g, n_rows, plan, static_cast<float*>(workspace), st);
     }
+    if constexpr (W8 && SWIGLU) {
+        const int waves = gather_fits(g) ? few_rows_waves(g, n_rows) : 0;
+        if (waves > 0) return launch_few_rows(g, n_rows, waves, st);
+    }
     if (max_rows <= 16 && gather_fits(g) && thin_pays(g, n_rows, nullptr)) return launch_thin<SWIGLU, W8>(g, n_rows, nullptr, call, st);
     GemmPair pair{};
     pair.claims = next_claims(call);
-    if (!both_kinds<W8>(n_rows, g.E) || !persistent_fits(g)) {
-        g.alone = 1;
+    // (One MLP of up to 192 rows has tiles of one workgroup alone too, and the sums of a call of both kinds.  As such a call its
+    // persistent workgroups found no tile and took the first 5 us: DeepSeek-V3's dense MLP, 128 / 160 / 192 tokens 167 / 183 / 203 -> 152 / 175 /
+    // 189 us with one upload less.)
+    const bool one_kind = !both_kinds<W8>(n_rows, g.E) || !persistent_fits(g);
+    if (one_kind || (g.E == 1 && n_rows <= 192)) {
+        g.alone = one_kind;
         if (!W8 && (long)g.E * g.n_tiles_n <= cu_count()) g.cut_cus = cu_count();
         pair.p[0] = g;
         return launch_tiles<4, SWIGLU, W8>(pair, n_rows, st);

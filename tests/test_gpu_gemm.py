@@ -1283,3 +1283,45 @@ def test_bf16_down_projection_of_few_tiles_is_cut_in_rows(h, E, counts):
         a, b = int(offsets[e]), int(offsets[e + 1])
         parts = [down(act[i:min(i + 64, b)].contiguous(), [downs[e]], [0, min(i + 64, b) - i]) for i in range(a, b, 64)]
         assert torch.equal(y[a:b], torch.cat(parts)), f"expert {e} ({b - a} rows)"
+
+
+@pytest.mark.parametrize("n,I", [(1, 18432), (16, 14464), (17, 16384), (33, 16512), (48, 18432), (64, 20480), (65, 18432), (80, 20480), (81, 16384), (96, 16512), (97, 14464),
+                                 (113, 20480), (128, 18432)])       # 8, 9 and 10 waves a workgroup on 256 CUs, last tiles whole and ragged; past 96 rows
+@pytest.mark.parametrize("h", [128, 640])                           # 1 and 5 blocks of 128 k: less than the stages of a ring, and more
+def test_wide_fp8_mlp_of_few_rows(n, I, h):
+    """Gate and up projection of one wide fp8 MLP.  A token row that is 1 at one k reads a column of both matrices exactly, so that
+    act is pinned to one bf16 step (silu by the hardware exponential); dense rows against the oracle, also gathered in another
+    order with an entry outside x, bit for bit the same where the row is."""
+    from moe_gen_amd import ops
+    print(f"wide mlp n={n} I={I} h={h}", flush=True)
+    mats = make_experts(1, h, I, True, 7)[0]
+    dm = [tuple(t.cuda() for t in m) for m in mats]
+    ptrs = ops.expert_pointers(*([m[0]] for m in dm), *([m[1]] for m in dm))
+    off = torch.tensor([0, n], dtype=torch.int32, device="cuda")
+
+    def gate_up(x, row_map=None):
+        m, act, _ = ops.mlp_group(x, row_map, ptrs, off, n, n)
+        act.fill_(7.0)
+        ops.grouped_swiglu_joint(m, None, h, True, ops.PHASE_GATE_UP)
+        return act
+
+    g = torch.Generator().manual_seed(n + I)
+    k = torch.randint(0, h, (n,), generator=g)
+    one = torch.zeros(n, h)
+    one[torch.arange(n), k] = 1.0
+    gate, up = (torch.from_numpy(f32_of(m)) for m in mats[:2])
+    want = torch.nn.functional.silu(gate[:, k].t().to(torch.bfloat16)).float() * up[:, k].t().to(torch.bfloat16).float()
+    got = gate_up(one.to(torch.bfloat16).cuda()).cpu().float()
+    assert ((got - want).abs() <= 2.0 ** -6 * want.abs()).all()
+
+    x = torch.randn(n, h, generator=g).to(torch.bfloat16)
+    y = gate_up(x.cuda())
+    a = x.float() @ gate.t()
+    ref = torch.nn.functional.silu(a) * (x.float() @ up.t())
+    assert rel_max(O.bf16_to_f32(bits(y)), ref.numpy()) <= TOL
+    rm = torch.randperm(n, generator=g).to(torch.int32)
+    bad = rm.clone()
+    bad[n // 2] = n + 5
+    z = gate_up(x.cuda(), bad.cuda())
+    keep = torch.arange(n) != n // 2
+    assert torch.equal(z.cpu()[keep], y.cpu()[rm.long()][keep]) and (z.cpu()[n // 2].float() == 0).all()
