@@ -123,9 +123,8 @@ class SwiGLUMLP(nn.Module):
             raise RuntimeError("SwiGLUMLP.forward: engine-backed weights are handled by the MoE block")
         # (tables and row range travel in kernel arguments: a copy from the host would stop the stream, and tables kept
         # for the next call would hide a weight or scale that has been replaced in between)
-        ptrs = collect_pointers([self], None)
-        offsets = ops._upload_words([n << 32], x.device).view(torch.int32)
-        return ops.grouped_swiglu_one(x2d, ptrs, offsets, n).view(*shape)
+        ptrs = _pointer_table([_tensors_of(self)], one_call=True, words=(n << 32,))
+        return ops.grouped_swiglu_one(x2d, ptrs, ptrs.words.view(torch.int32), n).view(*shape)
 
 
 def _unwrap(expert):
@@ -321,12 +320,12 @@ def _addresses(rows):
     return [None if t is None else t.data_ptr() for row in rows for t in row]
 
 
-def _pointer_table(rows, one_call):
+def _pointer_table(rows, one_call, words=()):
     """ExpertPointers from a list of (gate, up, down, s_gate, s_up, s_down) tuples."""
     cols = list(zip(*rows))
     fp8 = cols[0][0].dtype == FP8
     return ops.expert_pointers(list(cols[0]), list(cols[1]), list(cols[2]),
-                               *((list(c) for c in cols[3:]) if fp8 else (None, None, None)), one_call=one_call)
+                               *((list(c) for c in cols[3:]) if fp8 else (None, None, None)), one_call=one_call, words=words)
 
 
 def engine_backed(expert) -> bool:

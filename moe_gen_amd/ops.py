@@ -167,9 +167,10 @@ class ExpertPointers:
         self.__post_init__()
 
 
-def expert_pointers(gates, ups, downs, s_gates=None, s_ups=None, s_downs=None, device=None, one_call=False) -> ExpertPointers:
+def expert_pointers(gates, ups, downs, s_gates=None, s_ups=None, s_downs=None, device=None, one_call=False, words=()) -> ExpertPointers:
     """Build pointer tables from lists of per-expert tensors: gate/up [I,h], down [h,I]
-    (bf16, or float8_e4m3fn with fp32 scales [ceil(r/128), ceil(c/128)])."""
+    (bf16, or float8_e4m3fn with fp32 scales [ceil(r/128), ceil(c/128)]).  words: 64-bit words that travel with the tables, on the
+    device as `.words`."""
     E = len(gates)
     I, h = gates[0].shape
     fp8 = gates[0].dtype == torch.float8_e4m3fn
@@ -191,10 +192,13 @@ def expert_pointers(gates, ups, downs, s_gates=None, s_ups=None, s_downs=None, d
     # All tables in one array.  The copy from the host returns when they are there, for a later call on any stream; tables
     # of one call (one_call) are written on its own stream by a small launch, without a wait.
     dev = device or gates[0].device
+    vals += words
     t = _upload_words(vals, dev) if one_call else torch.tensor(vals, dtype=torch.int64).to(dev)
     tab = [t[c * E:(c + 1) * E] for c in range(len(cols))]
     keep = tuple(tuple(ts) for _, ts, _, _ in cols)
-    return ExpertPointers(E, h, I, fp8, tab[0], tab[1], tab[2], *(tab[3:] if fp8 else (None, None, None)), keep)
+    ptrs = ExpertPointers(E, h, I, fp8, tab[0], tab[1], tab[2], *(tab[3:] if fp8 else (None, None, None)), keep)
+    ptrs.words = t[len(cols) * E:]
+    return ptrs
 
 
 def _upload_words(values, device) -> torch.Tensor:
