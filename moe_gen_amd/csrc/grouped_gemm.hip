@@ -1350,22 +1350,24 @@ __device__ __forceinline__ int sum_over_experts(const GemmArgs& g, int tid, int*
 // before the next stage's barrier leaves only the 4 weight instructions behind them in flight.
 // Weight row R of a stage (LDS row R, brought by wave R / 32): column n0 + R; gate and up: gate column n0 + R,
 // R < 128, up column n0 + R - 128 above.  k starts at stage 0 unless the kernel has the call to itself.
-template <int TG, bool SWIGLU, bool SHARED, typename C>   // TG: 16-row token groups multiplied (1 .. 12); SHARED: another tile reads these weights
+// NW waves: 8, or 4 with half the weight rows (down projection, up to 64 rows)
+template <int TG, bool SWIGLU, bool SHARED, typename C, int NW = 8>   // TG: 16-row token groups multiplied (1 .. 12); SHARED: another tile reads these weights
 __device__ __forceinline__ void stream16_tile(const GemmArgs& g, uint8_t* w0, uint8_t* w1, uint8_t* w2, uint8_t* t0, uint8_t* t1,
                                               int e, int row0, int row_end, int n_tile, C& claims) {
-    constexpr int NBLK = SWIGLU ? 128 : 256;
+    constexpr int NBLK = SWIGLU ? 128 : 32 * NW;
     constexpr int WM = TG >= 5 ? 2 : 1;           // sets of waves across the token groups
     constexpr int TH = (TG + WM - 1) / WM;        // token groups per wave (an odd TG: the second set's last group is padding)
     constexpr int NF = 2 * WM;                    // 16-row weight fragments per wave
     constexpr int NDW = 4;                        // weight DMA instructions per wave and stage
-    constexpr int NDT = (2 * TG + 7) / 8;         // token DMA instructions per wave and stage (8 rows each; 64 rows per round of the waves)
+    constexpr int NDT = (2 * TG + NW - 1) / NW;   // token DMA instructions per wave and stage (8 rows each; 8 NW rows per round of the waves)
+    static_assert(NW == 8 || (NW == 4 && !SWIGLU && TG <= 4), "halves");
     static_assert(TG >= 1 && TG <= 12, "token rows staged");
     const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
     const int wm = WM == 2 ? wave >> 2 : 0, wn = WM == 2 ? wave & 3 : wave;
     const int n0 = n_tile * NBLK;
     const int K = g.K, N = g.N;
     const int nk = K / BK;
-    const int prot = k_rotation<false>(n_tile, nk);
+    const int prot = k_rotation<false>(n0 / (SWIGLU ? 128 : 256), nk);
 
     // ---- DMA coordinates: lane l supplies row +l/8 of an instruction's 8 rows and the 16 bytes that belong at physical chunk l%8 ----
     const int lr = lane >> 3, pp = lane & 7;
@@ -1379,8 +1381,8 @@ __device__ __forceinline__ void stream16_tile(const GemmArgs& g, uint8_t* w0, ui
     const uint8_t* a_base = reinterpret_cast<const uint8_t*>(g.a) + (g.row_map ? (size_t)0 : (size_t)row0 * K * 2);
     const int a_records = g.row_map ? (int)(uint32_t)g.a_bytes : (row_end - row0) * K * 2;
 #pragma unroll
-    for (int i = 0; i < NDT; ++i) {               // token rows 64 i + 8 wave + lr; rows past the tile's last: zeros, no request
-        const int tr = 64 * i + 8 * wave + lr;
+    for (int i = 0; i < NDT; ++i) {               // token rows 8 NW i + 8 wave + lr; rows past the tile's last: zeros, no request
+        const int tr = 8 * NW * i + 8 * wave + lr;
         const int r = min(row0 + tr, row_end - 1);
         const int src = g.row_map ? ((gptr_i32)(uintptr_t)g.row_map)[r] : r - row0;
         t_voff[i] = (uint32_t)src * (uint32_t)(K * 2) + (uint32_t)((pp ^ swz(tr)) << 4);
@@ -1400,7 +1402,7 @@ __device__ __forceinline__ void stream16_tile(const GemmArgs& g, uint8_t* w0, ui
     auto dma_t = [&](int kt_pipe, uint8_t* tb, int i) __attribute__((always_inline)) {
         const int live = uni(kt_pipe < nk ? -1 : 0);
         const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)a_base, 0, live & a_records, 0x00020000);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_u8)(tb + (64 * i + 8 * wave) * ROW_B), 16, t_voff[i], stage_off(kt_pipe), 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_u8)(tb + (8 * NW * i + 8 * wave) * ROW_B), 16, t_voff[i], stage_off(kt_pipe), 0, 0);
     };
 
     // ---- operand coordinates: fragment j of the wave is LDS rows wrow(j) .. + 15 ----
@@ -1659,6 +1661,50 @@ __global__ __launch_bounds__(128 * WN) void grouped_gemm_kernel(GemmPair pair_of
             __syncthreads();
             gemm_tile<2, WN, SWIGLU, W8, false>(g, stage(0), stage(1), e, t0 + 128, t1, n_tile);
         }
+    }
+}
+
+// ---- half tiles: bf16 down projections of few tiles ----
+//
+// A down projection of few experts, or of small ones, has a fraction of a round or little more than one of 256-column tiles: the CUs left
+// over idle, and so does the memory.  Here a tile is 128 columns x up to 64 rows, a workgroup 4 waves with half the LDS, two of which
+// run on a CU: as many bytes in flight, twice as many pieces to fill the CUs with, and one's start and end beside the other's loop.  Experts
+// above 64 rows are cut evenly into neighbours that share the weights through their XCD's L2.  The bits are those of whole tiles.  (Rule and
+// figures: half_tiles_pay.)
+constexpr int HALF_ROWS = 64;
+inline __host__ __device__ int half_tiles_of(int count) { return (count + HALF_ROWS - 1) / HALF_ROWS; }
+__global__ __launch_bounds__(256, 2) void grouped_gemm_half_kernel(GemmPair pair_of) {
+    constexpr int NT = 256;
+    __shared__ __attribute__((aligned(1024))) uint8_t lw0[S8_WBYTES / 2];
+    __shared__ __attribute__((aligned(1024))) uint8_t lw1[S8_WBYTES / 2];
+    __shared__ __attribute__((aligned(1024))) uint8_t lw2[S8_WBYTES / 2];
+    __shared__ __attribute__((aligned(1024))) uint8_t lt0[HALF_ROWS * ROW_B];
+    __shared__ __attribute__((aligned(1024))) uint8_t lt1[HALF_ROWS * ROW_B];
+    __shared__ int s_pref[MAX_E + 1];
+    __shared__ int s_wtot[NT / 64];
+    const int tid = threadIdx.x;
+    int v = dealt_tile(blockIdx.x & 7, blockIdx.x >> 3);
+    const bool in_front = v < pair_of.shared_tiles;
+    if (!in_front) v -= pair_of.shared_tiles;
+    const GemmArgs& g = pair_of.p[in_front ? 1 : 0];
+    ExpertOfThread mine;
+    const int run = mtile_prefix_scan<NT>(g, tid, s_pref, s_wtot, mine, half_tiles_of, [](int, int, int) {});
+    if (v >= run * g.n_tiles_n) return;
+    if (tid == 0) s_pref[g.E] = run;
+    __syncthreads();
+    const ExpertAt x = expert_at(s_pref, g.E, v / g.n_tiles_n);
+    const int first_row = uni(g.offsets[x.e]), rows_e = uni(g.offsets[x.e + 1]) - first_row;
+    int m_tile, n_tile;
+    tile_in_expert(v - x.first * g.n_tiles_n, x.tiles, g.n_tiles_n, m_tile, n_tile);
+    const int slice = ((rows_e + x.tiles - 1) / x.tiles + 15) & ~15;
+    const int r0 = first_row + m_tile * slice, r1 = min(first_row + rows_e, r0 + slice);
+    if (r0 >= r1) return;                        // (heights are whole groups of 16)
+    OneTile one;
+    switch ((x.tiles > 1 ? 4 : 0) + ((r1 - r0 + 15) >> 4)) {
+#define MOE_HALF_CASE(n, shared) case n + 4 * shared: stream16_tile<n, false, shared, OneTile, 4>(g, lw0, lw1, lw2, lt0, lt1, x.e, r0, r1, n_tile, one); break;
+    MOE_HALF_CASE(1, false) MOE_HALF_CASE(2, false) MOE_HALF_CASE(3, false) MOE_HALF_CASE(4, false)
+    MOE_HALF_CASE(1, true) MOE_HALF_CASE(2, true) MOE_HALF_CASE(3, true) MOE_HALF_CASE(4, true)
+#undef MOE_HALF_CASE
     }
 }
 
@@ -2630,25 +2676,6 @@ __global__ __launch_bounds__(512) void grouped_gemm_persistent_split_kernel(Gemm
     persistent_body<false, true, false, true>(pair_of, split, PersistentLds{a0a, a0b, a1a, a1b, b0, b1, ptr, &tables}, (int)gridDim.x);
 }
 
-// tiles of one workgroup each, whole rounds of 8 groups of 4
-inline long tile_grid(long tiles) { return (tiles + 31) / 32 * 32; }
-
-template <int WN, bool SWIGLU, bool W8>
-int launch_tiles(const GemmPair& pair, int n_rows, hipStream_t st) {
-    auto kern = grouped_gemm_kernel<WN, SWIGLU, W8>;
-    const GemmArgs& g = pair.p[0];
-    long tiles = ((long)n_rows / 128 + g.E) * g.n_tiles_n;             // sum_e tiles_of(c_e) <= sum_e (c_e / 128 + 1)
-    if (tiles < g.cut_cus) tiles = g.cut_cus;                          // (no more than that where rows are cut lower)
-    const long grid = tile_grid(tiles + pair.shared_tiles);
-    if (grid > 0x7fffffffL) {
-        set_error("grouped gemm: %ld workgroups exceed the grid limit", grid);
-        return MOE_ERR_INVALID;
-    }
-    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(128 * WN), 0, st, pair);
-    MOE_HIP_CHECK(hipGetLastError());
-    return MOE_OK;
-}
-
 // CUs of the current device (one persistent workgroup on each)
 inline int cu_count() {
     static int cached[64] = {0};
@@ -2660,6 +2687,50 @@ inline int cu_count() {
         cached[dev] = n;
     }
     return cached[dev];
+}
+
+// tiles of one workgroup each, whole rounds of 8 groups of 4
+inline long tile_grid(long tiles) { return (tiles + 31) / 32 * 32; }
+
+// Whether a bf16 down projection of tiles of one workgroup alone runs in half tiles: whole ones for at most half of the CUs, and rows that
+// few experts have more than HALF_ROWS of; or whole ones for a second, part-filled round, and so few rows that hardly any expert is cut.
+// Layers, us, whole -> half.  Half a round, Mixtral-8x7B, 20 / 64 / 128 / 200 tokens (means of 5 to 50 rows) 505 / 520 / 537 / 557 -> 459 / 471 / 485 /
+// 500, 256 570 -> 576; two rounds, DeepSeek-V2-Lite, 20 / 32 / 64 / 128 (2 to 12) 130 / 137 / 152 / 176 -> 124 / 129 / 147 / 166, 256 and 400 the same and
+// 205 -> 212.  Three quarters of a round, Mixtral-8x22B, 20 / 64 / 256: 775 / 755 / 834 whole, 790 / 778 / 937 in halves.
+bool half_tiles_pay(const GemmArgs& g, int n_rows) {
+    const long tiles = (long)(g.E < n_rows ? g.E : n_rows) * g.n_tiles_n, cus = cu_count();
+    if (2 * tiles <= cus) return n_rows <= 48L * g.E;
+    return tiles > cus && tiles <= 2 * cus && n_rows <= 16L * g.E;
+}
+int launch_half(GemmPair pair, int n_rows, hipStream_t st) {
+    if (pair.shared_tiles > 0) {                 // (as many 256-column tiles of up to 192 rows; the host's bound of its rows follows)
+        pair.p[1].n_tiles_n = (pair.p[1].N + 127) / 128;
+        pair.shared_tiles = half_tiles_of(pair.shared_rows) * pair.p[1].n_tiles_n;
+    }
+    GemmArgs& g = pair.p[0];
+    g.n_tiles_n = (g.N + 127) / 128;
+    const long grid = tile_grid(((long)n_rows / HALF_ROWS + g.E) * g.n_tiles_n + pair.shared_tiles);
+    hipLaunchKernelGGL(grouped_gemm_half_kernel, dim3((unsigned)grid), dim3(256), 0, st, pair);
+    MOE_HIP_CHECK(hipGetLastError());
+    return MOE_OK;
+}
+
+template <int WN, bool SWIGLU, bool W8>
+int launch_tiles(const GemmPair& pair, int n_rows, hipStream_t st) {
+    auto kern = grouped_gemm_kernel<WN, SWIGLU, W8>;
+    const GemmArgs& g = pair.p[0];
+    if constexpr (!W8 && !SWIGLU)
+        if (half_tiles_pay(g, n_rows)) return launch_half(pair, n_rows, st);
+    long tiles = ((long)n_rows / 128 + g.E) * g.n_tiles_n;             // sum_e tiles_of(c_e) <= sum_e (c_e / 128 + 1)
+    if (tiles < g.cut_cus) tiles = g.cut_cus;                          // (no more than that where rows are cut lower)
+    const long grid = tile_grid(tiles + pair.shared_tiles);
+    if (grid > 0x7fffffffL) {
+        set_error("grouped gemm: %ld workgroups exceed the grid limit", grid);
+        return MOE_ERR_INVALID;
+    }
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(128 * WN), 0, st, pair);
+    MOE_HIP_CHECK(hipGetLastError());
+    return MOE_OK;
 }
 
 // waves of 32 columns that the thin kernel's down projection has at most
@@ -2927,6 +2998,7 @@ int launch_joint(const GemmArgs& routed, int n_rows, int max_rows, const GemmArg
     if (!both_kinds<W8>(n_rows, routed.E)) {
         pair.p[0].alone = 1;
         pair.shared_tiles = tiles_of<!W8>(n_shared) * shared.n_tiles_n;
+        pair.shared_rows = n_shared;
         return launch_tiles<4, SWIGLU, W8>(pair, n_rows, st);
     }
     pair.p[0] = both_kernels<W8>(routed);

@@ -1325,3 +1325,38 @@ def test_wide_fp8_mlp_of_few_rows(n, I, h):
     z = gate_up(x.cuda(), bad.cuda())
     keep = torch.arange(n) != n // 2
     assert torch.equal(z.cpu()[keep], y.cpu()[rm.long()][keep]) and (z.cpu()[n // 2].float() == 0).all()
+
+
+@pytest.mark.parametrize("h,I,E,counts", [
+    (192, 320, 12, [1, 0, 16, 17, 63, 64, 65, 100, 128, 3, 33, 48]),      # a ragged last half tile, 5 stages of 64 k; up to two slices
+    (4096, 64, 8, [48, 47, 1, 129, 90, 0, 60, 9]),                        # 128 whole tiles: half a round; one stage; three slices
+    (2048, 704, 40, [5] * 20 + [0] * 10 + [40, 64, 65, 130, 1, 2, 17, 33, 9, 20]),     # 320 whole tiles: a part-filled second round
+    (64, 448, 1, [40])])                                                  # half of a half tile
+def test_bf16_half_tiles_of_a_down_projection(h, I, E, counts):
+    """Tiles of 128 columns and up to 64 rows: rows equal, bit for bit, those of a call with 192-row tiles and persistent ones (an
+    expert of many rows behind them)."""
+    from moe_gen_amd import ops
+    print(f"half tiles h={h} I={I} {counts}", flush=True)
+    offsets = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    n, more = int(offsets[-1]), 130 * (E + 1)
+    g = torch.Generator().manual_seed(h + I)
+    act = torch.randn(n + more, I, generator=g).to(torch.bfloat16).cuda()
+    downs = [(torch.randn(h, I, generator=g) * 0.05).to(torch.bfloat16).cuda() for _ in range(E + 1)]
+    other = torch.zeros(I, h, dtype=torch.bfloat16, device="cuda")
+
+    def down(rows, mats, off):
+        ptrs = ops.expert_pointers([other] * len(mats), [other] * len(mats), mats)
+        y = torch.full((rows.shape[0], h), 7.0, dtype=torch.bfloat16, device="cuda")
+        x = torch.zeros(rows.shape[0], h, dtype=torch.bfloat16, device="cuda")
+        m, _, _ = ops.mlp_group(x, None, ptrs, torch.tensor(off, dtype=torch.int32, device="cuda"), rows.shape[0], rows.shape[0], act=rows, y=y)
+        ops.grouped_swiglu_joint(m, None, h, False, ops.PHASE_DOWN)
+        return y
+
+    y = down(act[:n].contiguous(), downs[:E], offsets.tolist())
+    big = down(act, downs, offsets.tolist() + [n + more])
+    assert torch.equal(y, big[:n])
+    ref = act[:n].float().cpu()
+    for e in range(E):
+        a, b = int(offsets[e]), int(offsets[e + 1])
+        if b > a:
+            assert rel_max(O.bf16_to_f32(bits(y[a:b])), (ref[a:b] @ downs[e].float().cpu().t()).numpy()) <= TOL
