@@ -99,7 +99,7 @@ struct GemmArgs {
     int alone;                  // 1 (fp8): no persistent tile's sums have to be matched: k_rotation, and the stage order of
                                 // stream8_tile for tiles of up to 64 rows
     int tail_cus;               // > 0: the persistent workgroups run whole rounds of this many tiles (one per CU); what
-                                // is left goes to workgroups of 128-row half tiles if that pays (tail_tiles)
+                                // is left goes to workgroups of one piece of a tile each if that pays (tail_of)
     int cut_cus;                // > 0 (bf16, tiles of one workgroup alone): the CUs, see cut_rows
 };
 
@@ -1246,25 +1246,34 @@ __host__ __device__ __forceinline__ int persistent_tiles(const GemmArgs& g, int 
 // which share their panels (strips of any 8 CUs: DeepSeek-V2-236B, 32768 tokens, and DeepSeek-V3, 65536, 1 and 2 % slower
 // than without any).
 // A last round of a few tiles costs as much as a full one.  Where the others do not fill the CUs that it leaves over, and cut into
-// 128-row halves its tiles make the sum of both kinds' rounds shorter (a round of halves and others counted kHalfCost), it goes
-// to workgroups of one tile.  Every workgroup evaluates all this on the same offsets[].
+// pieces its tiles make the sum of both kinds' rounds shorter, it goes to workgroups of one tile: as 128-row halves, or, where no
+// others share the round, in as many as three or four pieces that fit in it (next to others, which take as long as a half, they end no
+// sooner).  Every workgroup evaluates all this on the same offsets[].  Halves -> up to four pieces, us: Mixtral-8x7B, layer, 2000 / 4000 / 8000
+// tokens 1426 / 2302 / 4306 -> 1408 / 2278 / 4288; dense MLP of DeepSeek-V3, 2800 / 5000 tokens 1820 / 3186 -> 1797 / 3138 (1000: the same, a
+// quarter's weights take as long to convert as a half's).  16 other calls of those and Mixtral-8x22B: -1.0 ... +0.7 %, as one build against itself.
 // Layers, us, every CU at the persistent tiles first and one workgroup launched per tile of the others -> this (and Claims): DeepSeek-V2-Lite
 // 1400 / 2000 / 3000 / 4096 tokens 387 / 461 / 551 / 655 -> 339 / 411 / 499 / 623, DeepSeek-V2-236B 4000 / 8000 / 16000 / 32768 2223 / 3391 /
 // 5709 / 10523 -> 2054 / 3163 / 5540 / 10405, Mixtral-8x22B 700 / 2000 1172 / 2312 -> 1076 / 2220, Mixtral-8x7B 1500 1122 -> 1056,
 // DeepSeek-V3 4096 / 8000 / 65536 3906 / 6753 / 45436 -> 3824 / 6653 / 44486.  (Strips of up to 192 CUs instead of 128: the same
 // to 0.6 % slower.  kStreamCost 40 and 62: -0.2 ... +5.5 % and -3.6 ... +1.5 %, 0.5 % slower and 0.2 % faster in the mean of 22 calls.)
-constexpr int kStreamCost = 50, kHalfCost = 72, kMostAside = 128;
-struct RoundCost { int keep, move; };       // hundredths of a round, with the last one persistent / as halves
+constexpr int kStreamCost = 50, kMostAside = 128;
+struct RoundCost { int keep, move, pieces; };       // hundredths of a round, with the last one persistent / in so many pieces a tile
 __host__ __device__ __forceinline__ RoundCost round_cost(int total, int own, int cus) {
-    const int whole = 100 * ((total + cus - 1) / cus), shared = (100 * total + kStreamCost * own) / cus;
-    return RoundCost{whole > shared ? whole : shared, 100 * (total / cus) + kHalfCost * ((own + 2 * (total % cus) + cus - 1) / cus)};
+    const int whole = 100 * ((total + cus - 1) / cus), shared = (100 * total + kStreamCost * own) / cus, tail = total % cus;
+    RoundCost c{whole > shared ? whole : shared, 72 * ((own + 2 * tail + cus - 1) / cus), 2};
+    if (own == 0 && 3 * tail <= cus) { c.move = 54; c.pieces = 3; }
+    if (own == 0 && 4 * tail <= cus) { c.move = 44; c.pieces = 4; }
+    c.move += 100 * (total / cus);
+    return c;
 }
-__device__ __forceinline__ int tail_tiles(const GemmArgs& g, int total, int own) {
-    if (g.tail_cus <= 0) return 0;
+__host__ __device__ __forceinline__ int piece_rows(int pieces) { return pieces == 2 ? 128 : pieces == 3 ? 96 : 64; }
+struct Tail { int tiles, pieces; };
+__device__ __forceinline__ Tail tail_of(const GemmArgs& g, int total, int own) {
+    if (g.tail_cus <= 0) return Tail{0, 2};
     const int tail = total % g.tail_cus;
-    if (tail == 0) return 0;
+    if (tail == 0) return Tail{0, 2};
     const RoundCost c = round_cost(total, own, g.tail_cus);
-    return c.move < c.keep ? tail : 0;
+    return Tail{c.move < c.keep ? tail : 0, c.pieces};
 }
 struct PersistentPlan { int full, width; };
 // of `grid` persistent workgroups with `total` tiles.  (Less than a round of tiles: an eighth of them on each XCD; all of an XCD's places
@@ -2174,7 +2183,7 @@ __device__ __forceinline__ void persistent_body(const GemmPair& pair_of, const S
     const int ptiles1 = second_tiles.persistent;
     const int own = g.tail_cus > 0 ? sum_over_experts<NT>(g, tid, s_wtot, [&](int c) { return own_tiles<W8>(g, c); }) * g.n_tiles_n + second_tiles.own : 0;
     const int slice_tiles = run * g.n_tiles_n;   // SPLIT: tiles of one slice
-    const int all = SPLIT ? slice_tiles * split.plan.slices : slice_tiles + ptiles1, total = all - tail_tiles(g, all, own);
+    const int all = SPLIT ? slice_tiles * split.plan.slices : slice_tiles + ptiles1, total = all - tail_of(g, all, own).tiles;
     const PersistentPlan plan = SPLIT ? PersistentPlan{0, grid} : persistent_plan(g, total, own, grid);
     const int xcd = blockIdx.x & 7, place = blockIdx.x >> 3;
     // this workgroup's it-th tile, `total` or more past its last one
@@ -2579,16 +2588,17 @@ __device__ __forceinline__ void tile_body(const GemmPair& pair_of, const TileLds
     SharedTiles s{0, 0, 0, 0};
     if (pair_of.shared_rows > 0) s = shared_tiles_of<W8>(pair_of.p[1], uni(shared_first), uni(shared_end));
     const int own = run * ga.n_tiles_n;
-    int v = dealt_tile(xcd, block >> 3), total_p = 0, tail = 0;
+    int v = dealt_tile(xcd, block >> 3), total_p = 0;
+    Tail tail{0, 2};
     __syncthreads();                     // t.wtot has been read, t.own is whole
     if (claiming || v >= own + s.own) {
         const int run_p = mtile_prefix_scan<NT>(ga, tid, t.persistent, t.wtot, mine, [&](int c) { return persistent_tiles(ga, c); }, [](int, int, int) {});
         if (tid == 0) t.persistent[ga.E] = run_p;
         total_p = run_p * ga.n_tiles_n + s.persistent;
-        tail = tail_tiles(ga, total_p, own + s.own);
+        tail = tail_of(ga, total_p, own + s.own);
         __syncthreads();
     }
-    const int limit = own + s.own + 2 * tail;
+    const int limit = own + s.own + tail.pieces * tail.tiles;
     Claims claims{pair_of.claims, xcd, limit, 0};
     if (claiming) {
         claims.ask();
@@ -2598,12 +2608,12 @@ __device__ __forceinline__ void tile_body(const GemmPair& pair_of, const TileLds
     }
     for (; v >= 0; v = claims.take(&t.claim)) {
     const int* pref = t.own;
-    int half = -1, shared = 0, at = v;   // shared: tiles of the shared expert in front of the routed experts' in the space `at` counts in
+    int piece = -1, shared = 0, at = v;   // shared: tiles of the shared expert in front of the routed experts' in the space `at` counts in
     bool of_shared = false;
-    if (v >= own + s.own) {              // a half of one of the last persistent tiles
-        const int h = v - own - s.own;
-        at = total_p - tail + (h >> 1);
-        half = h & 1;
+    if (v >= own + s.own) {              // a piece of one of the last persistent tiles
+        const int h = v - own - s.own, of = h / tail.pieces;
+        at = total_p - tail.tiles + of;
+        piece = h - of * tail.pieces;
         pref = t.persistent;
         shared = s.persistent;
         of_shared = at < shared;
@@ -2620,9 +2630,9 @@ __device__ __forceinline__ void tile_body(const GemmPair& pair_of, const TileLds
     tile_in_expert(at - x.first * g.n_tiles_n, mt_e, g.n_tiles_n, m_tile, n_tile);
     int r0, r1;
     bool neighbours = true;
-    if (half >= 0) {                     // half of a 256-row tile of the persistent body's space
-        r0 = o0 + m_tile * 256 + half * 128;
-        r1 = min(min(row_end, o0 + (m_tile + 1) * 256), r0 + 128);
+    if (piece >= 0) {                    // of a 256-row tile of the persistent body's space
+        r0 = o0 + m_tile * 256 + piece * piece_rows(tail.pieces);
+        r1 = min(min(row_end, o0 + (m_tile + 1) * 256), r0 + piece_rows(tail.pieces));
         if (r0 >= r1) {
             claims.ask();
             continue;
@@ -2966,7 +2976,7 @@ int launch_mt(const GemmArgs& g0, int n_rows, int max_rows, void* workspace, siz
     // 3584 / 4096 / 8192 tokens 4.53 -> 3.99, 4.64 -> 4.31, 7.50 -> 7.41 ms (at 4096 tokens 109 of the 256 experts hold
     // 129 to 192 rows, which were padded 256-row tiles).  With bf16
     // weights it is break-even (Mixtral-8x7B 9.28 -> 9.23 ms, DeepSeek-V2-236B 11.34 -> 11.42) and not done.
-    // Last round of the persistent body (tail_tiles above): Mixtral-8x22B, 8192 tokens, down projection (6.4 rounds
+    // Last round of the persistent body (tail_of above), as halves: Mixtral-8x22B, 8192 tokens, down projection (6.4 rounds
     // of 0.4 ms) 2.82 -> 2.66 ms, step 8.31 -> 8.13; Mixtral-8x7B 9.39 -> 9.27 ms; DeepSeek-V2-Lite 0.855 -> 0.821 ms
     // (its shared expert's 128 down tiles become 256 half tiles: 0.071 -> 0.055 ms); DeepSeek-V2-236B 11.43 -> 11.46,
     // DeepSeek-V3 46.56 -> 46.54: short rounds gain nothing, a partial round of few CUs runs at a higher clock anyway.

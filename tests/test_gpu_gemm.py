@@ -1360,3 +1360,28 @@ def test_bf16_half_tiles_of_a_down_projection(h, I, E, counts):
         a, b = int(offsets[e]), int(offsets[e + 1])
         if b > a:
             assert rel_max(O.bf16_to_f32(bits(y[a:b])), (ref[a:b] @ downs[e].float().cpu().t()).numpy()) <= TOL
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("h,I", [(3072, 1536),      # 60 tiles both ways: quarters
+                                 (4352, 2176),      # 85: thirds, one workgroup less than CUs
+                                 (4608, 2304),      # 90: too many for thirds
+                                 (256, 6912)])      # gate/up: a round and 14 tiles in quarters
+def test_last_tiles_in_three_and_four_pieces(fp8, h, I):
+    """Experts of persistent tiles alone, ragged ones (230 and 193 rows) with pieces of few rows or none.  Rows equal, bit for bit, those of
+    a call that ends with an expert of 12 tiles more, where the persistent workgroups hold these."""
+    from moe_gen_amd import ops
+    counts = [512, 230, 449, 3072]
+    n, E = sum(counts[:3]), 3
+    print(f"pieces fp8={fp8} h={h} I={I}", flush=True)
+    g = torch.Generator().manual_seed(h + I)
+    x = torch.randn(sum(counts), h, generator=g).to(torch.bfloat16).cuda()
+    mats = [[[t.cuda() for t in (m if fp8 else [m])] for m in one] for one in make_experts(E + 1, h, I, fp8, I)]
+
+    def call(e, rows):
+        ptrs = ops.expert_pointers(*([m[j][part] for m in mats[:e]] for part in range(1 + fp8) for j in range(3)))
+        off = np.concatenate([[0], np.cumsum(counts[:e])]).astype(np.int32)
+        return ops.grouped_swiglu(rows, None, ptrs, torch.from_numpy(off).cuda(), rows.shape[0])
+
+    y = call(E, x[:n].contiguous())
+    assert torch.isfinite(y).all() and y.any() and torch.equal(y, call(E + 1, x)[:n])
