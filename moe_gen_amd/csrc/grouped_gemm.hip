@@ -1551,9 +1551,13 @@ template <int NT>
 __device__ __forceinline__ int cut_rows(const GemmArgs& g, int tid, int* s_wtot) {
     if (g.cut_cus <= 0) return 0;
     const int low = sum_over_experts<NT>(g, tid, s_wtot, [](int c) { return (c + 95) / 96; });
-    if ((long)low * g.n_tiles_n <= g.cut_cus) return 96;
-    const int high = sum_over_experts<NT>(g, tid, s_wtot, [](int c) { return (c + 127) / 128; });
-    return (long)high * g.n_tiles_n <= g.cut_cus ? 128 : 0;
+    int rows = 96;
+    if ((long)low * g.n_tiles_n > g.cut_cus) {
+        const int high = sum_over_experts<NT>(g, tid, s_wtot, [](int c) { return (c + 127) / 128; });
+        rows = (long)high * g.n_tiles_n <= g.cut_cus ? 128 : 0;
+    }
+    __syncthreads();                 // every wave has read s_wtot, which the scan behind this writes first thing
+    return rows;
 }
 
 // One workgroup per (M tile, N tile), in calls without persistent tiles (few rows per expert, odd K).  (tile_body is its counterpart in calls
