@@ -26,9 +26,10 @@
 //    grid is an upper bound on the tile count, surplus workgroups exit at once; the tile height (16 ... 192 rows in steps of 16)
 //    follows the expert.  They run through the weight streamers (stream16_tile, stream8x_tile, stream8_tile): weights AND token
 //    rows reach LDS by DMA, three weight buffers, one barrier per stage.
-// Kernels: grouped_gemm_both_kernel has both kinds in one launch, the persistent workgroups first (calls of a mean of 128 rows per
-// expert or more); grouped_gemm_kernel one-workgroup tiles alone (fewer rows, and what the persistent body cannot address);
-// grouped_gemm_thin_kernel waves of 16 columns (up to 16 rows per expert); the split kernels slices of k of one fp8 MLP.
+// Kernels: grouped_gemm_both_kernel has both kinds in one launch, the persistent workgroups first (calls of many rows per
+// expert: both_kinds); grouped_gemm_kernel one-workgroup tiles alone (fewer rows, and what the persistent body cannot address);
+// grouped_gemm_half_kernel halves of those (bf16 down projections of few tiles); grouped_gemm_thin_kernel waves of 16 columns (up to
+// 16 rows per expert); gate_up_few_rows_kernel a tile per CU of one wide fp8 MLP; the split kernels slices of k of one.
 //
 // Workgroup = 8 waves, two per SIMD.  v_mfma_f32_16x16x32_bf16 throughout: on real (non-zero) data this
 // chip is power-limited under MFMA load; the 16x16x32 shape moves a third less accumulator data per flop
@@ -110,7 +111,7 @@ struct GemmArgs {
 //  * a call of one kind of tiles: `shared_tiles` workgroups in front of the routed experts' are the shared expert's; those past
 //    its rows return at once.
 //  * a call of both: `shared_rows` > 0 bounds its rows, and its tiles are counted as any expert's (persistent ones in front of the
-//    routed experts'; one-workgroup tiles behind them, in front of the half tiles).
+//    routed experts'; one-workgroup tiles behind them, in front of the pieces of last tiles).
 struct GemmPair {
     GemmArgs p[2];              // routed, shared
     int shared_tiles, shared_rows;
@@ -930,7 +931,7 @@ __device__ __forceinline__ void stream8_tile(const GemmArgs& g, SBuf buf0, SBuf 
 //
 // The same division of labour as stream8_tile (8 waves x 32 weight rows, fp8 weights by DMA in whole lines, every wave
 // multiplies all token rows, a weight is converted once, by the wave that multiplies it), for tiles whose rows another
-// kernel might have computed: what an fp8 expert's full 256-row tiles leave over, the halves of the persistent body's last
+// kernel might have computed: what an fp8 expert's full 256-row tiles leave over, the pieces of the persistent body's last
 // tiles, and in calls that this kernel serves alone the experts (or 128-row slices of experts) above 64 rows.  A row's bits
 // must then not depend on who computes it, so every matrix instruction gets the k values the persistent body gives it,
 // in the same lanes: lane group q holds k = 32 s + 8 f(q) + (0..7) of k-step s, f = 0, 2, 1, 3.  Those are the 16-byte token
@@ -2182,7 +2183,7 @@ __device__ __forceinline__ void persistent_body(const GemmPair& pair_of, const S
         if (W8 && SWIGLU) s_ptr1[3] = (unsigned long long)(uintptr_t)s.s1[0];
     }
     __syncthreads();
-    // whole rounds, and the last one unless it is better off as half tiles: one-workgroup tiles, whose own are counted for that
+    // whole rounds, and the last one unless it is better off in pieces: one-workgroup tiles, whose own are counted for that
     const SharedTiles second_tiles = PAIRED ? shared_tiles_of<W8>(pair_of.p[1], uni(s_off1[0]), uni(s_off1[1])) : SharedTiles{0, 0, 0, 0};
     const int ptiles1 = second_tiles.persistent;
     const int own = g.tail_cus > 0 ? sum_over_experts<NT>(g, tid, s_wtot, [&](int c) { return own_tiles<W8>(g, c); }) * g.n_tiles_n + second_tiles.own : 0;
@@ -2557,17 +2558,17 @@ __device__ __forceinline__ void persistent_body(const GemmPair& pair_of, const S
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no DMA may land in LDS after the workgroup has gone
 }
 
-// ---- both kinds of tiles in one launch: calls of a mean of 128 rows per expert or more ----
+// ---- both kinds of tiles in one launch: calls of many rows per expert (both_kinds) ----
 //
 // One persistent workgroup per CU comes first; the tiles of one workgroup run on CUs that the plan leaves to them or as CUs fall free,
-// claimed by the workgroups that are there or in workgroups of their own (Claims), so that the two kinds overlap and the launch drains once.  As two launches, one behind the other, the second's workgroups waited
-// for the first's last tile (a second stream costs more than it gains).  Layers, us, two launches -> this: DeepSeek-V2-Lite, 1500 / 2200 /
+// claimed by the workgroups that are there or in workgroups of their own (Claims), so that the two kinds overlap and the launch
+// drains once.  As two launches, one behind the other, the second's workgroups waited for the first's last tile (a second stream costs more than it gains).  Layers, us, two launches -> this: DeepSeek-V2-Lite, 1500 / 2200 /
 // 3000 / 4096 tokens 423 / 514 / 589 / 701 -> 411 / 493 / 577 / 689, DeepSeek-V3 4500 / 9000 4385 / 7907 -> 4276 / 7840, DeepSeek-V2-236B
 // 4000 / 9000 2286 / 3743 -> 2276 / 3735, Mixtral-8x7B 700 / 2500 714 / 1694 -> 692 / 1687; 16384 tokens and more the same.
 // The two bodies take the call's arguments from two copies of them: loads that both need would move in front of the branch, and so
 // many scalar registers alive there cost the down projection 320 to 376 bytes of spills (236 -> 308 us, DeepSeek-V2-Lite, 4096 tokens).
 //
-// A workgroup of one tile: the routed experts' own tiles, the shared expert's, then the halves of the tiles that the persistent
+// A workgroup of one tile: the routed experts' own tiles, the shared expert's, then the pieces of the tiles that the persistent
 // workgroups leave at the end of THEIR tile space, neighbours on one XCD (the prefix is rebuilt over that space).
 struct TileTables {
     int own[PE + 1], persistent[PE + 1], off[PE + 1], wtot[8], claim;      // M tiles of either kind in front of an expert, its first row
@@ -2919,7 +2920,7 @@ int launch_both(const GemmPair& pair, int n_rows, hipStream_t st) {
     const SharedTiles shared = pair.shared_rows > 0 ? shared_tiles_bound<W8>(pair.p[1], pair.shared_rows) : SharedTiles{};
     const long ncu = (cu_count() / 8) * 8, own = ((long)n_rows / 256 + g.E) * g.n_tiles_n + shared.persistent;
     const long persistent = own < ncu ? (own + 7) / 8 * 8 : ncu;
-    // one tile per expert that has rows (bf16 weights: two), the shared expert's, and a last round's halves
+    // one tile per expert that has rows (bf16 weights: two), the shared expert's, and a last round's pieces (at most two for each CU)
     const long tiles = tile_grid((W8 ? 1 : 2) * (long)(g.E < n_rows ? g.E : n_rows) * g.n_tiles_n + shared.own + 2 * g.tail_cus);
     const long grid = pair.claims ? ncu : persistent + tiles;
     if (grid > 0x7fffffffL) {
