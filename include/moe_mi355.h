@@ -168,15 +168,18 @@ int moe_dispatch_static(const int32_t* topk_idx, int32_t n_tokens, int32_t top_k
  * larger experts run on 256-row tiles of persistent workgroups (with fp8 weights: their full 256-row tiles, and the
  * rows these leave over as one tile of the first kind if they are at most 192; those of a single expert, E = 1, as a padded tile
  * of the second kind where that shortens the call).  The persistent workgroups,
- * one per CU, take whole rounds of tiles; a last, partial round is cut into 128-row halves, which join the first kind, when that
+ * one per CU, take whole rounds of tiles, the last of them on fewer CUs where tiles of the first kind use the others; a last, partial
+ * round is cut into 128-row halves (thirds or quarters where they fit), which join the first kind, when that
  * shortens the rounds of both (alone: if it is at most half the CUs' worth of tiles).  Below a mean of 128 rows per expert
- * (n_rows / E), with K not a multiple of 128, with more than 512 experts or with 4 GiB or more of gathered x, all tiles are of the
- * first kind (larger experts cut into 128-row tiles).  With bf16 weights an output row's bits depend on the row and its
+ * (n_rows / E; bf16 weights: 64 from 32 experts on, 32 from 128 on), with K not a multiple of 128, with more than 512 experts or with
+ * 4 GiB or more of gathered x, all tiles are of the
+ * first kind (larger experts cut into tiles of 128 rows, or with bf16 weights and few tiles of fewer).  With bf16 weights an output row's bits depend on the row and its
  * expert's weights alone, never on the row's place among its expert's rows, on any expert's count, on the kernel that
- * computes it or on the call.  With fp8 weights that holds inside a call with both kinds of tiles, and two things
+ * computes it or on the call.  With fp8 weights that holds inside a call with both kinds of tiles, and three things
  * change the order in which a row's products are added, and with it the last bit: a call of the first kind
  * alone starts its k loops at other stages, and there an expert of up to 64 rows
- * adds the products of a stage in another order than one of more.  (The scratch of moe_mlp_workspace_bytes changes it too.)
+ * adds the products of a stage in another order than one of more; and the gate and up projection of a single wide MLP of up to 96
+ * rows (on 256 CUs 14337 to 20480 columns) starts them at stages of its own.  (The scratch of moe_mlp_workspace_bytes changes it too.)
  * Calls in which no expert has more than 16 rows run on a kernel of one wave per 32 weight rows where that is the faster one.
  */
 enum { MOE_PHASE_GATE_UP = 1, MOE_PHASE_DOWN = 2, MOE_PHASE_BOTH = 3 };
@@ -242,7 +245,7 @@ size_t moe_mlp_workspace_bytes(const moe_mlp_group* group, int32_t hidden);
  * of any intermediate size, n_experts == 1) in one call, both of the same weight type (fp8 != 0: fp8 with block scales).
  * Where moe_shared_joins says 1 they share their launches: the shared expert's tiles run next to the routed experts';
  * otherwise they run one after the other.  shared == NULL: the routed experts alone.  The bits are those of separate calls,
- * but for one case: with fp8 weights, below a mean of 128 rows per routed expert, a shared expert that is small (256-row
+ * but for two cases: an fp8 shared expert of 14337 to 20480 columns and up to 96 rows sums as in a larger call; and with fp8 weights, below a mean of 128 rows per routed expert, a shared expert that is small (256-row
  * tiles for less than 3/8 of the CUs) starts its sums at other stages than a call of its own with 128 rows or more does,
  * and is not cut into slices of k as that is if it brings scratch.
  */
