@@ -378,7 +378,7 @@ def run_workload(name: str, args, with_cpu: bool):
     torch.cuda.synchronize()
     mean_rows = w.n * w.k // w.E
     # which tiles a grouped GEMM call has follows from the mean rows per expert (grouped_gemm.hip, launch_mt):
-    # below 128 (bf16 weights: below 64 from 32 experts on, 32 from 128 on) tiles of one workgroup each alone; else both kinds (of the former, bf16: experts of up to 192 rows;
+    # below 128 (bf16 weights: below 86 from 32 experts on, 32 from 128 on) tiles of one workgroup each alone; else both kinds (of the former, bf16: experts of up to 192 rows;
     # fp8: what an expert's full 256-row tiles leave over, if at most 192 rows; either: the last round of persistent
     # tiles, in pieces, if it is at most half a round; most rows, and the time, on persistent tiles)
     persistent = mean_rows >= 128 and w.E <= 512 and w.h % 128 == 0

@@ -725,11 +725,12 @@ struct TileLds {
 // fp8 weights: from 128 rows on; sums start elsewhere in calls of one kind (k_rotation).  bf16 weights, whose sums do not depend on it:
 // the more experts there are, the lower the mean at which some of them hold most of the rows (and would be 128-row tiles that
 // fetch their weights again and again).  Layers, us, one kind -> both: 160 experts, DeepSeek-V2-236B, 500 / 900 / 1500 / 2000 / 3000 tokens
-// (means of 18 to 112) 1189 / 1407 / 1607 / 1773 / 2075 -> 1189 / 1364 / 1496 / 1583 / 1850; 64 experts, DeepSeek-V2-Lite, 350 / 512 / 700 /
-// 1000 / 1300 (32 to 121) 196 / 218 / 271 / 301 / 344 -> 234 / 225 / 261 / 286 / 332; 8 experts, Mixtral-8x7B and 8x22B, 256 and 400 (64 and
+// (means of 18 to 112) 1189 / 1407 / 1607 / 1773 / 2075 -> 1189 / 1364 / 1496 / 1583 / 1850; 64 experts, DeepSeek-V2-Lite, 350 / 512 /
+// 1000 / 1300 (32 to 121) 196 / 218 / 301 / 344 -> 234 / 225 / 286 / 332, from 700 to 895 tokens (66 to 84) 7 % slower to 6 % faster by how
+// the rounds fall out, from 910 on (85; five inputs each) never slower and 2.5 % faster in the mean; 8 experts, Mixtral-8x7B and 8x22B, 256 and 400 (64 and
 // 100) the same to 1 % slower.
 template <bool W8>
-inline bool both_kinds(long n_rows, int E) { return E > 0 && n_rows / E >= (W8 || E < 32 ? 128 : E < 128 ? 64 : 32); }
+inline bool both_kinds(long n_rows, int E) { return E > 0 && n_rows / E >= (W8 || E < 32 ? 128 : E < 128 ? 86 : 32); }
 
 // How the down projection of one MLP is cut when its k is: row tiles of `rows` (256: on the persistent body, else on the split
 // kernel), k into `slices` of up to `blocks` blocks of 128.  part: where the fp32 sums go, [slices][n_rows][N].
