@@ -1256,7 +1256,8 @@ __host__ __device__ __forceinline__ int persistent_tiles(const GemmArgs& g, int 
 // Layers, us, every CU at the persistent tiles first and one workgroup launched per tile of the others -> this (and Claims): DeepSeek-V2-Lite
 // 1400 / 2000 / 3000 / 4096 tokens 387 / 461 / 551 / 655 -> 339 / 411 / 499 / 623, DeepSeek-V2-236B 4000 / 8000 / 16000 / 32768 2223 / 3391 /
 // 5709 / 10523 -> 2054 / 3163 / 5540 / 10405, Mixtral-8x22B 700 / 2000 1172 / 2312 -> 1076 / 2220, Mixtral-8x7B 1500 1122 -> 1056,
-// DeepSeek-V3 4096 / 8000 / 65536 3906 / 6753 / 45436 -> 3824 / 6653 / 44486.  (Strips of up to 192 CUs instead of 128: the same
+// DeepSeek-V3 4096 / 8000 / 65536 3906 / 6753 / 45436 -> 3824 / 6653 / 44486.  Between sizes it goes by how the rounds fall out: of three pairs of
+// inputs Mixtral-8x22B, 750 / 800 / 850 tokens, three are 12 % faster, three 1.3 to 2.5 % slower (1315 -> 1348).  (Strips of up to 192 CUs instead of 128: the same
 // to 0.6 % slower.  kStreamCost 40 and 62: -0.2 ... +5.5 % and -3.6 ... +1.5 %, 0.5 % slower and 0.2 % faster in the mean of 22 calls.)
 constexpr int kStreamCost = 50, kMostAside = 128;
 struct RoundCost { int keep, move, pieces; };       // hundredths of a round, with the last one persistent / in so many pieces a tile
@@ -1548,7 +1549,7 @@ __device__ __forceinline__ ExpertAt expert_at(const int* pref, int E, int q) {
 // tiles_of says.  A call of few tiles, a down projection of a few experts, leaves CUs without any while its tallest tiles, bound
 // by the matrix cores above about 100 rows, take longest: cut as long as every tile has a CU.  Every workgroup finds the same.
 // Mixtral-8x22B, layers of 256 / 350 tokens (tallest experts 181 and 250 rows, 192 tiles for 256 CUs) 847 / 915 -> 831 / 899 us, of fewer tokens
-// and Mixtral-8x7B the same.
+// the same, Mixtral-8x7B of 256 to 400 tokens 0 to 0.5 % slower, which is the counting.
 template <int NT>
 __device__ __forceinline__ int cut_rows(const GemmArgs& g, int tid, int* s_wtot) {
     if (g.cut_cus <= 0) return 0;
