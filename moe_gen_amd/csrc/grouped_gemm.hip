@@ -3006,13 +3006,13 @@ inline bool joint_thin(const GemmArgs& routed, int n_rows, int max_rows, const G
     return max_rows <= 16 && n_shared <= 16 && thin_pays(routed, n_rows, &shared);
 }
 
-// The shared expert's tiles in the routed experts' launches.  shared.alone: see joint_alone.
+// The shared expert's tiles in the routed experts' launches.  both: see joint_both; shared.alone: see joint_alone.
 template <bool SWIGLU, bool W8>
-int launch_joint(const GemmArgs& routed, int n_rows, int max_rows, const GemmArgs& shared, int n_shared, LayerCall* call, hipStream_t st) {
+int launch_joint(const GemmArgs& routed, int n_rows, int max_rows, const GemmArgs& shared, int n_shared, bool both, LayerCall* call, hipStream_t st) {
     if (joint_thin(routed, n_rows, max_rows, shared, n_shared))
         return launch_thin<SWIGLU, W8>(routed, n_rows, SWIGLU && call && call->shared_gate_up_done ? nullptr : &shared, call, st);
     GemmPair pair{{routed, shared}, 0, 0, next_claims(call)};
-    if (!both_kinds<W8>(n_rows, routed.E)) {
+    if (!both) {
         pair.p[0].alone = 1;
         pair.shared_tiles = tiles_of<!W8>(n_shared) * shared.n_tiles_n;
         pair.shared_rows = n_shared;
@@ -3075,24 +3075,31 @@ bool sliced(const moe_mlp_group& m, int32_t hidden) {
 // Whether 256-row tiles of the group (its gate and up projection) are fewer than 3/8 of the CUs
 bool few_tiles(const moe_mlp_group& m, long cus) { return (long)(m.n_rows / 256 + 1) * ((m.inter + 127) / 128) * 8 < 3 * cus; }
 
-// Whether the shared expert's tiles join the routed experts' launches.  Where the routed call has both kinds of tiles they do if a
+// Whether a joint call has tiles of both kinds: the routed experts' call would, and the persistent body can address both problems.
+// (Where it cannot, for sizes that are odd multiples of 64, the call has one kind of tiles, like one of a lower mean.)
+bool joint_both(bool w8, const moe_mlp_group& routed, const moe_mlp_group& shared, int32_t hidden) {
+    return (w8 ? both_kinds<true>(routed.n_rows, routed.n_experts) : both_kinds<false>(routed.n_rows, routed.n_experts)) &&
+           shared.n_rows >= 128 && hidden % 128 == 0 && routed.inter % 128 == 0 && shared.inter % 128 == 0 && routed.n_experts <= 512 &&
+           cu_count() >= 8;
+}
+
+// Whether the shared expert's tiles join the routed experts' launches.  Where the joint call has both kinds of tiles they do if a
 // call of its own would have both as well (128 rows, no slices of k), up to four rounds of tiles of its own (beyond, the same
-// within 0.2 %): the two then fill their last rounds together.  Where the routed call has one-workgroup tiles (or the
-// thin kernel's waves) alone, a few tiles always do; more of them up to two of that kernel's 128-row tiles, all that
+// within 0.2 %): the two then fill their last rounds together.  Where it has one-workgroup tiles (or the
+// thin kernel's waves) alone, below a mean of 128 rows, a few tiles always do; more of them up to two of that kernel's 128-row tiles, all that
 // the shared expert gets there, per CU, unless its own call is in slices.
 // Layers, us, apart -> joined.  Both kinds: DeepSeek-V2-Lite 1400 / 2000 / 2777 / 4096 tokens 439 / 514 / 585 / 725 -> 397 / 470 /
 // 563 / 699; DeepSeek-V3 4096 / 6000 4046 / 5498 -> 4004 / 5367, 16384 the same.  One kind: DeepSeek-V2-Lite 1024 / 1300 366 /
-// 409 -> 322 / 351; DeepSeek-V2-236B 1024 / 1500 1463 / 1641 -> 1416 / 1615, 2048 the same, 3000 2074 -> 2090 (not joined: 576 tiles);
+// 409 -> 322 / 351, its hidden size 2112 instead of 2048, 1000 tokens, 335 -> 316; DeepSeek-V2-236B 1024 / 1500 1463 / 1641 -> 1416 / 1615, 2048 the same, 3000 2074 -> 2090 (not joined: 576 tiles);
 // DeepSeek-V3 1500 / 2997 / 4000 2507 / 3437 / 4139 -> 2470 / 3382 / 4120.
 bool joins(const moe_mlp_group& routed, const moe_mlp_group& shared, int32_t hidden) {
     if (routed.n_rows < 1 || shared.n_rows < 1 || routed.n_experts < 1 || shared.n_experts != 1 || hidden < 1) return false;
     if (routed.row_map && (size_t)routed.x_rows * (size_t)hidden * 2 >= (1ull << 32)) return false;
     if (shared.row_map && (size_t)shared.x_rows * (size_t)hidden * 2 >= (1ull << 32)) return false;
     const long cus = cu_count(), cols = (shared.inter + 127) / 128, rows = shared.n_rows;
-    if (routed.fp8 ? both_kinds<true>(routed.n_rows, routed.n_experts) : both_kinds<false>(routed.n_rows, routed.n_experts))
-        return rows >= 128 && (rows + 255) / 256 * cols <= 4 * cus && hidden % 128 == 0 && routed.inter % 128 == 0 &&
-               shared.inter % 128 == 0 && routed.n_experts <= 512 && cus >= 8 && !sliced(shared, hidden);
-    return few_tiles(shared, cus) || ((rows + 127) / 128 * cols <= 2 * cus && !sliced(shared, hidden));
+    if (joint_both(routed.fp8, routed, shared, hidden)) return (rows + 255) / 256 * cols <= 4 * cus && !sliced(shared, hidden);
+    return routed.n_rows / routed.n_experts < 128 &&
+           (few_tiles(shared, cus) || ((rows + 127) / 128 * cols <= 2 * cus && !sliced(shared, hidden)));
 }
 
 // fp8 weights, a joint call that one kernel serves: whether the shared expert's sums start at the stages of that kernel's own
@@ -3127,11 +3134,12 @@ int grouped_swiglu_joint(const moe_mlp_group& r, const moe_mlp_group& s, int32_t
     }
     hipStream_t st = as_stream(stream);
     GemmArgs gate_up = gate_up_args(s, hidden), down = down_args(s, hidden);
+    const bool both = joint_both(W8, r, s, hidden);
     if (W8) gate_up.alone = down.alone = joint_alone(s);
     if (phases & MOE_PHASE_GATE_UP)
-        rc = launch_joint<true, W8>(gate_up_args(r, hidden), r.n_rows, row_bound(r), gate_up, s.n_rows, call, st);
+        rc = launch_joint<true, W8>(gate_up_args(r, hidden), r.n_rows, row_bound(r), gate_up, s.n_rows, both, call, st);
     if (rc == MOE_OK && (phases & MOE_PHASE_DOWN))
-        rc = launch_joint<false, W8>(down_args(r, hidden), r.n_rows, row_bound(r), down, s.n_rows, call, st);
+        rc = launch_joint<false, W8>(down_args(r, hidden), r.n_rows, row_bound(r), down, s.n_rows, both, call, st);
     return rc;
 }
 

@@ -896,6 +896,37 @@ def test_shared_expert_in_the_launches_of_both_kernels(fp8, n, E, I, shared_inte
     assert torch.equal(y1, y2) and torch.equal(sh1, sh2)
 
 
+@pytest.mark.parametrize("n,E,k,h,I,shared_inter", [
+    (1100, 130, 4, 320, 1152, 384), (1100, 130, 4, 384, 1088, 384), (1100, 130, 4, 384, 1152, 448),     # one size an odd multiple of 64
+    (1000, 64, 6, 320, 2176, 384),
+    (120, 130, 36, 384, 1152, 384)])                                                                    # fewer rows than 128
+def test_bf16_shared_expert_stays_in_the_launches_where_persistent_tiles_cannot_have_it(n, E, k, h, I, shared_inter):
+    """Means of 33 and 93 rows, at which the routed experts' own call has both kinds of tiles where the persistent body can address it:
+    a joint call that it cannot serve has one kind.  Bit for bit two calls apart."""
+    from moe_gen_amd import ops
+    print(f"joint, one kind n={n} E={E} h={h} I={I} shared_inter={shared_inter}", flush=True)
+    g = torch.Generator().manual_seed(n)
+    tables = []
+    for count, inter, seed in ((E, I, 61), (1, shared_inter, 62)):
+        one = [m.cuda() for m in make_experts(1, h, inter, False, seed)[0]]
+        tables.append(ops.expert_pointers(*([m] * count for m in one)))
+    idx = (torch.rand((n, E), generator=g) + 0.004 * torch.arange(E)).topk(k, dim=1).indices.to(torch.int32)
+    x = torch.randn(n, h, generator=g).to(torch.bfloat16).cuda()
+    d = ops.dispatch(idx.cuda(), E, None, want_row_map=True)
+    so = torch.tensor([0, n], dtype=torch.int32, device="cuda")
+    r1, _, y1 = ops.mlp_group(x, d.row_map, tables[0], d.offsets, n * k, n)
+    s1, _, sh1 = ops.mlp_group(x, None, tables[1], so, n)
+    y1.fill_(7.0); sh1.fill_(7.0)
+    assert ops.shared_joins(r1, s1, h)
+    ops.grouped_swiglu_joint(r1, s1, h, False)
+    r2, _, y2 = ops.mlp_group(x, d.row_map, tables[0], d.offsets, n * k, n)
+    s2, _, sh2 = ops.mlp_group(x, None, tables[1], so, n)
+    ops.grouped_swiglu_joint(r2, None, h, False)
+    ops.grouped_swiglu_joint(s2, None, h, False)
+    torch.cuda.synchronize()
+    assert torch.equal(y1, y2) and torch.equal(sh1, sh2) and torch.isfinite(y1).all()
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("E", [2, 16])          # routed experts of 256 rows (both kinds of tiles) and of 32 (one kind)
 @pytest.mark.parametrize("n_rows,rows", [
