@@ -171,7 +171,7 @@ int moe_dispatch_static(const int32_t* topk_idx, int32_t n_tokens, int32_t top_k
  * one per CU, take whole rounds of tiles, the last of them on fewer CUs where tiles of the first kind use the others; a last, partial
  * round is cut into 128-row halves (thirds or quarters where they fit), which join the first kind, when that
  * shortens the rounds of both (alone: if it is at most half the CUs' worth of tiles).  Below a mean of 128 rows per expert
- * (n_rows / E; bf16 weights: 86 from 32 experts on, 32 from 128 on), with K not a multiple of 128, with more than 512 experts or with
+ * (n_rows / E; 64 experts and more of bf16 weights: down to 32 rows, the larger the weights the fewer), with K not a multiple of 128, with more than 512 experts or with
  * 4 GiB or more of gathered x, all tiles are of the
  * first kind (larger experts cut into tiles of 128 rows, or with bf16 weights and few tiles of fewer).  With bf16 weights an output row's bits depend on the row and its
  * expert's weights alone, never on the row's place among its expert's rows, on any expert's count, on the kernel that

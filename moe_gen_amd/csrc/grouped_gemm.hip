@@ -721,16 +721,22 @@ struct TileLds {
     uint8_t *w0, *w1, *w2, *t0, *t1, *t2;
 };
 
-// Whether a call of a group has tiles of both kinds (where the persistent body can address its rows), by the mean of its rows per expert.
-// fp8 weights: from 128 rows on; sums start elsewhere in calls of one kind (k_rotation).  bf16 weights, whose sums do not depend on it:
-// the more experts there are, the lower the mean at which some of them hold most of the rows (and would be 128-row tiles that
-// fetch their weights again and again).  Layers, us, one kind -> both: 160 experts, DeepSeek-V2-236B, 500 / 900 / 1500 / 2000 / 3000 tokens
-// (means of 18 to 112) 1189 / 1407 / 1607 / 1773 / 2075 -> 1189 / 1364 / 1496 / 1583 / 1850; 64 experts, DeepSeek-V2-Lite, 350 / 512 /
-// 1000 / 1300 (32 to 121) 196 / 218 / 301 / 344 -> 234 / 225 / 286 / 332, from 700 to 895 tokens (66 to 84) 7 % slower to 6 % faster by how
-// the rounds fall out, from 910 on (85; five inputs each) never slower and 2.5 % faster in the mean; 8 experts, Mixtral-8x7B and 8x22B, 256 and 400 (64 and
-// 100) the same to 1 % slower.
+// Whether a call of a group has tiles of both kinds (where the persistent body can address its rows): from a mean of 128 rows per expert
+// on; sums of fp8 weights start elsewhere in calls of one kind (k_rotation).  Sums of bf16 weights do not depend on it: with many
+// experts some hold most of the rows well below that mean (and would be 128-row tiles that fetch their weights again and again), and all
+// gain by the other rounds.  Both kinds cost a call 7 to 10 us in front of the first tiles, against a gain that grows with the weights and
+// with the mean: below 128 rows the call has to be long enough for the one, and its rows enough for the other.  Layers, us, one kind ->
+// both.  Above the line: 160 experts, DeepSeek-V2-236B, 900 / 1500 / 2500 tokens (means of 33 to 93 rows) skewed 1403 / 1591 / 1911 -> 1357 / 1491 /
+// 1693, even 1405 / 1518 / 1704 -> 1336 / 1467 / 1644; 64, DeepSeek-V2-Lite, 920 / 1100 / 1300 skewed 284 / 310 / 340 -> 277 / 301 / 332, even the
+// same.  Below it (hidden x intermediate size): 64 experts, 2048 x 1024, 939 tokens 225 -> 241, 1024 x 1024 119 -> 142, 2048 x 768, 1259 202 -> 211; 128,
+// 2048 x 512, 726 149 -> 156; 256, 1024 x 384, 1451 107 -> 117.  32 experts, above it too: 2048 x 4096, 470 / 630 415 / 461 -> 442 / 470.  138 calls of
+// 64 to 256 experts, even and skewed: above it both kinds are 3.9 per cent faster in the mean, 1.6 slower at most; below it 1.8 slower.
 template <bool W8>
-inline bool both_kinds(long n_rows, int E) { return E > 0 && n_rows / E >= (W8 || E < 32 ? 128 : E < 128 ? 86 : 32); }
+inline bool both_kinds(long n_rows, int E, int K, int N) {
+    const long mean = E > 0 ? n_rows / E : 0;
+    const double weights = (double)E * K * N;      // of one matrix
+    return mean >= 128 || (!W8 && E >= 64 && mean >= 32 && weights >= 1.6e8 && weights * mean * mean >= 1.33e12);
+}
 
 // How the down projection of one MLP is cut when its k is: row tiles of `rows` (256: on the persistent body, else on the split
 // kernel), k into `slices` of up to `blocks` blocks of 128.  part: where the fp32 sums go, [slices][n_rows][N].
@@ -2962,7 +2968,7 @@ int launch_mt(const GemmArgs& g0, int n_rows, int max_rows, void* workspace, siz
     // (One MLP of up to 192 rows has tiles of one workgroup alone too, and the sums of a call of both kinds.  As such a call its
     // persistent workgroups found no tile and took the first 5 us: DeepSeek-V3's dense MLP, 128 / 160 / 192 tokens 167 / 183 / 203 -> 152 / 175 /
     // 189 us with one upload less.)
-    const bool one_kind = !both_kinds<W8>(n_rows, g.E) || !persistent_fits(g);
+    const bool one_kind = !both_kinds<W8>(n_rows, g.E, g.K, g.N) || !persistent_fits(g);
     if (one_kind || (g.E == 1 && n_rows <= 192)) {
         g.alone = one_kind;
         if (!W8 && (long)g.E * g.n_tiles_n <= cu_count()) g.cut_cus = cu_count();
@@ -3078,7 +3084,7 @@ bool few_tiles(const moe_mlp_group& m, long cus) { return (long)(m.n_rows / 256 
 // Whether a joint call has tiles of both kinds: the routed experts' call would, and the persistent body can address both problems.
 // (Where it cannot, for sizes that are odd multiples of 64, the call has one kind of tiles, like one of a lower mean.)
 bool joint_both(bool w8, const moe_mlp_group& routed, const moe_mlp_group& shared, int32_t hidden) {
-    return (w8 ? both_kinds<true>(routed.n_rows, routed.n_experts) : both_kinds<false>(routed.n_rows, routed.n_experts)) &&
+    return (w8 ? both_kinds<true> : both_kinds<false>)(routed.n_rows, routed.n_experts, hidden, routed.inter) &&
            shared.n_rows >= 128 && hidden % 128 == 0 && routed.inter % 128 == 0 && shared.inter % 128 == 0 && routed.n_experts <= 512 &&
            cu_count() >= 8;
 }

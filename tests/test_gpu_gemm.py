@@ -897,9 +897,9 @@ def test_shared_expert_in_the_launches_of_both_kernels(fp8, n, E, I, shared_inte
 
 
 @pytest.mark.parametrize("n,E,k,h,I,shared_inter", [
-    (1100, 130, 4, 320, 1152, 384), (1100, 130, 4, 384, 1088, 384), (1100, 130, 4, 384, 1152, 448),     # one size an odd multiple of 64
-    (1000, 64, 6, 320, 2176, 384),
-    (120, 130, 36, 384, 1152, 384)])                                                                    # fewer rows than 128
+    (1100, 130, 4, 2624, 4096, 384), (1100, 130, 4, 2560, 4160, 384), (1100, 130, 4, 2560, 4096, 448),     # one size an odd multiple of 64
+    (1000, 64, 6, 2112, 1408, 384),
+    (120, 130, 36, 2560, 4096, 384)])                                                                      # fewer rows than 128
 def test_bf16_shared_expert_stays_in_the_launches_where_persistent_tiles_cannot_have_it(n, E, k, h, I, shared_inter):
     """Means of 33 and 93 rows, at which the routed experts' own call has both kinds of tiles where the persistent body can address it:
     a joint call that it cannot serve has one kind.  Bit for bit two calls apart."""
@@ -1257,22 +1257,26 @@ def test_kernel_choice_for_few_rows_leaves_the_bits(fp8, E, h, I):
         assert torch.equal(call(rows, 16), want[:, :rows]), rows
 
 
-@pytest.mark.parametrize("E,mean", [(8, 127), (8, 128), (40, 85), (40, 86), (130, 31), (130, 32)])     # both sides of the line of both_kinds
-def test_bf16_skewed_experts_around_the_line_between_one_and_both_kinds(E, mean):
+@pytest.mark.parametrize("E,mean,h,I", [        # both sides of the lines of both_kinds
+    (8, 127, 384, 320), (8, 128, 384, 320),
+    (64, 89, 2048, 1280), (64, 90, 2048, 1280), (63, 90, 2048, 1280),      # mean * mean * weights; experts
+    (64, 120, 2048, 1152), (64, 120, 2048, 1280),                          # weights
+    (130, 31, 2560, 4096), (130, 32, 2560, 4096)])                         # mean
+def test_bf16_skewed_experts_around_the_line_between_one_and_both_kinds(E, mean, h, I):
     """A few experts hold most of the rows: 256-row tiles, pairs and slices next to small ones.  Every expert's rows equal, bit
     for bit, those of a call with that expert alone."""
     from moe_gen_amd import ops
-    h, I = 384, 320
     rows = E * mean
     counts = np.full(E, 3, np.int64)
     counts[[1, 3, 4]] = rows // 4, 300, 190
     counts[6] += rows - counts.sum()
     offsets = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
-    print(f"skewed experts E={E} mean={mean}", flush=True)
+    print(f"skewed experts E={E} mean={mean} h={h} I={I}", flush=True)
     assert counts.min() > 0 and offsets[-1] == rows
     g = torch.Generator().manual_seed(E + mean)
     x = torch.randn(rows, h, generator=g).to(torch.bfloat16).cuda()
-    mats = [[m.cuda() for m in one] for one in make_experts(E, h, I, False, E)]
+    few = [[m.cuda() for m in one] for one in make_experts(3, h, I, False, E)]
+    mats = [few[e % 3] for e in range(E)]
     call = lambda xs, ms, off: ops.grouped_swiglu(xs, None, ops.expert_pointers(*([m[j] for m in ms] for j in range(3))),
                                                   torch.tensor(off, dtype=torch.int32, device="cuda"), xs.shape[0])
     y = call(x, mats, offsets.tolist())
