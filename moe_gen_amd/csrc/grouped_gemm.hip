@@ -1555,25 +1555,43 @@ __device__ __forceinline__ ExpertAt expert_at(const int* pref, int E, int q) {
 // tiles_of says.  A call of few tiles, a down projection of a few experts, leaves CUs without any while its tallest tiles, bound
 // by the matrix cores above about 100 rows, take longest: cut as long as every tile has a CU.  Every workgroup finds the same.
 // Mixtral-8x22B, layers of 256 / 350 tokens (tallest experts 181 and 250 rows, 192 tiles for 256 CUs) 847 / 915 -> 831 / 899 us, of fewer tokens
-// the same, Mixtral-8x7B of 256 to 400 tokens 0 to 0.5 % slower, which is the counting.
+// the same, Mixtral-8x7B of 256 to 400 tokens 0 to 0.5 % slower, which is the counting.  (At most NT experts; s_sums: LDS of its own,
+// NT / 64 pairs.)
 template <int NT>
-__device__ __forceinline__ int cut_rows(const GemmArgs& g, int tid, int* s_wtot) {
-    if (g.cut_cus <= 0) return 0;
-    const int low = sum_over_experts<NT>(g, tid, s_wtot, [](int c) { return (c + 95) / 96; });
-    int rows = 96;
-    if ((long)low * g.n_tiles_n > g.cut_cus) {
-        const int high = sum_over_experts<NT>(g, tid, s_wtot, [](int c) { return (c + 127) / 128; });
-        rows = (long)high * g.n_tiles_n <= g.cut_cus ? 128 : 0;
+__device__ __forceinline__ int cut_rows(const GemmArgs& g, int tid, int* s_sums) {
+    int low = 0, high = 0;                       // tiles of up to 96 and of up to 128 rows
+    if (tid < g.E) {
+        const int c = g.offsets[tid + 1] - g.offsets[tid];
+        low = (c + 95) / 96;
+        high = (c + 127) / 128;
     }
-    __syncthreads();                 // every wave has read s_wtot, which the scan behind this writes first thing
-    return rows;
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) {
+        low += __shfl_xor(low, d);
+        high += __shfl_xor(high, d);
+    }
+    if ((tid & 63) == 0) {
+        s_sums[tid >> 5] = low;
+        s_sums[(tid >> 5) + 1] = high;
+    }
+    __syncthreads();
+    long l = 0, h = 0;
+#pragma unroll
+    for (int w = 0; w < NT / 64; ++w) {
+        l += s_sums[2 * w];
+        h += s_sums[2 * w + 1];
+    }
+    return l * g.n_tiles_n <= g.cut_cus ? 96 : h * g.n_tiles_n <= g.cut_cus ? 128 : 0;
 }
 
 // One workgroup per (M tile, N tile), in calls without persistent tiles (few rows per expert, odd K).  (tile_body is its counterpart in calls
 // of both kinds: which rows a tile has, and which streamer computes them, is the same there, since a row's bits follow from it.)
-template <int WN, bool SWIGLU, bool W8>
+// CUT: rows are cut lower where that fills the CUs (cut_rows), in an instantiation of its own: the other calls, DeepSeek-V2-Lite of 256 to
+// 500 tokens, were 1 to 2 % slower with the few instructions in front of their tiles.
+template <int WN, bool SWIGLU, bool W8, bool CUT>
 __global__ __launch_bounds__(128 * WN) void grouped_gemm_kernel(GemmPair pair_of) {
     constexpr int NT = 128 * WN;
+    static_assert(!(W8 && CUT), "fp8 rows are not cut: their sums follow the tile");
     // Three weight arrays of 32 KiB and token arrays of 16 KiB (fp8 weights: three, 128 rows; the second one 24 KiB)
     // or 24 KiB (bf16: two, 192 rows) -- the buffers of the weight streamers, written by DMA, as separate objects so
     // that a read of one waits for no DMA into another; gemm_tile's two stages (up to 128 token rows + 256 weight
@@ -1603,7 +1621,11 @@ __global__ __launch_bounds__(128 * WN) void grouped_gemm_kernel(GemmPair pair_of
     // ---- M-tile prefix over experts ----
     const GemmArgs& g = pair_of.p[in_front ? 1 : 0];
     ExpertOfThread mine;
-    const int cut = W8 || in_front ? 0 : cut_rows<NT>(g, tid, s_wtot);
+    int cut = 0;
+    if constexpr (CUT) {
+        __shared__ int s_sums[NT / 32];
+        cut = cut_rows<NT>(g, tid, s_sums);
+    }
     const int run = mtile_prefix_scan<NT>(g, tid, s_pref, s_wtot, mine, [&](int c) { return cut ? (c + cut - 1) / cut : tiles_of<!W8>(c); }, [](int, int, int) {});
     if (v >= run * g.n_tiles_n) return;
     const bool s8_ok = !g.row_map || g.a_bytes < (1ull << 32);   // (the weight streamer addresses gathered rows with 32-bit offsets)
@@ -1660,7 +1682,7 @@ __global__ __launch_bounds__(128 * WN) void grouped_gemm_kernel(GemmPair pair_of
     const bool pair = !W8 && rows_e >= PAIR_LO && rows_e <= PAIR_HI;
     const int slice = cut ? ((rows_e + mt_e - 1) / mt_e + 15) & ~15 : pair ? half_rows(rows_e) : 128;
     const int t0 = mt_e > 1 ? first_row + m_tile * slice : first_row, t1 = mt_e > 1 ? min(row_end, t0 + slice) : row_end;
-    if (t0 >= t1) return;           // (heights are whole groups of 16)
+    if (CUT && t0 >= t1) return;    // (heights are whole groups of 16)
     if (!W8 && s8_ok) {
         // bf16 weights: the weight streamer in the persistent body's order
         if (mt_e == 1) stream16<SWIGLU, false>(g, lw0, lw1, lw2, lt0, lt1, e, t0, t1, n_tile, one);
@@ -2740,12 +2762,16 @@ int launch_half(GemmPair pair, int n_rows, hipStream_t st) {
 
 template <int WN, bool SWIGLU, bool W8>
 int launch_tiles(const GemmPair& pair, int n_rows, hipStream_t st) {
-    auto kern = grouped_gemm_kernel<WN, SWIGLU, W8>;
+    auto kern = grouped_gemm_kernel<WN, SWIGLU, W8, false>;
     const GemmArgs& g = pair.p[0];
     if constexpr (!W8 && !SWIGLU)
         if (half_tiles_pay(g, n_rows)) return launch_half(pair, n_rows, st);
     long tiles = ((long)n_rows / 128 + g.E) * g.n_tiles_n;             // sum_e tiles_of(c_e) <= sum_e (c_e / 128 + 1)
-    if (tiles < g.cut_cus) tiles = g.cut_cus;                          // (no more than that where rows are cut lower)
+    if constexpr (!W8)
+        if (g.cut_cus > 0) {
+            kern = grouped_gemm_kernel<WN, SWIGLU, W8, true>;
+            if (tiles < g.cut_cus) tiles = g.cut_cus;                  // (no more than that where rows are cut lower)
+        }
     const long grid = tile_grid(tiles + pair.shared_tiles);
     if (grid > 0x7fffffffL) {
         set_error("grouped gemm: %ld workgroups exceed the grid limit", grid);
