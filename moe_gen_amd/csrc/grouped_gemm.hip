@@ -101,7 +101,7 @@ struct GemmArgs {
                                 // stream8_tile for tiles of up to 64 rows
     int tail_cus;               // > 0: the persistent workgroups run whole rounds of this many tiles (one per CU); what
                                 // is left goes to workgroups of one piece of a tile each if that pays (tail_of)
-    int cut_cus;                // > 0 (bf16, tiles of one workgroup alone): the CUs, see cut_rows
+    int cut_cus;                // > 0 (bf16, tiles of one workgroup alone): the CUs, see cut_prefix_scan
 };
 
 // What a launch works on: the routed experts and a second problem of one expert with matrices, sizes and buffers of its own,
@@ -1551,42 +1551,54 @@ __device__ __forceinline__ ExpertAt expert_at(const int* pref, int E, int q) {
     }
 }
 
-// Rows above which an expert is cut into tiles of equal height (neighbours on one XCD, which share its weights through the L2), 0: as
-// tiles_of says.  A call of few tiles, a down projection of a few experts, leaves CUs without any while its tallest tiles, bound
-// by the matrix cores above about 100 rows, take longest: cut as long as every tile has a CU.  Every workgroup finds the same.
-// Mixtral-8x22B, layers of 256 / 350 tokens (tallest experts 181 and 250 rows, 192 tiles for 256 CUs) 847 / 915 -> 831 / 899 us, of fewer tokens
-// the same, Mixtral-8x7B of 256 to 400 tokens 0 to 0.5 % slower, which is the counting.  (At most NT experts; s_sums: LDS of its own,
-// NT / 64 pairs.)
+// The scan of a call whose experts may be cut lower: `cut` rows above which an expert is cut into tiles of equal height (neighbours on one
+// XCD, which share its weights through the L2), 0: as tiles_of says.  A call of few tiles, a down projection of a few experts, leaves CUs
+// without any while its tallest tiles, bound by the matrix cores above about 100 rows, take longest: cut as long as every tile has a
+// CU.  Every workgroup finds the same.  Mixtral-8x22B, layers of 256 / 350 tokens (tallest experts 181 and 250 rows, 192 tiles for 256 CUs)
+// 847 / 915 -> 831 / 899 us, of fewer tokens the same.  The three ways to count are scanned side by side: as a pass of its own in front of
+// the scan, where the counts of Mixtral-8x7B at 256 to 400 tokens (66 to 110 rows) are not cut, it cost 2 to 5 of 570 us.
+// At most NT experts; s_wtot: 3 NT / 64.
 template <int NT>
-__device__ __forceinline__ int cut_rows(const GemmArgs& g, int tid, int* s_sums) {
-    int low = 0, high = 0;                       // tiles of up to 96 and of up to 128 rows
+__device__ __forceinline__ int cut_prefix_scan(const GemmArgs& g, int tid, int* s_wtot, ExpertOfThread& mine, int& cut) {
+    const int lane = tid & 63, wave = tid >> 6;
+    mine = ExpertOfThread{0, 0, 0, 0};
     if (tid < g.E) {
-        const int c = g.offsets[tid + 1] - g.offsets[tid];
-        low = (c + 95) / 96;
-        high = (c + 127) / 128;
+        mine.o0 = g.offsets[tid];
+        mine.o1 = g.offsets[tid + 1];
+    }
+    const int c = mine.o1 - mine.o0, n[3] = {(c + 95) / 96, (c + 127) / 128, tiles_of<true>(c)};
+    int inc[3] = {n[0], n[1], n[2]};
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            const int o = __shfl_up(inc[j], d);
+            if (lane >= d) inc[j] += o;
+        }
     }
 #pragma unroll
-    for (int d = 32; d > 0; d >>= 1) {
-        low += __shfl_xor(low, d);
-        high += __shfl_xor(high, d);
-    }
-    if ((tid & 63) == 0) {
-        s_sums[tid >> 5] = low;
-        s_sums[(tid >> 5) + 1] = high;
-    }
+    for (int j = 0; j < 3; ++j)
+        if (lane == 63) s_wtot[3 * wave + j] = inc[j];
     __syncthreads();
-    long l = 0, h = 0;
+    int before[3] = {0, 0, 0}, all[3] = {0, 0, 0};
 #pragma unroll
     for (int w = 0; w < NT / 64; ++w) {
-        l += s_sums[2 * w];
-        h += s_sums[2 * w + 1];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            if (w < wave) before[j] += s_wtot[3 * w + j];
+            all[j] += s_wtot[3 * w + j];
+        }
     }
-    return l * g.n_tiles_n <= g.cut_cus ? 96 : h * g.n_tiles_n <= g.cut_cus ? 128 : 0;
+    const bool low = (long)all[0] * g.n_tiles_n <= g.cut_cus, high = (long)all[1] * g.n_tiles_n <= g.cut_cus;
+    cut = low ? 96 : high ? 128 : 0;
+    mine.mt = low ? n[0] : high ? n[1] : n[2];
+    mine.start = (low ? before[0] + inc[0] : high ? before[1] + inc[1] : before[2] + inc[2]) - mine.mt;
+    return low ? all[0] : high ? all[1] : all[2];
 }
 
 // One workgroup per (M tile, N tile), in calls without persistent tiles (few rows per expert, odd K).  (tile_body is its counterpart in calls
 // of both kinds: which rows a tile has, and which streamer computes them, is the same there, since a row's bits follow from it.)
-// CUT: rows are cut lower where that fills the CUs (cut_rows), in an instantiation of its own: the other calls, DeepSeek-V2-Lite of 256 to
+// CUT: rows are cut lower where that fills the CUs (cut_prefix_scan), in an instantiation of its own: the other calls, DeepSeek-V2-Lite of 256 to
 // 500 tokens, were 1 to 2 % slower with the few instructions in front of their tiles.
 template <int WN, bool SWIGLU, bool W8, bool CUT>
 __global__ __launch_bounds__(128 * WN) void grouped_gemm_kernel(GemmPair pair_of) {
@@ -1609,7 +1621,7 @@ __global__ __launch_bounds__(128 * WN) void grouped_gemm_kernel(GemmPair pair_of
     const SBuf sb0{lw0, lt0}, sb1{lw1, lt1}, sb2{lw2, lt2};
     const TileLds lds{lw0, lw1, lw2, lt0, lt1, lt2};
     __shared__ int s_pref[MAX_E + 1];
-    __shared__ int s_wtot[NT / 64];
+    __shared__ int s_wtot[(CUT ? 3 : 1) * (NT / 64)];
     __shared__ int s_sel[5];
     const int tid = threadIdx.x;
 
@@ -1621,19 +1633,16 @@ __global__ __launch_bounds__(128 * WN) void grouped_gemm_kernel(GemmPair pair_of
     // ---- M-tile prefix over experts ----
     const GemmArgs& g = pair_of.p[in_front ? 1 : 0];
     ExpertOfThread mine;
-    int cut = 0;
-    if constexpr (CUT) {
-        __shared__ int s_sums[NT / 32];
-        cut = cut_rows<NT>(g, tid, s_sums);
-    }
-    const int run = mtile_prefix_scan<NT>(g, tid, s_pref, s_wtot, mine, [&](int c) { return cut ? (c + cut - 1) / cut : tiles_of<!W8>(c); }, [](int, int, int) {});
+    int cut = 0, run;
+    if constexpr (CUT) run = cut_prefix_scan<NT>(g, tid, s_wtot, mine, cut);
+    else run = mtile_prefix_scan<NT>(g, tid, s_pref, s_wtot, mine, [](int c) { return tiles_of<!W8>(c); }, [](int, int, int) {});
     if (v >= run * g.n_tiles_n) return;
     const bool s8_ok = !g.row_map || g.a_bytes < (1ull << 32);   // (the weight streamer addresses gathered rows with 32-bit offsets)
     const int q = v / g.n_tiles_n;  // global M-tile number
     // find e with prefix[e] <= q < prefix[e+1].  Up to NT experts every thread still holds its own
     // expert's prefix, tile count and row range: the one that owns q publishes them (one barrier,
     // no search, no second trip to memory for the offsets).  More experts: binary search in LDS.
-    if (g.E <= NT) {
+    if (CUT || g.E <= NT) {
         if (tid < g.E && mine.start <= q && q < mine.start + mine.mt) {
             s_sel[0] = tid; s_sel[1] = mine.start; s_sel[2] = mine.mt; s_sel[3] = mine.o0; s_sel[4] = mine.o1;
         }
