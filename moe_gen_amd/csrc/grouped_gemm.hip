@@ -3116,11 +3116,14 @@ bool sliced(const moe_mlp_group& m, int32_t hidden) {
 // Whether 256-row tiles of the group (its gate and up projection) are fewer than 3/8 of the CUs
 bool few_tiles(const moe_mlp_group& m, long cus) { return (long)(m.n_rows / 256 + 1) * ((m.inter + 127) / 128) * 8 < 3 * cus; }
 
+bool both_kinds_of(bool w8, const moe_mlp_group& m, int32_t hidden) {
+    return (w8 ? both_kinds<true> : both_kinds<false>)(m.n_rows, m.n_experts, hidden, m.inter);
+}
+
 // Whether a joint call has tiles of both kinds: the routed experts' call would, and the persistent body can address both problems.
 // (Where it cannot, for sizes that are odd multiples of 64, the call has one kind of tiles, like one of a lower mean.)
 bool joint_both(bool w8, const moe_mlp_group& routed, const moe_mlp_group& shared, int32_t hidden) {
-    return (w8 ? both_kinds<true> : both_kinds<false>)(routed.n_rows, routed.n_experts, hidden, routed.inter) &&
-           shared.n_rows >= 128 && hidden % 128 == 0 && routed.inter % 128 == 0 && shared.inter % 128 == 0 && routed.n_experts <= 512 &&
+    return both_kinds_of(w8, routed, hidden) && shared.n_rows >= 128 && hidden % 128 == 0 && routed.inter % 128 == 0 && shared.inter % 128 == 0 && routed.n_experts <= 512 &&
            cu_count() >= 8;
 }
 
@@ -3229,6 +3232,12 @@ bool layer_shared_first(const moe_mlp_group& routed, const moe_mlp_group& shared
            check_group(shared, hidden, shared.fp8, "moe_layer_forward") == MOE_OK && joins(routed, shared, hidden) &&
            joint_thin(gate_up_args(routed, hidden), routed.n_rows, row_bound(routed), gate_up_args(shared, hidden), shared.n_rows);
 }
+
+bool layer_claims(const moe_mlp_group& routed, const moe_mlp_group* shared, int32_t hidden) {
+    return both_kinds_of(routed.fp8, routed, hidden) || (shared && both_kinds_of(shared->fp8, *shared, hidden));
+}
+
+bool layer_joins(const moe_mlp_group& routed, const moe_mlp_group& shared, int32_t hidden) { return joins(routed, shared, hidden); }
 
 int layer_experts(const moe_mlp_group& routed, const moe_mlp_group* shared, int32_t hidden, int32_t fp8, LayerCall* call, void* stream) {
     return swiglu_groups(routed, shared, hidden, fp8, MOE_PHASE_BOTH, call, stream);

@@ -32,7 +32,10 @@ Layout layout_of(const moe_layer_args& a) {
     l.row_map = take(nk * 4);
     l.segments = take(moe_dispatch_workspace_bytes(p.n_tokens, p.top_k, p.n_experts));
     l.arrivals = take(n <= kTailTokens ? tail_arrivals(p.hidden) * 4 : 0);
-    l.claims = take(kLayerClaims * 4);
+    moe_mlp_group routed = *a.routed, shared = a.shared ? *a.shared : moe_mlp_group{};
+    routed.n_rows = (int32_t)nk;
+    shared.n_rows = (int32_t)n;
+    l.claims = take(layer_claims(routed, a.shared ? &shared : nullptr, p.hidden) ? kLayerClaims * 4 : 0);
     l.act = take(nk * (size_t)a.routed->inter * 2);
     l.y = take(nk * h * 2);
     if (a.shared) {
@@ -104,8 +107,6 @@ extern "C" int moe_layer_forward(const moe_layer_args* args, void* stream) {
     }
     LayerCall call;
     call.tail = may_combine ? &tail : nullptr;
-    call.claims = d.claims = ints(l.claims);
-    d.n_claims = kLayerClaims;
 
     moe_mlp_group routed = *a.routed;
     routed.x = x; routed.x_rows = n; routed.n_rows = n * k; routed.row_map = d.row_map; routed.offsets = d.offsets;
@@ -125,6 +126,10 @@ extern "C" int moe_layer_forward(const moe_layer_args* args, void* stream) {
         first = SharedFirst{shared.w_gate, shared.w_up, shared.s_gate, shared.s_up, static_cast<const uint16_t*>(x),
                             static_cast<uint16_t*>(shared.act), n, h, shared.inter, shared.fp8, 0};
         call.shared_gate_up_done = true;
+    }
+    if (layer_claims(routed, a.shared && !(join && layer_joins(routed, shared, h)) ? &shared : nullptr, h)) {
+        call.claims = d.claims = ints(l.claims);
+        d.n_claims = kLayerClaims;
     }
     const SharedFirst* const with = call.shared_gate_up_done ? &first : nullptr;
 

@@ -50,8 +50,11 @@ struct LayerCall {
     const CombineTail* tail = nullptr;   // the combine, for a down projection that can end with it
     bool combined = false;               // (result) it did
     bool shared_gate_up_done = false;
-    int32_t* claims = nullptr;           // counters that the dispatch sets to 0, kClaimInts for each launch of the call
+    int32_t* claims = nullptr;           // counters that the dispatch sets to 0, kClaimInts for each launch of the call; NULL: none
 };
+// Whether a launch of the call can have use for them: one with both kinds of tiles.  shared: NULL, or a shared expert with launches of its own
+bool layer_claims(const moe_mlp_group& routed, const moe_mlp_group* shared, int32_t hidden);
+bool layer_joins(const moe_mlp_group& routed, const moe_mlp_group& shared, int32_t hidden);      // moe_shared_joins
 constexpr int kClaimStride = 32, kClaimInts = 8 * kClaimStride;      // a line per XCD
 constexpr int kLayerClaims = 4 * kClaimInts;                         // two projections, the shared expert's apart
 int layer_experts(const moe_mlp_group& routed, const moe_mlp_group* shared, int32_t hidden, int32_t fp8, LayerCall* call, void* stream);

@@ -3,6 +3,8 @@
 import os
 import re
 
+import pytest
+
 from moe_gen_amd import _native as N
 
 HEADER = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "include", "moe_mi355.h")
@@ -77,3 +79,26 @@ assert lib.moe_grouped_swiglu_joint(ctypes.byref(good), ctypes.byref(none), 64, 
     r = subprocess.run([sys.executable, "-c", code], cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
                        capture_output=True, text=True)
     assert r.returncode == 0, (r.returncode, r.stderr)
+
+
+@pytest.mark.parametrize("fp8", [0, 1])
+def test_a_layer_call_holds_tile_counters_only_where_it_can_claim_tiles(fp8):
+    """4 KiB that the dispatch would clear: from a mean of 128 rows per expert on (64 experts, each with every token), or, with a
+    shared expert, from 128 tokens on.  Of these sizes every other buffer grows by a multiple of 256 bytes a token."""
+    import ctypes
+    lib, first = N.lib(), 128
+
+    def need(n, k, shared):
+        p = N.RouterParams(n, 128, 64, k, 1, 1, 0, 0, 0, 1, 0, 0, 1e-20, 1.0)
+        group = lambda E: N.MlpGroup(1, 1, 0, None, 1, 1, 1, 1, 1, 1, None, E, 128, 0, fp8, None, None, None, 0)
+        r, s = group(64), group(1)
+        a = N.LayerArgs(1, None, 1, None, ctypes.addressof(p), ctypes.addressof(r), ctypes.addressof(s) if shared else None, 1, 1, 1, None, 1,
+                        None, 0, 0.0, 0, 1)
+        size = lib.moe_layer_workspace_bytes(ctypes.byref(a))
+        assert size > 0, N.last_error()
+        return size - lib.moe_dispatch_workspace_bytes(n, k, 64)
+
+    for k, shared in ((64, False), (64, True), (32, True)):
+        step = [need(n + 1, k, shared) - need(n, k, shared) for n in range(first - 4, first + 4)]
+        assert [d - min(step) >= 4096 for d in step] == [n + 1 == first for n in range(first - 4, first + 4)], (k, shared, step)
+    assert len({need(n + 8, 32, False) - need(n, 32, False) for n in range(120, 136, 8)}) == 1          # a mean of 64
