@@ -1251,25 +1251,23 @@ __host__ __device__ __forceinline__ int persistent_tiles(const GemmArgs& g, int 
 // one takes 60: DeepSeek-V2-Lite, 4096 tokens, gate and up), rounded down: what is left of the others then runs on every CU, in
 // small pieces.  The places that the persistent tiles leave free in those rounds are taken in the longest stretch of the narrowest
 // strip that holds nearly all of them, of whole 32 CUs: the tiles that an XCD has at a time then stay whole blocks of 4 M tiles,
-// which share their panels (strips of any 8 CUs: DeepSeek-V2-236B, 32768 tokens, and DeepSeek-V3, 65536, 1 and 2 % slower
-// than without any).
-// A last round of a few tiles costs as much as a full one.  Where the others do not fill the CUs that it leaves over, and cut into
-// pieces its tiles make the sum of both kinds' rounds shorter, it goes to workgroups of one tile: as 128-row halves, or, where no
-// others share the round, in as many as three or four pieces that fit in it (next to others, which take as long as a half, they end no
-// sooner).  Every workgroup evaluates all this on the same offsets[].  Halves -> up to four pieces, us: Mixtral-8x7B, layer, 2000 / 4000 / 8000
-// tokens 1426 / 2302 / 4306 -> 1408 / 2278 / 4288; dense MLP of DeepSeek-V3, 2800 / 5000 tokens 1820 / 3186 -> 1797 / 3138 (1000: the same, a
-// quarter's weights take as long to convert as a half's).  16 other calls of those and Mixtral-8x22B: -1.0 ... +0.7 %, as one build against itself.
+// which share their panels.
+// A last round of a few tiles costs as much as a full one.  Where the others do not fill the CUs that it leaves over, or fill them up
+// to twice with tall ones among them (two of which, one behind the other, take longer than a persistent tile), and cut into pieces its
+// tiles make the sum of both kinds' rounds shorter, it goes to workgroups of one tile: as 128-row halves, or, where no others share the
+// round, in as many as three or four pieces that fit in it (next to others, which take as long as a half, they end no sooner).  Every
+// workgroup evaluates all this on the same offsets[].
 // Layers, us, every CU at the persistent tiles first and one workgroup launched per tile of the others -> this (and Claims): DeepSeek-V2-Lite
-// 1400 / 2000 / 3000 / 4096 tokens 387 / 461 / 551 / 655 -> 339 / 411 / 499 / 623, DeepSeek-V2-236B 4000 / 8000 / 16000 / 32768 2223 / 3391 /
-// 5709 / 10523 -> 2054 / 3163 / 5540 / 10405, Mixtral-8x22B 700 / 2000 1172 / 2312 -> 1076 / 2220, Mixtral-8x7B 1500 1122 -> 1056,
-// DeepSeek-V3 4096 / 8000 / 65536 3906 / 6753 / 45436 -> 3824 / 6653 / 44486.  Between sizes it goes by how the rounds fall out: of three pairs of
-// inputs Mixtral-8x22B, 750 / 800 / 850 tokens, three are 12 % faster, three 1.3 to 2.5 % slower (1315 -> 1348).  (Strips of up to 192 CUs instead of 128: the same
-// to 0.6 % slower.  kStreamCost 40 and 62: -0.2 ... +5.5 % and -3.6 ... +1.5 %, 0.5 % slower and 0.2 % faster in the mean of 22 calls.)
-constexpr int kStreamCost = 50, kMostAside = 128;
+// 1400 / 2400 / 4096 tokens 379 / 483 / 662 -> 342 / 458 / 635, DeepSeek-V2-236B 1500 / 4000 / 8000 1594 / 2238 / 3384 -> 1479 / 2054 / 3150, DeepSeek-V3
+// 6000 5296 -> 5195.  Mixtral-8x22B, 8 experts, goes by how the rounds fall out: 640 / 760 / 850 1121 / 1266 / 1300 -> 1042 / 1130 / 1161, 820 / 920 / 1100 /
+// 1200 1323 / 1353 / 1451 / 1561 -> 1304 / 1356 / 1453 / 1561; there the down projection has 96 to 144 tiles of 256 rows and 144 to 192
+// others, and without the count of tall ones (kTwoTall) it was 22 to 39 us longer: 1336 / 1393 / 1491 / 1598.
+constexpr int kStreamCost = 50, kTwoTall = 150, kMostAside = 128;
 struct RoundCost { int keep, move, pieces; };       // hundredths of a round, with the last one persistent / in so many pieces a tile
-__host__ __device__ __forceinline__ RoundCost round_cost(int total, int own, int cus) {
+__host__ __device__ __forceinline__ RoundCost round_cost(int total, int own, bool tall, int cus) {
     const int whole = 100 * ((total + cus - 1) / cus), shared = (100 * total + kStreamCost * own) / cus, tail = total % cus;
     RoundCost c{whole > shared ? whole : shared, 72 * ((own + 2 * tail + cus - 1) / cus), 2};
+    if (tall && total < cus && own > cus - total && own <= 2 * (cus - total)) c.keep = kTwoTall;
     if (own == 0 && 3 * tail <= cus) { c.move = 54; c.pieces = 3; }
     if (own == 0 && 4 * tail <= cus) { c.move = 44; c.pieces = 4; }
     c.move += 100 * (total / cus);
@@ -1277,11 +1275,11 @@ __host__ __device__ __forceinline__ RoundCost round_cost(int total, int own, int
 }
 __host__ __device__ __forceinline__ int piece_rows(int pieces) { return pieces == 2 ? 128 : pieces == 3 ? 96 : 64; }
 struct Tail { int tiles, pieces; };
-__device__ __forceinline__ Tail tail_of(const GemmArgs& g, int total, int own) {
+__device__ __forceinline__ Tail tail_of(const GemmArgs& g, int total, int own, bool tall) {
     if (g.tail_cus <= 0) return Tail{0, 2};
     const int tail = total % g.tail_cus;
     if (tail == 0) return Tail{0, 2};
-    const RoundCost c = round_cost(total, own, g.tail_cus);
+    const RoundCost c = round_cost(total, own, tall, g.tail_cus);
     return Tail{c.move < c.keep ? tail : 0, c.pieces};
 }
 struct PersistentPlan { int full, width; };
@@ -1327,16 +1325,27 @@ __host__ __device__ __forceinline__ int own_tiles(const GemmArgs& g, int c) {
     return (g.rem_split ? c > g.cold_max : !is_cold(g, c)) ? 0 : tiles_of<!W8>(c);
 }
 
+// Whether the tallest of them has more than kTallRows: two in a row then outlast a persistent tile by so much that its halves in front of or
+// behind one are the shorter way (round_cost).  DeepSeek-V3's dense MLP, fp8, one such tile a column: 400 / 420 / 440 tokens (144 / 164 / 184 rows)
+// with the persistent tiles kept 354 / 375 / 391 us, in halves 363 / 373 / 382.
+constexpr int kTallRows = 150;
+template <bool W8>
+__device__ __forceinline__ bool has_tall_tile(const GemmArgs& g, int c) {
+    const int tiles = own_tiles<W8>(g, c), rows = g.rem_split ? c & 255 : c;
+    return tiles == 1 ? rows > kTallRows : !W8 && tiles == 2 && rows >= PAIR_LO && half_rows(rows) > kTallRows;
+}
+
 // The shared expert's rows and its tiles of either kind in a call of both, all 0 without one
-struct SharedTiles { int first, end, own, persistent; };
+struct SharedTiles { int first, end, own, persistent; bool tall; };
 template <bool W8>
 __host__ __device__ __forceinline__ SharedTiles shared_tiles_of(const GemmArgs& g, int first, int end) {
-    return SharedTiles{first, end, own_tiles<W8>(g, end - first) * g.n_tiles_n, persistent_tiles(g, end - first) * g.n_tiles_n};
+    return SharedTiles{first, end, own_tiles<W8>(g, end - first) * g.n_tiles_n, persistent_tiles(g, end - first) * g.n_tiles_n,
+                       has_tall_tile<W8>(g, end - first)};
 }
 // The most tiles of each kind that up to `rows` rows can have (fewer rows can have more: 200 rows one 256-row tile, 300 none)
 template <bool W8>
 inline SharedTiles shared_tiles_bound(const GemmArgs& g, int rows) {
-    return SharedTiles{0, rows, (!W8 && rows >= PAIR_LO ? 2 : 1) * g.n_tiles_n, rows > g.cold_max ? ((rows + 255) >> 8) * g.n_tiles_n : 0};
+    return SharedTiles{0, rows, (!W8 && rows >= PAIR_LO ? 2 : 1) * g.n_tiles_n, rows > g.cold_max ? ((rows + 255) >> 8) * g.n_tiles_n : 0, false};
 }
 
 // sum over the experts of f(count) (every thread gets it; two barriers)
@@ -2223,11 +2232,14 @@ __device__ __forceinline__ void persistent_body(const GemmPair& pair_of, const S
     }
     __syncthreads();
     // whole rounds, and the last one unless it is better off in pieces: one-workgroup tiles, whose own are counted for that
-    const SharedTiles second_tiles = PAIRED ? shared_tiles_of<W8>(pair_of.p[1], uni(s_off1[0]), uni(s_off1[1])) : SharedTiles{0, 0, 0, 0};
+    const SharedTiles second_tiles = PAIRED ? shared_tiles_of<W8>(pair_of.p[1], uni(s_off1[0]), uni(s_off1[1])) : SharedTiles{};
     const int ptiles1 = second_tiles.persistent;
-    const int own = g.tail_cus > 0 ? sum_over_experts<NT>(g, tid, s_wtot, [&](int c) { return own_tiles<W8>(g, c); }) * g.n_tiles_n + second_tiles.own : 0;
+    // (of up to 512 experts: at most 1024 M tiles, the experts with a tall one above them)
+    const int sums = g.tail_cus > 0 ? sum_over_experts<NT>(g, tid, s_wtot, [&](int c) { return own_tiles<W8>(g, c) + (has_tall_tile<W8>(g, c) ? 1 << 16 : 0); }) : 0;
+    const int own = (sums & 0xffff) * g.n_tiles_n + second_tiles.own;
+    const bool tall = (sums >> 16) > 0 || second_tiles.tall;
     const int slice_tiles = run * g.n_tiles_n;   // SPLIT: tiles of one slice
-    const int all = SPLIT ? slice_tiles * split.plan.slices : slice_tiles + ptiles1, total = all - tail_of(g, all, own).tiles;
+    const int all = SPLIT ? slice_tiles * split.plan.slices : slice_tiles + ptiles1, total = all - tail_of(g, all, own, tall).tiles;
     const PersistentPlan plan = SPLIT ? PersistentPlan{0, grid} : persistent_plan(g, total, own, grid);
     const int xcd = blockIdx.x & 7, place = blockIdx.x >> 3;
     // this workgroup's it-th tile, `total` or more past its last one
@@ -2610,7 +2622,7 @@ __device__ __forceinline__ void persistent_body(const GemmPair& pair_of, const S
 // A workgroup of one tile: the routed experts' own tiles, the shared expert's, then the pieces of the tiles that the persistent
 // workgroups leave at the end of THEIR tile space, neighbours on one XCD (the prefix is rebuilt over that space).
 struct TileTables {
-    int own[PE + 1], persistent[PE + 1], off[PE + 1], wtot[8], claim;      // M tiles of either kind in front of an expert, its first row
+    int own[PE + 1], persistent[PE + 1], off[PE + 1], wtot[8], tall[8], claim;      // M tiles of either kind in front of an expert, its first row
 };
 template <bool SWIGLU, bool W8>
 __device__ __forceinline__ void tile_body(const GemmPair& pair_of, const TileLds& lds, TileTables& t, int block) {
@@ -2629,7 +2641,9 @@ __device__ __forceinline__ void tile_body(const GemmPair& pair_of, const TileLds
         if (e == ga.E - 1) t.off[ga.E] = o1;
     });
     if (tid == 0) t.own[ga.E] = run;
-    SharedTiles s{0, 0, 0, 0};
+    const uint64_t tall_lanes = __ballot(has_tall_tile<W8>(ga, mine.o1 - mine.o0));
+    if ((tid & 63) == 0) t.tall[tid >> 6] = tall_lanes != 0;
+    SharedTiles s{};
     if (pair_of.shared_rows > 0) s = shared_tiles_of<W8>(pair_of.p[1], uni(shared_first), uni(shared_end));
     const int own = run * ga.n_tiles_n;
     int v = dealt_tile(xcd, block >> 3), total_p = 0;
@@ -2639,7 +2653,10 @@ __device__ __forceinline__ void tile_body(const GemmPair& pair_of, const TileLds
         const int run_p = mtile_prefix_scan<NT>(ga, tid, t.persistent, t.wtot, mine, [&](int c) { return persistent_tiles(ga, c); }, [](int, int, int) {});
         if (tid == 0) t.persistent[ga.E] = run_p;
         total_p = run_p * ga.n_tiles_n + s.persistent;
-        tail = tail_of(ga, total_p, own + s.own);
+        int tall = s.tall;
+#pragma unroll
+        for (int w = 0; w < NT / 64; ++w) tall |= t.tall[w];
+        tail = tail_of(ga, total_p, own + s.own, uni(tall) != 0);
         __syncthreads();
     }
     const int limit = own + s.own + tail.pieces * tail.tiles;
@@ -3036,7 +3053,7 @@ int launch_mt(const GemmArgs& g0, int n_rows, int max_rows, void* workspace, siz
     // instead of 534 / 816 / 2265.
     if (W8 && g.E == 1 && own_tiles<W8>(pair.p[0], n_rows) > 0) {
         const int cus = pair.p[0].tail_cus, full = (n_rows >> 8) * g.n_tiles_n;
-        const RoundCost apart = round_cost(full, g.n_tiles_n, cus), padded = round_cost(full + g.n_tiles_n, 0, cus);
+        const RoundCost apart = round_cost(full, g.n_tiles_n, (n_rows & 255) > kTallRows, cus), padded = round_cost(full + g.n_tiles_n, 0, false, cus);
         const int a = apart.move < apart.keep ? apart.move : apart.keep, b = padded.move < padded.keep ? padded.move : padded.keep;
         if (b < a) pair.p[0].cold_max = 0;
     }

@@ -175,17 +175,17 @@ def test_experts_split_between_the_two_kernels(fp8):
 
 
 @pytest.mark.parametrize("fp8", [False, True])
-@pytest.mark.parametrize("I,counts", [(1280, [700, 520, 300, 1300, 90]),      # gate/up: less than half a round
-                                      (2048, [700, 520, 300, 1300, 90]),      # gate/up: 192 tiles next to 48 of one workgroup each
-                                      (2560, [700, 520, 300, 1300, 90]),      # gate/up: a round and a few tiles
-                                      (1664, [2100, 2300, 2500, 1500, 10])])  # gate/up: 442 tiles, a round + 186, next to 13
+@pytest.mark.parametrize("I,counts", [(1280, [700, 520, 300, 1300, 90]),      # 120 tiles next to 30 of one workgroup (fp8: 100 and 50, halves)
+                                      (2048, [700, 520, 300, 1300, 90]),      # 192 and 48 (160 and 80)
+                                      (2560, [700, 520, 300, 1300, 90]),      # 240 and 60 (200 and 100, tall: halves)
+                                      (1664, [2100, 2300, 2500, 1500, 10]),   # a round, and 186 next to 13 (173, 26)
+                                      (896, [700, 520, 300, 90]),             # 42 and 21: halves (35 and 28: halves)
+                                      (3072, [700, 520, 300, 160, 170, 180, 90])])      # 144 and 144, tall: halves (120 and 168, too)
 def test_rounds_of_the_persistent_kernel_and_its_last_tiles(fp8, I, counts):
-    """The persistent workgroups (one per CU) take whole rounds of 256 tiles; their last, partial round becomes
-    128-row halves of one workgroup each when that shortens the rounds of both kinds: alone, a round of at most 128 tiles;
-    next to one-workgroup tiles also a longer one (192 + 48 tiles: 432 half and whole tiles
-    of one workgroup; 186 of 442 likewise).  Tile counts in the comments are for bf16 weights (with fp8
-    weights only an expert's full tiles and ragged tiles above 128 rows count).  The down projections of these cases
-    have a few dozen tiles, all of them half tiles.  Against the oracle."""
+    """The persistent workgroups (one per CU) take whole rounds of 256 tiles, the last of them on fewer CUs next to tiles of one workgroup; a
+    partial round that leaves too few CUs to these, or costs more than its 128-row halves next to them, becomes such halves.  In the
+    comments: the gate and up projection's tiles on 256 CUs, kept unless they say halves, with bf16 (fp8) weights.  The down
+    projections of these cases have a few dozen tiles, all of them half tiles.  Against the oracle."""
     from moe_gen_amd import ops
     E, h = len(counts), 256
     print(f"rounds fp8={fp8} I={I} counts={counts}", flush=True)
