@@ -1322,7 +1322,7 @@ def test_bf16_down_projection_of_few_tiles_is_cut_in_rows(h, E, counts):
 
 @pytest.mark.parametrize("n,I", [(1, 18432), (16, 14464), (17, 16384), (33, 16512), (48, 18432), (64, 20480), (65, 18432), (80, 20480), (81, 16384), (96, 16512), (97, 14464),
                                  (113, 20480), (128, 18432)])       # 8, 9 and 10 waves a workgroup on 256 CUs, last tiles whole and ragged; past 96 rows
-@pytest.mark.parametrize("h", [128, 640])                           # 1 and 5 blocks of 128 k: less than the stages of a ring, and more
+@pytest.mark.parametrize("h", [128, 640])                           # 1 and 5 blocks of 128 k, for rings of 3 (65 rows and more) to 6 stages (up to 16)
 def test_wide_fp8_mlp_of_few_rows(n, I, h):
     """Gate and up projection of one wide fp8 MLP.  A token row that is 1 at one k reads a column of both matrices exactly, so that
     act is pinned to one bf16 step (silu by the hardware exponential); dense rows against the oracle, also gathered in another
@@ -1360,6 +1360,39 @@ def test_wide_fp8_mlp_of_few_rows(n, I, h):
     z = gate_up(x.cuda(), bad.cuda())
     keep = torch.arange(n) != n // 2
     assert torch.equal(z.cpu()[keep], y.cpu()[rm.long()][keep]) and (z.cpu()[n // 2].float() == 0).all()
+
+
+@pytest.mark.parametrize("n,I,h", [(1, 18432, 2048), (16, 14464, 2048), (17, 16384, 2048), (32, 20480, 2048), (48, 14464, 2048), (96, 18432, 2048),
+                                   (1, 14464, 8320), (16, 16512, 8320), (32, 18432, 8320), (64, 14464, 8320), (96, 14464, 8320)])
+def test_wide_fp8_mlp_of_few_rows_at_long_k(n, I, h):
+    """16 blocks of 128 k: every ring turns several times, whatever its stages; 65: the block scales, 64 of which a wave holds, are
+    loaded again.  Rows that are 1 at one k pin a column of both matrices, and so its block's scales; dense rows against float64."""
+    from moe_gen_amd import ops
+    from moe_gen_amd.synthetic import quantize_fp8_block128
+    print(f"wide mlp n={n} I={I} h={h}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(n + h)
+    mats = [quantize_fp8_block128(torch.randn(I, h, generator=g, device="cuda") * (0.02 + 0.02 * torch.rand(1, h, generator=g, device="cuda"))) for _ in range(2)]
+    down = (torch.zeros(h, I, dtype=torch.uint8, device="cuda").view(torch.float8_e4m3fn), torch.ones(h // 128, I // 128, device="cuda"))
+    ptrs = ops.expert_pointers(*([m[0]] for m in (*mats, down)), *([m[1]] for m in (*mats, down)))
+    off = torch.tensor([0, n], dtype=torch.int32, device="cuda")
+
+    def gate_up(x):
+        m, act, _ = ops.mlp_group(x, None, ptrs, off, n, n)
+        act.fill_(7.0)
+        ops.grouped_swiglu_joint(m, None, h, True, ops.PHASE_GATE_UP)
+        return act
+
+    full = [(q.float() * s.repeat_interleave(128, 0).repeat_interleave(128, 1)).to(torch.bfloat16) for q, s in mats]
+    k = torch.randint(0, h, (n,), generator=g, device="cuda")
+    k[: min(n, 2)] = torch.tensor([h - 1, 64 * 128 if h > 64 * 128 else 0], device="cuda")[: min(n, 2)]
+    one = torch.zeros(n, h, device="cuda")
+    one[torch.arange(n, device="cuda"), k] = 1.0
+    want = torch.nn.functional.silu(full[0][:, k].t()).float() * full[1][:, k].t().float()
+    assert ((gate_up(one.to(torch.bfloat16)).float() - want).abs() <= 2.0 ** -6 * want.abs()).all()
+    x = torch.randn(n, h, generator=g, device="cuda").to(torch.bfloat16)
+    a, b = (x.double() @ w.double().t() for w in full)
+    y, ref = gate_up(x).double(), torch.nn.functional.silu(a) * b
+    assert ((y - ref).abs().max() / ref.abs().max()).item() <= TOL
 
 
 @pytest.mark.parametrize("h,I,E,counts", [
