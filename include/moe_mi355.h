@@ -167,7 +167,7 @@ int moe_dispatch_static(const int32_t* topk_idx, int32_t n_tokens, int32_t top_k
  * (bf16 weights: also experts of 257 to 384 rows, as two such tiles);
  * larger experts run on 256-row tiles of persistent workgroups (with fp8 weights: their full 256-row tiles, and the
  * rows these leave over as one tile of the first kind if they are at most 192; those of a single expert, E = 1, as a padded tile
- * of the second kind where that shortens the call).  The persistent workgroups,
+ * of the second kind where the last round is then cut into thirds or quarters).  The persistent workgroups,
  * one per CU, take whole rounds of tiles, the last of them on fewer CUs where tiles of the first kind use the others; a last, partial
  * round is cut into 128-row halves (thirds or quarters where they fit), which join the first kind, when that
  * shortens the rounds of both (alone: if it is at most half the CUs' worth of tiles).  Below a mean of 128 rows per expert

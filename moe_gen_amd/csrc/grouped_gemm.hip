@@ -3046,11 +3046,12 @@ int launch_mt(const GemmArgs& g0, int n_rows, int max_rows, void* workspace, siz
     // (its shared expert's 128 down tiles become 256 half tiles: 0.071 -> 0.055 ms); DeepSeek-V2-236B 11.43 -> 11.46,
     // DeepSeek-V3 46.56 -> 46.54: short rounds gain nothing, a partial round of few CUs runs at a higher clock anyway.
     pair.p[0] = both_kernels<W8>(g);
-    // One fp8 expert (a dense MLP): the rows are known here.  What its full tiles leave over goes to the persistent body too,
-    // as a padded tile, where that shortens the rounds by the same count: the last one has room, or the other kind is
-    // saved.  DeepSeek-V3's dense MLP, us: 1300 / 1800 / 2200 / 4000 / 6000 tokens (leftovers of 20, 8, 152, 160 and 112 rows) 1129 /
-    // 1352 / 1567 / 2726 / 3998 -> 1015 / 1263 / 1465 / 2606 / 3887; done always, 600 / 1100 / 3500 tokens would be 616 / 931 / 2370
-    // instead of 534 / 816 / 2265.
+    // One fp8 expert (a dense MLP): the rows are known here.  What its full tiles leave over goes to the persistent body's space too,
+    // as a padded tile, where that shortens the rounds by the same count.  It does where the last round then runs in three or four
+    // pieces a tile, which tiles of another kind beside it rule out: calls of few tiles, and of a few more than whole rounds.  Whole MLP
+    // without scratch, us, apart -> padded: hidden 5120, intermediate 3072, 300 / 440 / 660 rows 118 / 148 / 133 -> 100 / 99 / 115, 7168 x 2048 129 /
+    // 163 / 146 -> 112 / 110 / 117, 2048 x 4096 93 / 117 / 104 -> 83 / 84 / 87, DeepSeek-V3's (its down projection) 377 / 548 / 583 -> 352 / 452 / 575.  Done
+    // always, it would be 441 instead of 352 at 300 rows, 726 (651) at 800, 1070 (985) at 1300, 1489 (1396) at 2100.
     if (W8 && g.E == 1 && own_tiles<W8>(pair.p[0], n_rows) > 0) {
         const int cus = pair.p[0].tail_cus, full = (n_rows >> 8) * g.n_tiles_n;
         const RoundCost apart = round_cost(full, g.n_tiles_n, (n_rows & 255) > kTallRows, cus), padded = round_cost(full + g.n_tiles_n, 0, false, cus);

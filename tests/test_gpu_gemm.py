@@ -1040,13 +1040,15 @@ def test_joint_call_leaves_apart_what_its_own_call_sums_in_another_way(E, rows, 
 
 
 @pytest.mark.parametrize("left", [1, 72, 192])
-def test_dense_fp8_leftover_rows_as_a_padded_tile(left):
-    """One fp8 MLP of 11 full tiles and a leftover whose gate and up tiles (240 of 128 columns with the leftover's) fit one round
-    of the persistent kernel: it takes them all.  The last rows come out bit for bit as in a call of their own, where
-    the other kernel serves the leftover, and the first as in a call without one."""
+@pytest.mark.parametrize("tiles", [13,      # gate and up: 260 tiles and 20 padded ones, of which 24 run in quarters: the rest of the padded ones persistent
+                                   11,      # 220 and 20 of one workgroup beside them; down projection: 12 tiles, the padded one among them, in quarters
+                                   1])      # 20 and 20 padded ones, all in quarters
+def test_dense_fp8_leftover_rows_as_a_padded_tile(tiles, left):
+    """One fp8 MLP whose leftover rows are a padded tile of the persistent kernel's space where the last round then runs in quarters.  The
+    rows come out bit for bit as in calls of fewer tiles, where the other kernel serves the leftover, and as in one without it."""
     from moe_gen_amd import ops
-    h, I, n = 256, 2560, 11 * 256 + left
-    print(f"padded leftover {left}", flush=True)
+    h, I, n = 256, 2560, tiles * 256 + left
+    print(f"padded leftover {tiles} {left}", flush=True)
     g = torch.Generator().manual_seed(left)
     x = torch.randn(n, h, generator=g).to(torch.bfloat16).cuda()
     mats = [tuple(t.cuda() for t in m) for m in make_experts(1, h, I, True, 31)[0]]
@@ -1054,8 +1056,10 @@ def test_dense_fp8_leftover_rows_as_a_padded_tile(left):
     def call(rows):
         return ops.grouped_swiglu(rows, None, ptrs, torch.tensor([0, len(rows)], dtype=torch.int32, device="cuda"), len(rows))
     y = call(x)
-    assert torch.equal(y[10 * 256:], call(x[10 * 256:].contiguous()))
-    assert torch.equal(y[:11 * 256], call(x[:11 * 256].contiguous()))
+    assert torch.isfinite(y).all() and y.any()
+    for first in (tiles - 1, max(tiles - 11, 0)):
+        assert torch.equal(y[first * 256:], call(x[first * 256:].contiguous())), first
+    assert torch.equal(y[:tiles * 256], call(x[:tiles * 256].contiguous()))
 
 
 @pytest.mark.parametrize("I", [4096, 4224, 18432])      # 32 blocks of 128 k (the rule's least), 33 (a short last slice), DeepSeek-V3's
