@@ -377,11 +377,13 @@ def run_workload(name: str, args, with_cpu: bool):
         blk(x)
     torch.cuda.synchronize()
     mean_rows = w.n * w.k // w.E
-    # which tiles a grouped GEMM call has follows from the mean rows per expert (grouped_gemm.hip, launch_mt):
-    # below 128 (bf16 weights: below 86 from 32 experts on, 32 from 128 on) tiles of one workgroup each alone; else both kinds (of the former, bf16: experts of up to 192 rows;
-    # fp8: what an expert's full 256-row tiles leave over, if at most 192 rows; either: the last round of persistent
-    # tiles, in pieces, if it is at most half a round; most rows, and the time, on persistent tiles)
-    persistent = mean_rows >= 128 and w.E <= 512 and w.h % 128 == 0
+    # which tiles a grouped GEMM call has follows from the mean rows per expert and the sizes (grouped_gemm.hip, both_kinds, launch_mt):
+    # tiles of one workgroup each alone, or both kinds (of the former, bf16: experts of up to 192 rows;
+    # fp8: what an expert's full 256-row tiles leave over, if at most 192 rows; either: a short last round of persistent
+    # tiles, in pieces; most rows, and the time, on persistent tiles)
+    weights = float(w.E) * w.h * w.I
+    both_kinds = mean_rows >= 128 or (not w.fp8 and w.E >= 64 and mean_rows >= 32 and weights >= 1.6e8 and weights * mean_rows ** 2 >= 1.33e12)
+    persistent = both_kinds and w.E <= 512 and w.h % 128 == 0 and w.I % 128 == 0
     # yardsticks of this box, taken right before and right after the timed passes (MFMA-bound workloads)
     cal = [calibrate(w)] if persistent and not args.no_calibration else []
 
