@@ -2624,11 +2624,11 @@ __device__ __forceinline__ void persistent_body(const GemmPair& pair_of, const S
 struct TileTables {
     int own[PE + 1], persistent[PE + 1], off[PE + 1], wtot[8], tall[8], claim;      // M tiles of either kind in front of an expert, its first row
 };
-template <bool SWIGLU, bool W8>
+template <bool SWIGLU, bool W8, bool CLAIMS>
 __device__ __forceinline__ void tile_body(const GemmPair& pair_of, const TileLds& lds, TileTables& t, int block) {
     constexpr int NT = 512;
     const int tid = threadIdx.x, xcd = block & 7;
-    const bool claiming = pair_of.claims != nullptr;
+    const bool claiming = CLAIMS && pair_of.claims != nullptr;
     const GemmArgs& ga = pair_of.p[0];
     int shared_first = 0, shared_end = 0;    // (requested here, so that the answer comes with that to the scan's loads)
     if (pair_of.shared_rows > 0) {
@@ -2645,14 +2645,14 @@ __device__ __forceinline__ void tile_body(const GemmPair& pair_of, const TileLds
     if ((tid & 63) == 0) t.tall[tid >> 6] = tall_lanes != 0;
     SharedTiles s{};
     if (pair_of.shared_rows > 0) s = shared_tiles_of<W8>(pair_of.p[1], uni(shared_first), uni(shared_end));
-    const int own = run * ga.n_tiles_n;
+    const int own = uni(run) * ga.n_tiles_n;
     int v = dealt_tile(xcd, block >> 3), total_p = 0;
     Tail tail{0, 2};
     __syncthreads();                     // t.wtot has been read, t.own is whole
     if (claiming || v >= own + s.own) {
         const int run_p = mtile_prefix_scan<NT>(ga, tid, t.persistent, t.wtot, mine, [&](int c) { return persistent_tiles(ga, c); }, [](int, int, int) {});
         if (tid == 0) t.persistent[ga.E] = run_p;
-        total_p = run_p * ga.n_tiles_n + s.persistent;
+        total_p = uni(run_p) * ga.n_tiles_n + s.persistent;
         int tall = s.tall;
 #pragma unroll
         for (int w = 0; w < NT / 64; ++w) tall |= t.tall[w];
@@ -2660,7 +2660,7 @@ __device__ __forceinline__ void tile_body(const GemmPair& pair_of, const TileLds
         __syncthreads();
     }
     const int limit = own + s.own + tail.pieces * tail.tiles;
-    Claims claims{pair_of.claims, xcd, limit, 0};
+    Claims claims{CLAIMS ? pair_of.claims : nullptr, xcd, limit, 0};
     if (claiming) {
         claims.ask();
         v = claims.take(&t.claim);
@@ -2684,7 +2684,9 @@ __device__ __forceinline__ void tile_body(const GemmPair& pair_of, const TileLds
         shared = s.own;
         of_shared = true;
     }
-    const GemmArgs& g = pair_of.p[of_shared ? 1 : 0];
+    int which = uni(of_shared ? 1 : 0);
+    asm volatile("" : "+s"(which));      // (else the arguments of both problems are loaded and prepared in front of the loop)
+    const GemmArgs& g = pair_of.p[which];
     const ExpertAt x = of_shared ? ExpertAt{0, 0, shared / g.n_tiles_n} : expert_at(pref, g.E, at / g.n_tiles_n);
     const int e = x.e, o0 = of_shared ? s.first : uni(t.off[e]), row_end = of_shared ? s.end : uni(t.off[e + 1]), mt_e = x.tiles;
     int m_tile, n_tile;
@@ -2710,7 +2712,11 @@ __device__ __forceinline__ void tile_body(const GemmPair& pair_of, const TileLds
     else stream16<SWIGLU, false>(g, lds.w0, lds.w1, lds.w2, lds.t0, lds.t1, e, r0, r1, n_tile, claims);
     }
 }
-template <bool SWIGLU, bool W8, bool PAIRED>
+// CLAIMS: the call may bring counters.  Calls that do not (one MLP, the stand-alone entry points) have an instantiation without the loop:
+// what the compiler prepares in front of it for every form of tile cost their launches 1.5 to 3 us (one fp8 MLP, 1100 rows, hidden 4096,
+// intermediate 2048, gate and up / down 62.0 / 38.8 -> 59.0 / 37.2 us; 800 rows, 5120 x 3072, 74.1 / 48.2 -> 71.0 / 46.7).  A joint
+// call without counters, a layer's stages one by one, runs in that with them.
+template <bool SWIGLU, bool W8, bool PAIRED, bool CLAIMS>
 __global__ __launch_bounds__(512) void grouped_gemm_both_kernel(GemmPair persistent_of, GemmPair tiles_of, int persistent_grid) {
     // The streamers' three weight buffers and token buffers.  The persistent body has its weights in the first two and its token
     // rows in the lower 16 KiB of the others, with its tables behind two of those.  (bf16: the whole LDS of a CU.)
@@ -2727,11 +2733,11 @@ __global__ __launch_bounds__(512) void grouped_gemm_both_kernel(GemmPair persist
         persistent_body<SWIGLU, W8, PAIRED, false>(persistent_of, SplitArgs{}, PersistentLds{lt0, lt1, lt2, lw2, lw0, lw1,
                                                    reinterpret_cast<unsigned long long*>(lw2 + TOKENS),
                                                    reinterpret_cast<PersistentTables*>(lt1 + TOKENS)}, persistent_grid);
-        if (tiles_of.claims == nullptr) return;
+        if (!CLAIMS || tiles_of.claims == nullptr) return;
         __syncthreads();                 // every wave has left the persistent body's LDS
     }
     TileTables& t = *reinterpret_cast<TileTables*>(W8 ? tile_tables : lt2);      // (the bf16 streamer has two token buffers)
-    tile_body<SWIGLU, W8>(tiles_of, TileLds{lw0, lw1, lw2, lt0, lt1, lt2}, t, (int)blockIdx.x - (tiles_of.claims ? 0 : persistent_grid));
+    tile_body<SWIGLU, W8, CLAIMS>(tiles_of, TileLds{lw0, lw1, lw2, lt0, lt1, lt2}, t, (int)blockIdx.x - (CLAIMS && tiles_of.claims ? 0 : persistent_grid));
 }
 
 // The persistent body alone: one MLP's down projection in slices of k
@@ -2987,8 +2993,10 @@ int launch_both(const GemmPair& pair, int n_rows, hipStream_t st) {
         set_error("grouped gemm: %ld workgroups exceed the grid limit", grid);
         return MOE_ERR_INVALID;
     }
-    if (pair.shared_rows > 0) hipLaunchKernelGGL((grouped_gemm_both_kernel<SWIGLU, W8, true>), dim3((unsigned)grid), dim3(512), 0, st, pair, pair, (int)persistent);
-    else hipLaunchKernelGGL((grouped_gemm_both_kernel<SWIGLU, W8, false>), dim3((unsigned)grid), dim3(512), 0, st, pair, pair, (int)persistent);
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(512), 0, st, pair, pair, (int)persistent); };
+    if (pair.shared_rows > 0) launch(grouped_gemm_both_kernel<SWIGLU, W8, true, true>);
+    else if (pair.claims) launch(grouped_gemm_both_kernel<SWIGLU, W8, false, true>);
+    else launch(grouped_gemm_both_kernel<SWIGLU, W8, false, false>);
     MOE_HIP_CHECK(hipGetLastError());
     return MOE_OK;
 }
