@@ -2668,48 +2668,48 @@ __device__ __forceinline__ void tile_body(const GemmPair& pair_of, const TileLds
         return;
     }
     for (; v >= 0; v = claims.take(&t.claim)) {
-    const int* pref = t.own;
-    int piece = -1, shared = 0, at = v;   // shared: tiles of the shared expert in front of the routed experts' in the space `at` counts in
-    bool of_shared = false;
-    if (v >= own + s.own) {              // a piece of one of the last persistent tiles
-        const int h = v - own - s.own, of = h / tail.pieces;
-        at = total_p - tail.tiles + of;
-        piece = h - of * tail.pieces;
-        pref = t.persistent;
-        shared = s.persistent;
-        of_shared = at < shared;
-        if (!of_shared) at -= shared;
-    } else if (v >= own) {
-        at = v - own;
-        shared = s.own;
-        of_shared = true;
-    }
-    int which = uni(of_shared ? 1 : 0);
-    asm volatile("" : "+s"(which));      // (else the arguments of both problems are loaded and prepared in front of the loop)
-    const GemmArgs& g = pair_of.p[which];
-    const ExpertAt x = of_shared ? ExpertAt{0, 0, shared / g.n_tiles_n} : expert_at(pref, g.E, at / g.n_tiles_n);
-    const int e = x.e, o0 = of_shared ? s.first : uni(t.off[e]), row_end = of_shared ? s.end : uni(t.off[e + 1]), mt_e = x.tiles;
-    int m_tile, n_tile;
-    tile_in_expert(at - x.first * g.n_tiles_n, mt_e, g.n_tiles_n, m_tile, n_tile);
-    int r0, r1;
-    bool neighbours = true;
-    if (piece >= 0) {                    // of a 256-row tile of the persistent body's space
-        r0 = o0 + m_tile * 256 + piece * piece_rows(tail.pieces);
-        r1 = min(min(row_end, o0 + (m_tile + 1) * 256), r0 + piece_rows(tail.pieces));
-        if (r0 >= r1) {
-            claims.ask();
-            continue;
+        const int* pref = t.own;
+        int piece = -1, shared = 0, at = v;   // shared: tiles of the shared expert in front of the routed experts' in the space `at` counts in
+        bool of_shared = false;
+        if (v >= own + s.own) {              // a piece of one of the last persistent tiles
+            const int h = v - own - s.own, of = h / tail.pieces;
+            at = total_p - tail.tiles + of;
+            piece = h - of * tail.pieces;
+            pref = t.persistent;
+            shared = s.persistent;
+            of_shared = at < shared;
+            if (!of_shared) at -= shared;
+        } else if (v >= own) {
+            at = v - own;
+            shared = s.own;
+            of_shared = true;
         }
-    } else {
-        const int first_row = o0 + (g.rem_split ? ((row_end - o0) & ~255) : 0), rows_e = row_end - first_row;
-        const int slice = !W8 && rows_e >= PAIR_LO ? half_rows(rows_e) : 128;
-        r0 = mt_e > 1 ? first_row + m_tile * slice : first_row;
-        r1 = mt_e > 1 ? min(row_end, r0 + slice) : row_end;
-        neighbours = mt_e > 1;
-    }
-    if (W8) stream8x<SWIGLU>(g, lds, e, r0, r1, n_tile, false, claims);
-    else if (neighbours) stream16<SWIGLU, true>(g, lds.w0, lds.w1, lds.w2, lds.t0, lds.t1, e, r0, r1, n_tile, claims);
-    else stream16<SWIGLU, false>(g, lds.w0, lds.w1, lds.w2, lds.t0, lds.t1, e, r0, r1, n_tile, claims);
+        int which = uni(of_shared ? 1 : 0);
+        asm volatile("" : "+s"(which));      // (else the arguments of both problems are loaded and prepared in front of the loop)
+        const GemmArgs& g = pair_of.p[which];
+        const ExpertAt x = of_shared ? ExpertAt{0, 0, shared / g.n_tiles_n} : expert_at(pref, g.E, at / g.n_tiles_n);
+        const int e = x.e, o0 = of_shared ? s.first : uni(t.off[e]), row_end = of_shared ? s.end : uni(t.off[e + 1]), mt_e = x.tiles;
+        int m_tile, n_tile;
+        tile_in_expert(at - x.first * g.n_tiles_n, mt_e, g.n_tiles_n, m_tile, n_tile);
+        int r0, r1;
+        bool neighbours = true;
+        if (piece >= 0) {                    // of a 256-row tile of the persistent body's space
+            r0 = o0 + m_tile * 256 + piece * piece_rows(tail.pieces);
+            r1 = min(min(row_end, o0 + (m_tile + 1) * 256), r0 + piece_rows(tail.pieces));
+            if (r0 >= r1) {
+                claims.ask();
+                continue;
+            }
+        } else {
+            const int first_row = o0 + (g.rem_split ? ((row_end - o0) & ~255) : 0), rows_e = row_end - first_row;
+            const int slice = !W8 && rows_e >= PAIR_LO ? half_rows(rows_e) : 128;
+            r0 = mt_e > 1 ? first_row + m_tile * slice : first_row;
+            r1 = mt_e > 1 ? min(row_end, r0 + slice) : row_end;
+            neighbours = mt_e > 1;
+        }
+        if (W8) stream8x<SWIGLU>(g, lds, e, r0, r1, n_tile, false, claims);
+        else if (neighbours) stream16<SWIGLU, true>(g, lds.w0, lds.w1, lds.w2, lds.t0, lds.t1, e, r0, r1, n_tile, claims);
+        else stream16<SWIGLU, false>(g, lds.w0, lds.w1, lds.w2, lds.t0, lds.t1, e, r0, r1, n_tile, claims);
     }
 }
 // CLAIMS: the call may bring counters.  Calls that do not (one MLP, the stand-alone entry points) have an instantiation without the loop:
@@ -3149,8 +3149,8 @@ bool both_kinds_of(bool w8, const moe_mlp_group& m, int32_t hidden) {
 // Whether a joint call has tiles of both kinds: the routed experts' call would, and the persistent body can address both problems.
 // (Where it cannot, for sizes that are odd multiples of 64, the call has one kind of tiles, like one of a lower mean.)
 bool joint_both(bool w8, const moe_mlp_group& routed, const moe_mlp_group& shared, int32_t hidden) {
-    return both_kinds_of(w8, routed, hidden) && shared.n_rows >= 128 && hidden % 128 == 0 && routed.inter % 128 == 0 && shared.inter % 128 == 0 && routed.n_experts <= 512 &&
-           cu_count() >= 8;
+    return both_kinds_of(w8, routed, hidden) && shared.n_rows >= 128 && hidden % 128 == 0 && routed.inter % 128 == 0 &&
+           shared.inter % 128 == 0 && routed.n_experts <= 512 && cu_count() >= 8;
 }
 
 // Whether the shared expert's tiles join the routed experts' launches.  Where the joint call has both kinds of tiles they do if a
