@@ -728,7 +728,8 @@ struct TileLds {
 // with the mean: below 128 rows the call has to be long enough for the one, and its rows enough for the other.  Layers, us, one kind ->
 // both.  Above the line: 160 experts, DeepSeek-V2-236B, 900 / 1500 / 2500 tokens (means of 33 to 93 rows) skewed 1403 / 1591 / 1911 -> 1357 / 1491 /
 // 1693, even 1405 / 1518 / 1704 -> 1336 / 1467 / 1644; 64, DeepSeek-V2-Lite, 920 / 1100 / 1300 skewed 284 / 310 / 340 -> 277 / 301 / 332, even the
-// same.  Below it (hidden x intermediate size): 64 experts, 2048 x 1024, 939 tokens 225 -> 241, 1024 x 1024 119 -> 142, 2048 x 768, 1259 202 -> 211; 128,
+// same; 96 of 5120 x 1536 (hidden x intermediate size), 689 / 961 (43 / 60 rows) skewed 914 / 1025 -> 878 / 980, even 916 / 970 -> 847 / 908.  Below it:
+// 64 experts, 2048 x 1024, 939 tokens 225 -> 241, 1024 x 1024 119 -> 142, 2048 x 768, 1259 202 -> 211; 128,
 // 2048 x 512, 726 149 -> 156; 256, 1024 x 384, 1451 107 -> 117.  32 experts, above it too: 2048 x 4096, 470 / 630 415 / 461 -> 442 / 470.  138 calls of
 // 64 to 256 experts, even and skewed: above it both kinds are 3.9 per cent faster in the mean, 1.6 slower at most; below it 1.8 slower.
 template <bool W8>
